@@ -1,0 +1,512 @@
+// Grouped GEMM for launches that do not fill the chip with large tiles: small batches, generation, short training batches.
+//
+// Same operands, packed weights and epilogues as grouped_gemm.hip (bf16 and OCP fp8, row maps on either side, activations,
+// kept pre-activations, block-quantised hidden activations).  What differs is the shape of the work: one tile of BM x 128
+// outputs per workgroup of four waves, several workgroups per compute unit (the barriers and epilogues of one run under the
+// MFMAs of the others), a plain ring of LDS stages, and the K range of every tile cut into P parts when there are fewer tiles
+// than workgroups the chip can hold.  The parts of a tile leave their fp32 sums in the workspace; the workgroup that finishes
+// last adds them in part order (so the result does not depend on who that is) and applies the epilogue: one launch, where
+// the large-tile path needs a launch for whole tiles, one for the parts and one for their reduction.
+#include "gg_common.h"
+#include <algorithm>
+#include <atomic>
+#include <math.h>
+#include <time.h>
+#include <type_traits>
+
+namespace moe_gg {
+
+constexpr int GS_BN = 128;
+constexpr int GS_THREADS = 256;
+constexpr int GS_CTR_BYTES = 16384;  // arrival counters at the start of the workspace: one 64-bit word per tile
+constexpr int GS_MIN_PART_STAGES = 32;  // K stages per part at least: what the hand-over of a split tile costs is worth about as many
+constexpr int GS_LDO = GS_BN + 4;    // pitch of the epilogue's fp32 tile in LDS
+
+template <int BM>
+struct GsShape {
+    static constexpr int WM = BM == 32 ? 1 : 2, WN = 4 / WM;  // waves along rows and columns
+    static constexpr int WR = BM / WM, WC = GS_BN / WN;       // rows and columns of a wave
+    static constexpr int NST = 3;                             // ring slots, a pair of 64-byte stages each (two workgroups fit a compute unit)
+    static constexpr int RA = BM < 64 ? 1 : BM / 64;          // activation loads per wave and stage (1 KB each)
+    static constexpr int RB = GS_BN / 64;
+};
+template <int BM, bool BSA>
+constexpr int gs_lds_bytes() {
+    using S = GsShape<BM>;
+    const int ring = S::NST * (BM + GS_BN) * 2 * ROWB + (BSA ? 4 * S::NST * 256 : 0);
+    const int epi = BM * GS_LDO * 4;
+    return ring > epi ? ring : epi;
+}
+
+struct GsParams {
+    GemmParams g;
+    int ncols;                 // packed columns that exist (N, or 2 N for SwiGLU)
+    int slots;                 // units up to which tiles are split: one workgroup per compute unit
+    unsigned long long nonce;  // what this launch's arrival counters carry in their upper bits
+};
+
+// How many parts every tile's K range is cut into.
+__host__ __device__ inline int gs_parts(long long tiles, int slots, int nk, int max_units) {
+    if (tiles <= 0) return 1;
+    const long long most = slots < max_units ? slots : max_units;
+    int P = (int)(most / tiles < GG_MAX_PARTS ? most / tiles : GG_MAX_PARTS);
+    while (P > 1 && (gg_part_stages(nk, P) < GS_MIN_PART_STAGES || (P - 1) * gg_part_stages(nk, P) >= nk)) --P;
+    return P < 1 ? 1 : P;
+}
+
+__device__ __forceinline__ int gs_scan(int v) {
+#pragma unroll
+    for (int off = 1; off < WAVE; off <<= 1) {
+        const int o = __shfl_up(v, off, WAVE);
+        if (lane_id() >= off) v += o;
+    }
+    return v;
+}
+
+template <int BM, bool FP8, int EPI, bool BSA>
+__global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParams q) {
+    using S = GsShape<BM>;
+    constexpr int ES = FP8 ? 1 : 2;
+    constexpr int MT = FP8 ? 32 : 16, CF = FP8 ? 2 : 1;
+    constexpr int TM = S::WR / MT, TN = S::WC / MT;
+    constexpr int NST = S::NST, RA = S::RA, RB = S::RB;
+    constexpr int LPS = 2 * (RA + RB) + (BSA ? 1 : 0);
+    constexpr int ASZ = BM * ROWB, BSZ = GS_BN * ROWB;  // bytes of a stage (a ring slot holds two)
+    constexpr bool QOUT = FP8 && EPI == EPI_SWIGLU;
+    static_assert(TM >= 1 && TN >= 1, "wave tile");
+    extern __shared__ __align__(1024) uint8_t lds[];
+    __shared__ int s_last;
+    const GemmParams& p = q.g;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / S::WN, wn = wave % S::WN;
+
+    // ---- this workgroup's unit: group, column tile, row tile, part.  Every wave scans the row counts by itself (64 groups at
+    // a time); counts that claim more rows than the buffers hold are cut at S_rows.
+    const int nt_all = (q.ncols + GS_BN - 1) / GS_BN;
+    int mt_all = 0;
+    {
+        int rows = 0;
+        for (int g0 = 0; g0 < p.E_l; g0 += WAVE) {
+            const int c = g0 + lane < p.E_l ? max(p.cnt[g0 + lane], 0) : 0;
+            const int inc = gs_scan(c), rs = min(rows + inc - c, p.S_rows);
+            const int t = (min(c, p.S_rows - rs) + BM - 1) / BM;
+            int ts = t;
+#pragma unroll
+            for (int off = 1; off < WAVE; off <<= 1) ts += __shfl_xor(ts, off, WAVE);
+            mt_all += ts;
+            rows = min(rows + __shfl(inc, WAVE - 1, WAVE), p.S_rows);
+        }
+    }
+    const int nk = (p.K * ES) / ROWB;
+    const int P = __builtin_amdgcn_readfirstlane(p.part_ws ? gs_parts((long long)mt_all * nt_all, q.slots, nk, p.max_units) : 1);
+    const int units = __builtin_amdgcn_readfirstlane(mt_all * nt_all * P);
+    // consecutive units share an XCD (workgroups b, b + 8, ... do): parts of a tile, then the row tiles of a weight panel
+    const int per = (units + 7) / 8;
+    const int unit = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
+    if (((int)blockIdx.x >> 3) >= per || unit >= units) return;
+    const int tile = unit / P, part = unit % P;
+    int g = 0, row0 = 0, rv = 0, nt = 0;
+    {
+        int rows = 0, tiles = 0;
+        for (int g0 = 0; g0 < p.E_l; g0 += WAVE) {
+            const int c = g0 + lane < p.E_l ? max(p.cnt[g0 + lane], 0) : 0;
+            const int inc = gs_scan(c), rs = min(rows + inc - c, p.S_rows);
+            const int cc = min(c, p.S_rows - rs);
+            const int mt = (cc + BM - 1) / BM;
+            const int ti = gs_scan(mt), t0 = (tiles + ti - mt) * nt_all;
+            const unsigned long long hit = __ballot(mt > 0 && tile >= t0 && tile < t0 + mt * nt_all);
+            if (hit) {
+                const int l = __builtin_ctzll(hit);
+                const int mt_g = __shfl(mt, l, WAVE), in = tile - __shfl(t0, l, WAVE);
+                g = g0 + l;
+                nt = in / mt_g;
+                const int m = in % mt_g;
+                row0 = __shfl(rs, l, WAVE) + m * BM;
+                rv = min(BM, __shfl(cc, l, WAVE) - m * BM);
+                break;
+            }
+            rows = min(rows + __shfl(inc, WAVE - 1, WAVE), p.S_rows);
+            tiles += __shfl(ti, WAVE - 1, WAVE);
+        }
+    }
+    g = __builtin_amdgcn_readfirstlane(g); nt = __builtin_amdgcn_readfirstlane(nt);
+    row0 = __builtin_amdgcn_readfirstlane(row0); rv = __builtin_amdgcn_readfirstlane(rv);
+    const int nkp = P > 1 ? gg_part_stages(nk, P) : nk;
+    const int ks0 = part * nkp, nks = min(nkp, nk - ks0);
+
+    // ---- addresses.  LDS tiles as in the large kernel: 64-byte rows, chunk c of row r at position c ^ ((r >> 2) & 3).
+    const int lchunk = (lane & 3) ^ ((lane >> 4) & 3);
+    const uint32_t ldk = (uint32_t)(p.K * ES);
+    const uint8_t* Ab = (p.a_map ? p.A : p.A + (size_t)row0 * ldk) + (size_t)ks0 * ROWB;
+    const size_t b_slab = (size_t)p.Npad * ROWB;
+    const uint8_t* Bb = p.B + (size_t)g * p.Npad * ldk + (size_t)nt * GS_BN * ROWB + (size_t)ks0 * b_slab;
+    uint32_t aoff[RA], boff[RB];
+#pragma unroll
+    for (int r = 0; r < RA; ++r) {
+        const int wr = BM < 64 ? (wave & 1) : wave;  // (32 rows: two waves move them, the other two repeat that)
+        const int lr = min(r * 64 + wr * WROWS + (lane >> 2), rv - 1);
+        aoff[r] = (uint32_t)(p.a_map ? max(p.a_map[row0 + lr], 0) : lr) * ldk + lchunk * 16;
+    }
+#pragma unroll
+    for (int r = 0; r < RB; ++r) boff[r] = (uint32_t)(r * 64 + wave * WROWS + (lane >> 2)) * ROWB + lchunk * 16;
+    uint8_t* const sA = lds;
+    uint8_t* const sB = lds + NST * 2 * ASZ;
+    uint32_t* const sS = (uint32_t*)(lds + NST * 2 * (ASZ + BSZ)) + wave * NST * 64;  // (BSA) the wave's scale dwords, one per row
+    const uint32_t la0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr_t)sA) + (BM < 64 ? (wave & 1) : wave) * WROWS * ROWB;
+    const uint32_t lb0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr_t)sB) + wave * WROWS * ROWB;
+    [[maybe_unused]] const uint32_t ls0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr_t)sS);
+    [[maybe_unused]] const uint32_t soff = BSA ? (uint32_t)(row0 + min(wm * S::WR + (lane & (S::WR - 1)), rv - 1)) * (uint32_t)p.bs_pitch : 0u;
+
+    const int npair = nks / 2;
+    // load d (0 .. LPS - 1) of the pair whose first stage lies at ap / bp: activations, weights, (BSA) scale dwords
+    auto load = [&](int d, const uint8_t* ap, const uint8_t* bp, const uint8_t* sp, int slot) {
+        if (d < 2 * RA) gg_dma16(ap + (d & 1) * ROWB, aoff[d >> 1], la0 + slot * 2 * ASZ + (d & 1) * ASZ + (d >> 1) * 64 * ROWB);
+        else if (d < 2 * (RA + RB)) {
+            const int e = d - 2 * RA;
+            gg_dma16(bp + (e / RB) * b_slab, boff[e % RB], lb0 + slot * 2 * BSZ + (e / RB) * BSZ + (e % RB) * 64 * ROWB);
+        } else if constexpr (BSA) gg_dma4(sp, soff, ls0 + slot * 256);
+    };
+#define GS_PAIR_PTRS(pr)                                                    \
+    const int st_ = 2 * min((pr), npair - 1);                               \
+    const uint8_t* ap_ = gg_uniform(Ab + (size_t)st_ * ROWB);               \
+    const uint8_t* bp_ = gg_uniform(Bb + (size_t)st_ * b_slab);             \
+    const uint8_t* sp_ = BSA ? gg_uniform(p.a_bscale + (((ks0 + st_) >> 1) << 2)) : nullptr;
+
+    typedef typename std::conditional<FP8, floatx16, floatx4>::type acc_t;
+    acc_t acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int v = 0; v < (FP8 ? 16 : 4); ++v) acc[i][j][v] = 0.f;
+
+    // ---- K loop.  While a pair of stages is multiplied, the fragments of the next one are read into the other set of registers
+    // and the pair NST behind it is requested into the slot that has just been read out; one barrier per pair (it says that the
+    // next pair's loads of every wave have landed and that nobody reads the slot the new loads go to any more).
+    const int fpos = (FP8 ? (lane >> 5) : (lane >> 4)) ^ ((lane >> 2) & 3);
+    const uint4* fa = (const uint4*)sA + (wm * S::WR + (lane & (MT - 1))) * CHUNKS;
+    const uint4* fb = (const uint4*)sB + (wn * S::WC + (lane & (MT - 1))) * CHUNKS;
+    struct Frag {
+        uint4 a[2][TM][CF], b[2][TN][CF];
+        uint32_t sc[TM];
+    } f0, f1;
+    auto read = [&](Frag& f, int slot) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const uint4* as = fa + (slot * 2 + u) * (ASZ / 16);
+            const uint4* bs = fb + (slot * 2 + u) * (BSZ / 16);
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int h = 0; h < CF; ++h) f.b[u][j][h] = bs[j * MT * CHUNKS + (fpos ^ (2 * h))];
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int h = 0; h < CF; ++h) f.a[u][i][h] = as[i * MT * CHUNKS + (fpos ^ (2 * h))];
+        }
+        if constexpr (BSA) {
+            // lane 32 h + r: the scale bytes of row r, block h of either stage (see mma_fp8_k64_bs), in bytes 0 and 2
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+                f.sc[i] = ((sS[slot * 64 + i * MT + (lane & 31)] >> ((lane >> 5) * 8)) & 0x00ff00ffu) + (uint32_t)(127 - GG_WSCALE) * 0x00010001u;
+        }
+    };
+#pragma unroll
+    for (int d = 0; d < NST; ++d) {
+        GS_PAIR_PTRS(d)
+#pragma unroll
+        for (int l = 0; l < LPS; ++l) load(l, ap_, bp_, sp_, d);
+    }
+    gg_wait<(NST - 1) * LPS, 0>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    read(f0, 0);
+    int slot = 0;
+    // The loads go between the MFMAs: issued in one go they keep the wave from its MFMAs for as long as the load path needs
+    // to take them (64 bytes a cycle and compute unit).
+    auto step = [&](const Frag& f, Frag& nxt, int s) {
+        asm volatile("" ::: "memory");
+        gg_wait<(NST - 2) * LPS, 0>();
+        __builtin_amdgcn_s_barrier();
+        GS_PAIR_PTRS(s + NST)
+        const int fill = slot;
+        slot = slot == NST - 1 ? 0 : slot + 1;
+        asm volatile("" ::: "memory");
+        read(nxt, slot);
+        __builtin_amdgcn_sched_barrier(0);
+        constexpr int NM = 2 * TM * TN, STEP = NM / LPS > 0 ? NM / LPS : 1, PER = (LPS + NM - 1) / NM;  // MFMAs per load, loads per MFMA
+#pragma unroll
+        for (int m = 0; m < NM; ++m) {
+            const int u = m / (TM * TN), i = (m % (TM * TN)) / TN, jj = m % TN, j = (i & 1) ? TN - 1 - jj : jj;
+            if constexpr (FP8 && BSA) {
+                if (u == 0) mma_fp8_k64_bs<false, 0>(acc[i][j], f.b[u][j][0], f.b[u][j][CF - 1], f.a[u][i][0], f.a[u][i][CF - 1], (int)f.sc[i]);
+                else mma_fp8_k64_bs<false, 2>(acc[i][j], f.b[u][j][0], f.b[u][j][CF - 1], f.a[u][i][0], f.a[u][i][CF - 1], (int)f.sc[i]);
+            } else if constexpr (FP8) mma_fp8_k64(acc[i][j], f.b[u][j][0], f.b[u][j][CF - 1], f.a[u][i][0], f.a[u][i][CF - 1]);
+            else mma_bf16_k32(acc[i][j], f.b[u][j][0], f.a[u][i][0]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int e = 0; e < PER; ++e) {
+                const int d = PER > 1 ? m * PER + e : m % STEP == 0 ? m / STEP : LPS;
+                if (d < LPS) load(d, ap_, bp_, sp_, fill);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    for (int s = 0; s < npair; s += 2) {
+        step(f0, f1, s);
+        if (s + 1 < npair) step(f1, f0, s + 1);
+    }
+    asm volatile("" ::: "memory");
+    gg_wait<0, 0>();
+    __syncthreads();
+
+    // ---- epilogue, row by row: the accumulators change into row-major order in LDS, then a thread takes eight consecutive output
+    // columns of a row.  Parts write their sums to the workspace instead; the last one of a tile goes through the same code
+    // with the sums read back from there.
+    float* const so = (float*)lds;
+    constexpr int OCW = EPI == EPI_SWIGLU ? GS_BN / 2 : GS_BN;  // output columns of the tile
+    constexpr int TPR = OCW / 8, RPP = GS_THREADS / TPR;         // threads per row, rows per pass
+    const int oc = (tid % TPR) * 8;                              // the thread's first output column inside the tile
+    const int pc = EPI == EPI_SWIGLU ? (oc / 32) * 64 + oc % 32 : oc;  // its packed column inside the tile
+    const int gp = nt * GS_BN + pc;
+    const int col = EPI == EPI_SWIGLU ? (gp / 64) * 32 + gp % 32 : gp;
+    float cg[8], cu[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) cg[e] = cu[e] = 1.f;
+    if constexpr (FP8) {
+        if (col < p.N) {
+            const float4* c0 = (const float4*)(p.col_scale + (size_t)g * p.ncs + col);
+            const float4 u0 = c0[0], u1 = c0[1];
+            cg[0] = u0.x; cg[1] = u0.y; cg[2] = u0.z; cg[3] = u0.w; cg[4] = u1.x; cg[5] = u1.y; cg[6] = u1.z; cg[7] = u1.w;
+            if constexpr (EPI == EPI_SWIGLU) {
+                const float4* c1 = (const float4*)(p.col_scale2 + (size_t)g * p.ncs + col);
+                const float4 v0 = c1[0], v1 = c1[1];
+                cu[0] = v0.x; cu[1] = v0.y; cu[2] = v0.z; cu[3] = v0.w; cu[4] = v1.x; cu[5] = v1.y; cu[6] = v1.z; cu[7] = v1.w;
+            }
+        }
+    }
+    auto finish = [&](int r, const float* x0, const float* x1) {  // row r of the tile; x0: the eight (gate) sums, x1: the up sums
+        const int grow = row0 + min(r, rv - 1);
+        const int crow = p.c_map ? p.c_map[grow] : grow;
+        float rs = 1.f;
+        if constexpr (FP8 || EPI == EPI_GATE) rs = p.row_scale ? p.row_scale[grow] : 1.f;
+        float y[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            float v = x0[e];
+            if constexpr (FP8) v *= cg[e] * rs;
+            if constexpr (!FP8 && EPI == EPI_GATE) v *= rs;
+            if constexpr (EPI == EPI_SWIGLU) {
+                float u = x1[e];
+                if constexpr (FP8) u *= cu[e] * rs;
+                v = act_silu_fast(v) * u;
+            }
+            if constexpr (EPI == EPI_GELU) v = act_gelu(v);
+            if constexpr (EPI == EPI_SILU) v = act_silu_fast(v);
+            y[e] = v;
+        }
+        if constexpr (QOUT) {  // four threads hold a block of 32 columns: one scale byte, 32 codes
+            float am = 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) am = fmaxf(am, fabsf(y[e]));
+            if (col >= p.N) am = 0.f;
+            am = fmaxf(am, __shfl_xor(am, 1, WAVE));
+            am = fmaxf(am, __shfl_xor(am, 2, WAVE));
+            const int sbyte = gg_block_scale_byte(__float_as_uint(am));
+            const float inv = __uint_as_float(gg_block_inv_bits(sbyte));
+            int lo = 0, hi = 0;
+            lo = __builtin_amdgcn_cvt_pk_fp8_f32(__fmul_rn(y[0], inv), __fmul_rn(y[1], inv), lo, false);
+            lo = __builtin_amdgcn_cvt_pk_fp8_f32(__fmul_rn(y[2], inv), __fmul_rn(y[3], inv), lo, true);
+            hi = __builtin_amdgcn_cvt_pk_fp8_f32(__fmul_rn(y[4], inv), __fmul_rn(y[5], inv), hi, false);
+            hi = __builtin_amdgcn_cvt_pk_fp8_f32(__fmul_rn(y[6], inv), __fmul_rn(y[7], inv), hi, true);
+            if (r < rv && crow >= 0 && col < p.N) {
+                *(uint2*)((uint8_t*)p.C + (size_t)crow * p.ldc + col) = make_uint2((uint32_t)lo, (uint32_t)hi);
+                if ((col & 31) == 0) p.c_bscale[(size_t)crow * p.bs_pitch + col / 32] = (uint8_t)sbyte;
+            }
+            return;
+        }
+        if (r >= rv || crow < 0 || col >= p.N) return;
+        *(uint4*)((bf16_t*)p.C + (size_t)crow * p.ldc + col) =
+            make_uint4(gg_pack_bf16(y[0], y[1]), gg_pack_bf16(y[2], y[3]), gg_pack_bf16(y[4], y[5]), gg_pack_bf16(y[6], y[7]));
+        if constexpr (!FP8 && EPI != EPI_NONE && EPI != EPI_GATE) {
+            if (p.C2) {  // the values before the activation (rows are never remapped where they are kept)
+                constexpr int W2 = EPI == EPI_SWIGLU ? 2 : 1;
+                bf16_t* r2 = (bf16_t*)p.C2 + (size_t)crow * p.ldc * W2 + (EPI == EPI_SWIGLU ? gp : col);
+                *(uint4*)r2 = make_uint4(gg_pack_bf16(x0[0], x0[1]), gg_pack_bf16(x0[2], x0[3]), gg_pack_bf16(x0[4], x0[5]), gg_pack_bf16(x0[6], x0[7]));
+                if constexpr (EPI == EPI_SWIGLU)
+                    *(uint4*)(r2 + 32) = make_uint4(gg_pack_bf16(x1[0], x1[1]), gg_pack_bf16(x1[2], x1[3]), gg_pack_bf16(x1[4], x1[5]), gg_pack_bf16(x1[6], x1[7]));
+            }
+        }
+    };
+    float* const ws = P > 1 ? (float*)((uint8_t*)p.part_ws + GS_CTR_BYTES) : nullptr;
+    constexpr int NQ = FP8 ? 4 : 1;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int v = 0; v < NQ; ++v) {
+                // four consecutive rows of the weight tile are four consecutive columns
+                const int r = wm * S::WR + i * MT + (lane & (MT - 1));
+                const int c = gg_packed_col<FP8>(wn * S::WC + j * MT + (FP8 ? 8 * v + 4 * (lane >> 5) : 4 * (lane >> 4)));
+                *(float4*)(so + r * GS_LDO + c) = make_float4(acc[i][j][4 * v], acc[i][j][4 * v + 1], acc[i][j][4 * v + 2], acc[i][j][4 * v + 3]);
+            }
+    __syncthreads();
+    // (whole passes of RPP rows: the threads that hold a block of columns of a row stay together)
+    const int r_end = min((rv + RPP - 1) & ~(RPP - 1), BM);
+    if (P == 1) {
+        for (int r = tid / TPR; r < r_end; r += RPP) {
+            float x0[8], x1[8];
+            *(float4*)x0 = *(const float4*)(so + r * GS_LDO + pc);
+            *(float4*)(x0 + 4) = *(const float4*)(so + r * GS_LDO + pc + 4);
+            if constexpr (EPI == EPI_SWIGLU) {
+                *(float4*)x1 = *(const float4*)(so + r * GS_LDO + pc + 32);
+                *(float4*)(x1 + 4) = *(const float4*)(so + r * GS_LDO + pc + 36);
+            }
+            finish(r, x0, x1);
+        }
+        return;
+    }
+    unsigned long long* const o = (unsigned long long*)(ws + (size_t)unit * (BM * GS_BN));
+    for (int i = tid; i < rv * (GS_BN / 2); i += GS_THREADS)
+        __hip_atomic_store(o + i, *(const unsigned long long*)(so + (i / (GS_BN / 2)) * GS_LDO + 2 * (i % (GS_BN / 2))), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    // arrival: the sums above are written through to memory; once they are acknowledged the part counts itself in.  The
+    // counter starts from whatever the workspace holds: only a word that carries this launch's nonce counts.
+    gg_wait<0, 0>();
+    __syncthreads();
+    if (tid == 0) {
+        unsigned long long* ctr = (unsigned long long*)p.part_ws + tile;
+        unsigned long long seen = __hip_atomic_load(ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        while ((seen >> 8) != q.nonce)  // the first to arrive starts the count (once it has, the others add to it without a retry)
+            if (__hip_atomic_compare_exchange_strong(ctr, &seen, q.nonce << 8, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) break;
+        const bool last = (int)(__hip_atomic_fetch_add(ctr, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 255) == P - 1;
+        // (the last part leaves a word without the nonce: a replay of a captured launch carries the same one)
+        if (last) __hip_atomic_store(ctr, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        s_last = last;
+    }
+    __syncthreads();
+    if (!s_last) return;
+    const float* w0 = ws + (size_t)tile * P * (BM * GS_BN);
+    for (int r = tid / TPR; r < r_end; r += RPP) {
+        float x0[8], x1[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x0[e] = x1[e] = 0.f;
+        if (r < rv) {
+            const unsigned long long* w = (const unsigned long long*)(w0 + (size_t)r * GS_BN + pc);
+            constexpr int NV = EPI == EPI_SWIGLU ? 8 : 4, PU = 32 / NV;  // 64-bit loads per part; parts requested together
+            for (int k0 = 0; k0 < P; k0 += PU) {
+                unsigned long long v[PU][NV];
+#pragma unroll
+                for (int k = 0; k < PU; ++k)
+                    if (k0 + k < P)
+#pragma unroll
+                        for (int e = 0; e < NV; ++e)
+                            v[k][e] = __hip_atomic_load(w + (size_t)(k0 + k) * (BM * GS_BN / 2) + (e & 3) + (e >> 2) * 16, __ATOMIC_RELAXED,
+                                                        __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+                for (int k = 0; k < PU; ++k)
+                    if (k0 + k < P)
+#pragma unroll
+                        for (int e = 0; e < NV; ++e) {
+                            float* x = (e >> 2 ? x1 : x0) + 2 * (e & 3);
+                            x[0] += __uint_as_float((uint32_t)v[k][e]);
+                            x[1] += __uint_as_float((uint32_t)(v[k][e] >> 32));
+                        }
+            }
+        }
+        finish(r, x0, x1);
+    }
+}
+
+// A number no earlier launch of this process used (and no stale workspace word is likely to hold): 56 bits.
+static unsigned long long gs_nonce() {
+    static const unsigned long long base = [] {
+        unsigned long long z = (unsigned long long)(uintptr_t)&gs_nonce ^ (unsigned long long)clock() * 0x9e3779b97f4a7c15ull;
+        z = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ull;
+        z = (z ^ (z >> 27)) * 0x94d049bb133111ebull;
+        return (z ^ (z >> 31)) | (1ull << 40);
+    }();
+    static std::atomic<unsigned long long> n{0};
+    return (base + n.fetch_add(1, std::memory_order_relaxed)) & ((1ull << 56) - 1);
+}
+
+template <int BM, bool FP8, int EPI, bool BSA>
+static void gs_launch(const GsParams& q0, void* part_ws, size_t part_ws_bytes, int cus, hipStream_t s) {
+    GsParams q = q0;
+    constexpr int lds = gs_lds_bytes<BM, BSA>();
+    q.slots = (int)std::min<long long>(cus, (8 << 20) / (BM * GS_BN * 4));  // (units worth splitting for)
+    q.g.part_ws = nullptr;
+    q.g.max_units = 0;
+    const long long unit_bytes = (long long)BM * GS_BN * 4;
+    if (part_ws && part_ws_bytes > (size_t)GS_CTR_BYTES) {
+        q.g.max_units = (int)std::min<long long>((long long)(part_ws_bytes - GS_CTR_BYTES) / unit_bytes, GS_CTR_BYTES / 8);
+        q.g.part_ws = (float*)part_ws;
+    }
+    const int nt = (q.ncols + GS_BN - 1) / GS_BN;
+    const long long ub = ((long long)q.g.S_rows + (long long)std::min(q.g.E_l, q.g.S_rows) * (BM - 1)) / BM * nt;  // most tiles there can be
+    const long long units = std::max<long long>(ub, q.g.part_ws ? std::min<long long>(q.slots, ub * GG_MAX_PARTS) : 0);
+    q.nonce = gs_nonce();
+    gemm_small_kernel<BM, FP8, EPI, BSA><<<(unsigned)((units + 7) / 8 * 8), GS_THREADS, lds, s>>>(q);
+}
+
+template <bool FP8>
+static int gs_dispatch(const GsParams& q, int bm, int epi, void* ws, size_t bytes, int cus, hipStream_t s) {
+#define GS_BM(EPIv, BSAv)                                                              \
+    do {                                                                               \
+        if (bm == 32) gs_launch<32, FP8, EPIv, BSAv>(q, ws, bytes, cus, s);            \
+        else gs_launch<64, FP8, EPIv, BSAv>(q, ws, bytes, cus, s);                     \
+    } while (0)
+    if constexpr (FP8) {
+        if (epi == EPI_NONE) GS_BM(EPI_NONE, true);
+        else GS_BM(EPI_SWIGLU, false);
+    } else {
+        switch (epi) {
+            case EPI_NONE: GS_BM(EPI_NONE, false); break;
+            case EPI_GELU: GS_BM(EPI_GELU, false); break;
+            case EPI_SILU: GS_BM(EPI_SILU, false); break;
+            case EPI_SWIGLU: GS_BM(EPI_SWIGLU, false); break;
+            default: GS_BM(EPI_GATE, false); break;
+        }
+    }
+#undef GS_BM
+    return moe_check_launch("grouped_gemm");
+}
+
+// Tile height for a launch (32 or 64 rows), or 0: large tiles.  Both paths' times in us are estimated from what the host knows
+// -- the row total, not its split over the groups (every group adds about half a tile of ragged tail) -- with coefficients
+// fitted to 90 launches drawn over rows 16 .. 16384, 1 .. 32 groups, K and N 512 .. 8192, bf16 and fp8, even and skewed:
+//   large tiles: rounds of the persistent grid, each 0.70 us (256 rows) or 0.45 us (128 rows) per 64 bytes of K, 4 us between
+//     tiles, 14 us for a launch with its K-split and reduction launches;
+//   small tiles: 0.26 / 0.29 us per 128 bytes of K while every workgroup has a compute unit to itself, then in proportion to
+//     their number (times 1.2, fp8 1.4: the load path is shared); 5 us for the hand-over of a split tile.
+// Over those launches the choice made from these estimates is within 2 % (geometric mean) of the better of the two, and 1.4 times
+// faster than large tiles alone: 27.5 -> 9.0 us at 512 rows x 1024 x 1024 (2 groups, bf16), 31 -> 21 us at 512 x 2048 x 4096,
+// 49 -> 20 us for an fp8 MLP of 300 rows; the line lies at one to two rounds of large tiles.
+int gs_choose_bm(int S_rows, int E_l, int K, int ncols, bool fp8, int cus) {
+    const double E = std::min(E_l, S_rows), nk = (double)K * (fp8 ? 1 : 2) / ROWB;
+    const int nt = (ncols + GG_BN - 1) / GG_BN, nts = (ncols + GS_BN - 1) / GS_BN;
+    const double r256 = ceil((S_rows / 256.0 + 0.5 * E) * nt / cus), r128 = ceil((S_rows / 128.0 + 0.5 * E) * nt / cus);
+    const bool small_m = 0.62 * r128 < r256;
+    double best = 14 + (small_m ? r128 : r256) * (nk * (small_m ? 0.45 : 0.70) + 4);
+    int bm_best = 0;
+    for (int bm : {32, 64}) {
+        const double units = (S_rows / (double)bm + 0.5 * E) * nts;
+        const double P = units < cus ? std::max(1.0, std::min(std::min(floor(cus / units), floor(nk / GS_MIN_PART_STAGES)), (double)GG_MAX_PARTS)) : 1.0;
+        const double x = units * P / cus, share = x <= 1 ? 1.0 : std::max(1.0, x * (fp8 ? 1.4 : 1.2));
+        const double t = 6 + (P > 1 ? 5 : 0) + nk / 2 / P * (bm == 32 ? 0.26 : 0.29) * share + 2 * std::max(1.0, x / 2);
+        if (t < best) { best = t; bm_best = bm; }
+    }
+    return bm_best;
+}
+
+int launch_gemm_small(const GemmParams& p, bool fp8, int bm, int epi, void* ws, size_t bytes, int cus, hipStream_t s) {
+    GsParams q{};
+    q.g = p;
+    q.ncols = epi == EPI_SWIGLU ? 2 * p.N : p.N;
+    return fp8 ? gs_dispatch<true>(q, bm, epi, ws, bytes, cus, s) : gs_dispatch<false>(q, bm, epi, ws, bytes, cus, s);
+}
+
+}  // namespace moe_gg

@@ -17,23 +17,13 @@
 //     a 16 x 16 super-tile;
 //   * a last round of the persistent grid that would leave most compute units idle is split along K over all
 //     of them (second launch + a reduction kernel that applies the epilogue), given a workspace.
-#include "common.h"
+#include "gg_common.h"
 #include <algorithm>
 #include <type_traits>
 
 namespace moe_gg {
 
-typedef __attribute__((address_space(3))) void* lds_ptr_t;
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-
-constexpr int ROWB = 64;   // bytes of K per tile row per LDS ring stage
-constexpr int CHUNKS = ROWB / 16;
-constexpr int NRING = 4;   // LDS ring stages
-constexpr int WROWS = 64 / CHUNKS;  // tile rows moved by one wave-wide 16-byte-per-lane load
 constexpr int SUP = 16;  // super-tile edge, in tiles
-constexpr int GG_MAXG = MOE_MAX_EXPERTS;
-constexpr int GG_BN = 256;
 #ifndef GG_BIG_NWM
 #define GG_BIG_NWM 2  // waves along M of the 256-row tile (x 2 along N)
 #endif
@@ -46,53 +36,8 @@ constexpr int GG_BN = 256;
 #define GG_FP8_BSA_NWM 4  // the fp8 down projection (block-scaled activations): waves along M, as for the other fp8 GEMM
 #endif
 
-struct GemmParams {
-    const uint8_t* A;         // [S_rows, K] activations (bf16 or fp8)
-    const uint8_t* B;         // packed weights [E_l, Npad, K]
-    void* C;                  // [S_rows, ldc] bf16
-    void* C2;                 // optional (bf16 kernels with an activation): the values BEFORE the activation, bf16, row pitch ldc
-                              // (SwiGLU: 2 ldc, in the packed gate / up column order), kept for the backward pass
-    const int32_t* cnt;       // [E_l] rows per group
-    const float* row_scale;   // fp8: [S_rows] per-row activation scale; bf16 with EPI_GATE: [S_rows] per-row gate
-    const float* col_scale;   // fp8: [E_l, ncs] per-output-channel scale (gate for SwiGLU)
-    const float* col_scale2;  // fp8 SwiGLU: [E_l, ncs] up scales
-    // fp8, block-scaled hidden activation (one power-of-two scale, an E8M0 exponent byte, per row and 32 columns; bs_pitch
-    // bytes per row): written beside the codes by the gate/up kernel's epilogue (c_bscale, rows as C's), read by the down
-    // kernel as the scale operand of its MFMAs (a_bscale, rows as A's).
-    uint8_t* c_bscale;
-    const uint8_t* a_bscale;
-    int bs_pitch;
-    const int32_t* a_map;     // optional: logical row -> row of A (gather while loading), else A is row r itself
-    const int32_t* c_map;     // optional: logical row -> row of C (scatter while storing)
-    int E_l, K, N, Npad, ldc, S_rows, ncs;
-    // Optional split of the last, partly filled round of the persistent grid along K: when that round holds at
-    // most a quarter of a grid of tiles, each of them is cut into P parts of the K range, one per otherwise idle
-    // workgroup, which store their fp32 partial sums here (max_units part tiles of BM x 256 floats); a second
-    // kernel adds the parts of a tile in part order and applies the epilogue.  NULL: no split.
-    float* part_ws;
-    int max_units;
-    // Weight-gradient mode (template flag DW): C[g] (dw_rows x N, at C + g * c_group_stride elements) = A_g^T-like product
-    // whose reduction runs over the rows of group g.  A is then the TRANSPOSED activation matrix [dw_rows, K] with
-    // K = the padded row total (every group's rows padded to a multiple of 64, zero filled), B the output gradients
-    // re-tiled like weights over the same padded rows; group g owns K stages [kstart_g, kstart_g + 2 ceil(cnt_g / 64)).
-    int dw_rows;
-    int dw_src_rows;  // rows of the untransposed operands: the counts are clamped to it, as the operand kernels clamp them
-    size_t c_group_stride;
-    // Time stamps (the TRACE instantiation only; see moe_diag_gemm_trace): GG_TRACE_TILE_WORDS words per workgroup -- for
-    // every tile the wall clock (100 MHz) at the start of its K loop, at the end of its K loop and at the end of its
-    // epilogue -- then GG_TRACE_BLOCK_WORDS words of workgroup 0: the clock at the end of each of its MFMA blocks.
-    // trace_flags & 1: the epilogue computes but stores nothing.
-    unsigned long long* trace;
-    int trace_flags;
-};
-constexpr int GG_TRACE_TILE_WORDS = 256, GG_TRACE_BLOCK_WORDS = 4096;
 
-constexpr int GG_MAX_PARTS = 16;   // parts per tile at most
 constexpr int GG_RED_SLABS = 32;   // blocks per tile in the reduction of the parts
-constexpr int GG_MIN_PART_STAGES = 8;  // K stages per part at least (64 bytes of K each)
-
-// stages per part when nk stages (even) are cut into P parts: even, and P of them cover nk
-__host__ __device__ inline int gg_part_stages(int nk, int P) { return ((nk + P - 1) / P + 1) & ~1; }
 
 // How the tiles of a launch are walked: tiles [0, full) whole, tiles [full, total) in P parts each.
 struct GgPlan {
@@ -113,116 +58,6 @@ __host__ __device__ inline GgPlan gg_plan(int total, int grid, int nk, bool spli
     return pl;
 }
 
-// Where a packed weight column sits inside its aligned group of 32 rows of the packed matrix.  The MFMA leaves a lane
-// with runs of FOUR consecutive rows of the weight operand (bf16 16x16: rows 4q .. 4q+3 of a tile for the lanes 16q ..
-// 16q+15; fp8 32x32: rows 8Q + 4h .. + 3 for the register quad Q and the lanes 32h .. 32h+31).  The rows of a group are
-// ordered so that two of a lane's runs are EIGHT consecutive output columns, which leave as one 16-byte store:
-//   bf16: column 8q + 4t + v of the group (t = 0, 1: the group's two MFMA tiles) at row 16t + 4q + v;
-//   fp8 : column 16P + 8h + 4t + v (P = 0, 1; quads 2P + t) at row 8 (2P + t) + 4h + v.
-// Runs of four columns that start at a multiple of four stay runs of four rows.
-template <bool FP8>
-__host__ __device__ inline int gg_col_to_row32(int c) {  // c in [0, 32)
-    if (FP8) return ((c >> 4) * 2 + ((c >> 2) & 1)) * 8 + ((c >> 3) & 1) * 4 + (c & 3);
-    return ((c >> 2) & 1) * 16 + (c >> 3) * 4 + (c & 3);
-}
-template <bool FP8>
-__host__ __device__ inline int gg_row_to_col32(int r) {  // the inverse
-    if (FP8) return (r >> 4) * 16 + ((r >> 2) & 1) * 8 + ((r >> 3) & 1) * 4 + (r & 3);
-    return ((r >> 2) & 3) * 8 + (r >> 4) * 4 + (r & 3);
-}
-template <bool FP8>
-__host__ __device__ inline int gg_packed_row(int col) { return (col & ~31) | gg_col_to_row32<FP8>(col & 31); }
-template <bool FP8>
-__host__ __device__ inline int gg_packed_col(int row) { return (row & ~31) | gg_row_to_col32<FP8>(row & 31); }
-
-// x * sigmoid(x) with the hardware reciprocal (1 ulp) instead of an IEEE division: the SwiGLU epilogue of a
-// 128 x 128 wave tile evaluates this 8192 times per lane-row, and the division was most of its cost
-// two fp32 -> packed bf16 (round to nearest even) in one hardware conversion
-typedef __bf16 gg_bf16x2 __attribute__((ext_vector_type(2)));
-typedef float gg_f32x2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ uint32_t gg_pack_bf16(float lo, float hi) {
-    const gg_f32x2 v = {lo, hi};
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, gg_bf16x2));
-}
-__device__ __forceinline__ float act_silu_fast(float x) { return x * __builtin_amdgcn_rcpf(1.0f + __expf(-x)); }
-__device__ __forceinline__ float act_silu(float x) { return x / (1.0f + __expf(-x)); }
-__device__ __forceinline__ float act_gelu(float x) { return 0.5f * x * (1.0f + erff(x * 0.70710678118654752440f)); }
-
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-// bf16: one 16x16x32 MFMA; lanes 16q .. 16q+15 hold K elements 8q .. 8q+7 (16 bytes) of rows 0 .. 15 of both operands
-// (Z: the sum starts here -- the MFMA takes a constant zero as its C operand, so no accumulator is cleared beforehand)
-template <bool Z = false>
-__device__ __forceinline__ void mma_bf16_k32(floatx4& acc, const uint4& a, const uint4& b) {
-    if constexpr (Z) {
-        const floatx4 z = {0.f, 0.f, 0.f, 0.f};
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), z, 0, 0, 0);
-    } else {
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), acc, 0, 0, 0);
-    }
-}
-
-// fp8: one 32x32x64 MFMA on 32 bytes of K per lane and operand (two 16-byte LDS chunks); both operands
-// are split over the lanes and registers in the same way, so every k is multiplied exactly once
-typedef int gg_i32x8 __attribute__((ext_vector_type(8)));
-template <bool Z = false>
-__device__ __forceinline__ void mma_fp8_k64(floatx16& acc, const uint4& a_lo, const uint4& a_hi, const uint4& b_lo, const uint4& b_hi) {
-    const gg_i32x8 a = {(int)a_lo.x, (int)a_lo.y, (int)a_lo.z, (int)a_lo.w, (int)a_hi.x, (int)a_hi.y, (int)a_hi.z, (int)a_hi.w};
-    const gg_i32x8 b = {(int)b_lo.x, (int)b_lo.y, (int)b_lo.z, (int)b_lo.w, (int)b_hi.x, (int)b_hi.y, (int)b_hi.z, (int)b_hi.w};
-    // format selectors 0/0 = fp8 (e4m3) for both operands, no block scales
-    if constexpr (Z) {
-        const floatx16 z = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, z, 0, 0, 0, 0, 0, 0);
-    } else {
-        acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, acc, 0, 0, 0, 0, 0, 0);
-    }
-}
-
-// The same MFMA with block scales on the activation operand (the instruction's B: the kernels multiply transposed, weights
-// as A).  For row r of the operand and block b of 32 k (b = 0: the first four registers of the lanes 0-31 and 32-63, i.e. k
-// 0-15 and 16-31 of the step; b = 1: the other four registers), the scale is the E8M0 byte OPSEL of the scale register of
-// lane 32 b + r (established with a one-wave probe on the chip); the weight operand takes 2^0 everywhere.
-constexpr int GG_WSCALE = 64;
-// ASMV: the instruction written out, accumulator in ordinary vector registers (the layout of eight waves per workgroup,
-// where a wave's 256 registers hold accumulators and fragments alike).  Through the builtin, the compiler moves the scaled
-// MFMAs of that layout across the scheduling fences that pin the K loop, bunches them, and spills accumulators and
-// fragments inside the loop; a volatile asm statement stays where it is written.  The compiler does not know that the
-// statement is an MFMA: what it would insert between such an instruction and a dependent one is added by hand where the
-// accumulators are next read (GG_MFMA_SETTLE).
-template <bool Z, int OPSEL, bool ASMV = false>
-__device__ __forceinline__ void mma_fp8_k64_bs(floatx16& acc, const uint4& a_lo, const uint4& a_hi, const uint4& b_lo, const uint4& b_hi,
-                                               int scale_b) {
-    const gg_i32x8 a = {(int)a_lo.x, (int)a_lo.y, (int)a_lo.z, (int)a_lo.w, (int)a_hi.x, (int)a_hi.y, (int)a_hi.z, (int)a_hi.w};
-    const gg_i32x8 b = {(int)b_lo.x, (int)b_lo.y, (int)b_lo.z, (int)b_lo.w, (int)b_hi.x, (int)b_hi.y, (int)b_hi.z, (int)b_hi.w};
-    if constexpr (ASMV) {
-        static_assert(!Z, "the written-out form accumulates");
-        const int wsc = GG_WSCALE;
-        if constexpr (OPSEL == 0)
-            asm volatile("v_mfma_scale_f32_32x32x64_f8f6f4 %0, %1, %2, %0, %3, %4 op_sel_hi:[0,0,0]" : "+v"(acc) : "v"(a), "v"(b), "v"(wsc), "v"(scale_b));
-        else
-            asm volatile("v_mfma_scale_f32_32x32x64_f8f6f4 %0, %1, %2, %0, %3, %4 op_sel_hi:[0,1,0]" : "+v"(acc) : "v"(a), "v"(b), "v"(wsc), "v"(scale_b));
-        return;
-    }
-    // (the weight operand's scale byte is GG_WSCALE = 64, a constant the instruction can take without a register; the
-    // activation side adds the 63 that are missing to 2^0 to its own bytes: the product of the two scales is what counts)
-    if constexpr (Z) {
-        const floatx16 z = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, z, 0, 0, 0, GG_WSCALE, OPSEL, scale_b);
-    } else {
-        acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, acc, 0, 0, 0, GG_WSCALE, OPSEL, scale_b);
-    }
-}
-
-// Block scale of the fp8 hidden activation: the smallest power of two X = 2^(byte - 127) with amax / X <= 448 (the largest
-// e4m3 value), from the bits of amax >= 0: amax = m 2^p, 1 <= m < 2, fits when p - e < 8, or p - e = 8 and m <= 1.75 -- so
-// byte = p + 127 - 8, one more when the mantissa exceeds that of 1.75; never below 0 (amax = 0, or tiny).  Integer work:
-// the CPU checker computes the same byte from the same bits.
-__host__ __device__ inline int gg_block_scale_byte(uint32_t amax_bits) {
-    const int b = (int)((amax_bits + 0x1fffffu) >> 23) - 8;
-    return b < 0 ? 0 : b;
-}
-// 1 / X as a float: 2^(127 - byte), exact (byte <= 247 for finite amax)
-__host__ __device__ inline uint32_t gg_block_inv_bits(int byte) { return (uint32_t)(254 - byte) << 23; }
-
 __device__ __forceinline__ int seg_of(const int* off, int n, int r) {
     int lo = 0, hi = n;
     while (hi - lo > 1) {
@@ -231,11 +66,6 @@ __device__ __forceinline__ int seg_of(const int* off, int n, int r) {
     }
     return lo;
 }
-
-// EPI_GATE: no activation, and every result row is multiplied by its row's gate (GemmParams::row_scale, one fp32
-// multiplication before the rounding to bf16): the down projection of an expert whose rows return already weighted.
-// (The fp8 kernels have a row scale as it is: a gate is folded into it by the caller.)
-enum { EPI_NONE = 0, EPI_GELU = 1, EPI_SILU = 2, EPI_SWIGLU = 3, EPI_GATE = 4 };
 
 // One output tile of the walk: group g, n tile nt, first row row0, rv valid rows (rv <= 0: none).
 struct GgTile {
@@ -354,44 +184,6 @@ __device__ __forceinline__ GgTile gg_walk(int4* s_tiles, const int* g_tile_start
     return t;
 }
 
-
-// ---- pieces of the main loop ---------------------------------------------------------------------
-// HBM -> LDS, 16 bytes per lane, no register staging.  One instruction moves 16 tile rows of one ring
-// stage (64 lanes x 16 B = 16 rows x 64 B); wave w of a round moves rows [w*16, w*16+16) of that round.
-// Written as inline assembly to get the scalar-base + 32-bit-lane-offset form (the builtin expands to a
-// 64-bit per-lane address); M0 holds the LDS byte address of the wave's 1 KB destination.
-__device__ __forceinline__ void gg_dma16(const uint8_t* sbase, uint32_t voff, uint32_t lds_addr) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %0" : : "s"(sbase), "v"(voff), "s"(lds_addr) : "memory");
-}
-
-// The lane id read afresh (two instructions) where it is needed.  What the epilogue and the tile set-up derive from it
-// is then computed there, once per tile, instead of being hoisted out of the tile loop as a dozen lane-constant
-// invariants that occupy -- or spill -- registers across the whole K loop.
-__device__ __forceinline__ int gg_lane_now() {
-    int l;
-    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
-    return l;
-}
-
-// One dword per lane, HBM -> LDS: lane l's value lands at lds_addr + 4 l.
-__device__ __forceinline__ void gg_dma4(const uint8_t* sbase, uint32_t voff, uint32_t lds_addr) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %1, %0" : : "s"(sbase), "v"(voff), "s"(lds_addr) : "memory");
-}
-
-// a wave-uniform value forced into scalar registers
-__device__ __forceinline__ const uint8_t* gg_uniform(const uint8_t* p) {
-    const uint64_t v = (uint64_t)p;
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-    return (const uint8_t*)(((uint64_t)hi << 32) | lo);
-}
-
-// s_waitcnt through the builtin (not inline asm) so that the compiler's own wait-count bookkeeping
-// sees it.  gfx9 encoding: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt[5:4] << 14.
-template <int VM, int LGKM>
-__device__ __forceinline__ void gg_wait() {
-    static_assert(VM >= 0 && VM <= 63 && LGKM >= 0 && LGKM <= 15, "wait counts");
-    __builtin_amdgcn_s_waitcnt((VM & 15) | (7 << 4) | (LGKM << 8) | ((VM >> 4) << 14));
-}
 
 // NWM x 2 wave64s per workgroup; every wave owns a (BM/NWM) x 128 block of the tile.
 //
@@ -1770,6 +1562,11 @@ int launch_gemm(const GemmParams& p_in, int epi, hipStream_t s, void* part_ws = 
         p.trace = g_trace.buf;
         p.trace_flags = g_trace.flags;
         part_ws = nullptr;
+    }
+    // launches that large tiles would leave mostly idle: see gemm_small.hip
+    if (!traced) {
+        const int bm_small = gs_choose_bm(p.S_rows, p.E_l, p.K, epi == EPI_SWIGLU ? 2 * p.N : p.N, FP8, grid);
+        if (bm_small) return launch_gemm_small(p, FP8, bm_small, epi, part_ws, part_ws_bytes, grid, s);
     }
     // 256-row or 128-row tiles: the host knows only the total row count, so it compares the estimated number
     // of rounds of the persistent grid (every group adds about half a tile of ragged tail); a 128-row tile

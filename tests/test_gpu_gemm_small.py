@@ -1,0 +1,96 @@
+"""The small-tile grouped GEMM (csrc/gemm_small.hip) at the edges of its tiles, stages and parts, against fp32 products of the
+same operands.  The sizes are ones the dispatch gives to it: few rows, or few columns, or both."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import O
+from iris_testing_amd import ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _close(got, ref, what):
+    err = (got.float() - ref).abs()
+    bar = 2.0 ** -7 * ref.abs() + 2.0 ** -8 * ref.abs().amax()
+    assert bool(torch.isfinite(got.float()).all()) and bool((err <= bar).all()), f"{what}: {float((err - bar).max())} over the bar"
+
+
+# (rows per group, K, N, activation): one row; a tile's edge on either side; one pair of stages and an odd number of pairs;
+# a partly filled group of 32 columns, a partly filled tile; K ranges long enough to be cut into parts; more groups than lanes
+CASES = [((1,), 64, 8, "none"), ((31, 32, 33), 192, 136, "none"), ((63, 0, 64, 65), 320, 96, "swiglu"), ((5, 130), 64, 264, "gelu"),
+         ((17,), 8192, 256, "none"), ((40, 3), 4096, 512, "swiglu"), ((64,), 7168, 1032, "silu"), (tuple([1, 0, 2] * 30), 128, 128, "none")]
+
+
+@pytest.mark.parametrize("cnt,K,N,act", CASES, ids=[f"{len(c[0])}g_{sum(c[0])}x{c[1]}x{c[2]}_{c[3]}" for c in CASES])
+@pytest.mark.parametrize("workspace", [False, True], ids=["whole", "parts"])
+def test_small_gemm_edges(cnt, K, N, act, workspace):
+    rng = np.random.default_rng(K + N)
+    E_l, S = len(cnt), sum(cnt)
+    base = torch.from_numpy(rng.standard_normal((S + 9, K)).astype(np.float32)).to(DEV).bfloat16()
+    w, wu = (torch.from_numpy((rng.standard_normal((E_l, K, N)) * K ** -0.5).astype(np.float32)).to(DEV).bfloat16() for _ in range(2))
+    packed = ops.prepack_weights(w, wu if act == "swiglu" else None)
+    a_map, c_map = (torch.from_numpy(rng.permutation(S + 9)[:S].astype(np.int32)).to(DEV) for _ in range(2))
+    if S > 4:
+        c_map[3] = -1  # a row without a place in the output
+    cnt_t = torch.tensor(cnt, dtype=torch.int32, device=DEV)
+    ws = ops.gemm_part_workspace(DEV) if workspace else None
+    if workspace:
+        ws.fill_(float("nan"))
+    out = torch.full((S + 9, N), -7.0, dtype=torch.bfloat16, device=DEV)
+    run = lambda: ops.grouped_gemm_mapped(base, a_map, packed, cnt_t, S, N, act, out, c_map, part_ws=ws)  # noqa: E731
+    run()
+    x, ref, r0 = base[a_map.long()].float().cpu(), torch.empty(S, N), 0
+    for e, c in enumerate(cnt):
+        g = x[r0:r0 + c] @ w[e].float().cpu()
+        if act == "swiglu":
+            g = torch.nn.functional.silu(g) * (x[r0:r0 + c] @ wu[e].float().cpu())
+        elif act != "none":
+            g = getattr(torch.nn.functional, act)(g)
+        ref[r0:r0 + c] = g
+        r0 += c
+    kept = (c_map >= 0).cpu()
+    first = out.clone()
+    _close(first.cpu()[c_map.cpu().long()[kept]], ref[kept], f"{cnt} {K} {N} {act}")
+    rest = torch.ones(S + 9, dtype=torch.bool)
+    rest[c_map.cpu().long()[kept]] = False
+    assert bool((first.cpu()[rest] == -7.0).all()), "a row outside the map was written"
+    # the same bits again: called again, and replayed from a graph (the counters of the parts are left as a launch finds them)
+    for _ in range(2):
+        run()
+        assert torch.equal(out.view(torch.int16), first.view(torch.int16))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        run()
+    for _ in range(3):
+        out.fill_(-7.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), first.view(torch.int16))
+
+
+@pytest.mark.parametrize("cnt,H,F", [((1,), 128, 128), ((33, 0, 64), 384, 256), ((65,), 4096, 640), ((20, 7), 2048, 2176)])
+@pytest.mark.parametrize("workspace", [False, True], ids=["whole", "parts"])
+def test_small_fp8_mlp_edges(cnt, H, F, workspace):
+    rng = np.random.default_rng(H + F)
+    E_l, S = len(cnt), sum(cnt)
+    x = torch.from_numpy((rng.standard_normal((S, H)) * rng.uniform(0.3, 3.0, (S, 1))).astype(np.float32)).to(DEV).bfloat16()
+    (gq, gs), (uq, us), (dq, ds) = [tuple(torch.from_numpy(t).to(DEV) for t in O.quantize_cols_fp8((rng.standard_normal(sh) * sc).astype(np.float32)))
+                                    for sh, sc in (((E_l, H, F), H ** -0.5), ((E_l, H, F), H ** -0.5), ((E_l, F, H), F ** -0.5))]
+    ws = ops.fp8_workspace(S, H, F, DEV)
+    part = ops.gemm_part_workspace(DEV) if workspace else None
+    y = ops.grouped_mlp_fp8(x, torch.tensor(cnt, dtype=torch.int32, device=DEV), F, ops.prepack_weights_fp8(gq, uq), gs, us,
+                            ops.prepack_weights_fp8(dq), ds, ws=ws, part_ws=part)
+    dec = lambda t: t.view(torch.float8_e4m3fn).float().cpu()  # noqa: E731
+    xd, hd, r0 = dec(ws["xq"]), ops.dequantize_hidden_fp8(ws["hq"], ws["hsc"]).cpu(), 0
+    for e, c in enumerate(cnt):
+        if c:
+            sx = ws["xs"][r0:r0 + c, None].cpu()
+            h = torch.nn.functional.silu((xd[r0:r0 + c] @ dec(gq[e])) * sx * gs[e].cpu()) * ((xd[r0:r0 + c] @ dec(uq[e])) * sx * us[e].cpu())
+            # a code is at most half a step of its block's grid away (one step where a sum sits on a boundary)
+            blk = h.view(c, -1, 32).abs().amax(-1, keepdim=True)
+            err = (hd[r0:r0 + c] - h).abs().view(c, -1, 32)
+            assert bool((err <= h.abs().view(c, -1, 32) * 2.0 ** -3.9 + blk * 2.0 ** -14 + 1e-6).all()), f"hidden of group {e}"
+            _close(y[r0:r0 + c].cpu(), (hd[r0:r0 + c] @ dec(dq[e])) * ds[e].cpu(), f"down, group {e}")
+        r0 += c
