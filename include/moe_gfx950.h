@@ -316,8 +316,8 @@ int moe_grouped_mlp_fp8_q_mapped(const uint8_t* a_q, const float* a_scale, int a
  *                    (w, w_up) is transposed together in the fused gate/up column order, N = columns of ONE matrix,
  *                    twice the bytes); fp32: moe_transpose_weights_f32 then moe_grouped_gemm.
  *   d w[g]         = x[rows of g]^T @ d out[rows of g] : moe_grouped_gemm_dw, one launch for all groups, the ragged row
- *                    count being the reduction dimension (both operands are first rewritten row-index-fastest, every
- *                    group padded to a multiple of 64 rows with zeros, into ws of moe_dw_workspace_bytes bytes);
+ *                    count being the reduction dimension (both operands are read as they are; ws is not used and
+ *                    moe_dw_workspace_bytes is 0);
  *                    groups without rows get zeros.  split_F > 0 (bf16): dy is [S_rows, 2 split_F] in the fused
  *                    gate/up column order and dw comes out as [E_l, K, 2 split_F] = [d w_gate | d w_up] side by side.
  * moe_mlp_act_backward: gradient through the activation of the expert MLP; a1 = pre-activations ([rows,F]; SwiGLU:
@@ -339,6 +339,24 @@ int moe_prepack_weights_transposed(const void* w, const void* w_up, int dtype, i
 size_t moe_dw_workspace_bytes(int S_rows, int E_l, int K, int N);
 int moe_grouped_gemm_dw(const void* x, const void* dy, const int32_t* expert_cnt, int dtype, int S_rows, int K, int N,
                         int E_l, int split_F, void* dw, void* ws, size_t ws_bytes, moe_stream_t stream);
+/* moe_grouped_gemm_dw with split_F = F whose halves go to two matrices of their own, dw_gate and dw_up [E_l,K,F] (bf16). */
+int moe_grouped_gemm_dw_pair(const void* x, const void* dy, const int32_t* expert_cnt, int S_rows, int K, int F, int E_l,
+                             void* dw_gate, void* dw_up, moe_stream_t stream);
+/* moe_prepack_weights and moe_prepack_weights_transposed in one pass over the weight (K and N multiples of 64, bf16). */
+int moe_prepack_weights_both(const void* w, const void* w_up, int dtype, int E_l, int K, int N, void* packed, void* packed_t,
+                             moe_stream_t stream);
+/* The expert MLP of a training step, one call per direction (bf16; H and F multiples of 64; act GELU, SiLU or SwiGLU; the
+ * reference's backward, layers/expert.py:62-64, is an empty stub).
+ * forward:  hidden [S,F] = act(x w1), pre_act as moe_grouped_gemm_act_keep, out [S,H] = hidden w2; w1 / w2 packed.
+ * backward: dh [S,F] and d_pre (layout of pre_act) are scratch; dx [S,H], dw1 / dw_up [E_l,H,F] (dw_up: SwiGLU only), dw2
+ * [E_l,F,H]; w1_t / w2_t as moe_prepack_weights_transposed makes them.
+ * Rows of out and dx past the counted total are zeroed. */
+int moe_mlp_train_forward(const void* x, const int32_t* expert_cnt, int S_rows, int H, int F, int E_l, int act, const void* w1,
+                          const void* w2, void* hidden, void* pre_act, void* out, void* part_ws, size_t part_ws_bytes,
+                          moe_stream_t stream);
+int moe_mlp_train_backward(const void* x, const void* hidden, const void* pre_act, const void* dy, const int32_t* expert_cnt,
+                           int S_rows, int H, int F, int E_l, int act, const void* w1_t, const void* w2_t, void* dh, void* d_pre,
+                           void* dx, void* dw1, void* dw_up, void* dw2, void* part_ws, size_t part_ws_bytes, moe_stream_t stream);
 int moe_transpose_weights_f32(const float* w, int E_l, int K, int N, float* out, moe_stream_t stream);
 int moe_mlp_act_backward(const void* a1, const void* dh, int dtype, int rows, int F, int act, void* d_a1,
                          moe_stream_t stream);

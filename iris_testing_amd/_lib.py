@@ -73,6 +73,10 @@ _SIGNATURES = {
     "moe_prepack_weights_transposed": (c_int, [P, P, c_int, c_int, c_int, c_int, P, P]),
     "moe_dw_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int]),
     "moe_grouped_gemm_dw": (c_int, [P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, P, P, c_size_t, P]),
+    "moe_grouped_gemm_dw_pair": (c_int, [P, P, P, c_int, c_int, c_int, c_int, P, P, P]),
+    "moe_prepack_weights_both": (c_int, [P, P, c_int, c_int, c_int, c_int, P, P, P]),
+    "moe_mlp_train_forward": (c_int, [P, P, c_int, c_int, c_int, c_int, c_int, P, P, P, P, P, P, c_size_t, P]),
+    "moe_mlp_train_backward": (c_int, [P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, P, P, P, P, P, P, P, P, P, c_size_t, P]),
     "moe_transpose_weights_f32": (c_int, [P, c_int, c_int, c_int, P, P]),
     "moe_mlp_act_backward": (c_int, [P, P, c_int, c_int, c_int, c_int, P, P]),
     "moe_combine_backward": (c_int, [P, P, c_int, c_int, c_int, c_int, P, P, P, P, P, c_int, c_int, c_int, P, P, P]),

@@ -97,6 +97,7 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
             mt_all += ts;
             rows = min(rows + __shfl(inc, WAVE - 1, WAVE), p.S_rows);
         }
+        if constexpr (!FP8) gg_zero_tail(p, rows);
     }
     const int nk = (p.K * ES) / ROWB;
     const int P = __builtin_amdgcn_readfirstlane(p.part_ws ? gs_parts((long long)mt_all * nt_all, q.slots, nk, p.max_units) : 1);

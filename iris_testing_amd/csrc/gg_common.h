@@ -35,18 +35,22 @@ struct GemmParams {
     const int32_t* a_map;     // optional: logical row -> row of A (gather while loading), else A is row r itself
     const int32_t* c_map;     // optional: logical row -> row of C (scatter while storing)
     int E_l, K, N, Npad, ldc, S_rows, ncs;
+    int zero_tail;            // rows [counted total, S_rows) of C are zeroed (no c_map then)
     // Optional split of the last, partly filled round of the persistent grid along K: when that round holds at
     // most a quarter of a grid of tiles, each of them is cut into P parts of the K range, one per otherwise idle
     // workgroup, which store their fp32 partial sums here (max_units part tiles of BM x 256 floats); a second
     // kernel adds the parts of a tile in part order and applies the epilogue.  NULL: no split.
     float* part_ws;
     int max_units;
-    // Weight-gradient mode (template flag DW): C[g] (dw_rows x N, at C + g * c_group_stride elements) = A_g^T-like product
-    // whose reduction runs over the rows of group g.  A is then the TRANSPOSED activation matrix [dw_rows, K] with
-    // K = the padded row total (every group's rows padded to a multiple of 64, zero filled), B the output gradients
-    // re-tiled like weights over the same padded rows; group g owns K stages [kstart_g, kstart_g + 2 ceil(cnt_g / 64)).
+    // Weight-gradient mode (template flag DW): C[g] (dw_rows x N, at C + g * c_group_stride elements) = x_g^T dy_g, the reduction
+    // running over the rows of group g.  A is x [rows, dw_rows] and B is dy [rows, N], both as they are: the reduction index is
+    // the slow one, a K stage is 32 rows of each, and the fragments are transposed on their way out of LDS.  With dw_split (F)
+    // dy's columns are in the fused gate / up order (32 gate, 32 up, ...): gate column n of a row goes to column n, up column n
+    // to the element dw_delta further.
     int dw_rows;
-    int dw_src_rows;  // rows of the untransposed operands: the counts are clamped to it, as the operand kernels clamp them
+    int dw_src_rows;  // rows of the operands: the counts are clamped to it
+    int dw_split;
+    long long dw_delta;
     size_t c_group_stride;
     // Time stamps (the TRACE instantiation only; see moe_diag_gemm_trace): GG_TRACE_TILE_WORDS words per workgroup -- for
     // every tile the wall clock (100 MHz) at the start of its K loop, at the end of its K loop and at the end of its
@@ -181,6 +185,30 @@ __device__ __forceinline__ void gg_dma16(const uint8_t* sbase, uint32_t voff, ui
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %0" : : "s"(sbase), "v"(voff), "s"(lds_addr) : "memory");
 }
 
+// The same through a buffer descriptor: bytes at or past its range arrive as zeros.
+typedef int gg_i32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void gg_dma16(const gg_i32x4& srd, uint32_t voff, uint32_t lds_addr) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %0, 0 offen lds" : : "s"(srd), "v"(voff), "s"(lds_addr) : "memory");
+}
+// Descriptor of `left` bytes at p (none when left <= 0), in scalar registers.
+__device__ __forceinline__ gg_i32x4 gg_range(const uint8_t* p, long long left) {
+    const uint64_t v = (uint64_t)p;
+    const long long n = left < 0 ? 0 : left > 0xfffffff0ll ? 0xfffffff0ll : left;
+    const gg_i32x4 d = {__builtin_amdgcn_readfirstlane((int)(uint32_t)v), __builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32)) & 0xffff,
+                        __builtin_amdgcn_readfirstlane((int)(uint32_t)n), 0x00020000};
+    return d;
+}
+
+// Half h of a fragment of a 16 x 16 x 32 MFMA out of an LDS tile whose rows run along k (row pitch 512 bytes): lanes 16 q ..
+// 16 q + 15 end with k 8 q + 4 h .. + 3 of columns 0 .. 15.  `addr`: the lane's LDS byte address of k = 8 q + (lane % 16) / 4, four
+// columns from column 4 (lane % 4) on; the instruction transposes within the 16 lanes.
+typedef short gg_i16x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ uint2 gg_read_tr(uint32_t addr, int h) {
+    typedef __attribute__((address_space(3))) char* lds_char;
+    typedef __attribute__((address_space(3))) gg_i16x4* lds_v4;
+    return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4)((lds_char)(uintptr_t)addr + h * 4 * 512)));
+}
+
 // The lane id read afresh (two instructions) where it is needed.  What the epilogue and the tile set-up derive from it
 // is then computed there, once per tile, instead of being hoisted out of the tile loop as a dozen lane-constant
 // invariants that occupy -- or spill -- registers across the whole K loop.
@@ -214,6 +242,15 @@ constexpr int GG_MAX_PARTS = 16;       // parts a tile's K range is cut into, at
 constexpr int GG_MIN_PART_STAGES = 8;  // K stages per part at least (64 bytes of K each)
 // stages per part when nk stages (even) are cut into P parts: even, and P of them cover nk
 __host__ __device__ inline int gg_part_stages(int nk, int P) { return ((nk + P - 1) / P + 1) & ~1; }
+
+// GemmParams::zero_tail, by all workgroups of a launch
+__device__ __forceinline__ void gg_zero_tail(const GemmParams& p, int total) {
+    if (!p.zero_tail || total >= p.S_rows) return;
+    const int nv = p.N / 8;
+    const size_t n = (size_t)(p.S_rows - total) * nv;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
+        *(uint4*)((bf16_t*)p.C + (size_t)(total + i / nv) * p.ldc + (i % nv) * 8) = make_uint4(0, 0, 0, 0);
+}
 
 // gemm_small.hip: the tile height (32, 64 or 128 rows) of the small-tile kernel for a launch, 0 where the large tiles are the
 // better choice; and that launch.

@@ -76,7 +76,7 @@ struct GgTile {
 
 // lin -> tile: group-major, 16-row bands, 16-column super-columns (see the XCD-aware walk above)
 // DW (weight-gradient mode): every non-empty group has the same ceil(dw_rows / BM) x Nt tiles, rows [0, dw_rows) of its own
-// output matrix; g_row_start then holds the groups' first K stages (set by the caller from it).
+// output matrix; its K stages are its rows, 32 at a time (an even number of stages: the last ones may be partly or wholly past them).
 template <int BM, bool DW = false>
 __device__ __forceinline__ GgTile gg_decode(const int* g_tile_start, const int* g_row_start, int E_l, int Nt, int S_rows, int lin,
                                             int dw_rows = 0) {
@@ -130,8 +130,8 @@ __device__ __forceinline__ GgTile gg_peek(const int4* s_tiles, const int* g_row_
         t.g = __builtin_amdgcn_readfirstlane(e.x); t.nt = __builtin_amdgcn_readfirstlane(e.y);
         t.row0 = __builtin_amdgcn_readfirstlane(e.z); t.rv = max(__builtin_amdgcn_readfirstlane(e.w), 0);
         if constexpr (DW) {
-            t.ks0 = g_row_start[t.g];
-            t.nks = g_row_start[t.g + 1] - t.ks0;
+            t.ks0 = g_row_start[t.g];  // (the group's first row)
+            t.nks = (g_row_start[t.g + 1] - t.ks0 + 63) / 64 * 2;
         }
         if constexpr (SPLIT) {
             const int lin = round * stride + my;
@@ -171,7 +171,7 @@ __device__ __forceinline__ GgTile gg_walk(int4* s_tiles, const int* g_tile_start
             t.row0 = __builtin_amdgcn_readfirstlane(e.z); t.rv = rv;
             if constexpr (DW) {
                 t.ks0 = g_row_start[t.g];
-                t.nks = g_row_start[t.g + 1] - t.ks0;
+                t.nks = (g_row_start[t.g + 1] - t.ks0 + 63) / 64 * 2;
             }
             if constexpr (SPLIT) {
                 t.ks0 = (lin % pl.P) * pl.nkp;
@@ -184,6 +184,13 @@ __device__ __forceinline__ GgTile gg_walk(int4* s_tiles, const int* g_tile_start
     return t;
 }
 
+
+// Where the loads of a stage read: a scalar pointer, or (RANGE) a descriptor that ends where the group does.
+template <bool RANGE>
+__device__ __forceinline__ auto gg_stage_src(const uint8_t* base, size_t off, long long left) {
+    if constexpr (RANGE) return gg_range(base + off, left - (long long)off);
+    else return gg_uniform(base + off);
+}
 
 // NWM x 2 wave64s per workgroup; every wave owns a (BM/NWM) x 128 block of the tile.
 //
@@ -221,7 +228,8 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
     constexpr int CF = FP8 ? 2 : 1;                    // 16-byte LDS chunks per fragment and lane
     constexpr int TM = BM / (NWM * MT), TN = BN / (2 * MT);  // MFMA tiles per wave
     constexpr int NT = TM * TN;                        // MFMAs per K stage and wave
-    constexpr int NRD = (TM + TN) * CF;                // fragment reads per K stage and wave
+    constexpr int RPF = DW ? 2 : CF;                   // LDS reads per fragment (DW: two transposing reads of 8 bytes)
+    constexpr int NRD = (TM + TN) * RPF;               // fragment reads per K stage and wave
     constexpr int LR = NW * WROWS;                     // rows fetched per load round (16 per wave)
     constexpr int RA = BM / LR, RB = BN / LR;          // load rounds per stage
     constexpr int LPS = RA + RB;                       // HBM->LDS loads per lane per stage
@@ -263,17 +271,15 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
 
     if (tid == 0) {
         int ts = 0, rs = 0;
-        [[maybe_unused]] int dw_seen = 0;
         for (int g = 0; g < p.E_l; ++g) {
             g_tile_start[g] = ts;
             g_row_start[g] = rs;
             int c = max(p.cnt[g], 0);
             if constexpr (DW) {
-                // tiles of the group's own dw_rows x N output; its K stages: the rows padded to 64 (two stages of 32)
-                c = min(c, max(p.dw_src_rows - dw_seen, 0));
-                dw_seen += c;
+                // tiles of the group's own dw_rows x N output
+                c = min(c, max(p.dw_src_rows - rs, 0));
                 ts += c > 0 ? ((p.dw_rows + BM - 1) / BM) * Nt : 0;
-                rs += ((c + 63) / 64) * 2;
+                rs += c;
             } else {
                 // (counts that claim more rows than the buffers hold are cut at S_rows: the host's bound on the number of
                 // tiles, which decides whether the whole-tile launch is left out, counts on it)
@@ -286,6 +292,20 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
         g_row_start[p.E_l] = rs;
     }
     __syncthreads();
+    if constexpr (DW) {
+        // the gradient of a group without rows is zero (it has no tile below)
+        for (int g = 0; g < p.E_l; ++g) {
+            if (g_row_start[g + 1] > g_row_start[g]) continue;
+            const int nv = (p.dw_split ? p.dw_split : p.N) / 8;  // 16-byte vectors per output row (and half, where split)
+            bf16_t* c = (bf16_t*)p.C + (size_t)g * p.c_group_stride;
+            for (int i = blockIdx.x * NW * WAVE + threadIdx.x; i < p.dw_rows * nv; i += gridDim.x * NW * WAVE) {
+                bf16_t* o = c + (size_t)(i / nv) * p.ldc + (i % nv) * 8;
+                *(uint4*)o = make_uint4(0, 0, 0, 0);
+                if (p.dw_split) *(uint4*)(o + p.dw_delta) = make_uint4(0, 0, 0, 0);
+            }
+        }
+    }
+    if constexpr (!DW && !FP8) gg_zero_tail(p, g_row_start[p.E_l]);
     const int nk = (p.K * ES) / ROWB;  // ring stages per tile; even (K * ES is a multiple of 2 * ROWB)
     const GgPlan plan = gg_plan(g_tile_start[p.E_l], (int)gridDim.x, nk, !DW && p.part_ws != nullptr, p.max_units);
     if (SPLIT && plan.P == 1) return;  // nothing was left over for this launch
@@ -314,26 +334,54 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
     const uint32_t la0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr_t)(sA + wave * WROWS * CHUNKS));
     const uint32_t lb0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr_t)(sB + wave * WROWS * CHUNKS));
 
-    const uint32_t ldk = (uint32_t)(p.K * ES);
+    const uint32_t ldk = DW ? (uint32_t)p.dw_rows * 2u : (uint32_t)(p.K * ES);  // row pitch of A in bytes
+    [[maybe_unused]] const uint32_t ldb = (uint32_t)p.N * 2u;                     // (DW) of B
     const size_t b_slab = (size_t)p.Npad * ROWB;  // packed weights are slab-major: [group][K slab][Npad rows][ROWB bytes]
     // per-round lane offsets into the weight slab (vector registers: no scalar address arithmetic per load)
     uint32_t b_off[RB];
 #pragma unroll
-    for (int r = 0; r < RB; ++r) b_off[r] = (uint32_t)(r * LR + lrow) * ROWB + lchunk * 16;
+    for (int r = 0; r < RB; ++r) {
+        if constexpr (DW) b_off[r] = (uint32_t)(2 * (r * NW + wave) + (lane >> 5)) * ldb + (uint32_t)((lane & 31) ^ (4 * ((2 * wave + (lane >> 5)) & 3))) * 16u;
+        else b_off[r] = (uint32_t)(r * LR + lrow) * ROWB + lchunk * 16;
+    }
+    // DW: an LDS stage holds 32 rows of 512 bytes per operand (a 1 KB load brings two of them); 16-byte chunk c of row k lies at
+    // position c ^ f(k), which spreads the eight rows that half a wave reads together over the banks: f = 2 (k % 4 + 4 (k / 8 % 2))
+    // for A, read 32 contiguous bytes a row, f = 4 (k % 4) for B, read 8 bytes of four chunks in a row (the permuted columns).
+    [[maybe_unused]] uint32_t tr_a = 0, tr_b = 0;
+    if constexpr (DW) {
+        const int kq = (lane >> 4) * 8 + ((lane & 15) >> 2), k4 = (lane & 15) >> 2, q4 = lane & 3;  // first k, its low bits, column quad
+        tr_a = (uint32_t)(uintptr_t)(lds_ptr_t)sA + kq * 512 + (((wm * 16 + (q4 >> 1)) ^ (2 * (k4 + 4 * ((lane >> 4) & 1)))) * 16) + (q4 & 1) * 8;
+        tr_b = (uint32_t)(uintptr_t)(lds_ptr_t)sB + kq * 512 + (((wn * 16 + q4) ^ (4 * k4)) * 16);
+    }
+    // LDS address of fragment i of A (16 rows of the product) / j of B (its columns 32 (j / 2) + 8 q + 4 (j % 2) ..) in ring slot sl
+#define GG_TR_A(i, sl) ((tr_a ^ ((i) * 32)) + (sl) * (ASLOT * 16))
+#define GG_TR_B(j, sl) ((tr_b ^ (((j) >> 1) * 64)) + (sl) * (BSLOT * 16) + ((j) & 1) * 8)
 
 #define GG_MAPROW_GLOBAL(t, l) p.a_map[(t).row0 + (l)]   /* the first tile: straight from memory */
 #define GG_MAPROW_LDS(t, l) s_amap[(l)]                  /* later tiles: fetched into LDS one tile ahead */
 #define GG_TILE_PTRS(t, Ab_, Bb_, aoff_, MAPROW_)                                                          \
-    const uint8_t* Ab_ = (p.a_map ? p.A : p.A + (size_t)(t).row0 * p.K * ES) + (size_t)(t).ks0 * ROWB;      \
-    const uint8_t* Bb_ = p.B + (DW ? (size_t)0 : (size_t)(t).g * p.Npad * p.K * ES) + (size_t)(t).nt * BN * ROWB + (size_t)(t).ks0 * b_slab; \
+    const uint8_t* Ab_ = DW ? p.A + (size_t)(t).ks0 * ldk + (size_t)(t).row0 * 2                             \
+                            : (p.a_map ? p.A : p.A + (size_t)(t).row0 * p.K * ES) + (size_t)(t).ks0 * ROWB;  \
+    const uint8_t* Bb_ = DW ? p.B + (size_t)(t).ks0 * ldb + (size_t)(t).nt * BN * 2                           \
+                            : p.B + (size_t)(t).g * p.Npad * p.K * ES + (size_t)(t).nt * BN * ROWB + (size_t)(t).ks0 * b_slab; \
     uint32_t aoff_[RA];                                                                                     \
     const int ln_ = gg_lane_now();  /* lrow and lchunk again, derived per tile */                              \
-    const int lrow_ = wave_s * WROWS + (ln_ >> 2);                                                            \
-    const uint32_t lcb_ = (uint32_t)(((ln_ & 3) ^ ((ln_ >> 4) & 3)) * 16);                                     \
-    _Pragma("unroll") for (int r = 0; r < RA; ++r) {                                                         \
-        const int lr_ = max(min(r * LR + lrow_, (t).rv - 1), 0);  /* tile row this lane fetches, clamped */    \
-        aoff_[r] = (uint32_t)(p.a_map ? max(MAPROW_(t, lr_), 0) : lr_) * ldk + lcb_;                       \
+    if constexpr (DW) {                                                                                      \
+        const long long rows_ = g_row_start[(t).g + 1] - (t).ks0;                                            \
+        dw_left_a = rows_ * ldk - (long long)(t).row0 * 2;                                                    \
+        dw_left_b = rows_ * ldb - (long long)(t).nt * BN * 2;                                                 \
+        _Pragma("unroll") for (int r = 0; r < RA; ++r)                                                        \
+            aoff_[r] = (uint32_t)(2 * (r * NW + wave_s) + (ln_ >> 5)) * ldk +                                   \
+                       (uint32_t)((ln_ & 31) ^ (2 * (((2 * wave_s + (ln_ >> 5)) & 3) + 4 * (r & 1)))) * 16u;      \
+    } else {                                                                                                 \
+        const int lrow_ = wave_s * WROWS + (ln_ >> 2);                                                         \
+        const uint32_t lcb_ = (uint32_t)(((ln_ & 3) ^ ((ln_ >> 4) & 3)) * 16);                                  \
+        _Pragma("unroll") for (int r = 0; r < RA; ++r) {                                                      \
+            const int lr_ = max(min(r * LR + lrow_, (t).rv - 1), 0);  /* tile row this lane fetches, clamped */ \
+            aoff_[r] = (uint32_t)(p.a_map ? max(MAPROW_(t, lr_), 0) : lr_) * ldk + lcb_;                      \
+        }                                                                                                     \
     }
+    [[maybe_unused]] long long dw_left_a = 0, dw_left_b = 0;  // (DW) bytes of the operands from the tile's corner to the end of the group
     // load d (0 .. LPS-1) of one stage: A rounds first, then B rounds
 #define GG_LD(d, ap_, bp_, aoff_, slot)                                                                       \
     do {                                                                                                      \
@@ -344,8 +392,8 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
     // of another tile, and a repeated load of the last stage lands in a slot nobody reads again)
 #define GG_STAGE_PTRS(Ab_, Bb_, st, ap_, bp_, nks_)                                            \
     const int st_ = min((st), (nks_) - 1);                                                     \
-    const uint8_t* ap_ = gg_uniform(Ab_ + (size_t)st_ * ROWB);                                 \
-    const uint8_t* bp_ = gg_uniform(Bb_ + (size_t)st_ * b_slab);
+    const auto ap_ = gg_stage_src<DW>(Ab_, (size_t)st_ * (DW ? (size_t)32 * ldk : (size_t)ROWB), dw_left_a);  \
+    const auto bp_ = gg_stage_src<DW>(Bb_, (size_t)st_ * (DW ? (size_t)32 * ldb : b_slab), dw_left_b);
 #define GG_ISSUE_RANGE(Ab_, Bb_, aoff_, st, slot, first, count, nks_)                          \
     do {                                                                                       \
         GG_STAGE_PTRS(Ab_, Bb_, st, ap_i, bp_i, nks_)                                          \
@@ -455,8 +503,13 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
         // fragment read R of the next stage: operand R / CF (activation rows first, then weight rows), chunk R % CF
 #define GG_RD(R, NA_, NB_)                                                                               \
     do {                                                                                                 \
-        constexpr int ro_ = (R) / CF, rh_ = (R) % CF;                                                    \
-        if constexpr (ro_ < TM) NA_[ro_ * CF + rh_] = nfa_[ro_ * MT * CHUNKS + (fpos ^ (rh_ * FSTEP))];  \
+        constexpr int ro_ = (R) / RPF, rh_ = (R) % RPF;                                                  \
+        if constexpr (DW) {                                                                              \
+            const uint2 v_ = gg_read_tr(ro_ < TM ? GG_TR_A(ro_, nsl_) : GG_TR_B((ro_ < TM ? 0 : ro_ - TM), nsl_), rh_); \
+            uint4& f_ = ro_ < TM ? NA_[ro_ < TM ? ro_ : 0] : NB_[ro_ < TM ? 0 : ro_ - TM];               \
+            if constexpr (rh_ == 0) { f_.x = v_.x; f_.y = v_.y; } else { f_.z = v_.x; f_.w = v_.y; }      \
+        }                                                                                                \
+        else if constexpr (ro_ < TM) NA_[ro_ * CF + rh_] = nfa_[ro_ * MT * CHUNKS + (fpos ^ (rh_ * FSTEP))];  \
         else NB_[(ro_ - TM) * CF + rh_] = nfb_[(ro_ - TM) * MT * CHUNKS + (fpos ^ (rh_ * FSTEP))];       \
     } while (0)
 #define GG_ML(I, FA_, FB_, NA_, NB_, slot, Z_, EVEN_, SET_)                                                \
@@ -504,6 +557,7 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
             GG_SC_DMA((s) + 4 - kbase, nks_ld, SET_ * 2);                                                \
         }                                                                                                \
         GG_STAGE_PTRS(Ab, Bb, (s) + 4 - kbase, ap_, bp_, nks_ld)                                         \
+        [[maybe_unused]] const int nsl_ = ((SL) + 1) & 3;                                                \
         const uint4* nfa_ = fa + (((SL) + 1) & 3) * ASLOT;                                               \
         const uint4* nfb_ = fb + (((SL) + 1) & 3) * BSLOT;                                               \
         /* (written-out MFMAs: two wait states between the vector instructions above and an MFMA that reads their results) */ \
@@ -574,6 +628,18 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
             if (!pre) {
                 const uint4* fa0 = fa + phi * ASLOT;
                 const uint4* fb0 = fb + phi * BSLOT;
+                if constexpr (DW) {
+#pragma unroll
+                    for (int i = 0; i < TM; ++i) {
+                        const uint2 lo = gg_read_tr(GG_TR_A(i, phi), 0), hi = gg_read_tr(GG_TR_A(i, phi), 1);
+                        fA0[i] = make_uint4(lo.x, lo.y, hi.x, hi.y);
+                    }
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) {
+                        const uint2 lo = gg_read_tr(GG_TR_B(j, phi), 0), hi = gg_read_tr(GG_TR_B(j, phi), 1);
+                        fB0[j] = make_uint4(lo.x, lo.y, hi.x, hi.y);
+                    }
+                } else {
 #pragma unroll
                 for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -582,6 +648,7 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
                 for (int j = 0; j < TN; ++j)
 #pragma unroll
                     for (int h = 0; h < CF; ++h) fB0[j * CF + h] = fb0[j * MT * CHUNKS + (fpos ^ (h * FSTEP))];
+                }
                 GG_SC_READ(0);  // (a tile that starts here starts in slot 0)
                 // the first slot is refilled from the first block on: every wave must hold its stage-0 fragments first
                 gg_wait<63, 0>();
@@ -736,7 +803,9 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
                 if (jg % 2 == 1) continue;  // an up group: consumed together with its gate group
             }
             const int pcol = nt * BN + cbase_e + jg * 32;  // first packed column of the group
-            const int colg = EPI == EPI_SWIGLU ? (pcol / 64) * 32 : pcol;  // its first output column
+            const bool pair = EPI == EPI_SWIGLU || (DW && p.dw_split);
+            const int colg = pair ? (pcol / 64) * 32 : pcol;  // its first output column
+            [[maybe_unused]] const long long cshift = DW && p.dw_split && (pcol & 32) ? p.dw_delta : 0;
             [[maybe_unused]] uint4 pk[2];  // fp8: the lane's two 16-byte units of the group, stored after they changed lanes
             [[maybe_unused]] float xq[2][8];  // quantised output: the lane's sixteen values of the group's block of 32 columns
 #pragma unroll
@@ -791,8 +860,8 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
                 o4.w = gg_pack_bf16(x[6], x[7]);
                 if constexpr (FP8) {
                     pk[u] = o4;
-                } else if (ok[i][0] && col < p.N) {
-                    *(uint4*)(crow[i][0] + col) = o4;
+                } else if (ok[i][0] && col + (pair && DW ? pcol - colg : 0) < p.N) {
+                    *(uint4*)(crow[i][0] + col + (DW ? cshift : 0)) = o4;
                     if constexpr (EPI != EPI_NONE && EPI != EPI_GATE) {
                         if (p.C2) {
                             // same row, in a matrix whose rows are as long (SwiGLU: twice as long, packed column order)
@@ -895,6 +964,8 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
 #undef GG_PROLOGUE
 #undef GG_SC_DMA
 #undef GG_SC_READ
+#undef GG_TR_A
+#undef GG_TR_B
 }
 
 // ---- second half of a K-split tile: add its parts in part order, then the epilogue of the GEMM kernel ------------
@@ -1049,6 +1120,53 @@ __global__ __launch_bounds__(256) void prepack_kernel(const T* __restrict__ w, c
             }
         }
         __syncthreads();
+    }
+}
+
+// The same for 16-bit weights with K a multiple of 64 and N of 8 (what the GEMMs take): 64 k x 128 n through LDS, 16 bytes per load
+// and store; and, where out_t is given, the re-tiling of the transposed product (prepack_t below) from the same tile, so that
+// a weight which both directions need is read once.  Columns [N, Npad) of the one and rows [K, Kpad) of the other leave as zeros.
+__global__ __launch_bounds__(256) void prepack16_kernel(const uint16_t* __restrict__ w, const uint16_t* __restrict__ w_up,
+                                                         uint16_t* __restrict__ out, uint16_t* __restrict__ out_t, int K, int N, int Npad,
+                                                         int Kpad) {
+    constexpr int TN = 128, LD = TN + 8;
+    __shared__ __align__(16) uint16_t tile[64][LD];
+    const int passes = w_up ? 2 : 1, e = blockIdx.z / passes, pass = blockIdx.z % passes;
+    const int k0 = blockIdx.y * 64, n0 = blockIdx.x * TN;
+    const uint16_t* s = (pass ? w_up : w) + (size_t)e * K * N;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int v = threadIdx.x + i * 256, kk = v / 16, nn = (v % 16) * 8;
+        uint4 x = make_uint4(0, 0, 0, 0);
+        if (k0 < K && n0 + nn < N) x = *(const uint4*)(s + (size_t)(k0 + kk) * N + n0 + nn);
+        *(uint4*)&tile[kk][nn] = x;
+    }
+    __syncthreads();
+    constexpr int SK = 32;
+    if (out && k0 < K) {
+        uint16_t* dst = out + (size_t)e * Npad * K;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int v = threadIdx.x + i * 256, k8 = (v % 4) * 8, row = v / 4;  // row: (slab of the tile, row of the packed columns)
+            const int slab = row / TN, rr = row % TN;
+            const int nn = gg_packed_col<false>(rr);  // (consecutive threads write consecutive packed rows)
+            const int pr = w_up ? ((n0 + rr) >> 5) * 64 + pass * 32 + (rr & 31) : n0 + rr;
+            if (pr >= Npad) continue;
+            uint32_t o[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) o[q] = (uint32_t)tile[slab * SK + k8 + 2 * q][nn] | ((uint32_t)tile[slab * SK + k8 + 2 * q + 1][nn] << 16);
+            *(uint4*)(dst + ((size_t)(k0 / SK + slab) * Npad + pr) * SK + k8) = make_uint4(o[0], o[1], o[2], o[3]);
+        }
+    }
+    if (out_t) {
+        uint16_t* dst = out_t + (size_t)e * Kpad * N * passes;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int v = threadIdx.x + i * 256, q = v % 4, kr = (v / 4) % 64, slab = v / 256;
+            if (n0 + slab * SK >= N) continue;
+            const int kc = gg_packed_col<false>(kr);
+            *(uint4*)(dst + ((size_t)((n0 / SK + slab) * passes + pass) * Kpad + k0 + kr) * SK + q * 8) = *(const uint4*)&tile[kc][slab * SK + q * 8];
+        }
     }
 }
 
@@ -1366,76 +1484,6 @@ __global__ __launch_bounds__(256) void prepack_t_kernel(const T* __restrict__ w,
     }
 }
 
-// Operands of the weight-gradient product d w[g] = x_g^T @ dy_g, whose reduction runs over the rows of group g: both
-// matrices are needed with the row index fastest.  Rows are renumbered s -> s' so that every group starts at a
-// multiple of 64 (two K stages of the GEMM) and its tail up to the next multiple of 64 is zero.  A block moves 64 rows
-// (one group's, never two) x 64 columns through LDS.
-//   SLAB = false: out = x^T, [cols, ld_out] row-major                       (the GEMM's activation operand)
-//   SLAB = true : out = the weight layout over the padded rows, [ld_out / SK][Npad][SK]  (the GEMM's weight operand)
-//                with split_F > 0 the input columns are in the fused gate/up order (32 gate, 32 up, ...) and leave in
-//                the order [all gate | all up], so that the product's columns are the two weight gradients side by side
-template <bool SLAB>
-__global__ __launch_bounds__(256) void dw_operand_kernel(const uint16_t* __restrict__ in, const int32_t* __restrict__ cnt, int E_l,
-                                                          int S_rows, int cols, uint16_t* __restrict__ out, int ld_out, int Npad,
-                                                          int split_F) {
-    __shared__ uint16_t tile[64][64 + 2];
-    __shared__ int s_src0, s_valid;
-    if (threadIdx.x == 0) {
-        // padded block blockIdx.y -> (first source row, valid rows); blocks past the padded total have nothing to do
-        int pb = 0, rs = 0, src0 = -1, valid = 0;
-        for (int g = 0; g < E_l; ++g) {
-            const int c = min(max(cnt[g], 0), max(S_rows - rs, 0));
-            const int nb = (c + 63) / 64;
-            if ((int)blockIdx.y < pb + nb) {
-                const int j = blockIdx.y - pb;
-                src0 = rs + j * 64;
-                valid = min(64, c - j * 64);
-                break;
-            }
-            pb += nb;
-            rs += c;
-        }
-        s_src0 = src0;
-        s_valid = valid;
-    }
-    __syncthreads();
-    const int src0 = s_src0, valid = s_valid;
-    if (src0 < 0) return;
-    const int c0 = blockIdx.x * 64;
-    for (int i = threadIdx.x; i < 64 * 64; i += 256) {
-        const int r = i / 64, c = i % 64;
-        tile[r][c] = (r < valid && c0 + c < cols) ? in[(size_t)(src0 + r) * cols + c0 + c] : (uint16_t)0;
-    }
-    __syncthreads();
-    const int sp0 = blockIdx.y * 64;  // first padded row of the block
-    constexpr int SK = ROWB / 2;
-    for (int i = threadIdx.x; i < 64 * 64; i += 256) {
-        const int c = i / 64, r = i % 64;  // consecutive threads walk the rows: contiguous in both output layouts
-        if (c0 + c >= (SLAB ? Npad : cols)) continue;
-        const uint16_t v = tile[r][c];  // (columns in [cols, Npad) were loaded as zeros)
-        const int sp = sp0 + r;
-        if constexpr (SLAB) {
-            int oc = c0 + c;
-            if (split_F > 0 && oc < 2 * split_F) oc = ((oc % 64) / 32) * split_F + (oc / 64) * 32 + oc % 32;
-            out[((size_t)(sp / SK) * Npad + gg_packed_row<false>(oc)) * SK + sp % SK] = v;
-        } else {
-            out[(size_t)(c0 + c) * ld_out + sp] = v;
-        }
-    }
-}
-
-// d w[g] <- 0 for the groups that received no row (the GEMM has no tile for them)
-__global__ __launch_bounds__(256) void dw_zero_empty_kernel(uint4* __restrict__ dw, const int32_t* __restrict__ cnt,
-                                                             size_t vec_per_group, int src_rows) {
-    // (a group whose rows all lie past the end of the operands counts as empty, as in the GEMM's own tables)
-    int before = 0;
-    for (int e = 0; e < (int)blockIdx.y; ++e) before += max(cnt[e], 0);
-    if (min(max(cnt[blockIdx.y], 0), max(src_rows - before, 0)) > 0) return;
-    uint4* d = dw + (size_t)blockIdx.y * vec_per_group;
-    const uint4 z = make_uint4(0, 0, 0, 0);
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < vec_per_group; i += (size_t)gridDim.x * blockDim.x) d[i] = z;
-}
-
 // Gradient through the activation of the expert MLP.  a1: the pre-activations as the first GEMM produces them without an
 // epilogue ([rows, F] for GELU / SiLU; [rows, 2F] in the fused gate/up column order -- 32 gate columns, their 32 up
 // columns, ... -- for SwiGLU); dh: gradient of the hidden activation [rows, F]; out: gradient of a1, same layout as a1.
@@ -1472,6 +1520,52 @@ __global__ __launch_bounds__(256) void act_backward_kernel(const T* __restrict__
                 dv = d * (s * (1.0f + x * (1.0f - s)));
             }
             store_f32<T>(out + i, dv);
+        }
+    }
+}
+
+// The bf16 form: eight consecutive columns per thread, 16 bytes per load and store (F a multiple of 8; the gate and the up column of
+// a SwiGLU unit lie 32 columns apart).  Memory-bound: 10 bytes per hidden value for SwiGLU.
+template <int EPI>
+__global__ __launch_bounds__(256) void act_backward_vec_kernel(const uint4* __restrict__ a1, const uint4* __restrict__ dh, uint4* __restrict__ out,
+                                                                unsigned total, unsigned F8) {
+    auto unpack = [](const uint4& v, float* f) {
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) { f[2 * i] = __uint_as_float(w[i] << 16); f[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u); }
+    };
+    auto pack = [](const float* f) {
+        return make_uint4(gg_pack_bf16(f[0], f[1]), gg_pack_bf16(f[2], f[3]), gg_pack_bf16(f[4], f[5]), gg_pack_bf16(f[6], f[7]));
+    };
+    for (unsigned i = blockIdx.x * 256 + threadIdx.x; i < total; i += gridDim.x * 256) {
+        float d[8], x[8], o[8];
+        unpack(dh[i], d);
+        if constexpr (EPI == EPI_SWIGLU) {
+            const unsigned r = i / F8, n8 = i % F8;  // (four vectors per group of 32 columns)
+            const size_t base = (size_t)r * 2 * F8 + (n8 / 4) * 8 + n8 % 4;
+            float u[8], ou[8];
+            unpack(a1[base], x);
+            unpack(a1[base + 4], u);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float s = __builtin_amdgcn_rcpf(1.0f + __expf(-x[e]));
+                o[e] = d[e] * u[e] * (s * (1.0f + x[e] * (1.0f - s)));
+                ou[e] = d[e] * (x[e] * s);
+            }
+            out[base] = pack(o);
+            out[base + 4] = pack(ou);
+        } else {
+            unpack(a1[i], x);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                if constexpr (EPI == EPI_GELU)
+                    o[e] = d[e] * (0.5f * (1.0f + erff(x[e] * 0.70710678118654752440f)) + x[e] * 0.39894228040143267794f * __expf(-0.5f * x[e] * x[e]));
+                else {
+                    const float s = __builtin_amdgcn_rcpf(1.0f + __expf(-x[e]));
+                    o[e] = d[e] * (s * (1.0f + x[e] * (1.0f - s)));
+                }
+            }
+            out[i] = pack(o);
         }
     }
 }
@@ -1646,6 +1740,12 @@ template <typename T>
 int launch_prepack(const T* w, const T* w_up, int E_l, int K, int N, T* out, hipStream_t s) {
     const int n_eff = N * (w_up ? 2 : 1);
     const int Npad = round_up(n_eff, GG_BN);
+    if constexpr (sizeof(T) == 2) {
+        if (K % 64 == 0 && N % 8 == 0) {
+            prepack16_kernel<<<dim3(ceil_div(w_up ? Npad / 2 : Npad, 128), K / 64, E_l * (w_up ? 2 : 1)), 256, 0, s>>>(w, w_up, out, nullptr, K, N, Npad, 0);
+            return moe_check_launch("prepack_weights");
+        }
+    }
     const int n_zero = w_up ? n_eff : std::min(round_up(N, 64), Npad);  // (the re-tiling kernel writes the zeros up to there)
     if (Npad > n_zero) zero_pad_rows_kernel<T><<<dim3(64, E_l), 256, 0, s>>>(out, K, n_zero, Npad);
     prepack_kernel<T><<<dim3(ceil_div(N, 64), ceil_div(K, 64), E_l), 256, 0, s>>>(w, w_up, out, K, N, Npad);
@@ -1677,6 +1777,18 @@ extern "C" int moe_prepack_weights(const void* w, const void* w_up, int dtype, i
     MOE_REQUIRE(E_l > 0 && K > 0 && N > 0 && w && packed, MOE_ERR_INVALID, "prepack_weights: bad arguments");
     MOE_REQUIRE(!w_up || N % 32 == 0, MOE_ERR_UNSUPPORTED, "prepack_weights: gate/up interleave needs N %% 32 == 0 (N=%d)", N);
     return launch_prepack<uint16_t>((const uint16_t*)w, (const uint16_t*)w_up, E_l, K, N, (uint16_t*)packed, (hipStream_t)stream);
+}
+
+// Both re-tilings of a weight (moe_prepack_weights and moe_prepack_weights_transposed) in one pass over it.
+extern "C" int moe_prepack_weights_both(const void* w, const void* w_up, int dtype, int E_l, int K, int N, void* packed, void* packed_t,
+                                        moe_stream_t stream) {
+    MOE_REQUIRE(dtype == MOE_BF16, MOE_ERR_INVALID, "prepack_weights_both: bf16 only (dtype %d)", dtype);
+    MOE_REQUIRE(E_l > 0 && K > 0 && N > 0 && w && packed && packed_t, MOE_ERR_INVALID, "prepack_weights_both: bad arguments");
+    MOE_REQUIRE(K % 64 == 0 && N % 64 == 0, MOE_ERR_UNSUPPORTED, "prepack_weights_both: needs K and N multiples of 64 (K=%d N=%d)", K, N);
+    const int passes = w_up ? 2 : 1, Npad = round_up(N * passes, GG_BN), Kpad = round_up(K, GG_BN);
+    prepack16_kernel<<<dim3(ceil_div(Npad / passes, 128), Kpad / 64, E_l * passes), 256, 0, (hipStream_t)stream>>>(
+        (const uint16_t*)w, (const uint16_t*)w_up, (uint16_t*)packed, (uint16_t*)packed_t, K, N, Npad, Kpad);
+    return moe_check_launch("prepack_weights_both");
 }
 
 extern "C" int moe_prepack_weights_fp8(const uint8_t* w, const uint8_t* w_up, int E_l, int K, int N, uint8_t* packed,
@@ -1963,15 +2075,25 @@ extern "C" int moe_prepack_weights_transposed(const void* w, const void* w_up, i
     return moe_check_launch("prepack_weights_transposed");
 }
 
-extern "C" size_t moe_dw_workspace_bytes(int S_rows, int E_l, int K, int N) {
-    if (S_rows < 0 || E_l <= 0 || K <= 0 || N <= 0) return 0;
-    const size_t spad = (size_t)round_up(S_rows, 64) + (size_t)64 * E_l;
-    return spad * ((size_t)K + (size_t)round_up(N, GG_BN)) * 2;
+// (the operands were rewritten with the row index fastest here once; the kernel reads them as they are now)
+extern "C" size_t moe_dw_workspace_bytes(int, int, int, int) { return 0; }
+
+// split_F > 0: dy's columns in the fused gate / up order; gate columns go to dw (row pitch ldc), up columns dw_delta elements further
+static int launch_dw(const void* x, const void* dy, const int32_t* expert_cnt, int S_rows, int K, int N, int E_l, int split_F, void* dw,
+                     int ldc, long long dw_delta, hipStream_t s) {
+    MOE_REQUIRE(N % 8 == 0 && K % 8 == 0, MOE_ERR_UNSUPPORTED, "grouped_gemm_dw: bf16 needs K, N multiples of 8 (K=%d N=%d)", K, N);
+    GemmParams p{};
+    p.A = (const uint8_t*)x; p.B = (const uint8_t*)dy; p.C = dw; p.cnt = expert_cnt;
+    p.E_l = E_l; p.K = 64; p.N = N; p.Npad = round_up(N, GG_BN); p.ldc = ldc; p.S_rows = K;
+    p.dw_rows = K; p.dw_src_rows = S_rows; p.dw_split = split_F; p.dw_delta = dw_delta; p.c_group_stride = (size_t)K * ldc;
+    grouped_gemm_kernel<256, GG_BIG_NWM, EPI_NONE, false, false, true><<<num_cus(), GG_BIG_NWM * 2 * WAVE, 0, s>>>(p);
+    return moe_check_launch("grouped_gemm_dw");
 }
 
 extern "C" int moe_grouped_gemm_dw(const void* x, const void* dy, const int32_t* expert_cnt, int dtype, int S_rows, int K, int N,
                                    int E_l, int split_F, void* dw, void* ws, size_t ws_bytes, moe_stream_t stream) {
     hipStream_t s = (hipStream_t)stream;
+    (void)ws; (void)ws_bytes;
     MOE_REQUIRE(S_rows >= 0 && K > 0 && N > 0 && E_l > 0 && E_l <= GG_MAXG, MOE_ERR_INVALID, "grouped_gemm_dw: bad shape");
     MOE_REQUIRE(expert_cnt && dw && (S_rows == 0 || (x && dy)), MOE_ERR_INVALID, "grouped_gemm_dw: null pointer");
     MOE_REQUIRE(split_F == 0 || (dtype == MOE_BF16 && split_F % 32 == 0 && N == 2 * split_F), MOE_ERR_INVALID,
@@ -1982,27 +2104,61 @@ extern "C" int moe_grouped_gemm_dw(const void* x, const void* dy, const int32_t*
         return moe_check_launch("grouped_gemm_dw_f32");
     }
     MOE_REQUIRE(dtype == MOE_BF16, MOE_ERR_INVALID, "grouped_gemm_dw: dtype %d", dtype);
-    MOE_REQUIRE(N % 8 == 0 && K % 8 == 0, MOE_ERR_UNSUPPORTED, "grouped_gemm_dw: bf16 needs K, N multiples of 8 (K=%d N=%d)", K, N);
-    MOE_REQUIRE(ws && ws_bytes >= moe_dw_workspace_bytes(S_rows, E_l, K, N), MOE_ERR_WORKSPACE, "grouped_gemm_dw: workspace %zu < %zu",
-                ws_bytes, moe_dw_workspace_bytes(S_rows, E_l, K, N));
-    const int spad = round_up(S_rows, 64) + 64 * E_l;  // upper bound of the padded row total, and the operands' pitch
-    MOE_REQUIRE((unsigned long long)K * (unsigned long long)spad * 2ull < (1ull << 32), MOE_ERR_UNSUPPORTED,
-                "grouped_gemm_dw: the transposed activations must stay under 4 GiB (%d x %d)", K, spad);
-    const int Npad = round_up(N, GG_BN);
-    uint16_t* xT = (uint16_t*)ws;                       // [K, spad]
-    uint16_t* dyP = xT + (size_t)K * spad;              // [spad / 32][Npad][32]
-    const int pblocks = spad / 64;
-    dw_zero_empty_kernel<<<dim3(256, E_l), 256, 0, s>>>((uint4*)dw, expert_cnt, (size_t)K * N * 2 / 16, S_rows);
-    if (S_rows > 0) {
-        dw_operand_kernel<false><<<dim3(ceil_div(K, 64), pblocks), 256, 0, s>>>((const uint16_t*)x, expert_cnt, E_l, S_rows, K, xT, spad, 0, 0);
-        dw_operand_kernel<true><<<dim3(Npad / 64, pblocks), 256, 0, s>>>((const uint16_t*)dy, expert_cnt, E_l, S_rows, N, dyP, spad, Npad, split_F);
-        GemmParams p{};
-        p.A = (const uint8_t*)xT; p.B = (const uint8_t*)dyP; p.C = dw; p.cnt = expert_cnt;
-        p.E_l = E_l; p.K = spad; p.N = N; p.Npad = Npad; p.ldc = N; p.S_rows = K;
-        p.dw_rows = K; p.dw_src_rows = S_rows; p.c_group_stride = (size_t)K * N;
-        grouped_gemm_kernel<256, GG_BIG_NWM, EPI_NONE, false, false, true><<<num_cus(), GG_BIG_NWM * 2 * WAVE, 0, s>>>(p);
-    }
-    return moe_check_launch("grouped_gemm_dw");
+    return launch_dw(x, dy, expert_cnt, S_rows, K, N, E_l, split_F, dw, N, split_F, s);
+}
+
+extern "C" int moe_grouped_gemm_dw_pair(const void* x, const void* dy, const int32_t* expert_cnt, int S_rows, int K, int F, int E_l,
+                                        void* dw_gate, void* dw_up, moe_stream_t stream) {
+    MOE_REQUIRE(S_rows >= 0 && K > 0 && F > 0 && F % 32 == 0 && E_l > 0 && E_l <= GG_MAXG, MOE_ERR_INVALID, "grouped_gemm_dw_pair: bad shape");
+    MOE_REQUIRE(expert_cnt && dw_gate && dw_up && (S_rows == 0 || (x && dy)), MOE_ERR_INVALID, "grouped_gemm_dw_pair: null pointer");
+    return launch_dw(x, dy, expert_cnt, S_rows, K, 2 * F, E_l, F, dw_gate, F, (bf16_t*)dw_up - (bf16_t*)dw_gate, (hipStream_t)stream);
+}
+
+// ---- the expert MLP of a training step, one call per direction (bf16).  Weights as moe_prepack_weights (forward) and
+// moe_prepack_weights_transposed (backward) re-tile them; pre_act as moe_grouped_gemm_act_keep leaves it.
+extern "C" int moe_mlp_train_forward(const void* x, const int32_t* expert_cnt, int S_rows, int H, int F, int E_l, int act, const void* w1,
+                                     const void* w2, void* hidden, void* pre_act, void* out, void* part_ws, size_t part_ws_bytes,
+                                     moe_stream_t stream) {
+    MOE_REQUIRE(S_rows > 0 && H > 0 && F > 0 && E_l > 0 && E_l <= GG_MAXG, MOE_ERR_INVALID, "mlp_train_forward: bad shape");
+    MOE_REQUIRE(act > EPI_NONE && act <= EPI_SWIGLU, MOE_ERR_INVALID, "mlp_train_forward: activation %d", act);
+    MOE_REQUIRE(H % 64 == 0 && F % 64 == 0, MOE_ERR_UNSUPPORTED, "mlp_train_forward: needs H, F multiples of 64 (H=%d F=%d)", H, F);
+    MOE_REQUIRE(x && expert_cnt && w1 && w2 && hidden && pre_act && out, MOE_ERR_INVALID, "mlp_train_forward: null pointer");
+    hipStream_t s = (hipStream_t)stream;
+    GemmParams p{};
+    p.A = (const uint8_t*)x; p.B = (const uint8_t*)w1; p.C = hidden; p.C2 = pre_act; p.cnt = expert_cnt;
+    p.E_l = E_l; p.K = H; p.N = F; p.ldc = F; p.S_rows = S_rows; p.Npad = round_up(act == EPI_SWIGLU ? 2 * F : F, GG_BN);
+    const int rc = launch_gemm<false>(p, act, s, part_ws, part_ws_bytes);
+    if (rc) return rc;
+    GemmParams q{};
+    q.A = (const uint8_t*)hidden; q.B = (const uint8_t*)w2; q.C = out; q.cnt = expert_cnt; q.zero_tail = 1;
+    q.E_l = E_l; q.K = F; q.N = H; q.ldc = H; q.S_rows = S_rows; q.Npad = round_up(H, GG_BN);
+    return launch_gemm<false>(q, EPI_NONE, s, part_ws, part_ws_bytes);
+}
+
+extern "C" int moe_mlp_train_backward(const void* x, const void* hidden, const void* pre_act, const void* dy, const int32_t* expert_cnt,
+                                      int S_rows, int H, int F, int E_l, int act, const void* w1_t, const void* w2_t, void* dh, void* d_pre,
+                                      void* dx, void* dw1, void* dw_up, void* dw2, void* part_ws, size_t part_ws_bytes, moe_stream_t stream) {
+    MOE_REQUIRE(S_rows > 0 && H > 0 && F > 0 && E_l > 0 && E_l <= GG_MAXG, MOE_ERR_INVALID, "mlp_train_backward: bad shape");
+    MOE_REQUIRE(act > EPI_NONE && act <= EPI_SWIGLU, MOE_ERR_INVALID, "mlp_train_backward: activation %d", act);
+    MOE_REQUIRE(H % 64 == 0 && F % 64 == 0, MOE_ERR_UNSUPPORTED, "mlp_train_backward: needs H, F multiples of 64 (H=%d F=%d)", H, F);
+    MOE_REQUIRE(x && hidden && pre_act && dy && expert_cnt && w1_t && w2_t && dh && d_pre && dx && dw1 && dw2 && (act != EPI_SWIGLU || dw_up),
+                MOE_ERR_INVALID, "mlp_train_backward: null pointer");
+    hipStream_t s = (hipStream_t)stream;
+    const int NP = act == EPI_SWIGLU ? 2 * F : F;
+    GemmParams p{};
+    p.A = (const uint8_t*)dy; p.B = (const uint8_t*)w2_t; p.C = dh; p.cnt = expert_cnt;
+    p.E_l = E_l; p.K = H; p.N = F; p.ldc = F; p.S_rows = S_rows; p.Npad = round_up(F, GG_BN);
+    int rc = launch_gemm<false>(p, EPI_NONE, s, part_ws, part_ws_bytes);
+    if (!rc) rc = launch_dw(hidden, dy, expert_cnt, S_rows, F, H, E_l, 0, dw2, H, 0, s);
+    if (!rc) rc = moe_mlp_act_backward(pre_act, dh, MOE_BF16, S_rows, F, act, d_pre, stream);
+    if (rc) return rc;
+    GemmParams q{};
+    q.A = (const uint8_t*)d_pre; q.B = (const uint8_t*)w1_t; q.C = dx; q.cnt = expert_cnt; q.zero_tail = 1;
+    q.E_l = E_l; q.K = NP; q.N = H; q.ldc = H; q.S_rows = S_rows; q.Npad = round_up(H, GG_BN);
+    rc = launch_gemm<false>(q, EPI_NONE, s, part_ws, part_ws_bytes);
+    if (rc) return rc;
+    if (act == EPI_SWIGLU) return launch_dw(x, d_pre, expert_cnt, S_rows, H, NP, E_l, F, dw1, F, (bf16_t*)dw_up - (bf16_t*)dw1, s);
+    return launch_dw(x, d_pre, expert_cnt, S_rows, H, NP, E_l, 0, dw1, F, 0, s);
 }
 
 extern "C" int moe_transpose_weights_f32(const float* w, int E_l, int K, int N, float* out, moe_stream_t stream) {
@@ -2020,15 +2176,28 @@ extern "C" int moe_mlp_act_backward(const void* a1, const void* dh, int dtype, i
     MOE_REQUIRE(act != EPI_SWIGLU || F % 32 == 0, MOE_ERR_UNSUPPORTED, "mlp_act_backward: swiglu needs F %% 32 == 0");
     if (rows == 0) return MOE_OK;
     MOE_REQUIRE(a1 && dh && d_a1, MOE_ERR_INVALID, "mlp_act_backward: null pointer");
-    const int blocks = (int)std::min<size_t>(((size_t)rows * F + 255) / 256, (size_t)num_cus() * 32);
     hipStream_t s = (hipStream_t)stream;
+    if (dtype == MOE_BF16 && F % 8 == 0) {
+        const int F8 = F / 8, chunk = (int)std::min<long long>(rows, (1ll << 31) / F8);  // rows per launch: 32-bit indices
+        for (int r0 = 0; r0 < rows; r0 += chunk) {
+            const unsigned total = (unsigned)std::min(chunk, rows - r0) * (unsigned)F8;
+            const int blocks = (int)std::min<unsigned>((total + 255) / 256, (unsigned)num_cus() * 32);
+            const size_t off = (size_t)r0 * F8, off1 = off * (act == EPI_SWIGLU ? 2 : 1);
+#define GG_ACTV(EPIv) act_backward_vec_kernel<EPIv><<<blocks, 256, 0, s>>>((const uint4*)a1 + off1, (const uint4*)dh + off, (uint4*)d_a1 + off1, total, F8)
+            if (act == EPI_GELU) GG_ACTV(EPI_GELU);
+            else if (act == EPI_SILU) GG_ACTV(EPI_SILU);
+            else GG_ACTV(EPI_SWIGLU);
+#undef GG_ACTV
+        }
+        return moe_check_launch("mlp_act_backward");
+    }
+    const int blocks = (int)std::min<size_t>(((size_t)rows * F + 255) / 256, (size_t)num_cus() * 32);
 #define GG_ACTB(EPIv, Tv) act_backward_kernel<EPIv, Tv><<<blocks, 256, 0, s>>>((const Tv*)a1, (const Tv*)dh, (Tv*)d_a1, (size_t)rows, F)
     if (dtype == MOE_F32) {
         if (act == EPI_GELU) GG_ACTB(EPI_GELU, float);
         else GG_ACTB(EPI_SILU, float);
     } else if (act == EPI_GELU) GG_ACTB(EPI_GELU, bf16_t);
-    else if (act == EPI_SILU) GG_ACTB(EPI_SILU, bf16_t);
-    else GG_ACTB(EPI_SWIGLU, bf16_t);
+    else GG_ACTB(EPI_SILU, bf16_t);  // (SwiGLU has F a multiple of 32)
 #undef GG_ACTB
     return moe_check_launch("mlp_act_backward");
 }

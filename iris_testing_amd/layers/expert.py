@@ -3,6 +3,7 @@ expert MLP the workloads define (Linear-act-Linear, SwiGLU, fp8) which the refer
 """
 from __future__ import annotations
 
+import weakref
 from dataclasses import dataclass, field
 from typing import Optional
 
@@ -19,17 +20,31 @@ _PACKED = {}
 _PART_WS = {}
 
 
+def _pack_key(kind: str, w: torch.Tensor, w_up: Optional[torch.Tensor]):
+    return (kind, w.data_ptr(), w._version, None if w_up is None else (w_up.data_ptr(), w_up._version), tuple(w.shape), w.dtype, w.device)
+
+
+def _drop_packs(kind: str, w: torch.Tensor) -> None:
+    for k in [k for k, v in _PACKED.items() if v[0]() is None or (v[0]() is w and k[0] == kind)]:
+        del _PACKED[k]
+
+
 def _cached_pack(kind: str, w: torch.Tensor, w_up: Optional[torch.Tensor], build) -> torch.Tensor:
-    import weakref
-    key = (kind, w.data_ptr(), w._version, None if w_up is None else (w_up.data_ptr(), w_up._version), tuple(w.shape), w.dtype,
-           w.device)
+    key = _pack_key(kind, w, w_up)
     hit = _PACKED.get(key)
     if hit is not None and hit[0]() is w:
         return hit[1]
-    for k in [k for k, v in _PACKED.items() if v[0]() is None or (v[0]() is w and k[0] == kind)]:
-        del _PACKED[k]
+    _drop_packs(kind, w)
     packed = build(w, w_up)
     _PACKED[key] = (weakref.ref(w), packed)
+    return packed
+
+
+def _pack_both(w: torch.Tensor, w_up: Optional[torch.Tensor]) -> torch.Tensor:
+    """_packed_weights' and _packed_weights_t's re-tilings in one pass over the weight; the second one is left in the cache."""
+    _drop_packs("T", w)
+    packed, packed_t = ops.prepack_weights_both(w, w_up)
+    _PACKED[_pack_key("T", w, w_up)] = (weakref.ref(w), packed_t)
     return packed
 
 
@@ -153,7 +168,13 @@ class ExpertWeights:
         step): the forward pass would otherwise multiply with the weights of before the update while the backward pass,
         which re-tiles the transposes by tensor version, uses the new ones."""
         if self.raw is not None and self._versions(self.raw) != self.raw_versions:
-            self.w1, self.w2, self.w_up = self._derive(self.raw)
+            w1, w2, w_up = self.raw
+            if w1.dtype == torch.bfloat16 and self.hidden % 64 == 0 and self.ffn % 64 == 0 and torch.is_grad_enabled() and \
+                    all(t is None or (t.requires_grad and t.is_contiguous()) for t in self.raw):
+                # weights in training: the backward pass of this step will want their transposes too
+                self.w1, self.w2, self.w_up = _pack_both(w1, w_up), _pack_both(w2, None), None
+            else:
+                self.w1, self.w2, self.w_up = self._derive(self.raw)
             self.raw_versions = self._versions(self.raw)
         return self
 
@@ -174,16 +195,12 @@ class ExpertMLP(torch.autograd.Function):
     def forward(ctx, tokens, cnt, ew, w1, w2, w_up):
         tokens = tokens.contiguous()
         S, F = tokens.shape[0], ew.ffn
-        hidden = torch.empty((S, F), dtype=tokens.dtype, device=tokens.device)
         a1 = None
         if tokens.dtype == torch.bfloat16 and ew.act != "none" and S:
             # the first GEMM also keeps what it feeds to the activation: the backward pass would otherwise run it again
-            ws = _part_ws(tokens.device)
-            a1 = torch.empty((S, 2 * F if ew.act == "swiglu" else F), dtype=tokens.dtype, device=tokens.device)
-            ops.grouped_gemm_act_keep(tokens, ew.w1, cnt, S, F, ew.act, hidden, a1, part_ws=ws)
-            out = torch.zeros((S, ew.hidden), dtype=tokens.dtype, device=tokens.device)  # (rows past the counted total stay zero)
-            ops.grouped_gemm_mapped(hidden, None, ew.w2, cnt, S, ew.hidden, "none", out, part_ws=ws)
+            out, hidden, a1 = ops.mlp_train_forward(tokens, cnt, ew.act, ew.w1, ew.w2, F, part_ws=_part_ws(tokens.device))
         else:
+            hidden = torch.empty((S, F), dtype=tokens.dtype, device=tokens.device)
             out = ops.grouped_mlp(tokens, cnt, ew.act, ew.w1, ew.w2, ew.w_up, F=F, hidden_ws=hidden)
         ctx.save_for_backward(tokens, hidden, cnt, w1, w2, w_up, a1)
         ctx.ew = ew
@@ -211,15 +228,18 @@ class ExpertMLP(torch.autograd.Function):
             dw1 = ops.grouped_gemm_dw(tokens, da1, cnt)
             return dx, None, None, dw1, dw2, None
         ws = _part_ws(tokens.device)
+        if a1 is not None:
+            dx, dw1, dw2, dw_up = ops.mlp_train_backward(tokens, hidden, a1, dy, cnt, ew.act, _packed_weights_t(w1, w_up), _packed_weights_t(w2),
+                                                         part_ws=ws)
+            return dx, None, None, dw1, dw2, dw_up
         NP = 2 * F if swiglu else F
         dh = torch.zeros((S, F), dtype=dy.dtype, device=dy.device)
         dx = torch.zeros((S, H), dtype=dy.dtype, device=dy.device)
         if S:
             ops.grouped_gemm_mapped(dy, None, _packed_weights_t(w2), cnt, S, F, "none", dh, part_ws=ws)
-        if a1 is None:  # (no rows, or an MLP without an activation)
-            a1 = torch.zeros((S, NP), dtype=dy.dtype, device=dy.device)
-            if S:
-                ops.grouped_gemm_mapped(tokens, None, ew.w1, cnt, S, NP, "none", a1, part_ws=ws)
+        a1 = torch.zeros((S, NP), dtype=dy.dtype, device=dy.device)  # (no rows, or an MLP without an activation)
+        if S:
+            ops.grouped_gemm_mapped(tokens, None, ew.w1, cnt, S, NP, "none", a1, part_ws=ws)
         dw2 = ops.grouped_gemm_dw(hidden, dy, cnt)
         da1 = ops.mlp_act_backward(a1, dh, ew.act)
         if S:

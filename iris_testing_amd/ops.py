@@ -618,6 +618,57 @@ def prepack_weights_transposed(w: torch.Tensor, w_up: Optional[torch.Tensor] = N
     return out
 
 
+def prepack_weights_both(w: torch.Tensor, w_up: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, torch.Tensor]:
+    """(prepack_weights(w, w_up), prepack_weights_transposed(w, w_up)) in one pass over the weights."""
+    _req_cuda(w, "weights")
+    assert w.dtype == torch.bfloat16
+    E_l, K, N = w.shape
+    if w_up is not None:
+        _req_cuda(w_up, "w_up")
+        assert w_up.shape == w.shape and w_up.dtype == w.dtype
+    n_tot = N * (2 if w_up is not None else 1)
+    lib = L.lib()
+    out = torch.empty(lib.moe_prepack_bytes(L.MOE_BF16, E_l, K, n_tot), dtype=torch.uint8, device=w.device)
+    out_t = torch.empty(lib.moe_prepack_bytes(L.MOE_BF16, E_l, n_tot, K), dtype=torch.uint8, device=w.device)
+    L.check(lib.moe_prepack_weights_both(L.ptr(w), L.ptr(w_up), L.MOE_BF16, E_l, K, N, L.ptr(out), L.ptr(out_t), L.stream_ptr()))
+    return out, out_t
+
+
+def mlp_train_forward(x: torch.Tensor, expert_cnt: torch.Tensor, act: str, w1: torch.Tensor, w2: torch.Tensor, F: int,
+                      part_ws: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """(out [S,H], hidden [S,F], pre_act) of the bf16 expert MLP with what its backward pass needs kept; w1 / w2 prepacked."""
+    _req_cuda(x, "x")
+    _req_i32(expert_cnt, "expert_cnt")
+    assert x.dtype == torch.bfloat16
+    S, H = x.shape
+    hidden = torch.empty((S, F), dtype=x.dtype, device=x.device)
+    pre = torch.empty((S, 2 * F if act == "swiglu" else F), dtype=x.dtype, device=x.device)
+    out = torch.empty_like(x)
+    L.check(L.lib().moe_mlp_train_forward(x.data_ptr(), expert_cnt.data_ptr(), S, H, F, expert_cnt.numel(), L.ACT[act], w1.data_ptr(),
+                                          w2.data_ptr(), hidden.data_ptr(), pre.data_ptr(), out.data_ptr(), L.ptr(part_ws),
+                                          0 if part_ws is None else part_ws.numel() * part_ws.element_size(), L.stream_ptr()))
+    return out, hidden, pre
+
+
+def mlp_train_backward(x: torch.Tensor, hidden: torch.Tensor, pre: torch.Tensor, dy: torch.Tensor, expert_cnt: torch.Tensor, act: str,
+                       w1_t: torch.Tensor, w2_t: torch.Tensor, part_ws: Optional[torch.Tensor] = None):
+    """(dx, dw1, dw2, dw_up or None) of mlp_train_forward; w1_t / w2_t: prepack_weights_transposed of (w1, w_up) and w2."""
+    _req_cuda(dy, "dy")
+    _req_i32(expert_cnt, "expert_cnt")
+    assert dy.dtype == torch.bfloat16 and dy.shape == x.shape
+    S, H = x.shape
+    F, E_l, dev = hidden.shape[1], expert_cnt.numel(), x.device
+    swiglu = act == "swiglu"
+    dh, d_pre, dx = torch.empty_like(hidden), torch.empty_like(pre), torch.empty_like(x)
+    dw1, dw2 = torch.empty((E_l, H, F), dtype=x.dtype, device=dev), torch.empty((E_l, F, H), dtype=x.dtype, device=dev)
+    dw_up = torch.empty_like(dw1) if swiglu else None
+    L.check(L.lib().moe_mlp_train_backward(x.data_ptr(), hidden.data_ptr(), pre.data_ptr(), dy.data_ptr(), expert_cnt.data_ptr(), S, H, F,
+                                           E_l, L.ACT[act], w1_t.data_ptr(), w2_t.data_ptr(), dh.data_ptr(), d_pre.data_ptr(), dx.data_ptr(),
+                                           dw1.data_ptr(), L.ptr(dw_up), dw2.data_ptr(), L.ptr(part_ws),
+                                           0 if part_ws is None else part_ws.numel() * part_ws.element_size(), L.stream_ptr()))
+    return dx, dw1, dw2, dw_up
+
+
 def transpose_weights_f32(w: torch.Tensor) -> torch.Tensor:
     """[E_l,K,N] fp32 -> [E_l,N,K]."""
     _req_cuda(w, "weights")
@@ -641,10 +692,8 @@ def grouped_gemm_dw(x: torch.Tensor, dy: torch.Tensor, expert_cnt: torch.Tensor,
     E_l = expert_cnt.numel()
     code = L.dtype_code(x.dtype)
     dw = torch.empty((E_l, K, N), dtype=x.dtype, device=x.device)
-    nbytes = L.lib().moe_dw_workspace_bytes(S, E_l, K, N) if x.dtype == torch.bfloat16 else 0
-    ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=x.device)
-    L.check(L.lib().moe_grouped_gemm_dw(L.ptr(x), L.ptr(dy), L.ptr(expert_cnt), code, S, K, N, E_l, split_F, L.ptr(dw), L.ptr(ws),
-                                        nbytes, L.stream_ptr()))
+    L.check(L.lib().moe_grouped_gemm_dw(L.ptr(x), L.ptr(dy), L.ptr(expert_cnt), code, S, K, N, E_l, split_F, L.ptr(dw), None, 0,
+                                        L.stream_ptr()))
     return dw
 
 

@@ -184,3 +184,33 @@ def test_expert_mlp_follows_in_place_weight_updates():
     # inference path (no autograd) sees the update too
     with torch.no_grad():
         assert _rel(expert_mlp(xd, ew, cnt_d), want1) < 2.0 ** -6
+
+
+@pytest.mark.parametrize("K,F,cnt", [(8, 32, (1,)), (264, 96, (31, 0, 33)), (256, 128, (64, 65, 63)), (520, 160, (127, 2, 129, 256))])
+def test_weight_gradient_pair_and_both_re_tilings_at_tile_edges(K, F, cnt):
+    """The weight-gradient kernel reads its operands with the row index slow and ends every group's range in the load descriptor: row
+    counts around a stage (32) and a pair of stages, partly filled tiles in both directions, both halves of a gate / up pair."""
+    rng = np.random.default_rng(K + F)
+    E_l, S = len(cnt), sum(cnt)
+    x = torch.from_numpy(rng.standard_normal((S + 3, K)).astype(np.float32)).bfloat16()
+    dy = torch.from_numpy(rng.standard_normal((S + 3, 2 * F)).astype(np.float32)).bfloat16()
+    x[S:] = float("nan")  # (rows past the counted total take no part)
+    c = torch.tensor(cnt, dtype=torch.int32, device=DEV)
+    dg, du = (torch.full((E_l, K, F), -7.0, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    from iris_testing_amd import _lib as L
+    xd, dyd = x.to(DEV), dy.to(DEV)
+    L.check(L.lib().moe_grouped_gemm_dw_pair(xd.data_ptr(), dyd.data_ptr(), c.data_ptr(), S + 3, K, F, E_l, dg.data_ptr(), du.data_ptr(), L.stream_ptr()))
+    d4, r = dy.view(S + 3, F // 32, 2, 32), 0
+    for e, n in enumerate(cnt):
+        for got, half in ((dg, 0), (du, 1)):
+            want = x[r:r + n].double().T @ d4[r:r + n, :, half].reshape(n, F).double()
+            if n:
+                assert _rel(got[e], want) < 2.0 ** -7, (e, half)
+            else:
+                assert bool((got[e] == 0).all())
+        r += n
+    if K % 64 == 0 and F % 64 == 0:
+        w, wu = (torch.from_numpy(rng.standard_normal((E_l, K, F)).astype(np.float32)).bfloat16().to(DEV) for _ in range(2))
+        for up in (None, wu):
+            packed, packed_t = ops.prepack_weights_both(w, up)
+            assert torch.equal(packed, ops.prepack_weights(w, up)) and torch.equal(packed_t, ops.prepack_weights_transposed(w, up))
