@@ -147,9 +147,8 @@ int moe_pack_tokens_fp8_gated(const void* x_bf16, int T, int H, const int32_t* t
  * token_buf[e,s,j,:] = recv[s, expert_offs_s[e]+j, :] for j < recv_counts[s,e], else zeros;
  * pca[e,s] = recv_counts[s,e].  status (nullable): 1 on count > CAP, or when a counted row lies at or
  * past row M of its slot (the sender's pack dropped it: it reads as zeros).
- * map_ws (here and in every entry point below that takes one): int32 scratch of
- * moe_recv_map_ints(W, E_l, n_out) elements (prefix tables over the counts; n_out = rows of the
- * output buffer, which no longer enters the size). */
+ * map_ws (here and in every entry point below that takes one): unused (the prefix tables live on the chip;
+ * kept for ABI stability, may be NULL), as is moe_recv_map_ints. */
 size_t moe_recv_map_ints(int W, int E_l, int n_out);
 int moe_unpack_token_buf(const void* recv, int dtype, int W, int M, int H, const int32_t* recv_counts, int E_l,
                          int CAP, void* token_buf, int32_t* pca, int32_t* map_ws, int32_t* status,
@@ -281,9 +280,15 @@ size_t moe_gemm_part_workspace_bytes(void);
 int moe_gemm_split_plan(int total_tiles, int grid, int k_stages, int max_units, int32_t* out);
 int moe_zero_padding_rows(void* buf, int dtype, int W, int M, int H, const int32_t* recv_counts, int E_l,
                           moe_stream_t stream);
+/* moe_recv_prepare: everything the destination side derives from recv_counts in one launch: the row map of moe_recv_row_map (M >= 1) or
+ * moe_recv_row_map_flat (M == 0), row_gate as in moe_recv_row_map_gated (recv_gate / row_gate: both or neither), row_scale[r] =
+ * the fp8 scale of row r's source row (recv_scale / row_scale: both or neither; rows without a source take that of row 0),
+ * the per-expert totals, and, if ret is given ([W,M,H] of `dtype`), moe_zero_padding_rows on it. */
+int moe_recv_prepare(const int32_t* recv_counts, int W, int E_l, int M, int n_rows, const float* recv_gate, const float* recv_scale,
+                     int32_t* row_map, float* row_gate, float* row_scale, int32_t* expert_cnt, void* ret, int dtype, int H,
+                     moe_stream_t stream);
 /* Gradient of moe_shuffle (the reference leaves TokenShuffle.backward empty, token_shuffle.py:58-60):
- * grad_token_buf[e,s,j,:] = grad_rows[off[e,s]+j,:] for j < pca[e,s], zeros in the padding; off as in moe_shuffle.
- * map_ws >= moe_recv_map_ints(W,E_l,0) ints. */
+ * grad_token_buf[e,s,j,:] = grad_rows[off[e,s]+j,:] for j < pca[e,s], zeros in the padding; off as in moe_shuffle. */
 int moe_shuffle_backward(const void* grad_rows, int dtype, int E_l, int W, int CAP, int H, const int32_t* pca,
                          void* grad_token_buf, int32_t* map_ws, moe_stream_t stream);
 /* moe_grouped_mlp_fp8 with the same row indirection: the row quantisation reads input row r from row
@@ -301,7 +306,8 @@ int moe_grouped_mlp_fp8_mapped(const void* a_base_bf16, int a_rows, const int32_
 /* moe_grouped_mlp_fp8_mapped for rows that arrive quantised (moe_pack_tokens_fp8): a_q [a_rows,H] codes and a_scale
  * [a_rows] scales, gathered through a_row_map (nullable) by the first GEMM as it loads them; xs_ws [S_rows] receives the
  * scales in the GEMM's row order.  Everything else as in moe_grouped_mlp_fp8_mapped, whose result it reproduces bit for
- * bit when a_q / a_scale are the quantised rows of that call's input. */
+ * bit when a_q / a_scale are the quantised rows of that call's input.  a_scale == NULL: xs_ws holds them already
+ * (moe_recv_prepare). */
 int moe_grouped_mlp_fp8_q_mapped(const uint8_t* a_q, const float* a_scale, int a_rows, const int32_t* a_row_map,
                                  const int32_t* expert_cnt, int S_rows, int H, int F, int E_l, const uint8_t* wgu_packed,
                                  const float* sg, const float* su, const uint8_t* wd_packed, const float* sd, float* xs_ws,
@@ -360,6 +366,8 @@ int moe_mlp_train_backward(const void* x, const void* hidden, const void* pre_ac
 int moe_transpose_weights_f32(const float* w, int E_l, int K, int N, float* out, moe_stream_t stream);
 int moe_mlp_act_backward(const void* a1, const void* dh, int dtype, int rows, int F, int act, void* d_a1,
                          moe_stream_t stream);
+/* (moe_combine_backward: dst_sizes may be NULL where all T*k slots are routed: a destination's rows then end where the next one's
+ * start, the last one's at T*k) */
 int moe_combine_backward(const void* d_out, const void* ret, int dtype, int W, int M, int H, const int32_t* topk_idx,
                          const int32_t* pos, const float* gate, const int32_t* dst_sizes, const int32_t* dst_offsets, int T,
                          int k, int E_l, void* d_ret, float* d_gate, moe_stream_t stream);
@@ -403,6 +411,50 @@ int moe_diag_mfma_loop(int fp8, int random_data, int iters, int workgroups, floa
  * launches compute the same results (unless bit 0 is set).  Used by `bench.py --gemm-phases`. */
 size_t moe_diag_gemm_trace_words(void);
 int moe_diag_gemm_trace(unsigned long long* trace, size_t words, int flags);
+
+/* ---- the whole hot path of one step as one call -------------------------------------------------------------------
+ * What rank 0 does for one batch (route, count, pack; row map, expert MLP, return; combine), through the entry points above
+ * with the arguments named alike there; only enqueues, as they do.  Modes: fused = the GEMMs gather from / scatter into the transfer
+ * buffers; flat = padding-free payloads (fused); gated = gates travel with the rows (fused); quant = fp8 experts; q_dispatch
+ * = rows travel quantised (fused, quant, not flat); f32_weights = the weights are those of moe_grouped_mlp (not fused).  Pointers that a mode does not use may be NULL. */
+typedef struct moe_step_args {
+    int32_t tokens, hidden, experts, topk, world, ffn, act, dtype, M, S; /* S: rows received */
+    int32_t fused, flat, gated, quant, q_dispatch, f32_weights;
+    /* source side */
+    const void *x, *router;
+    const float* bias;
+    float* logits;
+    int32_t* idx;
+    float* gate;
+    void* route_ws;
+    size_t route_ws_bytes;
+    int32_t *send_counts, *expert_offs, *dst_sizes, *dst_offsets, *caps, *pos, *row_token;
+    void* count_ws;
+    size_t count_ws_bytes;
+    void* send; /* [W,M,H] rows, fp8 codes (q_dispatch) or the payload (flat) */
+    float *send_scale, *send_gate;
+    int32_t* status;
+    /* destination side */
+    const void* recv; /* [W,M,H] rows, fp8 codes (q_dispatch) or the flat payload (flat) */
+    const float *recv_scale, *recv_gate;
+    const int32_t* recv_counts;
+    int32_t *row_map, *expert_cnt;
+    float* row_gate;
+    const void *w1, *w_up, *w2; /* packed; w_up: fp32 SwiGLU only */
+    const float *s1, *s_up, *s2; /* fp8 weight scales */
+    void *rows, *y, *hidden_ws; /* expert-major rows and results (not fused), hidden activation (not quant) */
+    uint8_t *xq, *hq, *hscale;
+    float* xs;
+    int32_t *unpack_map, *ret_map; /* (not fused) */
+    void* part_ws;
+    size_t part_ws_bytes;
+    void* ret; /* [W,M,H], or [S,H] (flat) */
+    /* source side again */
+    const void* returned;
+    const int32_t* zero_off; /* one zero (flat) */
+    void* out;
+} moe_step_args;
+int moe_step(const moe_step_args* args /* host */, moe_stream_t stream);
 
 #ifdef __cplusplus
 }

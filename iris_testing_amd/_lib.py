@@ -28,6 +28,17 @@ class MoeLibraryError(RuntimeError):
         self.text = text
 
 
+class StepArgs(ctypes.Structure):
+    """moe_step_args of include/moe_gfx950.h: integers, then pointers; *_bytes are sizes."""
+    _fields_ = [(n, c_int32) for n in (
+        "tokens hidden experts topk world ffn act dtype M S fused flat gated quant q_dispatch f32_weights").split()] + [
+        (n, c_size_t if n.endswith("_bytes") else c_void_p) for n in (
+        "x router bias logits idx gate route_ws route_ws_bytes send_counts expert_offs dst_sizes dst_offsets caps "
+        "pos row_token count_ws count_ws_bytes send send_scale send_gate status recv recv_scale recv_gate "
+        "recv_counts row_map expert_cnt row_gate w1 w_up w2 s1 s_up s2 rows y hidden_ws xq hq hscale xs unpack_map "
+        "ret_map part_ws part_ws_bytes ret returned zero_off out").split()]
+
+
 P = c_void_p
 _SIGNATURES = {
     "moe_abi_version": (c_int, []),
@@ -82,6 +93,8 @@ _SIGNATURES = {
     "moe_combine_backward": (c_int, [P, P, c_int, c_int, c_int, c_int, P, P, P, P, P, c_int, c_int, c_int, P, P, P]),
     "moe_gemm_split_plan": (c_int, [c_int, c_int, c_int, c_int, P]),
     "moe_zero_padding_rows": (c_int, [P, c_int, c_int, c_int, c_int, P, c_int, P]),
+    "moe_recv_prepare": (c_int, [P, c_int, c_int, c_int, c_int, P, P, P, P, P, P, P, c_int, c_int, P]),
+    "moe_step": (c_int, [POINTER(StepArgs), P]),
     "moe_grouped_mlp_fp8_mapped": (c_int, [P, c_int, P, P, c_int, c_int, c_int, c_int, P, P, P, P, P, P, P, P, P, P, P, c_int, P, P,
                                            c_size_t, P]),  # (.., xq_ws, xs_ws, hq_ws, hscale_ws, row_gate, out, out_rows, ..)
     "moe_diag_mfma_loop_sink_floats": (c_size_t, []),

@@ -9,16 +9,17 @@
 // Order of rows inside a (dst, el) bucket is ascending token index (utils.py:210-219).  An
 // atomic-counter scatter would not reproduce that, so the position of every routed slot is
 // computed as   expert_start[ex] + (rows of ex in earlier 64-token blocks) + (rows of ex in
-// earlier lanes of this block),  with LDS histograms, a wave prefix scan and per-expert lane masks.
+// earlier lanes of this block),  with LDS histograms and per-expert lane masks.
 // All integer work: results are bit-exact by construction.
 #include "common.h"
 #include <atomic>
+#include <type_traits>
 
 namespace {
 
 constexpr int CB = MOE_COUNT_BLOCK;  // 64 tokens = one wave per counting block
 
-// ---- 1. per-block histogram: hist[e][b] = #slots of block b routed to expert e --------------------
+// ---- 1. per-block histogram: hist[b][e] = #slots of block b routed to expert e --------------------
 __global__ __launch_bounds__(256) void block_hist_kernel(const int32_t* __restrict__ idx, int32_t* __restrict__ hist,
                                                           int T, int k, int E, int NB) {
     extern __shared__ int32_t lds_hist[];  // [4][E]
@@ -36,7 +37,7 @@ __global__ __launch_bounds__(256) void block_hist_kernel(const int32_t* __restri
     }
     __syncthreads();
     if (b < NB)
-        for (int e = lane_id(); e < E; e += WAVE) hist[(size_t)e * NB + b] = my[e];
+        for (int e = lane_id(); e < E; e += WAVE) hist[(size_t)b * E + e] = my[e];
 }
 
 __device__ __forceinline__ int wave_incl_scan(int v) {
@@ -48,30 +49,13 @@ __device__ __forceinline__ int wave_incl_scan(int v) {
     return v;
 }
 
-// ---- 2. per-expert exclusive scan over blocks (one wave per expert) --------------------------------
-__global__ __launch_bounds__(WAVE) void scan_blocks_kernel(const int32_t* __restrict__ hist, int32_t* __restrict__ base,
-                                                            int32_t* __restrict__ counts, int NB) {
-    const int e = blockIdx.x;
-    int running = 0;
-    for (int c = 0; c < NB; c += WAVE) {
-        const int b = c + lane_id();
-        const int v = b < NB ? hist[(size_t)e * NB + b] : 0;
-        const int inc = wave_incl_scan(v);
-        if (b < NB) base[(size_t)e * NB + b] = running + inc - v;
-        running += __shfl(inc, WAVE - 1, WAVE);
-    }
-    if (lane_id() == 0) counts[e] = running;
-}
-
-// ---- 3. expert prefix -> all count/offset outputs (one wave) ---------------------------------------
-// ONE_WAVE = false: every wave of the calling block runs this with the same inputs and writes the same values (es is
-// shared; the barrier inside is a block barrier that all of them reach).  ONE_WAVE = true: a single wave runs it, whatever
-// else the block holds, and the hand-over through es is a wave-local one (no block barrier in divergent control flow).
-template <bool ONE_WAVE>
-__device__ __forceinline__ void offsets_body(const int32_t* counts, int E, int W, int32_t* es /*[E+1], LDS*/,
-                                             int32_t* expert_start /*[E+1]*/, int32_t* __restrict__ send_counts,
-                                             int32_t* __restrict__ expert_offs, int32_t* __restrict__ dst_sizes,
-                                             int32_t* __restrict__ dst_offsets, int32_t* __restrict__ caps) {
+// ---- 2. expert prefix -> all count/offset outputs (one wave) ---------------------------------------
+// A single wave runs it, whatever else its block holds; the lanes hand over through es in LDS.  es[e] = rows of the experts
+// before e; with `write` the results also go to memory.
+__device__ __forceinline__ void offsets_body(const int32_t* counts /*LDS*/, int E, int W, int32_t* es /*[E+1], LDS*/, bool write,
+                                             int32_t* __restrict__ send_counts, int32_t* __restrict__ expert_offs,
+                                             int32_t* __restrict__ dst_sizes, int32_t* __restrict__ dst_offsets,
+                                             int32_t* __restrict__ caps) {
     const int lane = lane_id();
     const int per = (E + WAVE - 1) / WAVE;
     const int lo = min(lane * per, E), hi = min(lo + per, E);
@@ -81,18 +65,14 @@ __device__ __forceinline__ void offsets_body(const int32_t* counts, int E, int W
     int run = incl - sum;
     for (int e = lo; e < hi; ++e) { es[e] = run; run += counts[e]; }
     if (lane == WAVE - 1) es[E] = incl;
+    if (!write) return;
 #pragma unroll
     for (int off = WAVE / 2; off >= 1; off >>= 1) cmax = max(cmax, __shfl_xor(cmax, off, WAVE));
-    if constexpr (ONE_WAVE) {
-        // the lanes' LDS writes above are read by other lanes of the same wave below
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    } else {
-        __syncthreads();
-    }
+    // the lanes' LDS writes above are read by other lanes of the same wave below
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     const int E_l = E / W;
-    for (int e = lane; e <= E; e += WAVE) expert_start[e] = es[e];
     for (int e = lane; e < E; e += WAVE) {
         send_counts[e] = counts[e];
         expert_offs[e] = es[e] - es[(e / E_l) * E_l];
@@ -109,122 +89,89 @@ __device__ __forceinline__ void offsets_body(const int32_t* counts, int E, int W
     if (lane == 0) { caps[0] = max(mmax, 1); caps[1] = max(cmax, 1); }
 }
 
-__global__ __launch_bounds__(WAVE) void offsets_kernel(const int32_t* __restrict__ counts, int E, int W,
-                                                        int32_t* __restrict__ expert_start /*[E+1]*/,
-                                                        int32_t* __restrict__ send_counts, int32_t* __restrict__ expert_offs,
-                                                        int32_t* __restrict__ dst_sizes, int32_t* __restrict__ dst_offsets,
-                                                        int32_t* __restrict__ caps) {
-    __shared__ int32_t es[MOE_MAX_EXPERTS + 1];
-    offsets_body<true>(counts, E, W, es, expert_start, send_counts, expert_offs, dst_sizes, dst_offsets, caps);
-}
-
-// Steps 2 and 3 in one launch when the histogram is small enough for one workgroup (every wave scans the experts
-// w, w + 16, ...; then one wave derives the offsets): a launch saved on a stage that is all launches.
-constexpr int SCAN1_MAXCELLS = 1 << 16;
-__global__ __launch_bounds__(1024) void scan_offsets_kernel(const int32_t* __restrict__ hist, int32_t* __restrict__ base,
-                                                             int32_t* __restrict__ counts, int NB, int E, int W,
-                                                             int32_t* __restrict__ expert_start, int32_t* __restrict__ send_counts,
-                                                             int32_t* __restrict__ expert_offs, int32_t* __restrict__ dst_sizes,
-                                                             int32_t* __restrict__ dst_offsets, int32_t* __restrict__ caps) {
-    __shared__ int32_t es[MOE_MAX_EXPERTS + 1];
-    __shared__ int32_t s_counts[MOE_MAX_EXPERTS];
-    const int wave = threadIdx.x / WAVE, nw = blockDim.x / WAVE;
-    for (int e = wave; e < E; e += nw) {
-        int running = 0;
-        for (int c = 0; c < NB; c += WAVE) {
-            const int b = c + lane_id();
-            const int v = b < NB ? hist[(size_t)e * NB + b] : 0;
-            const int inc = wave_incl_scan(v);
-            if (b < NB) base[(size_t)e * NB + b] = running + inc - v;
-            running += __shfl(inc, WAVE - 1, WAVE);
+// ---- 3. stable positions.  A workgroup of 16 waves ranks RBLK consecutive blocks of 64 tokens, 16 / RBLK waves to a block, each with
+// every (16 / RBLK)-th of a token's slots: the waves OR their lane bits into a 64-bit mask per block and expert in LDS (a token holds
+// an expert at most once), and the rank of a slot inside its expert is the rows of the expert in earlier workgroups' blocks +
+// the popcounts of the earlier blocks' masks + the popcount of its own mask below the lane.
+// What the earlier blocks hold every workgroup sums up for itself from the histogram (NB x E words from L2: 8 KB for 16384 tokens
+// and 8 experts, 256 KB for 16384 and 256, in 16-byte loads where E allows them), and the offsets with it: no scan launch between the
+// two (it took 5 to 22 us on its own, one workgroup walking its experts' rows one after the other).  Four blocks to a workgroup:
+// with 16 the popcounts of up to 15 masks per slot and four workgroups in all took 22 us for 4096 tokens x 8 of 256, so 9.
+// (scan and rank took 22 us as launches of their own.)
+// ONE = true (up to 1024 tokens): a single workgroup holds all 16 blocks, counts for itself and is the only launch.
+constexpr int RANK_WAVES = 16;
+template <bool ONE>
+constexpr int rank_blocks() { return ONE ? 16 : 4; }
+template <bool ONE>
+__global__ __launch_bounds__(RANK_WAVES * WAVE) void rank_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict__ hist, int T,
+                                                                  int k, int E, int W, int NB, int32_t* __restrict__ send_counts,
+                                                                  int32_t* __restrict__ expert_offs, int32_t* __restrict__ dst_sizes,
+                                                                  int32_t* __restrict__ dst_offsets, int32_t* __restrict__ caps,
+                                                                  int32_t* __restrict__ pos, int32_t* __restrict__ row_token) {
+    constexpr int RBLK = rank_blocks<ONE>(), PARTS = RANK_WAVES / RBLK, SLOTS = MOE_MAX_TOPK / PARTS;
+    extern __shared__ unsigned long long masks[];  // [RBLK][E]
+    __shared__ int32_t tot[MOE_MAX_EXPERTS], pre[MOE_MAX_EXPERTS], es[MOE_MAX_EXPERTS + 1];
+    const int tid = threadIdx.x, wave = tid / WAVE, lane = lane_id(), blk = wave / PARTS, part = wave % PARTS;
+    const int b0 = blockIdx.x * RBLK, t = (b0 + blk) * CB + lane;
+    const bool live = b0 + blk < NB && t < T;
+    int mine[SLOTS];
+#pragma unroll
+    for (int j = 0; j < SLOTS; ++j) mine[j] = (live && j * PARTS + part < k) ? idx[(size_t)t * k + j * PARTS + part] : -1;
+    for (int e = tid; e < E; e += blockDim.x) tot[e] = pre[e] = 0;
+    for (int i = tid; i < RBLK * E; i += blockDim.x) masks[i] = 0ull;
+    __syncthreads();
+    unsigned long long* my = masks + blk * E;
+#pragma unroll
+    for (int j = 0; j < SLOTS; ++j)
+        if ((unsigned)mine[j] < (unsigned)E) {
+            atomicOr(&my[mine[j]], 1ull << lane);
+            if constexpr (ONE) atomicAdd(&tot[mine[j]], 1);
         }
-        if (lane_id() == 0) { counts[e] = running; s_counts[e] = running; }
+    if constexpr (!ONE) {
+        // column sums of the histogram: thread = (V experts, slice of the blocks)
+        auto sums = [&](auto vec) {
+            constexpr int V = decltype(vec)::value;
+            const int cols = E / V, slices = blockDim.x / cols, c = tid % cols, sl = tid / cols;
+            if (sl >= slices) return;
+            int all[V] = {}, before[V] = {};
+#pragma unroll 8
+            for (int b = sl; b < NB; b += slices) {
+                int v[V];
+                if constexpr (V == 4) {
+                    const int4 q = reinterpret_cast<const int4*>(hist + (size_t)b * E)[c];
+                    v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+                } else {
+                    v[0] = hist[(size_t)b * E + c];
+                }
+#pragma unroll
+                for (int i = 0; i < V; ++i) {
+                    all[i] += v[i];
+                    before[i] += b < b0 ? v[i] : 0;
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < V; ++i) {
+                atomicAdd(&tot[c * V + i], all[i]);
+                atomicAdd(&pre[c * V + i], before[i]);
+            }
+        };
+        if (E % 4 == 0) sums(std::integral_constant<int, 4>{});
+        else sums(std::integral_constant<int, 1>{});
     }
     __syncthreads();
-    if (wave == 0) offsets_body<true>(s_counts, E, W, es, expert_start, send_counts, expert_offs, dst_sizes, dst_offsets, caps);
-}
-
-// ---- 4. stable positions: one wave per 64-token block ----------------------------------------------
-// One wave ranks the slots of token block b: the rank of a slot among the block's slots of the same expert is the
-// number of lower lanes that hold that expert (a token holds an expert at most once), read off a 64-bit lane
-// mask per expert that the wave builds in LDS with one atomic OR per slot.  Called by every thread of a block
-// (it contains block barriers); waves without a block pass active = false.
-__device__ __forceinline__ void rank_block(const int32_t* __restrict__ idx, const int32_t* base, const int32_t* expert_start,
-                                           int32_t* __restrict__ pos, int32_t* __restrict__ row_token, int T, int k, int E,
-                                           int NB, int b, bool active, unsigned long long* mask /*[E], LDS, per wave*/) {
-    const int lane = lane_id();
-    const int t = b * CB + lane;
-    const bool live = active && t < T;
-    int mine[MOE_MAX_TOPK];
-#pragma unroll
-    for (int j = 0; j < MOE_MAX_TOPK; ++j) mine[j] = (live && j < k) ? idx[(size_t)t * k + j] : -1;
-    if (active)
-        for (int e = lane; e < E; e += WAVE) mask[e] = 0ull;
+    if (wave == 0) offsets_body(tot, E, W, es, blockIdx.x == 0, send_counts, expert_offs, dst_sizes, dst_offsets, caps);
     __syncthreads();
+    const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (WAVE - lane));
 #pragma unroll
-    for (int j = 0; j < MOE_MAX_TOPK; ++j)
-        if ((unsigned)mine[j] < (unsigned)E) atomicOr(&mask[mine[j]], 1ull << lane);
-    __syncthreads();
-    const unsigned long long lt_mask = (lane == 0) ? 0ull : (~0ull >> (WAVE - lane));
-#pragma unroll
-    for (int j = 0; j < MOE_MAX_TOPK; ++j) {
+    for (int j = 0; j < SLOTS; ++j) {
         const int e = mine[j];
         if ((unsigned)e < (unsigned)E) {
-            const int p = expert_start[e] + base[(size_t)e * NB + b] + __popcll(mask[e] & lt_mask);
-            pos[(size_t)t * k + j] = p;
+            int p = es[e] + pre[e] + __popcll(my[e] & below);
+            for (int w = 0; w < blk; ++w) p += __popcll(masks[w * E + e]);
+            pos[(size_t)t * k + j * PARTS + part] = p;
             row_token[p] = t;
         }
     }
-    __syncthreads();  // the masks are reused by the caller's next block
-}
-
-__global__ __launch_bounds__(256) void rank_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict__ base,
-                                                    const int32_t* __restrict__ expert_start, int32_t* __restrict__ pos,
-                                                    int32_t* __restrict__ row_token, int T, int k, int E, int NB) {
-    __shared__ unsigned long long masks[4][MOE_MAX_EXPERTS];
-    const int wave = threadIdx.x / WAVE;
-    const int b = blockIdx.x * 4 + wave;
-    rank_block(idx, base, expert_start, pos, row_token, T, k, E, NB, b, b < NB, masks[wave]);
-}
-
-// ---- the four steps above in one block, for few tokens (NB <= CS_MAXNB blocks of 64): launch latency is all that
-// such a count costs, so one launch instead of four.  Same arithmetic, tables in LDS instead of the workspace.
-constexpr int CS_MAXNB = 16;
-constexpr int CS_MAXCELLS = 4096;  // E * NB histogram cells held in LDS (twice: counts and prefixes)
-
-__global__ __launch_bounds__(256) void count_small_kernel(const int32_t* __restrict__ idx, int T, int k, int E, int W, int NB,
-                                                           int32_t* __restrict__ send_counts, int32_t* __restrict__ expert_offs,
-                                                           int32_t* __restrict__ dst_sizes, int32_t* __restrict__ dst_offsets,
-                                                           int32_t* __restrict__ caps, int32_t* __restrict__ pos,
-                                                           int32_t* __restrict__ row_token) {
-    __shared__ int32_t hist[CS_MAXCELLS];   // [e][b]
-    __shared__ int32_t base[CS_MAXCELLS];   // [e][b] rows of e in earlier blocks
-    __shared__ int32_t counts[MOE_MAX_EXPERTS];
-    __shared__ int32_t es[MOE_MAX_EXPERTS + 1];
-    __shared__ int32_t expert_start[MOE_MAX_EXPERTS + 1];
-    __shared__ unsigned long long masks[4][MOE_MAX_EXPERTS];
-    const int wave = threadIdx.x / WAVE, lane = lane_id();
-    for (int i = threadIdx.x; i < E * NB; i += blockDim.x) hist[i] = 0;
-    __syncthreads();
-    for (int b = wave; b < NB; b += 4) {
-        const int t = b * CB + lane;
-        if (t < T)
-            for (int j = 0; j < k; ++j) {
-                const int e = idx[(size_t)t * k + j];
-                if ((unsigned)e < (unsigned)E) atomicAdd(&hist[e * NB + b], 1);
-            }
-    }
-    __syncthreads();
-    for (int e = threadIdx.x; e < E; e += blockDim.x) {
-        int run = 0;
-        for (int b = 0; b < NB; ++b) { base[e * NB + b] = run; run += hist[e * NB + b]; }
-        counts[e] = run;
-    }
-    __syncthreads();
-    offsets_body<false>(counts, E, W, es, expert_start, send_counts, expert_offs, dst_sizes, dst_offsets, caps);
-    __syncthreads();
-    for (int b0 = 0; b0 < NB; b0 += 4)  // (uniform trip count: rank_block holds block barriers)
-        rank_block(idx, base, expert_start, pos, row_token, T, k, E, NB, b0 + wave, b0 + wave < NB, masks[wave]);
 }
 
 // ---- small integer helpers --------------------------------------------------------------------------
@@ -241,47 +188,6 @@ __global__ void max_floor1_kernel(const int32_t* __restrict__ v, int n, int32_t*
     if (threadIdx.x == 0) out[0] = red[0];
 }
 
-// Tables derived from recv_counts [W,E_l] (one block):
-//   src_off[s*E_l+e] = exclusive prefix over e of recv_counts[s,:]   (row inside slot s)
-//   row_off[e*W+s]   = exclusive prefix over flattened (e,s) of recv_counts[s,e]  (+ total at [E_l*W])
-//   flat_off[s*E_l+e]= exclusive prefix over flattened (s,e)         (row in a padding-free flat payload)
-__global__ __launch_bounds__(WAVE) void recv_tables_kernel(const int32_t* __restrict__ rc, int W, int E_l,
-                                                            int32_t* __restrict__ src_off, int32_t* __restrict__ row_off,
-                                                            int32_t* __restrict__ flat_off, int32_t* __restrict__ pca,
-                                                            int32_t* __restrict__ expert_cnt) {
-    const int n = W * E_l;
-    const int lane = lane_id();
-    const int per = (n + WAVE - 1) / WAVE;
-    const int lo = min(lane * per, n), hi = min(lo + per, n);
-    // (e,s)-major prefix
-    int sum = 0;
-    for (int i = lo; i < hi; ++i) sum += rc[(i % W) * E_l + (i / W)];
-    int incl = wave_incl_scan(sum);
-    int run = incl - sum;
-    for (int i = lo; i < hi; ++i) { row_off[i] = run; run += rc[(i % W) * E_l + (i / W)]; }
-    if (lane == WAVE - 1) row_off[n] = incl;
-    // (s,e)-major prefix
-    sum = 0;
-    for (int i = lo; i < hi; ++i) sum += rc[i];
-    incl = wave_incl_scan(sum);
-    run = incl - sum;
-    for (int i = lo; i < hi; ++i) { flat_off[i] = run; run += rc[i]; }
-    if (lane == WAVE - 1) flat_off[n] = incl;
-    // per-source prefix over experts, pca transpose, per-expert totals
-    for (int s = lane; s < W; s += WAVE) {
-        int r = 0;
-        for (int e = 0; e < E_l; ++e) { src_off[s * E_l + e] = r; r += rc[s * E_l + e]; }
-    }
-    for (int i = lane; i < n; i += WAVE) {
-        if (pca) pca[i] = rc[(i % W) * E_l + (i / W)];
-    }
-    if (expert_cnt)
-        for (int e = lane; e < E_l; e += WAVE) {
-            int c = 0;
-            for (int s = 0; s < W; ++s) c += rc[s * E_l + e];
-            expert_cnt[e] = c;
-        }
-}
 
 
 // expert_offs[d,e] = exclusive prefix over e of counts[d,:]; dst_sizes / dst_offsets over d (one wave)
@@ -321,10 +227,63 @@ struct RowSource {
     int mode;
     const int32_t* map;                                   // SRC_MAP / SRC_PACK: row_token
     const int32_t *dst_sizes, *dst_offsets;               // SRC_PACK
-    const int32_t *rc, *src_off, *row_off, *flat_off;     // recv-driven modes
+    const int32_t *rc, *src_off, *row_off, *flat_off;     // recv-driven modes: tables in LDS (recv_tables)
     int W, E_l, M, CAP;
     int32_t* status;
 };
+
+// What the recv-driven modes derive from recv_counts (W E_l <= MOE_MAX_EXPERTS entries; counts are read as
+// counts[s * pitch_s + e * pitch_e], so a matrix or its transpose will do):
+//   rc[s*E_l+e]      the counts themselves
+//   src_off[s*E_l+e] exclusive prefix over e of rc[s,:]                  (row inside slot s)
+//   row_off[e*W+s]   exclusive prefix over flattened (e,s)               (expert-major row; total at [E_l*W])
+//   flat_off[s*E_l+e] exclusive prefix over flattened (s,e)              (row in a padding-free flat payload)
+// Every workgroup of the copy makes its own set in LDS, one table to a wave (2 us with 256 counts, once per workgroup of a
+// grid that stays on the chip), instead of a launch of one wave in front of the copy (4.8 us in a graph, 5 to 15 at 256 counts).
+struct RecvCounts {
+    const int32_t* counts;
+    int pitch_s, pitch_e;
+    int32_t *pca, *expert_cnt;  // or NULL: counts[e][s], rows per expert (left by the first workgroup)
+};
+struct RecvTables {
+    int32_t rc[MOE_MAX_EXPERTS], src_off[MOE_MAX_EXPERTS], row_off[MOE_MAX_EXPERTS + 1], flat_off[MOE_MAX_EXPERTS];
+};
+__device__ __forceinline__ void recv_tables(RecvTables& t, const RecvCounts& q, int W, int E_l) {
+    const int n = W * E_l, wave = threadIdx.x / WAVE, lane = lane_id();
+    for (int i = threadIdx.x; i < n; i += blockDim.x) {
+        const int s = i / E_l, e = i % E_l, c = q.counts[(size_t)s * q.pitch_s + (size_t)e * q.pitch_e];
+        t.rc[i] = c;
+        if (q.pca && blockIdx.x == 0) q.pca[e * W + s] = c;
+    }
+    __syncthreads();
+    const int per = (n + WAVE - 1) / WAVE;
+    const int lo = min(lane * per, n), hi = min(lo + per, n);
+    if (wave == 0) {
+        int sum = 0;
+        for (int i = lo; i < hi; ++i) sum += t.rc[(i % W) * E_l + i / W];
+        const int incl = wave_incl_scan(sum);
+        int run = incl - sum;
+        for (int i = lo; i < hi; ++i) { t.row_off[i] = run; run += t.rc[(i % W) * E_l + i / W]; }
+        if (lane == WAVE - 1) t.row_off[n] = incl;
+    } else if (wave == 1) {
+        int sum = 0;
+        for (int i = lo; i < hi; ++i) sum += t.rc[i];
+        int run = wave_incl_scan(sum) - sum;
+        for (int i = lo; i < hi; ++i) { t.flat_off[i] = run; run += t.rc[i]; }
+    } else if (wave == 2) {
+        for (int s = lane; s < W; s += WAVE) {
+            int r = 0;
+            for (int e = 0; e < E_l; ++e) { t.src_off[s * E_l + e] = r; r += t.rc[s * E_l + e]; }
+        }
+    } else if (wave == 3 && q.expert_cnt && blockIdx.x == 0) {
+        for (int e = lane; e < E_l; e += WAVE) {
+            int c = 0;
+            for (int s = 0; s < W; ++s) c += t.rc[s * E_l + e];
+            q.expert_cnt[e] = c;
+        }
+    }
+    __syncthreads();
+}
 
 // largest i in [0,n) with off[i] <= r (off ascending, off[0] = 0): the whole wave looks at 64 entries
 // at a time and counts them with a ballot.  Equal offsets mark empty segments; the last of a run of
@@ -394,10 +353,17 @@ __device__ __forceinline__ int source_row(const RowSource& a, int r) {
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
-template <int WPB>
+template <int WPB, bool RECV>
 __global__ __launch_bounds__(WPB * WAVE) void gather_rows_kernel(const u32x4* __restrict__ src, u32x4* __restrict__ dst,
-                                                                  const RowSource a, int n_rows,
-                                                                  int row_vec /* 16-byte units per row */) {
+                                                                  const RowSource src_of, int n_rows,
+                                                                  int row_vec /* 16-byte units per row */, const RecvCounts q) {
+    RowSource a = src_of;
+    if constexpr (RECV) {
+        static_assert(WPB == 4, "one wave per table");
+        __shared__ RecvTables tables;
+        recv_tables(tables, q, a.W, a.E_l);
+        a.rc = tables.rc; a.src_off = tables.src_off; a.row_off = tables.row_off; a.flat_off = tables.flat_off;
+    }
     const int wave = threadIdx.x / WAVE, lane = lane_id();
     for (int r = blockIdx.x * WPB + wave; r < n_rows; r += gridDim.x * WPB) {
         const int m = source_row(a, r);
@@ -427,21 +393,29 @@ __global__ __launch_bounds__(WPB * WAVE) void gather_rows_kernel(const u32x4* __
 // routing most of the send buffer is padding).  Same bytes in send_buf as the slot-major gather (SRC_PACK), with x
 // read once instead of k times.
 constexpr int PACK_ZR = 8;
+// Waves per token row of the kernels that give a token to a wave: with few tokens a row is cut into runs of columns (64 vectors at
+// least), so that the chip holds some 2048 waves whatever the token count (24 rows of 14 KB, top-8: pack 12.8 -> 7.7 us, combine
+// 23 -> 5.8 us: a wave alone walks its row by 1 to 8 KB a memory round trip).
+inline int row_parts(int tokens, int row_vec) {
+    return max(1, min(2048 / max(tokens, 1), (row_vec + WAVE - 1) / WAVE));
+}
 template <int WPB>
 __global__ __launch_bounds__(WPB * WAVE) void pack_tokens_kernel(const u32x4* __restrict__ x, u32x4* __restrict__ send,
                                                                   const int32_t* __restrict__ idx, const int32_t* __restrict__ pos,
                                                                   const int32_t* __restrict__ dst_sizes,
                                                                   const int32_t* __restrict__ dst_offsets, int T, int k, int E_l,
                                                                   int W, int M, int row_vec, int32_t* __restrict__ status,
-                                                                  const float* __restrict__ gate, float* __restrict__ send_gate) {
+                                                                  const float* __restrict__ gate, float* __restrict__ send_gate, int parts) {
     // gate / send_gate (both or neither): the slot's top-k gate travels with its row, send_gate[d,m] = gate[t,kk], zero
     // in the padding slots -- for a destination that applies the gate to the expert's result before sending it back
+    // parts: waves per token, each with its own run of columns (see row_parts)
     const int wave = threadIdx.x / WAVE, lane = lane_id();
-    const int n_slots = W * M;
-    const int n_units = T + (n_slots + PACK_ZR - 1) / PACK_ZR;
-    for (int r = blockIdx.x * WPB + wave; r < n_units; r += gridDim.x * WPB) {
-        if (r >= T) {
-            const int s0 = (r - T) * PACK_ZR, s1 = min(s0 + PACK_ZR, n_slots);
+    const int n_slots = W * M, n_tok = T * parts;
+    const int per = ((row_vec + parts - 1) / parts + WAVE - 1) / WAVE * WAVE;
+    const int n_units = n_tok + (n_slots + PACK_ZR - 1) / PACK_ZR;
+    for (int unit = blockIdx.x * WPB + wave; unit < n_units; unit += gridDim.x * WPB) {
+        if (unit >= n_tok) {
+            const int s0 = (unit - n_tok) * PACK_ZR, s1 = min(s0 + PACK_ZR, n_slots);
             int d = s0 / M, m = s0 % M;
             int cnt = dst_sizes[d];
             const u32x4 z = {0u, 0u, 0u, 0u};
@@ -457,6 +431,7 @@ __global__ __launch_bounds__(WPB * WAVE) void pack_tokens_kernel(const u32x4* __
             }
             continue;
         }
+        const int r = unit / parts, c_lo = (unit % parts) * per, c_hi = min(c_lo + per, row_vec);
         // destination rows of the token's k slots (-1: beyond the pair capacity, dropped like the gather drops it)
         int drow[MOE_MAX_TOPK];
 #pragma unroll
@@ -467,23 +442,23 @@ __global__ __launch_bounds__(WPB * WAVE) void pack_tokens_kernel(const u32x4* __
                 const bool d_ok = (unsigned)d < (unsigned)W;  // (an expert id outside [0, W E_l): no slot, and no read of its offset)
                 const int m = pos[(size_t)r * k + j] - dst_offsets[d_ok ? d : 0];
                 if (d_ok && (unsigned)m < (unsigned)M) drow[j] = d * M + m;
-                if (send_gate && drow[j] >= 0 && lane == 0) send_gate[drow[j]] = gate[(size_t)r * k + j];
+                if (send_gate && drow[j] >= 0 && lane == 0 && c_lo == 0) send_gate[drow[j]] = gate[(size_t)r * k + j];
             }
         }
         const u32x4* src = x + (size_t)r * row_vec;
         // eight 16-byte loads in flight per lane (fewer at the end of a row, or when the row is shorter than 8 KB)
-        for (int c = lane; c < row_vec; c += 8 * WAVE) {
+        for (int c = c_lo + lane; c < c_hi; c += 8 * WAVE) {
             u32x4 v[8];
 #pragma unroll
             for (int u = 0; u < 8; ++u)
-                if (c + u * WAVE < row_vec) v[u] = __builtin_nontemporal_load(src + c + u * WAVE);
+                if (c + u * WAVE < c_hi) v[u] = __builtin_nontemporal_load(src + c + u * WAVE);
 #pragma unroll
             for (int j = 0; j < MOE_MAX_TOPK; ++j) {
                 if (j < k && drow[j] >= 0) {
                     u32x4* o = send + (size_t)drow[j] * row_vec + c;
 #pragma unroll
                     for (int u = 0; u < 8; ++u)
-                        if (c + u * WAVE < row_vec) __builtin_nontemporal_store(v[u], o + u * WAVE);
+                        if (c + u * WAVE < c_hi) __builtin_nontemporal_store(v[u], o + u * WAVE);
                 }
             }
         }
@@ -526,12 +501,14 @@ __global__ __launch_bounds__(WPB * WAVE) void combine_kernel(const uint4* __rest
                                                               const int32_t* __restrict__ pos, const float* __restrict__ gate,
                                                               const int32_t* __restrict__ dst_offsets, int T, int k_rt, int E_l,
                                                               int W, int M, int row_vec, uint4* __restrict__ out,
-                                                              int32_t* __restrict__ status) {
+                                                              int32_t* __restrict__ status, int parts) {
     constexpr int N = Vec16<XT>::N;
     constexpr int KMAX = KT ? KT : MOE_MAX_TOPK;
     const int k = KT ? KT : k_rt;
     const int wave = threadIdx.x / WAVE, lane = lane_id();
-    for (int t = blockIdx.x * WPB + wave; t < T; t += gridDim.x * WPB) {
+    const int per = ((row_vec + parts - 1) / parts + WAVE - 1) / WAVE * WAVE;  // columns per wave (see row_parts)
+    for (int unit = blockIdx.x * WPB + wave; unit < T * parts; unit += gridDim.x * WPB) {
+        const int t = unit / parts, c_lo = (unit % parts) * per, c_hi = min(c_lo + per, row_vec);
         // a slot whose destination or row lies outside the [W,M] layout was dropped by the pack (pair capacity
         // exceeded) and has no returned row: it is skipped, like the pack skipped it, and the status word is raised
         size_t rows[KMAX];
@@ -551,15 +528,15 @@ __global__ __launch_bounds__(WPB * WAVE) void combine_kernel(const uint4* __rest
             }
         }
         // U columns per lane and pass, so that sixteen 16-byte row reads are in flight per lane whatever k is
-        constexpr int U = KT ? (KT >= 16 ? 1 : 16 / KT) : 1;
-        for (int c0 = lane; c0 < row_vec; c0 += U * WAVE) {
+        constexpr int U = KT == 0 || KT >= 16 ? 1 : 16 / (KT ? KT : 1);
+        for (int c0 = c_lo + lane; c0 < c_hi; c0 += U * WAVE) {
             uint4 v[U][KMAX];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const int c = c0 + u * WAVE;
 #pragma unroll
                 for (int j = 0; j < KMAX; ++j)
-                    if (j < k && have[j] && c < row_vec) {
+                    if (j < k && have[j] && c < c_hi) {
                         // every returned row is read once: no cache retention wanted
                         const u32x4 raw = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(ret + rows[j] + c));
                         v[u][j] = make_uint4(raw.x, raw.y, raw.z, raw.w);
@@ -568,7 +545,7 @@ __global__ __launch_bounds__(WPB * WAVE) void combine_kernel(const uint4* __rest
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const int c = c0 + u * WAVE;
-                if (c >= row_vec) break;
+                if (c >= c_hi) break;
                 float acc[N];
 #pragma unroll
                 for (int i = 0; i < N; ++i) acc[i] = 0.f;
@@ -594,62 +571,108 @@ __global__ __launch_bounds__(WPB * WAVE) void combine_kernel(const uint4* __rest
 //   d ret[slot(t,kk)] = gate[t,kk] * d out[t]        (every slot belongs to one (t,kk): a scatter, like the pack)
 //   d gate[t,kk]      = < d out[t], ret[slot(t,kk)] > (fp32 sum over the row: per-lane partial sums in column order, then
 //                                                     a butterfly over the lanes -- reproducible from call to call)
-// Rows [0, T) of the launch are tokens (one wave each); rows [T, T + W*M) are the slots of d ret, which only get zeros when
-// they are padding (no (t,kk) maps there) -- as in pack_tokens_kernel.  Dropped slots (outside [W,M]) get no gradient.
-template <typename XT, int WPB>
+// Units [0, T) of the launch are tokens (one wave each); the units after them are runs of PACK_ZR slots of d ret, which only get
+// zeros when they are padding (no (t,kk) maps there) -- as in pack_tokens_kernel.  Dropped slots (outside [W,M]) get no
+// gradient.  A pass takes U columns of the token's d out and of its k slot rows together (some sixteen 16-byte loads in flight
+// per lane): d out is read once, not k times (4096 tokens x 8 rows of 14 KB: 299 -> 266 us, 4.4 TB/s with the padding).
+// dst_sizes == NULL: a destination's rows end where the next one's start (n_routed rows in all).
+template <typename XT, int KT, int WPB>
 __global__ __launch_bounds__(WPB * WAVE) void combine_backward_kernel(const uint4* __restrict__ dout, const uint4* __restrict__ ret,
                                                                        const int32_t* __restrict__ idx, const int32_t* __restrict__ pos,
                                                                        const float* __restrict__ gate,
                                                                        const int32_t* __restrict__ dst_sizes,
-                                                                       const int32_t* __restrict__ dst_offsets, int T, int k, int E_l,
+                                                                       const int32_t* __restrict__ dst_offsets, int T, int k_rt, int E_l,
                                                                        int W, int M, int row_vec, uint4* __restrict__ dret,
                                                                        float* __restrict__ dgate) {
     constexpr int N = Vec16<XT>::N;
+    constexpr int KMAX = KT ? KT : MOE_MAX_TOPK;
+    constexpr int U = KT ? (KT >= 8 ? 2 : KT >= 4 ? 4 : 8) : 1;
+    const int k = KT ? KT : k_rt;
     const int wave = threadIdx.x / WAVE, lane = lane_id();
-    const int n_rows = T + W * M;
-    for (int r = blockIdx.x * WPB + wave; r < n_rows; r += gridDim.x * WPB) {
+    const int n_slots = W * M, n_units = T + (n_slots + PACK_ZR - 1) / PACK_ZR;
+    for (int r = blockIdx.x * WPB + wave; r < n_units; r += gridDim.x * WPB) {
         if (r >= T) {
-            const int d = (r - T) / M, m = (r - T) % M;
-            if (m < dst_sizes[d]) continue;
-            uint4* o = dret + (size_t)(r - T) * row_vec;
-            for (int c = lane; c < row_vec; c += WAVE) o[c] = make_uint4(0, 0, 0, 0);
+            const int s0 = (r - T) * PACK_ZR, s1 = min(s0 + PACK_ZR, n_slots);
+            int d = s0 / M, m = s0 % M;
+            auto size_of = [&](int q) { return dst_sizes ? dst_sizes[q] : (q + 1 < W ? dst_offsets[q + 1] : T * k) - dst_offsets[q]; };
+            int cnt = size_of(d);
+            for (int sl = s0; sl < s1; ++sl) {
+                if (m >= cnt) {
+                    uint4* o = dret + (size_t)sl * row_vec;
+                    for (int c = lane; c < row_vec; c += WAVE) o[c] = make_uint4(0, 0, 0, 0);
+                }
+                if (++m == M && sl + 1 < s1) { m = 0; cnt = size_of(++d); }
+            }
             continue;
         }
         const uint4* drow = dout + (size_t)r * row_vec;
-        for (int j = 0; j < k; ++j) {
-            const int d = idx[(size_t)r * k + j] / E_l;
-            const bool d_ok = (unsigned)d < (unsigned)W;
-            const int m = pos[(size_t)r * k + j] - dst_offsets[d_ok ? d : 0];
-            const bool have = d_ok && (unsigned)m < (unsigned)M;
-            const float g = gate[(size_t)r * k + j];
-            float dot = 0.f;
-            if (have) {
-                const size_t slot = ((size_t)d * M + m) * row_vec;
-                for (int c = lane; c < row_vec; c += WAVE) {
-                    float dv[N], rv[N], ov[N];
-                    Vec16<XT>::unpack(drow[c], dv);
-                    Vec16<XT>::unpack(ret[slot + c], rv);
+        size_t slot[KMAX];
+        float g[KMAX], dot[KMAX];
+        bool have[KMAX];
 #pragma unroll
-                    for (int i = 0; i < N; ++i) {
-                        dot = __fadd_rn(dot, __fmul_rn(dv[i], rv[i]));
-                        ov[i] = __fmul_rn(g, dv[i]);
-                    }
-                    dret[slot + c] = Vec16<XT>::pack(ov);
-                }
+        for (int j = 0; j < KMAX; ++j) {
+            have[j] = false;
+            dot[j] = 0.f;
+            if (j < k) {
+                const int d = idx[(size_t)r * k + j] / E_l;
+                const bool d_ok = (unsigned)d < (unsigned)W;
+                const int m = pos[(size_t)r * k + j] - dst_offsets[d_ok ? d : 0];
+                have[j] = d_ok && (unsigned)m < (unsigned)M;
+                slot[j] = have[j] ? ((size_t)d * M + m) * row_vec : 0;
+                g[j] = gate[(size_t)r * k + j];
             }
-#pragma unroll
-            for (int off = WAVE / 2; off >= 1; off >>= 1) dot = __fadd_rn(dot, __shfl_xor(dot, off, WAVE));
-            if (lane == 0) dgate[(size_t)r * k + j] = dot;
         }
+        for (int c0 = lane; c0 < row_vec; c0 += U * WAVE) {
+            uint4 dv4[U], rv4[U][KMAX];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (c0 + u * WAVE < row_vec) {
+                    dv4[u] = drow[c0 + u * WAVE];
+#pragma unroll
+                    for (int j = 0; j < KMAX; ++j)
+                        if (j < k && have[j]) {
+                            const u32x4 raw = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(ret + slot[j] + c0 + u * WAVE));
+                            rv4[u][j] = make_uint4(raw.x, raw.y, raw.z, raw.w);
+                        }
+                }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (c0 + u * WAVE >= row_vec) break;
+                float dv[N];
+                Vec16<XT>::unpack(dv4[u], dv);
+#pragma unroll
+                for (int j = 0; j < KMAX; ++j)
+                    if (j < k && have[j]) {
+                        float rv[N], ov[N];
+                        Vec16<XT>::unpack(rv4[u][j], rv);
+#pragma unroll
+                        for (int i = 0; i < N; ++i) {
+                            dot[j] = __fadd_rn(dot[j], __fmul_rn(dv[i], rv[i]));
+                            ov[i] = __fmul_rn(g[j], dv[i]);
+                        }
+                        const uint4 o = Vec16<XT>::pack(ov);
+                        const u32x4 o4 = {o.x, o.y, o.z, o.w};
+                        __builtin_nontemporal_store(o4, reinterpret_cast<u32x4*>(dret + slot[j] + c0 + u * WAVE));
+                    }
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < KMAX; ++j)
+            if (j < k) {
+#pragma unroll
+                for (int off = WAVE / 2; off >= 1; off >>= 1) dot[j] = __fadd_rn(dot[j], __shfl_xor(dot[j], off, WAVE));
+                if (lane == 0) dgate[(size_t)r * k + j] = dot[j];
+            }
     }
 }
 
 template <typename XT>
 int launch_combine(const void* ret, const int32_t* idx, const int32_t* pos, const float* gate, const int32_t* dst_offsets, int T,
                    int k, int E_l, int W, int M, int row_vec, void* out, int32_t* status, hipStream_t s) {
-    const int blocks = min(ceil_div(T, 4), 65535 * 8);
+    const int parts = row_parts(T, row_vec);
+    const int blocks = min(ceil_div(T * parts, 4), 65535 * 8);
 #define MOE_COMBINE(KT) \
-    combine_kernel<XT, KT, 4><<<blocks, 4 * WAVE, 0, s>>>((const uint4*)ret, idx, pos, gate, dst_offsets, T, k, E_l, W, M, row_vec, (uint4*)out, status)
+    combine_kernel<XT, KT, 4><<<blocks, 4 * WAVE, 0, s>>>((const uint4*)ret, idx, pos, gate, dst_offsets, T, k, E_l, W, M, row_vec, (uint4*)out, status, parts)
     switch (k) {
         case 1: MOE_COMBINE(1); break;
         case 2: MOE_COMBINE(2); break;
@@ -664,8 +687,39 @@ int launch_combine(const void* ret, const int32_t* idx, const int32_t* pos, cons
 int gather_rows(const void* src, void* dst, const RowSource& a, int n_rows, int row_bytes, hipStream_t s) {
     if (n_rows == 0) return MOE_OK;
     const int blocks = min(ceil_div(n_rows, 4), 65535 * 8);
-    gather_rows_kernel<4><<<blocks, 4 * WAVE, 0, s>>>((const u32x4*)src, (u32x4*)dst, a, n_rows, row_bytes / 16);
+    gather_rows_kernel<4, false><<<blocks, 4 * WAVE, 0, s>>>((const u32x4*)src, (u32x4*)dst, a, n_rows, row_bytes / 16, RecvCounts{});
     return moe_check_launch("gather_rows");
+}
+
+// rows [size_s, M) of every slot s of a [W,M,row] buffer <- 0, size_s = sum over e of rc[s,e]; one wave per run of
+// PACK_ZR consecutive rows (the slot's size is summed once per run, or twice when the run crosses into the next slot)
+__device__ __forceinline__ int slot_size(const int32_t* __restrict__ rc, int s, int E_l, int lane) {
+    int size = 0;
+    for (int e = lane; e < E_l; e += WAVE) size += rc[s * E_l + e];
+#pragma unroll
+    for (int off = WAVE / 2; off >= 1; off >>= 1) size += __shfl_xor(size, off, WAVE);
+    return size;
+}
+__device__ __forceinline__ void zero_padding_rows(u32x4* __restrict__ buf, const int32_t* __restrict__ rc, int W, int E_l, int M,
+                                                  int row_vecs, int block) {
+    const int wave = threadIdx.x / WAVE, lane = lane_id();
+    const int r0 = (block * (blockDim.x / WAVE) + wave) * PACK_ZR, r1 = min(r0 + PACK_ZR, W * M);
+    if (r0 >= r1) return;
+    int s = r0 / M, m = r0 % M;
+    int size = slot_size(rc, s, E_l, lane);
+    const u32x4 z = {0u, 0u, 0u, 0u};
+    for (int r = r0; r < r1; ++r) {
+        if (m >= size) {
+            u32x4* row = buf + (size_t)r * row_vecs;
+            for (int c = lane; c < row_vecs; c += WAVE) __builtin_nontemporal_store(z, row + c);
+        }
+        if (++m == M && r + 1 < r1) { m = 0; size = slot_size(rc, ++s, E_l, lane); }
+    }
+}
+
+__global__ __launch_bounds__(256) void zero_padding_rows_kernel(u32x4* __restrict__ buf, const int32_t* __restrict__ rc, int W, int E_l,
+                                                                 int M, int row_vecs) {
+    zero_padding_rows(buf, rc, W, E_l, M, row_vecs, blockIdx.x);
 }
 
 // Expert-major row r of the receive side -> row of the [W,M,H] buffer that holds it (one thread per row, binary search in
@@ -678,10 +732,18 @@ int gather_rows(const void* src, void* dst, const RowSource& a, int n_rows, int 
 // reorder_flat_to_token_buf of the reference reads, baseline.py:204-218): the row of (e, s, j) is the exclusive prefix of the
 // counts over flattened (s, e) plus j, and no row can have been dropped.
 // recv_gate / row_gate (both or neither): the gates that arrived with the rows, [rows of the receive buffer], gathered
-// into expert-major order for the GEMM that applies them (0 for rows without a source).
+// into expert-major order for the GEMM that applies them (0 for rows without a source).  recv_scale / row_scale likewise: the
+// fp8 row scales (rows without a source take that of row 0, whose codes the GEMM reads for them).
+// zbuf (or NULL): the blocks from map_blocks on zero the padding rows of that [W,M,row_vecs] buffer, which depend on the same counts.
 __global__ __launch_bounds__(256) void row_map_from_counts_kernel(const int32_t* __restrict__ rc, int W, int E_l, int M, int n_rows,
                                                                    int32_t* __restrict__ map, int32_t* __restrict__ expert_cnt,
-                                                                   const float* __restrict__ recv_gate, float* __restrict__ row_gate) {
+                                                                   const float* __restrict__ recv_gate, float* __restrict__ row_gate,
+                                                                   const float* __restrict__ recv_scale, float* __restrict__ row_scale,
+                                                                   u32x4* __restrict__ zbuf, int row_vecs, int map_blocks) {
+    if ((int)blockIdx.x >= map_blocks) {
+        zero_padding_rows(zbuf, rc, W, E_l, M, row_vecs, blockIdx.x - map_blocks);
+        return;
+    }
     __shared__ int32_t s_row_off[MOE_MAX_EXPERTS + 1];
     __shared__ int32_t s_src_off[MOE_MAX_EXPERTS];
     const int n = W * E_l;
@@ -721,6 +783,7 @@ __global__ __launch_bounds__(256) void row_map_from_counts_kernel(const int32_t*
     if (r >= s_row_off[n]) {
         map[r] = 0;
         if (row_gate) row_gate[r] = 0.f;
+        if (row_scale) row_scale[r] = recv_scale[0];
         return;
     }
     int lo = 0, hi = n;  // s_row_off[0] = 0 <= r; the last of a run of equal offsets owns the row
@@ -733,36 +796,8 @@ __global__ __launch_bounds__(256) void row_map_from_counts_kernel(const int32_t*
     const int row = flat ? m : (m < M ? sr * M + m : -1);
     map[r] = row;
     if (row_gate) row_gate[r] = row >= 0 ? recv_gate[row] : 0.f;
+    if (row_scale) row_scale[r] = recv_scale[max(row, 0)];
 }
-
-// rows [size_s, M) of every slot s of a [W,M,row] buffer <- 0, size_s = sum over e of rc[s,e]; one wave per run of
-// PACK_ZR consecutive rows (the slot's size is summed once per run, or twice when the run crosses into the next slot)
-__device__ __forceinline__ int slot_size(const int32_t* __restrict__ rc, int s, int E_l, int lane) {
-    int size = 0;
-    for (int e = lane; e < E_l; e += WAVE) size += rc[s * E_l + e];
-#pragma unroll
-    for (int off = WAVE / 2; off >= 1; off >>= 1) size += __shfl_xor(size, off, WAVE);
-    return size;
-}
-__global__ __launch_bounds__(256) void zero_padding_rows_kernel(u32x4* __restrict__ buf, const int32_t* __restrict__ rc, int W,
-                                                                 int E_l, int M, int row_vecs) {
-    const int wave = threadIdx.x / WAVE, lane = lane_id();
-    const int r0 = (blockIdx.x * (blockDim.x / WAVE) + wave) * PACK_ZR, r1 = min(r0 + PACK_ZR, W * M);
-    if (r0 >= r1) return;
-    int s = r0 / M, m = r0 % M;
-    int size = slot_size(rc, s, E_l, lane);
-    const u32x4 z = {0u, 0u, 0u, 0u};
-    for (int r = r0; r < r1; ++r) {
-        if (m >= size) {
-            u32x4* row = buf + (size_t)r * row_vecs;
-            for (int c = lane; c < row_vecs; c += WAVE) __builtin_nontemporal_store(z, row + c);
-        }
-        if (++m == M && r + 1 < r1) { m = 0; size = slot_size(rc, ++s, E_l, lane); }
-    }
-}
-
-// map_ws of the recv-driven entry points: three prefix tables plus room for a transposed copy of the counts
-size_t recv_tables_ints(int W, int E_l) { return (size_t)3 * (W * E_l + 1) + (size_t)W * E_l; }
 
 int check_rows(const char* who, int dtype, int H) {
     if (dtype != MOE_F32 && dtype != MOE_BF16) return moe_fail(MOE_ERR_INVALID, "%s: dtype %d", who, dtype);
@@ -776,7 +811,7 @@ int check_rows(const char* who, int dtype, int H) {
 extern "C" size_t moe_count_workspace_bytes(int T, int k, int E) {
     (void)k;
     const size_t NB = (size_t)ceil_div(T > 0 ? T : 1, CB);
-    // hist[E][NB] + base[E][NB] + counts[E] + expert_start[E+1]
+    // hist[NB][E]; the size callers were always asked for (twice that and two rows)
     return sizeof(int32_t) * (2 * (size_t)E * NB + 2 * (size_t)E + 1);
 }
 
@@ -794,23 +829,15 @@ extern "C" int moe_count_and_offsets(const int32_t* topk_idx, int T, int k, int 
                 moe_count_workspace_bytes(T, k, E));
     const int NB = ceil_div(T > 0 ? T : 1, CB);
     int32_t* hist = (int32_t*)ws;
-    int32_t* base = hist + (size_t)E * NB;
-    int32_t* counts = base + (size_t)E * NB;
-    int32_t* expert_start = counts + E;
-    if (T > 0 && NB <= CS_MAXNB && E * NB <= CS_MAXCELLS) {
-        count_small_kernel<<<1, 256, 0, s>>>(topk_idx, T, k, E, W, NB, send_counts, expert_offs, dst_sizes, dst_offsets, caps, pos,
-                                             row_token);
+    auto lds = [&](int blocks) { return (size_t)blocks * E * sizeof(unsigned long long); };
+    if (NB <= rank_blocks<true>()) {  // (few tokens: one workgroup holds everything)
+        rank_kernel<true><<<1, RANK_WAVES * WAVE, lds(rank_blocks<true>()), s>>>(topk_idx, nullptr, T, k, E, W, NB, send_counts, expert_offs, dst_sizes, dst_offsets,
+                                                           caps, pos, row_token);
         return moe_check_launch("count_and_offsets");
     }
     block_hist_kernel<<<ceil_div(NB, 4), 256, 4 * E * sizeof(int32_t), s>>>(topk_idx, hist, T, k, E, NB);
-    if ((long long)E * NB <= SCAN1_MAXCELLS) {
-        scan_offsets_kernel<<<1, 1024, 0, s>>>(hist, base, counts, NB, E, W, expert_start, send_counts, expert_offs, dst_sizes,
-                                               dst_offsets, caps);
-    } else {
-        scan_blocks_kernel<<<E, WAVE, 0, s>>>(hist, base, counts, NB);
-        offsets_kernel<<<1, WAVE, 0, s>>>(counts, E, W, expert_start, send_counts, expert_offs, dst_sizes, dst_offsets, caps);
-    }
-    if (T > 0) rank_kernel<<<ceil_div(NB, 4), 256, 0, s>>>(topk_idx, base, expert_start, pos, row_token, T, k, E, NB);
+    rank_kernel<false><<<ceil_div(NB, rank_blocks<false>()), RANK_WAVES * WAVE, lds(rank_blocks<false>()), s>>>(
+        topk_idx, hist, T, k, E, W, NB, send_counts, expert_offs, dst_sizes, dst_offsets, caps, pos, row_token);
     return moe_check_launch("count_and_offsets");
 }
 
@@ -918,11 +945,12 @@ extern "C" int moe_pack_tokens_gated(const void* x, int dtype, int T, int H, con
     MOE_REQUIRE((long long)W * M + T < (1ll << 31), MOE_ERR_UNSUPPORTED, "pack_tokens: W*M + T too large");
     MOE_REQUIRE(send_buf && dst_sizes && dst_offsets, MOE_ERR_INVALID, "pack_tokens: null pointer");
     MOE_REQUIRE(T == 0 || (x && topk_idx && pos), MOE_ERR_INVALID, "pack_tokens: null pointer");
-    const int n_units = T + ceil_div(W * M, PACK_ZR);
+    const int parts = row_parts(T, H * dtype_size(dtype) / 16);
+    const int n_units = T * parts + ceil_div(W * M, PACK_ZR);
     const int blocks = min(ceil_div(n_units, 4), 65535 * 8);
     pack_tokens_kernel<4><<<blocks, 4 * WAVE, 0, (hipStream_t)stream>>>((const u32x4*)x, (u32x4*)send_buf, topk_idx, pos, dst_sizes,
                                                                         dst_offsets, T, k, E_l, W, M,
-                                                                        H * dtype_size(dtype) / 16, status, gate, send_gate);
+                                                                        H * dtype_size(dtype) / 16, status, gate, send_gate, parts);
     return moe_check_launch("pack_tokens");
 }
 
@@ -933,33 +961,27 @@ extern "C" int moe_pack_tokens(const void* x, int dtype, int T, int H, const int
                                  status, stream);
 }
 
-static int recv_driven(const char* who, int mode, const void* src, void* dst, int dtype, int H, const int32_t* rc_dev,
-                       int W, int E_l, int M, int CAP, int n_out, int32_t* pca, int32_t* expert_cnt, int32_t* map_ws,
-                       int32_t* status, hipStream_t s) {
+static int recv_driven(const char* who, int mode, const void* src, void* dst, int dtype, int H, const RecvCounts& q, int W, int E_l, int M,
+                       int CAP, int n_out, int32_t* status, hipStream_t s) {
     int rc = check_rows(who, dtype, H);
     if (rc) return rc;
     MOE_REQUIRE(W > 0 && E_l > 0 && W * E_l <= MOE_MAX_EXPERTS, MOE_ERR_INVALID, "%s: bad W=%d E_l=%d", who, W, E_l);
-    MOE_REQUIRE(n_out >= 0 && rc_dev && map_ws, MOE_ERR_INVALID, "%s: bad arguments", who);
-    int32_t* tables = map_ws;
-    const int n = W * E_l;
-    int32_t* src_off = tables;
-    int32_t* row_off = tables + (n + 1);
-    int32_t* flat_off = tables + 2 * (n + 1);
-    recv_tables_kernel<<<1, WAVE, 0, s>>>(rc_dev, W, E_l, src_off, row_off, flat_off, pca, expert_cnt);
-    if (n_out == 0) return moe_check_launch(who);
+    MOE_REQUIRE(n_out >= 0 && q.counts, MOE_ERR_INVALID, "%s: bad arguments", who);
     // (an empty flat payload or gradient has no storage: every output row is then padding and the source is never read)
-    MOE_REQUIRE(dst && (src || mode == SRC_REORDER || mode == SRC_UNSHUFFLE), MOE_ERR_INVALID, "%s: null pointer", who);
+    MOE_REQUIRE(n_out == 0 || (dst && (src || mode == SRC_REORDER || mode == SRC_UNSHUFFLE)), MOE_ERR_INVALID, "%s: null pointer", who);
     RowSource a{};
     a.mode = mode;
-    a.rc = rc_dev; a.src_off = src_off; a.row_off = row_off; a.flat_off = flat_off;
     a.W = W; a.E_l = E_l; a.M = M; a.CAP = CAP;
     a.status = status;
-    return gather_rows(src, dst, a, n_out, H * dtype_size(dtype), s);
+    // (one workgroup at least, for pca and the totals; at most what the chip holds at once, which then walks the rows)
+    const int blocks = max(1, min(ceil_div(n_out, 4), 256 * 7));
+    gather_rows_kernel<4, true><<<blocks, 4 * WAVE, 0, s>>>((const u32x4*)src, (u32x4*)dst, a, n_out, H * dtype_size(dtype) / 16, q);
+    return moe_check_launch(who);
 }
 
 extern "C" size_t moe_recv_map_ints(int W, int E_l, int n_out) {
-    (void)n_out;  // the per-row map of earlier versions is gone: rows are resolved inside the gather kernel
-    return recv_tables_ints(W, E_l);
+    (void)n_out;  // (nothing needs it any more: tables and rows are resolved inside the copies; callers keep allocating what they did)
+    return (size_t)3 * (W * E_l + 1) + (size_t)W * E_l;
 }
 
 extern "C" int moe_unpack_token_buf(const void* recv, int dtype, int W, int M, int H, const int32_t* recv_counts,
@@ -967,26 +989,54 @@ extern "C" int moe_unpack_token_buf(const void* recv, int dtype, int W, int M, i
                                     moe_stream_t stream) {
     MOE_REQUIRE(M >= 1 && CAP >= 1, MOE_ERR_INVALID, "unpack_token_buf: M=%d CAP=%d", M, CAP);
     MOE_REQUIRE((long long)E_l * W * CAP < (1ll << 31), MOE_ERR_UNSUPPORTED, "unpack_token_buf: too many rows");
-    return recv_driven("unpack_token_buf", SRC_TOKBUF, recv, token_buf, dtype, H, recv_counts, W, E_l, M, CAP, E_l * W * CAP, pca,
-                       nullptr, map_ws, status, (hipStream_t)stream);
+    (void)map_ws;
+    return recv_driven("unpack_token_buf", SRC_TOKBUF, recv, token_buf, dtype, H, {recv_counts, E_l, 1, pca, nullptr}, W, E_l, M, CAP,
+                       E_l * W * CAP, status, (hipStream_t)stream);
 }
 
 extern "C" int moe_reorder_flat_to_token_buf(const void* flat, int dtype, int R, int H, const int32_t* recv_counts,
                                              int W, int E_l, int CAP, void* token_buf, int32_t* map_ws, int32_t* status,
                                              moe_stream_t stream) {
-    (void)R;
+    (void)R, (void)map_ws;
     MOE_REQUIRE(CAP >= 1, MOE_ERR_INVALID, "reorder: CAP=%d", CAP);
     MOE_REQUIRE((long long)E_l * W * CAP < (1ll << 31), MOE_ERR_UNSUPPORTED, "reorder: too many rows");
-    return recv_driven("reorder_flat_to_token_buf", SRC_REORDER, flat, token_buf, dtype, H, recv_counts, W, E_l, 1, CAP,
-                       E_l * W * CAP, nullptr, nullptr, map_ws, status, (hipStream_t)stream);
+    return recv_driven("reorder_flat_to_token_buf", SRC_REORDER, flat, token_buf, dtype, H, {recv_counts, E_l, 1, nullptr, nullptr}, W, E_l, 1,
+                       CAP, E_l * W * CAP, status, (hipStream_t)stream);
 }
 
 extern "C" int moe_unpack_expert_major(const void* recv, int dtype, int W, int M, int H, const int32_t* recv_counts,
                                        int E_l, void* shuffled, int S_rows, int32_t* expert_cnt, int32_t* map_ws,
                                        moe_stream_t stream) {
+    (void)map_ws;
     MOE_REQUIRE(M >= 1, MOE_ERR_INVALID, "unpack_expert_major: M=%d", M);
-    return recv_driven("unpack_expert_major", SRC_UNPACK, recv, shuffled, dtype, H, recv_counts, W, E_l, M, 1, S_rows, nullptr,
-                       expert_cnt, map_ws, nullptr, (hipStream_t)stream);
+    return recv_driven("unpack_expert_major", SRC_UNPACK, recv, shuffled, dtype, H, {recv_counts, E_l, 1, nullptr, expert_cnt}, W, E_l, M, 1,
+                       S_rows, nullptr, (hipStream_t)stream);
+}
+
+static int launch_row_map(const int32_t* rc, int W, int E_l, int M, int n_rows, int32_t* map, int32_t* expert_cnt, const float* recv_gate,
+                          float* row_gate, const float* recv_scale, float* row_scale, void* zbuf, int row_bytes, hipStream_t s) {
+    // (at least one block, for the per-expert totals)
+    const int map_blocks = max(ceil_div(n_rows, 256), 1), zero_blocks = zbuf ? ceil_div(ceil_div(W * M, PACK_ZR), 4) : 0;
+    row_map_from_counts_kernel<<<map_blocks + zero_blocks, 256, 0, s>>>(rc, W, E_l, M, n_rows, map, expert_cnt, recv_gate, row_gate, recv_scale,
+                                                                        row_scale, (u32x4*)zbuf, row_bytes / 16, map_blocks);
+    return moe_check_launch("recv_row_map");
+}
+
+extern "C" int moe_recv_prepare(const int32_t* recv_counts, int W, int E_l, int M, int n_rows, const float* recv_gate, const float* recv_scale,
+                                int32_t* row_map, float* row_gate, float* row_scale, int32_t* expert_cnt, void* ret, int dtype, int H,
+                                moe_stream_t stream) {
+    MOE_REQUIRE(W > 0 && E_l > 0 && W * E_l <= MOE_MAX_EXPERTS, MOE_ERR_INVALID, "recv_prepare: bad W=%d E_l=%d", W, E_l);
+    MOE_REQUIRE(M >= 0 && n_rows >= 0 && recv_counts, MOE_ERR_INVALID, "recv_prepare: bad arguments");
+    MOE_REQUIRE((recv_gate == nullptr) == (row_gate == nullptr) && (recv_scale == nullptr) == (row_scale == nullptr), MOE_ERR_INVALID,
+                "recv_prepare: received and row-ordered values go together");
+    MOE_REQUIRE(n_rows == 0 || row_map, MOE_ERR_INVALID, "recv_prepare: null pointer");
+    if (ret) {
+        const int rc = check_rows("recv_prepare", dtype, H);
+        if (rc) return rc;
+        MOE_REQUIRE(M >= 1 && (long long)W * M < (1ll << 31), MOE_ERR_UNSUPPORTED, "recv_prepare: %d x %d rows", W, M);
+    }
+    return launch_row_map(recv_counts, W, E_l, M, n_rows, row_map, expert_cnt, recv_gate, row_gate, recv_scale, row_scale, ret,
+                          H * dtype_size(dtype), (hipStream_t)stream);
 }
 
 extern "C" int moe_recv_row_map(const int32_t* recv_counts, int W, int E_l, int M, int n_rows, int32_t* row_map,
@@ -997,9 +1047,7 @@ extern "C" int moe_recv_row_map(const int32_t* recv_counts, int W, int E_l, int 
     (void)map_ws;  // (the tables of earlier versions live in LDS now)
     MOE_REQUIRE(n_rows == 0 || row_map, MOE_ERR_INVALID, "recv_row_map: null pointer");
     // (one launch: every block rebuilds the prefix tables in LDS; at least one block, for the per-expert totals)
-    row_map_from_counts_kernel<<<max(ceil_div(n_rows, 256), 1), 256, 0, s>>>(recv_counts, W, E_l, M, n_rows, row_map, expert_cnt,
-                                                                             nullptr, nullptr);
-    return moe_check_launch("recv_row_map");
+    return launch_row_map(recv_counts, W, E_l, M, n_rows, row_map, expert_cnt, nullptr, nullptr, nullptr, nullptr, nullptr, 0, s);
 }
 
 extern "C" int moe_recv_row_map_gated(const int32_t* recv_counts, int W, int E_l, int M, int n_rows, const float* recv_gate,
@@ -1008,9 +1056,7 @@ extern "C" int moe_recv_row_map_gated(const int32_t* recv_counts, int W, int E_l
     MOE_REQUIRE(M >= 0 && n_rows >= 0 && recv_counts, MOE_ERR_INVALID, "recv_row_map_gated: bad arguments");
     MOE_REQUIRE((recv_gate == nullptr) == (row_gate == nullptr), MOE_ERR_INVALID, "recv_row_map_gated: recv_gate and row_gate go together");
     MOE_REQUIRE(n_rows == 0 || row_map, MOE_ERR_INVALID, "recv_row_map_gated: null pointer");
-    row_map_from_counts_kernel<<<max(ceil_div(n_rows, 256), 1), 256, 0, (hipStream_t)stream>>>(recv_counts, W, E_l, M, n_rows, row_map,
-                                                                                               expert_cnt, recv_gate, row_gate);
-    return moe_check_launch("recv_row_map_gated");
+    return launch_row_map(recv_counts, W, E_l, M, n_rows, row_map, expert_cnt, recv_gate, row_gate, nullptr, nullptr, nullptr, 0, (hipStream_t)stream);
 }
 
 extern "C" int moe_recv_row_map_flat(const int32_t* recv_counts, int W, int E_l, int n_rows, int32_t* row_map, int32_t* expert_cnt,
@@ -1029,22 +1075,14 @@ extern "C" int moe_zero_padding_rows(void* buf, int dtype, int W, int M, int H, 
     return moe_check_launch("zero_padding_rows");
 }
 
-// token_buf -> shuffled: pca is [E_l,W]; the tables kernel wants [W,E_l] counts, so transpose first.
-__global__ void transpose_counts_kernel(const int32_t* __restrict__ in, int rows, int cols, int32_t* __restrict__ out) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < rows * cols) out[(i % cols) * rows + (i / cols)] = in[i];
-}
-
 extern "C" int moe_shuffle(const void* token_buf, int dtype, int E_l, int W, int CAP, int H, const int32_t* pca,
                            void* shuffled, int S_rows, int32_t* expert_cnt, int32_t* map_ws, moe_stream_t stream) {
     hipStream_t s = (hipStream_t)stream;
     MOE_REQUIRE(W > 0 && E_l > 0 && W * E_l <= MOE_MAX_EXPERTS && CAP >= 1 && S_rows >= 0 && pca && map_ws,
                 MOE_ERR_INVALID, "shuffle: bad arguments");
-    // recv_counts[s,e] = pca[e,s], kept behind the tables in map_ws
-    int32_t* rc_t = map_ws + 3 * (W * E_l + 1);
-    transpose_counts_kernel<<<ceil_div(W * E_l, 256), 256, 0, s>>>(pca, E_l, W, rc_t);
-    return recv_driven("shuffle", SRC_SHUFFLE, token_buf, shuffled, dtype, H, rc_t, W, E_l, 1, CAP, S_rows, nullptr, expert_cnt,
-                       map_ws, nullptr, s);
+    // (pca[e,s] = recv_counts[s,e])
+    return recv_driven("shuffle", SRC_SHUFFLE, token_buf, shuffled, dtype, H, {pca, 1, W, nullptr, expert_cnt}, W, E_l, 1, CAP, S_rows,
+                       nullptr, s);
 }
 
 // gradient of moe_shuffle: grad_token_buf[e,s,j,:] = grad_rows[off[e,s] + j,:] for j < pca[e,s], zeros elsewhere
@@ -1054,19 +1092,17 @@ extern "C" int moe_shuffle_backward(const void* grad_rows, int dtype, int E_l, i
     MOE_REQUIRE(W > 0 && E_l > 0 && W * E_l <= MOE_MAX_EXPERTS && CAP >= 1 && pca && map_ws, MOE_ERR_INVALID,
                 "shuffle_backward: bad arguments");
     MOE_REQUIRE((long long)E_l * W * CAP < (1ll << 31), MOE_ERR_UNSUPPORTED, "shuffle_backward: too many rows");
-    int32_t* rc_t = map_ws + 3 * (W * E_l + 1);  // recv_counts[s,e] = pca[e,s], kept behind the tables
-    transpose_counts_kernel<<<ceil_div(W * E_l, 256), 256, 0, s>>>(pca, E_l, W, rc_t);
-    return recv_driven("shuffle_backward", SRC_UNSHUFFLE, grad_rows, grad_token_buf, dtype, H, rc_t, W, E_l, 1, CAP, E_l * W * CAP,
-                       nullptr, nullptr, map_ws, nullptr, s);
+    return recv_driven("shuffle_backward", SRC_UNSHUFFLE, grad_rows, grad_token_buf, dtype, H, {pca, 1, W, nullptr, nullptr}, W, E_l, 1, CAP,
+                       E_l * W * CAP, nullptr, s);
 }
 
 extern "C" int moe_return_pack(const void* y, int dtype, int S_rows, int H, const int32_t* recv_counts, int W, int E_l,
                                int M, void* ret, int32_t* map_ws, moe_stream_t stream) {
-    (void)S_rows;
+    (void)S_rows, (void)map_ws;
     MOE_REQUIRE(M >= 1, MOE_ERR_INVALID, "return_pack: M=%d", M);
     MOE_REQUIRE((long long)W * M < (1ll << 31), MOE_ERR_UNSUPPORTED, "return_pack: W*M too large");
-    return recv_driven("return_pack", SRC_RETURN, y, ret, dtype, H, recv_counts, W, E_l, M, 1, W * M, nullptr, nullptr, map_ws,
-                       nullptr, (hipStream_t)stream);
+    return recv_driven("return_pack", SRC_RETURN, y, ret, dtype, H, {recv_counts, E_l, 1, nullptr, nullptr}, W, E_l, M, 1, W * M, nullptr,
+                       (hipStream_t)stream);
 }
 
 extern "C" int moe_combine_backward(const void* d_out, const void* ret, int dtype, int W, int M, int H, const int32_t* topk_idx,
@@ -1078,17 +1114,25 @@ extern "C" int moe_combine_backward(const void* d_out, const void* ret, int dtyp
     MOE_REQUIRE(W > 0 && M >= 1 && T >= 0 && E_l > 0, MOE_ERR_INVALID, "combine_backward: bad shape");
     MOE_REQUIRE(k >= 1 && k <= MOE_MAX_TOPK, MOE_ERR_UNSUPPORTED, "combine_backward: topk=%d outside [1,%d]", k, MOE_MAX_TOPK);
     MOE_REQUIRE((long long)W * M + T < (1ll << 31), MOE_ERR_UNSUPPORTED, "combine_backward: W*M + T too large");
-    MOE_REQUIRE(d_ret && dst_sizes && dst_offsets, MOE_ERR_INVALID, "combine_backward: null pointer");
+    MOE_REQUIRE(d_ret && dst_offsets, MOE_ERR_INVALID, "combine_backward: null pointer");
     MOE_REQUIRE(T == 0 || (d_out && ret && topk_idx && pos && gate && d_gate), MOE_ERR_INVALID, "combine_backward: null pointer");
-    const int n_rows = T + W * M;
-    const int blocks = min(ceil_div(n_rows, 4), 65535 * 8);
+    const int blocks = min(ceil_div(T + ceil_div(W * M, PACK_ZR), 4), 65535 * 8);
     const int row_vec = H * dtype_size(dtype) / 16;
-    if (dtype == MOE_F32)
-        combine_backward_kernel<float, 4><<<blocks, 4 * WAVE, 0, s>>>((const uint4*)d_out, (const uint4*)ret, topk_idx, pos, gate, dst_sizes,
-                                                                      dst_offsets, T, k, E_l, W, M, row_vec, (uint4*)d_ret, d_gate);
-    else
-        combine_backward_kernel<bf16_t, 4><<<blocks, 4 * WAVE, 0, s>>>((const uint4*)d_out, (const uint4*)ret, topk_idx, pos, gate, dst_sizes,
-                                                                       dst_offsets, T, k, E_l, W, M, row_vec, (uint4*)d_ret, d_gate);
+#define MOE_CB(XT, KT) \
+    combine_backward_kernel<XT, KT, 4><<<blocks, 4 * WAVE, 0, s>>>((const uint4*)d_out, (const uint4*)ret, topk_idx, pos, gate, dst_sizes, \
+                                                                   dst_offsets, T, k, E_l, W, M, row_vec, (uint4*)d_ret, d_gate)
+#define MOE_CBK(XT)                                    \
+    switch (k) {                                       \
+        case 1: MOE_CB(XT, 1); break;                  \
+        case 2: MOE_CB(XT, 2); break;                  \
+        case 4: MOE_CB(XT, 4); break;                  \
+        case 8: MOE_CB(XT, 8); break;                  \
+        default: MOE_CB(XT, 0); break;                 \
+    }
+    if (dtype == MOE_F32) MOE_CBK(float)
+    else MOE_CBK(bf16_t)
+#undef MOE_CBK
+#undef MOE_CB
     return moe_check_launch("combine_backward");
 }
 

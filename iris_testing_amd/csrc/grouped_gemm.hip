@@ -2054,10 +2054,10 @@ extern "C" int moe_grouped_mlp_fp8_q_mapped(const uint8_t* a_q, const float* a_s
     MOE_REQUIRE((unsigned long long)S_rows * (unsigned long long)(F / 32) < (1ull << 32), MOE_ERR_UNSUPPORTED,
                 "grouped_mlp_fp8_q: the block scales must stay under 4 GiB");
     if (S_rows == 0) return MOE_OK;
-    MOE_REQUIRE(a_q && a_scale && expert_cnt && wgu_packed && sg && su && wd_packed && sd && xs_ws && hq_ws && hscale_ws && out,
+    MOE_REQUIRE(a_q && expert_cnt && wgu_packed && sg && su && wd_packed && sd && xs_ws && hq_ws && hscale_ws && out,
                 MOE_ERR_INVALID, "grouped_mlp_fp8_q: null pointer");
     // the row scales in the order of the GEMM's rows (the codes themselves are gathered by the GEMM as it loads them)
-    gather_scale_kernel<<<ceil_div(S_rows, 256), 256, 0, s>>>(a_scale, a_row_map, S_rows, xs_ws);
+    if (a_scale) gather_scale_kernel<<<ceil_div(S_rows, 256), 256, 0, s>>>(a_scale, a_row_map, S_rows, xs_ws);
     return fp8_mlp_gemms(a_q, a_row_map, xs_ws, expert_cnt, S_rows, H, F, E_l, wgu_packed, sg, su, wd_packed, sd, hq_ws, hscale_ws,
                          row_gate, out, c_row_map, part_ws, part_ws_bytes, s);
 }

@@ -1,0 +1,76 @@
+// One step of the hot path as one call: host code only, every stage is an entry point of its own.
+#include "common.h"
+
+// Stage by stage from Python a step costs 8 to 10 foreign calls with some fifteen arguments each (about 80 us of host time);
+// here one, so an eager step of a small model waits for the GPU and not for the host.  The destination side derives the row map, the
+// row scales, the gates and the zeroed padding rows from the received counts in one launch (a launch costs some 4.5 us
+// even when it has nothing to do).
+extern "C" int moe_step(const moe_step_args* a, moe_stream_t stream) {
+    MOE_REQUIRE(a, MOE_ERR_INVALID, "step: null arguments");
+    const int T = a->tokens, H = a->hidden, E = a->experts, k = a->topk, W = a->world, F = a->ffn, M = a->M, S = a->S;
+    MOE_REQUIRE(W > 0 && E > 0 && E % W == 0, MOE_ERR_INVALID, "step: %d experts on %d ranks", E, W);
+    MOE_REQUIRE(a->fused || !(a->flat || a->gated || a->q_dispatch), MOE_ERR_INVALID, "step: flat / gated / q_dispatch are fused modes");
+    MOE_REQUIRE(!a->q_dispatch || (a->quant && !a->flat), MOE_ERR_INVALID, "step: q_dispatch needs fp8 experts and fixed slots");
+    MOE_REQUIRE(!(a->flat && a->gated), MOE_ERR_INVALID, "step: flat and gated are separate modes");
+    const int E_l = E / W;
+    const float* out_gate = a->gated ? a->gate : nullptr;
+    int rc;
+#define MOE_STAGE(call)                           \
+    do {                                          \
+        if ((rc = (call)) != MOE_OK) return rc;   \
+    } while (0)
+    MOE_STAGE(moe_route_topk(a->x, a->router, a->bias, a->dtype, T, H, E, k, a->logits, a->idx, a->gate, a->route_ws, a->route_ws_bytes,
+                             stream));
+    MOE_STAGE(moe_count_and_offsets(a->idx, T, k, E, W, a->send_counts, a->expert_offs, a->dst_sizes, a->dst_offsets, a->caps, a->pos,
+                                    a->row_token, a->count_ws, a->count_ws_bytes, stream));
+    if (a->q_dispatch)
+        MOE_STAGE(moe_pack_tokens_fp8_gated(a->x, T, H, a->idx, a->pos, out_gate, k, E_l, a->dst_sizes, a->dst_offsets, W, M,
+                                            (uint8_t*)a->send, a->send_scale, a->gated ? a->send_gate : nullptr, a->status, stream));
+    else if (a->flat)
+        MOE_STAGE(moe_pack_payload(a->x, a->dtype, T, H, a->row_token, T * k, a->send, stream));
+    else if (a->gated)
+        MOE_STAGE(moe_pack_tokens_gated(a->x, a->dtype, T, H, a->idx, a->pos, a->gate, k, E_l, a->dst_sizes, a->dst_offsets, W, M, a->send,
+                                        a->send_gate, a->status, stream));
+    else
+        MOE_STAGE(moe_pack_tokens(a->x, a->dtype, T, H, a->idx, a->pos, k, E_l, a->dst_sizes, a->dst_offsets, W, M, a->send, a->status,
+                                  stream));
+    // destination: rows in expert-major order
+    if (a->fused)
+        MOE_STAGE(moe_recv_prepare(a->recv_counts, W, E_l, a->flat ? 0 : M, S, a->gated ? a->recv_gate : nullptr,
+                                   a->q_dispatch ? a->recv_scale : nullptr, a->row_map, a->gated ? a->row_gate : nullptr,
+                                   a->q_dispatch ? a->xs : nullptr, a->expert_cnt, a->flat ? nullptr : a->ret, a->dtype, H, stream));
+    else
+        MOE_STAGE(moe_unpack_expert_major(a->recv, a->dtype, W, M, H, a->recv_counts, E_l, a->rows, S, a->expert_cnt, a->unpack_map, stream));
+    const void* src = a->fused ? a->recv : a->rows;
+    void* dst = a->fused ? a->ret : a->y;
+    const int n_buf = a->fused && !a->flat ? W * M : S;
+    const int32_t* map = a->fused ? a->row_map : nullptr;
+    const float* row_gate = a->gated ? a->row_gate : nullptr;
+    if (a->q_dispatch)
+        MOE_STAGE(moe_grouped_mlp_fp8_q_mapped((const uint8_t*)src, nullptr, n_buf, map, a->expert_cnt, S, H, F, E_l, (const uint8_t*)a->w1,
+                                               a->s1, a->s_up, (const uint8_t*)a->w2, a->s2, a->xs, a->hq, a->hscale, row_gate, dst, n_buf,
+                                               map, a->part_ws, a->part_ws_bytes, stream));
+    else if (a->quant)
+        MOE_STAGE(moe_grouped_mlp_fp8_mapped(src, n_buf, map, a->expert_cnt, S, H, F, E_l, (const uint8_t*)a->w1, a->s1, a->s_up,
+                                             (const uint8_t*)a->w2, a->s2, a->xq, a->xs, a->hq, a->hscale, row_gate, dst, n_buf, map,
+                                             a->part_ws, a->part_ws_bytes, stream));
+    else if (a->f32_weights)
+        MOE_STAGE(moe_grouped_mlp(src, a->expert_cnt, a->dtype, S, H, F, E_l, a->act, a->w1, a->w_up, a->w2, a->hidden_ws, dst, stream));
+    else {
+        MOE_STAGE(moe_grouped_gemm_mapped(src, n_buf, map, a->w1, a->expert_cnt, S, H, F, E_l, a->act, a->hidden_ws, S, nullptr, a->part_ws,
+                                          a->part_ws_bytes, stream));
+        if (a->gated)
+            MOE_STAGE(moe_grouped_gemm_mapped_gated(a->hidden_ws, S, nullptr, a->w2, a->expert_cnt, S, F, H, E_l, row_gate, dst, n_buf, map,
+                                                    a->part_ws, a->part_ws_bytes, stream));
+        else
+            MOE_STAGE(moe_grouped_gemm_mapped(a->hidden_ws, S, nullptr, a->w2, a->expert_cnt, S, F, H, E_l, MOE_ACT_NONE, dst, n_buf, map,
+                                              a->part_ws, a->part_ws_bytes, stream));
+    }
+    if (!a->fused) MOE_STAGE(moe_return_pack(a->y, a->dtype, S, H, a->recv_counts, W, E_l, M, a->ret, a->ret_map, stream));
+    // the flat returned payload is indexed by position: one "destination" that holds all experts, offset 0
+    if (a->flat)
+        return moe_combine(a->returned, a->dtype, 1, T * k, H, a->idx, a->pos, a->gate, a->zero_off, T, k, E, a->out, a->status, stream);
+    return moe_combine(a->returned, a->dtype, W, M, H, a->idx, a->pos, a->gated ? nullptr : a->gate, a->dst_offsets, T, k, E_l, a->out,
+                       a->status, stream);
+#undef MOE_STAGE
+}

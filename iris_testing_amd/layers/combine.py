@@ -7,12 +7,6 @@ import torch
 from .. import ops
 
 
-def _dst_sizes(dst_offsets: torch.Tensor, routed_rows: int) -> torch.Tensor:
-    """Rows per destination from their exclusive prefix (the last one runs to the routed total)."""
-    end = torch.full((1,), routed_rows, dtype=dst_offsets.dtype, device=dst_offsets.device)
-    return torch.diff(dst_offsets, append=end).contiguous()
-
-
 class Combine(torch.autograd.Function):
 
     @staticmethod
@@ -26,8 +20,8 @@ class Combine(torch.autograd.Function):
     def backward(ctx, d_out):
         """d returned[slot(t,kk)] = gate[t,kk] * d out[t] (zeros in the padding); d gate[t,kk] = <d out[t], returned[slot(t,kk)]>."""
         returned, gate, idx, pos, dst_offsets = ctx.saved_tensors
-        sizes = _dst_sizes(dst_offsets, idx.numel())
-        d_ret, d_gate = ops.combine_backward(d_out.contiguous(), returned, idx, pos, gate.contiguous(), sizes, dst_offsets, ctx.e_local)
+        # (rows per destination: from one start to the next, derived where they are needed)
+        d_ret, d_gate = ops.combine_backward(d_out.contiguous(), returned, idx, pos, gate.contiguous(), None, dst_offsets, ctx.e_local)
         return d_ret, d_gate, None, None, None, None
 
 
@@ -52,10 +46,9 @@ class PackFixedM(torch.autograd.Function):
     @staticmethod
     def backward(ctx, d_send):
         """Every token row was copied to its k slots: its gradient is the sum of the k slot gradients, i.e. the combine
-        with unit gates (fp32 sum in slot order, one rounding)."""
+        without gates (fp32 sum in slot order, one rounding)."""
         idx, pos, dst_offsets = ctx.saved_tensors
-        ones = torch.ones(idx.shape, dtype=torch.float32, device=idx.device)
-        return ops.combine(d_send.contiguous(), idx, pos, ones, dst_offsets, ctx.e_local), None, None, None, None, None, None
+        return ops.combine(d_send.contiguous(), idx, pos, None, dst_offsets, ctx.e_local), None, None, None, None, None, None
 
 
 def pack_fixed_m(tokens: torch.Tensor, topk_idx: torch.Tensor, pos: torch.Tensor, dst_sizes: torch.Tensor,

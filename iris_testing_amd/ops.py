@@ -709,13 +709,16 @@ def mlp_act_backward(a1: torch.Tensor, dh: torch.Tensor, act: str) -> torch.Tens
 
 
 def combine_backward(d_out: torch.Tensor, ret: torch.Tensor, topk_idx: torch.Tensor, pos: torch.Tensor, gate: torch.Tensor,
-                     dst_sizes: torch.Tensor, dst_offsets: torch.Tensor, e_local: int) -> Tuple[torch.Tensor, torch.Tensor]:
-    """(d ret [W,M,H], d gate [T,k]) of out = combine(ret, ...)."""
+                     dst_sizes: Optional[torch.Tensor], dst_offsets: torch.Tensor,
+                     e_local: int) -> Tuple[torch.Tensor, torch.Tensor]:
+    """(d ret [W,M,H], d gate [T,k]) of out = combine(ret, ...).  dst_sizes None: every slot is routed, so a destination's rows
+    end where the next one's start."""
     _req_cuda(d_out, "d_out")
     _req_cuda(ret, "ret")
     _req_i32(topk_idx, "topk_idx")
     _req_i32(pos, "pos")
-    _req_i32(dst_sizes, "dst_sizes")
+    if dst_sizes is not None:
+        _req_i32(dst_sizes, "dst_sizes")
     _req_i32(dst_offsets, "dst_offsets")
     W, M, H = ret.shape
     T, k = topk_idx.shape

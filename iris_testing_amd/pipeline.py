@@ -15,8 +15,8 @@ With ``padding_free=True`` (fused) the rows cross as the reference's padding-fre
 fixed-M slots: "pack" gathers the payload, the GEMMs gather from / scatter into flat [S,H] buffers through a row map over
 the payload's source-major blocks, nothing is zero-filled, and the combine reads the returned payload by position.
 The two transfers in between are not part of a one-GPU build: the receive buffer and the returned
-buffer are assembled beforehand (harness.build_world) and stay fixed.  Each stage is one C-ABI call
-on the current stream; no stage synchronises or allocates.
+buffer are assembled beforehand (harness.build_world) and stay fixed.  A step is one C-ABI call on the current stream, and so
+is each stage on its own (for callers that time them one by one); none synchronises or allocates.
 """
 from __future__ import annotations
 
@@ -115,6 +115,34 @@ class DispatchPipeline:
             self.returned = returned if returned is not None else torch.zeros((W, M, H), dtype=dt, device=dev)
         self.out = torch.empty((T, H), dtype=dt, device=dev)
         self._p = L.ptr
+        self._args = self._step_args()
+
+    def _step_args(self) -> L.StepArgs:
+        """The argument block of moe_step: sizes, modes and this object's own buffers (step() fills in the rest)."""
+        c, ew, p = self.cfg, self.weights, self._p
+        get = lambda name: p(getattr(self, name, None))  # noqa: E731  (buffers a mode does not use do not exist)
+        return L.StepArgs(
+            tokens=c.tokens, hidden=c.hidden, experts=c.experts, topk=c.topk, world=c.world, ffn=c.ffn, act=L.ACT[ew.act],
+            dtype=self.code, M=self.world.M, S=self.S, fused=self.fused, flat=self.padding_free, gated=self.gated,
+            quant=ew.dtype == torch.uint8, q_dispatch=self.fp8_dispatch, f32_weights=ew.dtype == torch.float32,
+            send=p(self.send_q if self.fp8_dispatch else self.payload if self.padding_free else self.send),
+            hidden_ws=get("hidden"), hscale=get("hsc"), ret=p(self.ret_flat if self.padding_free else self.ret),
+            **{n: get(n) for n in ("logits idx gate route_ws send_counts expert_offs dst_sizes dst_offsets caps pos row_token count_ws "
+                                   "send_scale send_gate status row_map expert_cnt row_gate rows y xq hq xs unpack_map ret_map part_ws "
+                                   "zero_off out").split()},
+            route_ws_bytes=self.route_ws_bytes, count_ws_bytes=self.count_ws_bytes, part_ws_bytes=self.part_ws_bytes)
+
+    def _run(self, s):
+        """The stages of STAGES as one call (the map, scales, gates and padding of the destination side in one launch)."""
+        a, w, ew, p = self._args, self.world, self.weights, self._p
+        # what belongs to the caller is looked up on every step
+        a.x, a.router, a.bias, a.recv_counts = p(w.x0), p(w.router), p(w.bias), p(w.recv_counts)
+        a.recv = p(w.recv_q if self.fp8_dispatch else self.recv_flat if self.padding_free else w.recv)
+        a.recv_scale, a.recv_gate = p(w.recv_scale), p(self.recv_gate)
+        a.w1, a.w_up, a.w2, a.returned = p(ew.w1), p(ew.w_up), p(ew.w2), p(self.returned)
+        if ew.dtype == torch.uint8:
+            a.s1, a.s_up, a.s2 = (p(t) for t in ew.scales)
+        L.check(L.lib().moe_step(a, s))
 
     # each stage is a closure-free method so that callers can time them one by one
     def route(self, s):
@@ -259,17 +287,17 @@ class DispatchPipeline:
         """One pass of the hot path.  With ``events`` (a list), per-stage (start, end) torch.cuda.Event
         pairs of this step are appended to it."""
         s = L.stream_ptr()
-        rec = {} if events is not None else None
+        if events is None:
+            self._run(s)
+            return
+        rec = {}
         for name in STAGES:
-            if rec is not None:
-                a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-                a.record()
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
             getattr(self, name)(s)
-            if rec is not None:
-                b.record()
-                rec[name] = (a, b)
-        if events is not None:
-            events.append(rec)
+            b.record()
+            rec[name] = (a, b)
+        events.append(rec)
 
     def capture(self):
         """The whole step as one HIP graph (every stage only enqueues kernels: no allocation, no memset,

@@ -493,3 +493,57 @@ def test_pack_and_combine_at_other_top_k(k, dtype):
     ret = O.bf16_round(rng.standard_normal((W, M, H)).astype(np.float32)) if dtype == "bf16" else rng.standard_normal((W, M, H)).astype(np.float32)
     out = ops.combine(torch.from_numpy(ret).to(tdt).to(DEV), dev(idx), dev(pos), dev(gate), dev(offs), E_l)
     assert_bits_equal(out, O.combine(ret, idx, pos, gate, offs, E_l, dtype), "combine")
+
+
+@pytest.mark.parametrize("T", [1, 64, 65, 1024, 1025, 2049])
+@pytest.mark.parametrize("E,W,k", [(2, 2, 1), (60, 4, 3), (512, 8, 8)])
+def test_counts_and_positions_at_block_edges(T, E, W, k):
+    """The single-workgroup count (up to 1024 tokens) and the two-launch one, around the edges of their blocks of 64 and 1024."""
+    rng = np.random.default_rng(T + E)
+    p = rng.random(E) ** 4 + 1e-6
+    idx = np.stack([rng.choice(E, k, replace=False, p=p / p.sum()) for _ in range(T)]).astype(np.int32)
+    c = ops.count_and_offsets(torch.from_numpy(idx).to(DEV), E, W)
+    counts = O.send_counts(idx, W, E)
+    sizes, offs = O.dst_sizes_offsets(counts)
+    pos, row_token = O.payload_positions(idx, E)
+    assert_bits_equal(c.send_counts, counts, "send_counts")
+    assert_bits_equal(c.expert_offs, O.build_expert_offsets(counts), "expert_offs")
+    assert_bits_equal(c.dst_sizes, sizes, "dst_sizes")
+    assert_bits_equal(c.dst_offsets, offs, "dst_offsets")
+    assert_bits_equal(c.pos, pos, "pos")
+    assert_bits_equal(c.row_token, row_token, "row_token")
+    assert c.caps.tolist() == [max(1, int(sizes.max())), max(1, int(counts.max()))]
+
+
+@pytest.mark.parametrize("T,H,k", [(1, 520, 1), (5, 4096, 3), (33, 1032, 8), (700, 264, 2)])
+def test_row_copies_and_sums_cut_into_column_runs(T, H, k):
+    """Few tokens: a row is cut into runs of columns (whole, ragged, single); pack, combine and the gradient of combine."""
+    rng = np.random.default_rng(T)
+    E, W = 16, 4
+    E_l = E // W
+    x = O.bf16_round(rng.standard_normal((T, H)).astype(np.float32))
+    idx = np.stack([rng.permutation(E)[:k] for _ in range(T)]).astype(np.int32)
+    gate = rng.random((T, k)).astype(np.float32)
+    sizes, offs = O.dst_sizes_offsets(O.send_counts(idx, W, E))
+    pos, row_token = O.payload_positions(idx, E)
+    M = O.pair_capacity(sizes) + 1
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(DEV)  # noqa: E731
+    bf = lambda a: torch.from_numpy(a).bfloat16().to(DEV)  # noqa: E731
+    send = ops.pack_tokens(bf(x), dev(idx), dev(pos), dev(sizes), dev(offs), E_l, M)
+    assert_bits_equal(send, O.pack_fixed_m(O.send_payload(x, row_token), offs, sizes, M), "send")
+    ret = O.bf16_round(rng.standard_normal((W, M, H)).astype(np.float32))
+    out = ops.combine(bf(ret), dev(idx), dev(pos), dev(gate), dev(offs), E_l)
+    assert_bits_equal(out, O.combine(ret, idx, pos, gate, offs, E_l, "bf16"), "combine")
+    d_out = O.bf16_round(rng.standard_normal((T, H)).astype(np.float32))
+    want = np.zeros((W, M, H), np.float32)
+    want_g = np.zeros((T, k), np.float64)
+    for t in range(T):
+        for j in range(k):
+            d = idx[t, j] // E_l
+            m = pos[t, j] - offs[d]
+            want[d, m] = O.bf16_round(gate[t, j] * d_out[t])
+            want_g[t, j] = (d_out[t].astype(np.float64) * ret[d, m]).sum()
+    for known in (dev(sizes), None):  # (None: the sizes follow from the starts)
+        d_ret, d_gate = ops.combine_backward(bf(d_out), bf(ret), dev(idx), dev(pos), dev(gate), known, dev(offs), E_l)
+        assert_bits_equal(d_ret, want, "d returned")
+        np.testing.assert_allclose(to_np(d_gate), want_g, rtol=1e-4, atol=1e-3)

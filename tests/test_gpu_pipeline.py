@@ -86,6 +86,37 @@ def test_graph_replay_equals_eager(name, fused):
         torch.cuda.synchronize()
 
 
+@pytest.mark.parametrize("name,mode", [("plumbing", {}), ("small", dict(fused=False)), ("small", {}), ("small", dict(gated=True)),
+                                       ("small", dict(padding_free=True)), ("zipf_k4", {}), ("zipf_k4", dict(fp8_dispatch=False)),
+                                       ("zipf_k4", dict(gated=True)), ("zipf_k4", dict(padding_free=True))])
+def test_step_as_one_call_equals_its_stages(name, mode):
+    """step() is one library call; with events it runs stage by stage.  Every result must be the same bits."""
+    from dataclasses import replace
+    from iris_testing_amd.pipeline import DispatchPipeline
+    cfg = CONFIGS[name]
+    cfg = replace(cfg, tokens=min(cfg.tokens, 300))
+    world = harness.build_world(cfg, DEV)
+    ew, _, _ = harness.expert_weights(cfg, 0, DEV)
+    if mode.get("gated"):
+        mode = dict(mode, recv_gate=harness.recv_gates(world))
+    if mode.get("padding_free"):
+        mode = dict(mode, recv_flat=harness.recv_flat(world))
+    pipe = DispatchPipeline(world, ew, **mode)
+    pipe.returned.copy_(torch.randn(pipe.returned.shape, device=DEV).to(pipe.returned.dtype))
+    names = [n for n in ("logits idx gate send_counts expert_offs dst_sizes dst_offsets caps pos row_token send send_gate payload send_q "
+                         "send_scale expert_cnt row_map row_gate rows hidden y ret ret_flat xq xs hq hsc out").split()
+             if isinstance(getattr(pipe, n, None), torch.Tensor)]
+    def results(events):
+        for n in names:
+            getattr(pipe, n).zero_()
+        pipe.step(events)
+        torch.cuda.synchronize()
+        return {n: getattr(pipe, n).clone() for n in names}
+    one, stages = results(None), results([])
+    for n in names:
+        assert torch.equal(one[n], stages[n]), f"{n} differs"
+
+
 def test_entry_point_smoke_runs():
     """The smoke check of the repository's entry module (one small step against the oracle) must keep passing."""
     import importlib
