@@ -1184,103 +1184,130 @@ __global__ void zero_pad_rows_kernel(T* __restrict__ out, int K, int Nreal, int 
     }
 }
 
-// ---- fp32 path: plain tiled FMA kernel, weights in the reference layout ------------------------------
-// C[rows of g] = epi(A[rows of g] @ W[g] (, A @ Wup[g])); 64x64 tiles, 16x16 threads, 4x4 per thread; K in slabs
-// of 64 through LDS, the next slab fetched into registers while the current one is multiplied (the workloads of
-// this path are small: what counts is that no memory latency is left exposed per slab).
-template <int EPI>
+// fp32 grouped GEMM (the plumbing workload's experts, and the fp32 gradients to rows): tiles of 32R x 32R rows and columns, four waves
+// of 16R x 16R each, on the fp32 matrix instruction (16x16x4; products and sums of one k after the other, k ascending, the
+// order of a scalar fmaf chain).  Weights in the reference layout [E_l][K][N].
+// Bound at the plumbing sizes (512 rows, K 256 / 512) by the length of its chain: load, LDS, matrix instructions, slab by slab, with few
+// workgroups in flight; hence the long slabs (R = 1: 128 of K, twice the loads under way) and small tiles (256 workgroups of
+// 32 x 32 where 64 x 64 gives 64).  On the vector units with 64 x 64 tiles the two GEMMs took 32 and 56 us, now 10 and 14.
+// R = 2 for launches of many tiles: every operand value out of LDS feeds two matrix instructions.
+// A in LDS as [row][k % 4][k / 4]: the four values a lane needs in four consecutive steps are one 16-byte read; B as
+// [k][column], rows padded so that the four k of a step lie in different banks.
+template <int EPI, int R>
 __global__ __launch_bounds__(256) void grouped_gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ Wt,
                                                                 const float* __restrict__ Wup, float* __restrict__ C,
                                                                 const int32_t* __restrict__ cnt, int E_l, int K, int N,
-                                                                int S_rows) {
-    constexpr int KC = 64;                       // K per slab
-    constexpr int PT = 64 * KC / 256;            // elements of each operand per thread and slab
-    __shared__ float As[KC][64 + 4];
-    __shared__ float Bs[KC][64];
-    __shared__ float Us[EPI == EPI_SWIGLU ? KC : 1][64];
+                                                                int S_rows, bool vec) {
+    constexpr int TM = 32 * R, KC = 128 / R, PT = TM * KC / 4 / 256;  // PT: 16-byte units of each operand per thread and slab
+    constexpr int PA = KC + 4, PB = TM + 16;
+    constexpr bool UP = EPI == EPI_SWIGLU;
+    __shared__ float As[TM * PA], Bs[KC * PB], Us[UP ? KC * PB : 1];
     __shared__ int s_g, s_row0, s_rv;
-    if (threadIdx.x == 0) {
-        int mt = blockIdx.y, rs = 0, g = 0, found = 0;
-        for (; g < E_l; ++g) {
-            const int c = max(cnt[g], 0);
-            const int t = (c + 63) / 64;
-            if (mt < t) { found = 1; s_row0 = rs + mt * 64; s_rv = min(min(64, c - mt * 64), S_rows - (rs + mt * 64)); break; }
-            mt -= t;
-            rs += c;
+    const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+    if (wave == 0) {  // which expert's rows: 64 experts at a time, tiles and rows before them by a scan
+        int mt = blockIdx.y, rs = 0;
+        if (lane == 0) s_g = -1;
+        for (int base = 0; base < E_l; base += WAVE) {
+            const int c = base + lane < E_l ? max(cnt[base + lane], 0) : 0, t = (c + TM - 1) / TM;
+            int tiles = t, rows = c;
+#pragma unroll
+            for (int off = 1; off < WAVE; off <<= 1) {
+                const int o = __shfl_up(tiles, off, WAVE), q = __shfl_up(rows, off, WAVE);
+                if (lane >= off) { tiles += o; rows += q; }
+            }
+            const bool mine = mt < tiles && mt >= tiles - t;
+            if (mine) {
+                const int first = (mt - (tiles - t)) * TM, row0 = rs + rows - c + first;
+                s_g = base + lane; s_row0 = row0; s_rv = min(min(TM, c - first), S_rows - row0);
+            }
+            if (__ballot(mine)) break;
+            mt -= __shfl(tiles, WAVE - 1, WAVE);
+            rs += __shfl(rows, WAVE - 1, WAVE);
         }
-        s_g = found ? g : -1;
     }
     __syncthreads();
     const int g = s_g;
     if (g < 0 || s_rv <= 0) return;
-    const int row0 = s_row0, rv = s_rv, n0 = blockIdx.x * 64;
+    const int row0 = s_row0, rv = s_rv, n0 = blockIdx.x * TM;
     const float* W = Wt + (size_t)g * K * N;
-    const float* U = EPI == EPI_SWIGLU ? Wup + (size_t)g * K * N : nullptr;
-    const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
-    float acc[4][4] = {}, acu[4][4] = {};
-    float ra[PT], rb[PT], ru[EPI == EPI_SWIGLU ? PT : 1];
+    const float* U = UP ? Wup + (size_t)g * K * N : nullptr;
+    float4 ra[PT], rb[PT], ru[UP ? PT : 1];
+    // (vec: K, N and the bases allow 16-byte loads, so a unit lies wholly inside or outside)
+    auto load = [&](const float* p, int at, int end) {
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (vec) {
+            if (at < end) v = *reinterpret_cast<const float4*>(p + at);
+        } else {
+            if (at < end) v.x = p[at];
+            if (at + 1 < end) v.y = p[at + 1];
+            if (at + 2 < end) v.z = p[at + 2];
+            if (at + 3 < end) v.w = p[at + 3];
+        }
+        return v;
+    };
     auto fetch = [&](int k0) {
 #pragma unroll
         for (int q = 0; q < PT; ++q) {
             const int i = threadIdx.x + q * 256;
-            const int r = i / KC, kk = i % KC;          // A: consecutive threads walk K
-            ra[q] = (r < rv && k0 + kk < K) ? A[(size_t)(row0 + r) * K + k0 + kk] : 0.f;
-            const int kb = i / 64, nn = i % 64;          // W: consecutive threads walk N
-            const bool ok = k0 + kb < K && n0 + nn < N;
-            rb[q] = ok ? W[(size_t)(k0 + kb) * N + n0 + nn] : 0.f;
-            if constexpr (EPI == EPI_SWIGLU) ru[q] = ok ? U[(size_t)(k0 + kb) * N + n0 + nn] : 0.f;
+            const int r = i / (KC / 4), k4 = i % (KC / 4);     // A: consecutive threads walk K
+            ra[q] = load(A + (size_t)(row0 + min(r, rv - 1)) * K, k0 + 4 * k4, r < rv ? K : 0);
+            const int kb = i / (TM / 4), n4 = i % (TM / 4);     // W: consecutive threads walk N
+            const size_t row = (size_t)min(k0 + kb, K - 1) * N;
+            const int end = k0 + kb < K ? N : 0;
+            rb[q] = load(W + row, n0 + 4 * n4, end);
+            if constexpr (UP) ru[q] = load(U + row, n0 + 4 * n4, end);
         }
     };
+    const int wm = (wave / 2) * 16 * R, wn = (wave % 2) * 16 * R, l16 = lane % 16, kg = lane / 16;
+    floatx4 acc[R][R] = {}, acu[UP ? R : 1][R] = {};
     fetch(0);
     for (int k0 = 0; k0 < K; k0 += KC) {
 #pragma unroll
         for (int q = 0; q < PT; ++q) {
             const int i = threadIdx.x + q * 256;
-            As[i % KC][i / KC] = ra[q];
-            Bs[i / 64][i % 64] = rb[q];
-            if constexpr (EPI == EPI_SWIGLU) Us[i / 64][i % 64] = ru[q];
+            float* a = As + (i / (KC / 4)) * PA + i % (KC / 4);
+            a[0] = ra[q].x; a[KC / 4] = ra[q].y; a[2 * (KC / 4)] = ra[q].z; a[3 * (KC / 4)] = ra[q].w;
+            const int b = (i / (TM / 4)) * PB + (i % (TM / 4)) * 4;
+            *reinterpret_cast<float4*>(Bs + b) = rb[q];
+            if constexpr (UP) *reinterpret_cast<float4*>(Us + b) = ru[q];
         }
         __syncthreads();
         if (k0 + KC < K) fetch(k0 + KC);
         // slab positions past K hold zeros: adding +0 products leaves every sum as it is
-#pragma unroll 8
-        for (int kk = 0; kk < KC; ++kk) {
-            float a[4], b[4];
+        const int steps = min(KC, K - k0 + 15) / 16;
+        for (int s4 = 0; s4 < steps; ++s4) {
+            floatx4 a[R];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) a[i] = As[kk][ty * 4 + i];
+            for (int i = 0; i < R; ++i) a[i] = *reinterpret_cast<const floatx4*>(As + (wm + 16 * i + l16) * PA + kg * (KC / 4) + 4 * s4);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) b[j] = Bs[kk][tx * 4 + j];
+            for (int u = 0; u < 4; ++u)
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+                for (int j = 0; j < R; ++j) {
+                    const int b = (16 * s4 + 4 * u + kg) * PB + wn + 16 * j + l16;
+                    const float bv = Bs[b], uv = UP ? Us[UP ? b : 0] : 0.f;
 #pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
-            if constexpr (EPI == EPI_SWIGLU) {
-                float u[4];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) u[j] = Us[kk][tx * 4 + j];
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) acu[i][j] = fmaf(a[i], u[j], acu[i][j]);
-            }
+                    for (int i = 0; i < R; ++i) {
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][u], bv, acc[i][j], 0, 0, 0);
+                        if constexpr (UP) acu[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][u], uv, acu[i][j], 0, 0, 0);
+                    }
+                }
         }
         __syncthreads();
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int r = ty * 4 + i;
-        if (r >= rv) continue;
+    for (int i = 0; i < R; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int c = n0 + tx * 4 + j;
-            if (c >= N) continue;
-            float x = acc[i][j];
-            if constexpr (EPI == EPI_GELU) x = act_gelu(x);
-            if constexpr (EPI == EPI_SILU) x = act_silu(x);
-            if constexpr (EPI == EPI_SWIGLU) x = act_silu(x) * acu[i][j];
-            C[(size_t)(row0 + r) * N + c] = x;
-        }
-    }
+        for (int j = 0; j < R; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int r = wm + 16 * i + 4 * kg + q, c = n0 + wn + 16 * j + l16;
+                if (r >= rv || c >= N) continue;
+                float x = acc[i][j][q];
+                if constexpr (EPI == EPI_GELU) x = act_gelu(x);
+                if constexpr (EPI == EPI_SILU) x = act_silu(x);
+                if constexpr (UP) x = act_silu(x) * acu[i][j][q];
+                C[(size_t)(row0 + r) * N + c] = x;
+            }
 }
 
 // ---- per-row fp8 quantisation of bf16 rows (one wave per row) -------------------------------------
@@ -1725,14 +1752,24 @@ int launch_gemm(const GemmParams& p_in, int epi, hipStream_t s, void* part_ws = 
 int launch_f32(const float* A, const float* W, const float* U, float* C, const int32_t* cnt, int E_l, int K, int N, int S_rows,
                int epi, hipStream_t s) {
     if (S_rows == 0) return MOE_OK;
-    dim3 grid(ceil_div(N, 64), ceil_div(S_rows, 64) + E_l);
+    const bool vec = K % 4 == 0 && N % 4 == 0 && (((uintptr_t)A | (uintptr_t)W | (uintptr_t)U) & 15) == 0;
+    // 64 x 64 tiles once they give every compute unit two workgroups, 32 x 32 below
+    const bool big = (long long)ceil_div(N, 64) * ceil_div(S_rows, 64) >= 2 * num_cus();
+    const int tile = big ? 64 : 32;
+    dim3 grid(ceil_div(N, tile), ceil_div(S_rows, tile) + E_l);
+#define GG_F32(EPI)                                                                                                                  \
+    case EPI:                                                                                                                        \
+        if (big) grouped_gemm_f32_kernel<EPI, 2><<<grid, 256, 0, s>>>(A, W, U, C, cnt, E_l, K, N, S_rows, vec);                      \
+        else grouped_gemm_f32_kernel<EPI, 1><<<grid, 256, 0, s>>>(A, W, U, C, cnt, E_l, K, N, S_rows, vec);                          \
+        break
     switch (epi) {
-        case EPI_NONE: grouped_gemm_f32_kernel<EPI_NONE><<<grid, 256, 0, s>>>(A, W, U, C, cnt, E_l, K, N, S_rows); break;
-        case EPI_GELU: grouped_gemm_f32_kernel<EPI_GELU><<<grid, 256, 0, s>>>(A, W, U, C, cnt, E_l, K, N, S_rows); break;
-        case EPI_SILU: grouped_gemm_f32_kernel<EPI_SILU><<<grid, 256, 0, s>>>(A, W, U, C, cnt, E_l, K, N, S_rows); break;
-        case EPI_SWIGLU: grouped_gemm_f32_kernel<EPI_SWIGLU><<<grid, 256, 0, s>>>(A, W, U, C, cnt, E_l, K, N, S_rows); break;
+        GG_F32(EPI_NONE);
+        GG_F32(EPI_GELU);
+        GG_F32(EPI_SILU);
+        GG_F32(EPI_SWIGLU);
         default: return moe_fail(MOE_ERR_INVALID, "grouped_gemm: activation %d", epi);
     }
+#undef GG_F32
     return moe_check_launch("grouped_gemm_f32");
 }
 

@@ -70,6 +70,28 @@ def test_grouped_gemm(dtype, E_l, K, N, S):
     assert (to_np(out)[S_tot:] == 0).all(), "rows past sum(cnt) must stay untouched"
 
 
+@pytest.mark.parametrize("act,H,F,S", [("silu", 20, 33, 70), ("swiglu", 127, 66, 65), ("gelu", 132, 260, 31),
+                                       ("swiglu", 260, 1100, 2300), ("gelu", 97, 1026, 3100)])
+def test_fp32_expert_at_tile_edges(act, H, F, S):
+    """Both tile sizes of the fp32 GEMM (32 x 32 for few tiles, 64 x 64 for many), rows, K and N that fill no tile, slab or 16-byte
+    unit, and an expert without rows."""
+    rng = np.random.default_rng(H + F)
+    E_l = 3
+    cnt = _groups(rng, E_l, S)
+    cnt[1] = 0
+    S_tot = int(cnt.sum())
+    x = _randn(rng, S_tot, H, dtype="f32")
+    w1, w2 = _randn(rng, E_l, H, F, scale=H ** -0.5, dtype="f32"), _randn(rng, E_l, F, H, scale=F ** -0.5, dtype="f32")
+    wu = _randn(rng, E_l, H, F, scale=H ** -0.5, dtype="f32") if act == "swiglu" else None
+    c = torch.from_numpy(cnt).to(DEV)
+    hid = ops.grouped_gemm(_t(x, "f32"), _t(w1, "f32"), c)
+    _check(to_np(hid), O.grouped_gemm(x, w1, cnt, "f32").astype(np.float64), F32_RTOL, F32_ATOL, "fp32 GEMM")
+    if H % 4 == 0 and F % 4 == 0:
+        ew = ExpertWeights.prepare(act, _t(w1, "f32"), _t(w2, "f32"), None if wu is None else _t(wu, "f32"))
+        y = expert_mlp(_t(x, "f32"), ew, c)
+        _check(to_np(y), O.expert_mlp(x, cnt, w1, w2, act, "f32", w_up=wu).astype(np.float64), F32_RTOL, F32_ATOL, "fp32 MLP")
+
+
 def test_grouped_gemm_identity_is_exact():
     """Identity / one-hot weights: the GEMM must reproduce (permute) its input bit for bit."""
     rng = np.random.default_rng(3)
