@@ -412,6 +412,31 @@ int moe_diag_mfma_loop(int fp8, int random_data, int iters, int workgroups, floa
 size_t moe_diag_gemm_trace_words(void);
 int moe_diag_gemm_trace(unsigned long long* trace, size_t words, int flags);
 
+/* ---- the exchange of a simulated world, and what the shuffle has to know on the host ---------------------------------
+ * moe_a2a_place: what arrives at `rank` when every source sends its padding-free payload (the reference's custom_a2a moves these
+ *   rows between GPUs, layers/all_to_all.py:10-125): sources[s] (host array of W; payload NULL: sends nothing) gives the payload
+ *   [rows,H] of rank s, its counts for this rank [E_l] and where its block for this rank starts (one int32 in device memory).
+ *   token_buf [E_l,W,CAP,H] <- row block start + (rows of the experts before e) + j of source s at [e,s,j], zeros
+ *   past its count; pca[e,s] = counts; counts_ready / token_sync (n_ready / n_sync int32 each, nullable) <- W.
+ *   If a count exceeds CAP nothing is written.
+ * moe_a2a_max_count: *max_count (device-writable, e.g. pinned host memory) <- the largest count of moe_a2a_place, 0 if none.
+ * moe_shuffle_totals: out[0] <- sum of pca (n entries), out[1] <- smallest of token_sync (n_sync entries; 2^31 - 1 if none);
+ *   out device-writable, e.g. pinned host memory. */
+typedef struct moe_a2a_source {
+    const void* payload;
+    const int32_t* counts;
+    const int32_t* start;
+    long long rows;
+} moe_a2a_source;
+int moe_a2a_max_count(const moe_a2a_source* sources /* host */, int W, int E_l, int32_t* max_count, moe_stream_t stream);
+int moe_a2a_place(const moe_a2a_source* sources /* host */, int dtype, int W, int E_l, int CAP, int H, void* token_buf, int32_t* pca,
+                  int32_t* counts_ready, int n_ready, int32_t* token_sync, int n_sync, moe_stream_t stream);
+int moe_shuffle_totals(const int32_t* pca, int n, const int32_t* token_sync, int n_sync, int32_t* out, moe_stream_t stream);
+/* moe_expert_forward: moe_grouped_gemm_mapped without maps or activation on `packed`, with the rows of out past the counted
+ * total zeroed (the caller's out needs no clearing). */
+int moe_expert_forward(const void* tokens, const void* packed, const int32_t* expert_cnt, int S_rows, int K, int N, int E_l, void* out,
+                       void* part_ws, size_t part_ws_bytes, moe_stream_t stream);
+
 /* ---- the whole hot path of one step as one call -------------------------------------------------------------------
  * What rank 0 does for one batch (route, count, pack; row map, expert MLP, return; combine), through the entry points above
  * with the arguments named alike there; only enqueues, as they do.  Modes: fused = the GEMMs gather from / scatter into the transfer

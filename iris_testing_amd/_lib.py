@@ -39,6 +39,11 @@ class StepArgs(ctypes.Structure):
         "ret_map part_ws part_ws_bytes ret returned zero_off out").split()]
 
 
+class A2aSource(ctypes.Structure):
+    """moe_a2a_source of include/moe_gfx950.h."""
+    _fields_ = [("payload", c_void_p), ("counts", c_void_p), ("start", c_void_p), ("rows", ctypes.c_longlong)]
+
+
 P = c_void_p
 _SIGNATURES = {
     "moe_abi_version": (c_int, []),
@@ -94,6 +99,10 @@ _SIGNATURES = {
     "moe_gemm_split_plan": (c_int, [c_int, c_int, c_int, c_int, P]),
     "moe_zero_padding_rows": (c_int, [P, c_int, c_int, c_int, c_int, P, c_int, P]),
     "moe_recv_prepare": (c_int, [P, c_int, c_int, c_int, c_int, P, P, P, P, P, P, P, c_int, c_int, P]),
+    "moe_a2a_max_count": (c_int, [POINTER(A2aSource), c_int, c_int, P, P]),
+    "moe_a2a_place": (c_int, [POINTER(A2aSource), c_int, c_int, c_int, c_int, c_int, P, P, P, c_int, P, c_int, P]),
+    "moe_shuffle_totals": (c_int, [P, c_int, P, c_int, P, P]),
+    "moe_expert_forward": (c_int, [P, P, P, c_int, c_int, c_int, c_int, P, P, c_size_t, P]),
     "moe_step": (c_int, [POINTER(StepArgs), P]),
     "moe_grouped_mlp_fp8_mapped": (c_int, [P, c_int, P, P, c_int, c_int, c_int, c_int, P, P, P, P, P, P, P, P, P, P, P, c_int, P, P,
                                            c_size_t, P]),  # (.., xq_ws, xs_ws, hq_ws, hscale_ws, row_gate, out, out_rows, ..)
@@ -142,7 +151,8 @@ def ptr(t) -> int:
 
 
 def stream_ptr() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """The current stream of the current device (0.2 us; through a torch.cuda.Stream object it is 3 us, a fifth of a call)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def dtype_code(dt: torch.dtype) -> int:

@@ -806,6 +806,88 @@ int check_rows(const char* who, int dtype, int H) {
     return MOE_OK;
 }
 
+// The exchange of a simulated world (moe_a2a_place), up to A2A_SRC sources to a launch (their pointers travel as kernel
+// arguments).  A workgroup makes the tables of its sources in LDS, then its waves copy or zero rows (e, s, j) of token_buf.
+constexpr int A2A_SRC = 64;
+struct A2aSources {
+    moe_a2a_source src[A2A_SRC];
+};
+__device__ __forceinline__ int a2a_count(const moe_a2a_source& q, int e) { return q.payload ? max(q.counts[e], 0) : 0; }
+
+__global__ __launch_bounds__(256) void a2a_max_count_kernel(const A2aSources q, int ns, int E_l, int32_t* __restrict__ out, bool first) {
+    __shared__ int32_t most;
+    if (threadIdx.x == 0) most = first ? 0 : *out;
+    __syncthreads();
+    for (int i = threadIdx.x; i < ns * E_l; i += blockDim.x) {
+        const int c = a2a_count(q.src[i / E_l], i % E_l);
+        if (c > 0) atomicMax(&most, c);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) *out = most;
+}
+
+__global__ __launch_bounds__(256) void a2a_place_kernel(const A2aSources q, int s0, int ns, int W, int E_l, int CAP, int row_vec,
+                                                         u32x4* __restrict__ token_buf, int32_t* __restrict__ pca,
+                                                         int32_t* __restrict__ counts_ready, int n_ready,
+                                                         int32_t* __restrict__ token_sync, int n_sync) {
+    __shared__ int32_t cnt[MOE_MAX_EXPERTS], off[MOE_MAX_EXPERTS], most;
+    const int tid = threadIdx.x, lane = lane_id();
+    if (tid == 0) most = 0;
+    __syncthreads();
+    for (int i = tid; i < ns * E_l; i += blockDim.x) {
+        const int c = a2a_count(q.src[i / E_l], i % E_l);
+        cnt[i] = c;
+        if (c > CAP) atomicMax(&most, c);
+    }
+    __syncthreads();
+    if (most > CAP) return;
+    for (int s = tid; s < ns; s += blockDim.x) {
+        int r = q.src[s].payload ? *q.src[s].start : 0;
+        for (int e = 0; e < E_l; ++e) { off[s * E_l + e] = r; r += cnt[s * E_l + e]; }
+    }
+    if (blockIdx.x == 0) {
+        for (int i = tid; i < ns * E_l; i += blockDim.x) pca[(i % E_l) * W + s0 + i / E_l] = cnt[i];
+        for (int i = tid; i < n_ready; i += blockDim.x) counts_ready[i] = W;
+        for (int i = tid; i < n_sync; i += blockDim.x) token_sync[i] = W;
+    }
+    __syncthreads();
+    const int n_rows = E_l * ns * CAP, wpb = blockDim.x / WAVE;
+    for (int r = blockIdx.x * wpb + tid / WAVE; r < n_rows; r += gridDim.x * wpb) {
+        const int j = r % CAP, s = r / CAP % ns, e = r / CAP / ns;
+        u32x4* d = token_buf + (((size_t)e * W + s0 + s) * CAP + j) * row_vec;
+        const long long at = (long long)off[s * E_l + e] + j;
+        if (j < cnt[s * E_l + e] && at >= 0 && at < q.src[s].rows) {
+            const u32x4* src = (const u32x4*)q.src[s].payload + (size_t)at * row_vec;
+            int c = lane;
+            for (; c + 3 * WAVE < row_vec; c += 4 * WAVE) {
+                u32x4 v[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) v[u] = __builtin_nontemporal_load(src + c + u * WAVE);
+#pragma unroll
+                for (int u = 0; u < 4; ++u) d[c + u * WAVE] = v[u];
+            }
+            for (; c < row_vec; c += WAVE) d[c] = __builtin_nontemporal_load(src + c);
+        } else {
+            const u32x4 z = {0u, 0u, 0u, 0u};
+            for (int c = lane; c < row_vec; c += WAVE) d[c] = z;
+        }
+    }
+}
+
+__global__ __launch_bounds__(256) void shuffle_totals_kernel(const int32_t* __restrict__ pca, int n, const int32_t* __restrict__ sync,
+                                                              int n_sync, int32_t* __restrict__ out) {
+    __shared__ int32_t sum, least;
+    if (threadIdx.x == 0) { sum = 0; least = 0x7fffffff; }
+    __syncthreads();
+    int s = 0, m = 0x7fffffff;
+    for (int i = threadIdx.x; i < n; i += blockDim.x) s += pca[i];
+    for (int i = threadIdx.x; i < n_sync; i += blockDim.x) m = min(m, sync[i]);
+    atomicAdd(&sum, s);
+    atomicMin(&least, m);
+    __syncthreads();
+    if (threadIdx.x == 0) { out[0] = sum; out[1] = least; }
+}
+
 }  // namespace
 
 extern "C" size_t moe_count_workspace_bytes(int T, int k, int E) {
@@ -1077,8 +1159,9 @@ extern "C" int moe_zero_padding_rows(void* buf, int dtype, int W, int M, int H, 
 
 extern "C" int moe_shuffle(const void* token_buf, int dtype, int E_l, int W, int CAP, int H, const int32_t* pca,
                            void* shuffled, int S_rows, int32_t* expert_cnt, int32_t* map_ws, moe_stream_t stream) {
+    (void)map_ws;
     hipStream_t s = (hipStream_t)stream;
-    MOE_REQUIRE(W > 0 && E_l > 0 && W * E_l <= MOE_MAX_EXPERTS && CAP >= 1 && S_rows >= 0 && pca && map_ws,
+    MOE_REQUIRE(W > 0 && E_l > 0 && W * E_l <= MOE_MAX_EXPERTS && CAP >= 1 && S_rows >= 0 && pca,
                 MOE_ERR_INVALID, "shuffle: bad arguments");
     // (pca[e,s] = recv_counts[s,e])
     return recv_driven("shuffle", SRC_SHUFFLE, token_buf, shuffled, dtype, H, {pca, 1, W, nullptr, expert_cnt}, W, E_l, 1, CAP, S_rows,
@@ -1088,8 +1171,9 @@ extern "C" int moe_shuffle(const void* token_buf, int dtype, int E_l, int W, int
 // gradient of moe_shuffle: grad_token_buf[e,s,j,:] = grad_rows[off[e,s] + j,:] for j < pca[e,s], zeros elsewhere
 extern "C" int moe_shuffle_backward(const void* grad_rows, int dtype, int E_l, int W, int CAP, int H, const int32_t* pca,
                                     void* grad_token_buf, int32_t* map_ws, moe_stream_t stream) {
+    (void)map_ws;
     hipStream_t s = (hipStream_t)stream;
-    MOE_REQUIRE(W > 0 && E_l > 0 && W * E_l <= MOE_MAX_EXPERTS && CAP >= 1 && pca && map_ws, MOE_ERR_INVALID,
+    MOE_REQUIRE(W > 0 && E_l > 0 && W * E_l <= MOE_MAX_EXPERTS && CAP >= 1 && pca, MOE_ERR_INVALID,
                 "shuffle_backward: bad arguments");
     MOE_REQUIRE((long long)E_l * W * CAP < (1ll << 31), MOE_ERR_UNSUPPORTED, "shuffle_backward: too many rows");
     return recv_driven("shuffle_backward", SRC_UNSHUFFLE, grad_rows, grad_token_buf, dtype, H, {pca, 1, W, nullptr, nullptr}, W, E_l, 1, CAP,
@@ -1149,4 +1233,52 @@ extern "C" int moe_combine(const void* ret, int dtype, int W, int M, int H, cons
     const int row_vec = H * dtype_size(dtype) / 16;
     if (dtype == MOE_F32) return launch_combine<float>(ret, topk_idx, pos, gate, dst_offsets, T, k, E_l, W, M, row_vec, out, status, s);
     return launch_combine<bf16_t>(ret, topk_idx, pos, gate, dst_offsets, T, k, E_l, W, M, row_vec, out, status, s);
+}
+
+// ---- the exchange of a simulated world -----------------------------------------------------------
+static int a2a_check(const char* who, const moe_a2a_source* src, int W, int E_l) {
+    MOE_REQUIRE(src && W > 0 && E_l > 0 && W * E_l <= MOE_MAX_EXPERTS, MOE_ERR_INVALID, "%s: bad W=%d E_l=%d", who, W, E_l);
+    for (int s = 0; s < W; ++s)
+        MOE_REQUIRE(!src[s].payload || (src[s].counts && src[s].start && src[s].rows >= 0), MOE_ERR_INVALID, "%s: source %d is incomplete",
+                    who, s);
+    return MOE_OK;
+}
+static A2aSources a2a_slice(const moe_a2a_source* src, int s0, int ns) {
+    A2aSources q{};
+    for (int i = 0; i < ns; ++i) q.src[i] = src[s0 + i];
+    return q;
+}
+
+extern "C" int moe_a2a_max_count(const moe_a2a_source* sources, int W, int E_l, int32_t* max_count, moe_stream_t stream) {
+    const int rc = a2a_check("a2a_max_count", sources, W, E_l);
+    if (rc) return rc;
+    MOE_REQUIRE(max_count, MOE_ERR_INVALID, "a2a_max_count: null pointer");
+    for (int s0 = 0; s0 < W; s0 += A2A_SRC) {
+        const int ns = min(A2A_SRC, W - s0);
+        a2a_max_count_kernel<<<1, 256, 0, (hipStream_t)stream>>>(a2a_slice(sources, s0, ns), ns, E_l, max_count, s0 == 0);
+    }
+    return moe_check_launch("a2a_max_count");
+}
+
+extern "C" int moe_a2a_place(const moe_a2a_source* sources, int dtype, int W, int E_l, int CAP, int H, void* token_buf, int32_t* pca,
+                             int32_t* counts_ready, int n_ready, int32_t* token_sync, int n_sync, moe_stream_t stream) {
+    int rc = a2a_check("a2a_place", sources, W, E_l);
+    if (!rc) rc = check_rows("a2a_place", dtype, H);
+    if (rc) return rc;
+    MOE_REQUIRE(CAP >= 1 && (long long)E_l * W * CAP < (1ll << 31), MOE_ERR_UNSUPPORTED, "a2a_place: CAP=%d", CAP);
+    MOE_REQUIRE(token_buf && pca, MOE_ERR_INVALID, "a2a_place: null pointer");
+    for (int s0 = 0; s0 < W; s0 += A2A_SRC) {
+        const int ns = min(A2A_SRC, W - s0);
+        const int blocks = min(ceil_div(E_l * ns * CAP, 4), 256 * 8);
+        a2a_place_kernel<<<blocks, 256, 0, (hipStream_t)stream>>>(a2a_slice(sources, s0, ns), s0, ns, W, E_l, CAP, H * dtype_size(dtype) / 16,
+                                                                  (u32x4*)token_buf, pca, counts_ready, counts_ready && !s0 ? n_ready : 0,
+                                                                  token_sync, token_sync && !s0 ? n_sync : 0);
+    }
+    return moe_check_launch("a2a_place");
+}
+
+extern "C" int moe_shuffle_totals(const int32_t* pca, int n, const int32_t* token_sync, int n_sync, int32_t* out, moe_stream_t stream) {
+    MOE_REQUIRE(n >= 0 && n_sync >= 0 && out && (n == 0 || pca) && (n_sync == 0 || token_sync), MOE_ERR_INVALID, "shuffle_totals: bad arguments");
+    shuffle_totals_kernel<<<1, 256, 0, (hipStream_t)stream>>>(pca, n, token_sync, n_sync, out);
+    return moe_check_launch("shuffle_totals");
 }

@@ -1902,6 +1902,18 @@ extern "C" int moe_grouped_gemm_mapped(const void* a_base, int a_rows, const int
     return launch_gemm<false>(p, act, (hipStream_t)stream, part_ws, part_ws_bytes);
 }
 
+extern "C" int moe_expert_forward(const void* tokens, const void* packed, const int32_t* expert_cnt, int S_rows, int K, int N, int E_l,
+                                  void* out, void* part_ws, size_t part_ws_bytes, moe_stream_t stream) {
+    MOE_REQUIRE(S_rows >= 0 && K > 0 && N > 0 && E_l > 0 && E_l <= GG_MAXG, MOE_ERR_INVALID, "expert_forward: bad shape");
+    MOE_REQUIRE(K % 64 == 0 && N % 8 == 0, MOE_ERR_UNSUPPORTED, "expert_forward: needs K %% 64 == 0 and N %% 8 == 0 (K=%d N=%d)", K, N);
+    if (S_rows == 0) return MOE_OK;
+    MOE_REQUIRE(tokens && packed && expert_cnt && out, MOE_ERR_INVALID, "expert_forward: null pointer");
+    GemmParams p{};
+    p.A = (const uint8_t*)tokens; p.B = (const uint8_t*)packed; p.C = out; p.cnt = expert_cnt; p.zero_tail = 1;
+    p.E_l = E_l; p.K = K; p.N = N; p.ldc = N; p.S_rows = S_rows; p.Npad = round_up(N, GG_BN);
+    return launch_gemm<false>(p, EPI_NONE, (hipStream_t)stream, part_ws, part_ws_bytes);
+}
+
 extern "C" int moe_grouped_gemm_mapped_gated(const void* a_base, int a_rows, const int32_t* a_row_map, const void* packed,
                                              const int32_t* expert_cnt, int S_rows, int K, int N, int E_l, const float* row_gate,
                                              void* out, int out_rows, const int32_t* c_row_map, void* part_ws, size_t part_ws_bytes,

@@ -4,8 +4,9 @@ The reference's operator moves rows between GPUs with Iris puts (kernels.py:21-1
 inter-GPU transfer is not part of a one-GPU build; what is kept is the operator's contract: the
 10-argument signature, the in-place fill of ``local_pca`` / ``token_buf`` / the two completion
 counters, and the returned ``token_buf``.  The sends of the other simulated ranks are supplied
-through a ``SimulatedWorld``; placing the rows ([E_local, world, CAP, H], zero padded) is done by
-the HIP reorder kernel.
+through a ``SimulatedWorld``; one HIP kernel gathers the rows from all of them into place ([E_local, world, CAP, H], zero
+padded), with the counts and counters.  The host waits once, for the largest count (a kernel of its own in front leaves
+it in pinned memory), because an overflow raises.
 """
 from __future__ import annotations
 
@@ -63,27 +64,43 @@ class AllToAllOp(torch.autograd.Function):
         world.post(rank, tokens, dest_counts, dst_offsets)
 
         # what each source sends to `rank`: rows [dst_offsets[rank], +sum(dest_counts[rank,:]))
-        parts, counts = [], torch.zeros((world_size, e_local), dtype=torch.int32, device=tokens.device)
-        for src in range(world_size):
-            if src not in world.sends:
-                continue
-            p, dc, do = world.sends[src]
-            n = int(dc[rank].sum().item())
-            o = int(do[rank].item())
-            parts.append(p[o:o + n])
-            counts[src] = dc[rank]
-        flat = torch.cat(parts, dim=0) if parts else tokens[:0]
-        over = int(counts.max().item()) if counts.numel() else 0
+        sends, shape, where = [None] * world_size, (world_size, e_local), (tokens.device, torch.int32)
+        for src, (p, dc, do) in world.sends.items():
+            assert p.shape[1:] == tokens.shape[1:] and dc.shape == shape and do.numel() == world_size, "sends of different shapes"
+            # (as posted they are usually what the kernels read; otherwise a converted copy)
+            if p.dtype != tokens.dtype or not (p.is_cuda and p.is_contiguous()):
+                p = p.to(tokens.device, tokens.dtype).contiguous()
+            if dc.dtype != torch.int32 or not (dc.is_cuda and dc.is_contiguous()):
+                dc = dc.to(*where).contiguous()
+            if do.dtype != torch.int32 or not (do.is_cuda and do.is_contiguous()):
+                do = do.to(*where).contiguous()
+            sends[src] = (p, dc, do)
+        want = (e_local, world_size, capacity, tokens.shape[-1])
+        block, most = ops.a2a_sources(sends, rank), ops.pinned_i32(1)
+        fits = tuple(token_buf.shape) == want and token_buf.dtype == tokens.dtype
+        ops.a2a_max_count(block, e_local, most)
+        known = torch.cuda.Event()
+        known.record()
+        try:
+            if fits:  # (writes nothing if a count exceeds the capacity; the host learns of that while the rows move)
+                pca = local_pca if local_pca.is_contiguous() else torch.empty_like(local_pca, memory_format=torch.contiguous_format)
+                ready, sync = (t if t.dtype == torch.int32 and t.is_cuda and t.is_contiguous() else None for t in (counts_ready, token_sync))
+                ops.a2a_place(block, token_buf, pca, ready, sync)
+        finally:
+            known.synchronize()
+        over = int(most[0])
         if over > capacity:
             raise ValueError(f"capacity overflow: a (src, expert) pair sends {over} rows > CAP={capacity}")
-        if tuple(token_buf.shape) != (e_local, world_size, capacity, tokens.shape[-1]):
+        if not fits:
             raise ValueError(f"token_buf shape {tuple(token_buf.shape)} mismatch expected "
-                             f"({e_local},{world_size},{capacity},{tokens.shape[-1]}).")
-        ops.reorder_flat(flat.contiguous(), counts, capacity, token_buf)
-        local_pca.copy_(counts.t())
+                             f"({e_local},{world_size},{capacity},{tokens.shape[-1]}) of {tokens.dtype}.")
+        if pca is not local_pca:
+            local_pca.copy_(pca)
         # completion counters in their final state: every source has signalled (all_to_all.py:59-69)
-        counts_ready.fill_(world_size)
-        token_sync.fill_(world_size)
+        if ready is None:
+            counts_ready.fill_(world_size)
+        if sync is None:
+            token_sync.fill_(world_size)
         return token_buf
 
     @staticmethod

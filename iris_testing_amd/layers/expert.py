@@ -60,14 +60,10 @@ def _packed_weights_t(w: torch.Tensor, w_up: Optional[torch.Tensor] = None) -> t
 
 def _grouped_gemm_t(do: torch.Tensor, weights: torch.Tensor, cnt: torch.Tensor) -> torch.Tensor:
     """d tokens[rows of g] = do[rows of g] @ weights[g]^T; rows past sum(cnt) are zero."""
-    E_l, K, N = weights.shape
-    S = do.shape[0]
+    K = weights.shape[1]
     if do.dtype == torch.float32:
         return ops.grouped_gemm(do, ops.transpose_weights_f32(weights.contiguous()), cnt)
-    out = torch.zeros((S, K), dtype=do.dtype, device=do.device)
-    if S:
-        ops.grouped_gemm_mapped(do, None, _packed_weights_t(weights), cnt, S, K, "none", out, part_ws=_part_ws(do.device))
-    return out
+    return ops.expert_forward(do, _packed_weights_t(weights), cnt, K, _part_ws(do.device))
 
 
 def _part_ws(device) -> torch.Tensor:
@@ -82,12 +78,7 @@ def _grouped_gemm(tokens: torch.Tensor, weights: torch.Tensor, cnt: torch.Tensor
     """out[rows of g] = tokens[rows of g] @ weights[g]; rows past sum(cnt) are zero."""
     if tokens.dtype != torch.bfloat16 or weights.shape[1] % 64 or weights.shape[2] % 8:  # (what the MFMA kernel covers)
         return ops.grouped_gemm(tokens, weights, cnt)
-    S, N = tokens.shape[0], weights.shape[2]
-    out = torch.zeros((S, N), dtype=tokens.dtype, device=tokens.device)
-    if S:
-        ops.grouped_gemm_mapped(tokens, None, _packed_weights(weights), cnt, S, N, "none", out,
-                                part_ws=_part_ws(tokens.device))
-    return out
+    return ops.expert_forward(tokens, _packed_weights(weights), cnt, weights.shape[2], _part_ws(tokens.device))
 
 
 class Expert(torch.autograd.Function):

@@ -19,13 +19,19 @@ class TokenShuffle(torch.autograd.Function):
         assert dispatched_tokens.is_cuda, "dispatched_tokens must be CUDA"
         _assert_cuda_int32(pca, "pca")
         e_local, world_size = pca.shape
-        if token_sync is not None:
-            # the reference kernel spins until token_sync[e] >= world_size (kernels.py:192); on one
-            # GPU the data is either complete or never will be, so an incomplete counter is an error
-            if int(token_sync.min().item()) < world_size:
-                raise RuntimeError("token_sync shows an incomplete transfer (expected >= world_size)")
-        total = int(pca.sum().item())
-        out, _ = ops.shuffle_rows(dispatched_tokens.contiguous(), pca.contiguous(), total)
+        pca_c = pca.contiguous()
+        # the row count sizes the result, so the host has to wait for it: one kernel leaves it in pinned memory, with the state
+        # of the transfer
+        totals = ops.pinned_i32(2)
+        sync = None if token_sync is None else token_sync.to(pca.device, torch.int32).contiguous()
+        ops.shuffle_totals(pca_c, sync, totals)
+        torch.cuda.current_stream().synchronize()
+        total, done = totals.tolist()
+        # the reference kernel spins until token_sync[e] >= world_size (kernels.py:192); on one
+        # GPU the data is either complete or never will be, so an incomplete counter is an error
+        if sync is not None and done < world_size:
+            raise RuntimeError("token_sync shows an incomplete transfer (expected >= world_size)")
+        out, _ = ops.shuffle_rows(dispatched_tokens.contiguous(), pca_c, total)
         ctx.save_for_backward(pca)
         ctx.capacity = dispatched_tokens.shape[2]
         return out

@@ -6,6 +6,7 @@ unless the caller passes them in.
 """
 from __future__ import annotations
 
+import math
 from dataclasses import dataclass
 from typing import Optional, Tuple
 
@@ -26,6 +27,18 @@ def _req_i32(t: torch.Tensor, name: str) -> None:
 
 def _i32(n, device) -> torch.Tensor:
     return torch.empty(n, dtype=torch.int32, device=device)
+
+
+def _i32_parts(device, *shapes):
+    """Contiguous int32 tensors of these shapes in one allocation, each at a multiple of 16 bytes (a view costs half of what an
+    allocation does)."""
+    sizes = [math.prod(sh) for sh in shapes]
+    buf = _i32(sum(-(-n // 4) * 4 for n in sizes), device)
+    out, at = [], 0
+    for sh, n in zip(shapes, sizes):
+        out.append(buf.as_strided(sh, (sh[1], 1) if len(sh) == 2 else (1,), at))
+        at += -(-n // 4) * 4
+    return out
 
 
 # ---- a1 -------------------------------------------------------------------------------------
@@ -71,8 +84,7 @@ def count_and_offsets(topk_idx: torch.Tensor, num_experts_total: int, world_size
     E, W = num_experts_total, world_size
     dev = topk_idx.device
     e_l = E // W
-    out = Counts(_i32((W, e_l), dev), _i32((W, e_l), dev), _i32((W,), dev), _i32((W,), dev), _i32((2,), dev),
-                 _i32((T, k), dev), _i32((T * k,), dev))
+    out = Counts(*_i32_parts(dev, (W, e_l), (W, e_l), (W,), (W,), (2,)), *_i32_parts(dev, (T, k), (T * k,)))
     nbytes = L.lib().moe_count_workspace_bytes(T, k, E)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
     L.check(L.lib().moe_count_and_offsets(L.ptr(topk_idx), T, k, E, W, L.ptr(out.send_counts), L.ptr(out.expert_offs),
@@ -187,14 +199,6 @@ def pack_tokens_fp8(x: torch.Tensor, topk_idx: torch.Tensor, pos: torch.Tensor, 
 
 
 # ---- a9 / a10 -------------------------------------------------------------------------------
-def _map_ws(W, E_l, n_out, device, map_ws=None):
-    need = L.lib().moe_recv_map_ints(W, E_l, n_out)
-    if map_ws is None:
-        return _i32((need,), device)
-    assert map_ws.dtype == torch.int32 and map_ws.numel() >= need and map_ws.is_cuda
-    return map_ws
-
-
 def unpack_token_buf(recv: torch.Tensor, recv_counts: torch.Tensor, capacity: int,
                      token_buf: Optional[torch.Tensor] = None, pca: Optional[torch.Tensor] = None,
                      status: Optional[torch.Tensor] = None, map_ws=None) -> Tuple[torch.Tensor, torch.Tensor]:
@@ -211,9 +215,8 @@ def unpack_token_buf(recv: torch.Tensor, recv_counts: torch.Tensor, capacity: in
         raise ValueError(f"token_buf shape {tuple(token_buf.shape)} mismatch expected ({E_l},{W},{capacity},{H}).")
     if pca is None:
         pca = _i32((E_l, W), dev)
-    ws = _map_ws(W, E_l, E_l * W * capacity, dev, map_ws)
     L.check(L.lib().moe_unpack_token_buf(L.ptr(recv), L.dtype_code(recv.dtype), W, M, H, L.ptr(recv_counts), E_l,
-                                         capacity, L.ptr(token_buf), L.ptr(pca), L.ptr(ws), L.ptr(status),
+                                         capacity, L.ptr(token_buf), L.ptr(pca), None, L.ptr(status),
                                          L.stream_ptr()))
     return token_buf, pca
 
@@ -224,9 +227,8 @@ def reorder_flat(flat: torch.Tensor, recv_counts: torch.Tensor, capacity: int, t
     _req_i32(recv_counts, "recv_counts")
     R, H = flat.shape
     W, E_l = recv_counts.shape
-    ws = _map_ws(W, E_l, E_l * W * capacity, flat.device)
     L.check(L.lib().moe_reorder_flat_to_token_buf(L.ptr(flat), L.dtype_code(flat.dtype), R, H, L.ptr(recv_counts), W,
-                                                  E_l, capacity, L.ptr(token_buf), L.ptr(ws), L.ptr(status),
+                                                  E_l, capacity, L.ptr(token_buf), None, L.ptr(status),
                                                   L.stream_ptr()))
     return token_buf
 
@@ -242,10 +244,65 @@ def shuffle_rows(token_buf: torch.Tensor, pca: torch.Tensor, S_rows: int, out: O
         out = torch.empty((S_rows, H), dtype=token_buf.dtype, device=dev)
     if expert_cnt is None:
         expert_cnt = _i32((E_l,), dev)
-    ws = _map_ws(W, E_l, S_rows, dev, map_ws)
     L.check(L.lib().moe_shuffle(L.ptr(token_buf), L.dtype_code(token_buf.dtype), E_l, W, CAP, H, L.ptr(pca), L.ptr(out),
-                                S_rows, L.ptr(expert_cnt), L.ptr(ws), L.stream_ptr()))
+                                S_rows, L.ptr(expert_cnt), None, L.stream_ptr()))
     return out, expert_cnt
+
+
+def pinned_i32(n: int) -> torch.Tensor:
+    """n int32 in pinned host memory, which kernels write directly: read it after waiting for them (one wait, no copy)."""
+    return torch.empty(n, dtype=torch.int32, pin_memory=True)
+
+
+def a2a_sources(sends, rank: int):
+    """The argument block of a2a_max_count / a2a_place for ``rank`` (it only points into the tensors).  sends: per source rank None
+    or (payload [R,H], counts int32 [W,E_l], dst_offsets int32 [W]), contiguous and on the device."""
+    block = (L.A2aSource * len(sends))()
+    for q, send in zip(block, sends):
+        if send is not None and send[0].shape[0]:
+            payload, counts, starts = send
+            q.payload, q.rows = payload.data_ptr(), payload.shape[0]
+            q.counts, q.start = counts.data_ptr() + 4 * rank * counts.shape[1], starts.data_ptr() + 4 * rank
+    return block
+
+
+def a2a_max_count(block, e_local: int, out: torch.Tensor) -> None:
+    """out[0] (pinned or device int32) <- the largest count of any (source, expert)."""
+    L.check(L.lib().moe_a2a_max_count(block, len(block), e_local, L.ptr(out), L.stream_ptr()))
+
+
+def a2a_place(block, token_buf: torch.Tensor, pca: torch.Tensor, counts_ready: Optional[torch.Tensor],
+              token_sync: Optional[torch.Tensor]) -> None:
+    """The exchange of a simulated world into token_buf [E_l,W,CAP,H], with the counts and the completed counters."""
+    _req_cuda(token_buf, "token_buf")
+    for t, n in ((pca, "local_pca"), (counts_ready, "counts_ready"), (token_sync, "token_sync")):
+        if t is not None:
+            _req_i32(t, n)
+    E_l, W, CAP, H = token_buf.shape
+    assert W == len(block) and pca.shape == (E_l, W)
+    L.check(L.lib().moe_a2a_place(block, L.dtype_code(token_buf.dtype), W, E_l, CAP, H, L.ptr(token_buf), L.ptr(pca), L.ptr(counts_ready),
+                                  0 if counts_ready is None else counts_ready.numel(), L.ptr(token_sync),
+                                  0 if token_sync is None else token_sync.numel(), L.stream_ptr()))
+
+
+def shuffle_totals(pca: torch.Tensor, token_sync: Optional[torch.Tensor], out: torch.Tensor) -> None:
+    """out[0], out[1] (pinned or device int32) <- sum of pca, smallest of token_sync."""
+    _req_i32(pca, "pca")
+    if token_sync is not None:
+        _req_i32(token_sync, "token_sync")
+    L.check(L.lib().moe_shuffle_totals(L.ptr(pca), pca.numel(), L.ptr(token_sync), 0 if token_sync is None else token_sync.numel(),
+                                       L.ptr(out), L.stream_ptr()))
+
+
+def expert_forward(tokens: torch.Tensor, packed: torch.Tensor, expert_cnt: torch.Tensor, N: int, part_ws: torch.Tensor) -> torch.Tensor:
+    """out[rows of e] = tokens[rows of e] @ w[e] for bf16 rows and re-tiled weights; rows past the counted total are zero."""
+    _req_cuda(tokens, "tokens")
+    _req_i32(expert_cnt, "local_expert_cnt")
+    S, K = tokens.shape
+    out = torch.empty((S, N), dtype=tokens.dtype, device=tokens.device)
+    L.check(L.lib().moe_expert_forward(L.ptr(tokens), L.ptr(packed), L.ptr(expert_cnt), S, K, N, expert_cnt.numel(), L.ptr(out),
+                                       L.ptr(part_ws), part_ws.numel() * part_ws.element_size(), L.stream_ptr()))
+    return out
 
 
 def shuffle_rows_backward(grad_rows: torch.Tensor, pca: torch.Tensor, capacity: int) -> torch.Tensor:
@@ -255,9 +312,8 @@ def shuffle_rows_backward(grad_rows: torch.Tensor, pca: torch.Tensor, capacity: 
     E_l, W = pca.shape
     H = grad_rows.shape[1]
     out = torch.empty((E_l, W, capacity, H), dtype=grad_rows.dtype, device=grad_rows.device)
-    ws = _map_ws(W, E_l, 0, grad_rows.device)
     L.check(L.lib().moe_shuffle_backward(L.ptr(grad_rows), L.dtype_code(grad_rows.dtype), E_l, W, capacity, H, L.ptr(pca),
-                                         L.ptr(out), L.ptr(ws), L.stream_ptr()))
+                                         L.ptr(out), None, L.stream_ptr()))
     return out
 
 
@@ -273,9 +329,8 @@ def unpack_expert_major(recv: torch.Tensor, recv_counts: torch.Tensor, S_rows: i
         out = torch.empty((S_rows, H), dtype=recv.dtype, device=dev)
     if expert_cnt is None:
         expert_cnt = _i32((E_l,), dev)
-    ws = _map_ws(W, E_l, S_rows, dev, map_ws)
     L.check(L.lib().moe_unpack_expert_major(L.ptr(recv), L.dtype_code(recv.dtype), W, M, H, L.ptr(recv_counts), E_l,
-                                            L.ptr(out), S_rows, L.ptr(expert_cnt), L.ptr(ws), L.stream_ptr()))
+                                            L.ptr(out), S_rows, L.ptr(expert_cnt), None, L.stream_ptr()))
     return out, expert_cnt
 
 
@@ -431,9 +486,8 @@ def return_pack(y: torch.Tensor, recv_counts: torch.Tensor, M: int, out: Optiona
     W, E_l = recv_counts.shape
     if out is None:
         out = torch.empty((W, M, H), dtype=y.dtype, device=y.device)
-    ws = _map_ws(W, E_l, W * M, y.device, map_ws)
     L.check(L.lib().moe_return_pack(L.ptr(y), L.dtype_code(y.dtype), S, H, L.ptr(recv_counts), W, E_l, M, L.ptr(out),
-                                    L.ptr(ws), L.stream_ptr()))
+                                    None, L.stream_ptr()))
     return out
 
 
@@ -449,8 +503,7 @@ def recv_row_map(recv_counts: torch.Tensor, M: int, n_rows: int, row_map: Option
         row_map = _i32((max(n_rows, 1),), dev)
     if expert_cnt is None:
         expert_cnt = _i32((E_l,), dev)
-    ws = _map_ws(W, E_l, n_rows, dev, map_ws)
-    L.check(L.lib().moe_recv_row_map(L.ptr(recv_counts), W, E_l, M, n_rows, L.ptr(row_map), L.ptr(expert_cnt), L.ptr(ws),
+    L.check(L.lib().moe_recv_row_map(L.ptr(recv_counts), W, E_l, M, n_rows, L.ptr(row_map), L.ptr(expert_cnt), None,
                                      L.stream_ptr()))
     return row_map, expert_cnt
 

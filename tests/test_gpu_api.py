@@ -88,6 +88,49 @@ def test_custom_a2a_uniform_pattern(e_local, hidden_dim, cap):
                    bufs.token_sync, None, experts + 1, cap)
 
 
+@pytest.mark.parametrize("W,e_local,H,cap", [(2, 1, 8, 1), (4, 15, 520, 7), (70, 3, 2056, 5)])
+def test_custom_a2a_ragged_world(W, e_local, H, cap):
+    """Ragged and empty blocks, a silent source, more sources than one launch takes; an overflow raises and writes nothing."""
+    rng = np.random.default_rng(W)
+    counts = rng.integers(0, cap + 1, size=(W, W, e_local)).astype(np.int32)  # [src, dst, e]
+    counts[0, 0, 0], counts[-1] = cap, 0
+    rank, silent = W // 2, 0 if W > 2 else None
+    world, rows = SimulatedWorld(W, rank=rank), {}
+    for s in range(W):
+        sizes = counts[s].sum(1)
+        start = (np.cumsum(sizes) - sizes).astype(np.int32)
+        rows[s] = torch.randn((int(sizes.sum()), H), device=DEV).bfloat16()
+        if s != silent:
+            world.post(s, rows[s], torch.from_numpy(counts[s]).to(DEV), torch.from_numpy(start).to(DEV))
+    bufs = utils.alloc_shmem_buffers(None, W, e_local, cap, H, torch.bfloat16)
+    bufs.token_buf.fill_(9.0)
+    want_pca = counts[:, rank].T.copy()
+    if silent is not None:
+        want_pca[:, silent] = 0
+    args = lambda c: (*world.sends[rank], bufs.pca, bufs.token_buf[:, :, :c], bufs.counts_ready, bufs.token_sync,  # noqa: E731
+                      bufs.heap_bases, e_local * W, c)
+    with simulated_world(world):
+        if want_pca.max() == cap and cap > 1:
+            small = bufs.token_buf[:, :, : cap - 1].contiguous()
+            with pytest.raises(ValueError, match="capacity overflow"):
+                custom_a2a(*world.sends[rank], bufs.pca, small, bufs.counts_ready, bufs.token_sync, None, e_local * W, cap - 1)
+            assert W > 64 or (small == 9.0).all()
+        custom_a2a(*args(cap))
+    assert_bits_equal(bufs.pca, want_pca, "pca")
+    assert int(bufs.counts_ready) == W and (bufs.token_sync == W).all()
+    want = torch.zeros_like(bufs.token_buf)
+    for s in range(W):
+        sizes = counts[s].sum(1)
+        at = int((np.cumsum(sizes) - sizes)[rank])
+        for e in range(e_local):
+            n = int(want_pca[e, s])
+            want[e, s, :n] = rows[s][at:at + n]
+            at += int(counts[s, rank, e])
+    assert torch.equal(bufs.token_buf, want)
+    assert torch.equal(shuffle(bufs.token_buf, bufs.pca, bufs.token_sync),
+                       torch.cat([want[e, s, : int(want_pca[e, s])] for e in range(e_local) for s in range(W)]))
+
+
 def test_reorder_flat_to_token_buf_and_errors():
     rng = np.random.default_rng(0)
     W, E_l, H, CAP = 4, 3, 32, 9
