@@ -478,26 +478,34 @@ static int gs_dispatch(const GsParams& q, int bm, int epi, void* ws, size_t byte
 
 // Tile height for a launch (32 or 64 rows), or 0: large tiles.  Both paths' times in us are estimated from what the host knows
 // -- the row total, not its split over the groups (every group adds about half a tile of ragged tail) -- with coefficients
-// fitted to 90 launches drawn over rows 16 .. 16384, 1 .. 32 groups, K and N 512 .. 8192, bf16 and fp8, even and skewed:
-//   large tiles: rounds of the persistent grid, each 0.70 us (256 rows) or 0.45 us (128 rows) per 64 bytes of K, 4 us between
-//     tiles, 14 us for a launch with its K-split and reduction launches;
-//   small tiles: 0.26 / 0.29 us per 128 bytes of K while every workgroup has a compute unit to itself, then in proportion to
-//     their number (times 1.2, fp8 1.4: the load path is shared); 5 us for the hand-over of a split tile.
-// Over those launches the choice made from these estimates is within 2 % (geometric mean) of the better of the two, and 1.4 times
-// faster than large tiles alone: 27.5 -> 9.0 us at 512 rows x 1024 x 1024 (2 groups, bf16), 31 -> 21 us at 512 x 2048 x 4096,
-// 49 -> 20 us for an fp8 MLP of 300 rows; the line lies at one to two rounds of large tiles.
+// fitted to 490 launches drawn over rows 16 .. 16384, 1 .. 32 groups, K and N 512 .. 8192, bf16 and fp8, even and skewed:
+//   large tiles: whole rounds of the persistent grid, each 0.70 us (256 rows) or 0.40 us (128 rows) per 64 bytes of K (fp8 a fifth
+//     more) and 4 us between tiles; the tiles of the last, part-filled round split along K as far as there are
+//     compute units, at 12 us for its two launches; 10 us for the launch;
+//   small tiles: 0.24 / 0.30 us per 128 bytes of K while every workgroup has a compute unit to itself, then in proportion to
+//     their number (times 1.2, fp8 1.4: the load path is shared); 5 us for the hand-over of a split tile, 8 us for the launch.
+// Over those launches the choice made from these estimates is within 1 % (geometric mean) of the better of the two, 1.31 times
+// faster than large tiles alone and in one launch of 490 more than 7 % slower than them: 27.5 -> 9.0 us at 512 rows x 1024 x 1024
+// (2 groups, bf16), 31 -> 21 us at 512 x 2048 x 4096, 49 -> 20 us for an fp8 MLP of 300 rows; the line lies at about one round of
+// large tiles.
 int gs_choose_bm(int S_rows, int E_l, int K, int ncols, bool fp8, int cus) {
     const double E = std::min(E_l, S_rows), nk = (double)K * (fp8 ? 1 : 2) / ROWB;
     const int nt = (ncols + GG_BN - 1) / GG_BN, nts = (ncols + GS_BN - 1) / GS_BN;
-    const double r256 = ceil((S_rows / 256.0 + 0.5 * E) * nt / cus), r128 = ceil((S_rows / 128.0 + 0.5 * E) * nt / cus);
-    const bool small_m = 0.62 * r128 < r256;
-    double best = 14 + (small_m ? r128 : r256) * (nk * (small_m ? 0.45 : 0.70) + 4);
+    const double t256 = (S_rows / 256.0 + 0.5 * E) * nt, t128 = (S_rows / 128.0 + 0.5 * E) * nt;
+    const bool small_m = 0.62 * ceil(t128 / cus) < ceil(t256 / cus);
+    const double tiles = small_m ? t128 : t256, tile_us = nk * (small_m ? 0.40 : 0.70) * (fp8 ? 1.2 : 1.0);
+    const double full = floor(tiles / cus), rem = tiles - full * cus;
+    double best = 9.5 + full * (tile_us + 3.9);
+    if (rem > 0.5) {
+        const double P = std::max(1.0, std::min(std::min(floor(cus / rem), 8.0), floor(nk / 16)));
+        best += tile_us / P + 4.2 + (P > 1 ? 11.9 : 0);
+    }
     int bm_best = 0;
     for (int bm : {32, 64}) {
         const double units = (S_rows / (double)bm + 0.5 * E) * nts;
         const double P = units < cus ? std::max(1.0, std::min(std::min(floor(cus / units), floor(nk / GS_MIN_PART_STAGES)), (double)GG_MAX_PARTS)) : 1.0;
-        const double x = units * P / cus, share = x <= 1 ? 1.0 : std::max(1.0, x * (fp8 ? 1.4 : 1.2));
-        const double t = 6 + (P > 1 ? 5 : 0) + nk / 2 / P * (bm == 32 ? 0.26 : 0.29) * share + 2 * std::max(1.0, x / 2);
+        const double x = units * P / cus;
+        const double t = 8.3 + (P > 1 ? 5 : 0) + nk / 2 / P * (bm == 32 ? 0.24 : 0.30) * std::max(1.0, x * (fp8 ? 1.4 : 1.225)) + 1.8 * std::max(1.0, x / 2);
         if (t < best) { best = t; bm_best = bm; }
     }
     return bm_best;
