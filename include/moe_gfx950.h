@@ -29,6 +29,7 @@ extern "C" {
 typedef void* moe_stream_t; /* hipStream_t */
 
 enum { MOE_F32 = 0, MOE_BF16 = 1 };
+enum { MOE_W_TILED = 0, MOE_W_RAW = 1, MOE_W_RAW_T = 2 }; /* weights: re-tiled for the kernels, as they are, as they are and transposed */
 enum { MOE_ACT_NONE = 0, MOE_ACT_GELU = 1, MOE_ACT_SILU = 2, MOE_ACT_SWIGLU = 3 };
 enum {
     MOE_OK = 0,
@@ -348,21 +349,21 @@ int moe_grouped_gemm_dw(const void* x, const void* dy, const int32_t* expert_cnt
 /* moe_grouped_gemm_dw with split_F = F whose halves go to two matrices of their own, dw_gate and dw_up [E_l,K,F] (bf16). */
 int moe_grouped_gemm_dw_pair(const void* x, const void* dy, const int32_t* expert_cnt, int S_rows, int K, int F, int E_l,
                              void* dw_gate, void* dw_up, moe_stream_t stream);
-/* moe_prepack_weights and moe_prepack_weights_transposed in one pass over the weight (K and N multiples of 64, bf16). */
-int moe_prepack_weights_both(const void* w, const void* w_up, int dtype, int E_l, int K, int N, void* packed, void* packed_t,
-                             moe_stream_t stream);
 /* The expert MLP of a training step, one call per direction (bf16; H and F multiples of 64; act GELU, SiLU or SwiGLU; the
  * reference's backward, layers/expert.py:62-64, is an empty stub).
- * forward:  hidden [S,F] = act(x w1), pre_act as moe_grouped_gemm_act_keep, out [S,H] = hidden w2; w1 / w2 packed.
+ * forward:  hidden [S,F] = act(x w1), pre_act as moe_grouped_gemm_act_keep, out [S,H] = hidden w2.  layout MOE_W_TILED: w1 / w2
+ * re-tiled (w_up NULL); MOE_W_RAW: w1, w_up (SwiGLU) [E_l,H,F] and w2 [E_l,F,H] as they are.
  * backward: dh [S,F] and d_pre (layout of pre_act) are scratch; dx [S,H], dw1 / dw_up [E_l,H,F] (dw_up: SwiGLU only), dw2
- * [E_l,F,H]; w1_t / w2_t as moe_prepack_weights_transposed makes them.
+ * [E_l,F,H].  layout MOE_W_RAW_T: w1, w_up, w2 in the reference layout; MOE_W_TILED: w1 (of the pair) and w2 as
+ * moe_prepack_weights_transposed makes them (w_up NULL).
  * Rows of out and dx past the counted total are zeroed. */
-int moe_mlp_train_forward(const void* x, const int32_t* expert_cnt, int S_rows, int H, int F, int E_l, int act, const void* w1,
-                          const void* w2, void* hidden, void* pre_act, void* out, void* part_ws, size_t part_ws_bytes,
-                          moe_stream_t stream);
+int moe_mlp_train_forward(const void* x, const int32_t* expert_cnt, int S_rows, int H, int F, int E_l, int act, int layout,
+                          const void* w1, const void* w_up, const void* w2, void* hidden, void* pre_act, void* out, void* part_ws,
+                          size_t part_ws_bytes, moe_stream_t stream);
 int moe_mlp_train_backward(const void* x, const void* hidden, const void* pre_act, const void* dy, const int32_t* expert_cnt,
-                           int S_rows, int H, int F, int E_l, int act, const void* w1_t, const void* w2_t, void* dh, void* d_pre,
-                           void* dx, void* dw1, void* dw_up, void* dw2, void* part_ws, size_t part_ws_bytes, moe_stream_t stream);
+                           int S_rows, int H, int F, int E_l, int act, int layout, const void* w1, const void* w_up, const void* w2,
+                           void* dh, void* d_pre, void* dx, void* dw1, void* dw_up, void* dw2, void* part_ws, size_t part_ws_bytes,
+                           moe_stream_t stream);
 int moe_transpose_weights_f32(const float* w, int E_l, int K, int N, float* out, moe_stream_t stream);
 int moe_mlp_act_backward(const void* a1, const void* dh, int dtype, int rows, int F, int act, void* d_a1,
                          moe_stream_t stream);
@@ -432,10 +433,11 @@ int moe_a2a_max_count(const moe_a2a_source* sources /* host */, int W, int E_l, 
 int moe_a2a_place(const moe_a2a_source* sources /* host */, int dtype, int W, int E_l, int CAP, int H, void* token_buf, int32_t* pca,
                   int32_t* counts_ready, int n_ready, int32_t* token_sync, int n_sync, moe_stream_t stream);
 int moe_shuffle_totals(const int32_t* pca, int n, const int32_t* token_sync, int n_sync, int32_t* out, moe_stream_t stream);
-/* moe_expert_forward: moe_grouped_gemm_mapped without maps or activation on `packed`, with the rows of out past the counted
- * total zeroed (the caller's out needs no clearing). */
-int moe_expert_forward(const void* tokens, const void* packed, const int32_t* expert_cnt, int S_rows, int K, int N, int E_l, void* out,
-                       void* part_ws, size_t part_ws_bytes, moe_stream_t stream);
+/* moe_expert_forward: out[rows of g] = tokens[rows of g] @ w[g] (bf16) with the rows of out past the counted total zeroed (the
+ * caller's out needs no clearing).  layout MOE_W_TILED: weights as moe_prepack_weights makes them of [E_l,K,N]; MOE_W_RAW: [E_l,K,N]
+ * as they are; MOE_W_RAW_T: [E_l,N,K] as they are (out = tokens w^T). */
+int moe_expert_forward(const void* tokens, const void* weights, int layout, const int32_t* expert_cnt, int S_rows, int K, int N, int E_l,
+                       void* out, void* part_ws, size_t part_ws_bytes, moe_stream_t stream);
 
 /* ---- the whole hot path of one step as one call -------------------------------------------------------------------
  * What rank 0 does for one batch (route, count, pack; row map, expert MLP, return; combine), through the entry points above

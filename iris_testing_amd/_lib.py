@@ -15,6 +15,7 @@ LIB_PATH = os.path.join(_HERE, "csrc", "libmoe_gfx950.so")
 
 MOE_F32, MOE_BF16 = 0, 1
 ACT = {"none": 0, "gelu": 1, "silu": 2, "swiglu": 3}
+W_TILED, W_RAW, W_RAW_T = 0, 1, 2  # weight layouts: re-tiled, as they are, as they are and transposed
 MOE_MAX_EXPERTS = 512
 MOE_MAX_TOPK = 16
 
@@ -90,9 +91,8 @@ _SIGNATURES = {
     "moe_dw_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int]),
     "moe_grouped_gemm_dw": (c_int, [P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, P, P, c_size_t, P]),
     "moe_grouped_gemm_dw_pair": (c_int, [P, P, P, c_int, c_int, c_int, c_int, P, P, P]),
-    "moe_prepack_weights_both": (c_int, [P, P, c_int, c_int, c_int, c_int, P, P, P]),
-    "moe_mlp_train_forward": (c_int, [P, P, c_int, c_int, c_int, c_int, c_int, P, P, P, P, P, P, c_size_t, P]),
-    "moe_mlp_train_backward": (c_int, [P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, P, P, P, P, P, P, P, P, P, c_size_t, P]),
+    "moe_mlp_train_forward": (c_int, [P, P, c_int, c_int, c_int, c_int, c_int, c_int, P, P, P, P, P, P, P, c_size_t, P]),
+    "moe_mlp_train_backward": (c_int, [P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int, P, P, P, P, P, P, P, P, P, P, c_size_t, P]),
     "moe_transpose_weights_f32": (c_int, [P, c_int, c_int, c_int, P, P]),
     "moe_mlp_act_backward": (c_int, [P, P, c_int, c_int, c_int, c_int, P, P]),
     "moe_combine_backward": (c_int, [P, P, c_int, c_int, c_int, c_int, P, P, P, P, P, c_int, c_int, c_int, P, P, P]),
@@ -102,7 +102,7 @@ _SIGNATURES = {
     "moe_a2a_max_count": (c_int, [POINTER(A2aSource), c_int, c_int, P, P]),
     "moe_a2a_place": (c_int, [POINTER(A2aSource), c_int, c_int, c_int, c_int, c_int, P, P, P, c_int, P, c_int, P]),
     "moe_shuffle_totals": (c_int, [P, c_int, P, c_int, P, P]),
-    "moe_expert_forward": (c_int, [P, P, P, c_int, c_int, c_int, c_int, P, P, c_size_t, P]),
+    "moe_expert_forward": (c_int, [P, P, c_int, P, c_int, c_int, c_int, c_int, P, P, c_size_t, P]),
     "moe_step": (c_int, [POINTER(StepArgs), P]),
     "moe_grouped_mlp_fp8_mapped": (c_int, [P, c_int, P, P, c_int, c_int, c_int, c_int, P, P, P, P, P, P, P, P, P, P, P, c_int, P, P,
                                            c_size_t, P]),  # (.., xq_ws, xs_ws, hq_ws, hscale_ws, row_gate, out, out_rows, ..)

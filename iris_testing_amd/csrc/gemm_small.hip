@@ -63,8 +63,10 @@ __device__ __forceinline__ int gs_scan(int v) {
     return v;
 }
 
-template <int BM, bool FP8, int EPI, bool BSA>
+template <int BM, bool FP8, int EPI, bool BSA, int BMODE>
 __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParams q) {
+    constexpr bool BT = BMODE == GG_B_T, BN_PAIR = BMODE == GG_B_NP, BN_RAW = BMODE == GG_B_N || BN_PAIR;  // (see GG_B_*)
+    static_assert(!FP8 || BMODE == GG_B_PACKED, "raw weights are a bf16 matter");
     using S = GsShape<BM>;
     constexpr int ES = FP8 ? 1 : 2;
     constexpr int MT = FP8 ? 32 : 16, CF = FP8 ? 2 : 1;
@@ -140,8 +142,17 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
     const int lchunk = (lane & 3) ^ ((lane >> 4) & 3);
     const uint32_t ldk = (uint32_t)(p.K * ES);
     const uint8_t* Ab = (p.a_map ? p.A : p.A + (size_t)row0 * ldk) + (size_t)ks0 * ROWB;
-    const size_t b_slab = (size_t)p.Npad * ROWB;
-    const uint8_t* Bb = p.B + (size_t)g * p.Npad * ldk + (size_t)nt * GS_BN * ROWB + (size_t)ks0 * b_slab;
+    // weights: bytes from one stage to the next, from the start of the tensor to the tile's first stage, and (not re-tiled) of a tensor
+    [[maybe_unused]] const bool pair = p.B2 != nullptr;
+    [[maybe_unused]] const uint32_t ldb = BT ? (uint32_t)(pair ? p.K / 2 : p.K) * 2u : (uint32_t)p.N * 2u;
+    [[maybe_unused]] const size_t b_group = (size_t)p.K / (BT && pair ? 2 : 1) * p.N * 2;
+    [[maybe_unused]] const ptrdiff_t b2_delta = p.B2 - p.B;
+    const size_t b_slab = BT ? (size_t)ROWB : BN_RAW ? (size_t)32 * ldb : (size_t)p.Npad * ROWB;
+    const size_t b_at = BT ? (size_t)g * b_group + (size_t)nt * GS_BN * ldb + (size_t)ks0 / (pair ? 2 : 1) * ROWB
+                      : BN_RAW ? (size_t)g * b_group + (size_t)nt * (BN_PAIR ? GS_BN : 2 * GS_BN) + (size_t)ks0 * b_slab
+                               : (size_t)g * p.Npad * ldk + (size_t)nt * GS_BN * ROWB + (size_t)ks0 * b_slab;
+    const uint8_t* Bb = p.B + b_at;
+    [[maybe_unused]] const long long b_left = (long long)p.E_l * b_group - (long long)b_at;
     uint32_t aoff[RA], boff[RB];
 #pragma unroll
     for (int r = 0; r < RA; ++r) {
@@ -150,7 +161,15 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
         aoff[r] = (uint32_t)(p.a_map ? max(p.a_map[row0 + lr], 0) : lr) * ldk + lchunk * 16;
     }
 #pragma unroll
-    for (int r = 0; r < RB; ++r) boff[r] = (uint32_t)(r * 64 + wave * WROWS + (lane >> 2)) * ROWB + lchunk * 16;
+    for (int r = 0; r < RB; ++r) {
+        if constexpr (BT) boff[r] = (uint32_t)gg_packed_col<false>(r * 64 + wave * WROWS + (lane >> 2)) * ldb + lchunk * 16;
+        // BN_RAW: a stage is 32 rows of 256 bytes, four to a 1 KB load, chunk c of row k at position c ^ 4 (k % 4); a pair: 32 rows of
+        // 128 bytes of either matrix, eight to a load, chunk c at position c ^ 4 (k / 2 % 2)
+        else if constexpr (BN_PAIR) boff[r] = (uint32_t)(8 * wave + (lane >> 3)) * ldb + (uint32_t)((lane & 7) ^ (4 * ((lane >> 4) & 1))) * 16u;
+        else if constexpr (BN_RAW) boff[r] = (uint32_t)(4 * (r * 4 + wave) + (lane >> 4)) * ldb + (uint32_t)((lane & 15) ^ (4 * (lane >> 4))) * 16u;
+        else boff[r] = (uint32_t)(r * 64 + wave * WROWS + (lane >> 2)) * ROWB + lchunk * 16;
+    }
+    static_assert(!BN_RAW || RB == 2, "two loads per wave and stage");
     uint8_t* const sA = lds;
     uint8_t* const sB = lds + NST * 2 * ASZ;
     uint32_t* const sS = (uint32_t*)(lds + NST * 2 * (ASZ + BSZ)) + wave * NST * 64;  // (BSA) the wave's scale dwords, one per row
@@ -161,17 +180,25 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
 
     const int npair = nks / 2;
     // load d (0 .. LPS - 1) of the pair whose first stage lies at ap / bp: activations, weights, (BSA) scale dwords
-    auto load = [&](int d, const uint8_t* ap, const uint8_t* bp, const uint8_t* sp, int slot) {
+    // (bp[stage][matrix of a pair])
+    typedef typename std::conditional<BMODE == GG_B_PACKED, const uint8_t*, gg_i32x4>::type bsrc_t;
+    auto load = [&](int d, const uint8_t* ap, const bsrc_t (&bp)[2][2], const uint8_t* sp, int slot) {
         if (d < 2 * RA) gg_dma16(ap + (d & 1) * ROWB, aoff[d >> 1], la0 + slot * 2 * ASZ + (d & 1) * ASZ + (d >> 1) * 64 * ROWB);
         else if (d < 2 * (RA + RB)) {
             const int e = d - 2 * RA;
-            gg_dma16(bp + (e / RB) * b_slab, boff[e % RB], lb0 + slot * 2 * BSZ + (e / RB) * BSZ + (e % RB) * 64 * ROWB);
+            gg_dma16(bp[e / RB][BN_PAIR ? e % RB : 0], boff[e % RB], lb0 + slot * 2 * BSZ + (e / RB) * BSZ + (e % RB) * 64 * ROWB);
         } else if constexpr (BSA) gg_dma4(sp, soff, ls0 + slot * 256);
     };
 #define GS_PAIR_PTRS(pr)                                                    \
     const int st_ = 2 * min((pr), npair - 1);                               \
     const uint8_t* ap_ = gg_uniform(Ab + (size_t)st_ * ROWB);               \
-    const uint8_t* bp_ = gg_uniform(Bb + (size_t)st_ * b_slab);             \
+    bsrc_t bp_[2][2];                                                       \
+    _Pragma("unroll") for (int u_ = 0; u_ < 2; ++u_)                         \
+        _Pragma("unroll") for (int m_ = 0; m_ < (BN_PAIR ? 2 : 1); ++m_) {   \
+            const size_t so_ = BT && pair ? (size_t)(st_ >> 1) * ROWB : (size_t)(st_ + u_) * b_slab; \
+            if constexpr (BMODE == GG_B_PACKED) bp_[u_][m_] = gg_uniform(Bb + so_);                  \
+            else bp_[u_][m_] = gg_range((BN_PAIR ? m_ : BT && pair && u_) ? Bb + b2_delta + so_ : Bb + so_, b_left - (long long)so_); \
+        }                                                                   \
     const uint8_t* sp_ = BSA ? gg_uniform(p.a_bscale + (((ks0 + st_) >> 1) << 2)) : nullptr;
 
     typedef typename std::conditional<FP8, floatx16, floatx4>::type acc_t;
@@ -189,6 +216,18 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
     const int fpos = (FP8 ? (lane >> 5) : (lane >> 4)) ^ ((lane >> 2) & 3);
     const uint4* fa = (const uint4*)sA + (wm * S::WR + (lane & (MT - 1))) * CHUNKS;
     const uint4* fb = (const uint4*)sB + (wn * S::WC + (lane & (MT - 1))) * CHUNKS;
+    // (BN_RAW) LDS address of the lane's part of the first of the two fragments of each group of 32 columns (see gg_read_tr)
+    constexpr int BTR = BN_PAIR ? 128 : 256;
+    [[maybe_unused]] uint32_t trb[TN > 1 ? TN / 2 : 1];
+    if constexpr (BN_RAW) {
+        const int kq = (lane >> 4) * 8 + ((lane & 15) >> 2), k4 = (lane & 15) >> 2, q4 = lane & 3;
+#pragma unroll
+        for (int h = 0; h < TN / 2; ++h) {
+            const int grp = wn * (S::WC / 32) + h;
+            trb[h] = (uint32_t)(uintptr_t)(lds_ptr_t)sB + kq * BTR +
+                     (BN_PAIR ? (grp & 1) * (BSZ / 2) + ((((grp >> 1) * 4 + q4) ^ (4 * (k4 >> 1))) * 16) : (((grp * 4 + q4) ^ (4 * k4)) * 16));
+        }
+    }
     struct Frag {
         uint4 a[2][TM][CF], b[2][TN][CF];
         uint32_t sc[TM];
@@ -199,9 +238,16 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
             const uint4* as = fa + (slot * 2 + u) * (ASZ / 16);
             const uint4* bs = fb + (slot * 2 + u) * (BSZ / 16);
 #pragma unroll
-            for (int j = 0; j < TN; ++j)
+            for (int j = 0; j < TN; ++j) {
+                if constexpr (BN_RAW) {
+                    const uint32_t at = trb[j >> 1] + (slot * 2 + u) * BSZ + (j & 1) * 8;
+                    const uint2 lo = gg_read_tr<BTR>(at, 0), hi = gg_read_tr<BTR>(at, 1);
+                    f.b[u][j][0] = make_uint4(lo.x, lo.y, hi.x, hi.y);
+                } else {
 #pragma unroll
-                for (int h = 0; h < CF; ++h) f.b[u][j][h] = bs[j * MT * CHUNKS + (fpos ^ (2 * h))];
+                    for (int h = 0; h < CF; ++h) f.b[u][j][h] = bs[j * MT * CHUNKS + (fpos ^ (2 * h))];
+                }
+            }
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -434,7 +480,7 @@ static unsigned long long gs_nonce() {
     return (base + n.fetch_add(1, std::memory_order_relaxed)) & ((1ull << 56) - 1);
 }
 
-template <int BM, bool FP8, int EPI, bool BSA>
+template <int BM, bool FP8, int EPI, bool BSA, int BMODE>
 static void gs_launch(const GsParams& q0, void* part_ws, size_t part_ws_bytes, int cus, hipStream_t s) {
     GsParams q = q0;
     constexpr int lds = gs_lds_bytes<BM, BSA>();
@@ -450,19 +496,28 @@ static void gs_launch(const GsParams& q0, void* part_ws, size_t part_ws_bytes, i
     const long long ub = ((long long)q.g.S_rows + (long long)std::min(q.g.E_l, q.g.S_rows) * (BM - 1)) / BM * nt;  // most tiles there can be
     const long long units = std::max<long long>(ub, q.g.part_ws ? std::min<long long>(q.slots, ub * GG_MAX_PARTS) : 0);
     q.nonce = gs_nonce();
-    gemm_small_kernel<BM, FP8, EPI, BSA><<<(unsigned)((units + 7) / 8 * 8), GS_THREADS, lds, s>>>(q);
+    gemm_small_kernel<BM, FP8, EPI, BSA, BMODE><<<(unsigned)((units + 7) / 8 * 8), GS_THREADS, lds, s>>>(q);
 }
 
 template <bool FP8>
 static int gs_dispatch(const GsParams& q, int bm, int epi, void* ws, size_t bytes, int cus, hipStream_t s) {
-#define GS_BM(EPIv, BSAv)                                                              \
+#define GS_MODE(EPIv, BSAv, MODEv)                                                     \
     do {                                                                               \
-        if (bm == 32) gs_launch<32, FP8, EPIv, BSAv>(q, ws, bytes, cus, s);            \
-        else gs_launch<64, FP8, EPIv, BSAv>(q, ws, bytes, cus, s);                     \
+        if (bm == 32) gs_launch<32, FP8, EPIv, BSAv, MODEv>(q, ws, bytes, cus, s);     \
+        else gs_launch<64, FP8, EPIv, BSAv, MODEv>(q, ws, bytes, cus, s);              \
     } while (0)
+#define GS_BM(EPIv, BSAv) GS_MODE(EPIv, BSAv, GG_B_PACKED)
     if constexpr (FP8) {
         if (epi == EPI_NONE) GS_BM(EPI_NONE, true);
         else GS_BM(EPI_SWIGLU, false);
+    } else if (q.g.b_mode != GG_B_PACKED) {  // weights in the reference layout
+        const int mode = q.g.b_mode;
+        if (mode == GG_B_T && epi == EPI_NONE) GS_MODE(EPI_NONE, false, GG_B_T);
+        else if (mode == GG_B_N && epi == EPI_NONE) GS_MODE(EPI_NONE, false, GG_B_N);
+        else if (mode == GG_B_N && epi == EPI_GELU) GS_MODE(EPI_GELU, false, GG_B_N);
+        else if (mode == GG_B_N && epi == EPI_SILU) GS_MODE(EPI_SILU, false, GG_B_N);
+        else if (mode == GG_B_NP && epi == EPI_SWIGLU) GS_MODE(EPI_SWIGLU, false, GG_B_NP);
+        else return moe_fail(MOE_ERR_INVALID, "grouped_gemm: weight mode %d with activation %d", mode, epi);
     } else {
         switch (epi) {
             case EPI_NONE: GS_BM(EPI_NONE, false); break;
@@ -473,6 +528,7 @@ static int gs_dispatch(const GsParams& q, int bm, int epi, void* ws, size_t byte
         }
     }
 #undef GS_BM
+#undef GS_MODE
     return moe_check_launch("grouped_gemm");
 }
 

@@ -18,7 +18,9 @@ constexpr int GG_BN = 256;
 
 struct GemmParams {
     const uint8_t* A;         // [S_rows, K] activations (bf16 or fp8)
-    const uint8_t* B;         // packed weights [E_l, Npad, K]
+    const uint8_t* B;         // packed weights [E_l, Npad, K]; or (b_mode) weights in the reference layout, see GgB
+    const uint8_t* B2;        // the second matrix of a gate / up pair (GG_B_NP; GG_B_T with a pair, else NULL)
+    int b_mode;
     void* C;                  // [S_rows, ldc] bf16
     void* C2;                 // optional (bf16 kernels with an activation): the values BEFORE the activation, bf16, row pitch ldc
                               // (SwiGLU: 2 ldc, in the packed gate / up column order), kept for the backward pass
@@ -59,6 +61,22 @@ struct GemmParams {
     unsigned long long* trace;
     int trace_flags;
 };
+// How a kernel takes its weight operand (template parameter; the rows below are those of [E_l, rows, columns] bf16 tensors in the
+// reference layout, read as they are -- for weights that change from call to call, whose re-tiling would cost more than it saves):
+//   GG_B_PACKED  re-tiled (moe_prepack_weights): a K stage of a tile is one contiguous piece
+//   GG_B_DW      the weight-gradient mode (see dw_rows): columns are output columns, the rows of a group are the reduction
+//   GG_B_T       out = a w^T: rows are output columns, columns the reduction, 64 bytes of 256 rows to a stage, like an activation
+//                operand; with B2 the stages alternate between B and B2 (the fused gate / up order of a's columns)
+//   GG_B_N       out = a w: columns are output columns, rows the reduction: 32 rows of 256 columns to a stage, transposed on the way
+//                out of LDS like GG_B_DW's
+//   GG_B_NP      the same for a gate / up pair in the fused column order: 128 columns of B and the same 128 of B2 to a stage
+// What they cost against the re-tiled operand (33618 rows, 32 groups): a w 901 -> 942 us (K 2048, N 7168) and 872 -> 913 us (K 7168,
+// N 2048), a w^T 901 -> 927 and 872 -> 946 us; one group of 32768 rows 5 to 12 %.  Pieces of 64 or 256 bytes of rows far apart
+// instead of 16 contiguous KB load the L2 channels less evenly.  Re-tiling one such matrix set takes 0.8 ms per direction.
+// Reads past the end of a tensor (its last tile's columns past N) arrive as zeros; elsewhere they are other rows' values, in
+// columns that are not stored.
+enum { GG_B_PACKED = 0, GG_B_DW = 1, GG_B_T = 2, GG_B_N = 3, GG_B_NP = 4 };
+
 constexpr int GG_TRACE_TILE_WORDS = 256, GG_TRACE_BLOCK_WORDS = 4096;
 
 // Where a packed weight column sits inside its aligned group of 32 rows of the packed matrix.  The MFMA leaves a lane
@@ -199,14 +217,15 @@ __device__ __forceinline__ gg_i32x4 gg_range(const uint8_t* p, long long left) {
     return d;
 }
 
-// Half h of a fragment of a 16 x 16 x 32 MFMA out of an LDS tile whose rows run along k (row pitch 512 bytes): lanes 16 q ..
+// Half h of a fragment of a 16 x 16 x 32 MFMA out of an LDS tile whose rows run along k (row pitch PITCH bytes): lanes 16 q ..
 // 16 q + 15 end with k 8 q + 4 h .. + 3 of columns 0 .. 15.  `addr`: the lane's LDS byte address of k = 8 q + (lane % 16) / 4, four
 // columns from column 4 (lane % 4) on; the instruction transposes within the 16 lanes.
 typedef short gg_i16x4 __attribute__((ext_vector_type(4)));
+template <int PITCH>
 __device__ __forceinline__ uint2 gg_read_tr(uint32_t addr, int h) {
     typedef __attribute__((address_space(3))) char* lds_char;
     typedef __attribute__((address_space(3))) gg_i16x4* lds_v4;
-    return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4)((lds_char)(uintptr_t)addr + h * 4 * 512)));
+    return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4)((lds_char)(uintptr_t)addr + h * 4 * PITCH)));
 }
 
 // The lane id read afresh (two instructions) where it is needed.  What the epilogue and the tile set-up derive from it

@@ -203,8 +203,12 @@ __device__ __forceinline__ auto gg_stage_src(const uint8_t* base, size_t off, lo
 // under-filled last round in parts of the K range and leaves fp32 partial sums in the workspace (GemmParams).
 // BSA: the activation operand carries block scales (fp8 down projection: GemmParams::a_bscale), applied by the MFMAs.
 // TRACE: the same kernel with time stamps (GemmParams::trace); product launches never use it.
-template <int BM, int NWM, int EPI, bool FP8, bool SPLIT, bool DW = false, bool BSA = false, bool TRACE = false>
+template <int BM, int NWM, int EPI, bool FP8, bool SPLIT, int BMODE = GG_B_PACKED, bool BSA = false, bool TRACE = false>
 __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const GemmParams p) {
+    constexpr bool DW = BMODE == GG_B_DW, BT = BMODE == GG_B_T, BN_PAIR = BMODE == GG_B_NP, BN_RAW = BMODE == GG_B_N || BN_PAIR;
+    static_assert(!FP8 || BMODE == GG_B_PACKED, "raw weights are a bf16 matter");
+    static_assert(BMODE != GG_B_NP || EPI == EPI_SWIGLU || SPLIT, "pairs are what SwiGLU multiplies with");
+    constexpr int BTR = DW ? 512 : 256;   // (operands transposed out of LDS) row pitch of a stage of B
     static_assert(!TRACE || (!SPLIT && !DW), "time stamps: whole-tile forward launches only");
     [[maybe_unused]] int tr_tile = 0, tr_blk = 0;  // (TRACE) words written so far
 #define GG_TRACE_TILE()                                                                                                    \
@@ -228,8 +232,8 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
     constexpr int CF = FP8 ? 2 : 1;                    // 16-byte LDS chunks per fragment and lane
     constexpr int TM = BM / (NWM * MT), TN = BN / (2 * MT);  // MFMA tiles per wave
     constexpr int NT = TM * TN;                        // MFMAs per K stage and wave
-    constexpr int RPF = DW ? 2 : CF;                   // LDS reads per fragment (DW: two transposing reads of 8 bytes)
-    constexpr int NRD = (TM + TN) * RPF;               // fragment reads per K stage and wave
+    constexpr int RPA = DW ? 2 : CF, RPB = DW || BN_RAW ? 2 : CF;  // LDS reads per fragment (transposing reads bring 8 bytes)
+    constexpr int NRD = TM * RPA + TN * RPB;           // fragment reads per K stage and wave
     constexpr int LR = NW * WROWS;                     // rows fetched per load round (16 per wave)
     constexpr int RA = BM / LR, RB = BN / LR;          // load rounds per stage
     constexpr int LPS = RA + RB;                       // HBM->LDS loads per lane per stage
@@ -335,15 +339,21 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
     const uint32_t lb0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr_t)(sB + wave * WROWS * CHUNKS));
 
     const uint32_t ldk = DW ? (uint32_t)p.dw_rows * 2u : (uint32_t)(p.K * ES);  // row pitch of A in bytes
-    [[maybe_unused]] const uint32_t ldb = (uint32_t)p.N * 2u;                     // (DW) of B
+    // row pitch of B where it is not re-tiled: (BT) its columns are the reduction, half of it per matrix of a pair
+    [[maybe_unused]] const uint32_t ldb = BT ? (uint32_t)(p.B2 ? p.K / 2 : p.K) * 2u : (uint32_t)p.N * 2u;
+    [[maybe_unused]] const size_t b_group = (size_t)p.K / (BT && p.B2 ? 2 : 1) * p.N * 2;  // (BT, BN_RAW) bytes per group and matrix
     const size_t b_slab = (size_t)p.Npad * ROWB;  // packed weights are slab-major: [group][K slab][Npad rows][ROWB bytes]
     // per-round lane offsets into the weight slab (vector registers: no scalar address arithmetic per load)
     uint32_t b_off[RB];
 #pragma unroll
     for (int r = 0; r < RB; ++r) {
         if constexpr (DW) b_off[r] = (uint32_t)(2 * (r * NW + wave) + (lane >> 5)) * ldb + (uint32_t)((lane & 31) ^ (4 * ((2 * wave + (lane >> 5)) & 3))) * 16u;
+        else if constexpr (BT) b_off[r] = (uint32_t)gg_packed_col<false>(r * LR + lrow) * ldb + lchunk * 16;
+        // (BN_RAW: a 1 KB load brings four rows of 256 bytes, half of a stage's loads per region of 128 columns)
+        else if constexpr (BN_RAW) b_off[r] = (uint32_t)(4 * (r % (RB / 2) * NW + wave) + (lane >> 4)) * ldb + (uint32_t)((lane & 15) ^ (4 * (lane >> 4))) * 16u;
         else b_off[r] = (uint32_t)(r * LR + lrow) * ROWB + lchunk * 16;
     }
+    static_assert(!BN_RAW || (RB % 2 == 0 && RB / 2 * NW == 8), "eight loads per region");
     // DW: an LDS stage holds 32 rows of 512 bytes per operand (a 1 KB load brings two of them); 16-byte chunk c of row k lies at
     // position c ^ f(k), which spreads the eight rows that half a wave reads together over the banks: f = 2 (k % 4 + 4 (k / 8 % 2))
     // for A, read 32 contiguous bytes a row, f = 4 (k % 4) for B, read 8 bytes of four chunks in a row (the permuted columns).
@@ -353,17 +363,28 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
         tr_a = (uint32_t)(uintptr_t)(lds_ptr_t)sA + kq * 512 + (((wm * 16 + (q4 >> 1)) ^ (2 * (k4 + 4 * ((lane >> 4) & 1)))) * 16) + (q4 & 1) * 8;
         tr_b = (uint32_t)(uintptr_t)(lds_ptr_t)sB + kq * 512 + (((wn * 16 + q4) ^ (4 * k4)) * 16);
     }
+    // BN_RAW: a stage of B is two regions of 32 rows of 256 bytes: the two column halves of the tile, or its gate and its up columns;
+    // chunk c of row k at position c ^ 4 (k % 4), as in DW's B.
+    if constexpr (BN_RAW) {
+        const int kq = (lane >> 4) * 8 + ((lane & 15) >> 2), k4 = (lane & 15) >> 2, q4 = lane & 3;
+        tr_b = (uint32_t)(uintptr_t)(lds_ptr_t)sB + (BN_PAIR ? 0 : wn * (BSLOT * 8)) + kq * 256 + ((((BN_PAIR ? wn * 8 : 0) + q4) ^ (4 * k4)) * 16);
+    }
     // LDS address of fragment i of A (16 rows of the product) / j of B (its columns 32 (j / 2) + 8 q + 4 (j % 2) ..) in ring slot sl
 #define GG_TR_A(i, sl) ((tr_a ^ ((i) * 32)) + (sl) * (ASLOT * 16))
-#define GG_TR_B(j, sl) ((tr_b ^ (((j) >> 1) * 64)) + (sl) * (BSLOT * 16) + ((j) & 1) * 8)
+#define GG_TR_B(j, sl)                                                                                                  \
+    ((tr_b ^ (BN_PAIR ? ((j) >> 2) * 64 : ((j) >> 1) * 64)) + (BN_PAIR ? (((j) >> 1) & 1) * (BSLOT * 8) : 0) + (sl) * (BSLOT * 16) + ((j) & 1) * 8)
 
 #define GG_MAPROW_GLOBAL(t, l) p.a_map[(t).row0 + (l)]   /* the first tile: straight from memory */
 #define GG_MAPROW_LDS(t, l) s_amap[(l)]                  /* later tiles: fetched into LDS one tile ahead */
 #define GG_TILE_PTRS(t, Ab_, Bb_, aoff_, MAPROW_)                                                          \
     const uint8_t* Ab_ = DW ? p.A + (size_t)(t).ks0 * ldk + (size_t)(t).row0 * 2                             \
                             : (p.a_map ? p.A : p.A + (size_t)(t).row0 * p.K * ES) + (size_t)(t).ks0 * ROWB;  \
-    const uint8_t* Bb_ = DW ? p.B + (size_t)(t).ks0 * ldb + (size_t)(t).nt * BN * 2                           \
-                            : p.B + (size_t)(t).g * p.Npad * p.K * ES + (size_t)(t).nt * BN * ROWB + (size_t)(t).ks0 * b_slab; \
+    const size_t bo0_ = DW ? (size_t)(t).ks0 * ldb + (size_t)(t).nt * BN * 2                                  \
+                      : BT ? (size_t)(t).g * b_group + (size_t)(t).nt * BN * ldb + (size_t)(t).ks0 / (p.B2 ? 2 : 1) * ROWB \
+                      : BN_RAW ? (size_t)(t).g * b_group + (size_t)(t).nt * (BN_PAIR ? BN : 2 * BN) + (size_t)(t).ks0 * 32 * ldb \
+                               : (size_t)(t).g * p.Npad * p.K * ES + (size_t)(t).nt * BN * ROWB + (size_t)(t).ks0 * b_slab; \
+    const uint8_t* Bb_ = p.B + bo0_;                                                                          \
+    if constexpr (BT || BN_RAW) dw_left_b = (long long)p.E_l * b_group - (long long)bo0_;                      \
     uint32_t aoff_[RA];                                                                                     \
     const int ln_ = gg_lane_now();  /* lrow and lchunk again, derived per tile */                              \
     if constexpr (DW) {                                                                                      \
@@ -381,19 +402,24 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
             aoff_[r] = (uint32_t)(p.a_map ? max(MAPROW_(t, lr_), 0) : lr_) * ldk + lcb_;                      \
         }                                                                                                     \
     }
+    [[maybe_unused]] const ptrdiff_t b2_delta = p.B2 - p.B;
     [[maybe_unused]] long long dw_left_a = 0, dw_left_b = 0;  // (DW) bytes of the operands from the tile's corner to the end of the group
     // load d (0 .. LPS-1) of one stage: A rounds first, then B rounds
 #define GG_LD(d, ap_, bp_, aoff_, slot)                                                                       \
     do {                                                                                                      \
         if constexpr ((d) < RA) gg_dma16(ap_, aoff_[(d) < RA ? (d) : 0], la0 + ((slot) * ASLOT + (d) * LR * CHUNKS) * 16); \
-        else gg_dma16(bp_, b_off[(d) >= RA ? (d) - RA : 0], lb0 + ((slot) * BSLOT + ((d) - RA) * LR * CHUNKS) * 16); \
+        else gg_dma16(BN_RAW && (d) >= RA + RB / 2 ? bp_##2 : bp_, b_off[(d) >= RA ? (d) - RA : 0], lb0 + ((slot) * BSLOT + ((d) - RA) * LR * CHUNKS) * 16); \
     } while (0)
     // loads [first, first + count) of stage `st` (clamped to the last stage: the ring never holds data
     // of another tile, and a repeated load of the last stage lands in a slot nobody reads again)
 #define GG_STAGE_PTRS(Ab_, Bb_, st, ap_, bp_, nks_)                                            \
     const int st_ = min((st), (nks_) - 1);                                                     \
     const auto ap_ = gg_stage_src<DW>(Ab_, (size_t)st_ * (DW ? (size_t)32 * ldk : (size_t)ROWB), dw_left_a);  \
-    const auto bp_ = gg_stage_src<DW>(Bb_, (size_t)st_ * (DW ? (size_t)32 * ldb : b_slab), dw_left_b);
+    const size_t so_ = BT ? (size_t)(p.B2 ? st_ >> 1 : st_) * ROWB : (size_t)st_ * (DW || BN_RAW ? (size_t)32 * ldb : b_slab); \
+    const auto bp_ = gg_stage_src<BMODE != GG_B_PACKED>(BT && p.B2 && (st_ & 1) ? Bb_ + b2_delta : Bb_, so_, dw_left_b);   \
+    /* (BN_RAW: the second region, in the other matrix or 256 bytes further along the rows) */                  \
+    [[maybe_unused]] const auto bp_##2 = gg_stage_src<BMODE != GG_B_PACKED>(BN_RAW ? Bb_ + (BN_PAIR ? b2_delta : 256) : Bb_, so_, \
+                                                                            dw_left_b - (BN_RAW && !BN_PAIR ? 256 : 0));
 #define GG_ISSUE_RANGE(Ab_, Bb_, aoff_, st, slot, first, count, nks_)                          \
     do {                                                                                       \
         GG_STAGE_PTRS(Ab_, Bb_, st, ap_i, bp_i, nks_)                                          \
@@ -503,9 +529,10 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
         // fragment read R of the next stage: operand R / CF (activation rows first, then weight rows), chunk R % CF
 #define GG_RD(R, NA_, NB_)                                                                               \
     do {                                                                                                 \
-        constexpr int ro_ = (R) / RPF, rh_ = (R) % RPF;                                                  \
-        if constexpr (DW) {                                                                              \
-            const uint2 v_ = gg_read_tr(ro_ < TM ? GG_TR_A(ro_, nsl_) : GG_TR_B((ro_ < TM ? 0 : ro_ - TM), nsl_), rh_); \
+        constexpr bool ra_ = (R) < TM * RPA;                                                             \
+        constexpr int ro_ = ra_ ? (R) / RPA : TM + ((R) - TM * RPA) / RPB, rh_ = ra_ ? (R) % RPA : ((R) - TM * RPA) % RPB; \
+        if constexpr (ra_ ? DW : DW || BN_RAW) {                                                         \
+            const uint2 v_ = ra_ ? gg_read_tr<512>(GG_TR_A((ra_ ? ro_ : 0), nsl_), rh_) : gg_read_tr<BTR>(GG_TR_B((ra_ ? 0 : ro_ - TM), nsl_), rh_); \
             uint4& f_ = ro_ < TM ? NA_[ro_ < TM ? ro_ : 0] : NB_[ro_ < TM ? 0 : ro_ - TM];               \
             if constexpr (rh_ == 0) { f_.x = v_.x; f_.y = v_.y; } else { f_.z = v_.x; f_.w = v_.y; }      \
         }                                                                                                \
@@ -628,26 +655,25 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
             if (!pre) {
                 const uint4* fa0 = fa + phi * ASLOT;
                 const uint4* fb0 = fb + phi * BSLOT;
-                if constexpr (DW) {
 #pragma unroll
-                    for (int i = 0; i < TM; ++i) {
-                        const uint2 lo = gg_read_tr(GG_TR_A(i, phi), 0), hi = gg_read_tr(GG_TR_A(i, phi), 1);
+                for (int i = 0; i < TM; ++i) {
+                    if constexpr (DW) {
+                        const uint2 lo = gg_read_tr<512>(GG_TR_A(i, phi), 0), hi = gg_read_tr<512>(GG_TR_A(i, phi), 1);
                         fA0[i] = make_uint4(lo.x, lo.y, hi.x, hi.y);
-                    }
+                    } else {
 #pragma unroll
-                    for (int j = 0; j < TN; ++j) {
-                        const uint2 lo = gg_read_tr(GG_TR_B(j, phi), 0), hi = gg_read_tr(GG_TR_B(j, phi), 1);
+                        for (int h = 0; h < CF; ++h) fA0[i * CF + h] = fa0[i * MT * CHUNKS + (fpos ^ (h * FSTEP))];
+                    }
+                }
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    if constexpr (DW || BN_RAW) {
+                        const uint2 lo = gg_read_tr<BTR>(GG_TR_B(j, phi), 0), hi = gg_read_tr<BTR>(GG_TR_B(j, phi), 1);
                         fB0[j] = make_uint4(lo.x, lo.y, hi.x, hi.y);
+                    } else {
+#pragma unroll
+                        for (int h = 0; h < CF; ++h) fB0[j * CF + h] = fb0[j * MT * CHUNKS + (fpos ^ (h * FSTEP))];
                     }
-                } else {
-#pragma unroll
-                for (int i = 0; i < TM; ++i)
-#pragma unroll
-                    for (int h = 0; h < CF; ++h) fA0[i * CF + h] = fa0[i * MT * CHUNKS + (fpos ^ (h * FSTEP))];
-#pragma unroll
-                for (int j = 0; j < TN; ++j)
-#pragma unroll
-                    for (int h = 0; h < CF; ++h) fB0[j * CF + h] = fb0[j * MT * CHUNKS + (fpos ^ (h * FSTEP))];
                 }
                 GG_SC_READ(0);  // (a tile that starts here starts in slot 0)
                 // the first slot is refilled from the first block on: every wave must hold its stage-0 fragments first
@@ -1124,8 +1150,8 @@ __global__ __launch_bounds__(256) void prepack_kernel(const T* __restrict__ w, c
 }
 
 // The same for 16-bit weights with K a multiple of 64 and N of 8 (what the GEMMs take): 64 k x 128 n through LDS, 16 bytes per load
-// and store; and, where out_t is given, the re-tiling of the transposed product (prepack_t below) from the same tile, so that
-// a weight which both directions need is read once.  Columns [N, Npad) of the one and rows [K, Kpad) of the other leave as zeros.
+// and store; or, where out_t is given, the re-tiling of the transposed product (prepack_t below) from the same tile.
+// Columns [N, Npad) of the one and rows [K, Kpad) of the other leave as zeros.
 __global__ __launch_bounds__(256) void prepack16_kernel(const uint16_t* __restrict__ w, const uint16_t* __restrict__ w_up,
                                                          uint16_t* __restrict__ out, uint16_t* __restrict__ out_t, int K, int N, int Npad,
                                                          int Kpad) {
@@ -1711,27 +1737,40 @@ int launch_gemm(const GemmParams& p_in, int epi, hipStream_t s, void* part_ws = 
     const long long ub = ((long long)(p.S_rows + bm - 1) / bm + p.E_l) * nt;
     const bool all_split = p.part_ws && red_blocks > 0 && 4 * ub <= grid && nk >= 2 * GG_MIN_PART_STAGES && p.max_units >= 2 * ub;
     // fp8 without activation is the down projection of the expert MLP: its activation operand is block-scaled
-#define GG_LAUNCH(BMv, NWMv, EPIv)                                                                        \
+#define GG_LAUNCH(BMv, NWMv, EPIv, MODEv)                                                                      \
     do {                                                                                                  \
         constexpr bool BSAv = FP8 && EPIv == EPI_NONE;                                                    \
         if (traced) {                                                                                     \
             if constexpr (BMv == 256 && (EPIv == EPI_NONE || EPIv == EPI_SWIGLU))                         \
-                grouped_gemm_kernel<BMv, NWMv, EPIv, FP8, false, false, BSAv, true><<<grid, NWMv * 2 * WAVE, 0, s>>>(p); \
+                grouped_gemm_kernel<BMv, NWMv, EPIv, FP8, false, GG_B_PACKED, BSAv, true><<<grid, NWMv * 2 * WAVE, 0, s>>>(p); \
             else return moe_fail(MOE_ERR_UNSUPPORTED, "grouped_gemm: no time-stamping instantiation for this launch (256-row tiles, no activation or SwiGLU)"); \
             break;                                                                                        \
         }                                                                                                 \
-        if (!all_split) grouped_gemm_kernel<BMv, NWMv, EPIv, FP8, false, false, BSAv><<<grid, NWMv * 2 * WAVE, 0, s>>>(p); \
+        if (!all_split) grouped_gemm_kernel<BMv, NWMv, EPIv, FP8, false, MODEv, BSAv><<<grid, NWMv * 2 * WAVE, 0, s>>>(p); \
         if (p.part_ws && red_blocks > 0) {                                                                \
             /* (the launch that takes parts stores raw partial sums: one instantiation whatever the epilogue) */ \
-            grouped_gemm_kernel<BMv, NWMv, EPI_NONE, FP8, true, false, BSAv><<<grid, NWMv * 2 * WAVE, 0, s>>>(p); \
+            grouped_gemm_kernel<BMv, NWMv, EPI_NONE, FP8, true, MODEv, BSAv><<<grid, NWMv * 2 * WAVE, 0, s>>>(p); \
             gg_reduce_parts_kernel<BMv, EPIv, FP8><<<red_blocks, 256, 0, s>>>(p, grid);                    \
         }                                                                                                 \
     } while (0)
-#define GG_EPI(EPIv)                          \
-    do {                                      \
-        if (small_m) GG_LAUNCH(128, 2, EPIv); \
-        else GG_LAUNCH(256, (FP8 ? (EPIv == EPI_NONE ? GG_FP8_BSA_NWM : GG_FP8_NWM) : GG_BIG_NWM), EPIv); \
+#define GG_EPI_MODE(EPIv, MODEv)                     \
+    do {                                             \
+        if (small_m) GG_LAUNCH(128, 2, EPIv, MODEv); \
+        else GG_LAUNCH(256, (FP8 ? (EPIv == EPI_NONE ? GG_FP8_BSA_NWM : GG_FP8_NWM) : GG_BIG_NWM), EPIv, MODEv); \
     } while (0)
+#define GG_EPI(EPIv) GG_EPI_MODE(EPIv, GG_B_PACKED)
+    if constexpr (!FP8) {  // weights in the reference layout
+        if (p.b_mode != GG_B_PACKED) {
+            if (traced) return moe_fail(MOE_ERR_UNSUPPORTED, "grouped_gemm: no time-stamping instantiation for weights in the reference layout");
+            if (p.b_mode == GG_B_T && epi == EPI_NONE) GG_EPI_MODE(EPI_NONE, GG_B_T);
+            else if (p.b_mode == GG_B_N && epi == EPI_NONE) GG_EPI_MODE(EPI_NONE, GG_B_N);
+            else if (p.b_mode == GG_B_N && epi == EPI_GELU) GG_EPI_MODE(EPI_GELU, GG_B_N);
+            else if (p.b_mode == GG_B_N && epi == EPI_SILU) GG_EPI_MODE(EPI_SILU, GG_B_N);
+            else if (p.b_mode == GG_B_NP && epi == EPI_SWIGLU) GG_EPI_MODE(EPI_SWIGLU, GG_B_NP);
+            else return moe_fail(MOE_ERR_INVALID, "grouped_gemm: weight mode %d with activation %d", p.b_mode, epi);
+            return moe_check_launch("grouped_gemm");
+        }
+    }
     switch (epi) {
         case EPI_NONE:
             if (FP8 && !p.a_bscale) return moe_fail(MOE_ERR_INVALID, "grouped_gemm: the fp8 down projection needs block scales");
@@ -1745,6 +1784,7 @@ int launch_gemm(const GemmParams& p_in, int epi, hipStream_t s, void* part_ws = 
         default: return moe_fail(MOE_ERR_INVALID, "grouped_gemm: activation %d", epi);
     }
 #undef GG_EPI
+#undef GG_EPI_MODE
 #undef GG_LAUNCH
     return moe_check_launch("grouped_gemm");
 }
@@ -1816,18 +1856,6 @@ extern "C" int moe_prepack_weights(const void* w, const void* w_up, int dtype, i
     return launch_prepack<uint16_t>((const uint16_t*)w, (const uint16_t*)w_up, E_l, K, N, (uint16_t*)packed, (hipStream_t)stream);
 }
 
-// Both re-tilings of a weight (moe_prepack_weights and moe_prepack_weights_transposed) in one pass over it.
-extern "C" int moe_prepack_weights_both(const void* w, const void* w_up, int dtype, int E_l, int K, int N, void* packed, void* packed_t,
-                                        moe_stream_t stream) {
-    MOE_REQUIRE(dtype == MOE_BF16, MOE_ERR_INVALID, "prepack_weights_both: bf16 only (dtype %d)", dtype);
-    MOE_REQUIRE(E_l > 0 && K > 0 && N > 0 && w && packed && packed_t, MOE_ERR_INVALID, "prepack_weights_both: bad arguments");
-    MOE_REQUIRE(K % 64 == 0 && N % 64 == 0, MOE_ERR_UNSUPPORTED, "prepack_weights_both: needs K and N multiples of 64 (K=%d N=%d)", K, N);
-    const int passes = w_up ? 2 : 1, Npad = round_up(N * passes, GG_BN), Kpad = round_up(K, GG_BN);
-    prepack16_kernel<<<dim3(ceil_div(Npad / passes, 128), Kpad / 64, E_l * passes), 256, 0, (hipStream_t)stream>>>(
-        (const uint16_t*)w, (const uint16_t*)w_up, (uint16_t*)packed, (uint16_t*)packed_t, K, N, Npad, Kpad);
-    return moe_check_launch("prepack_weights_both");
-}
-
 extern "C" int moe_prepack_weights_fp8(const uint8_t* w, const uint8_t* w_up, int E_l, int K, int N, uint8_t* packed,
                                        moe_stream_t stream) {
     MOE_REQUIRE(E_l > 0 && K > 0 && N > 0 && w && packed, MOE_ERR_INVALID, "prepack_weights_fp8: bad arguments");
@@ -1846,11 +1874,9 @@ extern "C" int moe_grouped_gemm(const void* tokens, const void* weights, const i
                           EPI_NONE, s);
     MOE_REQUIRE(dtype == MOE_BF16, MOE_ERR_INVALID, "grouped_gemm: dtype %d", dtype);
     MOE_REQUIRE(K % 64 == 0 && N % 8 == 0, MOE_ERR_UNSUPPORTED, "grouped_gemm: bf16 needs K %% 64 == 0 and N %% 8 == 0 (K=%d N=%d)", K, N);
-    MOE_REQUIRE(ws && ws_bytes >= moe_prepack_bytes(dtype, E_l, K, N), MOE_ERR_WORKSPACE, "grouped_gemm: workspace too small");
-    int rc = launch_prepack<uint16_t>((const uint16_t*)weights, nullptr, E_l, K, N, (uint16_t*)ws, s);
-    if (rc) return rc;
+    // (the weights are taken as they are: a re-tiled copy per call would read and write them once more; ws is not used)
     GemmParams p{};
-    p.A = (const uint8_t*)tokens; p.B = (const uint8_t*)ws; p.C = out; p.cnt = expert_cnt;
+    p.A = (const uint8_t*)tokens; p.B = (const uint8_t*)weights; p.b_mode = GG_B_N; p.C = out; p.cnt = expert_cnt;
     p.E_l = E_l; p.K = K; p.N = N; p.Npad = round_up(N, GG_BN); p.ldc = N; p.S_rows = S_rows;
     return launch_gemm<false>(p, EPI_NONE, s);
 }
@@ -1902,14 +1928,16 @@ extern "C" int moe_grouped_gemm_mapped(const void* a_base, int a_rows, const int
     return launch_gemm<false>(p, act, (hipStream_t)stream, part_ws, part_ws_bytes);
 }
 
-extern "C" int moe_expert_forward(const void* tokens, const void* packed, const int32_t* expert_cnt, int S_rows, int K, int N, int E_l,
-                                  void* out, void* part_ws, size_t part_ws_bytes, moe_stream_t stream) {
+extern "C" int moe_expert_forward(const void* tokens, const void* weights, int layout, const int32_t* expert_cnt, int S_rows, int K, int N,
+                                  int E_l, void* out, void* part_ws, size_t part_ws_bytes, moe_stream_t stream) {
+    MOE_REQUIRE(layout >= MOE_W_TILED && layout <= MOE_W_RAW_T, MOE_ERR_INVALID, "expert_forward: weight layout %d", layout);
     MOE_REQUIRE(S_rows >= 0 && K > 0 && N > 0 && E_l > 0 && E_l <= GG_MAXG, MOE_ERR_INVALID, "expert_forward: bad shape");
     MOE_REQUIRE(K % 64 == 0 && N % 8 == 0, MOE_ERR_UNSUPPORTED, "expert_forward: needs K %% 64 == 0 and N %% 8 == 0 (K=%d N=%d)", K, N);
     if (S_rows == 0) return MOE_OK;
-    MOE_REQUIRE(tokens && packed && expert_cnt && out, MOE_ERR_INVALID, "expert_forward: null pointer");
+    MOE_REQUIRE(tokens && weights && expert_cnt && out, MOE_ERR_INVALID, "expert_forward: null pointer");
     GemmParams p{};
-    p.A = (const uint8_t*)tokens; p.B = (const uint8_t*)packed; p.C = out; p.cnt = expert_cnt; p.zero_tail = 1;
+    p.A = (const uint8_t*)tokens; p.B = (const uint8_t*)weights; p.C = out; p.cnt = expert_cnt; p.zero_tail = 1;
+    p.b_mode = layout == MOE_W_TILED ? GG_B_PACKED : layout == MOE_W_RAW ? GG_B_N : GG_B_T;
     p.E_l = E_l; p.K = K; p.N = N; p.ldc = N; p.S_rows = S_rows; p.Npad = round_up(N, GG_BN);
     return launch_gemm<false>(p, EPI_NONE, (hipStream_t)stream, part_ws, part_ws_bytes);
 }
@@ -2135,7 +2163,7 @@ static int launch_dw(const void* x, const void* dy, const int32_t* expert_cnt, i
     p.A = (const uint8_t*)x; p.B = (const uint8_t*)dy; p.C = dw; p.cnt = expert_cnt;
     p.E_l = E_l; p.K = 64; p.N = N; p.Npad = round_up(N, GG_BN); p.ldc = ldc; p.S_rows = K;
     p.dw_rows = K; p.dw_src_rows = S_rows; p.dw_split = split_F; p.dw_delta = dw_delta; p.c_group_stride = (size_t)K * ldc;
-    grouped_gemm_kernel<256, GG_BIG_NWM, EPI_NONE, false, false, true><<<num_cus(), GG_BIG_NWM * 2 * WAVE, 0, s>>>(p);
+    grouped_gemm_kernel<256, GG_BIG_NWM, EPI_NONE, false, false, GG_B_DW><<<num_cus(), GG_BIG_NWM * 2 * WAVE, 0, s>>>(p);
     return moe_check_launch("grouped_gemm_dw");
 }
 
@@ -2163,46 +2191,53 @@ extern "C" int moe_grouped_gemm_dw_pair(const void* x, const void* dy, const int
     return launch_dw(x, dy, expert_cnt, S_rows, K, 2 * F, E_l, F, dw_gate, F, (bf16_t*)dw_up - (bf16_t*)dw_gate, (hipStream_t)stream);
 }
 
-// ---- the expert MLP of a training step, one call per direction (bf16).  Weights as moe_prepack_weights (forward) and
-// moe_prepack_weights_transposed (backward) re-tile them; pre_act as moe_grouped_gemm_act_keep leaves it.
-extern "C" int moe_mlp_train_forward(const void* x, const int32_t* expert_cnt, int S_rows, int H, int F, int E_l, int act, const void* w1,
-                                     const void* w2, void* hidden, void* pre_act, void* out, void* part_ws, size_t part_ws_bytes,
-                                     moe_stream_t stream) {
+// ---- the expert MLP of a training step, one call per direction (bf16); pre_act as moe_grouped_gemm_act_keep leaves it.
+extern "C" int moe_mlp_train_forward(const void* x, const int32_t* expert_cnt, int S_rows, int H, int F, int E_l, int act, int layout,
+                                     const void* w1, const void* w_up, const void* w2, void* hidden, void* pre_act, void* out, void* part_ws,
+                                     size_t part_ws_bytes, moe_stream_t stream) {
     MOE_REQUIRE(S_rows > 0 && H > 0 && F > 0 && E_l > 0 && E_l <= GG_MAXG, MOE_ERR_INVALID, "mlp_train_forward: bad shape");
     MOE_REQUIRE(act > EPI_NONE && act <= EPI_SWIGLU, MOE_ERR_INVALID, "mlp_train_forward: activation %d", act);
     MOE_REQUIRE(H % 64 == 0 && F % 64 == 0, MOE_ERR_UNSUPPORTED, "mlp_train_forward: needs H, F multiples of 64 (H=%d F=%d)", H, F);
-    MOE_REQUIRE(x && expert_cnt && w1 && w2 && hidden && pre_act && out, MOE_ERR_INVALID, "mlp_train_forward: null pointer");
+    MOE_REQUIRE(layout == MOE_W_TILED || layout == MOE_W_RAW, MOE_ERR_INVALID, "mlp_train_forward: weight layout %d", layout);
+    const bool raw = layout == MOE_W_RAW, pair = raw && act == EPI_SWIGLU;
+    MOE_REQUIRE(x && expert_cnt && w1 && w2 && hidden && pre_act && out && (!pair || w_up), MOE_ERR_INVALID, "mlp_train_forward: null pointer");
     hipStream_t s = (hipStream_t)stream;
     GemmParams p{};
     p.A = (const uint8_t*)x; p.B = (const uint8_t*)w1; p.C = hidden; p.C2 = pre_act; p.cnt = expert_cnt;
+    p.B2 = pair ? (const uint8_t*)w_up : nullptr;
+    p.b_mode = pair ? GG_B_NP : raw ? GG_B_N : GG_B_PACKED;
     p.E_l = E_l; p.K = H; p.N = F; p.ldc = F; p.S_rows = S_rows; p.Npad = round_up(act == EPI_SWIGLU ? 2 * F : F, GG_BN);
     const int rc = launch_gemm<false>(p, act, s, part_ws, part_ws_bytes);
     if (rc) return rc;
     GemmParams q{};
     q.A = (const uint8_t*)hidden; q.B = (const uint8_t*)w2; q.C = out; q.cnt = expert_cnt; q.zero_tail = 1;
+    q.b_mode = raw ? GG_B_N : GG_B_PACKED;
     q.E_l = E_l; q.K = F; q.N = H; q.ldc = H; q.S_rows = S_rows; q.Npad = round_up(H, GG_BN);
     return launch_gemm<false>(q, EPI_NONE, s, part_ws, part_ws_bytes);
 }
 
 extern "C" int moe_mlp_train_backward(const void* x, const void* hidden, const void* pre_act, const void* dy, const int32_t* expert_cnt,
-                                      int S_rows, int H, int F, int E_l, int act, const void* w1_t, const void* w2_t, void* dh, void* d_pre,
-                                      void* dx, void* dw1, void* dw_up, void* dw2, void* part_ws, size_t part_ws_bytes, moe_stream_t stream) {
+                                      int S_rows, int H, int F, int E_l, int act, int layout, const void* w1, const void* w_up,
+                                      const void* w2, void* dh, void* d_pre, void* dx, void* dw1, void* dw_up, void* dw2, void* part_ws, size_t part_ws_bytes, moe_stream_t stream) {
     MOE_REQUIRE(S_rows > 0 && H > 0 && F > 0 && E_l > 0 && E_l <= GG_MAXG, MOE_ERR_INVALID, "mlp_train_backward: bad shape");
     MOE_REQUIRE(act > EPI_NONE && act <= EPI_SWIGLU, MOE_ERR_INVALID, "mlp_train_backward: activation %d", act);
     MOE_REQUIRE(H % 64 == 0 && F % 64 == 0, MOE_ERR_UNSUPPORTED, "mlp_train_backward: needs H, F multiples of 64 (H=%d F=%d)", H, F);
-    MOE_REQUIRE(x && hidden && pre_act && dy && expert_cnt && w1_t && w2_t && dh && d_pre && dx && dw1 && dw2 && (act != EPI_SWIGLU || dw_up),
+    MOE_REQUIRE(layout == MOE_W_TILED || layout == MOE_W_RAW_T, MOE_ERR_INVALID, "mlp_train_backward: weight layout %d", layout);
+    const bool raw = layout == MOE_W_RAW_T;
+    MOE_REQUIRE(x && hidden && pre_act && dy && expert_cnt && w1 && w2 && dh && d_pre && dx && dw1 && dw2 && (act != EPI_SWIGLU || (dw_up && (w_up || !raw))),
                 MOE_ERR_INVALID, "mlp_train_backward: null pointer");
     hipStream_t s = (hipStream_t)stream;
     const int NP = act == EPI_SWIGLU ? 2 * F : F;
     GemmParams p{};
-    p.A = (const uint8_t*)dy; p.B = (const uint8_t*)w2_t; p.C = dh; p.cnt = expert_cnt;
+    p.A = (const uint8_t*)dy; p.B = (const uint8_t*)w2; p.b_mode = raw ? GG_B_T : GG_B_PACKED; p.C = dh; p.cnt = expert_cnt;
     p.E_l = E_l; p.K = H; p.N = F; p.ldc = F; p.S_rows = S_rows; p.Npad = round_up(F, GG_BN);
     int rc = launch_gemm<false>(p, EPI_NONE, s, part_ws, part_ws_bytes);
     if (!rc) rc = launch_dw(hidden, dy, expert_cnt, S_rows, F, H, E_l, 0, dw2, H, 0, s);
     if (!rc) rc = moe_mlp_act_backward(pre_act, dh, MOE_BF16, S_rows, F, act, d_pre, stream);
     if (rc) return rc;
     GemmParams q{};
-    q.A = (const uint8_t*)d_pre; q.B = (const uint8_t*)w1_t; q.C = dx; q.cnt = expert_cnt; q.zero_tail = 1;
+    q.A = (const uint8_t*)d_pre; q.B = (const uint8_t*)w1; q.b_mode = raw ? GG_B_T : GG_B_PACKED; q.C = dx; q.cnt = expert_cnt; q.zero_tail = 1;
+    q.B2 = raw && act == EPI_SWIGLU ? (const uint8_t*)w_up : nullptr;
     q.E_l = E_l; q.K = NP; q.N = H; q.ldc = H; q.S_rows = S_rows; q.Npad = round_up(H, GG_BN);
     rc = launch_gemm<false>(q, EPI_NONE, s, part_ws, part_ws_bytes);
     if (rc) return rc;

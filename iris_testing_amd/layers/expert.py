@@ -9,11 +9,12 @@ from typing import Optional
 
 import torch
 
+from .. import _lib as L
 from .. import ops
 from ..utils import _assert_cuda_int32
 
 
-# Re-tiled copies of weight tensors the operator has seen, keyed on the tensor's storage and version counter, so that
+# Re-tiled copies of weight tensors the operator has seen (None: seen once, not re-tiled yet), keyed on the tensor's storage and version counter, so that
 # a weight that did not change between calls is re-tiled once, not on every call (the re-tiling reads and writes the
 # whole tensor).  Entries die with their tensors (weak references); an in-place update bumps the version and re-tiles.
 _PACKED = {}
@@ -40,17 +41,21 @@ def _cached_pack(kind: str, w: torch.Tensor, w_up: Optional[torch.Tensor], build
     return packed
 
 
-def _pack_both(w: torch.Tensor, w_up: Optional[torch.Tensor]) -> torch.Tensor:
-    """_packed_weights' and _packed_weights_t's re-tilings in one pass over the weight; the second one is left in the cache."""
-    _drop_packs("T", w)
-    packed, packed_t = ops.prepack_weights_both(w, w_up)
-    _PACKED[_pack_key("T", w, w_up)] = (weakref.ref(w), packed_t)
-    return packed
-
-
-def _packed_weights(w: torch.Tensor, w_up: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """Re-tiled w (with w_up: the fused gate/up pair) for the forward GEMM."""
-    return _cached_pack("N", w, w_up, ops.prepack_weights)
+def _weights_for(w: torch.Tensor, rows: int):
+    """(weights, layout) for the forward GEMM on `rows` rows.  The first call with a weight -- or with what an in-place update made of
+    it -- multiplies with the tensor as it is (see ExpertWeights.train_weights), the second one, if nothing has changed by
+    then, re-tiles it."""
+    key = _pack_key("N", w, None)
+    hit = _PACKED.get(key)
+    if hit is None or hit[0]() is not w:
+        _drop_packs("N", w)
+        raw = rows < 4096 * w.shape[0]
+        _PACKED[key] = hit = (weakref.ref(w), None if raw else ops.prepack_weights(w))
+        if raw:
+            return w, L.W_RAW
+    elif hit[1] is None:
+        _PACKED[key] = hit = (hit[0], ops.prepack_weights(w))
+    return hit[1], L.W_TILED
 
 
 def _packed_weights_t(w: torch.Tensor, w_up: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -60,10 +65,16 @@ def _packed_weights_t(w: torch.Tensor, w_up: Optional[torch.Tensor] = None) -> t
 
 def _grouped_gemm_t(do: torch.Tensor, weights: torch.Tensor, cnt: torch.Tensor) -> torch.Tensor:
     """d tokens[rows of g] = do[rows of g] @ weights[g]^T; rows past sum(cnt) are zero."""
-    K = weights.shape[1]
+    E_l, K, N = weights.shape
     if do.dtype == torch.float32:
         return ops.grouped_gemm(do, ops.transpose_weights_f32(weights.contiguous()), cnt)
-    return ops.expert_forward(do, _packed_weights_t(weights), cnt, K, _part_ws(do.device))
+    S = do.shape[0]
+    if N % 64 or K % 8 or S >= 4096 * E_l:  # (no whole stages of the reduction; or worth a re-tiled copy)
+        out = torch.zeros((S, K), dtype=do.dtype, device=do.device)
+        if S:
+            ops.grouped_gemm_mapped(do, None, _packed_weights_t(weights), cnt, S, K, "none", out, part_ws=_part_ws(do.device))
+        return out
+    return ops.expert_forward(do, weights.contiguous(), L.W_RAW_T, cnt, K, _part_ws(do.device))
 
 
 def _part_ws(device) -> torch.Tensor:
@@ -78,7 +89,8 @@ def _grouped_gemm(tokens: torch.Tensor, weights: torch.Tensor, cnt: torch.Tensor
     """out[rows of g] = tokens[rows of g] @ weights[g]; rows past sum(cnt) are zero."""
     if tokens.dtype != torch.bfloat16 or weights.shape[1] % 64 or weights.shape[2] % 8:  # (what the MFMA kernel covers)
         return ops.grouped_gemm(tokens, weights, cnt)
-    return ops.expert_forward(tokens, _packed_weights(weights), cnt, weights.shape[2], _part_ws(tokens.device))
+    w, layout = _weights_for(weights, tokens.shape[0])
+    return ops.expert_forward(tokens, w, layout, cnt, weights.shape[2], _part_ws(tokens.device))
 
 
 class Expert(torch.autograd.Function):
@@ -129,10 +141,11 @@ class ExpertWeights:
     w_up: Optional[torch.Tensor] = None
     scales: Optional[tuple] = None  # fp8: (sg, su, sd)
     # the tensors prepare() was given, in the reference layout: (w1, w2, w_up); the backward pass differentiates with
-    # respect to them and re-tiles their transposes on first use
+    # respect to them and multiplies with them as they are
     raw: Optional[tuple] = field(default=None, repr=False)
     # version counters of the raw tensors when w1 / w2 / w_up were last derived from them (refresh() compares)
     raw_versions: Optional[tuple] = field(default=None, repr=False)
+    seen_versions: Optional[tuple] = field(default=None, repr=False)  # ... when train_weights() last looked at them
 
     @staticmethod
     def _derive(raw):
@@ -157,17 +170,24 @@ class ExpertWeights:
     def refresh(self) -> "ExpertWeights":
         """Derive the kernels' copies again if a tensor prepare() was given has been updated in place since (an optimizer
         step): the forward pass would otherwise multiply with the weights of before the update while the backward pass,
-        which re-tiles the transposes by tensor version, uses the new ones."""
+        which takes the tensors as they are, uses the new ones."""
         if self.raw is not None and self._versions(self.raw) != self.raw_versions:
-            w1, w2, w_up = self.raw
-            if w1.dtype == torch.bfloat16 and self.hidden % 64 == 0 and self.ffn % 64 == 0 and torch.is_grad_enabled() and \
-                    all(t is None or (t.requires_grad and t.is_contiguous()) for t in self.raw):
-                # weights in training: the backward pass of this step will want their transposes too
-                self.w1, self.w2, self.w_up = _pack_both(w1, w_up), _pack_both(w2, None), None
-            else:
-                self.w1, self.w2, self.w_up = self._derive(self.raw)
+            self.w1, self.w2, self.w_up = self._derive(self.raw)
             self.raw_versions = self._versions(self.raw)
         return self
+
+    def train_weights(self, rows: int):
+        """(layout, w1, w_up, w2) for the forward pass of a bf16 training step on `rows` rows.  Weights that an optimizer has updated
+        since they were re-tiled are taken as they are if the rows per expert are few: the GEMMs read the reference layout at 0.88 to
+        0.96 of the rate, which costs more than re-tiling (reading and writing every weight in either direction) from some 4000
+        rows per expert on.  If they are still the same on the next call, they are re-tiled after all."""
+        now = self._versions(self.raw)
+        if now != self.raw_versions:
+            if now != self.seen_versions and rows < 4096 * self.e_local and all(t is None or t.is_contiguous() for t in self.raw):
+                self.seen_versions = now
+                return L.W_RAW, self.raw[0], self.raw[2], self.raw[1]
+            self.refresh()
+        return L.W_TILED, self.w1, None, self.w2
 
     @classmethod
     def prepare_fp8(cls, wg_q, sg, wu_q, su, wd_q, sd):
@@ -189,8 +209,11 @@ class ExpertMLP(torch.autograd.Function):
         a1 = None
         if tokens.dtype == torch.bfloat16 and ew.act != "none" and S:
             # the first GEMM also keeps what it feeds to the activation: the backward pass would otherwise run it again
-            out, hidden, a1 = ops.mlp_train_forward(tokens, cnt, ew.act, ew.w1, ew.w2, F, part_ws=_part_ws(tokens.device))
+            weights = ew.train_weights(S)
+            ctx.raw = weights[0] == L.W_RAW
+            out, hidden, a1 = ops.mlp_train_forward(tokens, cnt, ew.act, *weights, F, part_ws=_part_ws(tokens.device))
         else:
+            ew.refresh()
             hidden = torch.empty((S, F), dtype=tokens.dtype, device=tokens.device)
             out = ops.grouped_mlp(tokens, cnt, ew.act, ew.w1, ew.w2, ew.w_up, F=F, hidden_ws=hidden)
         ctx.save_for_backward(tokens, hidden, cnt, w1, w2, w_up, a1)
@@ -220,14 +243,15 @@ class ExpertMLP(torch.autograd.Function):
             return dx, None, None, dw1, dw2, None
         ws = _part_ws(tokens.device)
         if a1 is not None:
-            dx, dw1, dw2, dw_up = ops.mlp_train_backward(tokens, hidden, a1, dy, cnt, ew.act, _packed_weights_t(w1, w_up), _packed_weights_t(w2),
-                                                         part_ws=ws)
+            weights = (L.W_RAW_T, w1, w_up, w2) if ctx.raw else (L.W_TILED, _packed_weights_t(w1, w_up), None, _packed_weights_t(w2))
+            dx, dw1, dw2, dw_up = ops.mlp_train_backward(tokens, hidden, a1, dy, cnt, ew.act, *weights, part_ws=ws)
             return dx, None, None, dw1, dw2, dw_up
         NP = 2 * F if swiglu else F
         dh = torch.zeros((S, F), dtype=dy.dtype, device=dy.device)
         dx = torch.zeros((S, H), dtype=dy.dtype, device=dy.device)
         if S:
             ops.grouped_gemm_mapped(dy, None, _packed_weights_t(w2), cnt, S, F, "none", dh, part_ws=ws)
+        ew.refresh()
         a1 = torch.zeros((S, NP), dtype=dy.dtype, device=dy.device)  # (no rows, or an MLP without an activation)
         if S:
             ops.grouped_gemm_mapped(tokens, None, ew.w1, cnt, S, NP, "none", a1, part_ws=ws)
@@ -248,8 +272,9 @@ def expert_mlp(tokens: torch.Tensor, weights: ExpertWeights, local_expert_cnt: t
     if weights.dtype == torch.uint8:
         sg, su, sd = weights.scales
         return ops.grouped_mlp_fp8(tokens.contiguous(), local_expert_cnt, weights.ffn, weights.w1, sg, su, weights.w2, sd)
-    raw = weights.refresh().raw
+    raw = weights.raw
     if torch.is_grad_enabled() and raw is not None and (tokens.requires_grad or any(t is not None and t.requires_grad for t in raw)):
         return ExpertMLP.apply(tokens, local_expert_cnt.contiguous(), weights, raw[0], raw[1], raw[2])
+    weights.refresh()
     return ops.grouped_mlp(tokens.contiguous(), local_expert_cnt, weights.act, weights.w1, weights.w2, weights.w_up,
                            F=weights.ffn)

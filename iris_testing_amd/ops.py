@@ -294,13 +294,19 @@ def shuffle_totals(pca: torch.Tensor, token_sync: Optional[torch.Tensor], out: t
                                        L.ptr(out), L.stream_ptr()))
 
 
-def expert_forward(tokens: torch.Tensor, packed: torch.Tensor, expert_cnt: torch.Tensor, N: int, part_ws: torch.Tensor) -> torch.Tensor:
-    """out[rows of e] = tokens[rows of e] @ w[e] for bf16 rows and re-tiled weights; rows past the counted total are zero."""
+def expert_forward(tokens: torch.Tensor, weights: torch.Tensor, layout: int, expert_cnt: torch.Tensor, N: int,
+                   part_ws: torch.Tensor) -> torch.Tensor:
+    """out[rows of e] = tokens[rows of e] @ w[e] for bf16 rows; rows past the counted total are zero.  layout W_TILED: weights re-tiled
+    (prepack_weights of [E_l,K,N]); W_RAW: [E_l,K,N] as they are; W_RAW_T: [E_l,N,K] as they are, transposed in the product."""
     _req_cuda(tokens, "tokens")
+    _req_cuda(weights, "weights")
     _req_i32(expert_cnt, "local_expert_cnt")
     S, K = tokens.shape
+    assert tokens.dtype == torch.bfloat16
+    if layout != L.W_TILED:
+        assert weights.dtype == torch.bfloat16 and weights.shape == ((expert_cnt.numel(), K, N) if layout == L.W_RAW else (expert_cnt.numel(), N, K))
     out = torch.empty((S, N), dtype=tokens.dtype, device=tokens.device)
-    L.check(L.lib().moe_expert_forward(L.ptr(tokens), L.ptr(packed), L.ptr(expert_cnt), S, K, N, expert_cnt.numel(), L.ptr(out),
+    L.check(L.lib().moe_expert_forward(L.ptr(tokens), L.ptr(weights), layout, L.ptr(expert_cnt), S, K, N, expert_cnt.numel(), L.ptr(out),
                                        L.ptr(part_ws), part_ws.numel() * part_ws.element_size(), L.stream_ptr()))
     return out
 
@@ -362,11 +368,8 @@ def grouped_gemm(tokens: torch.Tensor, weights: torch.Tensor, expert_cnt: torch.
     assert K == K2 and expert_cnt.numel() == E_l
     if out is None:
         out = torch.zeros((S, N), dtype=tokens.dtype, device=tokens.device)
-    code = L.dtype_code(tokens.dtype)
-    nbytes = L.lib().moe_prepack_bytes(code, E_l, K, N)
-    ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=tokens.device)
-    L.check(L.lib().moe_grouped_gemm(L.ptr(tokens), L.ptr(weights), L.ptr(expert_cnt), code, S, K, N, E_l, L.ptr(out),
-                                     L.ptr(ws), nbytes, L.stream_ptr()))
+    L.check(L.lib().moe_grouped_gemm(L.ptr(tokens), L.ptr(weights), L.ptr(expert_cnt), L.dtype_code(tokens.dtype), S, K, N, E_l, L.ptr(out),
+                                     None, 0, L.stream_ptr()))
     return out
 
 
@@ -671,53 +674,51 @@ def prepack_weights_transposed(w: torch.Tensor, w_up: Optional[torch.Tensor] = N
     return out
 
 
-def prepack_weights_both(w: torch.Tensor, w_up: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, torch.Tensor]:
-    """(prepack_weights(w, w_up), prepack_weights_transposed(w, w_up)) in one pass over the weights."""
-    _req_cuda(w, "weights")
-    assert w.dtype == torch.bfloat16
-    E_l, K, N = w.shape
-    if w_up is not None:
-        _req_cuda(w_up, "w_up")
-        assert w_up.shape == w.shape and w_up.dtype == w.dtype
-    n_tot = N * (2 if w_up is not None else 1)
-    lib = L.lib()
-    out = torch.empty(lib.moe_prepack_bytes(L.MOE_BF16, E_l, K, n_tot), dtype=torch.uint8, device=w.device)
-    out_t = torch.empty(lib.moe_prepack_bytes(L.MOE_BF16, E_l, n_tot, K), dtype=torch.uint8, device=w.device)
-    L.check(lib.moe_prepack_weights_both(L.ptr(w), L.ptr(w_up), L.MOE_BF16, E_l, K, N, L.ptr(out), L.ptr(out_t), L.stream_ptr()))
-    return out, out_t
-
-
-def mlp_train_forward(x: torch.Tensor, expert_cnt: torch.Tensor, act: str, w1: torch.Tensor, w2: torch.Tensor, F: int,
-                      part_ws: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
-    """(out [S,H], hidden [S,F], pre_act) of the bf16 expert MLP with what its backward pass needs kept; w1 / w2 prepacked."""
+def mlp_train_forward(x: torch.Tensor, expert_cnt: torch.Tensor, act: str, layout: int, w1: torch.Tensor, w_up: Optional[torch.Tensor],
+                      w2: torch.Tensor, F: int, part_ws: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """(out [S,H], hidden [S,F], pre_act) of the bf16 expert MLP with what its backward pass needs kept.  layout W_TILED: w1 / w2 as
+    prepack_weights makes them; W_RAW: w1, w_up [E_l,H,F] and w2 [E_l,F,H] as they are."""
     _req_cuda(x, "x")
     _req_i32(expert_cnt, "expert_cnt")
     assert x.dtype == torch.bfloat16
     S, H = x.shape
+    swiglu, E_l = act == "swiglu", expert_cnt.numel()
+    if layout == L.W_RAW:
+        _req_raw_mlp(w1, w_up, w2, E_l, H, F, swiglu)
     hidden = torch.empty((S, F), dtype=x.dtype, device=x.device)
-    pre = torch.empty((S, 2 * F if act == "swiglu" else F), dtype=x.dtype, device=x.device)
+    pre = torch.empty((S, 2 * F if swiglu else F), dtype=x.dtype, device=x.device)
     out = torch.empty_like(x)
-    L.check(L.lib().moe_mlp_train_forward(x.data_ptr(), expert_cnt.data_ptr(), S, H, F, expert_cnt.numel(), L.ACT[act], w1.data_ptr(),
+    L.check(L.lib().moe_mlp_train_forward(x.data_ptr(), expert_cnt.data_ptr(), S, H, F, E_l, L.ACT[act], layout, w1.data_ptr(), L.ptr(w_up),
                                           w2.data_ptr(), hidden.data_ptr(), pre.data_ptr(), out.data_ptr(), L.ptr(part_ws),
                                           0 if part_ws is None else part_ws.numel() * part_ws.element_size(), L.stream_ptr()))
     return out, hidden, pre
 
 
+def _req_raw_mlp(w1, w_up, w2, E_l: int, H: int, F: int, swiglu: bool) -> None:
+    for t, shape, name in ((w1, (E_l, H, F), "w1"), (w2, (E_l, F, H), "w2")) + (((w_up, (E_l, H, F), "w_up"),) if swiglu else ()):
+        _req_cuda(t, name)
+        assert t.dtype == torch.bfloat16 and t.shape == shape, f"{name} must be bf16 {shape}"
+
+
 def mlp_train_backward(x: torch.Tensor, hidden: torch.Tensor, pre: torch.Tensor, dy: torch.Tensor, expert_cnt: torch.Tensor, act: str,
-                       w1_t: torch.Tensor, w2_t: torch.Tensor, part_ws: Optional[torch.Tensor] = None):
-    """(dx, dw1, dw2, dw_up or None) of mlp_train_forward; w1_t / w2_t: prepack_weights_transposed of (w1, w_up) and w2."""
+                       layout: int, w1: torch.Tensor, w_up: Optional[torch.Tensor], w2: torch.Tensor,
+                       part_ws: Optional[torch.Tensor] = None):
+    """(dx, dw1, dw2, dw_up or None) of mlp_train_forward.  layout W_RAW_T: the weights in the reference layout; W_TILED: as
+    prepack_weights_transposed makes them of (w1, w_up) and w2."""
     _req_cuda(dy, "dy")
     _req_i32(expert_cnt, "expert_cnt")
     assert dy.dtype == torch.bfloat16 and dy.shape == x.shape
     S, H = x.shape
     F, E_l, dev = hidden.shape[1], expert_cnt.numel(), x.device
     swiglu = act == "swiglu"
+    if layout == L.W_RAW_T:
+        _req_raw_mlp(w1, w_up, w2, E_l, H, F, swiglu)
     dh, d_pre, dx = torch.empty_like(hidden), torch.empty_like(pre), torch.empty_like(x)
     dw1, dw2 = torch.empty((E_l, H, F), dtype=x.dtype, device=dev), torch.empty((E_l, F, H), dtype=x.dtype, device=dev)
     dw_up = torch.empty_like(dw1) if swiglu else None
     L.check(L.lib().moe_mlp_train_backward(x.data_ptr(), hidden.data_ptr(), pre.data_ptr(), dy.data_ptr(), expert_cnt.data_ptr(), S, H, F,
-                                           E_l, L.ACT[act], w1_t.data_ptr(), w2_t.data_ptr(), dh.data_ptr(), d_pre.data_ptr(), dx.data_ptr(),
-                                           dw1.data_ptr(), L.ptr(dw_up), dw2.data_ptr(), L.ptr(part_ws),
+                                           E_l, L.ACT[act], layout, w1.data_ptr(), L.ptr(w_up), w2.data_ptr(), dh.data_ptr(), d_pre.data_ptr(),
+                                           dx.data_ptr(), dw1.data_ptr(), L.ptr(dw_up), dw2.data_ptr(), L.ptr(part_ws),
                                            0 if part_ws is None else part_ws.numel() * part_ws.element_size(), L.stream_ptr()))
     return dx, dw1, dw2, dw_up
 

@@ -134,7 +134,7 @@ class DispatchPipeline:
 
     def _run(self, s):
         """The stages of STAGES as one call (the map, scales, gates and padding of the destination side in one launch)."""
-        a, w, ew, p = self._args, self.world, self.weights, self._p
+        a, w, ew, p = self._args, self.world, self.weights.refresh(), self._p
         # what belongs to the caller is looked up on every step
         a.x, a.router, a.bias, a.recv_counts = p(w.x0), p(w.router), p(w.bias), p(w.recv_counts)
         a.recv = p(w.recv_q if self.fp8_dispatch else self.recv_flat if self.padding_free else w.recv)
@@ -200,7 +200,7 @@ class DispatchPipeline:
                                                 self._p(self.unpack_map), s))
 
     def mlp_up(self, s):
-        c, ew = self.cfg, self.weights
+        c, ew = self.cfg, self.weights.refresh()
         lib = L.lib()
         if ew.dtype == torch.uint8:
             sg, su, sd = ew.scales
@@ -242,7 +242,7 @@ class DispatchPipeline:
                                                 self.S, None, self._p(self.part_ws), self.part_ws_bytes, s))
 
     def mlp_down(self, s):
-        c, ew = self.cfg, self.weights
+        c, ew = self.cfg, self.weights.refresh()
         if ew.dtype == torch.bfloat16 and self.gated:
             w = self.world
             L.check(L.lib().moe_grouped_gemm_mapped_gated(self._p(self.hidden), self.S, None, self._p(ew.w2), self._p(self.expert_cnt),

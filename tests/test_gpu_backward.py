@@ -187,7 +187,7 @@ def test_expert_mlp_follows_in_place_weight_updates():
 
 
 @pytest.mark.parametrize("K,F,cnt", [(8, 32, (1,)), (264, 96, (31, 0, 33)), (256, 128, (64, 65, 63)), (520, 160, (127, 2, 129, 256))])
-def test_weight_gradient_pair_and_both_re_tilings_at_tile_edges(K, F, cnt):
+def test_weight_gradient_pair_at_tile_edges(K, F, cnt):
     """The weight-gradient kernel reads its operands with the row index slow and ends every group's range in the load descriptor: row
     counts around a stage (32) and a pair of stages, partly filled tiles in both directions, both halves of a gate / up pair."""
     rng = np.random.default_rng(K + F)
@@ -209,8 +209,55 @@ def test_weight_gradient_pair_and_both_re_tilings_at_tile_edges(K, F, cnt):
             else:
                 assert bool((got[e] == 0).all())
         r += n
-    if K % 64 == 0 and F % 64 == 0:
-        w, wu = (torch.from_numpy(rng.standard_normal((E_l, K, F)).astype(np.float32)).bfloat16().to(DEV) for _ in range(2))
-        for up in (None, wu):
-            packed, packed_t = ops.prepack_weights_both(w, up)
-            assert torch.equal(packed, ops.prepack_weights(w, up)) and torch.equal(packed_t, ops.prepack_weights_transposed(w, up))
+
+
+@pytest.mark.parametrize("S,cnt,K,N", [(70, (33, 0, 35), 128, 72), (300, (1, 256, 40), 192, 328), (9000, (3000, 0, 5999), 64, 2056),
+                                       (5200, (5190,), 576, 4104), (2600, (700, 900, 1000), 4096, 264)])
+def test_weights_as_they_are_give_the_bits_of_re_tiled_ones(S, cnt, K, N):
+    """The GEMM on weights in the reference layout, and on their transposes, in both tile sizes, with and without the K split, with
+    partly filled tiles in every direction, against the re-tiled operand: the same sums in the same order."""
+    from iris_testing_amd import _lib as L
+    g = torch.Generator(device=DEV).manual_seed(S)
+    E_l = len(cnt)
+    c = torch.tensor(cnt, dtype=torch.int32, device=DEV)
+    ws = ops.gemm_part_workspace(DEV)
+    x = torch.randn(S, K, generator=g, device=DEV).bfloat16()
+    w = torch.randn(E_l, K, N, generator=g, device=DEV).bfloat16()
+    want = ops.expert_forward(x, ops.prepack_weights(w), L.W_TILED, c, N, ws)
+    assert torch.equal(ops.expert_forward(x, w, L.W_RAW, c, N, ws), want)
+    rows = torch.split(x[:sum(cnt)].float(), list(cnt))
+    ref = torch.cat([r @ w[e].float() for e, r in enumerate(rows)])
+    assert _rel(want[:sum(cnt)], ref.double().cpu()) < 2.0 ** -7 and bool((want[sum(cnt):] == 0).all())
+    wt = w.transpose(1, 2).contiguous()  # [E_l,N,K]
+    assert torch.equal(ops.expert_forward(x, wt, L.W_RAW_T, c, N, ws), want)
+
+
+@pytest.mark.parametrize("act", ["gelu", "silu", "swiglu"])
+@pytest.mark.parametrize("cnt,H,F", [((40, 0, 61), 192, 320), ((2500, 1300), 320, 1088)])
+def test_training_pass_on_weights_as_they_are(act, cnt, H, F):
+    """Forward with the weights as they are against the re-tiled ones (same bits), backward against the products it stands for."""
+    from iris_testing_amd import _lib as L
+    g = torch.Generator(device=DEV).manual_seed(H)
+    S, E_l = sum(cnt), len(cnt)
+    rnd = lambda *s: (torch.randn(*s, generator=g, device=DEV) * s[-2] ** -0.5).bfloat16()  # noqa: E731
+    x, w1, w2, dy = rnd(S, H), rnd(E_l, H, F), rnd(E_l, F, H), rnd(S, H)
+    wu = rnd(E_l, H, F) if act == "swiglu" else None
+    c, ws = torch.tensor(cnt, dtype=torch.int32, device=DEV), ops.gemm_part_workspace(DEV)
+    tiled = ops.mlp_train_forward(x, c, act, L.W_TILED, ops.prepack_weights(w1, wu), None, ops.prepack_weights(w2), F, part_ws=ws)
+    raw = ops.mlp_train_forward(x, c, act, L.W_RAW, w1, wu, w2, F, part_ws=ws)
+    for a, b, n in zip(tiled, raw, ("out", "hidden", "pre_act")):
+        assert torch.equal(a, b), n
+    out, hidden, pre = raw
+    dx, dw1, dw2, dw_up = ops.mlp_train_backward(x, hidden, pre, dy, c, act, L.W_RAW_T, w1, wu, w2, part_ws=ws)
+    tiled_t = (L.W_TILED, ops.prepack_weights_transposed(w1, wu), None, ops.prepack_weights_transposed(w2))
+    for a, b in zip((dx, dw1, dw2, dw_up), ops.mlp_train_backward(x, hidden, pre, dy, c, act, *tiled_t, part_ws=ws)):
+        assert a is b is None or torch.equal(a, b)
+    dh = ops.expert_forward(dy, ops.prepack_weights_transposed(w2), L.W_TILED, c, F, ws)
+    d_pre = ops.mlp_act_backward(pre, dh, act)
+    NP = pre.shape[1]
+    want = torch.zeros_like(x)
+    ops.grouped_gemm_mapped(d_pre, None, ops.prepack_weights_transposed(w1, wu), c, S, H, "none", want, part_ws=ws)
+    assert torch.equal(dx, want), "dx"
+    dw = ops.grouped_gemm_dw(x, d_pre, c, split_F=F if act == "swiglu" else 0)
+    assert torch.equal(dw1, dw[..., :F]) and (dw_up is None or torch.equal(dw_up, dw[..., F:])) and NP == dw.shape[-1]
+    assert torch.equal(dw2, ops.grouped_gemm_dw(hidden, dy, c))
