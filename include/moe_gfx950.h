@@ -241,10 +241,10 @@ int moe_grouped_mlp_fp8(const void* tokens_bf16, const int32_t* expert_cnt, int 
  *                           Map entries must lie inside their buffers or be negative: a negative a_row_map
  *                           entry reads row 0, a negative c_row_map entry stores nothing.  part_ws (nullable, part_ws_bytes
  *                           bytes, moe_gemm_part_workspace_bytes() for the full benefit): scratch for fp32
- *                           partial sums; with it, when the last round of the persistent grid holds at most
- *                           a quarter of a grid of tiles, those tiles are cut along K over the idle compute
- *                           units and summed in a fixed order by a second kernel (same result for the same
- *                           shapes and counts on every call; last-bit differences against the unsplit sum).
+ *                           partial sums; with it, launches of few tiles cut them along K over the idle compute
+ *                           units and add the parts in a fixed order (same result for the same shapes and counts
+ *                           on every call; last-bit differences against the uncut sum).  One launch at a time may
+ *                           use it: launches that may overlap (other streams) take scratch of their own.
  *   moe_zero_padding_rows   rows [sum_e recv_counts[s,e], M) of every slot s of buf [W,M,H] <- 0: what
  *                           moe_return_pack writes besides the result rows. */
 int moe_recv_row_map(const int32_t* recv_counts, int W, int E_l, int M, int n_rows, int32_t* row_map,
@@ -274,10 +274,10 @@ int moe_grouped_gemm_mapped_gated(const void* a_base, int a_rows, const int32_t*
                                   int out_rows, const int32_t* c_row_map, void* part_ws, size_t part_ws_bytes,
                                   moe_stream_t stream);
 size_t moe_gemm_part_workspace_bytes(void);
-/* How a launch with total_tiles output tiles, a persistent grid of `grid` workgroups, k_stages 64-byte stages of K
- * (even) and room for max_units part tiles in the workspace is walked: out[0] = tiles taken whole, out[1] = parts
- * per remaining tile (1: no split), out[2] = K stages per part, out[3] = work units in all.  Host-only arithmetic
- * (the kernels evaluate the same function); no counterpart in the reference. */
+/* How the last round of a launch with total_tiles large tiles, a persistent grid of `grid` workgroups, k_stages 64-byte stages of K
+ * (even) and room for max_units part tiles would be cut along K: out[0] = tiles taken whole, out[1] = parts per remaining
+ * tile (1: no split), out[2] = K stages per part, out[3] = work units in all.  Host-only arithmetic (the launches hand such
+ * a round to small tiles instead); no counterpart in the reference. */
 int moe_gemm_split_plan(int total_tiles, int grid, int k_stages, int max_units, int32_t* out);
 int moe_zero_padding_rows(void* buf, int dtype, int W, int M, int H, const int32_t* recv_counts, int E_l,
                           moe_stream_t stream);
@@ -296,7 +296,7 @@ int moe_shuffle_backward(const void* grad_rows, int dtype, int E_l, int W, int C
  * a_row_map[r] of a_base_bf16 (a_rows rows of H), the down GEMM writes result row r to row c_row_map[r]
  * of out (out_rows rows of H); either map may be NULL.  row_gate (nullable, fp32 [S_rows], as moe_recv_row_map_gated
  * returns it): result row r is multiplied by row_gate[r] before the one rounding (the gated return).  part_ws
- * (nullable): the K-split scratch of moe_grouped_gemm_mapped, used by both GEMMs in turn. */
+ * (nullable): the scratch of moe_grouped_gemm_mapped, used by both GEMMs in turn. */
 int moe_grouped_mlp_fp8_mapped(const void* a_base_bf16, int a_rows, const int32_t* a_row_map,
                                const int32_t* expert_cnt, int S_rows, int H, int F, int E_l,
                                const uint8_t* wgu_packed, const float* sg, const float* su, const uint8_t* wd_packed,
@@ -402,7 +402,7 @@ int moe_diag_mfma_loop(int fp8, int random_data, int iters, int workgroups, floa
 /* moe_diag_gemm_trace: where time goes inside the grouped GEMM.  After a call with a device buffer of `words` >=
  * moe_diag_gemm_trace_words() 64-bit words, the forward grouped-GEMM launches of the calling process (through any entry point
  * above; 256-row tiles, no activation or SwiGLU) run an instantiation of the same kernel that writes the device's 100 MHz wall
- * clock into the buffer, take whole tiles only (no K split of the last round), and overwrite what the launch before left:
+ * clock into the buffer, take every tile (none is left to small ones), and overwrite what the launch before left:
  *   words [256 w, 256 w + 256) of workgroup w: for each of its tiles in turn, the clock at the start of the tile's K loop, at the
  *     end of its K loop and at the end of its epilogue (the first 85 tiles);
  *   words [256 G, 256 G + 4096), G = number of workgroups = compute units: the clock at the end of every MFMA block (one 64-byte

@@ -43,6 +43,7 @@ struct GsParams {
     int ncols;                 // packed columns that exist (N, or 2 N for SwiGLU)
     int slots;                 // units up to which tiles are split: one workgroup per compute unit
     unsigned long long nonce;  // what this launch's arrival counters carry in their upper bits
+    int big_bm, big_grid;      // the tail of a launch of large tiles of big_bm rows (g.tail_max); 0: all rows
 };
 
 // How many parts every tile's K range is cut into.
@@ -63,7 +64,7 @@ __device__ __forceinline__ int gs_scan(int v) {
     return v;
 }
 
-template <int BM, bool FP8, int EPI, bool BSA, int BMODE>
+template <int BM, bool FP8, int EPI, bool BSA, int BMODE, bool TAIL>
 __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParams q) {
     constexpr bool BT = BMODE == GG_B_T, BN_PAIR = BMODE == GG_B_NP, BN_RAW = BMODE == GG_B_N || BN_PAIR;  // (see GG_B_*)
     static_assert(!FP8 || BMODE == GG_B_PACKED, "raw weights are a bf16 matter");
@@ -85,14 +86,16 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
 
     // ---- this workgroup's unit: group, column tile, row tile, part.  Every wave scans the row counts by itself (64 groups at
     // a time); counts that claim more rows than the buffers hold are cut at S_rows.
-    const int nt_all = (q.ncols + GS_BN - 1) / GS_BN;
+    // TAIL: the tiles are those of a launch of large tiles that fill no round of its grid, each cut into tiles of this kernel.
+    const int nt_all = TAIL ? p.Npad / GG_BN : (q.ncols + GS_BN - 1) / GS_BN;  // (TAIL: large tiles)
+    const int tm = TAIL ? q.big_bm : BM, subs = TAIL ? tm / BM * (GG_BN / GS_BN) : 1;
     int mt_all = 0;
     {
         int rows = 0;
         for (int g0 = 0; g0 < p.E_l; g0 += WAVE) {
             const int c = g0 + lane < p.E_l ? max(p.cnt[g0 + lane], 0) : 0;
             const int inc = gs_scan(c), rs = min(rows + inc - c, p.S_rows);
-            const int t = (min(c, p.S_rows - rs) + BM - 1) / BM;
+            const int t = (min(c, p.S_rows - rs) + tm - 1) / tm;
             int ts = t;
 #pragma unroll
             for (int off = 1; off < WAVE; off <<= 1) ts += __shfl_xor(ts, off, WAVE);
@@ -102,37 +105,46 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
         if constexpr (!FP8) gg_zero_tail(p, rows);
     }
     const int nk = (p.K * ES) / ROWB;
-    const int P = __builtin_amdgcn_readfirstlane(p.part_ws ? gs_parts((long long)mt_all * nt_all, q.slots, nk, p.max_units) : 1);
-    const int units = __builtin_amdgcn_readfirstlane(mt_all * nt_all * P);
+    // the launch's tiles [first, first + tiles / subs) of mt_all * nt_all
+    const int first = TAIL ? gg_whole_tiles(mt_all * nt_all, q.big_grid, p.tail_max) : 0;
+    const int tiles = __builtin_amdgcn_readfirstlane((mt_all * nt_all - first) * subs);
+    const int P = __builtin_amdgcn_readfirstlane(p.part_ws ? gs_parts(tiles, q.slots, nk, p.max_units) : 1);
+    const int units = tiles * P;
     // consecutive units share an XCD (workgroups b, b + 8, ... do): parts of a tile, then the row tiles of a weight panel
     const int per = (units + 7) / 8;
     const int unit = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
     if (((int)blockIdx.x >> 3) >= per || unit >= units) return;
-    const int tile = unit / P, part = unit % P;
+    const int tile = unit / P, part = unit % P, whole = first + tile / subs;
     int g = 0, row0 = 0, rv = 0, nt = 0;
     {
-        int rows = 0, tiles = 0;
+        int rows = 0, before = 0;
         for (int g0 = 0; g0 < p.E_l; g0 += WAVE) {
             const int c = g0 + lane < p.E_l ? max(p.cnt[g0 + lane], 0) : 0;
             const int inc = gs_scan(c), rs = min(rows + inc - c, p.S_rows);
             const int cc = min(c, p.S_rows - rs);
-            const int mt = (cc + BM - 1) / BM;
-            const int ti = gs_scan(mt), t0 = (tiles + ti - mt) * nt_all;
-            const unsigned long long hit = __ballot(mt > 0 && tile >= t0 && tile < t0 + mt * nt_all);
+            const int mt = (cc + tm - 1) / tm;
+            const int ti = gs_scan(mt), t0 = (before + ti - mt) * nt_all;
+            const unsigned long long hit = __ballot(mt > 0 && whole >= t0 && whole < t0 + mt * nt_all);
             if (hit) {
                 const int l = __builtin_ctzll(hit);
-                const int mt_g = __shfl(mt, l, WAVE), in = tile - __shfl(t0, l, WAVE);
+                const int mt_g = __shfl(mt, l, WAVE), in = whole - __shfl(t0, l, WAVE);
                 g = g0 + l;
+                int m = in % mt_g;
                 nt = in / mt_g;
-                const int m = in % mt_g;
-                row0 = __shfl(rs, l, WAVE) + m * BM;
-                rv = min(BM, __shfl(cc, l, WAVE) - m * BM);
+                if constexpr (TAIL) {
+                    gg_patch(in, mt_g, nt_all, m, nt);
+                    nt = nt * (GG_BN / GS_BN) + tile % (GG_BN / GS_BN);
+                }
+                const int r = m * tm + (TAIL ? tile % subs / (GG_BN / GS_BN) * BM : 0);
+                row0 = __shfl(rs, l, WAVE) + r;
+                rv = min(BM, __shfl(cc, l, WAVE) - r);
                 break;
             }
             rows = min(rows + __shfl(inc, WAVE - 1, WAVE), p.S_rows);
-            tiles += __shfl(ti, WAVE - 1, WAVE);
+            before += __shfl(ti, WAVE - 1, WAVE);
         }
     }
+    if (TAIL && (rv <= 0 || nt * GS_BN >= q.ncols)) return;  // (past the rows or columns; all parts of the tile alike)
     g = __builtin_amdgcn_readfirstlane(g); nt = __builtin_amdgcn_readfirstlane(nt);
     row0 = __builtin_amdgcn_readfirstlane(row0); rv = __builtin_amdgcn_readfirstlane(rv);
     const int nkp = P > 1 ? gg_part_stages(nk, P) : nk;
@@ -494,9 +506,17 @@ static void gs_launch(const GsParams& q0, void* part_ws, size_t part_ws_bytes, i
     }
     const int nt = (q.ncols + GS_BN - 1) / GS_BN;
     const long long ub = ((long long)q.g.S_rows + (long long)std::min(q.g.E_l, q.g.S_rows) * (BM - 1)) / BM * nt;  // most tiles there can be
-    const long long units = std::max<long long>(ub, q.g.part_ws ? std::min<long long>(q.slots, ub * GG_MAX_PARTS) : 0);
+    auto units = [&](long long tiles) {
+        return (unsigned)((std::max<long long>(tiles, q.g.part_ws ? std::min<long long>(q.slots, tiles * GG_MAX_PARTS) : 0) + 7) / 8 * 8);
+    };
     q.nonce = gs_nonce();
-    gemm_small_kernel<BM, FP8, EPI, BSA, BMODE><<<(unsigned)((units + 7) / 8 * 8), GS_THREADS, lds, s>>>(q);
+    if constexpr (BM == 64) {
+        if (q.big_bm) {
+            gemm_small_kernel<BM, FP8, EPI, BSA, BMODE, true><<<units((long long)q.g.tail_max * (q.big_bm / BM) * (GG_BN / GS_BN)), GS_THREADS, lds, s>>>(q);
+            return;
+        }
+    }
+    gemm_small_kernel<BM, FP8, EPI, BSA, BMODE, false><<<units(ub), GS_THREADS, lds, s>>>(q);
 }
 
 template <bool FP8>
@@ -534,34 +554,36 @@ static int gs_dispatch(const GsParams& q, int bm, int epi, void* ws, size_t byte
 
 // Tile height for a launch (32 or 64 rows), or 0: large tiles.  Both paths' times in us are estimated from what the host knows
 // -- the row total, not its split over the groups (every group adds about half a tile of ragged tail) -- with coefficients
-// fitted to 490 launches drawn over rows 16 .. 16384, 1 .. 32 groups, K and N 512 .. 8192, bf16 and fp8, even and skewed:
-//   large tiles: whole rounds of the persistent grid, each 0.70 us (256 rows) or 0.40 us (128 rows) per 64 bytes of K (fp8 a fifth
-//     more) and 4 us between tiles; the tiles of the last, part-filled round split along K as far as there are
-//     compute units, at 12 us for its two launches; 10 us for the launch;
+// fitted to 470 launches drawn over rows 16 .. 16384, 1 .. 32 groups, K and N 512 .. 8192, bf16 and fp8, even and skewed:
+//   large tiles: whole rounds of the persistent grid, each 0.46 us per 64 bytes of K (fp8 a fifth more) and 3.3 us between tiles; a
+//     part-filled last round 0.57 us (256 rows) or 0.33 us (128 rows), or what small tiles take for it where they get it (gg_tail);
+//     6 us for the launch;
 //   small tiles: 0.24 / 0.30 us per 128 bytes of K while every workgroup has a compute unit to itself, then in proportion to
-//     their number (times 1.2, fp8 1.4: the load path is shared); 5 us for the hand-over of a split tile, 8 us for the launch.
-// Over those launches the choice made from these estimates is within 1 % (geometric mean) of the better of the two, 1.31 times
-// faster than large tiles alone and in one launch of 490 more than 7 % slower than them: 27.5 -> 9.0 us at 512 rows x 1024 x 1024
+//     their number (times 1.2, fp8 1.4: the load path is shared); 5 us for the hand-over of a split tile, 7 us for the launch.
+// Over those launches the choice made from these estimates is within 0.5 % (geometric mean) of the better of the two, 1.19 times
+// faster than large tiles alone and in one launch of 470 more than 6 % slower than them: 27.5 -> 9.0 us at 512 rows x 1024 x 1024
 // (2 groups, bf16), 31 -> 21 us at 512 x 2048 x 4096, 49 -> 20 us for an fp8 MLP of 300 rows; the line lies at about one round of
 // large tiles.
 int gs_choose_bm(int S_rows, int E_l, int K, int ncols, bool fp8, int cus) {
-    const double E = std::min(E_l, S_rows), nk = (double)K * (fp8 ? 1 : 2) / ROWB;
+    const double E = std::min(E_l, S_rows), nk = (double)K * (fp8 ? 1 : 2) / ROWB, share = fp8 ? 1.4 : 1.225;
     const int nt = (ncols + GG_BN - 1) / GG_BN, nts = (ncols + GS_BN - 1) / GS_BN;
     const double t256 = (S_rows / 256.0 + 0.5 * E) * nt, t128 = (S_rows / 128.0 + 0.5 * E) * nt;
     const bool small_m = 0.62 * ceil(t128 / cus) < ceil(t256 / cus);
-    const double tiles = small_m ? t128 : t256, tile_us = nk * (small_m ? 0.40 : 0.70) * (fp8 ? 1.2 : 1.0);
+    const double tiles = small_m ? t128 : t256, rate = fp8 ? 1.2 : 1.0;
     const double full = floor(tiles / cus), rem = tiles - full * cus;
-    double best = 9.5 + full * (tile_us + 3.9);
-    if (rem > 0.5) {
-        const double P = std::max(1.0, std::min(std::min(floor(cus / rem), 8.0), floor(nk / 16)));
-        best += tile_us / P + 4.2 + (P > 1 ? 11.9 : 0);
+    const GgTail tail = gg_tail((int)nk, small_m ? 128 : 256, fp8, cus);
+    double best = 6 + full * (nk * 0.46 * rate + 3.3), last = nk * (small_m ? 0.33 : 0.57) * rate + 5.1;
+    if (E > 1 && tail.worth) {
+        best += 9.2;
+        if (rem <= tail.most) last = std::min(last, 8 + 0.15 * nk * share * std::max(1.0, rem * (small_m ? 4 : 8) / cus));
     }
+    if (rem > 0.5) best += last;
     int bm_best = 0;
     for (int bm : {32, 64}) {
         const double units = (S_rows / (double)bm + 0.5 * E) * nts;
         const double P = units < cus ? std::max(1.0, std::min(std::min(floor(cus / units), floor(nk / GS_MIN_PART_STAGES)), (double)GG_MAX_PARTS)) : 1.0;
         const double x = units * P / cus;
-        const double t = 8.3 + (P > 1 ? 5 : 0) + nk / 2 / P * (bm == 32 ? 0.24 : 0.30) * std::max(1.0, x * (fp8 ? 1.4 : 1.225)) + 1.8 * std::max(1.0, x / 2);
+        const double t = 7.4 + (P > 1 ? 5 : 0) + nk / 2 / P * (bm == 32 ? 0.24 : 0.30) * std::max(1.0, x * share) + 1.5 * std::max(1.0, x / 2);
         if (t < best) { best = t; bm_best = bm; }
     }
     return bm_best;
@@ -572,6 +594,15 @@ int launch_gemm_small(const GemmParams& p, bool fp8, int bm, int epi, void* ws, 
     q.g = p;
     q.ncols = epi == EPI_SWIGLU ? 2 * p.N : p.N;
     return fp8 ? gs_dispatch<true>(q, bm, epi, ws, bytes, cus, s) : gs_dispatch<false>(q, bm, epi, ws, bytes, cus, s);
+}
+
+int launch_gemm_tail(const GemmParams& p, bool fp8, int bm_big, int epi, void* ws, size_t bytes, int grid, hipStream_t s) {
+    GsParams q{};
+    q.g = p;
+    q.ncols = epi == EPI_SWIGLU ? 2 * p.N : p.N;
+    q.big_bm = bm_big;
+    q.big_grid = grid;
+    return fp8 ? gs_dispatch<true>(q, 64, epi, ws, bytes, grid, s) : gs_dispatch<false>(q, 64, epi, ws, bytes, grid, s);
 }
 
 }  // namespace moe_gg

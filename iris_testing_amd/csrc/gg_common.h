@@ -38,12 +38,11 @@ struct GemmParams {
     const int32_t* c_map;     // optional: logical row -> row of C (scatter while storing)
     int E_l, K, N, Npad, ldc, S_rows, ncs;
     int zero_tail;            // rows [counted total, S_rows) of C are zeroed (no c_map then)
-    // Optional split of the last, partly filled round of the persistent grid along K: when that round holds at
-    // most a quarter of a grid of tiles, each of them is cut into P parts of the K range, one per otherwise idle
-    // workgroup, which store their fp32 partial sums here (max_units part tiles of BM x 256 floats); a second
-    // kernel adds the parts of a tile in part order and applies the epilogue.  NULL: no split.
+    // Small tiles (gemm_small.hip): scratch for the fp32 partial sums of tiles whose K range is cut (max_units part tiles), or NULL.
     float* part_ws;
     int max_units;
+    // Large tiles: a last round of the persistent grid with at most this many tiles is left to a launch of small ones.
+    int tail_max;
     // Weight-gradient mode (template flag DW): C[g] (dw_rows x N, at C + g * c_group_stride elements) = x_g^T dy_g, the reduction
     // running over the rows of group g.  A is x [rows, dw_rows] and B is dy [rows, N], both as they are: the reduction index is
     // the slow one, a K stage is 32 rows of each, and the fragments are transposed on their way out of LDS.  With dw_split (F)
@@ -257,6 +256,39 @@ __device__ __forceinline__ void gg_wait() {
     __builtin_amdgcn_s_waitcnt((VM & 15) | (7 << 4) | (LGKM << 8) | ((VM >> 4) << 14));
 }
 
+constexpr int SUP = 16;  // super-tile edge, in large tiles
+// Tile idx of a group of Mt x Nt large tiles in the order they are walked: bands of 16 rows, super-columns of 16 within them.
+__device__ __forceinline__ void gg_patch(int idx, int Mt, int Nt, int& mt, int& nt) {
+    const int band = idx / (SUP * Nt), rem = idx % (SUP * Nt);
+    const int hr = min(SUP, Mt - band * SUP);
+    const int sc = rem / (hr * SUP), rem2 = rem % (hr * SUP);
+    const int wc = min(SUP, Nt - sc * SUP);
+    mt = band * SUP + rem2 / wc;
+    nt = sc * SUP + rem2 % wc;
+}
+
+// Tiles of a launch that the large kernel takes: all of them, or whole rounds of the grid when the rest is left to small tiles.
+__host__ __device__ inline int gg_whole_tiles(int total, int grid, int tail_max) {
+    const int tail = total % grid;
+    return tail <= tail_max ? total - tail : total;
+}
+
+// Tiles of a last round that fills less than a third of the grid or so: 64 x 128 tiles (gemm_small.hip) fill the chip with them sooner
+// than large ones leave it.  Per 64-byte K stage a small tile takes 0.15 us of a compute unit (times 1.2, fp8 1.4, where units
+// share the load path), a large one 0.47 us (128 rows: 0.30) while most of the chip idles beside it.  The launch costs 5 us when
+// the counts leave it nothing to do, so several groups get it only where the round is long enough for the chance of some
+// most / grid to be worth that.  (Before, such tiles were cut along K by a second launch and summed by a third, 9 us without a
+// tail: 777 tokens x 2 of 60 fp8 experts 181 -> 153 us, half of it those launches.)
+struct GgTail {
+    int most;    // tiles left over at most for the small ones to be quicker
+    bool worth;  // worth a launch that may find nothing
+};
+static inline GgTail gg_tail(int nk, int bm, bool fp8, int grid) {
+    const double round_us = nk * (bm == 128 ? 0.30 : 0.47) + 4;
+    const int most = (int)((round_us - 8) / (0.15 * nk * (fp8 ? 1.4 : 1.225)) * grid / (bm / 64 * 2));
+    return {most < 0 ? 0 : most < grid ? most : grid - 1, round_us >= 45};
+}
+
 constexpr int GG_MAX_PARTS = 16;       // parts a tile's K range is cut into, at most
 constexpr int GG_MIN_PART_STAGES = 8;  // K stages per part at least (64 bytes of K each)
 // stages per part when nk stages (even) are cut into P parts: even, and P of them cover nk
@@ -271,8 +303,10 @@ __device__ __forceinline__ void gg_zero_tail(const GemmParams& p, int total) {
         *(uint4*)((bf16_t*)p.C + (size_t)(total + i / nv) * p.ldc + (i % nv) * 8) = make_uint4(0, 0, 0, 0);
 }
 
-// gemm_small.hip: the tile height (32, 64 or 128 rows) of the small-tile kernel for a launch, 0 where the large tiles are the
+// gemm_small.hip: the tile height (32 or 64 rows) of the small-tile kernel for a launch, 0 where the large tiles are the
 // better choice; and that launch.
 int gs_choose_bm(int S_rows, int E_l, int K, int ncols, bool fp8, int cus);
 int launch_gemm_small(const GemmParams& p, bool fp8, int bm, int epi, void* ws, size_t bytes, int cus, hipStream_t s);
+// The tiles of a launch of large tiles (bm_big rows, grid workgroups) that GemmParams::tail_max left over.
+int launch_gemm_tail(const GemmParams& p, bool fp8, int bm_big, int epi, void* ws, size_t bytes, int grid, hipStream_t s);
 }  // namespace moe_gg

@@ -15,15 +15,14 @@
 //   * ragged group tails are masked (the reference assumes full tiles, kernels.py:270,282);
 //   * the tile walk is XCD-aware: the 32 workgroups that share an L2 take a compact 4 x 8 patch of
 //     a 16 x 16 super-tile;
-//   * a last round of the persistent grid that would leave most compute units idle is split along K over all
-//     of them (second launch + a reduction kernel that applies the epilogue), given a workspace.
+//   * the tiles of a last round of the persistent grid that fills less than about half of it go to a second launch of
+//     small tiles (gemm_small.hip), which fills the chip with them.
 #include "gg_common.h"
 #include <algorithm>
 #include <type_traits>
 
 namespace moe_gg {
 
-constexpr int SUP = 16;  // super-tile edge, in tiles
 #ifndef GG_BIG_NWM
 #define GG_BIG_NWM 2  // waves along M of the 256-row tile (x 2 along N)
 #endif
@@ -37,13 +36,12 @@ constexpr int SUP = 16;  // super-tile edge, in tiles
 #endif
 
 
-constexpr int GG_RED_SLABS = 32;   // blocks per tile in the reduction of the parts
-
-// How the tiles of a launch are walked: tiles [0, full) whole, tiles [full, total) in P parts each.
+// How a last round of large tiles would be walked if its tiles were cut along K: tiles [0, full) whole, tiles [full, total) in P
+// parts each (moe_gemm_split_plan; host arithmetic only).
 struct GgPlan {
     int total, full, P, nkp, units;
 };
-__host__ __device__ inline GgPlan gg_plan(int total, int grid, int nk, bool split, int max_units) {
+static GgPlan gg_plan(int total, int grid, int nk, bool split, int max_units) {
     GgPlan pl;
     pl.total = total; pl.full = total; pl.P = 1; pl.nkp = nk;
     const int tail = total % grid;
@@ -70,8 +68,7 @@ __device__ __forceinline__ int seg_of(const int* off, int n, int r) {
 // One output tile of the walk: group g, n tile nt, first row row0, rv valid rows (rv <= 0: none).
 struct GgTile {
     int g, nt, row0, rv;
-    int ks0, nks;   // first K stage and number of K stages this workgroup multiplies (the whole K range, or a part)
-    int unit;       // part tile index in the partial-sum workspace, or -1 for a whole tile
+    int ks0, nks;   // first K stage and number of K stages
 };
 
 // lin -> tile: group-major, 16-row bands, 16-column super-columns (see the XCD-aware walk above)
@@ -84,14 +81,11 @@ __device__ __forceinline__ GgTile gg_decode(const int* g_tile_start, const int* 
     const int cnt_g = DW ? dw_rows : g_row_start[g + 1] - g_row_start[g];
     const int Mt = (cnt_g + BM - 1) / BM;
     const int idx = lin - g_tile_start[g];
-    const int band = idx / (SUP * Nt), rem = idx % (SUP * Nt);
-    const int hr = min(SUP, Mt - band * SUP);
-    const int sc = rem / (hr * SUP), rem2 = rem % (hr * SUP);
-    const int wc = min(SUP, Nt - sc * SUP);
-    const int mt = band * SUP + rem2 / wc;
+    int mt, nt;
+    gg_patch(idx, Mt, Nt, mt, nt);
     GgTile t;
     t.g = g;
-    t.nt = sc * SUP + rem2 % wc;
+    t.nt = nt;
     t.row0 = (DW ? 0 : g_row_start[g]) + mt * BM;
     t.rv = DW ? min(BM, cnt_g - mt * BM) : min(min(BM, cnt_g - mt * BM), S_rows - t.row0);
     return t;
@@ -101,15 +95,14 @@ __device__ __forceinline__ GgTile gg_decode(const int* g_tile_start, const int* 
 // Decoding one costs a search and five integer divisions, so the workgroup decodes GG_TT of them at a time, one per
 // thread, into a table in LDS; the walk itself is then one 16-byte LDS read per tile.
 constexpr int GG_TT = 256;
-template <int BM, bool SPLIT, bool DW>
+template <int BM, bool DW>
 __device__ __forceinline__ void gg_fill_table(int4* s_tiles, const int* g_tile_start, const int* g_row_start, int E_l, int Nt,
-                                              int S_rows, const GgPlan& pl, int my, int stride, int round0, int dw_rows) {
-    const int n = SPLIT ? pl.units - pl.full : pl.full;
+                                              int S_rows, int n, int my, int stride, int round0, int dw_rows) {
     for (int i = threadIdx.x; i < GG_TT; i += blockDim.x) {
         const int lin = (round0 + i) * stride + my;
         int4 e = make_int4(0, 0, 0, 0);  // (g, nt, row0, rv); rv <= 0: nothing there
         if ((round0 + i) < (n + stride - 1) / stride && lin < n) {
-            const GgTile t = gg_decode<BM, DW>(g_tile_start, g_row_start, E_l, Nt, S_rows, SPLIT ? pl.full + lin / pl.P : lin, dw_rows);
+            const GgTile t = gg_decode<BM, DW>(g_tile_start, g_row_start, E_l, Nt, S_rows, lin, dw_rows);
             e = make_int4(t.g, t.nt, t.row0, t.rv);
         }
         s_tiles[i] = e;
@@ -118,13 +111,13 @@ __device__ __forceinline__ void gg_fill_table(int4* s_tiles, const int* g_tile_s
 
 // The tile of round `round` if the table holds it and it has rows (rv = 0 otherwise: the caller then takes the general
 // walk below).  One LDS read; nothing is advanced, refilled or skipped.
-template <bool SPLIT, bool DW>
-__device__ __forceinline__ GgTile gg_peek(const int4* s_tiles, const int* g_row_start, const GgPlan& pl, int nk, int my, int stride,
+template <bool DW>
+__device__ __forceinline__ GgTile gg_peek(const int4* s_tiles, const int* g_row_start, int nk, int my, int stride,
                                           int round, int round0) {
     GgTile t;
     t.g = t.nt = t.row0 = 0;
     t.rv = 0;
-    t.ks0 = 0; t.nks = nk; t.unit = -1;
+    t.ks0 = 0; t.nks = nk;
     if (round < round0 + GG_TT) {  // (past the end of the walk the table holds empty entries)
         const int4 e = s_tiles[round - round0];
         t.g = __builtin_amdgcn_readfirstlane(e.x); t.nt = __builtin_amdgcn_readfirstlane(e.y);
@@ -133,12 +126,6 @@ __device__ __forceinline__ GgTile gg_peek(const int4* s_tiles, const int* g_row_
             t.ks0 = g_row_start[t.g];  // (the group's first row)
             t.nks = (g_row_start[t.g + 1] - t.ks0 + 63) / 64 * 2;
         }
-        if constexpr (SPLIT) {
-            const int lin = round * stride + my;
-            t.ks0 = (lin % pl.P) * pl.nkp;
-            t.nks = min(pl.nkp, nk - t.ks0);
-            t.unit = lin;
-        }
     }
     return t;
 }
@@ -146,24 +133,22 @@ __device__ __forceinline__ GgTile gg_peek(const int4* s_tiles, const int* g_row_
 // Next non-empty tile of this workgroup at or after round `round` (advanced past it); rv = 0 when there is none.
 // round0 is the round the table starts at; the table is refilled (by the whole workgroup: every wave makes the same
 // calls) when the walk leaves it.
-template <int BM, bool SPLIT, bool DW>
+template <int BM, bool DW>
 __device__ __forceinline__ GgTile gg_walk(int4* s_tiles, const int* g_tile_start, const int* g_row_start, int E_l, int Nt, int S_rows,
-                                          const GgPlan& pl, int nk, int my, int stride, int& round, int& round0, int dw_rows) {
+                                          int n, int nk, int my, int stride, int& round, int& round0, int dw_rows) {
     GgTile t;
     t.g = t.nt = t.row0 = 0;
     t.rv = 0;
-    t.ks0 = 0; t.nks = nk; t.unit = -1;
-    const int n = SPLIT ? pl.units - pl.full : pl.full;
+    t.ks0 = 0; t.nks = nk;
     const int rounds = (n + stride - 1) / stride;
     while (round < rounds) {
         if (round >= round0 + GG_TT) {
             __syncthreads();  // (every wave has read what it needed of the old table)
             round0 = round;
-            gg_fill_table<BM, SPLIT, DW>(s_tiles, g_tile_start, g_row_start, E_l, Nt, S_rows, pl, my, stride, round0, dw_rows);
+            gg_fill_table<BM, DW>(s_tiles, g_tile_start, g_row_start, E_l, Nt, S_rows, n, my, stride, round0, dw_rows);
             __syncthreads();
         }
         const int4 e = s_tiles[round - round0];
-        const int lin = round * stride + my;
         ++round;
         const int rv = __builtin_amdgcn_readfirstlane(e.w);
         if (rv > 0) {
@@ -172,11 +157,6 @@ __device__ __forceinline__ GgTile gg_walk(int4* s_tiles, const int* g_tile_start
             if constexpr (DW) {
                 t.ks0 = g_row_start[t.g];
                 t.nks = (g_row_start[t.g + 1] - t.ks0 + 63) / 64 * 2;
-            }
-            if constexpr (SPLIT) {
-                t.ks0 = (lin % pl.P) * pl.nkp;
-                t.nks = min(pl.nkp, nk - t.ks0);
-                t.unit = lin;
             }
             break;
         }
@@ -199,17 +179,15 @@ __device__ __forceinline__ auto gg_stage_src(const uint8_t* base, size_t off, lo
 // stage s during block s -- every wave took the fragments of stage s into registers one block earlier -- spread
 // over the block, so the load pipe sees a steady stream instead of a burst and every load has more than two
 // blocks of MFMA work to land.
-// SPLIT = false: the launch that takes whole tiles.  SPLIT = true: the launch that takes the tiles of an
-// under-filled last round in parts of the K range and leaves fp32 partial sums in the workspace (GemmParams).
 // BSA: the activation operand carries block scales (fp8 down projection: GemmParams::a_bscale), applied by the MFMAs.
 // TRACE: the same kernel with time stamps (GemmParams::trace); product launches never use it.
-template <int BM, int NWM, int EPI, bool FP8, bool SPLIT, int BMODE = GG_B_PACKED, bool BSA = false, bool TRACE = false>
+template <int BM, int NWM, int EPI, bool FP8, int BMODE = GG_B_PACKED, bool BSA = false, bool TRACE = false>
 __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const GemmParams p) {
     constexpr bool DW = BMODE == GG_B_DW, BT = BMODE == GG_B_T, BN_PAIR = BMODE == GG_B_NP, BN_RAW = BMODE == GG_B_N || BN_PAIR;
     static_assert(!FP8 || BMODE == GG_B_PACKED, "raw weights are a bf16 matter");
-    static_assert(BMODE != GG_B_NP || EPI == EPI_SWIGLU || SPLIT, "pairs are what SwiGLU multiplies with");
+    static_assert(BMODE != GG_B_NP || EPI == EPI_SWIGLU, "pairs are what SwiGLU multiplies with");
     constexpr int BTR = DW ? 512 : 256;   // (operands transposed out of LDS) row pitch of a stage of B
-    static_assert(!TRACE || (!SPLIT && !DW), "time stamps: whole-tile forward launches only");
+    static_assert(!TRACE || !DW, "time stamps: whole-tile forward launches only");
     [[maybe_unused]] int tr_tile = 0, tr_blk = 0;  // (TRACE) words written so far
 #define GG_TRACE_TILE()                                                                                                    \
     do {                                                                                                                   \
@@ -218,11 +196,11 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
             ++tr_tile;                                                                                                     \
         }                                                                                                                  \
     } while (0)
-    static_assert(!DW || (!SPLIT && !FP8 && EPI == EPI_NONE), "the weight-gradient mode is a plain bf16 GEMM");
+    static_assert(!DW || (!FP8 && EPI == EPI_NONE), "the weight-gradient mode is a plain bf16 GEMM");
     static_assert(!BSA || FP8, "block scales belong to the fp8 MFMA");
-    constexpr bool VARK = SPLIT || DW;  // the K range differs from tile to tile
+    constexpr bool VARK = DW;  // the K range differs from tile to tile
     constexpr bool PEEL = !VARK && !BSA;  // the tile's first two blocks written out apart (see below)
-    constexpr bool QOUT = FP8 && EPI == EPI_SWIGLU && !SPLIT;  // the epilogue stores e4m3 codes and block scales
+    constexpr bool QOUT = FP8 && EPI == EPI_SWIGLU;  // the epilogue stores e4m3 codes and block scales
     constexpr int BN = GG_BN;
     constexpr int ES = FP8 ? 1 : 2;
     constexpr int NW = NWM * 2;                        // waves per workgroup
@@ -311,8 +289,7 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
     }
     if constexpr (!DW && !FP8) gg_zero_tail(p, g_row_start[p.E_l]);
     const int nk = (p.K * ES) / ROWB;  // ring stages per tile; even (K * ES is a multiple of 2 * ROWB)
-    const GgPlan plan = gg_plan(g_tile_start[p.E_l], (int)gridDim.x, nk, !DW && p.part_ws != nullptr, p.max_units);
-    if (SPLIT && plan.P == 1) return;  // nothing was left over for this launch
+    const int n_tiles = gg_whole_tiles(g_tile_start[p.E_l], (int)gridDim.x, DW ? 0 : p.tail_max);
 
     // XCD-aware position inside a round of gridDim.x tiles: workgroups b, b+8, b+16, ... share an L2.
     int my = blockIdx.x;
@@ -478,9 +455,9 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
     } while (0)
 
     int round = 0, round0 = 0;
-    gg_fill_table<BM, SPLIT, DW>(s_tiles, g_tile_start, g_row_start, p.E_l, Nt, p.S_rows, plan, my, (int)gridDim.x, 0, p.dw_rows);
+    gg_fill_table<BM, DW>(s_tiles, g_tile_start, g_row_start, p.E_l, Nt, p.S_rows, n_tiles, my, (int)gridDim.x, 0, p.dw_rows);
     __syncthreads();
-    GgTile cur = gg_walk<BM, SPLIT, DW>(s_tiles, g_tile_start, g_row_start, p.E_l, Nt, p.S_rows, plan, nk, my, (int)gridDim.x, round, round0, p.dw_rows);
+    GgTile cur = gg_walk<BM, DW>(s_tiles, g_tile_start, g_row_start, p.E_l, Nt, p.S_rows, n_tiles, nk, my, (int)gridDim.x, round, round0, p.dw_rows);
     uint32_t a_off[RA];
     const uint8_t *Ab = p.A, *Bb = p.B;
     if (cur.rv > 0) {
@@ -504,7 +481,6 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
         const int g = __builtin_amdgcn_readfirstlane(cur.g), nt = __builtin_amdgcn_readfirstlane(cur.nt);
         const int row0 = __builtin_amdgcn_readfirstlane(cur.row0), rv = __builtin_amdgcn_readfirstlane(cur.rv);
         const int nks = VARK ? __builtin_amdgcn_readfirstlane(cur.nks) : nk;
-        const int unit = SPLIT ? __builtin_amdgcn_readfirstlane(cur.unit) : -1;
 
         typedef typename std::conditional<FP8, floatx16, floatx4>::type acc_t;
         acc_t acc[TM][TN];  // (not cleared where the MFMAs of the tile's first block start the sums)
@@ -568,7 +544,7 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
             /* from block nks - 4 on the loads fetch the next tile, if it is at hand; not in a tile's first block: the  \
                row map that the tile's top requested must have landed and been handed over (one block end at least) */ \
             if ((s) == nks - 4 && (s) > 0) {                                                             \
-                const GgTile pk_ = gg_peek<SPLIT, DW>(s_tiles, g_row_start, plan, nk, my, (int)gridDim.x, round, round0); \
+                const GgTile pk_ = gg_peek<DW>(s_tiles, g_row_start, nk, my, (int)gridDim.x, round, round0); \
                 if (pk_.rv > 0) {                                                                        \
                     GG_TILE_PTRS(pk_, Ab_s, Bb_s, a_off_s, GG_MAPROW_LDS);                               \
                     Ab = Ab_s;                                                                           \
@@ -620,14 +596,14 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
             if (p.a_map) {
                 // the input rows of the NEXT tile, one per thread, straight into LDS: the switch to the next tile inside
                 // this tile's K loop then reads them from there instead of waiting for memory
-                const GgTile pk = gg_peek<SPLIT, DW>(s_tiles, g_row_start, plan, nk, my, (int)gridDim.x, round, round0);
+                const GgTile pk = gg_peek<DW>(s_tiles, g_row_start, nk, my, (int)gridDim.x, round, round0);
                 if (pk.rv > 0 && wave_s * WAVE < BM) {
                     const int tid_a = wave_s * WAVE + gg_lane_now();
                     gg_dma4(gg_uniform((const uint8_t*)(p.a_map + pk.row0)), (uint32_t)min(tid_a, pk.rv - 1) * 4u,
                             __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr_t)(s_amap + wave_s * WAVE)));
                 }
             }
-            if constexpr (!SPLIT) {
+            {
                 // What the epilogue needs from global memory per tile row / column (fp8 scales, the output row map) is
                 // requested here, straight into LDS, one value per thread (into the copy the previous tile does not
                 // use): the loads land during the first K stages (they are older than every load the K loop waits
@@ -732,7 +708,7 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
         // have passed the barrier: the last fragments of this tile are already in registers)
         // (when the K loop has switched over, the walk only confirms what the look-ahead saw)
         GG_TRACE_TILE();
-        const GgTile nxt = gg_walk<BM, SPLIT, DW>(s_tiles, g_tile_start, g_row_start, p.E_l, Nt, p.S_rows, plan, nk, my, (int)gridDim.x, round, round0, p.dw_rows);
+        const GgTile nxt = gg_walk<BM, DW>(s_tiles, g_tile_start, g_row_start, p.E_l, Nt, p.S_rows, n_tiles, nk, my, (int)gridDim.x, round, round0, p.dw_rows);
         if (!seam && nxt.rv > 0) {
             GG_TILE_PTRS(nxt, Ab_n, Bb_n, a_off_n, GG_MAPROW_GLOBAL);
             Ab = Ab_n;
@@ -744,35 +720,6 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
             GG_PROLOGUE(Ab, Bb, a_off, (VARK ? nxt.nks : nk));
         }
         const int phi_n = seam ? ((phi + nks) & 3) : 0;
-
-        // ---- a part of a tile: its fp32 partial sums go to the workspace as they are (tile row major, 256
-        // columns; the lane's runs of four columns as 16-byte stores); the reduction kernel does the rest
-        if constexpr (SPLIT) {  // (every tile of this instantiation is a part; the epilogue below is the other one's)
-            float* wsT = p.part_ws + (size_t)unit * (BM * BN);
-            constexpr int NQp = FP8 ? 4 : 1;
-            const int lane_p = gg_lane_now(), rbase_p = (wave_s >> 1) * (BM / NWM);
-            const int clp = FP8 ? (lane_p >> 5) * 4 : (lane_p >> 4) * 4;
-#pragma unroll
-            for (int i = 0; i < TM; ++i) {
-                const int r = rbase_p + i * MT + (lane_p & (MT - 1));
-#pragma unroll
-                for (int j = 0; j < TN; ++j) {
-#pragma unroll
-                    for (int q = 0; q < NQp; ++q) {
-                        const int c = wn * (BN / 2) + j * MT + 8 * q + clp;
-                        const float4 v = make_float4(acc[i][j][4 * q + 0], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2],
-                                                     acc[i][j][4 * q + 3]);
-                        if (r < rv) *(float4*)(wsT + (size_t)r * BN + c) = v;
-                    }
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            cur = nxt;
-            pre = seam;
-            phi = phi_n;
-            tpar ^= 1;
-            continue;
-        }
 
         // ---- epilogue: acc -> (scales) -> activation -> bf16 -> C
         // acc(i,j) holds the TRANSPOSED MT x MT product (weights as the MFMA A operand, activations as B):
@@ -992,126 +939,6 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
 #undef GG_SC_READ
 #undef GG_TR_A
 #undef GG_TR_B
-}
-
-// ---- second half of a K-split tile: add its parts in part order, then the epilogue of the GEMM kernel ------------
-// Same tile tables and the same plan as the GEMM launch it follows (gemm_grid = that launch's grid).  A block takes
-// BM / GG_RED_SLABS rows of one split tile (many small blocks: the partial sums of a few tiles are tens of MB); a thread takes four consecutive output columns of a row (for SwiGLU the gate
-// columns and, 32 packed columns further, their up columns).
-template <int BM, int EPI, bool FP8>
-__global__ __launch_bounds__(256) void gg_reduce_parts_kernel(const GemmParams p, int gemm_grid) {
-    constexpr int BN = GG_BN;
-    constexpr int ES = FP8 ? 1 : 2;
-    constexpr int RSL = GG_RED_SLABS;  // row slabs (blocks) per tile
-    __shared__ int g_tile_start[GG_MAXG + 1];
-    __shared__ int g_row_start[GG_MAXG + 1];
-    const int Nt = p.Npad / BN;
-    if (threadIdx.x == 0) {
-        int ts = 0, rs = 0;
-        for (int g = 0; g < p.E_l; ++g) {
-            g_tile_start[g] = ts;
-            g_row_start[g] = rs;
-            const int c = min(max(p.cnt[g], 0), max(p.S_rows - rs, 0));  // (clamped like the GEMM launch clamps it)
-            ts += ((c + BM - 1) / BM) * Nt;
-            rs += c;
-        }
-        g_tile_start[p.E_l] = ts;
-        g_row_start[p.E_l] = rs;
-    }
-    __syncthreads();
-    const int nk = (p.K * ES) / ROWB;
-    const GgPlan plan = gg_plan(g_tile_start[p.E_l], gemm_grid, nk, true, p.max_units);
-    if (plan.P == 1) return;
-    const int ti = blockIdx.x / RSL, slab = blockIdx.x % RSL;
-    if (ti >= plan.total - plan.full) return;
-    const GgTile t = gg_decode<BM>(g_tile_start, g_row_start, p.E_l, Nt, p.S_rows, plan.full + ti);
-    if (t.rv <= 0) return;
-    const float* ws = p.part_ws + (size_t)ti * plan.P * (BM * BN);
-    constexpr int OC4 = (EPI == EPI_SWIGLU ? BN / 2 : BN) / 4;  // groups of four output columns per tile row
-    constexpr int RPP = 256 / OC4;                               // rows per pass of the block
-    const int oc = (threadIdx.x % OC4) * 4;                      // first output column of the thread inside the tile
-    const int pc = EPI == EPI_SWIGLU ? (oc / 32) * 64 + oc % 32 : oc;  // its packed column inside the tile
-    const int gp = t.nt * BN + pc;                               // packed column of the launch
-    const int col = EPI == EPI_SWIGLU ? (gp / 64) * 32 + gp % 32 : gp;  // output column
-    float4 sc0 = make_float4(1.f, 1.f, 1.f, 1.f), sc1 = sc0;
-    if (FP8 && col < p.N) {
-        sc0 = *(const float4*)(p.col_scale + (size_t)t.g * p.ncs + col);
-        if constexpr (EPI == EPI_SWIGLU) sc1 = *(const float4*)(p.col_scale2 + (size_t)t.g * p.ncs + col);
-    }
-    bf16_t* C = (bf16_t*)p.C;
-    const int r_end = min((slab + 1) * (BM / RSL), t.rv);
-    for (int r = slab * (BM / RSL) + threadIdx.x / OC4; r < r_end; r += RPP) {
-        const float* w = ws + (size_t)r * BN + gg_packed_row<FP8>(pc);  // (parts are stored by row of the weight tile)
-        float4 a = *(const float4*)w, b = make_float4(0.f, 0.f, 0.f, 0.f);
-        if constexpr (EPI == EPI_SWIGLU) b = *(const float4*)(w + 32);
-        for (int part = 1; part < plan.P; ++part) {
-            const float* wp = w + (size_t)part * (BM * BN);
-            const float4 v = *(const float4*)wp;
-            a.x += v.x; a.y += v.y; a.z += v.z; a.w += v.w;
-            if constexpr (EPI == EPI_SWIGLU) {
-                const float4 u = *(const float4*)(wp + 32);
-                b.x += u.x; b.y += u.y; b.z += u.z; b.w += u.w;
-            }
-        }
-        const size_t grow = (size_t)(t.row0 + r);
-        float rs = 1.f;
-        if constexpr (FP8 || EPI == EPI_GATE) rs = p.row_scale ? p.row_scale[grow] : 1.f;  // (fp8 down projection: a gate, or nothing)
-        float av[4] = {a.x, a.y, a.z, a.w}, bv[4] = {b.x, b.y, b.z, b.w};
-        if constexpr (!FP8 && EPI != EPI_NONE && EPI != EPI_GATE) {
-            if (p.C2 && col < p.N) {  // the values before the activation, kept for the backward pass (rows are never remapped there)
-                constexpr int W2 = EPI == EPI_SWIGLU ? 2 : 1;
-                bf16_t* r2 = (bf16_t*)p.C2 + grow * (size_t)p.ldc * W2 + (EPI == EPI_SWIGLU ? gp : col);
-                uint2 o2;
-                o2.x = gg_pack_bf16(av[0], av[1]); o2.y = gg_pack_bf16(av[2], av[3]);
-                *(uint2*)r2 = o2;
-                if constexpr (EPI == EPI_SWIGLU) {
-                    o2.x = gg_pack_bf16(bv[0], bv[1]); o2.y = gg_pack_bf16(bv[2], bv[3]);
-                    *(uint2*)(r2 + 32) = o2;
-                }
-            }
-        }
-        const float c0[4] = {sc0.x, sc0.y, sc0.z, sc0.w}, c1[4] = {sc1.x, sc1.y, sc1.z, sc1.w};
-        float x[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            if constexpr (EPI == EPI_SWIGLU) {
-                float gv = av[e], uv = bv[e];
-                if constexpr (FP8) { gv *= c0[e] * rs; uv *= c1[e] * rs; }
-                x[e] = act_silu_fast(gv) * uv;
-            } else {
-                float v = av[e];
-                if constexpr (FP8) v *= c0[e] * rs;
-                if constexpr (!FP8 && EPI == EPI_GATE) v *= rs;
-                if constexpr (EPI == EPI_GELU) v = act_gelu(v);
-                if constexpr (EPI == EPI_SILU) v = act_silu_fast(v);
-                x[e] = v;
-            }
-        }
-        const int crow = p.c_map ? p.c_map[grow] : 0;
-        if constexpr (FP8 && EPI == EPI_SWIGLU) {
-            // quantised output, as in the GEMM kernel's epilogue: the eight threads that hold a block of 32 columns of this
-            // row (consecutive lanes; every thread of the block is in the loop together: r depends on threadIdx.x / OC4 only)
-            float am = fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3])));
-            if (col >= p.N) am = 0.f;
-#pragma unroll
-            for (int off = 1; off < 8; off <<= 1) am = fmaxf(am, __shfl_xor(am, off, WAVE));
-            const int sbyte = gg_block_scale_byte(__float_as_uint(am));
-            const float inv = __uint_as_float(gg_block_inv_bits(sbyte));
-            int cd = 0;
-            cd = __builtin_amdgcn_cvt_pk_fp8_f32(__fmul_rn(x[0], inv), __fmul_rn(x[1], inv), cd, false);
-            cd = __builtin_amdgcn_cvt_pk_fp8_f32(__fmul_rn(x[2], inv), __fmul_rn(x[3], inv), cd, true);
-            if (col < p.N && crow >= 0) {
-                const size_t orow = p.c_map ? (size_t)crow : grow;
-                *(uint32_t*)((uint8_t*)p.C + orow * p.ldc + col) = (uint32_t)cd;
-                if ((col & 31) == 0) p.c_bscale[orow * p.bs_pitch + col / 32] = (uint8_t)sbyte;
-            }
-        } else if (col < p.N && crow >= 0) {
-            uint2 o;
-            o.x = gg_pack_bf16(x[0], x[1]);
-            o.y = gg_pack_bf16(x[2], x[3]);
-            *(uint2*)(C + (p.c_map ? (size_t)crow : grow) * p.ldc + col) = o;
-        }
-    }
 }
 
 // ---- one-time weight re-tiling: w [E_l,K,N] (N contiguous) -> out [E_l][K/SK][Npad][SK], SK = one LDS
@@ -1721,37 +1548,26 @@ int launch_gemm(const GemmParams& p_in, int epi, hipStream_t s, void* part_ws = 
     const int nt = p.Npad / GG_BN;
     const double t256 = ((double)p.S_rows / 256 + 0.5 * p.E_l) * nt, t128 = ((double)p.S_rows / 128 + 0.5 * p.E_l) * nt;
     const bool small_m = 0.62 * ceil(t128 / grid) < ceil(t256 / grid);
-    // with a workspace, the tiles of a last round that fills at most a quarter of the grid are split along K
-    // (decided on the device from the row counts); the reduction kernel finds nothing to do otherwise
-    p.part_ws = nullptr;
-    p.max_units = 0;
-    if (part_ws) {
-        p.max_units = (int)std::min<size_t>(part_ws_bytes / ((size_t)(small_m ? 128 : 256) * GG_BN * sizeof(float)), (size_t)grid);
-        if (p.max_units >= 2) p.part_ws = (float*)part_ws;
+    const int bm = small_m ? 128 : 256;
+    const GgTail t = gg_tail(p.K * (FP8 ? 1 : 2) / ROWB, bm, FP8, grid);
+    p.tail_max = traced ? 0 : t.most;
+    if (p.E_l == 1) {  // (no group but this one: the host knows what is left over)
+        const int total = ceil_div(p.S_rows, bm) * nt;
+        if (gg_whole_tiles(total, grid, p.tail_max) == total) p.tail_max = 0;
+    } else if (!t.worth) {
+        p.tail_max = 0;
     }
-    const int red_blocks = (grid / 4) * GG_RED_SLABS;
-    // A launch so small that all its tiles are certain to be split (whatever the row counts turn out to be, there are at most
-    // ub of them: every group adds at most one partly filled row of tiles) has no whole tile: the first kernel is left out.
-    // gg_plan finds two parts or more whenever 4 tail <= grid, the K range has 16 stages and the workspace holds 2 tail units.
-    const int bm = small_m ? 128 : 256, nk = p.K * (FP8 ? 1 : 2) / ROWB;
-    const long long ub = ((long long)(p.S_rows + bm - 1) / bm + p.E_l) * nt;
-    const bool all_split = p.part_ws && red_blocks > 0 && 4 * ub <= grid && nk >= 2 * GG_MIN_PART_STAGES && p.max_units >= 2 * ub;
     // fp8 without activation is the down projection of the expert MLP: its activation operand is block-scaled
 #define GG_LAUNCH(BMv, NWMv, EPIv, MODEv)                                                                      \
     do {                                                                                                  \
         constexpr bool BSAv = FP8 && EPIv == EPI_NONE;                                                    \
         if (traced) {                                                                                     \
             if constexpr (BMv == 256 && (EPIv == EPI_NONE || EPIv == EPI_SWIGLU))                         \
-                grouped_gemm_kernel<BMv, NWMv, EPIv, FP8, false, GG_B_PACKED, BSAv, true><<<grid, NWMv * 2 * WAVE, 0, s>>>(p); \
+                grouped_gemm_kernel<BMv, NWMv, EPIv, FP8, GG_B_PACKED, BSAv, true><<<grid, NWMv * 2 * WAVE, 0, s>>>(p); \
             else return moe_fail(MOE_ERR_UNSUPPORTED, "grouped_gemm: no time-stamping instantiation for this launch (256-row tiles, no activation or SwiGLU)"); \
             break;                                                                                        \
         }                                                                                                 \
-        if (!all_split) grouped_gemm_kernel<BMv, NWMv, EPIv, FP8, false, MODEv, BSAv><<<grid, NWMv * 2 * WAVE, 0, s>>>(p); \
-        if (p.part_ws && red_blocks > 0) {                                                                \
-            /* (the launch that takes parts stores raw partial sums: one instantiation whatever the epilogue) */ \
-            grouped_gemm_kernel<BMv, NWMv, EPI_NONE, FP8, true, MODEv, BSAv><<<grid, NWMv * 2 * WAVE, 0, s>>>(p); \
-            gg_reduce_parts_kernel<BMv, EPIv, FP8><<<red_blocks, 256, 0, s>>>(p, grid);                    \
-        }                                                                                                 \
+        grouped_gemm_kernel<BMv, NWMv, EPIv, FP8, MODEv, BSAv><<<grid, NWMv * 2 * WAVE, 0, s>>>(p); \
     } while (0)
 #define GG_EPI_MODE(EPIv, MODEv)                     \
     do {                                             \
@@ -1759,6 +1575,12 @@ int launch_gemm(const GemmParams& p_in, int epi, hipStream_t s, void* part_ws = 
         else GG_LAUNCH(256, (FP8 ? (EPIv == EPI_NONE ? GG_FP8_BSA_NWM : GG_FP8_NWM) : GG_BIG_NWM), EPIv, MODEv); \
     } while (0)
 #define GG_EPI(EPIv) GG_EPI_MODE(EPIv, GG_B_PACKED)
+    auto tail = [&]() -> int {
+        if (!p.tail_max) return moe_check_launch("grouped_gemm");
+        GemmParams q = p;
+        q.zero_tail = 0;
+        return launch_gemm_tail(q, FP8, bm, epi, part_ws, part_ws_bytes, grid, s);
+    };
     if constexpr (!FP8) {  // weights in the reference layout
         if (p.b_mode != GG_B_PACKED) {
             if (traced) return moe_fail(MOE_ERR_UNSUPPORTED, "grouped_gemm: no time-stamping instantiation for weights in the reference layout");
@@ -1768,7 +1590,7 @@ int launch_gemm(const GemmParams& p_in, int epi, hipStream_t s, void* part_ws = 
             else if (p.b_mode == GG_B_N && epi == EPI_SILU) GG_EPI_MODE(EPI_SILU, GG_B_N);
             else if (p.b_mode == GG_B_NP && epi == EPI_SWIGLU) GG_EPI_MODE(EPI_SWIGLU, GG_B_NP);
             else return moe_fail(MOE_ERR_INVALID, "grouped_gemm: weight mode %d with activation %d", p.b_mode, epi);
-            return moe_check_launch("grouped_gemm");
+            return tail();
         }
     }
     switch (epi) {
@@ -1786,7 +1608,7 @@ int launch_gemm(const GemmParams& p_in, int epi, hipStream_t s, void* part_ws = 
 #undef GG_EPI
 #undef GG_EPI_MODE
 #undef GG_LAUNCH
-    return moe_check_launch("grouped_gemm");
+    return tail();
 }
 
 int launch_f32(const float* A, const float* W, const float* U, float* C, const int32_t* cnt, int E_l, int K, int N, int S_rows,
@@ -2163,7 +1985,7 @@ static int launch_dw(const void* x, const void* dy, const int32_t* expert_cnt, i
     p.A = (const uint8_t*)x; p.B = (const uint8_t*)dy; p.C = dw; p.cnt = expert_cnt;
     p.E_l = E_l; p.K = 64; p.N = N; p.Npad = round_up(N, GG_BN); p.ldc = ldc; p.S_rows = K;
     p.dw_rows = K; p.dw_src_rows = S_rows; p.dw_split = split_F; p.dw_delta = dw_delta; p.c_group_stride = (size_t)K * ldc;
-    grouped_gemm_kernel<256, GG_BIG_NWM, EPI_NONE, false, false, GG_B_DW><<<num_cus(), GG_BIG_NWM * 2 * WAVE, 0, s>>>(p);
+    grouped_gemm_kernel<256, GG_BIG_NWM, EPI_NONE, false, GG_B_DW><<<num_cus(), GG_BIG_NWM * 2 * WAVE, 0, s>>>(p);
     return moe_check_launch("grouped_gemm_dw");
 }
 

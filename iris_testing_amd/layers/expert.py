@@ -4,6 +4,7 @@ expert MLP the workloads define (Linear-act-Linear, SwiGLU, fp8) which the refer
 from __future__ import annotations
 
 import weakref
+from collections import OrderedDict
 from dataclasses import dataclass, field
 from typing import Optional
 
@@ -18,7 +19,8 @@ from ..utils import _assert_cuda_int32
 # a weight that did not change between calls is re-tiled once, not on every call (the re-tiling reads and writes the
 # whole tensor).  Entries die with their tensors (weak references); an in-place update bumps the version and re-tiles.
 _PACKED = {}
-_PART_WS = {}
+_PART_WS = OrderedDict()
+_PART_WS_MAX = 4  # streams with a workspace of their own (67 MB each); the one not used for longest is given back
 
 
 def _pack_key(kind: str, w: torch.Tensor, w_up: Optional[torch.Tensor]):
@@ -78,10 +80,18 @@ def _grouped_gemm_t(do: torch.Tensor, weights: torch.Tensor, cnt: torch.Tensor) 
 
 
 def _part_ws(device) -> torch.Tensor:
-    """One partial-sum workspace per device for the K split of an under-filled last round of GEMM tiles."""
-    ws = _PART_WS.get(device)
+    """Partial-sum workspace for the K split of GEMMs of few tiles: one per device and stream, since launches that may overlap must not
+    share it."""
+    key = (device, L.stream_ptr())
+    ws = _PART_WS.pop(key, None)
     if ws is None:
-        ws = _PART_WS[device] = ops.gemm_part_workspace(device)
+        ws = ops.gemm_part_workspace(device)
+    _PART_WS[key] = ws  # (now the last)
+    while len(_PART_WS) > _PART_WS_MAX:
+        try:
+            _PART_WS.popitem(last=False)
+        except KeyError:  # (another thread was quicker)
+            break
     return ws
 
 

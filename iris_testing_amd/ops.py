@@ -571,7 +571,7 @@ def grouped_gemm_mapped(a_base: torch.Tensor, a_row_map: Optional[torch.Tensor],
                         c_row_map: Optional[torch.Tensor] = None, part_ws: Optional[torch.Tensor] = None) -> torch.Tensor:
     """grouped_gemm_packed with row indirection on the way in (a_base rows a_row_map[r]) and / or on the
     way out (out rows c_row_map[r]).  a_base and out are 2-D views [rows, K] / [rows, N].  part_ws: optional
-    scratch (gemm_part_workspace) that lets an under-filled last round of tiles be split along K."""
+    scratch (gemm_part_workspace) that lets launches of few tiles be cut along K."""
     _req_cuda(a_base, "a_base")
     _req_i32(expert_cnt, "expert_cnt")
     assert a_base.dtype == torch.bfloat16 and out.dtype == torch.bfloat16 and a_base.dim() == 2 and out.dim() == 2
@@ -609,7 +609,7 @@ def grouped_gemm_act_keep(a_base: torch.Tensor, packed: torch.Tensor, expert_cnt
 
 
 def gemm_part_workspace(device) -> torch.Tensor:
-    """fp32 scratch for the K-split of grouped_gemm_mapped, sized for any launch."""
+    """fp32 scratch for the K split of grouped_gemm_mapped, sized for any launch (one launch at a time may use it)."""
     return torch.empty(L.lib().moe_gemm_part_workspace_bytes() // 4, dtype=torch.float32, device=device)
 
 

@@ -100,7 +100,7 @@ class DispatchPipeline:
         self.ret = torch.empty((W, M, H), dtype=dt, device=dev) if not self.padding_free else None
         self.ret_map = i32(lib.moe_recv_map_ints(W, E_l, W * M))
         self.row_map = i32(max(S, 1))
-        # scratch for the K-split of an under-filled last round of GEMM tiles (bf16 and fp8 experts)
+        # scratch for GEMMs of few tiles, which are cut along K (bf16 and fp8 experts)
         self.part_ws_bytes = lib.moe_gemm_part_workspace_bytes() if weights.dtype in (torch.bfloat16, torch.uint8) else 0
         self.part_ws = torch.empty(self.part_ws_bytes // 4, dtype=torch.float32, device=dev) if self.part_ws_bytes else None
         if weights.dtype == torch.uint8:

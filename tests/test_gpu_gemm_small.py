@@ -20,7 +20,9 @@ def _close(got, ref, what):
 # (rows per group, K, N, activation): one row; a tile's edge on either side; one pair of stages and an odd number of pairs;
 # a partly filled group of 32 columns, a partly filled tile; K ranges long enough to be cut into parts; more groups than lanes
 CASES = [((1,), 64, 8, "none"), ((31, 32, 33), 192, 136, "none"), ((63, 0, 64, 65), 320, 96, "swiglu"), ((5, 130), 64, 264, "gelu"),
-         ((17,), 8192, 256, "none"), ((40, 3), 4096, 512, "swiglu"), ((64,), 7168, 1032, "silu"), (tuple([1, 0, 2] * 30), 128, 128, "none")]
+         ((17,), 8192, 256, "none"), ((40, 3), 4096, 512, "swiglu"), ((64,), 7168, 1032, "silu"), (tuple([1, 0, 2] * 30), 128, 128, "none"),
+         # launches of large tiles (128 and 256 rows) whose last round of tiles is handed to small ones
+         ((4701,), 2048, 4096, "none"), ((8900, 0, 1000), 3072, 2528, "swiglu")]
 
 
 @pytest.mark.parametrize("cnt,K,N,act", CASES, ids=[f"{len(c[0])}g_{sum(c[0])}x{c[1]}x{c[2]}_{c[3]}" for c in CASES])
@@ -70,7 +72,8 @@ def test_small_gemm_edges(cnt, K, N, act, workspace):
         assert torch.equal(out.view(torch.int16), first.view(torch.int16))
 
 
-@pytest.mark.parametrize("cnt,H,F", [((1,), 128, 128), ((33, 0, 64), 384, 256), ((65,), 4096, 640), ((20, 7), 2048, 2176)])
+@pytest.mark.parametrize("cnt,H,F", [((1,), 128, 128), ((33, 0, 64), 384, 256), ((65,), 4096, 640), ((20, 7), 2048, 2176),
+                                     ((6000,), 2048, 1408)])  # (the last: large tiles with 8 left over)
 @pytest.mark.parametrize("workspace", [False, True], ids=["whole", "parts"])
 def test_small_fp8_mlp_edges(cnt, H, F, workspace):
     rng = np.random.default_rng(H + F)
