@@ -66,6 +66,7 @@ struct VecLoad<float> {
 // router slab, with one 128-bit read each).
 typedef float rt_f4 __attribute__((ext_vector_type(4)));
 typedef float rt_f16 __attribute__((ext_vector_type(16)));
+typedef float rt_f32 __attribute__((ext_vector_type(32)));
 typedef unsigned int rt_u4 __attribute__((ext_vector_type(4)));
 
 // One segment chain of a team of NWV waves for NTOK tokens and EB experts: the accumulators of the calling wave.
@@ -85,7 +86,7 @@ __device__ __forceinline__ void rt_team_sync() {
 
 template <int SHAPE>
 struct RtAcc {
-    typedef typename std::conditional<SHAPE == 16, rt_f16, rt_f4>::type type;
+    typedef typename std::conditional<SHAPE == 32, rt_f32, typename std::conditional<SHAPE == 16, rt_f16, rt_f4>::type>::type type;
 };
 
 template <typename XT, int SHAPE, int TB, int G, int NWV, int CPR /* 16-byte chunks of a token row per slab */, bool TEAM1, int D>
@@ -296,6 +297,162 @@ __global__ __launch_bounds__(NWV * WAVE, (NWV == 4 && TB == 2 ? 2 : 1)) void rou
     }
 }
 
+// More than 16 experts, bf16, many tokens: four waves, NWE along the experts (SHAPE each), 4 / NWE along the tokens (64 each).
+// ALL = false: one segment per workgroup, its chains to a plane of the workspace; workgroups b, b + 8, ... share an L2 and a segment.
+// ALL = true: the segment chains one after the other; the sum so far stays in registers, a chain is folded into it where its segment
+// ends, and the finished logit leaves: no partial sums in memory (eight planes written and read back were 27 us for 8192
+// tokens x 768, 256 experts: 70 -> 45 us with the top-k), with 16 experts to a wave for twice the waves.
+// Bound by the fp32 rate, which K = 1 MFMAs and vector instructions share (95 us for 4096 x 7168 x 256, measured 136 with the
+// partial sums; the 32 x 32 shape reaches 0.95 of the rate from a single chain per wave, 16 x 16 0.82): what counts is how few
+// vector instructions surround the MFMAs.  9218 tokens x 5032, 32 experts 88 -> 60 us and 16384 x 4096, 32 experts 94 -> 55 us
+// (blocks 32 experts wide instead of 64), 2048 x 4096, 256 experts 64 -> 50 us, 9216 x 3072, 256 experts 179 -> 157 us.
+// Slabs of KC h are double-buffered in LDS; the conversion and the writes of the next slab sit piece by piece between this one's
+// MFMAs, whose chain would leave the issue slots empty.
+// LDS: tokens as [token][h] (the lane reads eight consecutive h of its token), the router as [h][expert] as it comes.
+template <int SHAPE, int NWE, int KC, int D /* slabs under way in registers */, bool ALL>
+__global__ __launch_bounds__(4 * WAVE, 2) void route_logits_bf16_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
+                                                                      const float* __restrict__ bias, float* __restrict__ out, int T, int Hrow,
+                                                                      int E) {
+    constexpr int NTOK = 4 / NWE * RT_TB, EB = NWE * SHAPE, NCH = KC / 8, PX = KC + 4;
+    constexpr int XPT = NTOK * NCH / 256, WPT = KC * EB / 4 / 256;  // 16-byte pieces of token rows, 8-byte pieces of the router, per thread and slab
+    static_assert(NTOK * NCH % 256 == 0 && KC * EB / 4 % 256 == 0 && XPT + WPT < 2 * NCH, "two pieces per chunk at most");
+    __shared__ __align__(16) float xs[2][NTOK][PX];
+    __shared__ __align__(16) float ws[2][KC][EB];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    // workgroups b, b + 8, ... share an L2: ALL: all expert blocks of a token block; else a segment
+    const int n_e = (E + EB - 1) / EB, local = (int)blockIdx.x >> 3, b8 = (int)blockIdx.x & 7;
+    static_assert(RT_P == 8, "a segment per group of workgroups");
+    const int tb = ALL ? local / n_e * 8 + b8 : local / n_e, eb0 = local % n_e * EB, t0 = tb * NTOK;
+    if (t0 >= T) return;
+    const int seg_len = route_segment_len(Hrow);
+    const int h0 = ALL ? 0 : min(b8 * seg_len, Hrow), H = ALL ? Hrow : min(seg_len, Hrow - h0);
+    const int wt = wave / NWE * RT_TB, we = wave % NWE * SHAPE;
+    const bf16_t *xp[XPT], *wp[WPT];
+    int xh[XPT], wh[WPT];  // first h of the piece inside its slab
+#pragma unroll
+    for (int i = 0; i < XPT; ++i) {
+        const int c = tid + i * 256;
+        xh[i] = c % NCH * 8;
+        xp[i] = x + (size_t)min(t0 + c / NCH, T - 1) * Hrow;
+    }
+#pragma unroll
+    for (int i = 0; i < WPT; ++i) {
+        const int c = tid + i * 256;
+        wh[i] = c / (EB / 4);
+        wp[i] = w + min(eb0 + c % (EB / 4) * 4, E - 4);
+    }
+    static_assert(D == 2 || D == 4, "slab s lies in buffer s % 2 and register set s % D");
+    rt_u4 xr[D][XPT];
+    uint2 wr[D][WPT];
+    // (pieces past the end of the rows repeat the last ones; what is past H is not consumed)
+    auto fetch = [&](int d, int k0) {
+#pragma unroll
+        for (int i = 0; i < XPT; ++i) xr[d][i] = *reinterpret_cast<const rt_u4*>(xp[i] + min(h0 + k0 + xh[i], Hrow - 8));
+#pragma unroll
+        for (int i = 0; i < WPT; ++i) wr[d][i] = *reinterpret_cast<const uint2*>(wp[i] + (size_t)min(h0 + k0 + wh[i], Hrow - 1) * E);
+    };
+    auto put_x = [&](int d, int b, int i) {
+        const int c = tid + i * 256;
+        const rt_u4 r = xr[d][i];
+        const rt_f4 lo = {__uint_as_float(r.x << 16), __uint_as_float(r.x & 0xffff0000u), __uint_as_float(r.y << 16), __uint_as_float(r.y & 0xffff0000u)};
+        const rt_f4 hi = {__uint_as_float(r.z << 16), __uint_as_float(r.z & 0xffff0000u), __uint_as_float(r.w << 16), __uint_as_float(r.w & 0xffff0000u)};
+        float* o = &xs[b][c / NCH][c % NCH * 8];
+        *reinterpret_cast<rt_f4*>(o) = lo;
+        *reinterpret_cast<rt_f4*>(o + 4) = hi;
+    };
+    auto put_w = [&](int d, int b, int i) {
+        const int c = tid + i * 256;
+        const uint2 r = wr[d][i];
+        const rt_f4 v = {__uint_as_float(r.x << 16), __uint_as_float(r.x & 0xffff0000u), __uint_as_float(r.y << 16), __uint_as_float(r.y & 0xffff0000u)};
+        *reinterpret_cast<rt_f4*>(&ws[b][c / (EB / 4)][c % (EB / 4) * 4]) = v;
+    };
+    constexpr int NACC = SHAPE == 32 ? 32 : 16;
+    typename RtAcc<SHAPE>::type acc, sum;
+#pragma unroll
+    for (int v = 0; v < NACC; ++v) acc[v] = sum[v] = 0.f;
+    int seg = 0, left = min(seg_len, H) / 8;  // the chain at hand, chunks of eight h until it ends
+    auto fold = [&]() {
+#pragma unroll
+        for (int v = 0; v < NACC; ++v) {
+            sum[v] = seg == 0 ? acc[v] : __fadd_rn(sum[v], acc[v]);
+            acc[v] = 0.f;
+        }
+        ++seg;
+        left = max(min(seg_len, H - seg * seg_len), 0) / 8;
+    };
+    struct Frag {
+        rt_f4 x[2];
+        float w[8];
+    } f[2];
+    auto read = [&](Frag& g, int b, int c) {
+        const float* xl = &xs[b][wt + lane][c * 8];
+        g.x[0] = *reinterpret_cast<const rt_f4*>(xl);
+        g.x[1] = *reinterpret_cast<const rt_f4*>(xl + 4);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) g.w[q] = ws[b][c * 8 + q][we + lane % SHAPE];
+    };
+    const int n_slab = (H + KC - 1) / KC;
+#pragma unroll
+    for (int d = 0; d < D; ++d) fetch(d, d * KC);
+#pragma unroll
+    for (int i = 0; i < XPT; ++i) put_x(0, 0, i);
+#pragma unroll
+    for (int i = 0; i < WPT; ++i) put_w(0, 0, i);
+    fetch(0, D * KC);
+    __syncthreads();
+    // slab s (s % D = S) from buffer S % 2; slab s + 1 (register set N) goes to the other one, slab s + 1 + D is requested in its place
+    auto slab = [&](auto idx, int s) {
+        constexpr int S = decltype(idx)::value, B = S % 2, N = (S + 1) % D;
+        const int n = min(NCH, (H - s * KC) / 8);
+        read(f[0], B, 0);
+#pragma unroll
+        for (int c = 0; c < NCH; ++c) {
+            Frag &cur = f[c & 1], &nxt = f[1 - (c & 1)];
+            if (c + 1 < NCH) read(nxt, B, c + 1);  // (chunks past H: what the slot holds, not used)
+            // piece i of what this slab does for the next ones: the next slab's conversion and writes, then the request
+            auto piece = [&](int i) {
+                if (i < XPT) put_x(N, 1 - B, i);
+                else if (i - XPT < WPT) put_w(N, 1 - B, i - XPT);
+                else if (i == XPT + WPT) fetch(N, (s + 1 + D) * KC);
+            };
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                __builtin_amdgcn_sched_barrier(0);
+                if (c < n) {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        if constexpr (SHAPE == 32) acc = __builtin_amdgcn_mfma_f32_32x32x1f32(cur.x[h][q], cur.w[4 * h + q], acc, 0, 0, 0);
+                        else acc = __builtin_amdgcn_mfma_f32_16x16x1f32(cur.x[h][q], cur.w[4 * h + q], acc, 0, 0, 0);
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                piece(2 * c + h);
+            }
+            if (ALL && c < n && --left == 0) fold();
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        __syncthreads();
+    };
+    for (int s = 0; s < n_slab; s += D) {
+        slab(std::integral_constant<int, 0>{}, s);
+        if (s + 1 < n_slab) slab(std::integral_constant<int, 1>{}, s + 1);
+        if constexpr (D == 4) {
+            if (s + 2 < n_slab) slab(std::integral_constant<int, 2>{}, s + 2);
+            if (s + 3 < n_slab) slab(std::integral_constant<int, 3>{}, s + 3);
+        }
+    }
+    while (ALL && seg < RT_P) fold();  // (empty segments: their chains are +0)
+    const int e = eb0 + we + lane % SHAPE;
+    if (e >= E) return;
+    const float be = ALL && bias ? bias[e] : 0.f;
+    float* o = ALL ? out : out + (size_t)b8 * T * E;
+#pragma unroll
+    for (int v = 0; v < NACC; ++v) {
+        const int t = t0 + wt + (SHAPE == 32 ? 32 * (v / 16) + 8 * (v % 16 / 4) + 4 * (lane / 32) + v % 4 : 16 * (v / 4) + 4 * (lane / 16) + v % 4);
+        if (t < T) o[(size_t)t * E + e] = !ALL ? acc[v] : bias ? __fadd_rn(sum[v], be) : sum[v];
+    }
+}
+
 // Softmax gates + top-k.  G lanes cooperate on one token (G = 8,16,32,64); lane gl holds the eight consecutive experts
 // 8 gl .. 8 gl + 7 (two 16-byte loads per segment plane when the rows are 16-byte multiples).  Selection key: (logit
 // descending, expert id ascending).
@@ -317,7 +474,8 @@ __device__ __forceinline__ unsigned tk_xchg(int off, unsigned x) {
 // One pass of a wave: TPW = 64 / G tokens from tbase on.  part: the segments' partial sums, plane p at part + p * plane,
 // token t's row at t_part * E inside a plane (global workspace: t_part = t, plane = T E; a workgroup's own LDS copy:
 // t_part = t - first token of the workgroup).
-template <int G>
+// FINAL: part already holds the logits, bias and all (one plane; nothing to add up or write back).
+template <int G, bool FINAL = false>
 __device__ __forceinline__ void topk_gate_pass(const float* __restrict__ part, size_t plane, int t_part0, const float* __restrict__ bias,
                                                float* __restrict__ logits, int32_t* __restrict__ idx, float* __restrict__ gate, int T,
                                                int E, int k, int tbase) {
@@ -337,7 +495,15 @@ __device__ __forceinline__ void topk_gate_pass(const float* __restrict__ part, s
             if (live && eh < E) {
                 // the segments' partial sums in segment order, then the bias: this fixes the logit's bits
                 const float* pp = part + (size_t)(t - t_part0) * E + eh;
-                if (vec) {  // (eh + 3 < E then)
+                if constexpr (FINAL) {
+#pragma unroll
+                    for (int c = 0; c < 4; ++c)
+                        if (!vec && eh + c < E) sum[c] = pp[c];
+                    if (vec) {
+                        const float4 q = *reinterpret_cast<const float4*>(pp);
+                        sum[0] = q.x; sum[1] = q.y; sum[2] = q.z; sum[3] = q.w;
+                    }
+                } else if (vec) {  // (eh + 3 < E then)
                     float4 sp[RT_P];
 #pragma unroll
                     for (int p = 0; p < RT_P; ++p) sp[p] = *reinterpret_cast<const float4*>(pp + (size_t)p * plane);
@@ -360,8 +526,9 @@ __device__ __forceinline__ void topk_gate_pass(const float* __restrict__ part, s
                 }
 #pragma unroll
                 for (int c = 0; c < 4; ++c)
-                    if (eh + c < E && bias) sum[c] = __fadd_rn(sum[c], bias[eh + c]);
-                if (vec) *reinterpret_cast<float4*>(logits + (size_t)t * E + eh) = make_float4(sum[0], sum[1], sum[2], sum[3]);
+                    if (!FINAL && eh + c < E && bias) sum[c] = __fadd_rn(sum[c], bias[eh + c]);
+                if (FINAL) {
+                } else if (vec) *reinterpret_cast<float4*>(logits + (size_t)t * E + eh) = make_float4(sum[0], sum[1], sum[2], sum[3]);
                 else {
 #pragma unroll
                     for (int c = 0; c < 4; ++c)
@@ -438,7 +605,7 @@ __device__ __forceinline__ void topk_gate_pass(const float* __restrict__ part, s
     }
 }
 
-template <int G>
+template <int G, bool FINAL>
 __global__ __launch_bounds__(256) void topk_gate_kernel(const float* __restrict__ part /*[RT_P][T][E]*/,
                                                          const float* __restrict__ bias, float* __restrict__ logits,
                                                          int32_t* __restrict__ idx, float* __restrict__ gate, int T, int E,
@@ -447,7 +614,7 @@ __global__ __launch_bounds__(256) void topk_gate_kernel(const float* __restrict_
     const int wave_global = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
     const int n_waves = (gridDim.x * blockDim.x) / WAVE;
     for (int tbase = wave_global * TPW; tbase < T; tbase += n_waves * TPW)
-        topk_gate_pass<G>(part, (size_t)T * E, 0, bias, logits, idx, gate, T, E, k, tbase);
+        topk_gate_pass<G, FINAL>(part, (size_t)T * E, 0, bias, logits, idx, gate, T, E, k, tbase);
 }
 
 // Logits and top-k in one launch, for up to 16 experts.  A workgroup takes 64 tokens; wave p runs the chains of segment p for
@@ -485,11 +652,11 @@ __global__ __launch_bounds__(RT_P * WAVE, 1) void route_fused_kernel(const XT* _
     topk_gate_pass<TG>(part, (size_t)RT_TB * E, t0, bias, logits, idx, gate, T, E, k, t0 + seg * (WAVE / TG));
 }
 
-// Block shapes.  Many tokens: 128 tokens per block and slabs of 64 h, so that every wave runs two chains per group of
-// experts side by side and T / 128 x 8 segments of blocks are resident together (four blocks of this size fit a
-// compute unit's LDS); two waves (one group of four experts each) up to 8 experts, four up to 16; beyond that 16
-// experts per instruction and four or eight waves (64 or 128 experts per block).  Few tokens: 64 tokens per block
-// and one chain per wave, for four times as many waves.
+// Block shapes of the segment kernel (what route_logits_bf16_kernel does not take).  Many tokens: 128 tokens per block and slabs of 64 h,
+// so that every wave runs two chains per group of experts side by side and T / 128 x 8 segments of blocks are resident together
+// (four blocks of this size fit a compute unit's LDS); two waves (one group of four experts each) up to 8 experts, four up to 16;
+// beyond that 16 experts per instruction and four or eight waves (64 or 128 experts per block).  Few tokens: 64 tokens per block and
+// one chain per wave, for four times as many waves.
 template <typename XT>
 int launch_logits(const XT* x, const XT* w, float* part, int T, int H, int E, hipStream_t s) {
     constexpr int CPR = 64 / VecLoad<XT>::N;  // slabs of 64 h
@@ -504,11 +671,9 @@ int launch_logits(const XT* x, const XT* w, float* part, int T, int H, int E, hi
         if (E <= 4) RT_LAUNCH(4, 2, 1, 1, CPR, 1);
         else if (E <= 8) RT_LAUNCH(4, 2, 1, 2, CPR, 1);
         else if (E <= 16) RT_LAUNCH(4, 2, 1, 4, CPR, 1);
-        else if (E <= 64) {
-            // (fp32 tokens: two token blocks per wave do not fit the registers at this shape -- 18 would be spilled)
-            if constexpr (sizeof(XT) == 4) RT_LAUNCH(16, 1, 1, 4, CPR, 1);
-            else RT_LAUNCH(16, 2, 1, 4, CPR, 1);
-        }
+        // (fp32 tokens: two token blocks per wave do not fit the registers at this shape -- 18 would be spilled)
+        else if constexpr (sizeof(XT) == 2) RT_LAUNCH(16, 2, 1, 4, CPR, ceil_div(E, 64));
+        else if (E <= 64) RT_LAUNCH(16, 1, 1, 4, CPR, ceil_div(E, 64));
         else RT_LAUNCH(16, 2, 1, 8, CPR, ceil_div(E, 128));
     }
 #undef RT_LAUNCH
@@ -557,8 +722,27 @@ extern "C" int moe_route_topk(const void* x, const void* router, const float* bi
         return moe_check_launch("route_fused");
     }
     float* part = (float*)ws;
-    int rc = dtype == MOE_F32 ? launch_logits<float>((const float*)x, (const float*)router, part, T, H, E, s)
+    bool final = false;
+    int rc;
+    if (dtype == MOE_BF16 && E % 4 == 0 && ((E > 64 && T > 512) || (E > 16 && E <= 32 && T > 2048))) {
+        // (33 to 64 experts: the segment kernel's block of 128 tokens x 64 experts is as good or better.)  All segments in one workgroup
+        // where the rows are so short that writing and reading the segments' sums takes as long as the products, and there are
+        // tiles enough (at 3072 h and more their number, 2.25 for every place on the chip, say, costs more than the sums do).
+        const int n_e16 = ceil_div(E, 64), tiles16 = ceil_div(T, RT_TB) * n_e16;
+        final = E > 64 && H <= 1024 && tiles16 >= 256;
+        const int tok_blocks = ceil_div(T, (E <= 32 ? 4 : 1) * RT_TB), n_e = ceil_div(E, 128);
+#define RT_BF16(SHv, NWEv, ALLv, groups)                                                                                       \
+    route_logits_bf16_kernel<SHv, NWEv, ALLv ? 64 : 32, ALLv ? 2 : 4, ALLv><<<8 * (groups), 4 * WAVE, 0, s>>>(                 \
+        (const bf16_t*)x, (const bf16_t*)router, bias, ALLv ? logits : part, T, H, E)
+        if (final) RT_BF16(16, 4, true, ceil_div(ceil_div(T, RT_TB), 8) * n_e16);
+        else if (E <= 32) RT_BF16(32, 1, false, tok_blocks);
+        else RT_BF16(32, 4, false, tok_blocks * n_e);
+#undef RT_BF16
+        rc = moe_check_launch("route_logits");
+    } else {
+        rc = dtype == MOE_F32 ? launch_logits<float>((const float*)x, (const float*)router, part, T, H, E, s)
                               : launch_logits<bf16_t>((const bf16_t*)x, (const bf16_t*)router, part, T, H, E, s);
+    }
     if (rc) return rc;
     // lanes per token: the fewest that hold all experts at TK_MAXV per lane (more tokens per wave, fewer shuffles)
     int G = 8;
@@ -567,11 +751,17 @@ extern "C" int moe_route_topk(const void* x, const void* router, const float* bi
     const int tpw = WAVE / G;
     const int waves = ceil_div(T, tpw);
     const int blocks = min(ceil_div(waves, 4), 4096);
+#define RT_TOPK(Gv)                                                                                                             \
+    do {                                                                                                                        \
+        if (final) topk_gate_kernel<Gv, true><<<blocks, 256, 0, s>>>(logits, nullptr, nullptr, topk_idx, topk_gate, T, E, k);    \
+        else topk_gate_kernel<Gv, false><<<blocks, 256, 0, s>>>(part, bias, logits, topk_idx, topk_gate, T, E, k);               \
+    } while (0)
     switch (G) {
-        case 8: topk_gate_kernel<8><<<blocks, 256, 0, s>>>(part, bias, logits, topk_idx, topk_gate, T, E, k); break;
-        case 16: topk_gate_kernel<16><<<blocks, 256, 0, s>>>(part, bias, logits, topk_idx, topk_gate, T, E, k); break;
-        case 32: topk_gate_kernel<32><<<blocks, 256, 0, s>>>(part, bias, logits, topk_idx, topk_gate, T, E, k); break;
-        default: topk_gate_kernel<64><<<blocks, 256, 0, s>>>(part, bias, logits, topk_idx, topk_gate, T, E, k); break;
+        case 8: RT_TOPK(8); break;
+        case 16: RT_TOPK(16); break;
+        case 32: RT_TOPK(32); break;
+        default: RT_TOPK(64); break;
     }
+#undef RT_TOPK
     return moe_check_launch("topk_gate");
 }

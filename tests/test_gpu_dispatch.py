@@ -547,3 +547,20 @@ def test_row_copies_and_sums_cut_into_column_runs(T, H, k):
         d_ret, d_gate = ops.combine_backward(bf(d_out), bf(ret), dev(idx), dev(pos), dev(gate), known, dev(offs), E_l)
         assert_bits_equal(d_ret, want, "d returned")
         np.testing.assert_allclose(to_np(d_gate), want_g, rtol=1e-4, atol=1e-3)
+
+
+# (the segment kernel below the token limits and at 33 to 64 experts; one segment per workgroup; all segments in one workgroup;
+# rows of 8 to 63 chunks of eight, so that segments end inside and at the end of slabs, some of them empty)
+@pytest.mark.parametrize("T,H,E,k,bias", [(511, 72, 72, 2, True), (513, 264, 68, 8, False), (2049, 504, 20, 1, True), (2177, 1032, 32, 4, False),
+                                          (2050, 296, 60, 2, True), (8192, 136, 260, 8, True), (4200, 8, 256, 2, False), (16385, 328, 100, 4, False)])
+def test_router_tiles_are_bit_exact(T, H, E, k, bias):
+    rng = np.random.default_rng(T)
+    x = O.bf16_round(rng.standard_normal((T, H)).astype(np.float32))
+    w = O.bf16_round(rng.standard_normal((H, E)).astype(np.float32))
+    b = rng.standard_normal(E).astype(np.float32) if bias else None
+    dev = lambda a: torch.from_numpy(a).to(DEV)  # noqa: E731
+    idx, gate, logits = ops.route_topk(dev(x).bfloat16(), dev(w).bfloat16(), k, None if b is None else dev(b))
+    o_idx, o_gate, o_logits = O.route(x, w, k, b)
+    assert_bits_equal(logits, o_logits, "router logits")
+    assert_bits_equal(idx, o_idx, "top-k indices")
+    np.testing.assert_allclose(to_np(gate), o_gate, rtol=1e-5, atol=1e-30)
