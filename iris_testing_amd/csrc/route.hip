@@ -662,10 +662,16 @@ int launch_logits(const XT* x, const XT* w, float* part, int T, int H, int E, hi
     constexpr int CPR = 64 / VecLoad<XT>::N;  // slabs of 64 h
 #define RT_LAUNCH(SHAPEv, TBv, Gv, NWVv, CPRv, gz) \
     route_logits_mfma_kernel<XT, SHAPEv, TBv, Gv, NWVv, CPRv><<<dim3(RT_P, ceil_div(T, TBv * RT_TB), gz), NWVv * WAVE, 0, s>>>(x, w, part, T, H, E)
+    // One workgroup of 64 tokens x 16 experts to a compute unit, or two, and the chain's latency is all that counts: a step of the
+    // 4 x 4 x 1 product is 14 cycles, of the 16 x 16 x 1 product 32 (7168 x 256: 24 tokens 24 -> 13 us, 128 tokens 24.5 -> 14.4; 256 tokens
+    // 25.8 -> 19.3 with two groups to a wave; 512 tokens 28.0 as before, 30.4 with two groups).
+    const int quads = ceil_div(T, RT_TB) * ceil_div(E, 16);
     if (T <= 2048) {
         if (E <= 4) RT_LAUNCH(4, 1, 1, 1, 16, 1);
         else if (E <= 8) RT_LAUNCH(4, 1, 1, 2, 16, 1);
         else if (E <= 64) RT_LAUNCH(4, 1, 1, 4, 16, ceil_div(E, 16));
+        else if (quads <= 32) RT_LAUNCH(4, 1, 1, 4, 16, ceil_div(E, 16));
+        else if (quads <= 64) RT_LAUNCH(4, 1, 2, 4, 16, ceil_div(E, 32));
         else RT_LAUNCH(16, 1, 1, 4, 16, ceil_div(E, 64));
     } else {
         if (E <= 4) RT_LAUNCH(4, 2, 1, 1, CPR, 1);
