@@ -399,6 +399,12 @@ constexpr int PACK_ZR = 8;
 inline int row_parts(int tokens, int row_vec) {
     return max(1, min(2048 / max(tokens, 1), (row_vec + WAVE - 1) / WAVE));
 }
+// The combine's: also with many tokens, so that the rows of fewer tokens are read at a time -- with a row to a wave 4096 x 8 rows of 14 KB
+// are 32768 places in memory at once.  Runs of 2 KB at least and at most four to a row (k = 8: 4096 x 14 KB 104 -> 97 us, 5.5 TB/s;
+// 8192 x 4 KB 61 -> 57; k = 2: 8192 x 8 KB 41 -> 36; eight runs 55 where four take 51 and one 54, runs of 1 KB 20 where one takes 17).
+inline int combine_parts(int tokens, int row_vec) {
+    return tokens < 2048 ? row_parts(tokens, row_vec) : max(1, min(min(16384 / tokens, row_vec / (2 * WAVE)), 4));
+}
 template <int WPB>
 __global__ __launch_bounds__(WPB * WAVE) void pack_tokens_kernel(const u32x4* __restrict__ x, u32x4* __restrict__ send,
                                                                   const int32_t* __restrict__ idx, const int32_t* __restrict__ pos,
@@ -506,7 +512,7 @@ __global__ __launch_bounds__(WPB * WAVE) void combine_kernel(const uint4* __rest
     constexpr int KMAX = KT ? KT : MOE_MAX_TOPK;
     const int k = KT ? KT : k_rt;
     const int wave = threadIdx.x / WAVE, lane = lane_id();
-    const int per = ((row_vec + parts - 1) / parts + WAVE - 1) / WAVE * WAVE;  // columns per wave (see row_parts)
+    const int per = ((row_vec + parts - 1) / parts + WAVE - 1) / WAVE * WAVE;  // columns per wave (see combine_parts)
     for (int unit = blockIdx.x * WPB + wave; unit < T * parts; unit += gridDim.x * WPB) {
         const int t = unit / parts, c_lo = (unit % parts) * per, c_hi = min(c_lo + per, row_vec);
         // a slot whose destination or row lies outside the [W,M] layout was dropped by the pack (pair capacity
@@ -571,12 +577,13 @@ __global__ __launch_bounds__(WPB * WAVE) void combine_kernel(const uint4* __rest
 //   d ret[slot(t,kk)] = gate[t,kk] * d out[t]        (every slot belongs to one (t,kk): a scatter, like the pack)
 //   d gate[t,kk]      = < d out[t], ret[slot(t,kk)] > (fp32 sum over the row: per-lane partial sums in column order, then
 //                                                     a butterfly over the lanes -- reproducible from call to call)
-// Units [0, T) of the launch are tokens (one wave each); the units after them are runs of PACK_ZR slots of d ret, which only get
-// zeros when they are padding (no (t,kk) maps there) -- as in pack_tokens_kernel.  Dropped slots (outside [W,M]) get no
+// The first workgroups take the tokens: a wave each (WPT = 1) or all waves together, whose sums then meet in LDS in wave order; the
+// others take runs of PACK_ZR slots of d ret, which only get zeros when they are padding (no (t,kk) maps there) -- as in
+// pack_tokens_kernel.  Dropped slots (outside [W,M]) get no
 // gradient.  A pass takes U columns of the token's d out and of its k slot rows together (some sixteen 16-byte loads in flight
 // per lane): d out is read once, not k times (4096 tokens x 8 rows of 14 KB: 299 -> 266 us, 4.4 TB/s with the padding).
 // dst_sizes == NULL: a destination's rows end where the next one's start (n_routed rows in all).
-template <typename XT, int KT, int WPB>
+template <typename XT, int KT, int WPB, int WPT /* waves per token: 1 or WPB */>
 __global__ __launch_bounds__(WPB * WAVE) void combine_backward_kernel(const uint4* __restrict__ dout, const uint4* __restrict__ ret,
                                                                        const int32_t* __restrict__ idx, const int32_t* __restrict__ pos,
                                                                        const float* __restrict__ gate,
@@ -588,11 +595,18 @@ __global__ __launch_bounds__(WPB * WAVE) void combine_backward_kernel(const uint
     constexpr int KMAX = KT ? KT : MOE_MAX_TOPK;
     constexpr int U = KT ? (KT >= 8 ? 2 : KT >= 4 ? 4 : 8) : 1;
     const int k = KT ? KT : k_rt;
+    static_assert(WPT == 1 || WPT == WPB, "a token to a wave or to a workgroup");
+    __shared__ float part[WPT == 1 ? 1 : WPT][KMAX];
     const int wave = threadIdx.x / WAVE, lane = lane_id();
-    const int n_slots = W * M, n_units = T + (n_slots + PACK_ZR - 1) / PACK_ZR;
-    for (int r = blockIdx.x * WPB + wave; r < n_units; r += gridDim.x * WPB) {
-        if (r >= T) {
-            const int s0 = (r - T) * PACK_ZR, s1 = min(s0 + PACK_ZR, n_slots);
+    // token rows first, WPB / WPT to a workgroup, in workgroups of their own; then the runs of slots, WPB to a workgroup
+    const int n_slots = W * M, n_runs = (n_slots + PACK_ZR - 1) / PACK_ZR;
+    const int tok_blocks = (T + WPB / WPT - 1) / (WPB / WPT), n_blocks = tok_blocks + (n_runs + WPB - 1) / WPB;
+    for (int b = blockIdx.x; b < n_blocks; b += gridDim.x) {
+        const int r = WPT == 1 ? b * WPB + wave : b, c_first = WPT == 1 ? lane : (int)threadIdx.x;
+        if (b >= tok_blocks) {
+            const int run = (b - tok_blocks) * WPB + wave;
+            if (run >= n_runs) continue;
+            const int s0 = run * PACK_ZR, s1 = min(s0 + PACK_ZR, n_slots);
             int d = s0 / M, m = s0 % M;
             auto size_of = [&](int q) { return dst_sizes ? dst_sizes[q] : (q + 1 < W ? dst_offsets[q + 1] : T * k) - dst_offsets[q]; };
             int cnt = size_of(d);
@@ -605,6 +619,7 @@ __global__ __launch_bounds__(WPB * WAVE) void combine_backward_kernel(const uint
             }
             continue;
         }
+        if (r >= T) continue;
         const uint4* drow = dout + (size_t)r * row_vec;
         size_t slot[KMAX];
         float g[KMAX], dot[KMAX];
@@ -622,22 +637,23 @@ __global__ __launch_bounds__(WPB * WAVE) void combine_backward_kernel(const uint
                 g[j] = gate[(size_t)r * k + j];
             }
         }
-        for (int c0 = lane; c0 < row_vec; c0 += U * WAVE) {
+        constexpr int CS = WPT * WAVE;  // columns from one to the next of a lane
+        for (int c0 = c_first; c0 < row_vec; c0 += U * CS) {
             uint4 dv4[U], rv4[U][KMAX];
 #pragma unroll
             for (int u = 0; u < U; ++u)
-                if (c0 + u * WAVE < row_vec) {
-                    dv4[u] = drow[c0 + u * WAVE];
+                if (c0 + u * CS < row_vec) {
+                    dv4[u] = drow[c0 + u * CS];
 #pragma unroll
                     for (int j = 0; j < KMAX; ++j)
                         if (j < k && have[j]) {
-                            const u32x4 raw = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(ret + slot[j] + c0 + u * WAVE));
+                            const u32x4 raw = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(ret + slot[j] + c0 + u * CS));
                             rv4[u][j] = make_uint4(raw.x, raw.y, raw.z, raw.w);
                         }
                 }
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                if (c0 + u * WAVE >= row_vec) break;
+                if (c0 + u * CS >= row_vec) break;
                 float dv[N];
                 Vec16<XT>::unpack(dv4[u], dv);
 #pragma unroll
@@ -652,7 +668,7 @@ __global__ __launch_bounds__(WPB * WAVE) void combine_backward_kernel(const uint
                         }
                         const uint4 o = Vec16<XT>::pack(ov);
                         const u32x4 o4 = {o.x, o.y, o.z, o.w};
-                        __builtin_nontemporal_store(o4, reinterpret_cast<u32x4*>(dret + slot[j] + c0 + u * WAVE));
+                        __builtin_nontemporal_store(o4, reinterpret_cast<u32x4*>(dret + slot[j] + c0 + u * CS));
                     }
             }
         }
@@ -661,15 +677,28 @@ __global__ __launch_bounds__(WPB * WAVE) void combine_backward_kernel(const uint
             if (j < k) {
 #pragma unroll
                 for (int off = WAVE / 2; off >= 1; off >>= 1) dot[j] = __fadd_rn(dot[j], __shfl_xor(dot[j], off, WAVE));
-                if (lane == 0) dgate[(size_t)r * k + j] = dot[j];
+                if (lane == 0) {
+                    if constexpr (WPT == 1) dgate[(size_t)r * k + j] = dot[j];
+                    else part[wave][j] = dot[j];
+                }
             }
+        if constexpr (WPT > 1) {
+            __syncthreads();
+            if ((int)threadIdx.x < k) {
+                float sum = part[0][threadIdx.x];
+#pragma unroll
+                for (int w = 1; w < WPT; ++w) sum = __fadd_rn(sum, part[w][threadIdx.x]);
+                dgate[(size_t)r * k + threadIdx.x] = sum;
+            }
+            __syncthreads();
+        }
     }
 }
 
 template <typename XT>
 int launch_combine(const void* ret, const int32_t* idx, const int32_t* pos, const float* gate, const int32_t* dst_offsets, int T,
                    int k, int E_l, int W, int M, int row_vec, void* out, int32_t* status, hipStream_t s) {
-    const int parts = row_parts(T, row_vec);
+    const int parts = combine_parts(T, row_vec);
     const int blocks = min(ceil_div(T * parts, 4), 65535 * 8);
 #define MOE_COMBINE(KT) \
     combine_kernel<XT, KT, 4><<<blocks, 4 * WAVE, 0, s>>>((const uint4*)ret, idx, pos, gate, dst_offsets, T, k, E_l, W, M, row_vec, (uint4*)out, status, parts)
@@ -1200,11 +1229,18 @@ extern "C" int moe_combine_backward(const void* d_out, const void* ret, int dtyp
     MOE_REQUIRE((long long)W * M + T < (1ll << 31), MOE_ERR_UNSUPPORTED, "combine_backward: W*M + T too large");
     MOE_REQUIRE(d_ret && dst_offsets, MOE_ERR_INVALID, "combine_backward: null pointer");
     MOE_REQUIRE(T == 0 || (d_out && ret && topk_idx && pos && gate && d_gate), MOE_ERR_INVALID, "combine_backward: null pointer");
-    const int blocks = min(ceil_div(T + ceil_div(W * M, PACK_ZR), 4), 65535 * 8);
     const int row_vec = H * dtype_size(dtype) / 16;
-#define MOE_CB(XT, KT) \
-    combine_backward_kernel<XT, KT, 4><<<blocks, 4 * WAVE, 0, s>>>((const uint4*)d_out, (const uint4*)ret, topk_idx, pos, gate, dst_sizes, \
-                                                                   dst_offsets, T, k, E_l, W, M, row_vec, (uint4*)d_ret, d_gate)
+    // (a token to a workgroup where its rows give every wave some 8 KB to move: 8192 tokens x 8 rows of 4 KB 138 -> 116 us, 4096 x 4 of
+    // 8 KB 78 -> 66, 64 x 8 of 14 KB 48 -> 18; rows of 1 KB 22 -> 41, 4096 x 2 of 4 KB 24 -> 26)
+    const bool wide = row_vec >= 512 || (row_vec >= 256 && k >= 4);
+    const int blocks = min(ceil_div(T, wide ? 1 : 4) + ceil_div(ceil_div(W * M, PACK_ZR), 4), 65535 * 8);
+#define MOE_CBW(XT, KT, WPT)                                                                                                           \
+    combine_backward_kernel<XT, KT, 4, WPT><<<blocks, 4 * WAVE, 0, s>>>((const uint4*)d_out, (const uint4*)ret, topk_idx, pos, gate,     \
+                                                                        dst_sizes, dst_offsets, T, k, E_l, W, M, row_vec, (uint4*)d_ret, \
+                                                                        d_gate)
+#define MOE_CB(XT, KT)             \
+    if (wide) MOE_CBW(XT, KT, 4);  \
+    else MOE_CBW(XT, KT, 1)
 #define MOE_CBK(XT)                                    \
     switch (k) {                                       \
         case 1: MOE_CB(XT, 1); break;                  \
@@ -1217,6 +1253,7 @@ extern "C" int moe_combine_backward(const void* d_out, const void* ret, int dtyp
     else MOE_CBK(bf16_t)
 #undef MOE_CBK
 #undef MOE_CB
+#undef MOE_CBW
     return moe_check_launch("combine_backward");
 }
 

@@ -515,9 +515,9 @@ def test_counts_and_positions_at_block_edges(T, E, W, k):
     assert c.caps.tolist() == [max(1, int(sizes.max())), max(1, int(counts.max()))]
 
 
-@pytest.mark.parametrize("T,H,k", [(1, 520, 1), (5, 4096, 3), (33, 1032, 8), (700, 264, 2)])
+@pytest.mark.parametrize("T,H,k", [(1, 520, 1), (5, 4096, 3), (33, 1032, 8), (700, 264, 2), (2050, 2056, 4)])
 def test_row_copies_and_sums_cut_into_column_runs(T, H, k):
-    """Few tokens: a row is cut into runs of columns (whole, ragged, single); pack, combine and the gradient of combine."""
+    """Rows cut into runs of columns (whole, ragged, single) where tokens are few, and for the sums where rows are long; pack, combine and the gradient of combine."""
     rng = np.random.default_rng(T)
     E, W = 16, 4
     E_l = E // W
@@ -551,7 +551,7 @@ def test_row_copies_and_sums_cut_into_column_runs(T, H, k):
 
 # (the segment kernel below the token limits and at 33 to 64 experts; one segment per workgroup; all segments in one workgroup;
 # rows of 8 to 63 chunks of eight, so that segments end inside and at the end of slabs, some of them empty)
-@pytest.mark.parametrize("T,H,E,k,bias", [(511, 72, 72, 2, True), (513, 264, 68, 8, False), (2049, 504, 20, 1, True), (2177, 1032, 32, 4, False),
+@pytest.mark.parametrize("T,H,E,k,bias", [(65, 520, 250, 8, True), (130, 72, 300, 3, False), (511, 72, 72, 2, True), (513, 264, 68, 8, False), (2049, 504, 20, 1, True), (2177, 1032, 32, 4, False),
                                           (2050, 296, 60, 2, True), (8192, 136, 260, 8, True), (4200, 8, 256, 2, False), (16385, 328, 100, 4, False)])
 def test_router_tiles_are_bit_exact(T, H, E, k, bias):
     rng = np.random.default_rng(T)
