@@ -420,9 +420,11 @@ int moe_diag_gemm_trace(unsigned long long* trace, size_t words, int flags);
  *   token_buf [E_l,W,CAP,H] <- row block start + (rows of the experts before e) + j of source s at [e,s,j], zeros
  *   past its count; pca[e,s] = counts; counts_ready / token_sync (n_ready / n_sync int32 each, nullable) <- W.
  *   If a count exceeds CAP nothing is written.
- * moe_a2a_max_count: *max_count (device-writable, e.g. pinned host memory) <- the largest count of moe_a2a_place, 0 if none.
+ * moe_a2a_max_count: max_count[0] (of two words, device-writable, e.g. pinned host memory) <- the largest count of moe_a2a_place, 0 if none.
  * moe_shuffle_totals: out[0] <- sum of pca (n entries), out[1] <- smallest of token_sync (n_sync entries; 2^31 - 1 if none);
- *   out device-writable, e.g. pinned host memory. */
+ *   out device-writable, e.g. pinned host memory.
+ * moe_wait_i32: returns when *value (pinned host memory that held `pending` before the launch on `stream` that writes it) is
+ *   another value; of moe_shuffle_totals' two, out[0] is written last. */
 typedef struct moe_a2a_source {
     const void* payload;
     const int32_t* counts;
@@ -432,6 +434,7 @@ typedef struct moe_a2a_source {
 int moe_a2a_max_count(const moe_a2a_source* sources /* host */, int W, int E_l, int32_t* max_count, moe_stream_t stream);
 int moe_a2a_place(const moe_a2a_source* sources /* host */, int dtype, int W, int E_l, int CAP, int H, void* token_buf, int32_t* pca,
                   int32_t* counts_ready, int n_ready, int32_t* token_sync, int n_sync, moe_stream_t stream);
+int moe_wait_i32(const int32_t* value, int32_t pending, moe_stream_t stream);
 int moe_shuffle_totals(const int32_t* pca, int n, const int32_t* token_sync, int n_sync, int32_t* out, moe_stream_t stream);
 /* moe_expert_forward: out[rows of g] = tokens[rows of g] @ w[g] (bf16) with the rows of out past the counted total zeroed (the
  * caller's out needs no clearing).  layout MOE_W_TILED: weights as moe_prepack_weights makes them of [E_l,K,N]; MOE_W_RAW: [E_l,K,N]

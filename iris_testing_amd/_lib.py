@@ -101,6 +101,7 @@ _SIGNATURES = {
     "moe_recv_prepare": (c_int, [P, c_int, c_int, c_int, c_int, P, P, P, P, P, P, P, c_int, c_int, P]),
     "moe_a2a_max_count": (c_int, [POINTER(A2aSource), c_int, c_int, P, P]),
     "moe_a2a_place": (c_int, [POINTER(A2aSource), c_int, c_int, c_int, c_int, c_int, P, P, P, c_int, P, c_int, P]),
+    "moe_wait_i32": (c_int, [P, c_int, P]),
     "moe_shuffle_totals": (c_int, [P, c_int, P, c_int, P, P]),
     "moe_expert_forward": (c_int, [P, P, c_int, P, c_int, c_int, c_int, c_int, P, P, c_size_t, P]),
     "moe_step": (c_int, [POINTER(StepArgs), P]),

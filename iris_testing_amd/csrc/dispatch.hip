@@ -843,16 +843,27 @@ struct A2aSources {
 };
 __device__ __forceinline__ int a2a_count(const moe_a2a_source& q, int e) { return q.payload ? max(q.counts[e], 0) : 0; }
 
-__global__ __launch_bounds__(256) void a2a_max_count_kernel(const A2aSources q, int ns, int E_l, int32_t* __restrict__ out, bool first) {
+// A value for a waiting host (moe_wait_i32): visible as soon as it is stored, not only when the kernel ends.
+__device__ __forceinline__ void tell_host(int32_t* out, int32_t v) {
+    __threadfence_system();  // (what was written for the host before goes first)
+    __hip_atomic_store(out, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// out[0] <- the result (last launch only: the host may be waiting for it), out[1]: what earlier launches found
+__global__ __launch_bounds__(256) void a2a_max_count_kernel(const A2aSources q, int ns, int E_l, int32_t* __restrict__ out, bool first,
+                                                             bool last) {
     __shared__ int32_t most;
-    if (threadIdx.x == 0) most = first ? 0 : *out;
+    if (threadIdx.x == 0) most = first ? 0 : out[1];
     __syncthreads();
     for (int i = threadIdx.x; i < ns * E_l; i += blockDim.x) {
         const int c = a2a_count(q.src[i / E_l], i % E_l);
         if (c > 0) atomicMax(&most, c);
     }
     __syncthreads();
-    if (threadIdx.x == 0) *out = most;
+    if (threadIdx.x == 0) {
+        if (last) tell_host(out, most);
+        else out[1] = most;
+    }
 }
 
 __global__ __launch_bounds__(256) void a2a_place_kernel(const A2aSources q, int s0, int ns, int W, int E_l, int CAP, int row_vec,
@@ -914,7 +925,10 @@ __global__ __launch_bounds__(256) void shuffle_totals_kernel(const int32_t* __re
     atomicAdd(&sum, s);
     atomicMin(&least, m);
     __syncthreads();
-    if (threadIdx.x == 0) { out[0] = sum; out[1] = least; }
+    if (threadIdx.x == 0) {
+        out[1] = least;
+        tell_host(out, sum);
+    }
 }
 
 }  // namespace
@@ -1292,7 +1306,7 @@ extern "C" int moe_a2a_max_count(const moe_a2a_source* sources, int W, int E_l, 
     MOE_REQUIRE(max_count, MOE_ERR_INVALID, "a2a_max_count: null pointer");
     for (int s0 = 0; s0 < W; s0 += A2A_SRC) {
         const int ns = min(A2A_SRC, W - s0);
-        a2a_max_count_kernel<<<1, 256, 0, (hipStream_t)stream>>>(a2a_slice(sources, s0, ns), ns, E_l, max_count, s0 == 0);
+        a2a_max_count_kernel<<<1, 256, 0, (hipStream_t)stream>>>(a2a_slice(sources, s0, ns), ns, E_l, max_count, s0 == 0, s0 + ns == W);
     }
     return moe_check_launch("a2a_max_count");
 }

@@ -76,18 +76,16 @@ class AllToAllOp(torch.autograd.Function):
                 do = do.to(*where).contiguous()
             sends[src] = (p, dc, do)
         want = (e_local, world_size, capacity, tokens.shape[-1])
-        block, most = ops.a2a_sources(sends, rank), ops.pinned_i32(1)
+        block, most = ops.a2a_sources(sends, rank), ops.pinned_i32(2)
         fits = tuple(token_buf.shape) == want and token_buf.dtype == tokens.dtype
         ops.a2a_max_count(block, e_local, most)
-        known = torch.cuda.Event()
-        known.record()
         try:
             if fits:  # (writes nothing if a count exceeds the capacity; the host learns of that while the rows move)
                 pca = local_pca if local_pca.is_contiguous() else torch.empty_like(local_pca, memory_format=torch.contiguous_format)
                 ready, sync = (t if t.dtype == torch.int32 and t.is_cuda and t.is_contiguous() else None for t in (counts_ready, token_sync))
                 ops.a2a_place(block, token_buf, pca, ready, sync)
         finally:
-            known.synchronize()
+            ops.wait_i32(most)
         over = int(most[0])
         if over > capacity:
             raise ValueError(f"capacity overflow: a (src, expert) pair sends {over} rows > CAP={capacity}")

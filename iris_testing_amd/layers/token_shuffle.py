@@ -25,7 +25,7 @@ class TokenShuffle(torch.autograd.Function):
         totals = ops.pinned_i32(2)
         sync = None if token_sync is None else token_sync.to(pca.device, torch.int32).contiguous()
         ops.shuffle_totals(pca_c, sync, totals)
-        torch.cuda.current_stream().synchronize()
+        ops.wait_i32(totals)
         total, done = totals.tolist()
         # the reference kernel spins until token_sync[e] >= world_size (kernels.py:192); on one
         # GPU the data is either complete or never will be, so an incomplete counter is an error

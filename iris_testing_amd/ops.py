@@ -250,8 +250,13 @@ def shuffle_rows(token_buf: torch.Tensor, pca: torch.Tensor, S_rows: int, out: O
 
 
 def pinned_i32(n: int) -> torch.Tensor:
-    """n int32 in pinned host memory, which kernels write directly: read it after waiting for them (one wait, no copy)."""
-    return torch.empty(n, dtype=torch.int32, pin_memory=True)
+    """n int32 of -1 in pinned host memory, which kernels write directly (no copy): read them after wait_i32."""
+    return torch.empty(n, dtype=torch.int32, pin_memory=True).fill_(-1)
+
+
+def wait_i32(value: torch.Tensor) -> None:
+    """Waits until the kernel enqueued on the current stream has written value[0] of a pinned_i32."""
+    L.check(L.lib().moe_wait_i32(L.ptr(value), -1, L.stream_ptr()))
 
 
 def a2a_sources(sends, rank: int):
@@ -267,7 +272,7 @@ def a2a_sources(sends, rank: int):
 
 
 def a2a_max_count(block, e_local: int, out: torch.Tensor) -> None:
-    """out[0] (pinned or device int32) <- the largest count of any (source, expert)."""
+    """out[0] (pinned or device int32 [2]) <- the largest count of any (source, expert)."""
     L.check(L.lib().moe_a2a_max_count(block, len(block), e_local, L.ptr(out), L.stream_ptr()))
 
 
