@@ -156,6 +156,11 @@ def stream_ptr() -> int:
     return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
+def capturing() -> bool:
+    """Whether the current stream is being captured into a graph: launches are recorded, and nothing has run yet."""
+    return torch.cuda.is_current_stream_capturing()
+
+
 def dtype_code(dt: torch.dtype) -> int:
     if dt == torch.float32:
         return MOE_F32

@@ -18,6 +18,9 @@ from ..utils import _assert_cuda_int32
 # Re-tiled copies of weight tensors the operator has seen (None: seen once, not re-tiled yet), keyed on the tensor's storage and version counter, so that
 # a weight that did not change between calls is re-tiled once, not on every call (the re-tiling reads and writes the
 # whole tensor).  Entries die with their tensors (weak references); an in-place update bumps the version and re-tiles.
+# While a stream is being captured nothing here changes and nothing from here is used: a re-tiling that was only recorded has not
+# happened for the next eager call or the next graph, a copy dropped after an update would be freed under the graph, and a graph
+# that holds an optimizer's update has to read the weights it left.  A captured call multiplies with the tensors as they are.
 _PACKED = {}
 _PART_WS = OrderedDict()
 _PART_WS_MAX = 4  # streams with a workspace of their own (67 MB each); the one not used for longest is given back
@@ -33,6 +36,8 @@ def _drop_packs(kind: str, w: torch.Tensor) -> None:
 
 
 def _cached_pack(kind: str, w: torch.Tensor, w_up: Optional[torch.Tensor], build) -> torch.Tensor:
+    if L.capturing():
+        return build(w, w_up)
     key = _pack_key(kind, w, w_up)
     hit = _PACKED.get(key)
     if hit is not None and hit[0]() is w:
@@ -47,6 +52,8 @@ def _weights_for(w: torch.Tensor, rows: int):
     """(weights, layout) for the forward GEMM on `rows` rows.  The first call with a weight -- or with what an in-place update made of
     it -- multiplies with the tensor as it is (see ExpertWeights.train_weights), the second one, if nothing has changed by
     then, re-tiles it."""
+    if L.capturing():
+        return w, L.W_RAW
     key = _pack_key("N", w, None)
     hit = _PACKED.get(key)
     if hit is None or hit[0]() is not w:
@@ -71,7 +78,7 @@ def _grouped_gemm_t(do: torch.Tensor, weights: torch.Tensor, cnt: torch.Tensor) 
     if do.dtype == torch.float32:
         return ops.grouped_gemm(do, ops.transpose_weights_f32(weights.contiguous()), cnt)
     S = do.shape[0]
-    if N % 64 or K % 8 or S >= 4096 * E_l:  # (no whole stages of the reduction; or worth a re-tiled copy)
+    if N % 64 or K % 8 or (S >= 4096 * E_l and not L.capturing()):  # (no whole stages of the reduction; or worth a re-tiled copy)
         out = torch.zeros((S, K), dtype=do.dtype, device=do.device)
         if S:
             ops.grouped_gemm_mapped(do, None, _packed_weights_t(weights), cnt, S, K, "none", out, part_ws=_part_ws(do.device))
@@ -156,15 +163,20 @@ class ExpertWeights:
     # version counters of the raw tensors when w1 / w2 / w_up were last derived from them (refresh() compares)
     raw_versions: Optional[tuple] = field(default=None, repr=False)
     seen_versions: Optional[tuple] = field(default=None, repr=False)  # ... when train_weights() last looked at them
+    copies: tuple = field(default=(None, None, None), repr=False)  # those of w1, w2, w_up that are copies made here
 
     @staticmethod
-    def _derive(raw):
-        """(w1, w2, w_up) as the kernels take them, from the tensors in the reference layout."""
-        w1, w2, w_up = raw
+    def _derive(raw, copies=(None, None, None)):
+        """((w1, w2, w_up) as the kernels take them, the copies among them), from the tensors in the reference layout; ``copies``:
+        those made before, which are written again."""
+        w1, w2, w_up = (None if t is None else t.detach() for t in raw)
         if w1.dtype == torch.float32:
-            return w1.contiguous(), w2.contiguous(), None if w_up is None else w_up.contiguous()
-        return (ops.prepack_weights(w1.contiguous(), None if w_up is None else w_up.contiguous()),
-                ops.prepack_weights(w2.contiguous()), None)
+            copies = tuple(None if t is None or t.is_contiguous() else t.contiguous() if c is None else c.copy_(t)
+                           for t, c in zip((w1, w2, w_up), copies))
+            return tuple(t if c is None else c for t, c in zip((w1, w2, w_up), copies)), copies
+        copies = (ops.prepack_weights(w1.contiguous(), None if w_up is None else w_up.contiguous(), out=copies[0]),
+                  ops.prepack_weights(w2.contiguous(), out=copies[1]), None)
+        return copies, copies
 
     @staticmethod
     def _versions(raw):
@@ -174,23 +186,30 @@ class ExpertWeights:
     def prepare(cls, act: str, w1: torch.Tensor, w2: torch.Tensor, w_up: Optional[torch.Tensor] = None):
         e_l, H, F = w1.shape
         raw = (w1, w2, w_up)
-        p1, p2, pu = cls._derive(raw)
-        return cls(act, H, F, e_l, w1.dtype, p1, p2, pu, raw=raw, raw_versions=cls._versions(raw))
+        (p1, p2, pu), copies = cls._derive(raw)
+        return cls(act, H, F, e_l, w1.dtype, p1, p2, pu, raw=raw, raw_versions=cls._versions(raw), copies=copies)
 
     def refresh(self) -> "ExpertWeights":
         """Derive the kernels' copies again if a tensor prepare() was given has been updated in place since (an optimizer
         step): the forward pass would otherwise multiply with the weights of before the update while the backward pass,
-        which takes the tensors as they are, uses the new ones."""
+        which takes the tensors as they are, uses the new ones.  The copies stay where they are (a captured step holds their
+        addresses).  Under capture the derivation is recorded, to happen on every replay, and not counted as done."""
         if self.raw is not None and self._versions(self.raw) != self.raw_versions:
-            self.w1, self.w2, self.w_up = self._derive(self.raw)
-            self.raw_versions = self._versions(self.raw)
+            now = self._versions(self.raw)
+            (self.w1, self.w2, self.w_up), self.copies = self._derive(self.raw, self.copies)
+            if not L.capturing():
+                self.raw_versions = now
         return self
 
     def train_weights(self, rows: int):
         """(layout, w1, w_up, w2) for the forward pass of a bf16 training step on `rows` rows.  Weights that an optimizer has updated
         since they were re-tiled are taken as they are if the rows per expert are few: the GEMMs read the reference layout at 0.88 to
         0.96 of the rate, which costs more than re-tiling (reading and writing every weight in either direction) from some 4000
-        rows per expert on.  If they are still the same on the next call, they are re-tiled after all."""
+        rows per expert on.  If they are still the same on the next call, they are re-tiled after all.  A captured call takes them as
+        they are (see _PACKED): its replays may come after updates that nobody on the host sees."""
+        if L.capturing():
+            w1, w2, w_up = (None if t is None else t.detach().contiguous() for t in self.raw)
+            return L.W_RAW, w1, w_up, w2
         now = self._versions(self.raw)
         if now != self.raw_versions:
             if now != self.seen_versions and rows < 4096 * self.e_local and all(t is None or t.is_contiguous() for t in self.raw):
@@ -253,7 +272,10 @@ class ExpertMLP(torch.autograd.Function):
             return dx, None, None, dw1, dw2, None
         ws = _part_ws(tokens.device)
         if a1 is not None:
-            weights = (L.W_RAW_T, w1, w_up, w2) if ctx.raw else (L.W_TILED, _packed_weights_t(w1, w_up), None, _packed_weights_t(w2))
+            if ctx.raw or L.capturing():
+                weights = (L.W_RAW_T, w1.contiguous(), None if w_up is None else w_up.contiguous(), w2.contiguous())
+            else:
+                weights = (L.W_TILED, _packed_weights_t(w1, w_up), None, _packed_weights_t(w2))
             dx, dw1, dw2, dw_up = ops.mlp_train_backward(tokens, hidden, a1, dy, cnt, ew.act, *weights, part_ws=ws)
             return dx, None, None, dw1, dw2, dw_up
         NP = 2 * F if swiglu else F

@@ -346,8 +346,9 @@ def unpack_expert_major(recv: torch.Tensor, recv_counts: torch.Tensor, S_rows: i
 
 
 # ---- a11 / a12 ------------------------------------------------------------------------------
-def prepack_weights(w: torch.Tensor, w_up: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """[E_l,K,N] (reference layout) -> the MFMA kernels' K-contiguous layout (one-time, per weight)."""
+def prepack_weights(w: torch.Tensor, w_up: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """[E_l,K,N] (reference layout) -> the MFMA kernels' K-contiguous layout (one-time, per weight).  out: an earlier result for the
+    same shape, written again."""
     _req_cuda(w, "weights")
     assert w.dtype == torch.bfloat16, "prepack is for bf16 weights (fp32 uses the reference layout as is)"
     E_l, K, N = w.shape
@@ -356,7 +357,9 @@ def prepack_weights(w: torch.Tensor, w_up: Optional[torch.Tensor] = None) -> tor
         assert w_up.shape == w.shape and w_up.dtype == w.dtype
     n_eff = N * (2 if w_up is not None else 1)
     nbytes = L.lib().moe_prepack_bytes(L.MOE_BF16, E_l, K, n_eff)
-    out = torch.empty(nbytes, dtype=torch.uint8, device=w.device)
+    if out is None:
+        out = torch.empty(nbytes, dtype=torch.uint8, device=w.device)
+    assert out.dtype == torch.uint8 and out.numel() == nbytes and out.is_contiguous()
     L.check(L.lib().moe_prepack_weights(L.ptr(w), L.ptr(w_up), L.MOE_BF16, E_l, K, N, L.ptr(out), L.stream_ptr()))
     return out
 

@@ -1,0 +1,141 @@
+"""Calls under stream capture: what a graph records must not be taken for done by later eager calls or other graphs, and what a graph
+holds must stay where it is as long as the graph does."""
+import importlib
+
+import pytest
+import torch
+
+from iris_testing_amd import _lib as L
+from iris_testing_amd import ops
+from iris_testing_amd.layers import ExpertWeights, expert, expert_mlp
+
+expert_mod = importlib.import_module("iris_testing_amd.layers.expert")  # (the package re-exports the function under this name)
+DEV = "cuda"
+
+
+def _rnd(g, *s):
+    return (torch.randn(*s, generator=g, device=g.device) * s[-2] ** -0.5).bfloat16()
+
+
+def test_nothing_is_kept_for_later_calls_while_capturing(monkeypatch):
+    """The caches of derived weights under capture, without a GPU: same state after as before, and the tensors as they are in use."""
+    made = []
+
+    def pack(w, w_up=None, out=None):
+        made.append(torch.empty(1, dtype=torch.uint8) if out is None else out)
+        return made[-1]
+
+    monkeypatch.setattr(ops, "prepack_weights", pack)
+    monkeypatch.setattr(ops, "prepack_weights_transposed", pack)
+    capturing = [False]
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
+    g = torch.Generator().manual_seed(0)
+    w = _rnd(g, 2, 64, 64)
+    assert expert_mod._weights_for(w, 10)[1] == L.W_RAW  # the warm-up call
+    before = dict(expert_mod._PACKED)
+    capturing[0] = True
+    for _ in range(2):
+        for rows in (10, 10 ** 6):
+            got, layout = expert_mod._weights_for(w, rows)
+            assert got is w and layout == L.W_RAW
+        expert_mod._packed_weights_t(w)
+    assert expert_mod._PACKED == before
+    capturing[0] = False
+    assert expert_mod._weights_for(w, 10)[1] == L.W_TILED  # the second eager call re-tiles
+    # the expert MLP's weights after an update, when the first passes that see it are captured ones
+    ws = [_rnd(g, 2, 64, 64).requires_grad_() for _ in range(2)]
+    ew = ExpertWeights.prepare("silu", *ws)
+    copies = (ew.w1, ew.w2)
+    with torch.no_grad():
+        ws[0].mul_(2)
+    state = (ew.raw_versions, ew.seen_versions)
+    capturing[0] = True
+    for _ in range(2):
+        layout, w1, _, w2 = ew.train_weights(10)
+        assert layout == L.W_RAW and w1.data_ptr() == ws[0].data_ptr() and w2.data_ptr() == ws[1].data_ptr()
+        n = len(made)
+        ew.refresh()  # (recorded on every call: replays derive the copies anew)
+        assert len(made) == n + 2 and (ew.w1 is copies[0]) and (ew.w2 is copies[1]) and (ew.raw_versions, ew.seen_versions) == state
+    capturing[0] = False
+    ew.refresh()
+    assert ew.w1 is copies[0] and ew.w2 is copies[1] and ew.raw_versions == ew._versions(ew.raw) != state[0]
+    # fp32 weights are taken as they are where they lie in order, else as a copy that stays in its place
+    f1, f2 = torch.randn(2, 8, 8), torch.randn(2, 8, 8).transpose(1, 2)
+    ew = ExpertWeights.prepare("silu", f1, f2)
+    assert ew.w1.data_ptr() == f1.data_ptr() and torch.equal(ew.w2, f2)
+    at = ew.w2.data_ptr()
+    f1.add_(1)
+    f2.add_(1)
+    ew.refresh()
+    assert ew.w1.data_ptr() == f1.data_ptr() and ew.w2.data_ptr() == at and torch.equal(ew.w2, f2)
+
+
+def _capture(fn):
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        fn()  # one warm-up call
+    torch.cuda.current_stream().wait_stream(s)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = fn()
+    return graph, out
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [150, 9000])
+def test_expert_captured_after_one_warm_up(rows):
+    """Eager calls between the capture and the first replay, a second graph replayed before the first, an update between replays."""
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    x, w = _rnd(g, rows, 256), _rnd(g, 2, 256, 192)
+    cnt = torch.tensor([rows // 3, rows - rows // 3], dtype=torch.int32, device=DEV)
+    fresh = lambda: expert(x, w.clone(), cnt, rows)  # noqa: E731  (a tensor no cache has seen)
+    want = fresh()
+    graphs = [_capture(lambda: expert(x, w, cnt, rows)) for _ in range(2)]
+    assert torch.equal(expert(x, w, cnt, rows), want)
+    for graph, out in reversed(graphs):
+        out.zero_()
+        graph.replay()
+        assert torch.equal(out, want)
+    w.mul_(2.0)  # exact in bf16
+    assert torch.equal(expert(x, w, cnt, rows), want * 2)
+    trash = [torch.full((1 << 18,), float("nan"), dtype=torch.bfloat16, device=DEV) for _ in range(4)]  # (what the update gave back)
+    for graph, out in graphs:
+        graph.replay()
+        assert torch.equal(out, want * 2)
+    del trash
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("act", ["silu", "swiglu"])
+def test_training_step_captured_after_one_warm_up(act):
+    """A captured pass with the weight update in it: every replay is what the eager pass makes of the weights it finds, and the call
+    without gradients sees them afterwards."""
+    g = torch.Generator(device=DEV).manual_seed(5)
+    S, H, F, cnt = 130, 128, 192, torch.tensor([70, 60], dtype=torch.int32, device=DEV)
+    x, dy = _rnd(g, S, H), _rnd(g, S, H)
+    start = [_rnd(g, 2, H, F), _rnd(g, 2, F, H)] + ([_rnd(g, 2, H, F)] if act == "swiglu" else [])
+
+    def leaves():
+        return [t.clone().requires_grad_() for t in start]
+
+    def step(w, ew):
+        grads = torch.autograd.grad(expert_mlp(x, ew, cnt), w, dy)
+        with torch.no_grad():
+            for t, d in zip(w, grads):
+                t.sub_(d, alpha=0.25)
+        return grads
+
+    we, wc = leaves(), leaves()
+    ee, ec = (ExpertWeights.prepare(act, *w) for w in (we, wc))
+    graph, got = _capture(lambda: step(wc, ec))
+    step(we, ee)
+    for _ in range(3):
+        want = step(we, ee)
+        graph.replay()
+        for a, b in zip(list(got) + wc, list(want) + we):
+            assert torch.equal(a, b)
+        with torch.no_grad():
+            for t in wc + we:
+                t.add_(0)  # (tells the host that the weights changed, which a replay does not)
+            assert torch.equal(expert_mlp(x, ec, cnt), expert_mlp(x, ee, cnt))
