@@ -20,6 +20,7 @@ constexpr int GS_BN = 128;
 constexpr int GS_THREADS = 256;
 constexpr int GS_CTR_BYTES = 16384;  // arrival counters at the start of the workspace: one 64-bit word per tile
 constexpr int GS_MIN_PART_STAGES = 32;  // K stages per part at least: what the hand-over of a split tile costs is worth about as many
+constexpr int GS_PART_BYTES = 8 << 20;  // room for parts that a launch uses at most: splits beyond that cost more than they give
 constexpr int GS_LDO = GS_BN + 4;    // pitch of the epilogue's fp32 tile in LDS
 
 template <int BM>
@@ -496,7 +497,7 @@ template <int BM, bool FP8, int EPI, bool BSA, int BMODE>
 static void gs_launch(const GsParams& q0, void* part_ws, size_t part_ws_bytes, int cus, hipStream_t s) {
     GsParams q = q0;
     constexpr int lds = gs_lds_bytes<BM, BSA>();
-    q.slots = (int)std::min<long long>(cus, (8 << 20) / (BM * GS_BN * 4));  // (units worth splitting for)
+    q.slots = (int)std::min<long long>(cus, GS_PART_BYTES / (BM * GS_BN * 4));  // (units worth splitting for)
     q.g.part_ws = nullptr;
     q.g.max_units = 0;
     const long long unit_bytes = (long long)BM * GS_BN * 4;
@@ -588,6 +589,8 @@ int gs_choose_bm(int S_rows, int E_l, int K, int ncols, bool fp8, int cus) {
     }
     return bm_best;
 }
+
+size_t gs_workspace_bytes(int cus) { return GS_CTR_BYTES + std::min<size_t>((size_t)cus * 64 * GS_BN * 4, GS_PART_BYTES); }
 
 int launch_gemm_small(const GemmParams& p, bool fp8, int bm, int epi, void* ws, size_t bytes, int cus, hipStream_t s) {
     GsParams q{};

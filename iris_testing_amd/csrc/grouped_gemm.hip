@@ -1727,7 +1727,7 @@ extern "C" int moe_gemm_split_plan(int total_tiles, int grid, int k_stages, int 
     return MOE_OK;
 }
 
-extern "C" size_t moe_gemm_part_workspace_bytes(void) { return (size_t)num_cus() * 256 * GG_BN * sizeof(float); }
+extern "C" size_t moe_gemm_part_workspace_bytes(void) { return gs_workspace_bytes(num_cus()); }
 
 extern "C" int moe_grouped_gemm_mapped(const void* a_base, int a_rows, const int32_t* a_row_map, const void* packed,
                                        const int32_t* expert_cnt, int S_rows, int K, int N, int E_l, int act, void* out,

@@ -4,7 +4,6 @@ expert MLP the workloads define (Linear-act-Linear, SwiGLU, fp8) which the refer
 from __future__ import annotations
 
 import weakref
-from collections import OrderedDict
 from dataclasses import dataclass, field
 from typing import Optional
 
@@ -22,8 +21,6 @@ from ..utils import _assert_cuda_int32
 # happened for the next eager call or the next graph, a copy dropped after an update would be freed under the graph, and a graph
 # that holds an optimizer's update has to read the weights it left.  A captured call multiplies with the tensors as they are.
 _PACKED = {}
-_PART_WS = OrderedDict()
-_PART_WS_MAX = 4  # streams with a workspace of their own (67 MB each); the one not used for longest is given back
 
 
 def _pack_key(kind: str, w: torch.Tensor, w_up: Optional[torch.Tensor]):
@@ -87,19 +84,9 @@ def _grouped_gemm_t(do: torch.Tensor, weights: torch.Tensor, cnt: torch.Tensor) 
 
 
 def _part_ws(device) -> torch.Tensor:
-    """Partial-sum workspace for the K split of GEMMs of few tiles: one per device and stream, since launches that may overlap must not
-    share it."""
-    key = (device, L.stream_ptr())
-    ws = _PART_WS.pop(key, None)
-    if ws is None:
-        ws = ops.gemm_part_workspace(device)
-    _PART_WS[key] = ws  # (now the last)
-    while len(_PART_WS) > _PART_WS_MAX:
-        try:
-            _PART_WS.popitem(last=False)
-        except KeyError:  # (another thread was quicker)
-            break
-    return ws
+    """Partial-sum workspace for the K split of GEMMs of few tiles, for one call: launches that may overlap must not share it, and under
+    capture it has to belong to the graph.  (8 MB of the caching allocator's, which costs the host what a lookup did.)"""
+    return ops.gemm_part_workspace(device)
 
 
 def _grouped_gemm(tokens: torch.Tensor, weights: torch.Tensor, cnt: torch.Tensor) -> torch.Tensor:

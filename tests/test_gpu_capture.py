@@ -139,3 +139,38 @@ def test_training_step_captured_after_one_warm_up(act):
             for t in wc + we:
                 t.add_(0)  # (tells the host that the weights changed, which a replay does not)
             assert torch.equal(expert_mlp(x, ec, cnt), expert_mlp(x, ee, cnt))
+
+
+def test_partial_sum_workspace_belongs_to_its_call(monkeypatch):
+    """No two calls share it (they may be on streams that overlap, or in a graph), and nothing else keeps or gives back one in use."""
+    import weakref
+    monkeypatch.setattr(L, "stream_ptr", lambda: 0)
+    first, second = expert_mod._part_ws("cpu"), expert_mod._part_ws("cpu")
+    assert first.data_ptr() != second.data_ptr()
+    assert first.numel() * first.element_size() == L.lib().moe_gemm_part_workspace_bytes() <= (8 << 20) + (1 << 16)
+    refs = [weakref.ref(first), weakref.ref(second)]
+    del first, second
+    assert all(r() is None for r in refs)
+
+
+@pytest.mark.gpu
+def test_graph_keeps_its_workspace_while_other_streams_come_and_go():
+    """A GEMM whose tiles are cut along K, captured on a stream of its own; the same call on more streams than any pool would hold,
+    then tensors over the memory that became free: the replays give the same bits and touch none of them."""
+    g = torch.Generator(device=DEV).manual_seed(3)
+    x, w, cnt = _rnd(g, 64, 8192), _rnd(g, 1, 8192, 512), torch.tensor([64], dtype=torch.int32, device=DEV)
+    want = expert(x, w, cnt, 64)
+    graph, out = _capture(lambda: expert(x, w, cnt, 64))
+    for _ in range(6):
+        s = torch.cuda.Stream()
+        s.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(s):
+            assert torch.equal(expert(x, w, cnt, 64), want)
+        torch.cuda.current_stream().wait_stream(s)
+    canaries = [torch.full((1 << 21,), 7.0, device=DEV) for _ in range(40)]  # 8 MB each
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+    assert all(bool((c == 7.0).all()) for c in canaries)
