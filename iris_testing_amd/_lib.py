@@ -6,6 +6,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import struct
 from ctypes import c_char_p, c_float, c_int, c_int32, c_size_t, c_uint8, c_void_p, POINTER
 
 import torch  # noqa: F401  (must be imported first: the library binds the HIP runtime torch loaded)
@@ -38,6 +39,10 @@ class StepArgs(ctypes.Structure):
         "pos row_token count_ws count_ws_bytes send send_scale send_gate status recv recv_scale recv_gate "
         "recv_counts row_map expert_cnt row_gate w1 w_up w2 s1 s_up s2 rows y hidden_ws xq hq hscale xs unpack_map "
         "ret_map part_ws part_ws_bytes ret returned zero_off out").split()]
+
+
+# StepArgs as struct.pack takes it: integers, then addresses and sizes
+STEP_LAYOUT = struct.Struct("".join("i" if t is c_int32 else "P" for _, t in StepArgs._fields_))
 
 
 class A2aSource(ctypes.Structure):

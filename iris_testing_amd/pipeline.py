@@ -80,6 +80,9 @@ class DispatchPipeline:
         self.count_ws_bytes = lib.moe_count_workspace_bytes(T, k, E)
         self.count_ws = torch.empty(self.count_ws_bytes, dtype=torch.uint8, device=dev)
         self.send = torch.empty((W, M, H), dtype=dt, device=dev) if not self.padding_free else None
+        # (buffers of modes that are off)
+        self.send_gate = self.row_gate = self.payload = self.ret_flat = self.zero_off = self.send_q = self.send_scale = None
+        self.xq = self.xs = self.hq = self.hsc = None
         if self.gated:
             self.send_gate = torch.empty((W, M), dtype=torch.float32, device=dev)
             self.row_gate = torch.empty((max(S, 1),), dtype=torch.float32, device=dev)
@@ -115,34 +118,35 @@ class DispatchPipeline:
             self.returned = returned if returned is not None else torch.zeros((W, M, H), dtype=dt, device=dev)
         self.out = torch.empty((T, H), dtype=dt, device=dev)
         self._p = L.ptr
-        self._args = self._step_args()
+        self._args = L.StepArgs()
 
-    def _step_args(self) -> L.StepArgs:
-        """The argument block of moe_step: sizes, modes and this object's own buffers (step() fills in the rest)."""
-        c, ew, p = self.cfg, self.weights, self._p
-        get = lambda name: p(getattr(self, name, None))  # noqa: E731  (buffers a mode does not use do not exist)
-        return L.StepArgs(
-            tokens=c.tokens, hidden=c.hidden, experts=c.experts, topk=c.topk, world=c.world, ffn=c.ffn, act=L.ACT[ew.act],
-            dtype=self.code, M=self.world.M, S=self.S, fused=self.fused, flat=self.padding_free, gated=self.gated,
-            quant=ew.dtype == torch.uint8, q_dispatch=self.fp8_dispatch, f32_weights=ew.dtype == torch.float32,
-            send=p(self.send_q if self.fp8_dispatch else self.payload if self.padding_free else self.send),
-            hidden_ws=get("hidden"), hscale=get("hsc"), ret=p(self.ret_flat if self.padding_free else self.ret),
-            **{n: get(n) for n in ("logits idx gate route_ws send_counts expert_offs dst_sizes dst_offsets caps pos row_token count_ws "
-                                   "send_scale send_gate status row_map expert_cnt row_gate rows y xq hq xs unpack_map ret_map part_ws "
-                                   "zero_off out").split()},
-            route_ws_bytes=self.route_ws_bytes, count_ws_bytes=self.count_ws_bytes, part_ws_bytes=self.part_ws_bytes)
+    def _fill(self) -> L.StepArgs:
+        """The argument block of moe_step, written anew for every step: any buffer may have been replaced since the last one (an
+        output kept by its reader, say).  All fields in one go, in the order of the structure: 7 us of host time, set one by
+        one 12."""
+        c, w, ew = self.cfg, self.world, self.weights.refresh()
+        s1, s_up, s2 = ew.scales or (None, None, None)
+        send, recv, ret = self.send, w.recv, self.ret
+        if self.fp8_dispatch:
+            send, recv = self.send_q, w.recv_q
+        elif self.padding_free:
+            send, recv, ret = self.payload, self.recv_flat, self.ret_flat
+        at = [0 if t is None else t.data_ptr() for t in (
+            w.x0, w.router, w.bias, self.logits, self.idx, self.gate, self.route_ws,
+            self.send_counts, self.expert_offs, self.dst_sizes, self.dst_offsets, self.caps, self.pos, self.row_token, self.count_ws,
+            send, self.send_scale, self.send_gate, self.status, recv, w.recv_scale, self.recv_gate, w.recv_counts, self.row_map,
+            self.expert_cnt, self.row_gate, ew.w1, ew.w_up, ew.w2, s1, s_up, s2, self.rows, self.y, self.hidden, self.xq, self.hq,
+            self.hsc, self.xs, self.unpack_map, self.ret_map, self.part_ws,
+            ret, self.returned, self.zero_off, self.out)]
+        L.STEP_LAYOUT.pack_into(
+            self._args, 0, c.tokens, c.hidden, c.experts, c.topk, c.world, c.ffn, L.ACT[ew.act], self.code, w.M, self.S, self.fused,
+            self.padding_free, self.gated, ew.dtype == torch.uint8, self.fp8_dispatch, ew.dtype == torch.float32,
+            *at[:7], self.route_ws_bytes, *at[7:15], self.count_ws_bytes, *at[15:42], self.part_ws_bytes, *at[42:])
+        return self._args
 
     def _run(self, s):
         """The stages of STAGES as one call (the map, scales, gates and padding of the destination side in one launch)."""
-        a, w, ew, p = self._args, self.world, self.weights.refresh(), self._p
-        # what belongs to the caller is looked up on every step
-        a.x, a.router, a.bias, a.recv_counts = p(w.x0), p(w.router), p(w.bias), p(w.recv_counts)
-        a.recv = p(w.recv_q if self.fp8_dispatch else self.recv_flat if self.padding_free else w.recv)
-        a.recv_scale, a.recv_gate = p(w.recv_scale), p(self.recv_gate)
-        a.w1, a.w_up, a.w2, a.returned = p(ew.w1), p(ew.w_up), p(ew.w2), p(self.returned)
-        if ew.dtype == torch.uint8:
-            a.s1, a.s_up, a.s2 = (p(t) for t in ew.scales)
-        L.check(L.lib().moe_step(a, s))
+        L.check(L.lib().moe_step(self._fill(), s))
 
     # each stage is a closure-free method so that callers can time them one by one
     def route(self, s):

@@ -171,3 +171,58 @@ def test_ctypes_table_has_the_argument_count_of_every_declaration():
         assert m, f"{name} is not declared"
         params = [x for x in m.group(1).split(",") if x.strip() and x.strip() != "void"]
         assert len(params) == len(args), f"{name}: header declares {len(params)} arguments, the ctypes table {len(args)}"
+
+
+@pytest.mark.parametrize("kind,mode", [("f32", {}), ("bf16", {}), ("bf16", dict(gated=True)), ("bf16", dict(padding_free=True)),
+                                       ("fp8", {}), ("fp8", dict(fp8_dispatch=False)), ("fp8", dict(gated=True)), ("fp8", dict(padding_free=True))])
+def test_step_takes_the_buffers_of_the_moment(monkeypatch, kind, mode):
+    """Every field of the step's argument block is what its name says, and a buffer that the caller has replaced, or given other
+    memory, is the one the next step gets.  (CPU tensors; the library call is replaced by a look at its argument.)"""
+    import types
+    from iris_testing_amd import _lib as L
+    from iris_testing_amd.configs import MoEConfig
+    from iris_testing_amd.harness import World
+    from iris_testing_amd.layers import ExpertWeights
+    from iris_testing_amd.pipeline import DispatchPipeline
+    T, H, E, k, W, F, M, S = 6, 128, 8, 2, 4, 256, 5, 11
+    cfg = MoEConfig("case", 0, T, H, "f32" if kind == "f32" else "bf16", E, k, W, F, "swiglu" if kind == "fp8" else "silu")
+    dt, e_l = cfg.torch_dtype, cfg.e_local
+    world = World(cfg, torch.empty(H, E, dtype=dt), torch.empty(E), torch.empty(T, H, dtype=dt), [], M, 3, torch.empty(W, M, H, dtype=dt),
+                  torch.empty(W, e_l, dtype=torch.int32), S)
+    w1, w2 = torch.empty(e_l, H, F, dtype=dt), torch.empty(e_l, F, H, dtype=dt)
+    if kind == "fp8":
+        world.recv_q, world.recv_scale = torch.empty(W, M, H, dtype=torch.uint8), torch.empty(W, M)
+        ew = ExpertWeights("swiglu", H, F, e_l, torch.uint8, w1, w2, scales=tuple(torch.empty(e_l, n) for n in (F, F, H)))
+    else:
+        ew = ExpertWeights("silu", H, F, e_l, dt, w1, w2)
+    pipe = DispatchPipeline(world, ew, recv_gate=torch.empty(W, M) if mode.get("gated") else None,
+                            recv_flat=torch.empty(S, H, dtype=dt) if mode.get("padding_free") else None, **mode)
+    seen = {}
+    stub = types.SimpleNamespace(moe_step=lambda a, s: seen.update({n: getattr(a, n) or 0 for n, _ in L.StepArgs._fields_}) or 0)
+    monkeypatch.setattr(L, "lib", lambda: stub)
+    monkeypatch.setattr(L, "stream_ptr", lambda: 0)
+
+    def want():
+        flat, q = pipe.padding_free, pipe.fp8_dispatch
+        out = dict(tokens=T, hidden=H, experts=E, topk=k, world=W, ffn=F, act=L.ACT[ew.act], dtype=pipe.code, M=M, S=S, fused=pipe.fused,
+                   flat=flat, gated=pipe.gated, quant=kind == "fp8", q_dispatch=q, f32_weights=kind == "f32",
+                   route_ws_bytes=pipe.route_ws_bytes, count_ws_bytes=pipe.count_ws_bytes, part_ws_bytes=pipe.part_ws_bytes)
+        t = dict(x=world.x0, router=world.router, bias=world.bias, recv_counts=world.recv_counts, recv_scale=world.recv_scale,
+                 recv=world.recv_q if q else pipe.recv_flat if flat else world.recv, w1=ew.w1, w_up=ew.w_up, w2=ew.w2,
+                 s1=ew.scales and ew.scales[0], s_up=ew.scales and ew.scales[1], s2=ew.scales and ew.scales[2],
+                 send=pipe.send_q if q else pipe.payload if flat else pipe.send, ret=pipe.ret_flat if flat else pipe.ret,
+                 hidden_ws=pipe.hidden, hscale=pipe.hsc)
+        t.update({n: getattr(pipe, n, None) for n, _ in L.StepArgs._fields_ if n not in out and n not in t})
+        out.update({n: 0 if v is None else v.data_ptr() for n, v in t.items()})
+        return {n: int(v) for n, v in out.items()}
+
+    pipe.step()
+    assert seen == want()
+    for n in [n for n, v in vars(pipe).items() if isinstance(v, torch.Tensor)]:
+        setattr(pipe, n, torch.empty_like(getattr(pipe, n)))  # (the old one is freed)
+        pipe.step()
+        assert seen == want(), n
+    keep = pipe.out.clone()
+    pipe.out.data = keep
+    pipe.step()
+    assert seen["out"] == keep.data_ptr()
