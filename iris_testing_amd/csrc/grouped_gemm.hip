@@ -1428,7 +1428,7 @@ __global__ __launch_bounds__(256) void act_backward_vec_kernel(const uint4* __re
             unpack(a1[base + 4], u);
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                const float s = __builtin_amdgcn_rcpf(1.0f + __expf(-x[e]));
+                const float s = 1.0f / (1.0f + __expf(-x[e]));
                 o[e] = d[e] * u[e] * (s * (1.0f + x[e] * (1.0f - s)));
                 ou[e] = d[e] * (x[e] * s);
             }
@@ -1441,7 +1441,7 @@ __global__ __launch_bounds__(256) void act_backward_vec_kernel(const uint4* __re
                 if constexpr (EPI == EPI_GELU)
                     o[e] = d[e] * (0.5f * (1.0f + erff(x[e] * 0.70710678118654752440f)) + x[e] * 0.39894228040143267794f * __expf(-0.5f * x[e] * x[e]));
                 else {
-                    const float s = __builtin_amdgcn_rcpf(1.0f + __expf(-x[e]));
+                    const float s = 1.0f / (1.0f + __expf(-x[e]));
                     o[e] = d[e] * (s * (1.0f + x[e] * (1.0f - s)));
                 }
             }

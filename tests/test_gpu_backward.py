@@ -261,3 +261,15 @@ def test_training_pass_on_weights_as_they_are(act, cnt, H, F):
     dw = ops.grouped_gemm_dw(x, d_pre, c, split_F=F if act == "swiglu" else 0)
     assert torch.equal(dw1, dw[..., :F]) and (dw_up is None or torch.equal(dw_up, dw[..., F:])) and NP == dw.shape[-1]
     assert torch.equal(dw2, ops.grouped_gemm_dw(hidden, dy, c))
+
+
+@pytest.mark.parametrize("act", ["gelu", "silu"])
+def test_activation_gradient_is_the_same_in_either_form(act):
+    """Eight columns per thread (F a multiple of 8) and one (F = 4) evaluate the same fp32 expression, division and all, on every
+    value: same bits, also at the ends of the range."""
+    g = torch.Generator(device=DEV).manual_seed(9)
+    x = (4 * torch.randn(1 << 20, generator=g, device=DEV)).bfloat16()
+    x[:6] = torch.tensor([0.0, -0.0, 88.0, -88.0, -3.3e38, 3.3e38], device=DEV).bfloat16()
+    dh = torch.randn(1 << 20, generator=g, device=DEV).bfloat16()
+    wide, narrow = (ops.mlp_act_backward(x.view(-1, F), dh.view(-1, F), act).view(-1) for F in (1024, 4))
+    assert torch.equal(wide.view(torch.int16), narrow.view(torch.int16))
