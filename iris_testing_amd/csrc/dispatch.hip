@@ -89,6 +89,54 @@ __device__ __forceinline__ void offsets_body(const int32_t* counts /*LDS*/, int 
     if (lane == 0) { caps[0] = max(mmax, 1); caps[1] = max(cmax, 1); }
 }
 
+// ---- 2b. many tokens: what the blocks before a ranking workgroup hold, by a scan over the histogram.  A workgroup takes SCAN_E experts,
+// thread (slice, expert) a run of ranking groups (rank_blocks<false>() rows each): sums per slice, a scan of them over the
+// lanes, then base[group][e] = rows of e in the groups before it, and after the last group the totals.  Two reads and a quarter
+// of a write per histogram cell, in rows of 64 bytes; bound by the latency of a slice's run (262144 tokens x 8 of 256: the count takes
+// 43 us, with the sums below 181, with one wave per expert along all blocks 101).
+constexpr int SCAN_E = 16, SCAN_SLICES = 64;
+constexpr int RANK_WAVES = 16;
+template <bool ONE>
+constexpr int rank_blocks() { return ONE ? 16 : 4; }
+__global__ __launch_bounds__(SCAN_E * SCAN_SLICES) void scan_hist_kernel(const int32_t* __restrict__ hist, int32_t* __restrict__ base, int NB,
+                                                                         int NG, int E) {
+    __shared__ int32_t sum[SCAN_E][SCAN_SLICES + 1];
+    constexpr int ROWS = rank_blocks<false>();
+    static_assert(SCAN_SLICES == WAVE, "a slice per lane, an expert per wave");
+    const int c = threadIdx.x % SCAN_E, sl = threadIdx.x / SCAN_E, e = blockIdx.x * SCAN_E + c;
+    const int per = (NG + SCAN_SLICES - 1) / SCAN_SLICES, g0 = min(sl * per, NG), g1 = min(g0 + per, NG);
+    auto group = [&](int g) {
+        int v = 0;
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) {
+            const int b = g * ROWS + r;
+            v += b < NB ? hist[(size_t)b * E + e] : 0;
+        }
+        return v;
+    };
+    int all = 0;
+    if (e < E) {
+#pragma unroll 4
+        for (int g = g0; g < g1; ++g) all += group(g);
+    }
+    sum[c][sl] = all;
+    __syncthreads();
+    const int wave = threadIdx.x / WAVE;  // (one wave per expert)
+    const int mine = sum[wave][lane_id()], incl = wave_incl_scan(mine);
+    __syncthreads();
+    sum[wave][lane_id()] = incl - mine;
+    if (lane_id() == WAVE - 1) sum[wave][SCAN_SLICES] = incl;
+    __syncthreads();
+    if (e >= E) return;
+    int run = sum[c][sl];
+#pragma unroll 4
+    for (int g = g0; g < g1; ++g) {
+        base[(size_t)g * E + e] = run;
+        run += group(g);
+    }
+    if (sl == 0) base[(size_t)NG * E + e] = sum[c][SCAN_SLICES];
+}
+
 // ---- 3. stable positions.  A workgroup of 16 waves ranks RBLK consecutive blocks of 64 tokens, 16 / RBLK waves to a block, each with
 // every (16 / RBLK)-th of a token's slots: the waves OR their lane bits into a 64-bit mask per block and expert in LDS (a token holds
 // an expert at most once), and the rank of a slot inside its expert is the rows of the expert in earlier workgroups' blocks +
@@ -99,11 +147,10 @@ __device__ __forceinline__ void offsets_body(const int32_t* counts /*LDS*/, int 
 // with 16 the popcounts of up to 15 masks per slot and four workgroups in all took 22 us for 4096 tokens x 8 of 256, so 9.
 // (scan and rank took 22 us as launches of their own.)
 // ONE = true (up to 1024 tokens): a single workgroup holds all 16 blocks, counts for itself and is the only launch.
-constexpr int RANK_WAVES = 16;
+// base (or NULL): what scan_hist_kernel left, where the sums, which grow with the square of the tokens, are too many (RANK_SUM_CELLS).
 template <bool ONE>
-constexpr int rank_blocks() { return ONE ? 16 : 4; }
-template <bool ONE>
-__global__ __launch_bounds__(RANK_WAVES * WAVE) void rank_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict__ hist, int T,
+__global__ __launch_bounds__(RANK_WAVES * WAVE) void rank_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict__ hist,
+                                                                  const int32_t* __restrict__ base, int T,
                                                                   int k, int E, int W, int NB, int32_t* __restrict__ send_counts,
                                                                   int32_t* __restrict__ expert_offs, int32_t* __restrict__ dst_sizes,
                                                                   int32_t* __restrict__ dst_offsets, int32_t* __restrict__ caps,
@@ -117,7 +164,10 @@ __global__ __launch_bounds__(RANK_WAVES * WAVE) void rank_kernel(const int32_t* 
     int mine[SLOTS];
 #pragma unroll
     for (int j = 0; j < SLOTS; ++j) mine[j] = (live && j * PARTS + part < k) ? idx[(size_t)t * k + j * PARTS + part] : -1;
-    for (int e = tid; e < E; e += blockDim.x) tot[e] = pre[e] = 0;
+    for (int e = tid; e < E; e += blockDim.x) {
+        tot[e] = !ONE && base ? base[(size_t)gridDim.x * E + e] : 0;
+        pre[e] = !ONE && base ? base[(size_t)blockIdx.x * E + e] : 0;
+    }
     for (int i = tid; i < RBLK * E; i += blockDim.x) masks[i] = 0ull;
     __syncthreads();
     unsigned long long* my = masks + blk * E;
@@ -155,8 +205,10 @@ __global__ __launch_bounds__(RANK_WAVES * WAVE) void rank_kernel(const int32_t* 
                 atomicAdd(&pre[c * V + i], before[i]);
             }
         };
-        if (E % 4 == 0) sums(std::integral_constant<int, 4>{});
-        else sums(std::integral_constant<int, 1>{});
+        if (!base) {
+            if (E % 4 == 0) sums(std::integral_constant<int, 4>{});
+            else sums(std::integral_constant<int, 1>{});
+        }
     }
     __syncthreads();
     if (wave == 0) offsets_body(tot, E, W, es, blockIdx.x == 0, send_counts, expert_offs, dst_sizes, dst_offsets, caps);
@@ -933,10 +985,16 @@ __global__ __launch_bounds__(256) void shuffle_totals_kernel(const int32_t* __re
 
 }  // namespace
 
+// Histogram cells that the ranking workgroups may read in all (the square of the tokens) before the scan in front of them, a third launch,
+// is the better choice.  Sums against scan in us: 8 experts 10.4 / 13.2 (65536 tokens, 2 M cells) and 14.0 / 12.6 (131072, 8 M);
+// 256 experts 11.7 / 12.7 (8192, 1 M), 13.5 / 13.1 (16384, 4 M), 17.2 / 14.0 (32768, 16 M) and 181 / 43 (262144, 1 G); 512 experts
+// 14.4 / 13.6 (8192, 2 M) and 18.1 / 14.0 (16384, 8 M).
+constexpr long long RANK_SUM_CELLS = 6ll << 20;
+
 extern "C" size_t moe_count_workspace_bytes(int T, int k, int E) {
     (void)k;
     const size_t NB = (size_t)ceil_div(T > 0 ? T : 1, CB);
-    // hist[NB][E]; the size callers were always asked for (twice that and two rows)
+    // hist[NB][E], base[NG + 1][E] (NG = ranking groups); the size callers were always asked for
     return sizeof(int32_t) * (2 * (size_t)E * NB + 2 * (size_t)E + 1);
 }
 
@@ -956,13 +1014,19 @@ extern "C" int moe_count_and_offsets(const int32_t* topk_idx, int T, int k, int 
     int32_t* hist = (int32_t*)ws;
     auto lds = [&](int blocks) { return (size_t)blocks * E * sizeof(unsigned long long); };
     if (NB <= rank_blocks<true>()) {  // (few tokens: one workgroup holds everything)
-        rank_kernel<true><<<1, RANK_WAVES * WAVE, lds(rank_blocks<true>()), s>>>(topk_idx, nullptr, T, k, E, W, NB, send_counts, expert_offs, dst_sizes, dst_offsets,
+        rank_kernel<true><<<1, RANK_WAVES * WAVE, lds(rank_blocks<true>()), s>>>(topk_idx, nullptr, nullptr, T, k, E, W, NB, send_counts, expert_offs, dst_sizes, dst_offsets,
                                                            caps, pos, row_token);
         return moe_check_launch("count_and_offsets");
     }
     block_hist_kernel<<<ceil_div(NB, 4), 256, 4 * E * sizeof(int32_t), s>>>(topk_idx, hist, T, k, E, NB);
-    rank_kernel<false><<<ceil_div(NB, rank_blocks<false>()), RANK_WAVES * WAVE, lds(rank_blocks<false>()), s>>>(
-        topk_idx, hist, T, k, E, W, NB, send_counts, expert_offs, dst_sizes, dst_offsets, caps, pos, row_token);
+    const int NG = ceil_div(NB, rank_blocks<false>());
+    int32_t* base = nullptr;
+    if ((long long)NG * NB * E > RANK_SUM_CELLS) {
+        base = hist + (size_t)NB * E;
+        scan_hist_kernel<<<ceil_div(E, SCAN_E), SCAN_E * SCAN_SLICES, 0, s>>>(hist, base, NB, NG, E);
+    }
+    rank_kernel<false><<<NG, RANK_WAVES * WAVE, lds(rank_blocks<false>()), s>>>(
+        topk_idx, hist, base, T, k, E, W, NB, send_counts, expert_offs, dst_sizes, dst_offsets, caps, pos, row_token);
     return moe_check_launch("count_and_offsets");
 }
 

@@ -515,6 +515,27 @@ def test_counts_and_positions_at_block_edges(T, E, W, k):
     assert c.caps.tolist() == [max(1, int(sizes.max())), max(1, int(counts.max()))]
 
 
+@pytest.mark.parametrize("T,E,W,k", [(14080, 512, 8, 4), (14081, 512, 8, 4), (14400, 511, 7, 1), (65600, 73, 1, 2), (81001, 17, 1, 3), (330000, 1, 1, 1)])
+def test_counts_and_positions_of_many_tokens(T, E, W, k):
+    """Either side of where the ranking workgroups' own sums over the histogram give way to a scan (6 M cells read in all), which takes
+    16 experts to a workgroup and 64 slices of groups of 4 blocks of tokens."""
+    rng = np.random.default_rng(T + E)
+    p = rng.random(E) ** 4 + 1e-6
+    # (k distinct experts per token, drawn in proportion to p: the smallest of exponential times)
+    idx = np.concatenate([np.argsort(rng.exponential(size=(min(8192, T - t), E)) / p, axis=1)[:, :k] for t in range(0, T, 8192)]).astype(np.int32)
+    c = ops.count_and_offsets(torch.from_numpy(idx).to(DEV), E, W)
+    counts = O.send_counts(idx, W, E)
+    sizes, offs = O.dst_sizes_offsets(counts)
+    pos, row_token = O.payload_positions(idx, E)
+    assert_bits_equal(c.send_counts, counts, "send_counts")
+    assert_bits_equal(c.expert_offs, O.build_expert_offsets(counts), "expert_offs")
+    assert_bits_equal(c.dst_sizes, sizes, "dst_sizes")
+    assert_bits_equal(c.dst_offsets, offs, "dst_offsets")
+    assert_bits_equal(c.pos, pos, "pos")
+    assert_bits_equal(c.row_token, row_token, "row_token")
+    assert c.caps.tolist() == [max(1, int(sizes.max())), max(1, int(counts.max()))]
+
+
 @pytest.mark.parametrize("T,H,k", [(1, 520, 1), (5, 4096, 3), (33, 1032, 8), (700, 264, 2), (2050, 2056, 4)])
 def test_row_copies_and_sums_cut_into_column_runs(T, H, k):
     """Rows cut into runs of columns (whole, ragged, single) where tokens are few, and for the sums where rows are long; pack, combine and the gradient of combine."""
