@@ -179,7 +179,8 @@ int moe_unpack_expert_major(const void* recv, int dtype, int W, int M, int H, co
  * out[rows of e] = tokens[rows of e] @ weights[e], fp32 accumulate, cast to `dtype`;
  * rows of e = [sum cnt[:e], +cnt[e]).  tokens [S_rows,K]; weights [E_l,K,N] (N contiguous, the
  * reference layout); out [S_rows,N].  Rows past sum(cnt) are left untouched.
- * For bf16 the weights are re-tiled into ws first (moe_prepack_bytes(...) bytes). */
+ * bf16 weights are multiplied as they are; only those that are not 16-byte aligned are re-tiled first, into ws (moe_prepack_bytes(...)
+ * bytes; else it may be NULL). */
 size_t moe_prepack_bytes(int dtype, int E_l, int K, int N);
 int moe_grouped_gemm(const void* tokens, const void* weights, const int32_t* expert_cnt, int dtype, int S_rows,
                      int K, int N, int E_l, void* out, void* ws, size_t ws_bytes, moe_stream_t stream);
@@ -356,7 +357,7 @@ int moe_grouped_gemm_dw_pair(const void* x, const void* dy, const int32_t* exper
  * backward: dh [S,F] and d_pre (layout of pre_act) are scratch; dx [S,H], dw1 / dw_up [E_l,H,F] (dw_up: SwiGLU only), dw2
  * [E_l,F,H].  layout MOE_W_RAW_T: w1, w_up, w2 in the reference layout; MOE_W_TILED: w1 (of the pair) and w2 as
  * moe_prepack_weights_transposed makes them (w_up NULL).
- * Rows of out and dx past the counted total are zeroed. */
+ * Weights must be 16-byte aligned.  Rows of out and dx past the counted total are zeroed. */
 int moe_mlp_train_forward(const void* x, const int32_t* expert_cnt, int S_rows, int H, int F, int E_l, int act, int layout,
                           const void* w1, const void* w_up, const void* w2, void* hidden, void* pre_act, void* out, void* part_ws,
                           size_t part_ws_bytes, moe_stream_t stream);
@@ -416,7 +417,7 @@ int moe_diag_gemm_trace(unsigned long long* trace, size_t words, int flags);
 /* ---- the exchange of a simulated world, and what the shuffle has to know on the host ---------------------------------
  * moe_a2a_place: what arrives at `rank` when every source sends its padding-free payload (the reference's custom_a2a moves these
  *   rows between GPUs, layers/all_to_all.py:10-125): sources[s] (host array of W; payload NULL: sends nothing) gives the payload
- *   [rows,H] of rank s, its counts for this rank [E_l] and where its block for this rank starts (one int32 in device memory).
+ *   [rows,H] of rank s (16-byte aligned), its counts for this rank [E_l] and where its block for this rank starts (one int32 in device memory).
  *   token_buf [E_l,W,CAP,H] <- row block start + (rows of the experts before e) + j of source s at [e,s,j], zeros
  *   past its count; pca[e,s] = counts; counts_ready / token_sync (n_ready / n_sync int32 each, nullable) <- W.
  *   If a count exceeds CAP nothing is written.
@@ -438,7 +439,7 @@ int moe_wait_i32(const int32_t* value, int32_t pending, moe_stream_t stream);
 int moe_shuffle_totals(const int32_t* pca, int n, const int32_t* token_sync, int n_sync, int32_t* out, moe_stream_t stream);
 /* moe_expert_forward: out[rows of g] = tokens[rows of g] @ w[g] (bf16) with the rows of out past the counted total zeroed (the
  * caller's out needs no clearing).  layout MOE_W_TILED: weights as moe_prepack_weights makes them of [E_l,K,N]; MOE_W_RAW: [E_l,K,N]
- * as they are; MOE_W_RAW_T: [E_l,N,K] as they are (out = tokens w^T). */
+ * as they are; MOE_W_RAW_T: [E_l,N,K] as they are (out = tokens w^T).  Weights must be 16-byte aligned. */
 int moe_expert_forward(const void* tokens, const void* weights, int layout, const int32_t* expert_cnt, int S_rows, int K, int N, int E_l,
                        void* out, void* part_ws, size_t part_ws_bytes, moe_stream_t stream);
 

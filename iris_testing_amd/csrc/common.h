@@ -43,3 +43,5 @@ __device__ __forceinline__ int lane_id() { return threadIdx.x & (WAVE - 1); }
 
 static inline int dtype_size(int dtype) { return dtype == MOE_F32 ? 4 : (dtype == MOE_BF16 ? 2 : 0); }
 static inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
+// whether 16-byte loads and stores may start at p (NULL: there is nothing to load)
+static inline bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }

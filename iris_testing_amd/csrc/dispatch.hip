@@ -206,7 +206,7 @@ __global__ __launch_bounds__(RANK_WAVES * WAVE) void rank_kernel(const int32_t* 
             }
         };
         if (!base) {
-            if (E % 4 == 0) sums(std::integral_constant<int, 4>{});
+            if (E % 4 == 0 && ((uintptr_t)hist & 15) == 0) sums(std::integral_constant<int, 4>{});
             else sums(std::integral_constant<int, 1>{});
         }
     }
@@ -1354,8 +1354,8 @@ extern "C" int moe_combine(const void* ret, int dtype, int W, int M, int H, cons
 static int a2a_check(const char* who, const moe_a2a_source* src, int W, int E_l) {
     MOE_REQUIRE(src && W > 0 && E_l > 0 && W * E_l <= MOE_MAX_EXPERTS, MOE_ERR_INVALID, "%s: bad W=%d E_l=%d", who, W, E_l);
     for (int s = 0; s < W; ++s)
-        MOE_REQUIRE(!src[s].payload || (src[s].counts && src[s].start && src[s].rows >= 0), MOE_ERR_INVALID, "%s: source %d is incomplete",
-                    who, s);
+        MOE_REQUIRE(!src[s].payload || (src[s].counts && src[s].start && src[s].rows >= 0 && aligned16(src[s].payload)), MOE_ERR_INVALID,
+                    "%s: source %d is incomplete, or its payload not at a multiple of 16 bytes", who, s);
     return MOE_OK;
 }
 static A2aSources a2a_slice(const moe_a2a_source* src, int s0, int ns) {

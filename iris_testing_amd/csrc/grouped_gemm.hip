@@ -976,7 +976,7 @@ __global__ __launch_bounds__(256) void prepack_kernel(const T* __restrict__ w, c
     }
 }
 
-// The same for 16-bit weights with K a multiple of 64 and N of 8 (what the GEMMs take): 64 k x 128 n through LDS, 16 bytes per load
+// The same for 16-bit weights with K a multiple of 64 and N of 8 (what the GEMMs take) at multiples of 16 bytes: 64 k x 128 n through LDS, 16 bytes per load
 // and store; or, where out_t is given, the re-tiling of the transposed product (prepack_t below) from the same tile.
 // Columns [N, Npad) of the one and rows [K, Kpad) of the other leave as zeros.
 __global__ __launch_bounds__(256) void prepack16_kernel(const uint16_t* __restrict__ w, const uint16_t* __restrict__ w_up,
@@ -1344,7 +1344,7 @@ __global__ __launch_bounds__(256) void gather_scale_kernel(const float* __restri
 // column order of the fused gate/up product, so the same call serves d tokens = [d gate | d up] @ [w_gate | w_up]^T.
 template <typename T>
 __global__ __launch_bounds__(256) void prepack_t_kernel(const T* __restrict__ w, const T* __restrict__ w_up, T* __restrict__ out,
-                                                         int K, int N, int Kpad) {
+                                                         int K, int N, int Kpad, bool vec) {
     constexpr int SK = ROWB / (int)sizeof(T);
     constexpr int VPS = ROWB / 16;  // 16-byte vectors per 64-byte run
     const int e = blockIdx.y;
@@ -1359,7 +1359,11 @@ __global__ __launch_bounds__(256) void prepack_t_kernel(const T* __restrict__ w,
         const T* src = (pass ? w_up : w) + (size_t)e * K * N;
         uint4 val = z;
         const int kc = gg_packed_col<sizeof(T) == 1>(k);  // the output column of the transposed product this row stands for
-        if (kc < K) val = *reinterpret_cast<const uint4*>(src + (size_t)kc * N + (size_t)ns * SK + v * (16 / (int)sizeof(T)));
+        const T* from = src + (size_t)kc * N + (size_t)ns * SK + v * (16 / (int)sizeof(T));
+        if (kc < K) {
+            if (vec) val = *reinterpret_cast<const uint4*>(from);
+            else __builtin_memcpy(&val, from, 16);  // (w or w_up not at a multiple of 16 bytes)
+        }
         *reinterpret_cast<uint4*>(out + (((size_t)e * nsl * passes + slab) * Kpad + k) * SK + v * (16 / (int)sizeof(T))) = val;
     }
 }
@@ -1404,7 +1408,7 @@ __global__ __launch_bounds__(256) void act_backward_kernel(const T* __restrict__
     }
 }
 
-// The bf16 form: eight consecutive columns per thread, 16 bytes per load and store (F a multiple of 8; the gate and the up column of
+// The bf16 form: eight consecutive columns per thread, 16 bytes per load and store (F a multiple of 8, aligned buffers; the gate and the up column of
 // a SwiGLU unit lie 32 columns apart).  Memory-bound: 10 bytes per hidden value for SwiGLU.
 template <int EPI>
 __global__ __launch_bounds__(256) void act_backward_vec_kernel(const uint4* __restrict__ a1, const uint4* __restrict__ dh, uint4* __restrict__ out,
@@ -1450,11 +1454,13 @@ __global__ __launch_bounds__(256) void act_backward_vec_kernel(const uint4* __re
     }
 }
 
-// fp32 path of the backward pass (plumbing-size workloads): d w[g] = x_g^T @ dy_g, 64 x 64 output tiles, the group's
-// rows in slabs of 32 through LDS; and the plain transposition w [E,K,N] -> [E,N,K] that d tokens = dy @ w^T needs.
-__global__ __launch_bounds__(256) void grouped_dw_f32_kernel(const float* __restrict__ x, const float* __restrict__ dy,
-                                                              const int32_t* __restrict__ cnt, int E_l, int K, int N, int S_rows,
-                                                              float* __restrict__ dw) {
+// fp32 path of the backward pass (plumbing-size workloads), and bf16 operands that 16-byte loads cannot start at: d w[g] = x_g^T @
+// dy_g, 64 x 64 output tiles, the group's rows in slabs of 32 through LDS, element by element; split, ldc and delta as in launch_dw.
+// And the plain transposition w [E,K,N] -> [E,N,K] that d tokens = dy @ w^T needs.
+template <typename T>
+__global__ __launch_bounds__(256) void grouped_dw_kernel(const T* __restrict__ x, const T* __restrict__ dy, const int32_t* __restrict__ cnt,
+                                                          int E_l, int K, int N, int S_rows, T* __restrict__ dw, int ldc, bool split,
+                                                          long long delta) {
     constexpr int SC = 32;
     __shared__ float xs[SC][64 + 1];
     __shared__ float ys[SC][64 + 1];
@@ -1468,8 +1474,8 @@ __global__ __launch_bounds__(256) void grouped_dw_f32_kernel(const float* __rest
         for (int i = threadIdx.x; i < SC * 64; i += 256) {
             const int r = i / 64, cc = i % 64;
             const bool live = s0 + r < c;
-            xs[r][cc] = (live && k0 + cc < K) ? x[(size_t)(row0 + s0 + r) * K + k0 + cc] : 0.f;
-            ys[r][cc] = (live && n0 + cc < N) ? dy[(size_t)(row0 + s0 + r) * N + n0 + cc] : 0.f;
+            xs[r][cc] = (live && k0 + cc < K) ? load_f32<T>(x + (size_t)(row0 + s0 + r) * K + k0 + cc) : 0.f;
+            ys[r][cc] = (live && n0 + cc < N) ? load_f32<T>(dy + (size_t)(row0 + s0 + r) * N + n0 + cc) : 0.f;
         }
         __syncthreads();
 #pragma unroll 4
@@ -1491,7 +1497,9 @@ __global__ __launch_bounds__(256) void grouped_dw_f32_kernel(const float* __rest
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int k = k0 + ty * 4 + i, n = n0 + tx * 4 + j;
-            if (k < K && n < N) dw[((size_t)g * K + k) * N + n] = acc[i][j];
+            if (k >= K || n >= N) continue;
+            T* row = dw + ((size_t)g * K + k) * ldc;
+            store_f32<T>(split ? row + (n / 64) * 32 + n % 32 + (n % 64 >= 32 ? delta : 0) : row + n, acc[i][j]);
         }
 }
 
@@ -1640,7 +1648,7 @@ int launch_prepack(const T* w, const T* w_up, int E_l, int K, int N, T* out, hip
     const int n_eff = N * (w_up ? 2 : 1);
     const int Npad = round_up(n_eff, GG_BN);
     if constexpr (sizeof(T) == 2) {
-        if (K % 64 == 0 && N % 8 == 0) {
+        if (K % 64 == 0 && N % 8 == 0 && aligned16(w) && aligned16(w_up) && aligned16(out)) {
             prepack16_kernel<<<dim3(ceil_div(w_up ? Npad / 2 : Npad, 128), K / 64, E_l * (w_up ? 2 : 1)), 256, 0, s>>>(w, w_up, out, nullptr, K, N, Npad, 0);
             return moe_check_launch("prepack_weights");
         }
@@ -1696,10 +1704,19 @@ extern "C" int moe_grouped_gemm(const void* tokens, const void* weights, const i
                           EPI_NONE, s);
     MOE_REQUIRE(dtype == MOE_BF16, MOE_ERR_INVALID, "grouped_gemm: dtype %d", dtype);
     MOE_REQUIRE(K % 64 == 0 && N % 8 == 0, MOE_ERR_UNSUPPORTED, "grouped_gemm: bf16 needs K %% 64 == 0 and N %% 8 == 0 (K=%d N=%d)", K, N);
-    // (the weights are taken as they are: a re-tiled copy per call would read and write them once more; ws is not used)
+    // (the weights are taken as they are: a re-tiled copy per call would read and write them once more.  Those that the kernels' 16-byte
+    // loads cannot start at are re-tiled into ws.)
     GemmParams p{};
     p.A = (const uint8_t*)tokens; p.B = (const uint8_t*)weights; p.b_mode = GG_B_N; p.C = out; p.cnt = expert_cnt;
     p.E_l = E_l; p.K = K; p.N = N; p.Npad = round_up(N, GG_BN); p.ldc = N; p.S_rows = S_rows;
+    if (!aligned16(weights)) {
+        MOE_REQUIRE(ws && ws_bytes >= moe_prepack_bytes(dtype, E_l, K, N), MOE_ERR_WORKSPACE,
+                    "grouped_gemm: weights that are not 16-byte aligned need a workspace of %zu bytes (%zu given)",
+                    moe_prepack_bytes(dtype, E_l, K, N), ws ? ws_bytes : (size_t)0);
+        const int rc = moe_prepack_weights(weights, nullptr, dtype, E_l, K, N, ws, stream);
+        if (rc) return rc;
+        p.B = (const uint8_t*)ws; p.b_mode = GG_B_PACKED;
+    }
     return launch_gemm<false>(p, EPI_NONE, s);
 }
 
@@ -1757,6 +1774,7 @@ extern "C" int moe_expert_forward(const void* tokens, const void* weights, int l
     MOE_REQUIRE(K % 64 == 0 && N % 8 == 0, MOE_ERR_UNSUPPORTED, "expert_forward: needs K %% 64 == 0 and N %% 8 == 0 (K=%d N=%d)", K, N);
     if (S_rows == 0) return MOE_OK;
     MOE_REQUIRE(tokens && weights && expert_cnt && out, MOE_ERR_INVALID, "expert_forward: null pointer");
+    MOE_REQUIRE(aligned16(weights), MOE_ERR_INVALID, "expert_forward: weights must be 16-byte aligned");
     GemmParams p{};
     p.A = (const uint8_t*)tokens; p.B = (const uint8_t*)weights; p.C = out; p.cnt = expert_cnt; p.zero_tail = 1;
     p.b_mode = layout == MOE_W_TILED ? GG_B_PACKED : layout == MOE_W_RAW ? GG_B_N : GG_B_T;
@@ -1970,7 +1988,7 @@ extern "C" int moe_prepack_weights_transposed(const void* w, const void* w_up, i
                 "prepack_weights_transposed: needs N %% 64 == 0 and K %% 8 == 0 (K=%d N=%d)", K, N);
     const int Kpad = round_up(K, GG_BN);
     prepack_t_kernel<uint16_t><<<dim3(1024, E_l), 256, 0, (hipStream_t)stream>>>((const uint16_t*)w, (const uint16_t*)w_up,
-                                                                               (uint16_t*)packed, K, N, Kpad);
+                                                                               (uint16_t*)packed, K, N, Kpad, aligned16(w) && aligned16(w_up));
     return moe_check_launch("prepack_weights_transposed");
 }
 
@@ -1981,6 +1999,11 @@ extern "C" size_t moe_dw_workspace_bytes(int, int, int, int) { return 0; }
 static int launch_dw(const void* x, const void* dy, const int32_t* expert_cnt, int S_rows, int K, int N, int E_l, int split_F, void* dw,
                      int ldc, long long dw_delta, hipStream_t s) {
     MOE_REQUIRE(N % 8 == 0 && K % 8 == 0, MOE_ERR_UNSUPPORTED, "grouped_gemm_dw: bf16 needs K, N multiples of 8 (K=%d N=%d)", K, N);
+    if (!(aligned16(x) && aligned16(dy) && aligned16(dw) && dw_delta % 8 == 0)) {
+        grouped_dw_kernel<bf16_t><<<dim3(ceil_div(N, 64), ceil_div(K, 64), E_l), 256, 0, s>>>(
+            (const bf16_t*)x, (const bf16_t*)dy, expert_cnt, E_l, K, N, S_rows, (bf16_t*)dw, ldc, split_F > 0, dw_delta);
+        return moe_check_launch("grouped_gemm_dw");
+    }
     GemmParams p{};
     p.A = (const uint8_t*)x; p.B = (const uint8_t*)dy; p.C = dw; p.cnt = expert_cnt;
     p.E_l = E_l; p.K = 64; p.N = N; p.Npad = round_up(N, GG_BN); p.ldc = ldc; p.S_rows = K;
@@ -1998,8 +2021,8 @@ extern "C" int moe_grouped_gemm_dw(const void* x, const void* dy, const int32_t*
     MOE_REQUIRE(split_F == 0 || (dtype == MOE_BF16 && split_F % 32 == 0 && N == 2 * split_F), MOE_ERR_INVALID,
                 "grouped_gemm_dw: split_F=%d needs bf16, split_F %% 32 == 0 and N == 2 split_F", split_F);
     if (dtype == MOE_F32) {
-        grouped_dw_f32_kernel<<<dim3(ceil_div(N, 64), ceil_div(K, 64), E_l), 256, 0, s>>>((const float*)x, (const float*)dy, expert_cnt,
-                                                                                       E_l, K, N, S_rows, (float*)dw);
+        grouped_dw_kernel<float><<<dim3(ceil_div(N, 64), ceil_div(K, 64), E_l), 256, 0, s>>>((const float*)x, (const float*)dy, expert_cnt, E_l, K,
+                                                                                              N, S_rows, (float*)dw, N, false, 0);
         return moe_check_launch("grouped_gemm_dw_f32");
     }
     MOE_REQUIRE(dtype == MOE_BF16, MOE_ERR_INVALID, "grouped_gemm_dw: dtype %d", dtype);
@@ -2023,6 +2046,7 @@ extern "C" int moe_mlp_train_forward(const void* x, const int32_t* expert_cnt, i
     MOE_REQUIRE(layout == MOE_W_TILED || layout == MOE_W_RAW, MOE_ERR_INVALID, "mlp_train_forward: weight layout %d", layout);
     const bool raw = layout == MOE_W_RAW, pair = raw && act == EPI_SWIGLU;
     MOE_REQUIRE(x && expert_cnt && w1 && w2 && hidden && pre_act && out && (!pair || w_up), MOE_ERR_INVALID, "mlp_train_forward: null pointer");
+    MOE_REQUIRE(aligned16(w1) && aligned16(w_up) && aligned16(w2), MOE_ERR_INVALID, "mlp_train_forward: weights must be 16-byte aligned");
     hipStream_t s = (hipStream_t)stream;
     GemmParams p{};
     p.A = (const uint8_t*)x; p.B = (const uint8_t*)w1; p.C = hidden; p.C2 = pre_act; p.cnt = expert_cnt;
@@ -2048,6 +2072,7 @@ extern "C" int moe_mlp_train_backward(const void* x, const void* hidden, const v
     const bool raw = layout == MOE_W_RAW_T;
     MOE_REQUIRE(x && hidden && pre_act && dy && expert_cnt && w1 && w2 && dh && d_pre && dx && dw1 && dw2 && (act != EPI_SWIGLU || (dw_up && (w_up || !raw))),
                 MOE_ERR_INVALID, "mlp_train_backward: null pointer");
+    MOE_REQUIRE(aligned16(w1) && aligned16(w_up) && aligned16(w2), MOE_ERR_INVALID, "mlp_train_backward: weights must be 16-byte aligned");
     hipStream_t s = (hipStream_t)stream;
     const int NP = act == EPI_SWIGLU ? 2 * F : F;
     GemmParams p{};
@@ -2083,7 +2108,7 @@ extern "C" int moe_mlp_act_backward(const void* a1, const void* dh, int dtype, i
     if (rows == 0) return MOE_OK;
     MOE_REQUIRE(a1 && dh && d_a1, MOE_ERR_INVALID, "mlp_act_backward: null pointer");
     hipStream_t s = (hipStream_t)stream;
-    if (dtype == MOE_BF16 && F % 8 == 0) {
+    if (dtype == MOE_BF16 && F % 8 == 0 && aligned16(a1) && aligned16(dh) && aligned16(d_a1)) {
         const int F8 = F / 8, chunk = (int)std::min<long long>(rows, (1ll << 31) / F8);  // rows per launch: 32-bit indices
         for (int r0 = 0; r0 < rows; r0 += chunk) {
             const unsigned total = (unsigned)std::min(chunk, rows - r0) * (unsigned)F8;
@@ -2103,7 +2128,8 @@ extern "C" int moe_mlp_act_backward(const void* a1, const void* dh, int dtype, i
         if (act == EPI_GELU) GG_ACTB(EPI_GELU, float);
         else GG_ACTB(EPI_SILU, float);
     } else if (act == EPI_GELU) GG_ACTB(EPI_GELU, bf16_t);
-    else GG_ACTB(EPI_SILU, bf16_t);  // (SwiGLU has F a multiple of 32)
+    else if (act == EPI_SILU) GG_ACTB(EPI_SILU, bf16_t);
+    else GG_ACTB(EPI_SWIGLU, bf16_t);
 #undef GG_ACTB
     return moe_check_launch("mlp_act_backward");
 }

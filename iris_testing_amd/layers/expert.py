@@ -55,7 +55,7 @@ def _weights_for(w: torch.Tensor, rows: int):
     hit = _PACKED.get(key)
     if hit is None or hit[0]() is not w:
         _drop_packs("N", w)
-        raw = rows < 4096 * w.shape[0]
+        raw = rows < 4096 * w.shape[0] and w.data_ptr() % 16 == 0
         _PACKED[key] = hit = (weakref.ref(w), None if raw else ops.prepack_weights(w))
         if raw:
             return w, L.W_RAW
@@ -75,7 +75,8 @@ def _grouped_gemm_t(do: torch.Tensor, weights: torch.Tensor, cnt: torch.Tensor) 
     if do.dtype == torch.float32:
         return ops.grouped_gemm(do, ops.transpose_weights_f32(weights.contiguous()), cnt)
     S = do.shape[0]
-    if N % 64 or K % 8 or (S >= 4096 * E_l and not L.capturing()):  # (no whole stages of the reduction; or worth a re-tiled copy)
+    # (no whole stages of the reduction; worth a re-tiled copy; or not where the kernel's loads can start)
+    if N % 64 or K % 8 or ((S >= 4096 * E_l or weights.data_ptr() % 16) and not L.capturing()):
         out = torch.zeros((S, K), dtype=do.dtype, device=do.device)
         if S:
             ops.grouped_gemm_mapped(do, None, _packed_weights_t(weights), cnt, S, K, "none", out, part_ws=_part_ws(do.device))
@@ -107,7 +108,7 @@ class Expert(torch.autograd.Function):
         _assert_cuda_int32(local_expert_cnt, "local_expert_cnt")
         assert weights.shape[0] == local_expert_cnt.numel(), "one row count per local expert"
         ctx.save_for_backward(tokens, weights, local_expert_cnt)
-        return _grouped_gemm(tokens.contiguous(), weights.contiguous(), local_expert_cnt.contiguous())
+        return _grouped_gemm(ops.aligned16(tokens.contiguous()), weights.contiguous(), local_expert_cnt.contiguous())
 
     @staticmethod
     def backward(ctx, do):
@@ -118,7 +119,7 @@ class Expert(torch.autograd.Function):
                                                                       reduction runs over the expert's (ragged) rows
         Rows past the counted total get a zero gradient, experts without rows a zero weight gradient."""
         tokens, weights, cnt = ctx.saved_tensors
-        do = do.contiguous()
+        do = ops.aligned16(do.contiguous())
         cnt = cnt.contiguous()
         d_tokens = _grouped_gemm_t(do, weights, cnt)
         d_weights = ops.grouped_gemm_dw(tokens.contiguous(), do, cnt)
@@ -199,7 +200,7 @@ class ExpertWeights:
             return L.W_RAW, w1, w_up, w2
         now = self._versions(self.raw)
         if now != self.raw_versions:
-            if now != self.seen_versions and rows < 4096 * self.e_local and all(t is None or t.is_contiguous() for t in self.raw):
+            if now != self.seen_versions and rows < 4096 * self.e_local and all(t is None or (t.is_contiguous() and t.data_ptr() % 16 == 0) for t in self.raw):
                 self.seen_versions = now
                 return L.W_RAW, self.raw[0], self.raw[2], self.raw[1]
             self.refresh()
@@ -220,7 +221,7 @@ class ExpertMLP(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, tokens, cnt, ew, w1, w2, w_up):
-        tokens = tokens.contiguous()
+        tokens = ops.aligned16(tokens.contiguous())
         S, F = tokens.shape[0], ew.ffn
         a1 = None
         if tokens.dtype == torch.bfloat16 and ew.act != "none" and S:
@@ -244,7 +245,7 @@ class ExpertMLP(torch.autograd.Function):
           d x  = d a1 @ W1^T        d W1 = x^T @ d a1          (SwiGLU: both halves in one launch each)"""
         tokens, hidden, cnt, w1, w2, w_up, a1 = ctx.saved_tensors
         ew = ctx.ew
-        dy = dy.contiguous()
+        dy = ops.aligned16(dy.contiguous())
         S, H, F = tokens.shape[0], ew.hidden, ew.ffn
         swiglu = ew.act == "swiglu"
         if tokens.dtype == torch.float32:
@@ -290,10 +291,10 @@ def expert_mlp(tokens: torch.Tensor, weights: ExpertWeights, local_expert_cnt: t
     _assert_cuda_int32(local_expert_cnt, "local_expert_cnt")
     if weights.dtype == torch.uint8:
         sg, su, sd = weights.scales
-        return ops.grouped_mlp_fp8(tokens.contiguous(), local_expert_cnt, weights.ffn, weights.w1, sg, su, weights.w2, sd)
+        return ops.grouped_mlp_fp8(ops.aligned16(tokens.contiguous()), local_expert_cnt, weights.ffn, weights.w1, sg, su, weights.w2, sd)
     raw = weights.raw
     if torch.is_grad_enabled() and raw is not None and (tokens.requires_grad or any(t is not None and t.requires_grad for t in raw)):
         return ExpertMLP.apply(tokens, local_expert_cnt.contiguous(), weights, raw[0], raw[1], raw[2])
     weights.refresh()
-    return ops.grouped_mlp(tokens.contiguous(), local_expert_cnt, weights.act, weights.w1, weights.w2, weights.w_up,
+    return ops.grouped_mlp(ops.aligned16(tokens.contiguous()), local_expert_cnt, weights.act, weights.w1, weights.w2, weights.w_up,
                            F=weights.ffn)

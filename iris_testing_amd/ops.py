@@ -25,6 +25,12 @@ def _req_i32(t: torch.Tensor, name: str) -> None:
     assert t.dtype == torch.int32, f"{name} must be int32"
 
 
+def aligned16(t: torch.Tensor) -> torch.Tensor:
+    """t if its elements start at a multiple of 16 bytes, where kernels may begin wide loads; else (a view into a flat buffer, say) a
+    copy that does."""
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 def _i32(n, device) -> torch.Tensor:
     return torch.empty(n, dtype=torch.int32, device=device)
 
@@ -310,6 +316,7 @@ def expert_forward(tokens: torch.Tensor, weights: torch.Tensor, layout: int, exp
     assert tokens.dtype == torch.bfloat16
     if layout != L.W_TILED:
         assert weights.dtype == torch.bfloat16 and weights.shape == ((expert_cnt.numel(), K, N) if layout == L.W_RAW else (expert_cnt.numel(), N, K))
+        weights = aligned16(weights)
     out = torch.empty((S, N), dtype=tokens.dtype, device=tokens.device)
     L.check(L.lib().moe_expert_forward(L.ptr(tokens), L.ptr(weights), layout, L.ptr(expert_cnt), S, K, N, expert_cnt.numel(), L.ptr(out),
                                        L.ptr(part_ws), part_ws.numel() * part_ws.element_size(), L.stream_ptr()))
@@ -374,6 +381,8 @@ def grouped_gemm(tokens: torch.Tensor, weights: torch.Tensor, expert_cnt: torch.
     S, K = tokens.shape
     E_l, K2, N = weights.shape
     assert K == K2 and expert_cnt.numel() == E_l
+    if tokens.dtype == torch.bfloat16:
+        weights = aligned16(weights)
     if out is None:
         out = torch.zeros((S, N), dtype=tokens.dtype, device=tokens.device)
     L.check(L.lib().moe_grouped_gemm(L.ptr(tokens), L.ptr(weights), L.ptr(expert_cnt), L.dtype_code(tokens.dtype), S, K, N, E_l, L.ptr(out),
@@ -692,7 +701,7 @@ def mlp_train_forward(x: torch.Tensor, expert_cnt: torch.Tensor, act: str, layou
     S, H = x.shape
     swiglu, E_l = act == "swiglu", expert_cnt.numel()
     if layout == L.W_RAW:
-        _req_raw_mlp(w1, w_up, w2, E_l, H, F, swiglu)
+        w1, w_up, w2 = _raw_mlp(w1, w_up, w2, E_l, H, F, swiglu)
     hidden = torch.empty((S, F), dtype=x.dtype, device=x.device)
     pre = torch.empty((S, 2 * F if swiglu else F), dtype=x.dtype, device=x.device)
     out = torch.empty_like(x)
@@ -702,10 +711,11 @@ def mlp_train_forward(x: torch.Tensor, expert_cnt: torch.Tensor, act: str, layou
     return out, hidden, pre
 
 
-def _req_raw_mlp(w1, w_up, w2, E_l: int, H: int, F: int, swiglu: bool) -> None:
+def _raw_mlp(w1, w_up, w2, E_l: int, H: int, F: int, swiglu: bool):
     for t, shape, name in ((w1, (E_l, H, F), "w1"), (w2, (E_l, F, H), "w2")) + (((w_up, (E_l, H, F), "w_up"),) if swiglu else ()):
         _req_cuda(t, name)
         assert t.dtype == torch.bfloat16 and t.shape == shape, f"{name} must be bf16 {shape}"
+    return aligned16(w1), aligned16(w_up) if swiglu else None, aligned16(w2)
 
 
 def mlp_train_backward(x: torch.Tensor, hidden: torch.Tensor, pre: torch.Tensor, dy: torch.Tensor, expert_cnt: torch.Tensor, act: str,
@@ -720,7 +730,7 @@ def mlp_train_backward(x: torch.Tensor, hidden: torch.Tensor, pre: torch.Tensor,
     F, E_l, dev = hidden.shape[1], expert_cnt.numel(), x.device
     swiglu = act == "swiglu"
     if layout == L.W_RAW_T:
-        _req_raw_mlp(w1, w_up, w2, E_l, H, F, swiglu)
+        w1, w_up, w2 = _raw_mlp(w1, w_up, w2, E_l, H, F, swiglu)
     dh, d_pre, dx = torch.empty_like(hidden), torch.empty_like(pre), torch.empty_like(x)
     dw1, dw2 = torch.empty((E_l, H, F), dtype=x.dtype, device=dev), torch.empty((E_l, F, H), dtype=x.dtype, device=dev)
     dw_up = torch.empty_like(dw1) if swiglu else None
@@ -749,6 +759,8 @@ def grouped_gemm_dw(x: torch.Tensor, dy: torch.Tensor, expert_cnt: torch.Tensor,
     _req_cuda(dy, "dy")
     _req_i32(expert_cnt, "expert_cnt")
     assert x.dtype == dy.dtype and x.shape[0] == dy.shape[0]
+    if x.dtype == torch.bfloat16:  # (the kernel that takes operands at any address is several times slower than the copy)
+        x, dy = aligned16(x), aligned16(dy)
     S, K = x.shape
     N = dy.shape[1]
     E_l = expert_cnt.numel()

@@ -131,6 +131,22 @@ def test_custom_a2a_ragged_world(W, e_local, H, cap):
                        torch.cat([want[e, s, : int(want_pca[e, s])] for e in range(e_local) for s in range(W)]))
 
 
+def test_custom_a2a_payloads_at_odd_addresses():
+    """A payload that is a slice of a flat buffer, at an address where no 16-byte load may start."""
+    W, H = 3, 8
+    counts = torch.tensor([[2], [1], [3]], dtype=torch.int32, device=DEV)
+    starts = torch.tensor([0, 2, 3], dtype=torch.int32, device=DEV)
+    flat = torch.randn(1 + 6 * H, device=DEV).bfloat16()
+    world = SimulatedWorld(W, rank=1)
+    for s in range(W):
+        world.post(s, flat[1:].view(6, H), counts, starts)
+    bufs = utils.alloc_shmem_buffers(None, W, 1, 3, H, torch.bfloat16)
+    with simulated_world(world):
+        out = custom_a2a(*world.sends[1], bufs.pca, bufs.token_buf, bufs.counts_ready, bufs.token_sync, None, W, 3)
+    for s in range(W):
+        assert torch.equal(out[0, s, :1], flat[1:].view(6, H)[2:3]) and bool((out[0, s, 1:] == 0).all())
+
+
 def test_reorder_flat_to_token_buf_and_errors():
     rng = np.random.default_rng(0)
     W, E_l, H, CAP = 4, 3, 32, 9

@@ -273,3 +273,78 @@ def test_activation_gradient_is_the_same_in_either_form(act):
     dh = torch.randn(1 << 20, generator=g, device=DEV).bfloat16()
     wide, narrow = (ops.mlp_act_backward(x.view(-1, F), dh.view(-1, F), act).view(-1) for F in (1024, 4))
     assert torch.equal(wide.view(torch.int16), narrow.view(torch.int16))
+
+
+def _odd(t, off):
+    """The same values in a contiguous view that starts ``off`` elements into its storage."""
+    flat = torch.empty(t.numel() + off, dtype=t.dtype, device=t.device)
+    flat[off:].copy_(t.detach().reshape(-1))
+    return flat[off:].view(t.shape)
+
+
+@pytest.mark.parametrize("off", [1, 4])
+@pytest.mark.parametrize("act", ["gelu", "swiglu"])
+def test_operands_at_odd_addresses(off, act):
+    """Weights, rows and gradients that are slices of a flat buffer, at addresses where no 16-byte load may start: same bits as the
+    aligned ones, through the layers, eager and captured, and through the entry points that take them as they are."""
+    from iris_testing_amd import _lib as L
+    from iris_testing_amd.layers import expert
+    g = torch.Generator(device=DEV).manual_seed(off)
+    cnt, H, F = (70, 0, 45), 128, 192
+    S, E_l, c = sum(cnt), len(cnt), torch.tensor(cnt, dtype=torch.int32, device=DEV)
+    rnd = lambda *s: (torch.randn(*s, generator=g, device=DEV) * s[-2] ** -0.5).bfloat16()  # noqa: E731
+    x, dy, w = rnd(S, H), rnd(S, H), [rnd(E_l, H, F), rnd(E_l, F, H)] + ([rnd(E_l, H, F)] if act == "swiglu" else [])
+
+    def train(x, dy, w, passes):
+        x, w = x.detach().requires_grad_(), [t.detach().requires_grad_() for t in w]
+        ew, out = ExpertWeights.prepare(act, *w), []
+        for _ in range(passes):  # (weights as they are, then re-tiled)
+            with torch.no_grad():
+                if not out:
+                    w[0].mul_(1.0)
+            y = expert_mlp(x, ew, c)
+            out.append([y.detach(), *torch.autograd.grad(y, [x, *w], dy)])
+        with torch.no_grad():
+            out.append([expert_mlp(x, ew, c)])
+        return [t for o in out for t in o]
+
+    def one(x, dy, w):
+        x, w = x.detach().requires_grad_(), w.detach().requires_grad_()
+        y = expert(x, w, c, E_l)
+        return [y.detach(), *torch.autograd.grad(y, [x, w], dy)]
+
+    odd = [_odd(t, off) for t in (x, dy, *w)]
+    assert all(t.is_contiguous() and t.data_ptr() % 16 for t in odd)
+    for a, b in zip(train(x, dy, w, 3), train(odd[0], odd[1], odd[2:], 3)):
+        assert torch.equal(a, b)
+    w2o = odd[3].transpose(1, 2).contiguous()  # [E_l,H,F], aligned; its odd twin below
+    for _ in range(2):
+        for a, b in zip(one(x, _odd(rnd(S, F) * 0 + 1, 0), w2o), one(odd[0], _odd(torch.ones(S, F, device=DEV).bfloat16(), off), _odd(w2o, off))):
+            assert torch.equal(a, b)
+    graph = torch.cuda.CUDAGraph()
+    w2odd, ref = _odd(w2o, off), expert(x, w2o, c, E_l)
+    expert(odd[0], w2odd, c, E_l)
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        got = expert(odd[0], w2odd, c, E_l)
+    for _ in range(2):
+        got.zero_()
+        graph.replay()
+        assert torch.equal(got, ref)
+    # the entry points
+    assert torch.equal(ops.grouped_gemm(x, _odd(w2o, off), c), ops.grouped_gemm(x, w2o, c))
+    out, ws = torch.zeros_like(ref), torch.empty(L.lib().moe_prepack_bytes(L.MOE_BF16, E_l, H, F), dtype=torch.uint8, device=DEV)
+    L.check(L.lib().moe_grouped_gemm(x.data_ptr(), w2odd.data_ptr(), c.data_ptr(), L.MOE_BF16, S, H, F, E_l, out.data_ptr(), ws.data_ptr(),
+                                     ws.numel(), L.stream_ptr()))
+    assert torch.equal(out, ref)
+    pre, dh = rnd(S, 2 * F if act == "swiglu" else F), rnd(S, F)
+    want = ops.mlp_act_backward(pre, dh, act)
+    assert torch.equal(ops.mlp_act_backward(_odd(pre, off), dh, act), want) and torch.equal(ops.mlp_act_backward(pre, _odd(dh, off), act), want)
+    assert torch.equal(ops.prepack_weights_transposed(_odd(w2o, off)), ops.prepack_weights_transposed(w2o))
+    split = F if act == "swiglu" else 0
+    want, got = ops.grouped_gemm_dw(x, pre, c, split_F=split), torch.empty((E_l, H, pre.shape[1]), dtype=torch.bfloat16, device=DEV)
+    ox, op = _odd(x, off), _odd(pre, off)
+    L.check(L.lib().moe_grouped_gemm_dw(ox.data_ptr(), op.data_ptr(), c.data_ptr(), L.MOE_BF16, S, H, pre.shape[1], E_l, split, got.data_ptr(),
+                                        None, 0, L.stream_ptr()))
+    # (fp32 sums in another order, one rounding to bf16 each)
+    assert _rel(got, want.double().cpu()) < 2.0 ** -8 and bool((got[1] == 0).all())

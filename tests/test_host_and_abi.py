@@ -72,6 +72,26 @@ def test_argument_errors_of_the_fused_variants_and_diagnostics_without_a_gpu():
     assert lib.moe_diag_mfma_loop_flops(0, 1, 1) == 2.0 * 4 * 128 * 128 * 32
 
 
+def test_operands_that_wide_loads_cannot_start_at_are_refused_without_a_gpu():
+    """Weights in the reference layout (and payloads) go through 16-byte loads: an entry point that has no other way refuses them before
+    it launches anything; moe_grouped_gemm re-tiles them if it is given room for that."""
+    import ctypes
+    from iris_testing_amd import _lib as L
+    lib = L.lib()
+    for layout in (L.W_TILED, L.W_RAW, L.W_RAW_T):
+        assert lib.moe_expert_forward(16, 18, layout, 16, 4, 64, 64, 1, 16, None, 0, None) == -1 and b"16-byte aligned" in lib.moe_last_error()
+    for w1, w_up, w2 in ((18, 16, 16), (16, 8, 16), (16, 16, 2)):
+        rc = lib.moe_mlp_train_forward(16, 16, 4, 64, 64, 1, L.ACT["swiglu"], L.W_RAW, w1, w_up, w2, 16, 16, 16, None, 0, None)
+        assert rc == -1 and b"16-byte aligned" in lib.moe_last_error()
+        rc = lib.moe_mlp_train_backward(16, 16, 16, 16, 16, 4, 64, 64, 1, L.ACT["swiglu"], L.W_RAW_T, w1, w_up, w2, 16, 16, 16, 16, 16, 16, None, 0, None)
+        assert rc == -1 and b"16-byte aligned" in lib.moe_last_error()
+    assert lib.moe_grouped_gemm(16, 18, 16, L.MOE_BF16, 4, 64, 64, 1, 16, None, 0, None) == -3 and b"workspace" in lib.moe_last_error()
+    block = (L.A2aSource * 2)()
+    block[1].payload, block[1].counts, block[1].start, block[1].rows = 24, 16, 16, 3
+    assert lib.moe_a2a_place(block, L.MOE_BF16, 2, 1, 4, 8, 16, 16, None, 0, None, 0, None) == -1 and b"16 bytes" in lib.moe_last_error()
+    assert ctypes.sizeof(L.A2aSource) == 32
+
+
 def test_static_scratch_count_rejects_oversized_inputs_without_a_gpu():
     """The allocation-free counting entry point checks its size limit before it touches the GPU."""
     from iris_testing_amd import _lib as L
