@@ -43,6 +43,7 @@ enum {
 #define MOE_MAX_EXPERTS 512
 #define MOE_MAX_TOPK 16
 #define MOE_COUNT_BLOCK 64 /* tokens per counting block */
+#define MOE_A2A_SOURCES 64 /* sources of the simulated exchange per launch */
 
 int moe_abi_version(void);
 /* Text of the last error on the calling thread ("" if none). host pointer, valid until the next call. */
@@ -420,7 +421,8 @@ int moe_diag_gemm_trace(unsigned long long* trace, size_t words, int flags);
  *   [rows,H] of rank s (16-byte aligned), its counts for this rank [E_l] and where its block for this rank starts (one int32 in device memory).
  *   token_buf [E_l,W,CAP,H] <- row block start + (rows of the experts before e) + j of source s at [e,s,j], zeros
  *   past its count; pca[e,s] = counts; counts_ready / token_sync (n_ready / n_sync int32 each, nullable) <- W.
- *   If a count exceeds CAP nothing is written.
+ *   If a count exceeds CAP nothing is written -- up to MOE_A2A_SOURCES sources.  More take a launch for each MOE_A2A_SOURCES of them, which
+ *   tests the counts of its own sources only: look at moe_a2a_max_count's result before the call then.
  * moe_a2a_max_count: max_count[0] (of two words, device-writable, e.g. pinned host memory) <- the largest count of moe_a2a_place, 0 if none.
  * moe_shuffle_totals: out[0] <- sum of pca (n entries), out[1] <- smallest of token_sync (n_sync entries; 2^31 - 1 if none);
  *   out device-writable, e.g. pinned host memory.

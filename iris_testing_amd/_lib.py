@@ -19,6 +19,7 @@ ACT = {"none": 0, "gelu": 1, "silu": 2, "swiglu": 3}
 W_TILED, W_RAW, W_RAW_T = 0, 1, 2  # weight layouts: re-tiled, as they are, as they are and transposed
 MOE_MAX_EXPERTS = 512
 MOE_MAX_TOPK = 16
+MOE_A2A_SOURCES = 64  # sources that one launch of moe_a2a_place takes
 
 
 class MoeLibraryError(RuntimeError):

@@ -889,7 +889,7 @@ int check_rows(const char* who, int dtype, int H) {
 
 // The exchange of a simulated world (moe_a2a_place), up to A2A_SRC sources to a launch (their pointers travel as kernel
 // arguments).  A workgroup makes the tables of its sources in LDS, then its waves copy or zero rows (e, s, j) of token_buf.
-constexpr int A2A_SRC = 64;
+constexpr int A2A_SRC = MOE_A2A_SOURCES;
 struct A2aSources {
     moe_a2a_source src[A2A_SRC];
 };

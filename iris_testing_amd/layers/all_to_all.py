@@ -15,6 +15,7 @@ from typing import Dict, Optional, Tuple
 
 import torch
 
+from .. import _lib as L
 from .. import ops
 from ..utils import _assert_cuda_int32
 
@@ -80,8 +81,13 @@ class AllToAllOp(torch.autograd.Function):
         block, most = ops.a2a_sources(sends, rank), ops.pinned_i32(2)
         fits = tuple(token_buf.shape) == want and token_buf.dtype == tokens.dtype
         ops.a2a_max_count(block, e_local, most)
+        # (an exchange of one launch writes nothing if a count exceeds the capacity, and the host learns of that while the rows move;
+        # of several, each launch knows its own sources' counts only, so the host looks at the largest of all first)
+        if world_size > L.MOE_A2A_SOURCES:
+            ops.wait_i32(most)
+            fits = fits and int(most[0]) <= capacity
         try:
-            if fits:  # (writes nothing if a count exceeds the capacity; the host learns of that while the rows move)
+            if fits:
                 pca = local_pca if local_pca.is_contiguous() else torch.empty_like(local_pca, memory_format=torch.contiguous_format)
                 ready, sync = (t if t.dtype == torch.int32 and t.is_cuda and t.is_contiguous() else None for t in (counts_ready, token_sync))
                 ops.a2a_place(block, token_buf, pca, ready, sync)

@@ -114,7 +114,9 @@ def test_custom_a2a_ragged_world(W, e_local, H, cap):
             small = bufs.token_buf[:, :, : cap - 1].contiguous()
             with pytest.raises(ValueError, match="capacity overflow"):
                 custom_a2a(*world.sends[rank], bufs.pca, small, bufs.counts_ready, bufs.token_sync, None, e_local * W, cap - 1)
-            assert W > 64 or (small == 9.0).all()
+            assert (small == 9.0).all()
+            for t in (bufs.pca, bufs.counts_ready, bufs.token_sync):
+                assert not bool(t.any()), "an exchange that raises must not count or signal"
         custom_a2a(*args(cap))
     assert_bits_equal(bufs.pca, want_pca, "pca")
     assert int(bufs.counts_ready) == W and (bufs.token_sync == W).all()
@@ -129,6 +131,35 @@ def test_custom_a2a_ragged_world(W, e_local, H, cap):
     assert torch.equal(bufs.token_buf, want)
     assert torch.equal(shuffle(bufs.token_buf, bufs.pca, bufs.token_sync),
                        torch.cat([want[e, s, : int(want_pca[e, s])] for e in range(e_local) for s in range(W)]))
+
+
+@pytest.mark.parametrize("W,over", [(4, 1), (64, 63), (70, 3), (70, 69), (130, 70)])
+def test_custom_a2a_overflow_of_one_source_writes_nothing(W, over):
+    """One source sends a row more than the capacity, all others fit: with more sources than a launch takes, its launch is one of
+    several, and none of them may write."""
+    cap, H = 2, 8
+    counts = torch.ones((W, W), dtype=torch.int32)
+    counts[over, 0] = cap + 1
+    world, dev = SimulatedWorld(W, rank=0), lambda t: t.to(torch.int32).to(DEV)  # noqa: E731
+    for s in range(W):
+        n = counts[s]
+        world.post(s, torch.full((int(n.sum()), H), float(s), device=DEV), dev(n[:, None]), dev(torch.cumsum(n, 0) - n))
+    bufs = utils.alloc_shmem_buffers(None, W, 1, cap, H, torch.float32)
+    args = lambda c, buf: (*world.sends[0], bufs.pca, buf, bufs.counts_ready, bufs.token_sync, None, W, c)  # noqa: E731
+    bufs.token_buf.fill_(9.0)
+    with simulated_world(world):
+        with pytest.raises(ValueError, match="capacity overflow"):
+            custom_a2a(*args(cap, bufs.token_buf))
+        torch.cuda.synchronize()
+        assert bool((bufs.token_buf == 9.0).all())
+        for t in (bufs.pca, bufs.counts_ready, bufs.token_sync):
+            assert not bool(t.any()), "an exchange that raises must not count or signal"
+        with pytest.raises(ValueError, match="mismatch"):
+            custom_a2a(*args(cap + 1, bufs.token_buf))
+        out = custom_a2a(*args(cap + 1, torch.full((1, W, cap + 1, H), 9.0, device=DEV)))
+    assert torch.equal(bufs.pca[0], dev(counts[:, 0])) and int(bufs.counts_ready) == W
+    want = torch.arange(W, device=DEV)[:, None] * (torch.arange(cap + 1, device=DEV)[None] < counts[:, :1].to(DEV))
+    assert torch.equal(out[0, :, :, 0], want.float()) and torch.equal(out[..., 0], out[..., H - 1])
 
 
 def test_custom_a2a_payloads_at_odd_addresses():
