@@ -37,12 +37,13 @@ def _i32(n, device) -> torch.Tensor:
 
 def _i32_parts(device, *shapes):
     """Contiguous int32 tensors of these shapes in one allocation, each at a multiple of 16 bytes (a view costs half of what an
-    allocation does)."""
+    allocation does).  Each with a version counter of its own (``.data``): one that is changed in place must not make autograd
+    refuse another that it saved."""
     sizes = [math.prod(sh) for sh in shapes]
     buf = _i32(sum(-(-n // 4) * 4 for n in sizes), device)
     out, at = [], 0
     for sh, n in zip(shapes, sizes):
-        out.append(buf.as_strided(sh, (sh[1], 1) if len(sh) == 2 else (1,), at))
+        out.append(buf.as_strided(sh, (sh[1], 1) if len(sh) == 2 else (1,), at).data)
         at += -(-n // 4) * 4
     return out
 

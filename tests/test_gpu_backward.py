@@ -140,6 +140,30 @@ def test_combine_and_pack_gradients_match_float64_autograd():
         assert _rel(xd.grad, want) < tol
 
 
+def test_counts_changed_in_place_after_the_pack_and_the_combine():
+    """A caller may clamp the capacities or take a maximum over ranks in place: what the operators saved for their gradients is not
+    touched by that."""
+    g = torch.Generator(device=DEV).manual_seed(6)
+    T, H, E, k, W = 70, 64, 8, 2, 4
+    idx = torch.rand(T, E, generator=g, device=DEV).topk(k).indices.int()
+    x = torch.randn(T, H, generator=g, device=DEV).requires_grad_()
+    gate = torch.rand(T, k, generator=g, device=DEV).requires_grad_()
+
+    def grads(change):
+        n = ops.count_and_offsets(idx, E, W)
+        M = int(n.caps[0])
+        send = pack_fixed_m(x, idx, n.pos, n.dst_sizes, n.dst_offsets, E // W, M)
+        out = combine(send, idx, n.pos, gate, n.dst_offsets, E // W)
+        if change:
+            n.caps.clamp_(max=1)
+            for t in (n.dst_sizes, n.send_counts, n.expert_offs, n.row_token):
+                t.mul_(2)
+        return torch.autograd.grad(out.square().sum(), [x, gate])
+
+    for a, b in zip(grads(True), grads(False)):
+        assert torch.equal(a, b)
+
+
 def test_expert_mlp_follows_in_place_weight_updates():
     """An optimizer step updates the raw weights in place between two calls: the second forward must multiply with the
     updated weights (the kernels' re-tiled copies are derived again), and its gradients must be those of the updated ones."""

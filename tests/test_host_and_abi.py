@@ -174,6 +174,17 @@ def test_gemm_split_plan_covers_every_tile_and_every_k_stage_once():
     assert lib.moe_gemm_split_plan(10, 0, 8, 4, out) != 0 and lib.moe_gemm_split_plan(10, 8, 7, 4, out) != 0
 
 
+def test_results_in_one_allocation_do_not_share_a_version_counter():
+    """What a caller changes in place must not look changed elsewhere: autograd refuses to use a saved tensor whose counter moved."""
+    from iris_testing_amd import ops
+    parts = ops._i32_parts("cpu", (3, 5), (7,), (1, 1))
+    for i, t in enumerate(parts):
+        t.fill_(i)
+    parts[1].clamp_(max=0)
+    assert [t._version for t in parts] == [1, 2, 1] and [int(t.max()) for t in parts] == [0, 0, 2]
+    assert [tuple(t.shape) for t in parts] == [(3, 5), (7,), (1, 1)] and all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in parts)
+
+
 def test_bench_refuses_more_than_one_gpu():
     """This build has no collectives: bench.py --gpus 2 must say so and exit non-zero without touching a GPU."""
     import subprocess
