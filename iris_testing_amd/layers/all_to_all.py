@@ -71,7 +71,6 @@ class AllToAllOp(torch.autograd.Function):
             # (as posted they are usually what the kernels read; otherwise a converted copy)
             if p.dtype != tokens.dtype or not (p.is_cuda and p.is_contiguous()):
                 p = p.to(tokens.device, tokens.dtype).contiguous()
-            p = ops.aligned16(p)
             if dc.dtype != torch.int32 or not (dc.is_cuda and dc.is_contiguous()):
                 dc = dc.to(*where).contiguous()
             if do.dtype != torch.int32 or not (do.is_cuda and do.is_contiguous()):

@@ -268,12 +268,17 @@ def wait_i32(value: torch.Tensor) -> None:
 
 def a2a_sources(sends, rank: int):
     """The argument block of a2a_max_count / a2a_place for ``rank`` (it only points into the tensors).  sends: per source rank None
-    or (payload [R,H], counts int32 [W,E_l], dst_offsets int32 [W]), contiguous and on the device."""
+    or (payload [R,H], counts int32 [W,E_l], dst_offsets int32 [W]), contiguous and on the device; a payload that the kernels' 16-byte
+    loads cannot start at is copied, and its entry replaced."""
     block = (L.A2aSource * len(sends))()
-    for q, send in zip(block, sends):
+    for i, (q, send) in enumerate(zip(block, sends)):
         if send is not None and send[0].shape[0]:
             payload, counts, starts = send
-            q.payload, q.rows = payload.data_ptr(), payload.shape[0]
+            at = payload.data_ptr()
+            if at % 16:
+                payload = aligned16(payload)
+                sends[i], at = (payload, counts, starts), payload.data_ptr()
+            q.payload, q.rows = at, payload.shape[0]
             q.counts, q.start = counts.data_ptr() + 4 * rank * counts.shape[1], starts.data_ptr() + 4 * rank
     return block
 
