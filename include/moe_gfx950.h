@@ -206,10 +206,14 @@ int moe_grouped_gemm_packed(const void* tokens, const void* packed, const int32_
  * with K=F, N=H; w_up must be NULL; H and F multiples of 64.
  * MOE_F32: w1 [E_l,H,F], w_up [E_l,H,F] (SwiGLU only, else NULL), w2 [E_l,F,H], reference layout.
  * hidden_ws: [S_rows,F] in `dtype`.  fp32 accumulation; hidden activation and output rounded
- * once to `dtype`. */
+ * once to `dtype`.
+ * moe_grouped_mlp_split: with the scratch of moe_grouped_gemm_mapped (nullable; bf16), used by both GEMMs in turn. */
 int moe_grouped_mlp(const void* tokens, const int32_t* expert_cnt, int dtype, int S_rows, int H, int F,
                     int E_l, int act, const void* w1, const void* w_up, const void* w2, void* hidden_ws,
                     void* out, moe_stream_t stream);
+int moe_grouped_mlp_split(const void* tokens, const int32_t* expert_cnt, int dtype, int S_rows, int H, int F,
+                          int E_l, int act, const void* w1, const void* w_up, const void* w2, void* hidden_ws,
+                          void* out, void* part_ws, size_t part_ws_bytes, moe_stream_t stream);
 
 /* fp8 (OCP e4m3) SwiGLU expert.  Weights: e4m3 codes pre-packed like the bf16 ones (1 byte per
  * element) with per-output-channel fp32 scales (sg, su [E_l,F]; sd [E_l,H]).  The input rows (bf16) are quantised per
@@ -276,6 +280,13 @@ int moe_grouped_gemm_mapped_gated(const void* a_base, int a_rows, const int32_t*
                                   int out_rows, const int32_t* c_row_map, void* part_ws, size_t part_ws_bytes,
                                   moe_stream_t stream);
 size_t moe_gemm_part_workspace_bytes(void);
+#define MOE_SPLIT_MIN_K_BYTES 3968 /* shorter rows of activations (1984 bf16, 3968 fp8) are never cut along K: part_ws is not used */
+/* What a grouped GEMM of S_rows rows in E_l groups, K x N, would do with part_ws_bytes of scratch on a device of `cus` compute units, if
+ * its groups came to `tiles` tiles of the height that it chooses: out[0] = that height (32 or 64: small tiles of 128 columns; 128 or 256:
+ * large ones of 256 columns), out[1] = tiles taken by large ones (the rest, a part-filled last round, goes to small tiles of 64 rows),
+ * out[2] = parts that the K range of every small tile is cut into (1: not cut), out[3] = 64-byte stages of K per part.  Host-only: the
+ * functions that the launches and kernels use; no counterpart in the reference. */
+int moe_gemm_launch_plan(int S_rows, int E_l, int K, int N, int act, int fp8, int cus, size_t part_ws_bytes, int tiles, int32_t* out);
 /* How the last round of a launch with total_tiles large tiles, a persistent grid of `grid` workgroups, k_stages 64-byte stages of K
  * (even) and room for max_units part tiles would be cut along K: out[0] = tiles taken whole, out[1] = parts per remaining
  * tile (1: no split), out[2] = K stages per part, out[3] = work units in all.  Host-only arithmetic (the launches hand such

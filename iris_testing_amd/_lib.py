@@ -19,6 +19,7 @@ ACT = {"none": 0, "gelu": 1, "silu": 2, "swiglu": 3}
 W_TILED, W_RAW, W_RAW_T = 0, 1, 2  # weight layouts: re-tiled, as they are, as they are and transposed
 MOE_MAX_EXPERTS = 512
 MOE_MAX_TOPK = 16
+MOE_SPLIT_MIN_K_BYTES = 3968  # shorter rows of a GEMM's activations are never cut along K
 MOE_A2A_SOURCES = 64  # sources that one launch of moe_a2a_place takes
 
 
@@ -82,6 +83,7 @@ _SIGNATURES = {
     "moe_grouped_gemm": (c_int, [P, P, P, c_int, c_int, c_int, c_int, c_int, P, P, c_size_t, P]),
     "moe_grouped_gemm_packed": (c_int, [P, P, P, c_int, c_int, c_int, c_int, c_int, P, P]),
     "moe_grouped_mlp": (c_int, [P, P, c_int, c_int, c_int, c_int, c_int, c_int, P, P, P, P, P, P]),
+    "moe_grouped_mlp_split": (c_int, [P, P, c_int, c_int, c_int, c_int, c_int, c_int, P, P, P, P, P, P, c_size_t, P]),
     "moe_prepack_weights_fp8": (c_int, [P, P, c_int, c_int, c_int, P, P]),
     "moe_quantize_rows_fp8": (c_int, [P, c_int, c_int, P, P, P, P]),
     "moe_grouped_mlp_fp8": (c_int, [P, P, c_int, c_int, c_int, c_int, P, P, P, P, P, P, P, P, P, P, P]),
@@ -102,6 +104,7 @@ _SIGNATURES = {
     "moe_transpose_weights_f32": (c_int, [P, c_int, c_int, c_int, P, P]),
     "moe_mlp_act_backward": (c_int, [P, P, c_int, c_int, c_int, c_int, P, P]),
     "moe_combine_backward": (c_int, [P, P, c_int, c_int, c_int, c_int, P, P, P, P, P, c_int, c_int, c_int, P, P, P]),
+    "moe_gemm_launch_plan": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_size_t, c_int, P]),
     "moe_gemm_split_plan": (c_int, [c_int, c_int, c_int, c_int, P]),
     "moe_zero_padding_rows": (c_int, [P, c_int, c_int, c_int, c_int, P, c_int, P]),
     "moe_recv_prepare": (c_int, [P, c_int, c_int, c_int, c_int, P, P, P, P, P, P, P, c_int, c_int, P]),

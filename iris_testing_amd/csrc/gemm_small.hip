@@ -20,6 +20,7 @@ constexpr int GS_BN = 128;
 constexpr int GS_THREADS = 256;
 constexpr int GS_CTR_BYTES = 16384;  // arrival counters at the start of the workspace: one 64-bit word per tile
 constexpr int GS_MIN_PART_STAGES = 32;  // K stages per part at least: what the hand-over of a split tile costs is worth about as many
+static_assert((2 * GS_MIN_PART_STAGES - 2) * ROWB == MOE_SPLIT_MIN_K_BYTES, "(two parts, the second a pair of stages shorter: what the header tells callers)");
 constexpr int GS_PART_BYTES = 8 << 20;  // room for parts that a launch uses at most: splits beyond that cost more than they give
 constexpr int GS_LDO = GS_BN + 4;    // pitch of the epilogue's fp32 tile in LDS
 
@@ -493,18 +494,25 @@ static unsigned long long gs_nonce() {
     return (base + n.fetch_add(1, std::memory_order_relaxed)) & ((1ull << 56) - 1);
 }
 
+// Part tiles of bm rows that a launch may use: one per compute unit at most, as many as the workspace has room and counters for.
+static int gs_slots(int bm, int cus) { return (int)std::min<long long>(cus, GS_PART_BYTES / (bm * GS_BN * 4)); }
+static int gs_max_units(int bm, const void* part_ws, size_t bytes) {
+    if (!part_ws || bytes <= (size_t)GS_CTR_BYTES) return 0;
+    return (int)std::min<long long>((long long)(bytes - GS_CTR_BYTES) / (bm * GS_BN * 4), GS_CTR_BYTES / 8);
+}
+
+int gs_plan_parts(long long tiles, int bm, int nk, int cus, const void* part_ws, size_t bytes) {
+    const int room = gs_max_units(bm, part_ws, bytes);
+    return room ? gs_parts(tiles, gs_slots(bm, cus), nk, room) : 1;
+}
+
 template <int BM, bool FP8, int EPI, bool BSA, int BMODE>
 static void gs_launch(const GsParams& q0, void* part_ws, size_t part_ws_bytes, int cus, hipStream_t s) {
     GsParams q = q0;
     constexpr int lds = gs_lds_bytes<BM, BSA>();
-    q.slots = (int)std::min<long long>(cus, GS_PART_BYTES / (BM * GS_BN * 4));  // (units worth splitting for)
-    q.g.part_ws = nullptr;
-    q.g.max_units = 0;
-    const long long unit_bytes = (long long)BM * GS_BN * 4;
-    if (part_ws && part_ws_bytes > (size_t)GS_CTR_BYTES) {
-        q.g.max_units = (int)std::min<long long>((long long)(part_ws_bytes - GS_CTR_BYTES) / unit_bytes, GS_CTR_BYTES / 8);
-        q.g.part_ws = (float*)part_ws;
-    }
+    q.slots = gs_slots(BM, cus);
+    q.g.max_units = gs_max_units(BM, part_ws, part_ws_bytes);
+    q.g.part_ws = q.g.max_units ? (float*)part_ws : nullptr;
     const int nt = (q.ncols + GS_BN - 1) / GS_BN;
     const long long ub = ((long long)q.g.S_rows + (long long)std::min(q.g.E_l, q.g.S_rows) * (BM - 1)) / BM * nt;  // most tiles there can be
     auto units = [&](long long tiles) {
@@ -560,12 +568,13 @@ static int gs_dispatch(const GsParams& q, int bm, int epi, void* ws, size_t byte
 //     part-filled last round 0.57 us (256 rows) or 0.33 us (128 rows), or what small tiles take for it where they get it (gg_tail);
 //     6 us for the launch;
 //   small tiles: 0.24 / 0.30 us per 128 bytes of K while every workgroup has a compute unit to itself, then in proportion to
-//     their number (times 1.2, fp8 1.4: the load path is shared); 5 us for the hand-over of a split tile, 7 us for the launch.
+//     their number (times 1.2, fp8 1.4: the load path is shared); 5 us for the hand-over of a split tile, 7 us for the launch.  Tiles are
+//     split only as far as the launch has a workspace for the parts.
 // Over those launches the choice made from these estimates is within 0.5 % (geometric mean) of the better of the two, 1.19 times
 // faster than large tiles alone and in one launch of 470 more than 6 % slower than them: 27.5 -> 9.0 us at 512 rows x 1024 x 1024
 // (2 groups, bf16), 31 -> 21 us at 512 x 2048 x 4096, 49 -> 20 us for an fp8 MLP of 300 rows; the line lies at about one round of
 // large tiles.
-int gs_choose_bm(int S_rows, int E_l, int K, int ncols, bool fp8, int cus) {
+int gs_choose_bm(int S_rows, int E_l, int K, int ncols, bool fp8, int cus, const void* part_ws, size_t part_ws_bytes) {
     const double E = std::min(E_l, S_rows), nk = (double)K * (fp8 ? 1 : 2) / ROWB, share = fp8 ? 1.4 : 1.225;
     const int nt = (ncols + GG_BN - 1) / GG_BN, nts = (ncols + GS_BN - 1) / GS_BN;
     const double t256 = (S_rows / 256.0 + 0.5 * E) * nt, t128 = (S_rows / 128.0 + 0.5 * E) * nt;
@@ -582,7 +591,8 @@ int gs_choose_bm(int S_rows, int E_l, int K, int ncols, bool fp8, int cus) {
     int bm_best = 0;
     for (int bm : {32, 64}) {
         const double units = (S_rows / (double)bm + 0.5 * E) * nts;
-        const double P = units < cus ? std::max(1.0, std::min(std::min(floor(cus / units), floor(nk / GS_MIN_PART_STAGES)), (double)GG_MAX_PARTS)) : 1.0;
+        const int room = std::min(gs_slots(bm, cus), gs_max_units(bm, part_ws, part_ws_bytes));
+        const double P = units < room ? std::max(1.0, std::min(std::min(floor(room / units), floor(nk / GS_MIN_PART_STAGES)), (double)GG_MAX_PARTS)) : 1.0;
         const double x = units * P / cus;
         const double t = 7.4 + (P > 1 ? 5 : 0) + nk / 2 / P * (bm == 32 ? 0.24 : 0.30) * std::max(1.0, x * share) + 1.5 * std::max(1.0, x / 2);
         if (t < best) { best = t; bm_best = bm; }

@@ -305,7 +305,8 @@ __device__ __forceinline__ void gg_zero_tail(const GemmParams& p, int total) {
 
 // gemm_small.hip: the tile height (32 or 64 rows) of the small-tile kernel for a launch, 0 where the large tiles are the
 // better choice; and that launch.
-int gs_choose_bm(int S_rows, int E_l, int K, int ncols, bool fp8, int cus);
+int gs_choose_bm(int S_rows, int E_l, int K, int ncols, bool fp8, int cus, const void* part_ws, size_t part_ws_bytes);
+int gs_plan_parts(long long tiles, int bm, int nk, int cus, const void* part_ws, size_t bytes);  // parts per tile, as its kernel finds them
 size_t gs_workspace_bytes(int cus);  // (what its partial sums take at most)
 int launch_gemm_small(const GemmParams& p, bool fp8, int bm, int epi, void* ws, size_t bytes, int cus, hipStream_t s);
 // The tiles of a launch of large tiles (bm_big rows, grid workgroups) that GemmParams::tail_max left over.

@@ -1535,6 +1535,30 @@ int round_up(int a, int b) { return (a + b - 1) / b * b; }
 // moe_diag_gemm_trace: where the next forward GEMM launches of this process leave time stamps (not thread-safe: a diagnostic)
 struct { unsigned long long* buf; int flags; } g_trace = {nullptr, 0};
 
+// What a launch of S_rows rows in E_l groups takes: the height of its tiles (32, 64: gemm_small.hip; 128, 256) and, for large ones,
+// GemmParams::tail_max.  The one place where that is decided (moe_gemm_launch_plan shows it).
+struct GgChoice {
+    int bm, tail_max;
+};
+static GgChoice gg_choose(int S_rows, int E_l, int K, int nt, int ncols, bool fp8, int grid, const void* part_ws, size_t part_ws_bytes,
+                          bool whole) {
+    // launches that large tiles would leave mostly idle
+    const int bm_small = whole ? 0 : gs_choose_bm(S_rows, E_l, K, ncols, fp8, grid, part_ws, part_ws_bytes);
+    if (bm_small) return {bm_small, 0};
+    // 256-row or 128-row tiles: the host knows only the total row count, so it compares the estimated number
+    // of rounds of the persistent grid (every group adds about half a tile of ragged tail); a 128-row tile
+    // costs about 0.62 of a 256-row one
+    const double t256 = ((double)S_rows / 256 + 0.5 * E_l) * nt, t128 = ((double)S_rows / 128 + 0.5 * E_l) * nt;
+    const int bm = 0.62 * ceil(t128 / grid) < ceil(t256 / grid) ? 128 : 256;
+    if (whole) return {bm, 0};
+    const GgTail t = gg_tail(K * (fp8 ? 1 : 2) / ROWB, bm, fp8, grid);
+    if (E_l == 1) {  // (no group but this one: the host knows what is left over)
+        const int total = ceil_div(S_rows, bm) * nt;
+        return {bm, gg_whole_tiles(total, grid, t.most) == total ? 0 : t.most};
+    }
+    return {bm, t.worth ? t.most : 0};
+}
+
 template <bool FP8>
 int launch_gemm(const GemmParams& p_in, int epi, hipStream_t s, void* part_ws = nullptr, size_t part_ws_bytes = 0) {
     const int grid = num_cus();
@@ -1545,26 +1569,11 @@ int launch_gemm(const GemmParams& p_in, int epi, hipStream_t s, void* part_ws = 
         p.trace_flags = g_trace.flags;
         part_ws = nullptr;
     }
-    // launches that large tiles would leave mostly idle: see gemm_small.hip
-    if (!traced) {
-        const int bm_small = gs_choose_bm(p.S_rows, p.E_l, p.K, epi == EPI_SWIGLU ? 2 * p.N : p.N, FP8, grid);
-        if (bm_small) return launch_gemm_small(p, FP8, bm_small, epi, part_ws, part_ws_bytes, grid, s);
-    }
-    // 256-row or 128-row tiles: the host knows only the total row count, so it compares the estimated number
-    // of rounds of the persistent grid (every group adds about half a tile of ragged tail); a 128-row tile
-    // costs about 0.62 of a 256-row one
-    const int nt = p.Npad / GG_BN;
-    const double t256 = ((double)p.S_rows / 256 + 0.5 * p.E_l) * nt, t128 = ((double)p.S_rows / 128 + 0.5 * p.E_l) * nt;
-    const bool small_m = 0.62 * ceil(t128 / grid) < ceil(t256 / grid);
-    const int bm = small_m ? 128 : 256;
-    const GgTail t = gg_tail(p.K * (FP8 ? 1 : 2) / ROWB, bm, FP8, grid);
-    p.tail_max = traced ? 0 : t.most;
-    if (p.E_l == 1) {  // (no group but this one: the host knows what is left over)
-        const int total = ceil_div(p.S_rows, bm) * nt;
-        if (gg_whole_tiles(total, grid, p.tail_max) == total) p.tail_max = 0;
-    } else if (!t.worth) {
-        p.tail_max = 0;
-    }
+    const GgChoice ch = gg_choose(p.S_rows, p.E_l, p.K, p.Npad / GG_BN, epi == EPI_SWIGLU ? 2 * p.N : p.N, FP8, grid, part_ws, part_ws_bytes, traced);
+    if (ch.bm < 128) return launch_gemm_small(p, FP8, ch.bm, epi, part_ws, part_ws_bytes, grid, s);
+    const int bm = ch.bm;
+    const bool small_m = bm == 128;
+    p.tail_max = ch.tail_max;
     // fp8 without activation is the down projection of the expert MLP: its activation operand is block-scaled
 #define GG_LAUNCH(BMv, NWMv, EPIv, MODEv)                                                                      \
     do {                                                                                                  \
@@ -1744,6 +1753,22 @@ extern "C" int moe_gemm_split_plan(int total_tiles, int grid, int k_stages, int 
     return MOE_OK;
 }
 
+extern "C" int moe_gemm_launch_plan(int S_rows, int E_l, int K, int N, int act, int fp8, int cus, size_t part_ws_bytes, int tiles, int32_t* out) {
+    MOE_REQUIRE(S_rows > 0 && E_l > 0 && K > 0 && N > 0 && act >= EPI_NONE && act <= EPI_SWIGLU && cus > 0 && tiles >= 0 && out, MOE_ERR_INVALID,
+                "gemm_launch_plan: bad arguments");
+    const int ncols = act == EPI_SWIGLU ? 2 * N : N, nk = K * (fp8 ? 1 : 2) / ROWB;
+    const void* ws = part_ws_bytes ? out : nullptr;  // (any address: only whether there is one counts)
+    const GgChoice ch = gg_choose(S_rows, E_l, K, ceil_div(ncols, GG_BN), ncols, fp8 != 0, cus, ws, part_ws_bytes, false);
+    const bool large = ch.bm >= 128;
+    const int whole = large ? gg_whole_tiles(tiles, cus, ch.tail_max) : 0;
+    const int small = large ? (tiles - whole) * (ch.bm / 64) * (GG_BN / 128) : tiles;  // small tiles of the launch, or of its last round
+    out[0] = ch.bm;
+    out[1] = whole;
+    out[2] = gs_plan_parts(small, large ? 64 : ch.bm, nk, cus, ws, part_ws_bytes);
+    out[3] = out[2] > 1 ? gg_part_stages(nk, out[2]) : nk;
+    return MOE_OK;
+}
+
 extern "C" size_t moe_gemm_part_workspace_bytes(void) { return gs_workspace_bytes(num_cus()); }
 
 extern "C" int moe_grouped_gemm_mapped(const void* a_base, int a_rows, const int32_t* a_row_map, const void* packed,
@@ -1823,6 +1848,12 @@ extern "C" int moe_grouped_gemm_act_keep(const void* a_base, int a_rows, const i
 extern "C" int moe_grouped_mlp(const void* tokens, const int32_t* expert_cnt, int dtype, int S_rows, int H, int F, int E_l,
                                int act, const void* w1, const void* w_up, const void* w2, void* hidden_ws, void* out,
                                moe_stream_t stream) {
+    return moe_grouped_mlp_split(tokens, expert_cnt, dtype, S_rows, H, F, E_l, act, w1, w_up, w2, hidden_ws, out, nullptr, 0, stream);
+}
+
+extern "C" int moe_grouped_mlp_split(const void* tokens, const int32_t* expert_cnt, int dtype, int S_rows, int H, int F, int E_l,
+                                     int act, const void* w1, const void* w_up, const void* w2, void* hidden_ws, void* out,
+                                     void* part_ws, size_t part_ws_bytes, moe_stream_t stream) {
     hipStream_t s = (hipStream_t)stream;
     MOE_REQUIRE(S_rows >= 0 && H > 0 && F > 0 && E_l > 0 && E_l <= GG_MAXG, MOE_ERR_INVALID, "grouped_mlp: bad shape");
     MOE_REQUIRE(act == EPI_GELU || act == EPI_SILU || act == EPI_SWIGLU || act == EPI_NONE, MOE_ERR_INVALID,
@@ -1844,12 +1875,12 @@ extern "C" int moe_grouped_mlp(const void* tokens, const int32_t* expert_cnt, in
     p.A = (const uint8_t*)tokens; p.B = (const uint8_t*)w1; p.C = hidden_ws; p.cnt = expert_cnt;
     p.E_l = E_l; p.K = H; p.N = F; p.ldc = F; p.S_rows = S_rows;
     p.Npad = round_up(act == EPI_SWIGLU ? 2 * F : F, GG_BN);
-    int rc = launch_gemm<false>(p, act, s);
+    int rc = launch_gemm<false>(p, act, s, part_ws, part_ws_bytes);
     if (rc) return rc;
     GemmParams q{};
     q.A = (const uint8_t*)hidden_ws; q.B = (const uint8_t*)w2; q.C = out; q.cnt = expert_cnt;
     q.E_l = E_l; q.K = F; q.N = H; q.Npad = round_up(H, GG_BN); q.ldc = H; q.S_rows = S_rows;
-    return launch_gemm<false>(q, EPI_NONE, s);
+    return launch_gemm<false>(q, EPI_NONE, s, part_ws, part_ws_bytes);
 }
 
 static int launch_quantize(const void* x_bf16, const int32_t* src_map, int rows, int cols, uint8_t* q, float* scale,

@@ -79,15 +79,16 @@ def _grouped_gemm_t(do: torch.Tensor, weights: torch.Tensor, cnt: torch.Tensor) 
     if N % 64 or K % 8 or ((S >= 4096 * E_l or weights.data_ptr() % 16) and not L.capturing()):
         out = torch.zeros((S, K), dtype=do.dtype, device=do.device)
         if S:
-            ops.grouped_gemm_mapped(do, None, _packed_weights_t(weights), cnt, S, K, "none", out, part_ws=_part_ws(do.device))
+            ops.grouped_gemm_mapped(do, None, _packed_weights_t(weights), cnt, S, K, "none", out, part_ws=_part_ws(do.device, 2 * N))
         return out
-    return ops.expert_forward(do, weights.contiguous(), L.W_RAW_T, cnt, K, _part_ws(do.device))
+    return ops.expert_forward(do, weights.contiguous(), L.W_RAW_T, cnt, K, _part_ws(do.device, 2 * N))
 
 
-def _part_ws(device) -> torch.Tensor:
-    """Partial-sum workspace for the K split of GEMMs of few tiles, for one call: launches that may overlap must not share it, and under
-    capture it has to belong to the graph.  (8 MB of the caching allocator's, which costs the host what a lookup did.)"""
-    return ops.gemm_part_workspace(device)
+def _part_ws(device, k_bytes: int = L.MOE_SPLIT_MIN_K_BYTES) -> Optional[torch.Tensor]:
+    """Partial-sum workspace for the K split of GEMMs of few tiles, for one call (none where its longest rows, k_bytes of K, are too short to
+    be cut): launches that may overlap must not share it, and under capture it has to belong to the graph.  (8 MB of the
+    caching allocator's, which costs the host what a lookup did.)"""
+    return ops.gemm_part_workspace(device) if k_bytes >= L.MOE_SPLIT_MIN_K_BYTES else None
 
 
 def _grouped_gemm(tokens: torch.Tensor, weights: torch.Tensor, cnt: torch.Tensor) -> torch.Tensor:
@@ -95,7 +96,7 @@ def _grouped_gemm(tokens: torch.Tensor, weights: torch.Tensor, cnt: torch.Tensor
     if tokens.dtype != torch.bfloat16 or weights.shape[1] % 64 or weights.shape[2] % 8:  # (what the MFMA kernel covers)
         return ops.grouped_gemm(tokens, weights, cnt)
     w, layout = _weights_for(weights, tokens.shape[0])
-    return ops.expert_forward(tokens, w, layout, cnt, weights.shape[2], _part_ws(tokens.device))
+    return ops.expert_forward(tokens, w, layout, cnt, weights.shape[2], _part_ws(tokens.device, 2 * weights.shape[1]))
 
 
 class Expert(torch.autograd.Function):
@@ -228,11 +229,12 @@ class ExpertMLP(torch.autograd.Function):
             # the first GEMM also keeps what it feeds to the activation: the backward pass would otherwise run it again
             weights = ew.train_weights(S)
             ctx.raw = weights[0] == L.W_RAW
-            out, hidden, a1 = ops.mlp_train_forward(tokens, cnt, ew.act, *weights, F, part_ws=_part_ws(tokens.device))
+            out, hidden, a1 = ops.mlp_train_forward(tokens, cnt, ew.act, *weights, F, part_ws=_part_ws(tokens.device, 2 * max(ew.hidden, F)))
         else:
             ew.refresh()
             hidden = torch.empty((S, F), dtype=tokens.dtype, device=tokens.device)
-            out = ops.grouped_mlp(tokens, cnt, ew.act, ew.w1, ew.w2, ew.w_up, F=F, hidden_ws=hidden)
+            out = ops.grouped_mlp(tokens, cnt, ew.act, ew.w1, ew.w2, ew.w_up, F=F, hidden_ws=hidden,
+                                  part_ws=_part_ws(tokens.device, 2 * max(ew.hidden, F)))
         ctx.save_for_backward(tokens, hidden, cnt, w1, w2, w_up, a1)
         ctx.ew = ew
         return out
@@ -258,7 +260,7 @@ class ExpertMLP(torch.autograd.Function):
             dx = ops.grouped_gemm(da1, ops.transpose_weights_f32(w1.contiguous()), cnt)
             dw1 = ops.grouped_gemm_dw(tokens, da1, cnt)
             return dx, None, None, dw1, dw2, None
-        ws = _part_ws(tokens.device)
+        ws = _part_ws(tokens.device, 2 * max(H, 2 * F if swiglu else F))
         if a1 is not None:
             if ctx.raw or L.capturing():
                 weights = (L.W_RAW_T, w1.contiguous(), None if w_up is None else w_up.contiguous(), w2.contiguous())
@@ -291,10 +293,11 @@ def expert_mlp(tokens: torch.Tensor, weights: ExpertWeights, local_expert_cnt: t
     _assert_cuda_int32(local_expert_cnt, "local_expert_cnt")
     if weights.dtype == torch.uint8:
         sg, su, sd = weights.scales
-        return ops.grouped_mlp_fp8(ops.aligned16(tokens.contiguous()), local_expert_cnt, weights.ffn, weights.w1, sg, su, weights.w2, sd)
+        return ops.grouped_mlp_fp8(ops.aligned16(tokens.contiguous()), local_expert_cnt, weights.ffn, weights.w1, sg, su, weights.w2, sd,
+                                   part_ws=_part_ws(tokens.device, max(weights.hidden, weights.ffn)))
     raw = weights.raw
     if torch.is_grad_enabled() and raw is not None and (tokens.requires_grad or any(t is not None and t.requires_grad for t in raw)):
         return ExpertMLP.apply(tokens, local_expert_cnt.contiguous(), weights, raw[0], raw[1], raw[2])
     weights.refresh()
     return ops.grouped_mlp(ops.aligned16(tokens.contiguous()), local_expert_cnt, weights.act, weights.w1, weights.w2, weights.w_up,
-                           F=weights.ffn)
+                           F=weights.ffn, part_ws=_part_ws(tokens.device, 2 * max(weights.hidden, weights.ffn)))

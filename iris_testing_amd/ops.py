@@ -312,7 +312,7 @@ def shuffle_totals(pca: torch.Tensor, token_sync: Optional[torch.Tensor], out: t
 
 
 def expert_forward(tokens: torch.Tensor, weights: torch.Tensor, layout: int, expert_cnt: torch.Tensor, N: int,
-                   part_ws: torch.Tensor) -> torch.Tensor:
+                   part_ws: Optional[torch.Tensor]) -> torch.Tensor:
     """out[rows of e] = tokens[rows of e] @ w[e] for bf16 rows; rows past the counted total are zero.  layout W_TILED: weights re-tiled
     (prepack_weights of [E_l,K,N]); W_RAW: [E_l,K,N] as they are; W_RAW_T: [E_l,N,K] as they are, transposed in the product."""
     _req_cuda(tokens, "tokens")
@@ -325,7 +325,7 @@ def expert_forward(tokens: torch.Tensor, weights: torch.Tensor, layout: int, exp
         weights = aligned16(weights)
     out = torch.empty((S, N), dtype=tokens.dtype, device=tokens.device)
     L.check(L.lib().moe_expert_forward(L.ptr(tokens), L.ptr(weights), layout, L.ptr(expert_cnt), S, K, N, expert_cnt.numel(), L.ptr(out),
-                                       L.ptr(part_ws), part_ws.numel() * part_ws.element_size(), L.stream_ptr()))
+                                       L.ptr(part_ws), 0 if part_ws is None else part_ws.numel() * part_ws.element_size(), L.stream_ptr()))
     return out
 
 
@@ -397,8 +397,9 @@ def grouped_gemm(tokens: torch.Tensor, weights: torch.Tensor, expert_cnt: torch.
 
 
 def grouped_mlp(tokens: torch.Tensor, expert_cnt: torch.Tensor, act: str, w1, w2, w_up=None, F: Optional[int] = None,
-                hidden_ws: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """Expert MLP on expert-major rows.
+                hidden_ws: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None,
+                part_ws: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """Expert MLP on expert-major rows.  part_ws (bf16): scratch that lets GEMMs of few tiles be cut along K (gemm_part_workspace).
 
     bf16: ``w1``/``w2`` are prepack_weights() results (``w1`` = prepack(Wg, Wu) for swiglu), ``F`` is
     required.  fp32: ``w1`` [E_l,H,F], ``w_up`` (swiglu only) [E_l,H,F], ``w2`` [E_l,F,H] in the
@@ -416,9 +417,10 @@ def grouped_mlp(tokens: torch.Tensor, expert_cnt: torch.Tensor, act: str, w1, w2
         hidden_ws = torch.empty((S, F), dtype=tokens.dtype, device=dev)
     if out is None:
         out = torch.zeros((S, H), dtype=tokens.dtype, device=dev)
-    L.check(L.lib().moe_grouped_mlp(L.ptr(tokens), L.ptr(expert_cnt), L.dtype_code(tokens.dtype), S, H, F, E_l,
-                                    L.ACT[act], L.ptr(w1), L.ptr(w_up), L.ptr(w2), L.ptr(hidden_ws), L.ptr(out),
-                                    L.stream_ptr()))
+    L.check(L.lib().moe_grouped_mlp_split(L.ptr(tokens), L.ptr(expert_cnt), L.dtype_code(tokens.dtype), S, H, F, E_l,
+                                          L.ACT[act], L.ptr(w1), L.ptr(w_up), L.ptr(w2), L.ptr(hidden_ws), L.ptr(out),
+                                          L.ptr(part_ws), 0 if part_ws is None else part_ws.numel() * part_ws.element_size(),
+                                          L.stream_ptr()))
     return out
 
 

@@ -299,6 +299,20 @@ def test_activation_gradient_is_the_same_in_either_form(act):
     assert torch.equal(wide.view(torch.int16), narrow.view(torch.int16))
 
 
+@pytest.mark.parametrize("act", ["silu", "swiglu"])
+def test_inference_is_the_training_forward(act):
+    """Few tiles and long rows, which are cut along K: the call without gradients takes the same tiles and parts, hence the same bits."""
+    g = torch.Generator(device=DEV).manual_seed(2)
+    S, H, F, c = 64, 2048, 4096, torch.tensor([40, 24], dtype=torch.int32, device=DEV)
+    rnd = lambda *s: (torch.randn(*s, generator=g, device=DEV) * s[-2] ** -0.5).bfloat16()  # noqa: E731
+    w = [rnd(2, H, F).requires_grad_(), rnd(2, F, H).requires_grad_()] + ([rnd(2, H, F).requires_grad_()] if act == "swiglu" else [])
+    x, ew = rnd(S, H), ExpertWeights.prepare(act, *w)
+    y = expert_mlp(x, ew, c)
+    assert y.requires_grad
+    with torch.no_grad():
+        assert torch.equal(expert_mlp(x, ew, c), y)
+
+
 def _odd(t, off):
     """The same values in a contiguous view that starts ``off`` elements into its storage."""
     flat = torch.empty(t.numel() + off, dtype=t.dtype, device=t.device)

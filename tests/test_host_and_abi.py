@@ -174,6 +174,38 @@ def test_gemm_split_plan_covers_every_tile_and_every_k_stage_once():
     assert lib.moe_gemm_split_plan(10, 0, 8, 4, out) != 0 and lib.moe_gemm_split_plan(10, 8, 7, 4, out) != 0
 
 
+def _launch_plan(S, E_l, K, N, act="none", fp8=False, cus=256, ws=None, tiles=0):
+    import ctypes
+    from iris_testing_amd import _lib as L
+    out = (ctypes.c_int32 * 4)()
+    ws = L.lib().moe_gemm_part_workspace_bytes() if ws is None else ws
+    assert L.lib().moe_gemm_launch_plan(S, E_l, K, N, L.ACT[act], fp8, cus, ws, tiles, out) == 0
+    return tuple(out)
+
+
+def test_tile_rule_counts_on_parts_only_where_there_is_room_for_them():
+    """The height of a launch's tiles is chosen with the K split in mind; without a workspace nothing is split, and the choice must be
+    the one of a launch that cannot be split (which short rows are anyway, workspace or not)."""
+    from iris_testing_amd import _lib as L
+    ctr, unit = 16384, 64 * 128 * 4
+    full = L.lib().moe_gemm_part_workspace_bytes()
+    differ = split = 0
+    for S in (1, 24, 64, 300, 443, 1003, 4096, 20000):
+        for E_l in (1, 2, 8, 32):
+            for N, act in ((256, "none"), (2048, "swiglu"), (7168, "none")):
+                for K in (512, 1024, 1920, 1984, 2048, 4096, 14336):
+                    for fp8 in (False, True):
+                        none = _launch_plan(S, E_l, K, N, act, fp8, ws=0, tiles=3)
+                        some = _launch_plan(S, E_l, K, N, act, fp8, tiles=3)
+                        assert none[2] == 1 and none == _launch_plan(S, E_l, K, N, act, fp8, ws=ctr, tiles=3)
+                        if K * (1 if fp8 else 2) < L.MOE_SPLIT_MIN_K_BYTES:
+                            assert some == none
+                        differ, split = differ + (some[0] != none[0]), split + (some[2] > 1)
+                        # room for one part tile is room for none
+                        assert _launch_plan(S, E_l, K, N, act, fp8, ws=ctr + unit // 2, tiles=3)[0] == none[0]
+    assert full == ctr + (8 << 20) and differ > 20 and split > 100
+
+
 def test_results_in_one_allocation_do_not_share_a_version_counter():
     """What a caller changes in place must not look changed elsewhere: autograd refuses to use a saved tensor whose counter moved."""
     from iris_testing_amd import ops
