@@ -287,10 +287,9 @@ size_t moe_gemm_part_workspace_bytes(void);
  * out[2] = parts that the K range of every small tile is cut into (1: not cut), out[3] = 64-byte stages of K per part.  Host-only: the
  * functions that the launches and kernels use; no counterpart in the reference. */
 int moe_gemm_launch_plan(int S_rows, int E_l, int K, int N, int act, int fp8, int cus, size_t part_ws_bytes, int tiles, int32_t* out);
-/* How the last round of a launch with total_tiles large tiles, a persistent grid of `grid` workgroups, k_stages 64-byte stages of K
- * (even) and room for max_units part tiles would be cut along K: out[0] = tiles taken whole, out[1] = parts per remaining
- * tile (1: no split), out[2] = K stages per part, out[3] = work units in all.  Host-only arithmetic (the launches hand such
- * a round to small tiles instead); no counterpart in the reference. */
+/* A plan that launches followed before they handed a part-filled last round to small tiles, kept for its callers: total_tiles large
+ * tiles on a grid of `grid` workgroups, k_stages 64-byte stages of K (even), room for max_units part tiles: out[0] = tiles taken whole,
+ * out[1] = parts per remaining tile (1: no split), out[2] = K stages per part, out[3] = work units in all. */
 int moe_gemm_split_plan(int total_tiles, int grid, int k_stages, int max_units, int32_t* out);
 int moe_zero_padding_rows(void* buf, int dtype, int W, int M, int H, const int32_t* recv_counts, int E_l,
                           moe_stream_t stream);

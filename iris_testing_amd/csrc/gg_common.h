@@ -290,7 +290,6 @@ static inline GgTail gg_tail(int nk, int bm, bool fp8, int grid) {
 }
 
 constexpr int GG_MAX_PARTS = 16;       // parts a tile's K range is cut into, at most
-constexpr int GG_MIN_PART_STAGES = 8;  // K stages per part at least (64 bytes of K each)
 // stages per part when nk stages (even) are cut into P parts: even, and P of them cover nk
 __host__ __device__ inline int gg_part_stages(int nk, int P) { return ((nk + P - 1) / P + 1) & ~1; }
 

@@ -36,8 +36,8 @@ namespace moe_gg {
 #endif
 
 
-// How a last round of large tiles would be walked if its tiles were cut along K: tiles [0, full) whole, tiles [full, total) in P
-// parts each (moe_gemm_split_plan; host arithmetic only).
+// moe_gemm_split_plan: a last round of large tiles cut along K, tiles [0, full) whole, tiles [full, total) in P parts each.
+constexpr int GG_MIN_PART_STAGES = 8;  // K stages per part at least (64 bytes of K each)
 struct GgPlan {
     int total, full, P, nkp, units;
 };
@@ -1743,8 +1743,7 @@ extern "C" int moe_grouped_gemm_packed(const void* tokens, const void* packed, c
     return launch_gemm<false>(p, act, (hipStream_t)stream);
 }
 
-// The tile walk of a launch as the kernels compute it (host side of the same function; no GPU needed):
-// out = {full, P, stages per part, work units}.  For callers that size workspaces and for tests.
+// (an earlier plan for part-filled last rounds, kept for its callers: no launch follows it any more)
 extern "C" int moe_gemm_split_plan(int total_tiles, int grid, int k_stages, int max_units, int32_t* out) {
     MOE_REQUIRE(total_tiles >= 0 && grid > 0 && k_stages >= 2 && k_stages % 2 == 0 && max_units >= 0 && out, MOE_ERR_INVALID,
                 "gemm_split_plan: bad arguments");

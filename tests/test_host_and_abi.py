@@ -139,8 +139,8 @@ def test_configs_and_generators_are_deterministic():
 
 
 def test_gemm_split_plan_covers_every_tile_and_every_k_stage_once():
-    """The walk of a grouped-GEMM launch (whole tiles, then the tiles of an under-filled last round cut along K) is
-    one host/device function; here its host side: every tile appears, the parts of a split tile tile its K range
+    """The plan of moe_gemm_split_plan (whole tiles, then the tiles of an under-filled last round cut along K; kept for its
+    callers, the launches follow moe_gemm_launch_plan): every tile appears, the parts of a split tile tile its K range
     exactly, every part has an even, non-zero number of stages, and the part tiles fit the workspace."""
     import ctypes
     import random
@@ -181,6 +181,49 @@ def _launch_plan(S, E_l, K, N, act="none", fp8=False, cus=256, ws=None, tiles=0)
     ws = L.lib().moe_gemm_part_workspace_bytes() if ws is None else ws
     assert L.lib().moe_gemm_launch_plan(S, E_l, K, N, L.ACT[act], fp8, cus, ws, tiles, out) == 0
     return tuple(out)
+
+
+def test_launch_plan_covers_every_tile_and_every_k_stage_once():
+    """What the launches and kernels decide by (the same functions): a large tile is taken whole or left, with the rest of a part-filled last
+    round, to small ones; the parts of a small tile tile its K range exactly, in pairs of stages, 32 or more of them but for the last,
+    and fit the workspace and the chip."""
+    import random
+    from iris_testing_amd import _lib as L
+    rnd, ctr = random.Random(5), 16384
+    seen = {"tail": 0, "whole": 0, "parts": 0, "cut_short": 0}
+    for _ in range(4000):
+        fp8, cus, act = rnd.random() < 0.4, rnd.choice([256, 256, 304, 64]), rnd.choice(["none", "swiglu"])
+        S, E_l = int(2 ** rnd.uniform(0, 16)), rnd.choice([1, 2, 8, 32])
+        K, N = 128 * int(2 ** rnd.uniform(0, 7)), 64 * int(2 ** rnd.uniform(0, 8))
+        room = rnd.choice([0, 1, 2, 7, 64, 256])
+        ws = ctr + room * 64 * 128 * 4 if room else 0
+        nk = K * (1 if fp8 else 2) // 64
+        bm = _launch_plan(S, E_l, K, N, act, fp8, cus, ws)[0]
+        cols = 2 * N if act == "swiglu" else N
+        tiles = rnd.randint(1, max(1, (-(-S // bm) + E_l) * -(-cols // (256 if bm >= 128 else 128))))
+        again, whole, P, nkp = _launch_plan(S, E_l, K, N, act, fp8, cus, ws, tiles)
+        assert again == bm and bm in (32, 64, 128, 256) and 1 <= P <= 16
+        if bm >= 128:
+            assert whole in (tiles, tiles - tiles % cus)
+            seen["tail" if whole < tiles else "whole"] += 1
+        else:
+            assert whole == 0
+        small = (tiles - whole) * (2 * (bm // 64) if bm >= 128 else 1)
+        if P == 1:
+            assert nkp == nk
+            continue
+        seen["parts"] += 1
+        assert ws and nkp % 2 == 0 and nkp >= 32
+        stages = [min(nkp, nk - i * nkp) for i in range(P)]
+        assert sum(stages) == nk and all(s >= 2 and s % 2 == 0 for s in stages)
+        seen["cut_short"] += stages[-1] < nkp
+        assert small * P <= min(cus, room * (2 if bm == 32 else 1))
+    assert min(seen.values()) > 30, seen
+    # one group: the host knows what is left over, and keeps the second launch for rounds it is quicker in
+    assert _launch_plan(8192, 1, 4096, 14336, "swiglu", tiles=32 * 112)[:2] == (256, 32 * 112)
+    assert _launch_plan(8192 + 256, 1, 4096, 14336, "swiglu", tiles=33 * 112)[1] in (33 * 112, 14 * 256)
+    out = (__import__("ctypes").c_int32 * 4)()
+    assert L.lib().moe_gemm_launch_plan(0, 1, 64, 64, 0, 0, 256, 0, 1, out) == -1 and L.lib().moe_gemm_launch_plan(1, 1, 64, 64, 9, 0, 256, 0, 1, out) == -1
 
 
 def test_tile_rule_counts_on_parts_only_where_there_is_room_for_them():
