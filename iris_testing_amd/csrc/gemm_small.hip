@@ -95,14 +95,13 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
     {
         int rows = 0;
         for (int g0 = 0; g0 < p.E_l; g0 += WAVE) {
-            const int c = g0 + lane < p.E_l ? max(p.cnt[g0 + lane], 0) : 0;
-            const int inc = gs_scan(c), rs = min(rows + inc - c, p.S_rows);
-            const int t = (min(c, p.S_rows - rs) + tm - 1) / tm;
+            const GgRows r = gg_rows(p.cnt, g0 + lane, p.E_l, rows, p.S_rows);
+            const int t = (r.n + tm - 1) / tm;
             int ts = t;
 #pragma unroll
             for (int off = 1; off < WAVE; off <<= 1) ts += __shfl_xor(ts, off, WAVE);
             mt_all += ts;
-            rows = min(rows + __shfl(inc, WAVE - 1, WAVE), p.S_rows);
+            rows = r.end;
         }
         if constexpr (!FP8) gg_zero_tail(p, rows);
     }
@@ -121,10 +120,8 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
     {
         int rows = 0, before = 0;
         for (int g0 = 0; g0 < p.E_l; g0 += WAVE) {
-            const int c = g0 + lane < p.E_l ? max(p.cnt[g0 + lane], 0) : 0;
-            const int inc = gs_scan(c), rs = min(rows + inc - c, p.S_rows);
-            const int cc = min(c, p.S_rows - rs);
-            const int mt = (cc + tm - 1) / tm;
+            const GgRows gr = gg_rows(p.cnt, g0 + lane, p.E_l, rows, p.S_rows);
+            const int mt = (gr.n + tm - 1) / tm;
             const int ti = gs_scan(mt), t0 = (before + ti - mt) * nt_all;
             const unsigned long long hit = __ballot(mt > 0 && whole >= t0 && whole < t0 + mt * nt_all);
             if (hit) {
@@ -138,11 +135,11 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
                     nt = nt * (GG_BN / GS_BN) + tile % (GG_BN / GS_BN);
                 }
                 const int r = m * tm + (TAIL ? tile % subs / (GG_BN / GS_BN) * BM : 0);
-                row0 = __shfl(rs, l, WAVE) + r;
-                rv = min(BM, __shfl(cc, l, WAVE) - r);
+                row0 = __shfl(gr.start, l, WAVE) + r;
+                rv = min(BM, __shfl(gr.n, l, WAVE) - r);
                 break;
             }
-            rows = min(rows + __shfl(inc, WAVE - 1, WAVE), p.S_rows);
+            rows = gr.end;
             before += __shfl(ti, WAVE - 1, WAVE);
         }
     }

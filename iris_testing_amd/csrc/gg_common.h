@@ -256,6 +256,34 @@ __device__ __forceinline__ void gg_wait() {
     __builtin_amdgcn_s_waitcnt((VM & 15) | (7 << 4) | (LGKM << 8) | ((VM >> 4) << 14));
 }
 
+// Where the rows of group g (one per lane, 64 in a row) lie: its first row, how many it has, and (the same in every lane) the end of the last of the
+// 64; `before`: rows of the groups before them.  Counts that claim more rows than the buffers hold are cut at S_rows -- each before they
+// are added up, so that no 64 of them wrap up to GG_SCAN_ROWS rows, and one by one beyond.
+constexpr int GG_SCAN_ROWS = (1 << 25) - 1;
+struct GgRows {
+    int start, n, end;
+};
+__device__ __forceinline__ GgRows gg_rows(const int32_t* cnt, int g, int E_l, int before, int S_rows) {
+    const int left = S_rows - before, c = g < E_l ? min(max(cnt[g], 0), left) : 0;
+    if (S_rows > GG_SCAN_ROWS) {
+        GgRows r = {0, 0, before};
+        for (int l = 0; l < WAVE; ++l) {
+            const int n = min(__shfl(c, l, WAVE), S_rows - r.end);
+            if (lane_id() == l) { r.start = r.end; r.n = n; }
+            r.end += n;
+        }
+        return r;
+    }
+    int inc = c;
+#pragma unroll
+    for (int off = 1; off < WAVE; off <<= 1) {
+        const int o = __shfl_up(inc, off, WAVE);
+        if (lane_id() >= off) inc += o;
+    }
+    const int ex = min(inc - c, left);
+    return {before + ex, min(c, left - ex), before + min(__shfl(inc, WAVE - 1, WAVE), left)};
+}
+
 constexpr int SUP = 16;  // super-tile edge, in large tiles
 // Tile idx of a group of Mt x Nt large tiles in the order they are walked: bands of 16 rows, super-columns of 16 within them.
 __device__ __forceinline__ void gg_patch(int idx, int Mt, int Nt, int& mt, int& nt) {

@@ -1061,21 +1061,22 @@ __global__ __launch_bounds__(256) void grouped_gemm_f32_kernel(const float* __re
         int mt = blockIdx.y, rs = 0;
         if (lane == 0) s_g = -1;
         for (int base = 0; base < E_l; base += WAVE) {
-            const int c = base + lane < E_l ? max(cnt[base + lane], 0) : 0, t = (c + TM - 1) / TM;
-            int tiles = t, rows = c;
+            const GgRows r = gg_rows(cnt, base + lane, E_l, rs, S_rows);
+            const int t = (r.n + TM - 1) / TM;
+            int tiles = t;
 #pragma unroll
             for (int off = 1; off < WAVE; off <<= 1) {
-                const int o = __shfl_up(tiles, off, WAVE), q = __shfl_up(rows, off, WAVE);
-                if (lane >= off) { tiles += o; rows += q; }
+                const int o = __shfl_up(tiles, off, WAVE);
+                if (lane >= off) tiles += o;
             }
             const bool mine = mt < tiles && mt >= tiles - t;
             if (mine) {
-                const int first = (mt - (tiles - t)) * TM, row0 = rs + rows - c + first;
-                s_g = base + lane; s_row0 = row0; s_rv = min(min(TM, c - first), S_rows - row0);
+                const int first = (mt - (tiles - t)) * TM;
+                s_g = base + lane; s_row0 = r.start + first; s_rv = min(TM, r.n - first);
             }
             if (__ballot(mine)) break;
             mt -= __shfl(tiles, WAVE - 1, WAVE);
-            rs += __shfl(rows, WAVE - 1, WAVE);
+            rs = r.end;
         }
     }
     __syncthreads();
@@ -1466,8 +1467,8 @@ __global__ __launch_bounds__(256) void grouped_dw_kernel(const T* __restrict__ x
     __shared__ float ys[SC][64 + 1];
     const int g = blockIdx.z, k0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
     int row0 = 0;
-    for (int e = 0; e < g; ++e) row0 += max(cnt[e], 0);
-    const int c = min(max(cnt[g], 0), max(S_rows - row0, 0));
+    for (int e = 0; e < g; ++e) row0 += min(max(cnt[e], 0), S_rows - row0);  // (counts that claim too much are cut, not added)
+    const int c = min(max(cnt[g], 0), S_rows - row0);
     const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
     float acc[4][4] = {};
     for (int s0 = 0; s0 < c; s0 += SC) {

@@ -97,3 +97,59 @@ def test_small_fp8_mlp_edges(cnt, H, F, workspace):
             assert bool((err <= h.abs().view(c, -1, 32) * 2.0 ** -3.9 + blk * 2.0 ** -14 + 1e-6).all()), f"hidden of group {e}"
             _close(y[r0:r0 + c].cpu(), (hd[r0:r0 + c] @ dec(dq[e])) * ds[e].cpu(), f"down, group {e}")
         r0 += c
+
+
+BIG = 2 ** 31 - 1
+
+
+@pytest.mark.parametrize("S,E_l,K,N", [(40, 3, 64, 128), (64, 130, 4096, 256), (443, 3, 2048, 512), (9900, 3, 3072, 2528)])
+@pytest.mark.parametrize("at", [0, 1])
+def test_counts_that_claim_far_too_much(S, E_l, K, N, at):
+    """Counts whose sum passes 2^31 are cut at the rows there are, one after the other, in every grouped GEMM: small tiles with and without
+    parts, large ones with a last round of small ones, fp32, and the weight gradients."""
+    g = torch.Generator(device=DEV).manual_seed(S)
+    claimed = torch.zeros(E_l, dtype=torch.int32)
+    claimed[0], claimed[at], claimed[at + 1], claimed[-1] = 7, BIG, BIG, BIG
+    cut, left = torch.zeros_like(claimed), S
+    for e in range(E_l):
+        cut[e] = min(int(claimed[e]), left)
+        left -= int(cut[e])
+    claimed, cut = claimed.to(DEV), cut.to(DEV)
+    x = (torch.randn(S, K, generator=g, device=DEV) / 8).bfloat16()
+    w = (torch.randn(E_l, K, N, generator=g, device=DEV) / 8).bfloat16()
+    packed = ops.prepack_weights(w)
+    for ws in (None, ops.gemm_part_workspace(DEV)):
+        got, want = (torch.full((S, N), -7.0, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+        ops.grouped_gemm_mapped(x, None, packed, claimed, S, N, "none", got, part_ws=ws)
+        ops.grouped_gemm_mapped(x, None, packed, cut, S, N, "none", want, part_ws=ws)
+        assert torch.equal(got, want) and not bool((got == -7.0).all(1).any())
+    dy = (torch.randn(S, N, generator=g, device=DEV) / 8).bfloat16()
+    assert torch.equal(ops.grouped_gemm_dw(x, dy, claimed), ops.grouped_gemm_dw(x, dy, cut))
+    if S < 1000:
+        xf, wf, dyf = x.float(), w.float(), dy.float()
+        assert torch.equal(ops.grouped_gemm(xf, wf, claimed), ops.grouped_gemm(xf, wf, cut))
+        assert torch.equal(ops.grouped_gemm_dw(xf, dyf, claimed), ops.grouped_gemm_dw(xf, dyf, cut))
+    if K % 128 == 0 and S < 1000:
+        F = 256
+        q = lambda *s: torch.randint(0, 120, s, generator=g, device=DEV, dtype=torch.uint8)  # noqa: E731  (finite e4m3 codes)
+        one = lambda n: torch.full((E_l, n), 2.0 ** -12, device=DEV)  # noqa: E731
+        up, down = ops.prepack_weights_fp8(q(E_l, K, F), q(E_l, K, F)), ops.prepack_weights_fp8(q(E_l, F, K))
+        for ws in (None, ops.gemm_part_workspace(DEV)):
+            got, want = (ops.grouped_mlp_fp8(x, c, F, up, one(F), one(F), down, one(K), part_ws=ws) for c in (claimed, cut))
+            assert torch.equal(got.view(torch.int16), want.view(torch.int16)) and bool(got.float().abs().amax(1).gt(0).all())
+
+
+def test_counts_that_claim_far_too_much_of_very_many_rows():
+    """Beyond 2^25 rows even cut counts would wrap a sum of 64 of them: the same rule, one count at a time."""
+    S = (1 << 25) + 77
+    g = torch.Generator(device=DEV).manual_seed(1)
+    x, w = torch.randn(S, 4, generator=g, device=DEV), torch.randn(66, 4, 4, generator=g, device=DEV)
+    claimed = torch.full((66,), BIG, dtype=torch.int32, device=DEV)
+    claimed[0], claimed[64] = 1 << 25, 5
+    claimed[1:60] = 1
+    got = ops.grouped_gemm(x, w, claimed)
+    at = 1 << 25
+    assert torch.allclose(got[:at], x[:at] @ w[0], rtol=1e-5, atol=1e-5)  # (four products each)
+    for e in range(1, 60):
+        assert torch.allclose(got[at + e - 1], x[at + e - 1] @ w[e], rtol=1e-5, atol=1e-5)
+    assert torch.allclose(got[at + 59:], x[at + 59:] @ w[60], rtol=1e-5, atol=1e-5)
