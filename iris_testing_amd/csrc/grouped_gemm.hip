@@ -977,11 +977,9 @@ __global__ __launch_bounds__(256) void prepack_kernel(const T* __restrict__ w, c
 }
 
 // The same for 16-bit weights with K a multiple of 64 and N of 8 (what the GEMMs take) at multiples of 16 bytes: 64 k x 128 n through LDS, 16 bytes per load
-// and store; or, where out_t is given, the re-tiling of the transposed product (prepack_t below) from the same tile.
-// Columns [N, Npad) of the one and rows [K, Kpad) of the other leave as zeros.
+// and store.  Columns [N, Npad) leave as zeros.
 __global__ __launch_bounds__(256) void prepack16_kernel(const uint16_t* __restrict__ w, const uint16_t* __restrict__ w_up,
-                                                         uint16_t* __restrict__ out, uint16_t* __restrict__ out_t, int K, int N, int Npad,
-                                                         int Kpad) {
+                                                         uint16_t* __restrict__ out, int K, int N, int Npad) {
     constexpr int TN = 128, LD = TN + 8;
     __shared__ __align__(16) uint16_t tile[64][LD];
     const int passes = w_up ? 2 : 1, e = blockIdx.z / passes, pass = blockIdx.z % passes;
@@ -991,35 +989,23 @@ __global__ __launch_bounds__(256) void prepack16_kernel(const uint16_t* __restri
     for (int i = 0; i < 4; ++i) {
         const int v = threadIdx.x + i * 256, kk = v / 16, nn = (v % 16) * 8;
         uint4 x = make_uint4(0, 0, 0, 0);
-        if (k0 < K && n0 + nn < N) x = *(const uint4*)(s + (size_t)(k0 + kk) * N + n0 + nn);
+        if (n0 + nn < N) x = *(const uint4*)(s + (size_t)(k0 + kk) * N + n0 + nn);
         *(uint4*)&tile[kk][nn] = x;
     }
     __syncthreads();
     constexpr int SK = 32;
-    if (out && k0 < K) {
-        uint16_t* dst = out + (size_t)e * Npad * K;
+    uint16_t* dst = out + (size_t)e * Npad * K;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int v = threadIdx.x + i * 256, k8 = (v % 4) * 8, row = v / 4;  // row: (slab of the tile, row of the packed columns)
-            const int slab = row / TN, rr = row % TN;
-            const int nn = gg_packed_col<false>(rr);  // (consecutive threads write consecutive packed rows)
-            const int pr = w_up ? ((n0 + rr) >> 5) * 64 + pass * 32 + (rr & 31) : n0 + rr;
-            if (pr >= Npad) continue;
-            uint32_t o[4];
+    for (int i = 0; i < 4; ++i) {
+        const int v = threadIdx.x + i * 256, k8 = (v % 4) * 8, row = v / 4;  // row: (slab of the tile, row of the packed columns)
+        const int slab = row / TN, rr = row % TN;
+        const int nn = gg_packed_col<false>(rr);  // (consecutive threads write consecutive packed rows)
+        const int pr = w_up ? ((n0 + rr) >> 5) * 64 + pass * 32 + (rr & 31) : n0 + rr;
+        if (pr >= Npad) continue;
+        uint32_t o[4];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) o[q] = (uint32_t)tile[slab * SK + k8 + 2 * q][nn] | ((uint32_t)tile[slab * SK + k8 + 2 * q + 1][nn] << 16);
-            *(uint4*)(dst + ((size_t)(k0 / SK + slab) * Npad + pr) * SK + k8) = make_uint4(o[0], o[1], o[2], o[3]);
-        }
-    }
-    if (out_t) {
-        uint16_t* dst = out_t + (size_t)e * Kpad * N * passes;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int v = threadIdx.x + i * 256, q = v % 4, kr = (v / 4) % 64, slab = v / 256;
-            if (n0 + slab * SK >= N) continue;
-            const int kc = gg_packed_col<false>(kr);
-            *(uint4*)(dst + ((size_t)((n0 / SK + slab) * passes + pass) * Kpad + k0 + kr) * SK + q * 8) = *(const uint4*)&tile[kc][slab * SK + q * 8];
-        }
+        for (int q = 0; q < 4; ++q) o[q] = (uint32_t)tile[slab * SK + k8 + 2 * q][nn] | ((uint32_t)tile[slab * SK + k8 + 2 * q + 1][nn] << 16);
+        *(uint4*)(dst + ((size_t)(k0 / SK + slab) * Npad + pr) * SK + k8) = make_uint4(o[0], o[1], o[2], o[3]);
     }
 }
 
@@ -1659,7 +1645,7 @@ int launch_prepack(const T* w, const T* w_up, int E_l, int K, int N, T* out, hip
     const int Npad = round_up(n_eff, GG_BN);
     if constexpr (sizeof(T) == 2) {
         if (K % 64 == 0 && N % 8 == 0 && aligned16(w) && aligned16(w_up) && aligned16(out)) {
-            prepack16_kernel<<<dim3(ceil_div(w_up ? Npad / 2 : Npad, 128), K / 64, E_l * (w_up ? 2 : 1)), 256, 0, s>>>(w, w_up, out, nullptr, K, N, Npad, 0);
+            prepack16_kernel<<<dim3(ceil_div(w_up ? Npad / 2 : Npad, 128), K / 64, E_l * (w_up ? 2 : 1)), 256, 0, s>>>(w, w_up, out, K, N, Npad);
             return moe_check_launch("prepack_weights");
         }
     }
