@@ -36,15 +36,20 @@ def _i32(n, device) -> torch.Tensor:
 
 
 def _i32_parts(device, *shapes):
-    """Contiguous int32 tensors of these shapes in one allocation, each at a multiple of 16 bytes (a view costs half of what an
-    allocation does).  Each with a version counter of its own (``.data``): one that is changed in place must not make autograd
-    refuse another that it saved."""
-    sizes = [math.prod(sh) for sh in shapes]
-    buf = _i32(sum(-(-n // 4) * 4 for n in sizes), device)
-    out, at = [], 0
-    for sh, n in zip(shapes, sizes):
-        out.append(buf.as_strided(sh, (sh[1], 1) if len(sh) == 2 else (1,), at).data)
-        at += -(-n // 4) * 4
+    """Contiguous int32 tensors of these shapes in one allocation, each at a multiple of 16 bytes (cheaper than an allocation each), and
+    each with a version counter of its own, which is what unsafe_split is for: one that is changed in place must not make
+    autograd refuse another that it saved."""
+    sizes = []
+    for sh in shapes:
+        n = math.prod(sh)
+        sizes += [n, -n % 4] if n % 4 else [n]
+    parts = iter(_i32(sum(sizes), device).unsafe_split_with_sizes(sizes))
+    out = []
+    for sh in shapes:
+        part = next(parts)
+        if part.shape[0] % 4:
+            next(parts)  # (the gap behind it)
+        out.append(part.view(sh) if len(sh) == 2 else part)
     return out
 
 
