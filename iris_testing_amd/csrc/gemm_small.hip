@@ -95,7 +95,7 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
     {
         int rows = 0;
         for (int g0 = 0; g0 < p.E_l; g0 += WAVE) {
-            const GgRows r = gg_rows(p.cnt, g0 + lane, p.E_l, rows, p.S_rows);
+            const GgRows r = gg_rows<false>(p.cnt, g0 + lane, p.E_l, rows, p.S_rows);
             const int t = (r.n + tm - 1) / tm;
             int ts = t;
 #pragma unroll
@@ -120,7 +120,7 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
     {
         int rows = 0, before = 0;
         for (int g0 = 0; g0 < p.E_l; g0 += WAVE) {
-            const GgRows gr = gg_rows(p.cnt, g0 + lane, p.E_l, rows, p.S_rows);
+            const GgRows gr = gg_rows<false>(p.cnt, g0 + lane, p.E_l, rows, p.S_rows);
             const int mt = (gr.n + tm - 1) / tm;
             const int ti = gs_scan(mt), t0 = (before + ti - mt) * nt_all;
             const unsigned long long hit = __ballot(mt > 0 && whole >= t0 && whole < t0 + mt * nt_all);

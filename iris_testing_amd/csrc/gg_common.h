@@ -258,15 +258,17 @@ __device__ __forceinline__ void gg_wait() {
 
 // Where the rows of group g (one per lane, 64 in a row) lie: its first row, how many it has, and (the same in every lane) the end of the last of the
 // 64; `before`: rows of the groups before them.  Counts that claim more rows than the buffers hold are cut at S_rows -- each before they
-// are added up, so that no 64 of them wrap up to GG_SCAN_ROWS rows, and one by one beyond.
+// are added up, so that no 64 of them wrap up to GG_SCAN_ROWS rows; beyond (ANY_ROWS), one by one.
 constexpr int GG_SCAN_ROWS = (1 << 25) - 1;
 struct GgRows {
     int start, n, end;
 };
+template <bool ANY_ROWS>
 __device__ __forceinline__ GgRows gg_rows(const int32_t* cnt, int g, int E_l, int before, int S_rows) {
     const int left = S_rows - before, c = g < E_l ? min(max(cnt[g], 0), left) : 0;
-    if (S_rows > GG_SCAN_ROWS) {
+    if (ANY_ROWS && S_rows > GG_SCAN_ROWS) {
         GgRows r = {0, 0, before};
+#pragma unroll 1
         for (int l = 0; l < WAVE; ++l) {
             const int n = min(__shfl(c, l, WAVE), S_rows - r.end);
             if (lane_id() == l) { r.start = r.end; r.n = n; }

@@ -1047,7 +1047,7 @@ __global__ __launch_bounds__(256) void grouped_gemm_f32_kernel(const float* __re
         int mt = blockIdx.y, rs = 0;
         if (lane == 0) s_g = -1;
         for (int base = 0; base < E_l; base += WAVE) {
-            const GgRows r = gg_rows(cnt, base + lane, E_l, rs, S_rows);
+            const GgRows r = gg_rows<true>(cnt, base + lane, E_l, rs, S_rows);
             const int t = (r.n + TM - 1) / TM;
             int tiles = t;
 #pragma unroll
@@ -1529,6 +1529,7 @@ struct GgChoice {
 };
 static GgChoice gg_choose(int S_rows, int E_l, int K, int nt, int ncols, bool fp8, int grid, const void* part_ws, size_t part_ws_bytes,
                           bool whole) {
+    whole |= S_rows > GG_SCAN_ROWS;
     // launches that large tiles would leave mostly idle
     const int bm_small = whole ? 0 : gs_choose_bm(S_rows, E_l, K, ncols, fp8, grid, part_ws, part_ws_bytes);
     if (bm_small) return {bm_small, 0};
