@@ -96,7 +96,7 @@ def count_and_offsets(topk_idx: torch.Tensor, num_experts_total: int, world_size
     E, W = num_experts_total, world_size
     dev = topk_idx.device
     e_l = E // W
-    out = Counts(*_i32_parts(dev, (W, e_l), (W, e_l), (W,), (W,), (2,)), *_i32_parts(dev, (T, k), (T * k,)))
+    out = Counts(*_i32_parts(dev, (W, e_l), (W, e_l), (W,), (W,), (2,)), _i32((T, k), dev), _i32((T * k,), dev))
     nbytes = L.lib().moe_count_workspace_bytes(T, k, E)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
     L.check(L.lib().moe_count_and_offsets(L.ptr(topk_idx), T, k, E, W, L.ptr(out.send_counts), L.ptr(out.expert_offs),
