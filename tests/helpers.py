@@ -72,3 +72,18 @@ def oracle_recv(cfg, xs, shards, M, dst):
                      for x, s in zip(xs, shards)])
     rc = np.stack([s["counts"][dst] for s in shards]).astype(np.int32)
     return recv, rc
+
+
+def gemm_parts(cnt, K, N, act="none", fp8=False, workspace=True):
+    """(tile rows, tiles that large ones take, parts per small tile) of a grouped GEMM launch on a GPU with 256 compute units, from the
+    functions the launches themselves use (moe_gemm_launch_plan)."""
+    import ctypes
+    from iris_testing_amd import _lib as L
+    lib, out = L.lib(), (ctypes.c_int32 * 4)()
+    ws, cols = lib.moe_gemm_part_workspace_bytes() if workspace else 0, 2 * N if act == "swiglu" else N
+    args = (int(sum(cnt)), len(cnt), K, N, L.ACT[act], int(fp8), 256, ws)
+    L.check(lib.moe_gemm_launch_plan(*args, 0, out))
+    bm = out[0]
+    tiles = sum(-(-int(c) // bm) for c in cnt) * -(-cols // (256 if bm >= 128 else 128))
+    L.check(lib.moe_gemm_launch_plan(*args, tiles, out))
+    return out[0], out[1], out[2]

@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import O, assert_bits_equal, err_stats, to_np
+from helpers import O, assert_bits_equal, err_stats, gemm_parts, to_np
 
 pytestmark = pytest.mark.gpu
 
@@ -204,13 +204,19 @@ def test_grouped_gemm_counts_that_claim_more_rows_than_there_are():
 
 @pytest.mark.parametrize("E_l,K,N,rows,act", [(2, 512, 1024, (200, 150), "none"), (2, 2048, 4096, (230, 213), "silu"),
                                               (3, 1024, 512, (300, 0, 77), "swiglu"), (1, 4096, 2048, (443,), "gelu"),
-                                              (1, 1024, 4096, (20836,), "swiglu")])
+                                              (1, 1024, 4096, (20836,), "swiglu"),
+                                              # cut into parts: few tiles, and the last round of a launch of large ones
+                                              (2, 4096, 512, (70, 33), "swiglu"), (3, 8192, 256, (40, 0, 5), "none"),
+                                              (1, 4096, 2048, (8448,), "silu")])
 def test_grouped_gemm_k_split_of_the_last_round(E_l, K, N, rows, act):
-    """With a partial-sum workspace the tiles of an under-filled last round are cut along K and summed by a second
-    kernel.  The result must be the oracle's within the bf16 bar, within a bf16 rounding step of the unsplit kernel's
-    (only the fp32 summation order differs), identical from call to call, and rows outside the map stay untouched."""
+    """With a partial-sum workspace the small tiles that a launch, or its last round, comes to are cut along K where rows are long, and the
+    last part of a tile to finish adds the sums.  The result must be the oracle's within the bf16 bar, within a bf16 rounding step of
+    the unsplit kernel's (only the fp32 summation order differs), identical from call to call, and rows outside the map stay
+    untouched."""
     rng = np.random.default_rng(K + N + len(rows))
     cnt = np.array(rows, dtype=np.int32)
+    height, whole, parts = gemm_parts(cnt, K, N, act)
+    assert (parts > 1) == (K >= 4096) and (height >= 128) == (whole > 0) and gemm_parts(cnt, K, N, act, workspace=False)[2] == 1
     S_tot = int(cnt.sum())
     x = _randn(rng, S_tot, K)
     w = _randn(rng, E_l, K, N, scale=K ** -0.5)
@@ -243,14 +249,16 @@ def test_grouped_gemm_k_split_of_the_last_round(E_l, K, N, rows, act):
 
 
 @pytest.mark.parametrize("E_l,K,N,rows,act", [(3, 256, 384, (300, 0, 77), "swiglu"), (2, 512, 256, (70, 333), "gelu"),
-                                              (1, 1024, 2048, (443,), "silu"), (1, 1024, 4096, (20836,), "swiglu")])
+                                              (1, 1024, 2048, (443,), "silu"), (1, 1024, 4096, (20836,), "swiglu"),
+                                              (2, 4096, 512, (60, 40), "swiglu"), (1, 4096, 256, (33,), "gelu")])
 @pytest.mark.parametrize("split", [False, True], ids=["whole_tiles", "k_split"])
 def test_grouped_gemm_act_keep_also_stores_the_pre_activations(E_l, K, N, rows, act, split):
     """The launch that keeps the values before the activation for the backward pass: its output is bit for bit that
     of the ordinary launch, and what it keeps is bit for bit what a launch without activation produces (SwiGLU: in
-    the fused gate / up column order) -- with and without the K split of the last round."""
+    the fused gate / up column order) -- with and without the K split, which long rows get."""
     rng = np.random.default_rng(K + N + len(rows))
     cnt = np.array(rows, dtype=np.int32)
+    assert (gemm_parts(cnt, K, N, act, workspace=split)[2] > 1) == (split and K >= 4096)
     S_tot = int(cnt.sum())
     x = _randn(rng, S_tot, K)
     w = _randn(rng, E_l, K, N, scale=K ** -0.5)
@@ -400,14 +408,16 @@ def test_expert_mlp_fp8(E_l, H, F, S):
     print("fp8 vs unquantised fp32 MLP (max-abs, max-abs / rms, max-rel):", err_stats(out, ref.astype(np.float64)), flush=True)
 
 
-@pytest.mark.parametrize("E_l,H,F,rows", [(2, 2048, 1408, (300, 220)), (1, 512, 1024, (450,)), (3, 1024, 2048, (130, 0, 260))])
+@pytest.mark.parametrize("E_l,H,F,rows", [(2, 2048, 1408, (300, 220)), (1, 512, 1024, (450,)), (3, 1024, 2048, (130, 0, 260)),
+                                           (1, 4096, 512, (90,)), (2, 512, 4096, (130, 60)), (1, 4096, 4096, (40,))])
 def test_expert_mlp_fp8_k_split_of_the_last_round(E_l, H, F, rows):
-    """The fp8 GEMMs with the partial-sum workspace: few tiles on an otherwise idle chip are cut along K and summed by the
-    reduction kernel, which applies the same scales, epilogue and block quantisation.  Each GEMM is held to the oracle on
+    """The fp8 GEMMs with the partial-sum workspace: few tiles with long rows (4096 and more) are cut along K, and the last part of a tile
+    adds the sums and applies the same scales, epilogue and block quantisation.  Each GEMM is held to the oracle on
     its own inputs (as in test_expert_mlp_fp8), the result is reproducible from call to call whatever the workspace held,
     and the hidden activation is that of the unsplit kernels but for values on a rounding boundary."""
     rng = np.random.default_rng(H + F + E_l)
     cnt = np.array(rows, dtype=np.int32)
+    assert [gemm_parts(cnt, *a, fp8=True)[2] > 1 for a in ((H, F, "swiglu"), (F, H, "none"))] == [H >= 4096, F >= 4096]
     S_tot = int(cnt.sum())
     x = _randn(rng, S_tot, H)
     wg, wu = _randn(rng, E_l, H, F, scale=H ** -0.5), _randn(rng, E_l, H, F, scale=H ** -0.5)

@@ -11,7 +11,7 @@ rows and columns of the kernels' outputs:
 * a plain fp32 PyTorch GEMM of the same operands, compared element by element (this is what pins the fused
   SwiGLU epilogue, which is not linear, and the fp8 path).
 
-Both run with and without the partial-sum workspace (the K split of the last round of tiles).
+Both run with and without the partial-sum workspace (the K split of a part-filled last round: mixtral's down projection).
 """
 import numpy as np
 import pytest
@@ -236,16 +236,26 @@ def test_more_rounds_than_the_tile_table_holds():
 def test_bf16_gemm_over_random_shapes_and_maps():
     """Thirty seeded launches over the corners of the kernel's shape space -- K from two ring stages up, column counts that
     are no multiple of a tile or of a 32-column group, empty and one-row groups, more tiles than workgroups or fewer, row
-    maps on either side with dropped (negative) rows, every epilogue, with and without the K-split workspace -- each
-    compared element by element with a plain fp32 product of the same operands."""
-    rng = np.random.default_rng(2024)
+    maps on either side with dropped (negative) rows, every epilogue, with and without the K-split workspace (which rows this
+    short leave alone) -- each compared element by element with a plain fp32 product of the same operands."""
+    _random_bf16_launches(np.random.default_rng(2024), 30, [1, 2, 3, 4, 5, 8, 11, 16])
+
+
+def test_bf16_gemm_over_random_shapes_cut_along_k():
+    """The same with rows long enough to be cut into parts where tiles are few."""
+    assert _random_bf16_launches(np.random.default_rng(3), 14, [32, 37, 64, 112, 130]) >= 5
+
+
+def _random_bf16_launches(rng, n_cases, k_blocks):
+    from helpers import gemm_parts
+    cut = 0
     prev = torch.backends.cuda.matmul.allow_tf32
     torch.backends.cuda.matmul.allow_tf32 = False
     ws = ops.gemm_part_workspace(DEV)
     try:
-        for case in range(30):
+        for case in range(n_cases):
             E_l = int(rng.integers(1, 7))
-            K = 64 * int(rng.choice([1, 2, 3, 4, 5, 8, 11, 16]))
+            K = 64 * int(rng.choice(k_blocks))
             act = str(rng.choice(["none", "none", "swiglu", "gelu", "silu"]))
             N = int(rng.choice([32, 96, 264, 1024, 2080, 4096])) if act != "swiglu" else int(rng.choice([32, 96, 512, 1504, 4096]))
             big = rng.random() < 0.4
@@ -257,6 +267,7 @@ def test_bf16_gemm_over_random_shapes_and_maps():
                 S = 5
             n_in, n_out = S + 37, S + 11
             use_amap, use_cmap, split = rng.random() < 0.6, rng.random() < 0.6, rng.random() < 0.5
+            cut += split and gemm_parts(cnt, K, N, act)[2] > 1
             print(f"case {case}: E_l={E_l} K={K} N={N} act={act} cnt={cnt.tolist()} a_map={use_amap} c_map={use_cmap} split={split}", flush=True)
             base = torch.from_numpy(rng.standard_normal((n_in, K)).astype(np.float32)).to(DEV).bfloat16()
             w = torch.from_numpy((rng.standard_normal((E_l, K, N)) * K ** -0.5).astype(np.float32)).to(DEV).bfloat16()
@@ -292,6 +303,7 @@ def test_bf16_gemm_over_random_shapes_and_maps():
             assert bool((out[torch.from_numpy(~written).to(DEV)] == -7.0).all()), f"case {case}: a row outside the map (or a dropped one) was written"
     finally:
         torch.backends.cuda.matmul.allow_tf32 = prev
+    return cut
 
 
 def test_fp8_mlp_over_random_shapes():

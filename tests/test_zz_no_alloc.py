@@ -63,3 +63,11 @@ def test_static_scratch_rejects_sizes_beyond_the_array():
     assert rc == -3 and b"scratch" in lib.moe_last_error()
     torch.cuda.synchronize()
     assert all(bool((t == -7).all()) for t in outs), "a rejected call must not touch its outputs"
+
+
+def test_static_scratch_count_with_the_scan():
+    """Tokens x experts enough for the scan over the histogram: its part of the scratch behind the histogram, at the largest size too."""
+    _both(14081, 2, 512, 8, 4)
+    T = 64 * 1022  # (just under the array)
+    assert L.lib().moe_count_workspace_bytes(T, 1, 512) <= L.lib().moe_count_static_scratch_bytes() < L.lib().moe_count_workspace_bytes(T + 64, 1, 512)
+    _both(T, 1, 512, 8, 5)
