@@ -174,3 +174,34 @@ def test_graph_keeps_its_workspace_while_other_streams_come_and_go():
         torch.cuda.synchronize()
         assert torch.equal(out, want)
     assert all(bool((c == 7.0).all()) for c in canaries)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["plumbing", "small"])
+def test_captured_step_after_a_weight_update(name):
+    """A captured pipeline step holds the addresses of the prepared weights: after an in-place update and a refresh (which every eager
+    call makes) a replay is the eager step with the new weights, whatever took the memory that was given back meanwhile."""
+    from dataclasses import replace
+
+    from iris_testing_amd import harness
+    from iris_testing_amd.configs import CONFIGS
+    from iris_testing_amd.pipeline import DispatchPipeline
+    cfg = replace(CONFIGS[name], tokens=200)
+    world = harness.build_world(cfg, DEV)
+    ew, _, _ = harness.expert_weights(cfg, 0, DEV)
+    pipe = DispatchPipeline(world, ew)
+    graph = pipe.capture()
+    before = pipe.ret.clone()
+    for _ in range(2):
+        for t in ew.raw:
+            if t is not None:
+                t.mul_(-2.0)
+        ew.refresh()
+        trash = [torch.full((t.numel() // 2,), float("nan"), device=DEV) for t in (ew.w1, ew.w2) for _ in range(3)]
+        pipe.ret.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        got = pipe.ret.clone()
+        pipe.step()
+        assert torch.equal(got, pipe.ret) and not torch.equal(got, before) and bool(torch.isfinite(got.float()).all())
+        del trash
