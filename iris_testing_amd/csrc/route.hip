@@ -730,7 +730,8 @@ extern "C" int moe_route_topk(const void* x, const void* router, const float* bi
     float* part = (float*)ws;
     bool final = false;
     int rc;
-    if (dtype == MOE_BF16 && E % 4 == 0 && ((E > 64 && T > 512) || (E > 16 && E <= 32 && T > 2048))) {
+    // (the kernel for many tokens reads the router in pieces of four experts: they must lie at 8 bytes; the other one reads values)
+    if (dtype == MOE_BF16 && E % 4 == 0 && ((uintptr_t)router & 7) == 0 && ((E > 64 && T > 512) || (E > 16 && E <= 32 && T > 2048))) {
         // (33 to 64 experts: the segment kernel's block of 128 tokens x 64 experts is as good or better.)  All segments in one workgroup
         // where the rows are so short that writing and reading the segments' sums takes as long as the products, and there are
         // tiles enough (at 3072 h and more their number, 2.25 for every place on the chip, say, costs more than the sums do).

@@ -178,6 +178,24 @@ def test_route_one_launch_edge_shapes(T, H, E, k, bias, dtype):
     np.testing.assert_allclose(to_np(gate), o_gate, rtol=1e-5, atol=1e-30)
 
 
+@pytest.mark.parametrize("off", [1, 2, 4])
+@pytest.mark.parametrize("T,H,E", [(2049, 136, 32), (600, 136, 128), (4200, 72, 256)])
+def test_route_of_a_router_at_an_odd_address(T, H, E, off):
+    """A router that is a slice of a flat buffer, at addresses where four experts' values do not lie at 8 bytes (off 4: they do):
+    bit-exact against the oracle, for each form of the kernel for many tokens."""
+    g = torch.Generator().manual_seed(T + E)
+    x, w = torch.randn(T, H, generator=g).bfloat16(), (torch.randn(H, E, generator=g) * H ** -0.5).bfloat16()
+    flat = torch.empty(H * E + off, dtype=torch.bfloat16, device=DEV)
+    router = flat[off:].view(H, E)
+    router.copy_(w)
+    assert router.is_contiguous() and router.data_ptr() % 8 == 2 * off % 8
+    idx, gate, logits = ops.route_topk(x.to(DEV), router, 4)
+    o_idx, o_gate, o_logits = O.route(to_np(x), to_np(w), 4)
+    assert_bits_equal(logits, o_logits, "logits")
+    assert_bits_equal(idx, o_idx, "top-k")
+    np.testing.assert_allclose(to_np(gate), o_gate, rtol=1e-5, atol=1e-30)
+
+
 @pytest.mark.parametrize("E,k,W", [(8, 8, 4), (512, 16, 64), (6, 1, 3), (60, 7, 1), (40, 12, 4), (16, 16, 2)])  # (the last two: more selections than lanes per token)
 def test_route_edge_shapes(E, k, W):
     T, H = 77, 72
