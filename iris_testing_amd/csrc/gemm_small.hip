@@ -149,8 +149,8 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
     const int nkp = P > 1 ? gg_part_stages(nk, P) : nk;
     const int ks0 = part * nkp, nks = min(nkp, nk - ks0);
 
-    // ---- addresses.  LDS tiles as in the large kernel: 64-byte rows, chunk c of row r at position c ^ ((r >> 2) & 3).
-    const int lchunk = (lane & 3) ^ ((lane >> 4) & 3);
+    // ---- addresses.  LDS tiles as in the large kernel: 64-byte rows, chunk c of row r at position c ^ gg_swz(r >> 2).
+    const int lchunk = (lane & 3) ^ gg_swz(lane >> 4);
     const uint32_t ldk = (uint32_t)(p.K * ES);
     const uint8_t* Ab = (p.a_map ? p.A : p.A + (size_t)row0 * ldk) + (size_t)ks0 * ROWB;
     // weights: bytes from one stage to the next, from the start of the tensor to the tile's first stage, and (not re-tiled) of a tensor
@@ -224,7 +224,7 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
     // ---- K loop.  While a pair of stages is multiplied, the fragments of the next one are read into the other set of registers
     // and the pair NST behind it is requested into the slot that has just been read out; one barrier per pair (it says that the
     // next pair's loads of every wave have landed and that nobody reads the slot the new loads go to any more).
-    const int fpos = (FP8 ? (lane >> 5) : (lane >> 4)) ^ ((lane >> 2) & 3);
+    const int fpos = (FP8 ? (lane >> 5) : (lane >> 4)) ^ gg_swz(lane >> 2);
     const uint4* fa = (const uint4*)sA + (wm * S::WR + (lane & (MT - 1))) * CHUNKS;
     const uint4* fb = (const uint4*)sB + (wn * S::WC + (lane & (MT - 1))) * CHUNKS;
     // (BN_RAW) LDS address of the lane's part of the first of the two fragments of each group of 32 columns (see gg_read_tr)

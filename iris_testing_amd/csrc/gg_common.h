@@ -216,6 +216,12 @@ __device__ __forceinline__ gg_i32x4 gg_range(const uint8_t* p, long long left) {
     return d;
 }
 
+// LDS tiles of 64-byte rows: 16-byte chunk c of row r lies at position c ^ gg_swz(r / 4).  A 128-bit read by all lanes takes 16 of them
+// at a time -- 0-3, 12-15, 20-27 (then the others of the first 32; the upper 32 likewise) -- so the fragment reads (lanes 16 q .. 16 q + 15: chunk q of rows 0 .. 15, or fp8 lanes
+// 32 h .. 32 h + 31: chunk h of rows 0 .. 31) meet 64 different banks each time when the swizzle maps 0, 1, 2, 3 to 0, 3, 2, 1.  With
+// 0, 1, 2, 3 itself lanes 0-3 and 20-23 share their banks: 303 bytes a ns and compute unit instead of 530 (reads alone).
+__device__ __forceinline__ int gg_swz(int r4) { return -r4 & 3; }
+
 // Half h of a fragment of a 16 x 16 x 32 MFMA out of an LDS tile whose rows run along k (row pitch PITCH bytes): lanes 16 q ..
 // 16 q + 15 end with k 8 q + 4 h .. + 3 of columns 0 .. 15.  `addr`: the lane's LDS byte address of k = 8 q + (lane % 16) / 4, four
 // columns from column 4 (lane % 4) on; the instruction transposes within the 16 lanes.

@@ -299,11 +299,11 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
     }
 
     // lane-constant pieces of the addressing.  A tile row is 4 chunks of 16 bytes; row r keeps logical
-    // chunk c at position c ^ ((r >> 2) & 3), which makes both the 16-rows-per-instruction DMA writes
+    // chunk c at position c ^ gg_swz(r >> 2), which makes both the 16-rows-per-instruction DMA writes
     // and the 128-bit fragment reads (rows = lane % 32) bank-conflict free.
     const int lrow = wave * WROWS + (lane >> 2);         // row inside a load round
-    const int lchunk = (lane & 3) ^ ((lane >> 4) & 3);   // global 16-byte chunk this lane fetches
-    const int fswz = (lane >> 2) & 3;                    // swizzle of the fragment row (tile rows start at multiples of 16)
+    const int lchunk = (lane & 3) ^ gg_swz(lane >> 4);   // global 16-byte chunk this lane fetches
+    const int fswz = gg_swz(lane >> 2);                  // swizzle of the fragment row (tile rows start at multiples of 16)
     // first 16-byte chunk of the lane's fragment: bf16 lanes 16q .. 16q+15 take chunk q of rows 0 .. 15;
     // fp8 lanes 32h .. 32h+31 take chunks h and h + 2 of rows 0 .. 31 (both operands alike, so every k meets its partner):
     // the MFMA's first four operand registers of the two lane halves are then bytes 0-31 of the stage and the other four
@@ -373,7 +373,7 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
                        (uint32_t)((ln_ & 31) ^ (2 * (((2 * wave_s + (ln_ >> 5)) & 3) + 4 * (r & 1)))) * 16u;      \
     } else {                                                                                                 \
         const int lrow_ = wave_s * WROWS + (ln_ >> 2);                                                         \
-        const uint32_t lcb_ = (uint32_t)(((ln_ & 3) ^ ((ln_ >> 4) & 3)) * 16);                                  \
+        const uint32_t lcb_ = (uint32_t)(((ln_ & 3) ^ gg_swz(ln_ >> 4)) * 16);                                  \
         _Pragma("unroll") for (int r = 0; r < RA; ++r) {                                                      \
             const int lr_ = max(min(r * LR + lrow_, (t).rv - 1), 0);  /* tile row this lane fetches, clamped */ \
             aoff_[r] = (uint32_t)(p.a_map ? max(MAPROW_(t, lr_), 0) : lr_) * ldk + lcb_;                      \
