@@ -198,8 +198,12 @@ enum { EPI_NONE = 0, EPI_GELU = 1, EPI_SILU = 2, EPI_SWIGLU = 3, EPI_GATE = 4 };
 // stage (64 lanes x 16 B = 16 rows x 64 B); wave w of a round moves rows [w*16, w*16+16) of that round.
 // Written as inline assembly to get the scalar-base + 32-bit-lane-offset form (the builtin expands to a
 // 64-bit per-lane address); M0 holds the LDS byte address of the wave's 1 KB destination.
+// A scalar register that a vector instruction wrote (v_readlane, where the compiler brings a spilled base back) may be a load's base
+// only five wait states later, and the compiler does not count them across the start of such a statement: the base goes
+// through a scalar move first (which needs no wait, and is the wait state that a load needs behind a write of M0).
 __device__ __forceinline__ void gg_dma16(const uint8_t* sbase, uint32_t voff, uint32_t lds_addr) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %0" : : "s"(sbase), "v"(voff), "s"(lds_addr) : "memory");
+    const uint8_t* b;
+    asm volatile("s_mov_b32 m0, %3\n\ts_mov_b64 %0, %1\n\tglobal_load_lds_dwordx4 %2, %0" : "=&s"(b) : "s"(sbase), "v"(voff), "s"(lds_addr) : "memory");
 }
 
 // The same through a buffer descriptor: bytes at or past its range arrive as zeros.
@@ -244,7 +248,8 @@ __device__ __forceinline__ int gg_lane_now() {
 
 // One dword per lane, HBM -> LDS: lane l's value lands at lds_addr + 4 l.
 __device__ __forceinline__ void gg_dma4(const uint8_t* sbase, uint32_t voff, uint32_t lds_addr) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %1, %0" : : "s"(sbase), "v"(voff), "s"(lds_addr) : "memory");
+    const uint8_t* b;
+    asm volatile("s_mov_b32 m0, %3\n\ts_mov_b64 %0, %1\n\tglobal_load_lds_dword %2, %0" : "=&s"(b) : "s"(sbase), "v"(voff), "s"(lds_addr) : "memory");
 }
 
 // a wave-uniform value forced into scalar registers
