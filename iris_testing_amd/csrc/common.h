@@ -4,6 +4,7 @@
 #include <stdint.h>
 #include <stdio.h>
 #include <stdarg.h>
+#include <type_traits>
 
 #include "../../include/moe_gfx950.h"
 
@@ -40,6 +41,54 @@ template <>
 __device__ __forceinline__ float load_f32<bf16_t>(const bf16_t* p) { return bf16_to_f32(*p); }
 
 __device__ __forceinline__ int lane_id() { return threadIdx.x & (WAVE - 1); }
+
+// Inclusive scan over the 64 lanes of a wave, all of them active: OP over the lanes up to the own one, from 0 (its neutral element: sums, maxima
+// of values >= 0).  Six DPP moves; a cross-lane read through LDS (__shfl) is a round trip of some 35 ns instead, and the scans
+// stand at the start of kernels that have little else to do.
+template <typename OP>
+__device__ __forceinline__ int wave_scan(int v, OP op) {
+    v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false));  // row_shr 1, 2, 4, 8: within 16 lanes
+    v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false));
+    v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false));
+    v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false));
+    v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false));  // row_bcast 15: the 16 lanes before, to rows 1 and 3
+    return op(v, __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false));  // row_bcast 31: the first half, to the second
+}
+__device__ __forceinline__ int wave_incl_scan(int v) {
+    return wave_scan(v, [](int a, int b) { return a + b; });
+}
+// lane ^ OFF's value, without LDS either (OFF a power of two; all lanes active)
+template <int OFF>
+__device__ __forceinline__ int wave_xor(int x) {
+    static_assert(OFF == 1 || OFF == 2 || OFF == 4 || OFF == 8 || OFF == 16 || OFF == 32, "");
+    if constexpr (OFF == 1) return __builtin_amdgcn_update_dpp(0, x, 0xB1, 0xf, 0xf, false);  // quad_perm [1,0,3,2]
+    else if constexpr (OFF == 2) return __builtin_amdgcn_update_dpp(0, x, 0x4E, 0xf, 0xf, false);  // quad_perm [2,3,0,1]
+    else if constexpr (OFF == 4) {  // row_shl 4 into lanes 0-3 and 8-11 of a row, row_shr 4 into the others
+        return __builtin_amdgcn_update_dpp(__builtin_amdgcn_update_dpp(0, x, 0x104, 0xf, 0x5, false), x, 0x114, 0xf, 0xa, false);
+    } else if constexpr (OFF == 8) return __builtin_amdgcn_update_dpp(0, x, 0x128, 0xf, 0xf, false);  // row_ror 8
+    else {
+        // the swaps leave the pairs' lower (r[0]) and upper (r[1]) rows or halves in both
+        if constexpr (OFF == 16) {
+            const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+            return (int)((lane_id() & 16) ? r[0] : r[1]);
+        } else {
+            const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+            return (int)((lane_id() & 32) ? r[0] : r[1]);
+        }
+    }
+}
+// f(integral constants 32, 16, 8, 4, 2, 1)
+template <typename F>
+__device__ __forceinline__ void wave_butterfly(F&& f) {
+    f(std::integral_constant<int, 32>{}); f(std::integral_constant<int, 16>{}); f(std::integral_constant<int, 8>{});
+    f(std::integral_constant<int, 4>{}); f(std::integral_constant<int, 2>{}); f(std::integral_constant<int, 1>{});
+}
+// the same value in every lane: lane l's (l the same in all), the sum of all, the largest (of values >= 0)
+__device__ __forceinline__ int wave_lane(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
+__device__ __forceinline__ int wave_sum(int v) { return wave_lane(wave_incl_scan(v), WAVE - 1); }
+__device__ __forceinline__ int wave_max0(int v) {
+    return wave_lane(wave_scan(v, [](int a, int b) { return max(a, b); }), WAVE - 1);
+}
 
 static inline int dtype_size(int dtype) { return dtype == MOE_F32 ? 4 : (dtype == MOE_BF16 ? 2 : 0); }
 static inline int ceil_div(int a, int b) { return (a + b - 1) / b; }

@@ -40,15 +40,6 @@ __global__ __launch_bounds__(256) void block_hist_kernel(const int32_t* __restri
         for (int e = lane_id(); e < E; e += WAVE) hist[(size_t)b * E + e] = my[e];
 }
 
-__device__ __forceinline__ int wave_incl_scan(int v) {
-#pragma unroll
-    for (int off = 1; off < WAVE; off <<= 1) {
-        const int o = __shfl_up(v, off, WAVE);
-        if (lane_id() >= off) v += o;
-    }
-    return v;
-}
-
 // ---- 2. expert prefix -> all count/offset outputs (one wave) ---------------------------------------
 // A single wave runs it, whatever else its block holds; the lanes hand over through es in LDS.  es[e] = rows of the experts
 // before e; with `write` the results also go to memory.
@@ -66,8 +57,7 @@ __device__ __forceinline__ void offsets_body(const int32_t* counts /*LDS*/, int 
     for (int e = lo; e < hi; ++e) { es[e] = run; run += counts[e]; }
     if (lane == WAVE - 1) es[E] = incl;
     if (!write) return;
-#pragma unroll
-    for (int off = WAVE / 2; off >= 1; off >>= 1) cmax = max(cmax, __shfl_xor(cmax, off, WAVE));
+    cmax = wave_max0(cmax);
     // the lanes' LDS writes above are read by other lanes of the same wave below
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -84,8 +74,7 @@ __device__ __forceinline__ void offsets_body(const int32_t* counts /*LDS*/, int 
         dst_offsets[d] = es[d * E_l];
         mmax = max(mmax, sz);
     }
-#pragma unroll
-    for (int off = WAVE / 2; off >= 1; off >>= 1) mmax = max(mmax, __shfl_xor(mmax, off, WAVE));
+    mmax = wave_max0(mmax);
     if (lane == 0) { caps[0] = max(mmax, 1); caps[1] = max(cmax, 1); }
 }
 
@@ -727,8 +716,7 @@ __global__ __launch_bounds__(WPB * WAVE) void combine_backward_kernel(const uint
 #pragma unroll
         for (int j = 0; j < KMAX; ++j)
             if (j < k) {
-#pragma unroll
-                for (int off = WAVE / 2; off >= 1; off >>= 1) dot[j] = __fadd_rn(dot[j], __shfl_xor(dot[j], off, WAVE));
+                wave_butterfly([&](auto off) { dot[j] = __fadd_rn(dot[j], __int_as_float(wave_xor<decltype(off)::value>(__float_as_int(dot[j])))); });
                 if (lane == 0) {
                     if constexpr (WPT == 1) dgate[(size_t)r * k + j] = dot[j];
                     else part[wave][j] = dot[j];
@@ -777,9 +765,7 @@ int gather_rows(const void* src, void* dst, const RowSource& a, int n_rows, int 
 __device__ __forceinline__ int slot_size(const int32_t* __restrict__ rc, int s, int E_l, int lane) {
     int size = 0;
     for (int e = lane; e < E_l; e += WAVE) size += rc[s * E_l + e];
-#pragma unroll
-    for (int off = WAVE / 2; off >= 1; off >>= 1) size += __shfl_xor(size, off, WAVE);
-    return size;
+    return wave_sum(size);
 }
 __device__ __forceinline__ void zero_padding_rows(u32x4* __restrict__ buf, const int32_t* __restrict__ rc, int W, int E_l, int M,
                                                   int row_vecs, int block) {

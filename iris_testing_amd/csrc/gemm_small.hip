@@ -57,15 +57,6 @@ __host__ __device__ inline int gs_parts(long long tiles, int slots, int nk, int 
     return P < 1 ? 1 : P;
 }
 
-__device__ __forceinline__ int gs_scan(int v) {
-#pragma unroll
-    for (int off = 1; off < WAVE; off <<= 1) {
-        const int o = __shfl_up(v, off, WAVE);
-        if (lane_id() >= off) v += o;
-    }
-    return v;
-}
-
 template <int BM, bool FP8, int EPI, bool BSA, int BMODE, bool TAIL>
 __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParams q) {
     constexpr bool BT = BMODE == GG_B_T, BN_PAIR = BMODE == GG_B_NP, BN_RAW = BMODE == GG_B_N || BN_PAIR;  // (see GG_B_*)
@@ -92,16 +83,16 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
     const int nt_all = TAIL ? p.Npad / GG_BN : (q.ncols + GS_BN - 1) / GS_BN;  // (TAIL: large tiles)
     const int tm = TAIL ? q.big_bm : BM, subs = TAIL ? tm / BM * (GG_BN / GS_BN) : 1;
     int mt_all = 0;
+    GgRows gr;
+    int mt, ti;  // row tiles of the lane's group, and of the groups up to it
     {
         int rows = 0;
         for (int g0 = 0; g0 < p.E_l; g0 += WAVE) {
-            const GgRows r = gg_rows<false>(p.cnt, g0 + lane, p.E_l, rows, p.S_rows);
-            const int t = (r.n + tm - 1) / tm;
-            int ts = t;
-#pragma unroll
-            for (int off = 1; off < WAVE; off <<= 1) ts += __shfl_xor(ts, off, WAVE);
-            mt_all += ts;
-            rows = r.end;
+            gr = gg_rows<false>(p.cnt, g0 + lane, p.E_l, rows, p.S_rows);
+            mt = (gr.n + tm - 1) / tm;
+            ti = wave_incl_scan(mt);
+            mt_all += wave_lane(ti, WAVE - 1);
+            rows = gr.end;
         }
         if constexpr (!FP8) gg_zero_tail(p, rows);
     }
@@ -120,13 +111,16 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
     {
         int rows = 0, before = 0;
         for (int g0 = 0; g0 < p.E_l; g0 += WAVE) {
-            const GgRows gr = gg_rows<false>(p.cnt, g0 + lane, p.E_l, rows, p.S_rows);
-            const int mt = (gr.n + tm - 1) / tm;
-            const int ti = gs_scan(mt), t0 = (before + ti - mt) * nt_all;
+            if (p.E_l > WAVE) {  // (else the lanes hold their groups as they are)
+                gr = gg_rows<false>(p.cnt, g0 + lane, p.E_l, rows, p.S_rows);
+                mt = (gr.n + tm - 1) / tm;
+                ti = wave_incl_scan(mt);
+            }
+            const int t0 = (before + ti - mt) * nt_all;
             const unsigned long long hit = __ballot(mt > 0 && whole >= t0 && whole < t0 + mt * nt_all);
             if (hit) {
                 const int l = __builtin_ctzll(hit);
-                const int mt_g = __shfl(mt, l, WAVE), in = whole - __shfl(t0, l, WAVE);
+                const int mt_g = wave_lane(mt, l), in = whole - wave_lane(t0, l);
                 g = g0 + l;
                 int m = in % mt_g;
                 nt = in / mt_g;
@@ -135,12 +129,12 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
                     nt = nt * (GG_BN / GS_BN) + tile % (GG_BN / GS_BN);
                 }
                 const int r = m * tm + (TAIL ? tile % subs / (GG_BN / GS_BN) * BM : 0);
-                row0 = __shfl(gr.start, l, WAVE) + r;
-                rv = min(BM, __shfl(gr.n, l, WAVE) - r);
+                row0 = wave_lane(gr.start, l) + r;
+                rv = min(BM, wave_lane(gr.n, l) - r);
                 break;
             }
             rows = gr.end;
-            before += __shfl(ti, WAVE - 1, WAVE);
+            before += wave_lane(ti, WAVE - 1);
         }
     }
     if (TAIL && (rv <= 0 || nt * GS_BN >= q.ncols)) return;  // (past the rows or columns; all parts of the tile alike)

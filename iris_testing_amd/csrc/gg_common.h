@@ -287,14 +287,9 @@ __device__ __forceinline__ GgRows gg_rows(const int32_t* cnt, int g, int E_l, in
         }
         return r;
     }
-    int inc = c;
-#pragma unroll
-    for (int off = 1; off < WAVE; off <<= 1) {
-        const int o = __shfl_up(inc, off, WAVE);
-        if (lane_id() >= off) inc += o;
-    }
+    const int inc = wave_incl_scan(c);
     const int ex = min(inc - c, left);
-    return {before + ex, min(c, left - ex), before + min(__shfl(inc, WAVE - 1, WAVE), left)};
+    return {before + ex, min(c, left - ex), before + min(wave_lane(inc, WAVE - 1), left)};
 }
 
 constexpr int SUP = 16;  // super-tile edge, in large tiles

@@ -1049,19 +1049,14 @@ __global__ __launch_bounds__(256) void grouped_gemm_f32_kernel(const float* __re
         for (int base = 0; base < E_l; base += WAVE) {
             const GgRows r = gg_rows<true>(cnt, base + lane, E_l, rs, S_rows);
             const int t = (r.n + TM - 1) / TM;
-            int tiles = t;
-#pragma unroll
-            for (int off = 1; off < WAVE; off <<= 1) {
-                const int o = __shfl_up(tiles, off, WAVE);
-                if (lane >= off) tiles += o;
-            }
+            const int tiles = wave_incl_scan(t);
             const bool mine = mt < tiles && mt >= tiles - t;
             if (mine) {
                 const int first = (mt - (tiles - t)) * TM;
                 s_g = base + lane; s_row0 = r.start + first; s_rv = min(TM, r.n - first);
             }
             if (__ballot(mine)) break;
-            mt -= __shfl(tiles, WAVE - 1, WAVE);
+            mt -= wave_lane(tiles, WAVE - 1);
             rs = r.end;
         }
     }
@@ -1201,8 +1196,7 @@ __global__ __launch_bounds__(256) void quantize_rows_fp8_kernel(const bf16_t* __
         } else {
             for (int c = lane; c < nv; c += WAVE) amax = fp8_row_amax(src[c], amax);
         }
-#pragma unroll
-        for (int off = WAVE / 2; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, WAVE));
+        amax = __int_as_float(wave_max0(__float_as_int(amax)));  // (never NaN, never below 0: the bits are ordered alike)
         const bool zero = amax == 0.f;
         const float inv = zero ? 1.f : __fdiv_rn(448.f, amax);
         if (lane == 0) scale[r] = zero ? 1.f : __fdiv_rn(amax, 448.f);
@@ -1282,8 +1276,7 @@ __global__ __launch_bounds__(256) void pack_tokens_fp8_kernel(const bf16_t* __re
         } else {
             for (int c = lane; c < nv; c += WAVE) amax = fp8_row_amax(src[c], amax);
         }
-#pragma unroll
-        for (int off = WAVE / 2; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, WAVE));
+        amax = __int_as_float(wave_max0(__float_as_int(amax)));  // (never NaN, never below 0: the bits are ordered alike)
         const bool zero = amax == 0.f;
         const float inv = zero ? 1.f : __fdiv_rn(448.f, amax);
         const float sc = zero ? 1.f : __fdiv_rn(amax, 448.f);

@@ -460,14 +460,15 @@ constexpr int TK_MAXV = 8;  // values per lane -> E <= 8*G
 
 // The value of the lane `off` away in the butterfly of a reduction over 2 off lanes (off a power of two).  Up to 8 it is
 // a DPP move (xor 1, xor 2, then the mirror images within 8 and within 16 lanes: by then the two halves are uniform, so
-// any lane of the other half will do); beyond that a cross-lane read.
+// any lane of the other half will do); beyond that rows or halves change places.
 __device__ __forceinline__ unsigned tk_xchg(int off, unsigned x) {
     switch (off) {
         case 1: return (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0xB1, 0xF, 0xF, false);   // quad_perm [1,0,3,2]
         case 2: return (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x4E, 0xF, 0xF, false);   // quad_perm [2,3,0,1]
         case 4: return (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x141, 0xF, 0xF, false);  // row_half_mirror
         case 8: return (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x140, 0xF, 0xF, false);  // row_mirror
-        default: return (unsigned)__shfl_xor((int)x, off, WAVE);
+        case 16: return (unsigned)wave_xor<16>((int)x);
+        default: return (unsigned)wave_xor<32>((int)x);
     }
 }
 
