@@ -1028,19 +1028,23 @@ __global__ void zero_pad_rows_kernel(T* __restrict__ out, int K, int Nreal, int 
 // order of a scalar fmaf chain).  Weights in the reference layout [E_l][K][N].
 // Bound at the plumbing sizes (512 rows, K 256 / 512) by the length of its chain: load, LDS, matrix instructions, slab by slab, with few
 // workgroups in flight; hence the long slabs (R = 1: 128 of K, twice the loads under way) and small tiles (256 workgroups of
-// 32 x 32 where 64 x 64 gives 64).  On the vector units with 64 x 64 tiles the two GEMMs took 32 and 56 us, now 10 and 14.
+// 32 x 32 where 64 x 64 gives 64).  KG = 2, where there are few tiles: eight waves to a tile, slabs twice as long, every set of four with half of
+// a slab's steps and the second half's sums added at the end: the two GEMMs 22.7 -> 17.1 us (with one set 21.3; on the vector
+// units with 64 x 64 tiles they took 32 and 56 us).
 // R = 2 for launches of many tiles: every operand value out of LDS feeds two matrix instructions.
 // A in LDS as [row][k % 4][k / 4]: the four values a lane needs in four consecutive steps are one 16-byte read; B as
 // [k][column], rows padded so that the four k of a step lie in different banks.
-template <int EPI, int R>
-__global__ __launch_bounds__(256) void grouped_gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ Wt,
+template <int EPI, int R, int KG>
+__global__ __launch_bounds__(256 * KG) void grouped_gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ Wt,
                                                                 const float* __restrict__ Wup, float* __restrict__ C,
                                                                 const int32_t* __restrict__ cnt, int E_l, int K, int N,
                                                                 int S_rows, bool vec) {
-    constexpr int TM = 32 * R, KC = 128 / R, PT = TM * KC / 4 / 256;  // PT: 16-byte units of each operand per thread and slab
+    // PT: 16-byte units of each operand per thread and slab
+    constexpr int TM = 32 * R, KC = 128 / R * KG, NTH = 256 * KG, PT = TM * KC / 4 / NTH, STEPS = KC / 16 / KG;
     constexpr int PA = KC + 4, PB = TM + 16;
     constexpr bool UP = EPI == EPI_SWIGLU;
-    __shared__ float As[TM * PA], Bs[KC * PB], Us[UP ? KC * PB : 1];
+    extern __shared__ __align__(16) float slab[];
+    float *const As = slab, *const Bs = As + TM * PA, *const Us = Bs + KC * PB;
     __shared__ int s_g, s_row0, s_rv;
     const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
     if (wave == 0) {  // which expert's rows: 64 experts at a time, tiles and rows before them by a scan
@@ -1083,7 +1087,7 @@ __global__ __launch_bounds__(256) void grouped_gemm_f32_kernel(const float* __re
     auto fetch = [&](int k0) {
 #pragma unroll
         for (int q = 0; q < PT; ++q) {
-            const int i = threadIdx.x + q * 256;
+            const int i = threadIdx.x + q * NTH;
             const int r = i / (KC / 4), k4 = i % (KC / 4);     // A: consecutive threads walk K
             ra[q] = load(A + (size_t)(row0 + min(r, rv - 1)) * K, k0 + 4 * k4, r < rv ? K : 0);
             const int kb = i / (TM / 4), n4 = i % (TM / 4);     // W: consecutive threads walk N
@@ -1093,13 +1097,14 @@ __global__ __launch_bounds__(256) void grouped_gemm_f32_kernel(const float* __re
             if constexpr (UP) ru[q] = load(U + row, n0 + 4 * n4, end);
         }
     };
-    const int wm = (wave / 2) * 16 * R, wn = (wave % 2) * 16 * R, l16 = lane % 16, kg = lane / 16;
+    const int half = wave / 4;  // which steps of a slab are this wave's
+    const int wm = (wave / 2 % 2) * 16 * R, wn = (wave % 2) * 16 * R, l16 = lane % 16, kg = lane / 16;
     floatx4 acc[R][R] = {}, acu[UP ? R : 1][R] = {};
     fetch(0);
     for (int k0 = 0; k0 < K; k0 += KC) {
 #pragma unroll
         for (int q = 0; q < PT; ++q) {
-            const int i = threadIdx.x + q * 256;
+            const int i = threadIdx.x + q * NTH;
             float* a = As + (i / (KC / 4)) * PA + i % (KC / 4);
             a[0] = ra[q].x; a[KC / 4] = ra[q].y; a[2 * (KC / 4)] = ra[q].z; a[3 * (KC / 4)] = ra[q].w;
             const int b = (i / (TM / 4)) * PB + (i % (TM / 4)) * 4;
@@ -1109,8 +1114,8 @@ __global__ __launch_bounds__(256) void grouped_gemm_f32_kernel(const float* __re
         __syncthreads();
         if (k0 + KC < K) fetch(k0 + KC);
         // slab positions past K hold zeros: adding +0 products leaves every sum as it is
-        const int steps = min(KC, K - k0 + 15) / 16;
-        for (int s4 = 0; s4 < steps; ++s4) {
+        const int steps = min(KC, K - k0 + 15) / 16 - half * STEPS;
+        auto step = [&](int s4) {
             floatx4 a[R];
 #pragma unroll
             for (int i = 0; i < R; ++i) a[i] = *reinterpret_cast<const floatx4*>(As + (wm + 16 * i + l16) * PA + kg * (KC / 4) + 4 * s4);
@@ -1126,8 +1131,35 @@ __global__ __launch_bounds__(256) void grouped_gemm_f32_kernel(const float* __re
                         if constexpr (UP) acu[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][u], uv, acu[i][j], 0, 0, 0);
                     }
                 }
+        };
+        if (steps >= STEPS) {  // (all of them in one piece: the reads of the next steps go under the products of this one)
+#pragma unroll
+            for (int s4 = 0; s4 < STEPS; ++s4) step(half * STEPS + s4);
+        } else {
+            for (int s4 = 0; s4 < steps; ++s4) step(half * STEPS + s4);
         }
         __syncthreads();
+    }
+    if constexpr (KG == 2) {  // the second half's sums, through LDS
+        float* const o = slab + (threadIdx.x & 255) * (R * R * 4 * (UP ? 2 : 1));
+        if (half) {
+#pragma unroll
+            for (int i = 0; i < R; ++i)
+#pragma unroll
+                for (int j = 0; j < R; ++j) {
+                    *reinterpret_cast<floatx4*>(o + (i * R + j) * 4) = acc[i][j];
+                    if constexpr (UP) *reinterpret_cast<floatx4*>(o + (R * R + i * R + j) * 4) = acu[i][j];
+                }
+        }
+        __syncthreads();
+        if (half) return;
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+#pragma unroll
+            for (int j = 0; j < R; ++j) {
+                acc[i][j] += *reinterpret_cast<const floatx4*>(o + (i * R + j) * 4);
+                if constexpr (UP) acu[i][j] += *reinterpret_cast<const floatx4*>(o + (R * R + i * R + j) * 4);
+            }
     }
 #pragma unroll
     for (int i = 0; i < R; ++i)
@@ -1609,6 +1641,10 @@ int launch_gemm(const GemmParams& p_in, int epi, hipStream_t s, void* part_ws = 
     return tail();
 }
 
+constexpr int gg_f32_lds(int R, int KG, bool up) {
+    const int KC = 128 / R * KG;
+    return (32 * R * (KC + 4) + (up ? 2 : 1) * KC * (32 * R + 16)) * 4;
+}
 int launch_f32(const float* A, const float* W, const float* U, float* C, const int32_t* cnt, int E_l, int K, int N, int S_rows,
                int epi, hipStream_t s) {
     if (S_rows == 0) return MOE_OK;
@@ -1617,10 +1653,16 @@ int launch_f32(const float* A, const float* W, const float* U, float* C, const i
     const bool big = (long long)ceil_div(N, 64) * ceil_div(S_rows, 64) >= 2 * num_cus();
     const int tile = big ? 64 : 32;
     dim3 grid(ceil_div(N, tile), ceil_div(S_rows, tile) + E_l);
+    // Two sets of waves to a tile up to two workgroups a compute unit (half a tile per group more than the rows fill): 344 tiles, K 1000
+    // 30.4 -> 21.7 us, but 832 tiles, K 1024 51.5 -> 58.0 (one such workgroup fits a compute unit, three of the others do).
+    const bool split = !big && K > 128 && (long long)ceil_div(N, 32) * (ceil_div(S_rows, 32) + E_l / 2) <= 2 * num_cus();
+#define GG_F32_K(EPI, R, KG)                                                                                                         \
+    grouped_gemm_f32_kernel<EPI, R, KG><<<grid, 256 * KG, gg_f32_lds(R, KG, EPI == EPI_SWIGLU), s>>>(A, W, U, C, cnt, E_l, K, N, S_rows, vec)
 #define GG_F32(EPI)                                                                                                                  \
     case EPI:                                                                                                                        \
-        if (big) grouped_gemm_f32_kernel<EPI, 2><<<grid, 256, 0, s>>>(A, W, U, C, cnt, E_l, K, N, S_rows, vec);                      \
-        else grouped_gemm_f32_kernel<EPI, 1><<<grid, 256, 0, s>>>(A, W, U, C, cnt, E_l, K, N, S_rows, vec);                          \
+        if (big) GG_F32_K(EPI, 2, 1);                                                                                                \
+        else if (split) GG_F32_K(EPI, 1, 2);                                                                                         \
+        else GG_F32_K(EPI, 1, 1);                                                                                                    \
         break
     switch (epi) {
         GG_F32(EPI_NONE);
@@ -1630,6 +1672,7 @@ int launch_f32(const float* A, const float* W, const float* U, float* C, const i
         default: return moe_fail(MOE_ERR_INVALID, "grouped_gemm: activation %d", epi);
     }
 #undef GG_F32
+#undef GG_F32_K
     return moe_check_launch("grouped_gemm_f32");
 }
 

@@ -153,3 +153,30 @@ def test_counts_that_claim_far_too_much_of_very_many_rows():
     for e in range(1, 60):
         assert torch.allclose(got[at + e - 1], x[at + e - 1] @ w[e], rtol=1e-5, atol=1e-5)
     assert torch.allclose(got[at + 59:], x[at + 59:] @ w[60], rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("cnt,K,N", [((33, 0, 31), 128, 36), ((1, 64), 129, 32), ((32, 5), 240, 33), ((40,), 256, 7), ((17, 65), 257, 100),
+                                     ((256, 256), 512, 256), ((3,), 1000, 64)])
+@pytest.mark.parametrize("act", ["none", "swiglu"])
+def test_f32_sums_by_one_and_two_sets_of_waves(cnt, K, N, act):
+    """Few tiles and more than one slab's K: a tile's sums are made in two halves.  Against float64, with the bound of any order of
+    K fp32 products and additions, (K + 1) 2^-24 of the sum of their magnitudes; a gated product adds its activation's rounding."""
+    g = torch.Generator(device=DEV).manual_seed(K + N)
+    S, E_l = sum(cnt), len(cnt)
+    x = torch.randn(S, K, generator=g, device=DEV)
+    w, wu = (torch.randn(E_l, K, N, generator=g, device=DEV) * K ** -0.5 for _ in range(2))
+    c = torch.tensor(cnt, dtype=torch.int32, device=DEV)
+    eye = torch.eye(N, K, device=DEV).expand(E_l, N, K).contiguous()
+    got = ops.grouped_gemm(x, w, c) if act == "none" else ops.grouped_mlp(x, c, "swiglu", w, eye, wu)[:, :N]
+    r0 = 0
+    for e, n in enumerate(cnt):
+        xd, a, b = x[r0:r0 + n].double(), w[e].double(), wu[e].double()
+        s, mag = xd @ a, xd.abs() @ a.abs()
+        bar = (K + 1) * 2.0 ** -24 * mag
+        if act == "swiglu":
+            u = xd @ b
+            # |silu'| < 1.1; exp, division and product: 8 roundings; the product with the identity adds none
+            bar = 1.1 * bar * u.abs() + torch.nn.functional.silu(s).abs() * (K + 1) * 2.0 ** -24 * (xd.abs() @ b.abs()) + 2.0 ** -21 * (s * u).abs()
+            s = torch.nn.functional.silu(s) * u
+        assert bool(((got[r0:r0 + n].double() - s).abs() <= bar + 1e-30).all()), (e, float(((got[r0:r0 + n].double() - s).abs() / (bar + 1e-30)).max()))
+        r0 += n
