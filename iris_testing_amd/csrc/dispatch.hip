@@ -394,7 +394,33 @@ __device__ __forceinline__ int source_row(const RowSource& a, int r) {
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
-template <int WPB, bool RECV>
+// Rows of a copy that a wave takes together: of 2 to 4 KB two (eight 16-byte loads of a lane in flight instead of four; 4096 x 2 rows of 3 KB:
+// payload 11.2 -> 10.2 us, unpack 11.6 -> 9.8, return 12.1 -> 10.4), where rows are many enough to keep every place on the chip taken (1024
+// rows one by one or two by two: the same).  Shorter rows gain nothing from four together (8192 x 2 of 1 KB 8.3 -> 9.2) and few rows lose.
+inline int copy_rows(int n_rows, int row_vec) { return row_vec > 2 * WAVE && row_vec <= 4 * WAVE && n_rows >= 4096 ? 2 : 1; }
+// RPW rows of at most 8 / RPW vectors a lane, row j from src[from[j]] (below 0: zeros) to dst[j]; NT_STORE: non-temporal stores
+template <int RPW, bool NT_STORE>
+__device__ __forceinline__ void copy_rows_together(const u32x4* const (&from)[RPW], u32x4* const (&to)[RPW], int row_vec, int lane) {
+    constexpr int V = 8 / RPW;
+    u32x4 v[RPW][V];
+#pragma unroll
+    for (int j = 0; j < RPW; ++j)
+#pragma unroll
+        for (int u = 0; u < V; ++u) {
+            v[j][u] = u32x4{0u, 0u, 0u, 0u};
+            if (from[j] && lane + u * WAVE < row_vec) v[j][u] = __builtin_nontemporal_load(from[j] + lane + u * WAVE);
+        }
+#pragma unroll
+    for (int j = 0; j < RPW; ++j)
+#pragma unroll
+        for (int u = 0; u < V; ++u)
+            if (to[j] && lane + u * WAVE < row_vec) {
+                if constexpr (NT_STORE) __builtin_nontemporal_store(v[j][u], to[j] + lane + u * WAVE);
+                else to[j][lane + u * WAVE] = v[j][u];
+            }
+}
+
+template <int WPB, bool RECV, int RPW>
 __global__ __launch_bounds__(WPB * WAVE) void gather_rows_kernel(const u32x4* __restrict__ src, u32x4* __restrict__ dst,
                                                                   const RowSource src_of, int n_rows,
                                                                   int row_vec /* 16-byte units per row */, const RecvCounts q) {
@@ -405,7 +431,22 @@ __global__ __launch_bounds__(WPB * WAVE) void gather_rows_kernel(const u32x4* __
         recv_tables(tables, q, a.W, a.E_l);
         a.rc = tables.rc; a.src_off = tables.src_off; a.row_off = tables.row_off; a.flat_off = tables.flat_off;
     }
-    const int wave = threadIdx.x / WAVE, lane = lane_id();
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = lane_id();
+    if constexpr (RPW > 1) {
+        for (unsigned r0 = (blockIdx.x * WPB + wave) * RPW; r0 < (unsigned)n_rows; r0 += gridDim.x * WPB * RPW) {
+            const u32x4* from[RPW];
+            u32x4* to[RPW];
+#pragma unroll
+            for (int j = 0; j < RPW; ++j) {
+                const bool live = r0 + j < (unsigned)n_rows;
+                const int m = live ? source_row(a, (int)(r0 + j)) : -1;
+                from[j] = m >= 0 ? src + (size_t)m * row_vec : nullptr;
+                to[j] = live ? dst + (size_t)(r0 + j) * row_vec : nullptr;
+            }
+            copy_rows_together<RPW, true>(from, to, row_vec, lane);
+        }
+        return;
+    }
     for (int r = blockIdx.x * WPB + wave; r < n_rows; r += gridDim.x * WPB) {
         const int m = source_row(a, r);
         u32x4* d = dst + (size_t)r * row_vec;
@@ -755,8 +796,11 @@ int launch_combine(const void* ret, const int32_t* idx, const int32_t* pos, cons
 
 int gather_rows(const void* src, void* dst, const RowSource& a, int n_rows, int row_bytes, hipStream_t s) {
     if (n_rows == 0) return MOE_OK;
-    const int blocks = min(ceil_div(n_rows, 4), 65535 * 8);
-    gather_rows_kernel<4, false><<<blocks, 4 * WAVE, 0, s>>>((const u32x4*)src, (u32x4*)dst, a, n_rows, row_bytes / 16, RecvCounts{});
+    const int rpw = copy_rows(n_rows, row_bytes / 16), blocks = min(ceil_div(n_rows, 4 * rpw), 65535 * 8);
+#define MOE_GATHER(R) gather_rows_kernel<4, false, R><<<blocks, 4 * WAVE, 0, s>>>((const u32x4*)src, (u32x4*)dst, a, n_rows, row_bytes / 16, RecvCounts{})
+    if (rpw == 2) MOE_GATHER(2);
+    else MOE_GATHER(1);
+#undef MOE_GATHER
     return moe_check_launch("gather_rows");
 }
 
@@ -893,10 +937,10 @@ __global__ __launch_bounds__(256) void a2a_max_count_kernel(const A2aSources q, 
     __shared__ int32_t most;
     if (threadIdx.x == 0) most = first ? 0 : out[1];
     __syncthreads();
-    for (int i = threadIdx.x; i < ns * E_l; i += blockDim.x) {
-        const int c = a2a_count(q.src[i / E_l], i % E_l);
-        if (c > 0) atomicMax(&most, c);
-    }
+    int c = 0;
+    for (int i = threadIdx.x; i < ns * E_l; i += blockDim.x) c = max(c, a2a_count(q.src[i / E_l], i % E_l));
+    c = wave_max0(c);  // (one atomic a wave: 256 of them on one word follow each other)
+    if (lane_id() == 0) atomicMax(&most, c);
     __syncthreads();
     if (threadIdx.x == 0) {
         if (last) tell_host(out, most);
@@ -904,6 +948,7 @@ __global__ __launch_bounds__(256) void a2a_max_count_kernel(const A2aSources q, 
     }
 }
 
+template <int RPW>
 __global__ __launch_bounds__(256) void a2a_place_kernel(const A2aSources q, int s0, int ns, int W, int E_l, int CAP, int row_vec,
                                                          u32x4* __restrict__ token_buf, int32_t* __restrict__ pca,
                                                          int32_t* __restrict__ counts_ready, int n_ready,
@@ -929,25 +974,39 @@ __global__ __launch_bounds__(256) void a2a_place_kernel(const A2aSources q, int 
         for (int i = tid; i < n_sync; i += blockDim.x) token_sync[i] = W;
     }
     __syncthreads();
-    const int n_rows = E_l * ns * CAP, wpb = blockDim.x / WAVE;
-    for (int r = blockIdx.x * wpb + tid / WAVE; r < n_rows; r += gridDim.x * wpb) {
-        const int j = r % CAP, s = r / CAP % ns, e = r / CAP / ns;
-        u32x4* d = token_buf + (((size_t)e * W + s0 + s) * CAP + j) * row_vec;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE), wpb = blockDim.x / WAVE;
+    const unsigned n_rows = (unsigned)(E_l * ns * CAP);
+    // row r of the launch: (e, s, j); the source's row, or NULL: zeros
+    auto row = [&](unsigned r, u32x4*& to) -> const u32x4* {
+        const int j = (int)(r % CAP), s = (int)(r / CAP) % ns, e = (int)(r / CAP) / ns;
+        to = token_buf + (((size_t)e * W + s0 + s) * CAP + j) * row_vec;
         const long long at = (long long)off[s * E_l + e] + j;
-        if (j < cnt[s * E_l + e] && at >= 0 && at < q.src[s].rows) {
-            const u32x4* src = (const u32x4*)q.src[s].payload + (size_t)at * row_vec;
+        return j < cnt[s * E_l + e] && at >= 0 && at < q.src[s].rows ? (const u32x4*)q.src[s].payload + (size_t)at * row_vec : nullptr;
+    };
+    for (unsigned r0 = (blockIdx.x * wpb + wave) * RPW; r0 < n_rows; r0 += gridDim.x * wpb * RPW) {
+        const u32x4* from[RPW];
+        u32x4* to[RPW];
+#pragma unroll
+        for (int i = 0; i < RPW; ++i) {
+            from[i] = nullptr;
+            to[i] = nullptr;
+            if (r0 + i < n_rows) from[i] = row(r0 + i, to[i]);
+        }
+        if constexpr (RPW > 1) {
+            copy_rows_together<RPW, false>(from, to, row_vec, lane);
+        } else if (from[0]) {
             int c = lane;
             for (; c + 3 * WAVE < row_vec; c += 4 * WAVE) {
                 u32x4 v[4];
 #pragma unroll
-                for (int u = 0; u < 4; ++u) v[u] = __builtin_nontemporal_load(src + c + u * WAVE);
+                for (int u = 0; u < 4; ++u) v[u] = __builtin_nontemporal_load(from[0] + c + u * WAVE);
 #pragma unroll
-                for (int u = 0; u < 4; ++u) d[c + u * WAVE] = v[u];
+                for (int u = 0; u < 4; ++u) to[0][c + u * WAVE] = v[u];
             }
-            for (; c < row_vec; c += WAVE) d[c] = __builtin_nontemporal_load(src + c);
+            for (; c < row_vec; c += WAVE) to[0][c] = __builtin_nontemporal_load(from[0] + c);
         } else {
             const u32x4 z = {0u, 0u, 0u, 0u};
-            for (int c = lane; c < row_vec; c += WAVE) d[c] = z;
+            for (int c = lane; c < row_vec; c += WAVE) to[0][c] = z;
         }
     }
 }
@@ -960,8 +1019,12 @@ __global__ __launch_bounds__(256) void shuffle_totals_kernel(const int32_t* __re
     int s = 0, m = 0x7fffffff;
     for (int i = threadIdx.x; i < n; i += blockDim.x) s += pca[i];
     for (int i = threadIdx.x; i < n_sync; i += blockDim.x) m = min(m, sync[i]);
-    atomicAdd(&sum, s);
-    atomicMin(&least, m);
+    s = wave_sum(s);
+    wave_butterfly([&](auto off) { m = min(m, wave_xor<decltype(off)::value>(m)); });
+    if (lane_id() == 0) {
+        atomicAdd(&sum, s);
+        atomicMin(&least, m);
+    }
     __syncthreads();
     if (threadIdx.x == 0) {
         out[1] = least;
@@ -1149,8 +1212,11 @@ static int recv_driven(const char* who, int mode, const void* src, void* dst, in
     a.W = W; a.E_l = E_l; a.M = M; a.CAP = CAP;
     a.status = status;
     // (one workgroup at least, for pca and the totals; at most what the chip holds at once, which then walks the rows)
-    const int blocks = max(1, min(ceil_div(n_out, 4), 256 * 7));
-    gather_rows_kernel<4, true><<<blocks, 4 * WAVE, 0, s>>>((const u32x4*)src, (u32x4*)dst, a, n_out, H * dtype_size(dtype) / 16, q);
+    const int row_vec = H * dtype_size(dtype) / 16, rpw = copy_rows(n_out, row_vec), blocks = max(1, min(ceil_div(n_out, 4 * rpw), 256 * 7));
+#define MOE_GATHER(R) gather_rows_kernel<4, true, R><<<blocks, 4 * WAVE, 0, s>>>((const u32x4*)src, (u32x4*)dst, a, n_out, row_vec, q)
+    if (rpw == 2) MOE_GATHER(2);
+    else MOE_GATHER(1);
+#undef MOE_GATHER
     return moe_check_launch(who);
 }
 
@@ -1370,10 +1436,17 @@ extern "C" int moe_a2a_place(const moe_a2a_source* sources, int dtype, int W, in
     MOE_REQUIRE(token_buf && pca, MOE_ERR_INVALID, "a2a_place: null pointer");
     for (int s0 = 0; s0 < W; s0 += A2A_SRC) {
         const int ns = min(A2A_SRC, W - s0);
-        const int blocks = min(ceil_div(E_l * ns * CAP, 4), 256 * 8);
-        a2a_place_kernel<<<blocks, 256, 0, (hipStream_t)stream>>>(a2a_slice(sources, s0, ns), s0, ns, W, E_l, CAP, H * dtype_size(dtype) / 16,
-                                                                  (u32x4*)token_buf, pca, counts_ready, counts_ready && !s0 ? n_ready : 0,
-                                                                  token_sync, token_sync && !s0 ? n_sync : 0);
+        // (four short rows to a wave where rows are many, see copy_rows: 28672 rows of 1.5 KB, 16384 of them copied 20.8 -> 18.6 us)
+        const int row_vec = H * dtype_size(dtype) / 16, n = E_l * ns * CAP, rpw = n >= 8192 && row_vec <= 2 * WAVE ? 4 : copy_rows(n, row_vec);
+        const int blocks = min(ceil_div(n, 4 * rpw), 256 * 8);
+#define MOE_PLACE(R)                                                                                                                      \
+    a2a_place_kernel<R><<<blocks, 256, 0, (hipStream_t)stream>>>(a2a_slice(sources, s0, ns), s0, ns, W, E_l, CAP, row_vec, (u32x4*)token_buf, \
+                                                                 pca, counts_ready, counts_ready && !s0 ? n_ready : 0, token_sync,        \
+                                                                 token_sync && !s0 ? n_sync : 0)
+        if (rpw == 4) MOE_PLACE(4);
+        else if (rpw == 2) MOE_PLACE(2);
+        else MOE_PLACE(1);
+#undef MOE_PLACE
     }
     return moe_check_launch("a2a_place");
 }

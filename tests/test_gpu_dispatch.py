@@ -11,8 +11,9 @@ from helpers import O, assert_bits_equal, oracle_recv, oracle_world, to_np
 
 pytestmark = pytest.mark.gpu
 
-from iris_testing_amd import ops  # noqa: E402
+from iris_testing_amd import ops, utils  # noqa: E402
 from iris_testing_amd.configs import CONFIGS, gen_router, gen_router_bias, gen_shard_tokens  # noqa: E402
+from iris_testing_amd.layers import SimulatedWorld, custom_a2a, simulated_world  # noqa: E402
 
 DEV = "cuda"
 
@@ -603,3 +604,62 @@ def test_router_tiles_are_bit_exact(T, H, E, k, bias):
     assert_bits_equal(logits, o_logits, "router logits")
     assert_bits_equal(idx, o_idx, "top-k indices")
     np.testing.assert_allclose(to_np(gate), o_gate, rtol=1e-5, atol=1e-30)
+
+
+@pytest.mark.parametrize("H", [1024, 1032, 2040, 2048, 2056])
+def test_copies_of_many_rows_two_and_four_to_a_wave(H):
+    """Rows of 2 to 4 KB are copied two, the exchange's shorter ones four to a wave when there are many.  A copy moves columns without
+    looking at them: the first 64 of every output are those of the same copy of 64-column rows, which go one by one."""
+    T, E, W, k, E_l = 2051, 24, 4, 2, 6
+    g = torch.Generator(device=DEV).manual_seed(H)
+    x = torch.randn(T, H, generator=g, device=DEV).bfloat16()
+    idx = torch.stack([torch.randperm(E, generator=torch.Generator().manual_seed(t))[:k] for t in range(T)]).to(torch.int32).to(DEV)
+    n = ops.count_and_offsets(idx, E, W)
+    M, counts, S, cap = int(n.caps[0]) - 3, n.send_counts, T * k, int(n.caps[1]) - 1  # (three rows of a pair and one of an expert have no place)
+    status = lambda: torch.zeros(1, dtype=torch.int32, device=DEV)  # noqa: E731
+
+    def chain(rows, C):
+        cols = lambda *s: torch.full((*s, C), 3.0, dtype=torch.bfloat16, device=DEV)  # noqa: E731
+        payload = ops.pack_payload(rows, n.row_token)
+        recv = ops.pack_fixed_m(rows, n.row_token, n.dst_sizes, n.dst_offsets, M, status=status())
+        buf, pca = ops.unpack_token_buf(recv, counts, cap, cols(E_l, W, cap), status=status())
+        flat = ops.reorder_flat(payload, counts, cap, cols(E_l, W, cap), status=status())
+        er = ops.unpack_expert_major(recv, counts, S)[0]
+        back = ops.return_pack(er, counts, M)
+        pca_cut = counts.T.clamp(max=cap).contiguous()
+        sh = ops.shuffle_rows(flat, pca_cut, int(pca_cut.sum()))[0]
+        return [payload, recv, buf, flat, er, back, sh, ops.shuffle_rows_backward(sh, pca_cut, cap)]
+
+    for i, (a, b) in enumerate(zip(chain(x, H), chain(x[:, :64].contiguous(), 64))):
+        assert torch.equal(a[..., :64].view(torch.int16), b.view(torch.int16)), i
+        assert a.numel() // H >= 4096 or i in (2, 3, 6, 7)
+    assert torch.equal(chain(x, H)[0].view(torch.int16), x[n.row_token.long()].view(torch.int16))
+
+
+@pytest.mark.parametrize("H", [8, 768, 1024, 1032, 2048, 2056])
+def test_exchange_of_many_rows(H):
+    """The exchange by one, two and four rows to a wave, with a source that sends nothing, one whose payload ends early, and an
+    odd number of rows."""
+    W, E_l, cap = 5, 3, 641
+    g = torch.Generator(device=DEV).manual_seed(H)
+    counts = torch.randint(0, cap + 1, (W, E_l), generator=torch.Generator().manual_seed(H)).to(torch.int32)
+    counts[0, 0], counts[1, 2] = cap, 0
+    world, rows = SimulatedWorld(W, rank=0), []
+    for s in range(W):
+        before, size = 7 * s, int(counts[s].sum())
+        rows.append(torch.randn(before + size, H, generator=g, device=DEV).bfloat16())
+        full = torch.zeros(W, E_l, dtype=torch.int32)
+        full[0] = counts[s]
+        if s != 3:
+            world.post(s, rows[s], full.to(DEV), torch.tensor([before] + [0] * (W - 1), dtype=torch.int32, device=DEV))
+    bufs = utils.alloc_shmem_buffers(None, W, E_l, cap, H, torch.bfloat16)
+    bufs.token_buf.fill_(9.0)
+    with simulated_world(world):
+        out = custom_a2a(*world.sends[0], bufs.pca, bufs.token_buf, bufs.counts_ready, bufs.token_sync, None, W * E_l, cap)
+    assert E_l * W * cap >= 8192
+    for s in range(W):
+        at = 7 * s
+        for e in range(E_l):
+            c = 0 if s == 3 else int(counts[s, e])
+            assert torch.equal(out[e, s, :c], rows[s][at:at + c]) and not bool(out[e, s, c:].any()), (s, e)
+            at += c
