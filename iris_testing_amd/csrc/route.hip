@@ -301,7 +301,7 @@ __global__ __launch_bounds__(NWV * WAVE, (NWV == 4 && TB == 2 ? 2 : 1)) void rou
 // ALL = false: one segment per workgroup, its chains to a plane of the workspace; workgroups b, b + 8, ... share an L2 and a segment.
 // ALL = true: the segment chains one after the other; the sum so far stays in registers, a chain is folded into it where its segment
 // ends, and the finished logit leaves: no partial sums in memory (eight planes written and read back were 27 us for 8192
-// tokens x 768, 256 experts: 70 -> 45 us with the top-k), with 16 experts to a wave for twice the waves.
+// tokens x 768, 256 experts: 70 -> 45 us with the top-k), with 16 experts to a wave for twice the waves where tiles are few.
 // Bound by the fp32 rate, which K = 1 MFMAs and vector instructions share (95 us for 4096 x 7168 x 256, measured 136 with the
 // partial sums; the 32 x 32 shape reaches 0.95 of the rate from a single chain per wave, 16 x 16 0.82): what counts is how few
 // vector instructions surround the MFMAs.  9218 tokens x 5032, 32 experts 88 -> 60 us and 16384 x 4096, 32 experts 94 -> 55 us
@@ -737,14 +737,19 @@ extern "C" int moe_route_topk(const void* x, const void* router, const float* bi
         // where the rows are so short that writing and reading the segments' sums takes as long as the products, and there are
         // tiles enough (at 3072 h and more their number, 2.25 for every place on the chip, say, costs more than the sums do).
         const int n_e16 = ceil_div(E, 64), tiles16 = ceil_div(T, RT_TB) * n_e16;
-        final = E > 64 && H <= 1024 && tiles16 >= 256;
-        const int tok_blocks = ceil_div(T, (E <= 32 ? 4 : 1) * RT_TB), n_e = ceil_div(E, 128);
-#define RT_BF16(SHv, NWEv, ALLv, groups)                                                                                       \
-    route_logits_bf16_kernel<SHv, NWEv, ALLv ? 64 : 32, ALLv ? 2 : 4, ALLv><<<8 * (groups), 4 * WAVE, 0, s>>>(                 \
+        const int tok_blocks = ceil_div(T, (E <= 32 ? 4 : 1) * RT_TB), n_e = ceil_div(E, 128), tok8 = ceil_div(ceil_div(T, RT_TB), 8);
+        // With two tiles of 64 tokens x 128 experts for nearly every compute unit that holds for rows of any length, and the 32 x 32 shape does
+        // it: 16384 tokens, 256 experts 71 -> 63 us (512 h), 108 -> 99 (1024), 180 -> 134 (1536), 215 -> 169 (2048), 541 -> 520
+        // (7168); 14336 tokens x 2048 182 -> 167; but 12288 tokens (384 tiles) 156 -> 165, 8192 (256: one to a compute unit) 107 -> 108.
+        const bool all32 = E > 64 && tok_blocks * n_e >= 448;
+        final = all32 || (E > 64 && H <= 1024 && tiles16 >= 256);
+#define RT_BF16(SHv, NWEv, KCv, Dv, ALLv, groups)                                                        \
+    route_logits_bf16_kernel<SHv, NWEv, KCv, Dv, ALLv><<<8 * (groups), 4 * WAVE, 0, s>>>(                \
         (const bf16_t*)x, (const bf16_t*)router, bias, ALLv ? logits : part, T, H, E)
-        if (final) RT_BF16(16, 4, true, ceil_div(ceil_div(T, RT_TB), 8) * n_e16);
-        else if (E <= 32) RT_BF16(32, 1, false, tok_blocks);
-        else RT_BF16(32, 4, false, tok_blocks * n_e);
+        if (all32) RT_BF16(32, 4, 32, 2, true, tok8 * n_e);
+        else if (final) RT_BF16(16, 4, 64, 2, true, tok8 * n_e16);
+        else if (E <= 32) RT_BF16(32, 1, 32, 4, false, tok_blocks);
+        else RT_BF16(32, 4, 32, 4, false, tok_blocks * n_e);
 #undef RT_BF16
         rc = moe_check_launch("route_logits");
     } else {

@@ -606,6 +606,13 @@ def test_router_tiles_are_bit_exact(T, H, E, k, bias):
     np.testing.assert_allclose(to_np(gate), o_gate, rtol=1e-5, atol=1e-30)
 
 
+@pytest.mark.parametrize("T,H,E,k,bias", [(14337, 136, 200, 8, True), (28673, 1032, 68, 2, False), (14500, 40, 132, 3, True)])
+def test_router_of_very_many_tokens_in_finished_logits(T, H, E, k, bias):
+    """Two tiles of 64 tokens x 128 experts for every compute unit: all segments in one workgroup, whatever the rows' length (empty and
+    partly filled segments among them)."""
+    test_router_tiles_are_bit_exact(T, H, E, k, bias)
+
+
 @pytest.mark.parametrize("H", [1024, 1032, 2040, 2048, 2056])
 def test_copies_of_many_rows_two_and_four_to_a_wave(H):
     """Rows of 2 to 4 KB are copied two, the exchange's shorter ones four to a wave when there are many.  A copy moves columns without
