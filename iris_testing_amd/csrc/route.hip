@@ -302,22 +302,23 @@ __global__ __launch_bounds__(NWV * WAVE, (NWV == 4 && TB == 2 ? 2 : 1)) void rou
 // ALL = true: the segment chains one after the other; the sum so far stays in registers, a chain is folded into it where its segment
 // ends, and the finished logit leaves: no partial sums in memory (eight planes written and read back were 27 us for 8192
 // tokens x 768, 256 experts: 70 -> 45 us with the top-k), with 16 experts to a wave for twice the waves where tiles are few.
-// Bound by the fp32 rate, which K = 1 MFMAs and vector instructions share (95 us for 4096 x 7168 x 256, measured 136 with the
-// partial sums; the 32 x 32 shape reaches 0.95 of the rate from a single chain per wave, 16 x 16 0.82): what counts is how few
+// Bound by the fp32 rate, which K = 1 MFMAs and vector instructions share (95 us for 4096 x 7168 x 256, measured 143 with the
+// partial sums and the top-k; the 32 x 32 shape reaches 0.95 of the rate from a single chain per wave, 16 x 16 0.82): what counts is how few
 // vector instructions surround the MFMAs.  9218 tokens x 5032, 32 experts 88 -> 60 us and 16384 x 4096, 32 experts 94 -> 55 us
 // (blocks 32 experts wide instead of 64), 2048 x 4096, 256 experts 64 -> 50 us, 9216 x 3072, 256 experts 179 -> 157 us.
 // Slabs of KC h are double-buffered in LDS; the conversion and the writes of the next slab sit piece by piece between this one's
 // MFMAs, whose chain would leave the issue slots empty.
+// NB = 1: one slab in LDS and four workgroups to a compute unit; the others' products cover a workgroup's conversion, writes and barriers.
 // LDS: tokens as [token][h] (the lane reads eight consecutive h of its token), the router as [h][expert] as it comes.
-template <int SHAPE, int NWE, int KC, int D /* slabs under way in registers */, bool ALL>
-__global__ __launch_bounds__(4 * WAVE, 2) void route_logits_bf16_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
+template <int SHAPE, int NWE, int KC, int D /* slabs under way in registers */, bool ALL, int NB = 2 /* slabs in LDS */>
+__global__ __launch_bounds__(4 * WAVE, NB == 1 ? 4 : 2) void route_logits_bf16_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
                                                                       const float* __restrict__ bias, float* __restrict__ out, int T, int Hrow,
                                                                       int E) {
     constexpr int NTOK = 4 / NWE * RT_TB, EB = NWE * SHAPE, NCH = KC / 8, PX = KC + 4;
     constexpr int XPT = NTOK * NCH / 256, WPT = KC * EB / 4 / 256;  // 16-byte pieces of token rows, 8-byte pieces of the router, per thread and slab
     static_assert(NTOK * NCH % 256 == 0 && KC * EB / 4 % 256 == 0 && XPT + WPT < 2 * NCH, "two pieces per chunk at most");
-    __shared__ __align__(16) float xs[2][NTOK][PX];
-    __shared__ __align__(16) float ws[2][KC][EB];
+    __shared__ __align__(16) float xs[NB][NTOK][PX];
+    __shared__ __align__(16) float ws[NB][KC][EB];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     // workgroups b, b + 8, ... share an L2: ALL: all expert blocks of a token block; else a segment
     const int n_e = (E + EB - 1) / EB, local = (int)blockIdx.x >> 3, b8 = (int)blockIdx.x & 7;
@@ -402,7 +403,7 @@ __global__ __launch_bounds__(4 * WAVE, 2) void route_logits_bf16_kernel(const bf
     __syncthreads();
     // slab s (s % D = S) from buffer S % 2; slab s + 1 (register set N) goes to the other one, slab s + 1 + D is requested in its place
     auto slab = [&](auto idx, int s) {
-        constexpr int S = decltype(idx)::value, B = S % 2, N = (S + 1) % D;
+        constexpr int S = decltype(idx)::value, B = S % NB, N = (S + 1) % D;
         const int n = min(NCH, (H - s * KC) / 8);
         read(f[0], B, 0);
 #pragma unroll
@@ -411,8 +412,8 @@ __global__ __launch_bounds__(4 * WAVE, 2) void route_logits_bf16_kernel(const bf
             if (c + 1 < NCH) read(nxt, B, c + 1);  // (chunks past H: what the slot holds, not used)
             // piece i of what this slab does for the next ones: the next slab's conversion and writes, then the request
             auto piece = [&](int i) {
-                if (i < XPT) put_x(N, 1 - B, i);
-                else if (i - XPT < WPT) put_w(N, 1 - B, i - XPT);
+                if (i < XPT) put_x(N, (B + 1) % NB, i);
+                else if (i - XPT < WPT) put_w(N, (B + 1) % NB, i - XPT);
                 else if (i == XPT + WPT) fetch(N, (s + 1 + D) * KC);
             };
 #pragma unroll
@@ -426,12 +427,20 @@ __global__ __launch_bounds__(4 * WAVE, 2) void route_logits_bf16_kernel(const bf
                     }
                 }
                 __builtin_amdgcn_sched_barrier(0);
-                piece(2 * c + h);
+                if (NB == 2) piece(2 * c + h);
             }
             if (ALL && c < n && --left == 0) fold();
             __builtin_amdgcn_sched_barrier(0);
         }
         __syncthreads();
+        if constexpr (NB == 1) {
+#pragma unroll
+            for (int i = 0; i < XPT; ++i) put_x(N, 0, i);
+#pragma unroll
+            for (int i = 0; i < WPT; ++i) put_w(N, 0, i);
+            fetch(N, (s + 1 + D) * KC);
+            __syncthreads();
+        }
     };
     for (int s = 0; s < n_slab; s += D) {
         slab(std::integral_constant<int, 0>{}, s);
@@ -742,14 +751,20 @@ extern "C" int moe_route_topk(const void* x, const void* router, const float* bi
         // it: 16384 tokens, 256 experts 71 -> 63 us (512 h), 108 -> 99 (1024), 180 -> 134 (1536), 215 -> 169 (2048), 541 -> 520
         // (7168); 14336 tokens x 2048 182 -> 167; but 12288 tokens (384 tiles) 156 -> 165, 8192 (256: one to a compute unit) 107 -> 108.
         const bool all32 = E > 64 && tok_blocks * n_e >= 448;
+        // The segments as workgroups: four to a compute unit (of 256; one slab of LDS each) where that takes no more than half the rounds that two (two slabs)
+        // take: 4096 tokens x 7168, 256 experts (1024 workgroups) 154 -> 143 us with the top-k, 8192 x 2048 (2048) 108 -> 102, 12288 x 2048 155 -> 151,
+        // 600 x 4096 31.4 -> 30.5; but 9216 x 3072 (2304: three rounds for five) 157 -> 163, 6000 x 4992, 160 experts (1504) 146 -> 161.
+        const int wgs = 8 * tok_blocks * n_e, pairs = ceil_div(wgs, 2 * 256);
+        const bool four = pairs == 1 || 2 * ceil_div(wgs, 4 * 256) <= pairs;
         final = all32 || (E > 64 && H <= 1024 && tiles16 >= 256);
-#define RT_BF16(SHv, NWEv, KCv, Dv, ALLv, groups)                                                        \
-    route_logits_bf16_kernel<SHv, NWEv, KCv, Dv, ALLv><<<8 * (groups), 4 * WAVE, 0, s>>>(                \
+#define RT_BF16(SHv, NWEv, KCv, Dv, ALLv, NBv, groups)                                                   \
+    route_logits_bf16_kernel<SHv, NWEv, KCv, Dv, ALLv, NBv><<<8 * (groups), 4 * WAVE, 0, s>>>(           \
         (const bf16_t*)x, (const bf16_t*)router, bias, ALLv ? logits : part, T, H, E)
-        if (all32) RT_BF16(32, 4, 32, 2, true, tok8 * n_e);
-        else if (final) RT_BF16(16, 4, 64, 2, true, tok8 * n_e16);
-        else if (E <= 32) RT_BF16(32, 1, 32, 4, false, tok_blocks);
-        else RT_BF16(32, 4, 32, 4, false, tok_blocks * n_e);
+        if (all32) RT_BF16(32, 4, 32, 2, true, 2, tok8 * n_e);
+        else if (final) RT_BF16(16, 4, 64, 2, true, 2, tok8 * n_e16);
+        else if (E <= 32) RT_BF16(32, 1, 32, 4, false, 2, tok_blocks);
+        else if (four) RT_BF16(32, 4, 32, 2, false, 1, tok_blocks * n_e);
+        else RT_BF16(32, 4, 32, 4, false, 2, tok_blocks * n_e);
 #undef RT_BF16
         rc = moe_check_launch("route_logits");
     } else {

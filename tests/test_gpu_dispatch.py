@@ -613,6 +613,12 @@ def test_router_of_very_many_tokens_in_finished_logits(T, H, E, k, bias):
     test_router_tiles_are_bit_exact(T, H, E, k, bias)
 
 
+@pytest.mark.parametrize("T,H,E,k,bias", [(4033, 264, 140, 8, True), (4097, 504, 130, 2, False), (7000, 72, 68, 4, True), (517, 40, 68, 2, True)])
+def test_router_segments_two_and_four_to_a_compute_unit(T, H, E, k, bias):
+    """One slab of LDS and four workgroups to a compute unit, or two and two, by what the rounds come to."""
+    test_router_tiles_are_bit_exact(T, H, E, k, bias)
+
+
 @pytest.mark.parametrize("H", [1024, 1032, 2040, 2048, 2056])
 def test_copies_of_many_rows_two_and_four_to_a_wave(H):
     """Rows of 2 to 4 KB are copied two, the exchange's shorter ones four to a wave when there are many.  A copy moves columns without
