@@ -302,6 +302,9 @@ __global__ __launch_bounds__(NWV * WAVE, (NWV == 4 && TB == 2 ? 2 : 1)) void rou
 // ALL = true: the segment chains one after the other; the sum so far stays in registers, a chain is folded into it where its segment
 // ends, and the finished logit leaves: no partial sums in memory (eight planes written and read back were 27 us for 8192
 // tokens x 768, 256 experts: 70 -> 45 us with the top-k), with 16 experts to a wave for twice the waves where tiles are few.
+// KG = 2: a second set of waves runs the segments 4 to 7 beside the first one's 0 to 3; its chains wait in registers and go through LDS at the
+// end, where the first set adds them in order, so the bits stay (256 tiles: 4096 tokens x 768 33 -> 28 us; 512: 8192 x 768 48 -> 46, half of it from
+// the rows' leaving through LDS in 16-byte pieces; the products run at 0.86 of the fp32 rate, the other 13 us are launch, first loads and stores).
 // Bound by the fp32 rate, which K = 1 MFMAs and vector instructions share (95 us for 4096 x 7168 x 256, measured 143 with the
 // partial sums and the top-k; the 32 x 32 shape reaches 0.95 of the rate from a single chain per wave, 16 x 16 0.82): what counts is how few
 // vector instructions surround the MFMAs.  9218 tokens x 5032, 32 experts 88 -> 60 us and 16384 x 4096, 32 experts 94 -> 55 us
@@ -310,23 +313,26 @@ __global__ __launch_bounds__(NWV * WAVE, (NWV == 4 && TB == 2 ? 2 : 1)) void rou
 // MFMAs, whose chain would leave the issue slots empty.
 // NB = 1: one slab in LDS and four workgroups to a compute unit; the others' products cover a workgroup's conversion, writes and barriers.
 // LDS: tokens as [token][h] (the lane reads eight consecutive h of its token), the router as [h][expert] as it comes.
-template <int SHAPE, int NWE, int KC, int D /* slabs under way in registers */, bool ALL, int NB = 2 /* slabs in LDS */>
-__global__ __launch_bounds__(4 * WAVE, NB == 1 ? 4 : 2) void route_logits_bf16_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
+template <int SHAPE, int NWE, int KC, int D /* slabs under way in registers */, bool ALL, int NB /* slabs in LDS */, int KG /* sets of waves */>
+__global__ __launch_bounds__(KG * 4 * WAVE, NB == 1 || KG == 2 ? 4 : 2) void route_logits_bf16_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
                                                                       const float* __restrict__ bias, float* __restrict__ out, int T, int Hrow,
                                                                       int E) {
     constexpr int NTOK = 4 / NWE * RT_TB, EB = NWE * SHAPE, NCH = KC / 8, PX = KC + 4;
     constexpr int XPT = NTOK * NCH / 256, WPT = KC * EB / 4 / 256;  // 16-byte pieces of token rows, 8-byte pieces of the router, per thread and slab
     static_assert(NTOK * NCH % 256 == 0 && KC * EB / 4 % 256 == 0 && XPT + WPT < 2 * NCH, "two pieces per chunk at most");
-    __shared__ __align__(16) float xs[NB][NTOK][PX];
-    __shared__ __align__(16) float ws[NB][KC][EB];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    __shared__ __align__(16) float xs[KG * NB][NTOK][PX];
+    __shared__ __align__(16) float ws[KG * NB][KC][EB];
+    const int set = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8);
+    const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
+    const int sb = set * NB;  // the set's first buffer
     // workgroups b, b + 8, ... share an L2: ALL: all expert blocks of a token block; else a segment
     const int n_e = (E + EB - 1) / EB, local = (int)blockIdx.x >> 3, b8 = (int)blockIdx.x & 7;
     static_assert(RT_P == 8, "a segment per group of workgroups");
     const int tb = ALL ? local / n_e * 8 + b8 : local / n_e, eb0 = local % n_e * EB, t0 = tb * NTOK;
     if (t0 >= T) return;
     const int seg_len = route_segment_len(Hrow);
-    const int h0 = ALL ? 0 : min(b8 * seg_len, Hrow), H = ALL ? Hrow : min(seg_len, Hrow - h0);
+    const int span = !ALL ? seg_len : KG == 1 ? Hrow : RT_P / 2 * seg_len;  // columns of the workgroup (KG = 2: of the set)
+    const int h0 = min((ALL ? set : b8) * span, Hrow), H = min(span, Hrow - h0);
     const int wt = wave / NWE * RT_TB, we = wave % NWE * SHAPE;
     const bf16_t *xp[XPT], *wp[WPT];
     int xh[XPT], wh[WPT];  // first h of the piece inside its slab
@@ -357,7 +363,7 @@ __global__ __launch_bounds__(4 * WAVE, NB == 1 ? 4 : 2) void route_logits_bf16_k
         const rt_u4 r = xr[d][i];
         const rt_f4 lo = {__uint_as_float(r.x << 16), __uint_as_float(r.x & 0xffff0000u), __uint_as_float(r.y << 16), __uint_as_float(r.y & 0xffff0000u)};
         const rt_f4 hi = {__uint_as_float(r.z << 16), __uint_as_float(r.z & 0xffff0000u), __uint_as_float(r.w << 16), __uint_as_float(r.w & 0xffff0000u)};
-        float* o = &xs[b][c / NCH][c % NCH * 8];
+        float* o = &xs[sb + b][c / NCH][c % NCH * 8];
         *reinterpret_cast<rt_f4*>(o) = lo;
         *reinterpret_cast<rt_f4*>(o + 4) = hi;
     };
@@ -365,18 +371,34 @@ __global__ __launch_bounds__(4 * WAVE, NB == 1 ? 4 : 2) void route_logits_bf16_k
         const int c = tid + i * 256;
         const uint2 r = wr[d][i];
         const rt_f4 v = {__uint_as_float(r.x << 16), __uint_as_float(r.x & 0xffff0000u), __uint_as_float(r.y << 16), __uint_as_float(r.y & 0xffff0000u)};
-        *reinterpret_cast<rt_f4*>(&ws[b][c / (EB / 4)][c % (EB / 4) * 4]) = v;
+        *reinterpret_cast<rt_f4*>(&ws[sb + b][c / (EB / 4)][c % (EB / 4) * 4]) = v;
     };
     constexpr int NACC = SHAPE == 32 ? 32 : 16;
-    typename RtAcc<SHAPE>::type acc, sum;
+    typename RtAcc<SHAPE>::type acc, sum, later[KG == 2 ? RT_P / 2 - 1 : 1];
 #pragma unroll
     for (int v = 0; v < NACC; ++v) acc[v] = sum[v] = 0.f;
+    if constexpr (KG == 2)
+#pragma unroll
+        for (int i = 0; i < RT_P / 2 - 1; ++i)
+#pragma unroll
+            for (int v = 0; v < NACC; ++v) later[i][v] = 0.f;
     int seg = 0, left = min(seg_len, H) / 8;  // the chain at hand, chunks of eight h until it ends
     auto fold = [&]() {
+        if (KG == 1 || set == 0) {
 #pragma unroll
-        for (int v = 0; v < NACC; ++v) {
-            sum[v] = seg == 0 ? acc[v] : __fadd_rn(sum[v], acc[v]);
-            acc[v] = 0.f;
+            for (int v = 0; v < NACC; ++v) {
+                sum[v] = seg == 0 ? acc[v] : __fadd_rn(sum[v], acc[v]);
+                acc[v] = 0.f;
+            }
+        } else {  // (the second set's chains are added behind the first set's: the last three wait in registers, the last one in sum)
+#pragma unroll
+            for (int v = 0; v < NACC; ++v) {
+                later[0][v] = later[1][v];
+                later[1][v] = later[2][v];
+                later[2][v] = sum[v];
+                sum[v] = acc[v];
+                acc[v] = 0.f;
+            }
         }
         ++seg;
         left = max(min(seg_len, H - seg * seg_len), 0) / 8;
@@ -384,15 +406,15 @@ __global__ __launch_bounds__(4 * WAVE, NB == 1 ? 4 : 2) void route_logits_bf16_k
     struct Frag {
         rt_f4 x[2];
         float w[8];
-    } f[2];
+    } f[KG == 2 ? 1 : 2];  // (two sets: the registers go to the waiting chains; four waves to a SIMD cover the reads)
     auto read = [&](Frag& g, int b, int c) {
-        const float* xl = &xs[b][wt + lane][c * 8];
+        const float* xl = &xs[sb + b][wt + lane][c * 8];
         g.x[0] = *reinterpret_cast<const rt_f4*>(xl);
         g.x[1] = *reinterpret_cast<const rt_f4*>(xl + 4);
 #pragma unroll
-        for (int q = 0; q < 8; ++q) g.w[q] = ws[b][c * 8 + q][we + lane % SHAPE];
+        for (int q = 0; q < 8; ++q) g.w[q] = ws[sb + b][c * 8 + q][we + lane % SHAPE];
     };
-    const int n_slab = (H + KC - 1) / KC;
+    const int n_slab = ((KG == 1 ? H : min(span, Hrow)) + KC - 1) / KC;  // (KG = 2: of the first set, which has no fewer)
 #pragma unroll
     for (int d = 0; d < D; ++d) fetch(d, d * KC);
 #pragma unroll
@@ -405,11 +427,12 @@ __global__ __launch_bounds__(4 * WAVE, NB == 1 ? 4 : 2) void route_logits_bf16_k
     auto slab = [&](auto idx, int s) {
         constexpr int S = decltype(idx)::value, B = S % NB, N = (S + 1) % D;
         const int n = min(NCH, (H - s * KC) / 8);
-        read(f[0], B, 0);
+        if (KG == 1) read(f[0], B, 0);
 #pragma unroll
         for (int c = 0; c < NCH; ++c) {
-            Frag &cur = f[c & 1], &nxt = f[1 - (c & 1)];
-            if (c + 1 < NCH) read(nxt, B, c + 1);  // (chunks past H: what the slot holds, not used)
+            Frag &cur = f[KG == 2 ? 0 : c & 1], &nxt = f[KG == 2 ? 0 : 1 - (c & 1)];
+            if (KG == 2) read(cur, B, c);
+            else if (c + 1 < NCH) read(nxt, B, c + 1);  // (chunks past H: what the slot holds, not used)
             // piece i of what this slab does for the next ones: the next slab's conversion and writes, then the request
             auto piece = [&](int i) {
                 if (i < XPT) put_x(N, (B + 1) % NB, i);
@@ -450,7 +473,49 @@ __global__ __launch_bounds__(4 * WAVE, NB == 1 ? 4 : 2) void route_logits_bf16_k
             if (s + 3 < n_slab) slab(std::integral_constant<int, 3>{}, s + 3);
         }
     }
-    while (ALL && seg < RT_P) fold();  // (empty segments: their chains are +0)
+    while (ALL && seg < RT_P / KG) fold();  // (empty segments: their chains are +0)
+    if constexpr (KG == 2) {
+        // (every wave is past its last look at the slabs)
+        constexpr int PLANE = 4 * WAVE * NACC, PO = EB + 4;
+        static_assert(ALL && sizeof(xs) >= RT_P / 4 * PLANE * 4 && sizeof(ws) >= RT_P / 4 * PLANE * 4 && sizeof(xs) >= NTOK * PO * 4, "half the chains to an array");
+        auto at = [&](int i) { return (i < RT_P / 4 ? &xs[0][0][0] : &ws[0][0][0]) + i % (RT_P / 4) * PLANE + wave * WAVE * NACC + lane * 4; };
+        if (set) {
+#pragma unroll
+            for (int i = 0; i < RT_P / 2; ++i)
+#pragma unroll
+                for (int v = 0; v < NACC; v += 4) {
+                    const auto& a = i < RT_P / 2 - 1 ? later[i < RT_P / 2 - 1 ? i : 0] : sum;
+                    *reinterpret_cast<rt_f4*>(at(i) + v * WAVE) = rt_f4{a[v], a[v + 1], a[v + 2], a[v + 3]};
+                }
+        }
+        __syncthreads();
+        if (!set) {
+#pragma unroll
+            for (int i = 0; i < RT_P / 2; ++i)
+#pragma unroll
+                for (int v = 0; v < NACC; v += 4) {
+                    const rt_f4 a = *reinterpret_cast<const rt_f4*>(at(i) + v * WAVE);
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) sum[v + u] = __fadd_rn(sum[v + u], a[u]);
+                }
+        }
+        __syncthreads();
+        // whole rows of the tile leave, 16 bytes a thread (E % 4 == 0, logits at 16 bytes)
+        float* const rows = &xs[0][0][0];
+        if (!set) {
+            const int el = we + lane % SHAPE;
+            const float be = bias && eb0 + el < E ? bias[eb0 + el] : 0.f;
+#pragma unroll
+            for (int v = 0; v < NACC; ++v) rows[(wt + 16 * (v / 4) + 4 * (lane / 16) + v % 4) * PO + el] = bias ? __fadd_rn(sum[v], be) : sum[v];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < NTOK * EB / 4 / (KG * 4 * WAVE); ++i) {
+            const int c = (int)threadIdx.x + i * KG * 4 * WAVE, t = t0 + c / (EB / 4), e = eb0 + c % (EB / 4) * 4;
+            if (t < T && e < E) *reinterpret_cast<rt_f4*>(out + (size_t)t * E + e) = *reinterpret_cast<const rt_f4*>(rows + c / (EB / 4) * PO + c % (EB / 4) * 4);
+        }
+        return;
+    }
     const int e = eb0 + we + lane % SHAPE;
     if (e >= E) return;
     const float be = ALL && bias ? bias[e] : 0.f;
@@ -743,9 +808,11 @@ extern "C" int moe_route_topk(const void* x, const void* router, const float* bi
     // (the kernel for many tokens reads the router in pieces of four experts: they must lie at 8 bytes; the other one reads values)
     if (dtype == MOE_BF16 && E % 4 == 0 && ((uintptr_t)router & 7) == 0 && ((E > 64 && T > 512) || (E > 16 && E <= 32 && T > 2048))) {
         // (33 to 64 experts: the segment kernel's block of 128 tokens x 64 experts is as good or better.)  All segments in one workgroup
-        // where the rows are so short that writing and reading the segments' sums takes as long as the products, and there are
-        // tiles enough (at 3072 h and more their number, 2.25 for every place on the chip, say, costs more than the sums do).
-        const int n_e16 = ceil_div(E, 64), tiles16 = ceil_div(T, RT_TB) * n_e16;
+        // (tiles of 64 x 64, two sets of waves) where that is quicker than segments as workgroups, whose sums are written and read back:
+        // 13 us + 0.0203 (one round: 0.0213) for each h and round of the chip against 17 us + 0.042 a tile + 0.0165 for each h and 256 tiles.  With the top-k, 256
+        // experts: 8192 tokens x 256 47 -> 26 us, x 768 63 -> 46, x 1536 90 -> 75, x 3072 147 -> 137, but x 7168 269 -> 288; 4096 x 768 37 -> 29, x 1536
+        // 49 -> 45, x 3072 75 -> 79; 6000 (376 tiles) x 768 51 -> 43, x 1536 70 -> 72; 2048 x 256 22 -> 15, x 768 equal; 1024 (64 tiles) x 256 equal.
+        const int n_e16 = ceil_div(E, 64), tiles16 = ceil_div(T, RT_TB) * n_e16, r16 = ceil_div(tiles16, 256);
         const int tok_blocks = ceil_div(T, (E <= 32 ? 4 : 1) * RT_TB), n_e = ceil_div(E, 128), tok8 = ceil_div(ceil_div(T, RT_TB), 8);
         // With two tiles of 64 tokens x 128 experts for nearly every compute unit that holds for rows of any length, and the 32 x 32 shape does
         // it: 16384 tokens, 256 experts 71 -> 63 us (512 h), 108 -> 99 (1024), 180 -> 134 (1536), 215 -> 169 (2048), 541 -> 520
@@ -756,15 +823,15 @@ extern "C" int moe_route_topk(const void* x, const void* router, const float* bi
         // 600 x 4096 31.4 -> 30.5; but 9216 x 3072 (2304: three rounds for five) 157 -> 163, 6000 x 4992, 160 experts (1504) 146 -> 161.
         const int wgs = 8 * tok_blocks * n_e, pairs = ceil_div(wgs, 2 * 256);
         const bool four = pairs == 1 || 2 * ceil_div(wgs, 4 * 256) <= pairs;
-        final = all32 || (E > 64 && H <= 1024 && tiles16 >= 256);
-#define RT_BF16(SHv, NWEv, KCv, Dv, ALLv, NBv, groups)                                                   \
-    route_logits_bf16_kernel<SHv, NWEv, KCv, Dv, ALLv, NBv><<<8 * (groups), 4 * WAVE, 0, s>>>(           \
+        final = all32 || (E > 64 && tiles16 >= 128 && H * ((r16 == 1 ? 0.0213 : 0.0203 * r16) - 0.0165 / 256 * tiles16) < 4 + 0.042 * tiles16);
+#define RT_BF16(SHv, NWEv, KCv, Dv, ALLv, NBv, KGv, groups)                                                   \
+    route_logits_bf16_kernel<SHv, NWEv, KCv, Dv, ALLv, NBv, KGv><<<8 * (groups), KGv * 4 * WAVE, 0, s>>>(      \
         (const bf16_t*)x, (const bf16_t*)router, bias, ALLv ? logits : part, T, H, E)
-        if (all32) RT_BF16(32, 4, 32, 2, true, 2, tok8 * n_e);
-        else if (final) RT_BF16(16, 4, 64, 2, true, 2, tok8 * n_e16);
-        else if (E <= 32) RT_BF16(32, 1, 32, 4, false, 2, tok_blocks);
-        else if (four) RT_BF16(32, 4, 32, 2, false, 1, tok_blocks * n_e);
-        else RT_BF16(32, 4, 32, 4, false, 2, tok_blocks * n_e);
+        if (all32) RT_BF16(32, 4, 32, 2, true, 2, 1, tok8 * n_e);
+        else if (final) RT_BF16(16, 4, 32, 2, true, 2, 2, tok8 * n_e16);
+        else if (E <= 32) RT_BF16(32, 1, 32, 4, false, 2, 1, tok_blocks);
+        else if (four) RT_BF16(32, 4, 32, 2, false, 1, 1, tok_blocks * n_e);
+        else RT_BF16(32, 4, 32, 4, false, 2, 1, tok_blocks * n_e);
 #undef RT_BF16
         rc = moe_check_launch("route_logits");
     } else {

@@ -619,6 +619,12 @@ def test_router_segments_two_and_four_to_a_compute_unit(T, H, E, k, bias):
     test_router_tiles_are_bit_exact(T, H, E, k, bias)
 
 
+@pytest.mark.parametrize("T,H,E,k,bias", [(2050, 264, 256, 8, True), (8191, 72, 68, 2, False), (4097, 1032, 132, 4, True), (2048, 8, 252, 2, False), (2113, 40, 256, 3, True)])
+def test_router_segments_by_two_sets_of_waves(T, H, E, k, bias):
+    """Tiles of 64 x 64 whose segments two sets of waves share: empty and partly filled segments in either set, ragged tiles."""
+    test_router_tiles_are_bit_exact(T, H, E, k, bias)
+
+
 @pytest.mark.parametrize("H", [1024, 1032, 2040, 2048, 2056])
 def test_copies_of_many_rows_two_and_four_to_a_wave(H):
     """Rows of 2 to 4 KB are copied two, the exchange's shorter ones four to a wave when there are many.  A copy moves columns without
