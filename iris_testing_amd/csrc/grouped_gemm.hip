@@ -1034,19 +1034,43 @@ __global__ void zero_pad_rows_kernel(T* __restrict__ out, int K, int Nreal, int 
 // R = 2 for launches of many tiles: every operand value out of LDS feeds two matrix instructions.
 // A in LDS as [row][k % 4][k / 4]: the four values a lane needs in four consecutive steps are one 16-byte read; B as
 // [k][column], rows padded so that the four k of a step lie in different banks.
-template <int EPI, int R, int KG>
+// RET: result rows go to their slots of the returned [W,M,N] buffer as well, and the workgroups from ret.tiles_y on zero its padding rows: a
+// launch that only copied the rows took 2.5 us of the 43 of the plumbing step.  The tile's rows belong to one expert, whose slots
+// start at the sums of the received counts before it.
+struct F32Return {
+    const int32_t* rc;  // received counts [W,E_l]
+    int W, M;
+    float* buf;
+    int tiles_y;
+};
+template <int EPI, int R, int KG, bool RET = false>
 __global__ __launch_bounds__(256 * KG) void grouped_gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ Wt,
                                                                 const float* __restrict__ Wup, float* __restrict__ C,
                                                                 const int32_t* __restrict__ cnt, int E_l, int K, int N,
-                                                                int S_rows, bool vec) {
+                                                                int S_rows, bool vec, const F32Return ret) {
     // PT: 16-byte units of each operand per thread and slab
     constexpr int TM = 32 * R, KC = 128 / R * KG, NTH = 256 * KG, PT = TM * KC / 4 / NTH, STEPS = KC / 16 / KG;
     constexpr int PA = KC + 4, PB = TM + 16;
     constexpr bool UP = EPI == EPI_SWIGLU;
     extern __shared__ __align__(16) float slab[];
     float *const As = slab, *const Bs = As + TM * PA, *const Us = Bs + KC * PB;
-    __shared__ int s_g, s_row0, s_rv;
+    __shared__ int s_g, s_row0, s_rv, s_first;
+    __shared__ int32_t s_from[RET ? MOE_MAX_EXPERTS : 1], s_slot[RET ? MOE_MAX_EXPERTS : 1], s_to[RET ? TM : 1];
     const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+    if constexpr (RET) {
+        if ((int)blockIdx.y >= ret.tiles_y) {  // padding rows: a wave's share of all slots, slot by slot
+            const int waves = (gridDim.y - ret.tiles_y) * gridDim.x * (NTH / WAVE);
+            const int w0 = ((blockIdx.y - ret.tiles_y) * gridDim.x + blockIdx.x) * (NTH / WAVE) + wave;
+            for (int sr = 0; sr < ret.W; ++sr) {
+                int rows = 0;
+                for (int e = lane; e < E_l; e += WAVE) rows += ret.rc[sr * E_l + e];
+                rows = max(wave_sum(rows), 0);
+                for (int m = rows + w0; m < ret.M; m += waves)
+                    for (int c = lane; c < N; c += WAVE) ret.buf[((size_t)sr * ret.M + m) * N + c] = 0.f;
+            }
+            return;
+        }
+    }
     if (wave == 0) {  // which expert's rows: 64 experts at a time, tiles and rows before them by a scan
         int mt = blockIdx.y, rs = 0;
         if (lane == 0) s_g = -1;
@@ -1057,7 +1081,7 @@ __global__ __launch_bounds__(256 * KG) void grouped_gemm_f32_kernel(const float*
             const bool mine = mt < tiles && mt >= tiles - t;
             if (mine) {
                 const int first = (mt - (tiles - t)) * TM;
-                s_g = base + lane; s_row0 = r.start + first; s_rv = min(TM, r.n - first);
+                s_g = base + lane; s_row0 = r.start + first; s_rv = min(TM, r.n - first); s_first = first;
             }
             if (__ballot(mine)) break;
             mt -= wave_lane(tiles, WAVE - 1);
@@ -1070,6 +1094,24 @@ __global__ __launch_bounds__(256 * KG) void grouped_gemm_f32_kernel(const float*
     const int row0 = s_row0, rv = s_rv, n0 = blockIdx.x * TM;
     const float* W = Wt + (size_t)g * K * N;
     const float* U = UP ? Wup + (size_t)g * K * N : nullptr;
+    if constexpr (RET) {
+        // where the rows of every source start among the expert's, and among the slots of the returned buffer (read behind the K loop's first barrier)
+        if (wave == 0) {
+            int run = 0;
+            for (int base = 0; base < ret.W; base += WAVE) {
+                const int sr = base + lane;
+                int mine = 0, before = 0;
+                if (sr < ret.W) {
+                    mine = ret.rc[sr * E_l + g];
+#pragma unroll 8
+                    for (int e = 0; e < g; ++e) before += ret.rc[sr * E_l + e];
+                }
+                const int incl = wave_incl_scan(mine);
+                if (sr < ret.W) { s_from[sr] = run + incl - mine; s_slot[sr] = before; }
+                run += wave_lane(incl, WAVE - 1);
+            }
+        }
+    }
     float4 ra[PT], rb[PT], ru[UP ? PT : 1];
     // (vec: K, N and the bases allow 16-byte loads, so a unit lies wholly inside or outside)
     auto load = [&](const float* p, int at, int end) {
@@ -1113,6 +1155,17 @@ __global__ __launch_bounds__(256 * KG) void grouped_gemm_f32_kernel(const float*
         }
         __syncthreads();
         if (k0 + KC < K) fetch(k0 + KC);
+        if constexpr (RET)
+            if (k0 == 0 && (int)threadIdx.x < rv) {
+                const int r = s_first + (int)threadIdx.x;  // of the expert's rows
+                int lo = 0, hi = ret.W;  // (the last of a run of equal starts owns the row)
+                while (hi - lo > 1) {
+                    const int mid = (lo + hi) >> 1;
+                    if (s_from[mid] <= r) lo = mid; else hi = mid;
+                }
+                const int m = s_slot[lo] + r - s_from[lo];
+                s_to[threadIdx.x] = (unsigned)m < (unsigned)ret.M ? lo * ret.M + m : -1;  // (past the pair capacity: the row has no slot)
+            }
         // slab positions past K hold zeros: adding +0 products leaves every sum as it is
         const int steps = min(KC, K - k0 + 15) / 16 - half * STEPS;
         auto step = [&](int s4) {
@@ -1174,6 +1227,8 @@ __global__ __launch_bounds__(256 * KG) void grouped_gemm_f32_kernel(const float*
                 if constexpr (EPI == EPI_SILU) x = act_silu(x);
                 if constexpr (UP) x = act_silu(x) * acu[i][j][q];
                 C[(size_t)(row0 + r) * N + c] = x;
+                if constexpr (RET)
+                    if (s_to[r] >= 0) ret.buf[(size_t)s_to[r] * N + c] = x;
             }
 }
 
@@ -1646,7 +1701,7 @@ constexpr int gg_f32_lds(int R, int KG, bool up) {
     return (32 * R * (KC + 4) + (up ? 2 : 1) * KC * (32 * R + 16)) * 4;
 }
 int launch_f32(const float* A, const float* W, const float* U, float* C, const int32_t* cnt, int E_l, int K, int N, int S_rows,
-               int epi, hipStream_t s) {
+               int epi, hipStream_t s, F32Return ret = {}) {
     if (S_rows == 0) return MOE_OK;
     const bool vec = K % 4 == 0 && N % 4 == 0 && (((uintptr_t)A | (uintptr_t)W | (uintptr_t)U) & 15) == 0;
     // 64 x 64 tiles once they give every compute unit two workgroups, 32 x 32 below
@@ -1656,8 +1711,16 @@ int launch_f32(const float* A, const float* W, const float* U, float* C, const i
     // Two sets of waves to a tile up to two workgroups a compute unit (half a tile per group more than the rows fill): 344 tiles, K 1000
     // 30.4 -> 21.7 us, but 832 tiles, K 1024 51.5 -> 58.0 (one such workgroup fits a compute unit, three of the others do).
     const bool split = !big && K > 128 && (long long)ceil_div(N, 32) * (ceil_div(S_rows, 32) + E_l / 2) <= 2 * num_cus();
+    // (a workgroup for every 16 rows of the returned buffer that S_rows cannot fill, up to a round of the chip)
+    ret.tiles_y = grid.y;
+    if (ret.buf) grid.y += std::min(ceil_div(std::max(ret.W * ret.M - S_rows, 1), 16 * (int)grid.x), ceil_div(num_cus(), (int)grid.x));
+#define GG_F32_L(EPI, R, KG, RET)                                                                                                    \
+    grouped_gemm_f32_kernel<EPI, R, KG, RET><<<grid, 256 * KG, gg_f32_lds(R, KG, EPI == EPI_SWIGLU), s>>>(A, W, U, C, cnt, E_l, K, N, S_rows, vec, ret)
 #define GG_F32_K(EPI, R, KG)                                                                                                         \
-    grouped_gemm_f32_kernel<EPI, R, KG><<<grid, 256 * KG, gg_f32_lds(R, KG, EPI == EPI_SWIGLU), s>>>(A, W, U, C, cnt, E_l, K, N, S_rows, vec)
+    do {                                                                                                                             \
+        if (EPI == EPI_NONE && ret.buf) GG_F32_L(EPI_NONE, R, KG, true);                                                             \
+        else GG_F32_L(EPI, R, KG, false);                                                                                            \
+    } while (0)
 #define GG_F32(EPI)                                                                                                                  \
     case EPI:                                                                                                                        \
         if (big) GG_F32_K(EPI, 2, 1);                                                                                                \
@@ -1673,6 +1736,7 @@ int launch_f32(const float* A, const float* W, const float* U, float* C, const i
     }
 #undef GG_F32
 #undef GG_F32_K
+#undef GG_F32_L
     return moe_check_launch("grouped_gemm_f32");
 }
 
@@ -1872,6 +1936,20 @@ extern "C" int moe_grouped_mlp(const void* tokens, const int32_t* expert_cnt, in
                                int act, const void* w1, const void* w_up, const void* w2, void* hidden_ws, void* out,
                                moe_stream_t stream) {
     return moe_grouped_mlp_split(tokens, expert_cnt, dtype, S_rows, H, F, E_l, act, w1, w_up, w2, hidden_ws, out, nullptr, 0, stream);
+}
+
+int moe_mlp_f32_return(const float* tokens, const int32_t* expert_cnt, int S_rows, int H, int F, int E_l, int act, const float* w1,
+                       const float* w_up, const float* w2, float* hidden_ws, float* y, const int32_t* recv_counts, int W, int M, float* ret,
+                       hipStream_t s) {
+    MOE_REQUIRE(S_rows > 0 && H > 0 && F > 0 && E_l > 0 && E_l <= GG_MAXG, MOE_ERR_INVALID, "grouped_mlp: bad shape");
+    MOE_REQUIRE(act == EPI_GELU || act == EPI_SILU || act == EPI_SWIGLU || act == EPI_NONE, MOE_ERR_INVALID,
+                "grouped_mlp: activation %d", act);
+    MOE_REQUIRE(tokens && expert_cnt && w1 && w2 && hidden_ws && y && (act != EPI_SWIGLU || w_up), MOE_ERR_INVALID, "grouped_mlp: null pointer");
+    MOE_REQUIRE(W > 0 && W * E_l <= MOE_MAX_EXPERTS && M >= 1 && recv_counts && ret, MOE_ERR_INVALID, "return_pack: bad arguments");
+    MOE_REQUIRE((long long)W * M < (1ll << 31), MOE_ERR_UNSUPPORTED, "return_pack: W*M too large");
+    const int rc = launch_f32(tokens, w1, w_up, hidden_ws, expert_cnt, E_l, H, F, S_rows, act, s);
+    if (rc) return rc;
+    return launch_f32(hidden_ws, w2, nullptr, y, expert_cnt, E_l, F, H, S_rows, EPI_NONE, s, {recv_counts, W, M, ret, 0});
 }
 
 extern "C" int moe_grouped_mlp_split(const void* tokens, const int32_t* expert_cnt, int dtype, int S_rows, int H, int F, int E_l,

@@ -117,6 +117,33 @@ def test_step_as_one_call_equals_its_stages(name, mode):
         assert torch.equal(one[n], stages[n]), f"{n} differs"
 
 
+@pytest.mark.parametrize("T,H,E,k,W,F,act,cut", [(37, 128, 8, 2, 4, 260, "gelu", 0), (5, 36, 3, 1, 1, 100, "silu", 0), (300, 256, 130, 2, 65, 512, "silu", 3),
+                                                 (2000, 132, 24, 4, 8, 200, "gelu", 40), (700, 512, 12, 2, 2, 1024, "silu", 1), (4, 64, 16, 1, 4, 64, "gelu", 0)])
+def test_fp32_results_go_to_their_slots_from_the_gemm(T, H, E, k, W, F, act, cut):
+    """A step of fp32 experts writes y and the returned buffer in one launch; stage by stage a copy follows the GEMMs.  Tiles of 32 and 64 rows, one
+    and two sets of waves, sources without rows, and (cut) rows past the pair capacity, which have no slot."""
+    from iris_testing_amd.configs import MoEConfig
+    from iris_testing_amd.pipeline import DispatchPipeline
+    cfg = MoEConfig("case", T, T, H, "f32", E, k, W, F, act)
+    world = harness.build_world(cfg, DEV)
+    if cut:
+        M = max(world.M - cut, 1)
+        world.M, world.recv = M, world.recv[:, :M].contiguous()
+    ew, _, _ = harness.expert_weights(cfg, 0, DEV)
+    pipe = DispatchPipeline(world, ew)
+    names = "expert_cnt rows hidden y ret".split()
+
+    def results(events):
+        for n in names:
+            getattr(pipe, n).fill_(3)
+        pipe.step(events)
+        torch.cuda.synchronize()
+        return {n: getattr(pipe, n).clone() for n in names}
+    one, stages = results(None), results([])
+    for n in names:
+        assert torch.equal(one[n], stages[n]), f"{n} differs"
+
+
 def test_entry_point_smoke_runs():
     """The smoke check of the repository's entry module (one small step against the oracle) must keep passing."""
     import importlib
