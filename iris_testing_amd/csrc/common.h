@@ -15,10 +15,10 @@ char* moe_err_buf();
 int moe_fail(int code, const char* fmt, ...);
 int moe_check_launch(const char* what);
 
-// grouped_gemm.hip, for step.hip: moe_grouped_mlp of fp32 rows and moe_return_pack of its result in two launches (S_rows > 0)
-int moe_mlp_f32_return(const float* tokens, const int32_t* expert_cnt, int S_rows, int H, int F, int E_l, int act, const float* w1,
-                       const float* w_up, const float* w2, float* hidden_ws, float* y, const int32_t* recv_counts, int W, int M, float* ret,
-                       hipStream_t s);
+// grouped_gemm.hip, for step.hip: moe_unpack_expert_major of fp32 rows, moe_grouped_mlp and moe_return_pack, in two launches where tiles are small (S_rows > 0)
+int moe_mlp_f32_slots(const float* recv, const int32_t* recv_counts, int W, int M, int S_rows, int H, int F, int E_l, int act, const float* w1,
+                      const float* w_up, const float* w2, float* rows, int32_t* expert_cnt, float* hidden_ws, float* y, float* ret,
+                      hipStream_t s);
 
 #define MOE_REQUIRE(cond, code, ...)                 \
     do {                                             \

@@ -1034,20 +1034,25 @@ __global__ void zero_pad_rows_kernel(T* __restrict__ out, int K, int Nreal, int 
 // R = 2 for launches of many tiles: every operand value out of LDS feeds two matrix instructions.
 // A in LDS as [row][k % 4][k / 4]: the four values a lane needs in four consecutive steps are one 16-byte read; B as
 // [k][column], rows padded so that the four k of a step lie in different banks.
-// RET: result rows go to their slots of the returned [W,M,N] buffer as well, and the workgroups from ret.tiles_y on zero its padding rows: a
-// launch that only copied the rows took 2.5 us of the 43 of the plumbing step.  The tile's rows belong to one expert, whose slots
-// start at the sums of the received counts before it.
-struct F32Return {
+// SIDE: the copy of the rows beside the GEMM.  F32_RETURN: result rows go to their slots of the returned [W,M,N] buffer as well, and the
+// workgroups from side.tiles_y on zero its padding rows.  F32_UNPACK: the rows come from their slots of the received [W,M,K] buffer, and the workgroups
+// of the first columns leave them in expert-major order in side.rows (zeros for rows past the pair capacity, and past the total), and the counts
+// per expert in side.cnt.  As launches of their own the two copies took 2.5 and 3 us of the 43 of the plumbing step.  A tile's rows belong to one
+// expert, whose slots start at the sums of the received counts before it.
+enum { F32_ROWS = 0, F32_RETURN = 1, F32_UNPACK = 2 };
+struct F32Side {
     const int32_t* rc;  // received counts [W,E_l]
     int W, M;
-    float* buf;
+    float* buf;         // [W,M,...]: written (F32_RETURN) or read
     int tiles_y;
+    float* rows;
+    int32_t* cnt;
 };
-template <int EPI, int R, int KG, bool RET = false>
+template <int EPI, int R, int KG, int SIDE = F32_ROWS>
 __global__ __launch_bounds__(256 * KG) void grouped_gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ Wt,
                                                                 const float* __restrict__ Wup, float* __restrict__ C,
                                                                 const int32_t* __restrict__ cnt, int E_l, int K, int N,
-                                                                int S_rows, bool vec, const F32Return ret) {
+                                                                int S_rows, bool vec, const F32Side side) {
     // PT: 16-byte units of each operand per thread and slab
     constexpr int TM = 32 * R, KC = 128 / R * KG, NTH = 256 * KG, PT = TM * KC / 4 / NTH, STEPS = KC / 16 / KG;
     constexpr int PA = KC + 4, PB = TM + 16;
@@ -1055,27 +1060,43 @@ __global__ __launch_bounds__(256 * KG) void grouped_gemm_f32_kernel(const float*
     extern __shared__ __align__(16) float slab[];
     float *const As = slab, *const Bs = As + TM * PA, *const Us = Bs + KC * PB;
     __shared__ int s_g, s_row0, s_rv, s_first;
-    __shared__ int32_t s_from[RET ? MOE_MAX_EXPERTS : 1], s_slot[RET ? MOE_MAX_EXPERTS : 1], s_to[RET ? TM : 1];
+    constexpr bool RET = SIDE == F32_RETURN, SRC = SIDE == F32_UNPACK;
+    __shared__ int32_t s_from[SIDE ? MOE_MAX_EXPERTS : 1], s_slot[SIDE ? MOE_MAX_EXPERTS : 1], s_at[SIDE ? TM : 1];
+    __shared__ int32_t s_rc[SRC ? MOE_MAX_EXPERTS : 1], s_cnt[SRC ? MOE_MAX_EXPERTS : 1];
     const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
     if constexpr (RET) {
-        if ((int)blockIdx.y >= ret.tiles_y) {  // padding rows: a wave's share of all slots, slot by slot
-            const int waves = (gridDim.y - ret.tiles_y) * gridDim.x * (NTH / WAVE);
-            const int w0 = ((blockIdx.y - ret.tiles_y) * gridDim.x + blockIdx.x) * (NTH / WAVE) + wave;
-            for (int sr = 0; sr < ret.W; ++sr) {
+        if ((int)blockIdx.y >= side.tiles_y) {  // padding rows: a wave's share of all slots, slot by slot
+            const int waves = (gridDim.y - side.tiles_y) * gridDim.x * (NTH / WAVE);
+            const int w0 = ((blockIdx.y - side.tiles_y) * gridDim.x + blockIdx.x) * (NTH / WAVE) + wave;
+            for (int sr = 0; sr < side.W; ++sr) {
                 int rows = 0;
-                for (int e = lane; e < E_l; e += WAVE) rows += ret.rc[sr * E_l + e];
+                for (int e = lane; e < E_l; e += WAVE) rows += side.rc[sr * E_l + e];
                 rows = max(wave_sum(rows), 0);
-                for (int m = rows + w0; m < ret.M; m += waves)
-                    for (int c = lane; c < N; c += WAVE) ret.buf[((size_t)sr * ret.M + m) * N + c] = 0.f;
+                for (int m = rows + w0; m < side.M; m += waves)
+                    for (int c = lane; c < N; c += WAVE) side.buf[((size_t)sr * side.M + m) * N + c] = 0.f;
             }
             return;
         }
     }
+    if constexpr (SRC) {
+        for (int i = threadIdx.x; i < side.W * E_l; i += NTH) s_rc[i] = side.rc[i];
+        __syncthreads();
+        for (int e = threadIdx.x; e < E_l; e += NTH) {
+            int c = 0;
+            for (int sr = 0; sr < side.W; ++sr) c += s_rc[sr * E_l + e];
+            s_cnt[e] = c;
+            if (blockIdx.x + blockIdx.y == 0) side.cnt[e] = c;
+        }
+        __syncthreads();
+    }
+    const int32_t* const counts = SRC ? s_cnt : cnt;
+    const int32_t* const rc = SRC ? s_rc : side.rc;
     if (wave == 0) {  // which expert's rows: 64 experts at a time, tiles and rows before them by a scan
         int mt = blockIdx.y, rs = 0;
+        bool found = false;
         if (lane == 0) s_g = -1;
         for (int base = 0; base < E_l; base += WAVE) {
-            const GgRows r = gg_rows<true>(cnt, base + lane, E_l, rs, S_rows);
+            const GgRows r = gg_rows<true>(counts, base + lane, E_l, rs, S_rows);
             const int t = (r.n + TM - 1) / TM;
             const int tiles = wave_incl_scan(t);
             const bool mine = mt < tiles && mt >= tiles - t;
@@ -1083,33 +1104,52 @@ __global__ __launch_bounds__(256 * KG) void grouped_gemm_f32_kernel(const float*
                 const int first = (mt - (tiles - t)) * TM;
                 s_g = base + lane; s_row0 = r.start + first; s_rv = min(TM, r.n - first); s_first = first;
             }
-            if (__ballot(mine)) break;
+            if (__ballot(mine)) { found = true; break; }
             mt -= wave_lane(tiles, WAVE - 1);
             rs = r.end;
         }
+        // (the workgroups behind the tiles are as many as the rows behind the total, and more)
+        if (SRC && lane == 0 && !found) { s_row0 = rs + mt * TM; s_rv = min(TM, S_rows - s_row0); }
     }
     __syncthreads();
     const int g = s_g;
+    if (SRC && g < 0 && blockIdx.x == 0)
+        for (int i = threadIdx.x; i < s_rv * K; i += NTH) side.rows[(size_t)s_row0 * K + i] = 0.f;
     if (g < 0 || s_rv <= 0) return;
     const int row0 = s_row0, rv = s_rv, n0 = blockIdx.x * TM;
     const float* W = Wt + (size_t)g * K * N;
     const float* U = UP ? Wup + (size_t)g * K * N : nullptr;
-    if constexpr (RET) {
-        // where the rows of every source start among the expert's, and among the slots of the returned buffer (read behind the K loop's first barrier)
+    auto place = [&](int i) {  // row i of the tile: its slot
+        const int r = s_first + i;  // of the expert's rows
+        int lo = 0, hi = side.W;    // (the last of a run of equal starts owns the row)
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if (s_from[mid] <= r) lo = mid; else hi = mid;
+        }
+        const int m = s_slot[lo] + r - s_from[lo];
+        s_at[i] = (unsigned)m < (unsigned)side.M ? lo * side.M + m : -1;  // (past the pair capacity: the row has no slot)
+    };
+    if constexpr (SIDE != F32_ROWS) {
+        // where the rows of every source start among the expert's, and among the slots
         if (wave == 0) {
             int run = 0;
-            for (int base = 0; base < ret.W; base += WAVE) {
+            for (int base = 0; base < side.W; base += WAVE) {
                 const int sr = base + lane;
                 int mine = 0, before = 0;
-                if (sr < ret.W) {
-                    mine = ret.rc[sr * E_l + g];
+                if (sr < side.W) {
+                    mine = rc[sr * E_l + g];
 #pragma unroll 8
-                    for (int e = 0; e < g; ++e) before += ret.rc[sr * E_l + e];
+                    for (int e = 0; e < g; ++e) before += rc[sr * E_l + e];
                 }
                 const int incl = wave_incl_scan(mine);
-                if (sr < ret.W) { s_from[sr] = run + incl - mine; s_slot[sr] = before; }
+                if (sr < side.W) { s_from[sr] = run + incl - mine; s_slot[sr] = before; }
                 run += wave_lane(incl, WAVE - 1);
             }
+        }
+        if constexpr (SRC) {
+            __syncthreads();
+            if ((int)threadIdx.x < rv) place(threadIdx.x);
+            __syncthreads();
         }
     }
     float4 ra[PT], rb[PT], ru[UP ? PT : 1];
@@ -1131,7 +1171,12 @@ __global__ __launch_bounds__(256 * KG) void grouped_gemm_f32_kernel(const float*
         for (int q = 0; q < PT; ++q) {
             const int i = threadIdx.x + q * NTH;
             const int r = i / (KC / 4), k4 = i % (KC / 4);     // A: consecutive threads walk K
-            ra[q] = load(A + (size_t)(row0 + min(r, rv - 1)) * K, k0 + 4 * k4, r < rv ? K : 0);
+            if constexpr (SRC) {
+                const int at = s_at[min(r, rv - 1)];
+                ra[q] = load(side.buf + (size_t)max(at, 0) * K, k0 + 4 * k4, r < rv && at >= 0 ? K : 0);
+            } else {
+                ra[q] = load(A + (size_t)(row0 + min(r, rv - 1)) * K, k0 + 4 * k4, r < rv ? K : 0);
+            }
             const int kb = i / (TM / 4), n4 = i % (TM / 4);     // W: consecutive threads walk N
             const size_t row = (size_t)min(k0 + kb, K - 1) * N;
             const int end = k0 + kb < K ? N : 0;
@@ -1148,6 +1193,10 @@ __global__ __launch_bounds__(256 * KG) void grouped_gemm_f32_kernel(const float*
         for (int q = 0; q < PT; ++q) {
             const int i = threadIdx.x + q * NTH;
             float* a = As + (i / (KC / 4)) * PA + i % (KC / 4);
+            if constexpr (SRC) {  // (rows are multiples of 16 bytes)
+                const int r = i / (KC / 4), k = k0 + i % (KC / 4) * 4;
+                if (blockIdx.x == 0 && r < rv && k < K) *reinterpret_cast<float4*>(side.rows + (size_t)(row0 + r) * K + k) = ra[q];
+            }
             a[0] = ra[q].x; a[KC / 4] = ra[q].y; a[2 * (KC / 4)] = ra[q].z; a[3 * (KC / 4)] = ra[q].w;
             const int b = (i / (TM / 4)) * PB + (i % (TM / 4)) * 4;
             *reinterpret_cast<float4*>(Bs + b) = rb[q];
@@ -1156,16 +1205,7 @@ __global__ __launch_bounds__(256 * KG) void grouped_gemm_f32_kernel(const float*
         __syncthreads();
         if (k0 + KC < K) fetch(k0 + KC);
         if constexpr (RET)
-            if (k0 == 0 && (int)threadIdx.x < rv) {
-                const int r = s_first + (int)threadIdx.x;  // of the expert's rows
-                int lo = 0, hi = ret.W;  // (the last of a run of equal starts owns the row)
-                while (hi - lo > 1) {
-                    const int mid = (lo + hi) >> 1;
-                    if (s_from[mid] <= r) lo = mid; else hi = mid;
-                }
-                const int m = s_slot[lo] + r - s_from[lo];
-                s_to[threadIdx.x] = (unsigned)m < (unsigned)ret.M ? lo * ret.M + m : -1;  // (past the pair capacity: the row has no slot)
-            }
+            if (k0 == 0 && (int)threadIdx.x < rv) place(threadIdx.x);  // (read behind the barrier below)
         // slab positions past K hold zeros: adding +0 products leaves every sum as it is
         const int steps = min(KC, K - k0 + 15) / 16 - half * STEPS;
         auto step = [&](int s4) {
@@ -1228,7 +1268,7 @@ __global__ __launch_bounds__(256 * KG) void grouped_gemm_f32_kernel(const float*
                 if constexpr (UP) x = act_silu(x) * acu[i][j][q];
                 C[(size_t)(row0 + r) * N + c] = x;
                 if constexpr (RET)
-                    if (s_to[r] >= 0) ret.buf[(size_t)s_to[r] * N + c] = x;
+                    if (s_at[r] >= 0) side.buf[(size_t)s_at[r] * N + c] = x;
             }
 }
 
@@ -1700,30 +1740,32 @@ constexpr int gg_f32_lds(int R, int KG, bool up) {
     const int KC = 128 / R * KG;
     return (32 * R * (KC + 4) + (up ? 2 : 1) * KC * (32 * R + 16)) * 4;
 }
+// 64 x 64 tiles once they give every compute unit two workgroups, 32 x 32 below
+bool gg_f32_big(int S_rows, int N) { return (long long)ceil_div(N, 64) * ceil_div(S_rows, 64) >= 2 * num_cus(); }
 int launch_f32(const float* A, const float* W, const float* U, float* C, const int32_t* cnt, int E_l, int K, int N, int S_rows,
-               int epi, hipStream_t s, F32Return ret = {}) {
+               int epi, hipStream_t s, int side = F32_ROWS, F32Side sd = {}) {
     if (S_rows == 0) return MOE_OK;
-    const bool vec = K % 4 == 0 && N % 4 == 0 && (((uintptr_t)A | (uintptr_t)W | (uintptr_t)U) & 15) == 0;
-    // 64 x 64 tiles once they give every compute unit two workgroups, 32 x 32 below
-    const bool big = (long long)ceil_div(N, 64) * ceil_div(S_rows, 64) >= 2 * num_cus();
+    const bool vec = K % 4 == 0 && N % 4 == 0 && (((uintptr_t)(side == F32_UNPACK ? sd.buf : A) | (uintptr_t)W | (uintptr_t)U) & 15) == 0;
+    const bool big = gg_f32_big(S_rows, N);
     const int tile = big ? 64 : 32;
     dim3 grid(ceil_div(N, tile), ceil_div(S_rows, tile) + E_l);
     // Two sets of waves to a tile up to two workgroups a compute unit (half a tile per group more than the rows fill): 344 tiles, K 1000
     // 30.4 -> 21.7 us, but 832 tiles, K 1024 51.5 -> 58.0 (one such workgroup fits a compute unit, three of the others do).
     const bool split = !big && K > 128 && (long long)ceil_div(N, 32) * (ceil_div(S_rows, 32) + E_l / 2) <= 2 * num_cus();
     // (a workgroup for every 16 rows of the returned buffer that S_rows cannot fill, up to a round of the chip)
-    ret.tiles_y = grid.y;
-    if (ret.buf) grid.y += std::min(ceil_div(std::max(ret.W * ret.M - S_rows, 1), 16 * (int)grid.x), ceil_div(num_cus(), (int)grid.x));
-#define GG_F32_L(EPI, R, KG, RET)                                                                                                    \
-    grouped_gemm_f32_kernel<EPI, R, KG, RET><<<grid, 256 * KG, gg_f32_lds(R, KG, EPI == EPI_SWIGLU), s>>>(A, W, U, C, cnt, E_l, K, N, S_rows, vec, ret)
+    sd.tiles_y = grid.y;
+    if (side == F32_RETURN) grid.y += std::min(ceil_div(std::max(sd.W * sd.M - S_rows, 1), 16 * (int)grid.x), ceil_div(num_cus(), (int)grid.x));
+#define GG_F32_L(EPI, R, KG, SIDE)                                                                                                   \
+    grouped_gemm_f32_kernel<EPI, R, KG, SIDE><<<grid, 256 * KG, gg_f32_lds(R, KG, EPI == EPI_SWIGLU), s>>>(A, W, U, C, cnt, E_l, K, N, S_rows, vec, sd)
 #define GG_F32_K(EPI, R, KG)                                                                                                         \
     do {                                                                                                                             \
-        if (EPI == EPI_NONE && ret.buf) GG_F32_L(EPI_NONE, R, KG, true);                                                             \
-        else GG_F32_L(EPI, R, KG, false);                                                                                            \
+        if (side == F32_UNPACK) GG_F32_L(EPI, R, KG, F32_UNPACK);                                                                    \
+        else if (EPI == EPI_NONE && side == F32_RETURN) GG_F32_L(EPI_NONE, R, KG, F32_RETURN);                                       \
+        else GG_F32_L(EPI, R, KG, F32_ROWS);                                                                                         \
     } while (0)
 #define GG_F32(EPI)                                                                                                                  \
     case EPI:                                                                                                                        \
-        if (big) GG_F32_K(EPI, 2, 1);                                                                                                \
+        if (big) GG_F32_L(EPI, 2, 1, F32_ROWS);                                                                                      \
         else if (split) GG_F32_K(EPI, 1, 2);                                                                                         \
         else GG_F32_K(EPI, 1, 1);                                                                                                    \
         break
@@ -1938,18 +1980,26 @@ extern "C" int moe_grouped_mlp(const void* tokens, const int32_t* expert_cnt, in
     return moe_grouped_mlp_split(tokens, expert_cnt, dtype, S_rows, H, F, E_l, act, w1, w_up, w2, hidden_ws, out, nullptr, 0, stream);
 }
 
-int moe_mlp_f32_return(const float* tokens, const int32_t* expert_cnt, int S_rows, int H, int F, int E_l, int act, const float* w1,
-                       const float* w_up, const float* w2, float* hidden_ws, float* y, const int32_t* recv_counts, int W, int M, float* ret,
-                       hipStream_t s) {
-    MOE_REQUIRE(S_rows > 0 && H > 0 && F > 0 && E_l > 0 && E_l <= GG_MAXG, MOE_ERR_INVALID, "grouped_mlp: bad shape");
+int moe_mlp_f32_slots(const float* recv, const int32_t* recv_counts, int W, int M, int S_rows, int H, int F, int E_l, int act, const float* w1,
+                      const float* w_up, const float* w2, float* rows, int32_t* expert_cnt, float* hidden_ws, float* y, float* ret,
+                      hipStream_t s) {
+    MOE_REQUIRE(S_rows > 0 && H > 0 && H % 4 == 0 && F > 0 && E_l > 0 && E_l <= GG_MAXG, MOE_ERR_INVALID, "grouped_mlp: bad shape");
     MOE_REQUIRE(act == EPI_GELU || act == EPI_SILU || act == EPI_SWIGLU || act == EPI_NONE, MOE_ERR_INVALID,
                 "grouped_mlp: activation %d", act);
-    MOE_REQUIRE(tokens && expert_cnt && w1 && w2 && hidden_ws && y && (act != EPI_SWIGLU || w_up), MOE_ERR_INVALID, "grouped_mlp: null pointer");
+    MOE_REQUIRE(recv && rows && expert_cnt && w1 && w2 && hidden_ws && y && (act != EPI_SWIGLU || w_up), MOE_ERR_INVALID, "grouped_mlp: null pointer");
     MOE_REQUIRE(W > 0 && W * E_l <= MOE_MAX_EXPERTS && M >= 1 && recv_counts && ret, MOE_ERR_INVALID, "return_pack: bad arguments");
     MOE_REQUIRE((long long)W * M < (1ll << 31), MOE_ERR_UNSUPPORTED, "return_pack: W*M too large");
-    const int rc = launch_f32(tokens, w1, w_up, hidden_ws, expert_cnt, E_l, H, F, S_rows, act, s);
+    // (with large tiles the rows' places, looked up slab by slab, cost more than the copies: H 512, F 1024, 54 940 rows 1443 -> 1635 us a step, 14 613 456 -> 480)
+    const bool up = !gg_f32_big(S_rows, F), down = !gg_f32_big(S_rows, H);
+    int rc = up ? MOE_OK : moe_unpack_expert_major(recv, MOE_F32, W, M, H, recv_counts, E_l, rows, S_rows, expert_cnt, nullptr, s);
     if (rc) return rc;
-    return launch_f32(hidden_ws, w2, nullptr, y, expert_cnt, E_l, F, H, S_rows, EPI_NONE, s, {recv_counts, W, M, ret, 0});
+    rc = launch_f32(rows, w1, w_up, hidden_ws, expert_cnt, E_l, H, F, S_rows, act, s, up ? F32_UNPACK : F32_ROWS,
+                    {recv_counts, W, M, const_cast<float*>(recv), 0, rows, expert_cnt});
+    if (rc) return rc;
+    rc = launch_f32(hidden_ws, w2, nullptr, y, expert_cnt, E_l, F, H, S_rows, EPI_NONE, s, down ? F32_RETURN : F32_ROWS,
+                    {recv_counts, W, M, ret, 0, nullptr, nullptr});
+    if (rc || down) return rc;
+    return moe_return_pack(y, MOE_F32, S_rows, H, recv_counts, W, E_l, M, ret, nullptr, s);
 }
 
 extern "C" int moe_grouped_mlp_split(const void* tokens, const int32_t* expert_cnt, int dtype, int S_rows, int H, int F, int E_l,

@@ -118,15 +118,17 @@ def test_step_as_one_call_equals_its_stages(name, mode):
 
 
 @pytest.mark.parametrize("T,H,E,k,W,F,act,cut", [(37, 128, 8, 2, 4, 260, "gelu", 0), (5, 36, 3, 1, 1, 100, "silu", 0), (300, 256, 130, 2, 65, 512, "silu", 3),
-                                                 (2000, 132, 24, 4, 8, 200, "gelu", 40), (700, 512, 12, 2, 2, 1024, "silu", 1), (4, 64, 16, 1, 4, 64, "gelu", 0)])
-def test_fp32_results_go_to_their_slots_from_the_gemm(T, H, E, k, W, F, act, cut):
-    """A step of fp32 experts writes y and the returned buffer in one launch; stage by stage a copy follows the GEMMs.  Tiles of 32 and 64 rows, one
-    and two sets of waves, sources without rows, and (cut) rows past the pair capacity, which have no slot."""
+                                                 (2000, 132, 24, 4, 8, 200, "gelu", 40), (700, 512, 12, 2, 2, 1024, "silu", 1), (4, 64, 16, 1, 4, 64, "gelu", 0), (40, 252, 8, 2, 2, 130, "swiglu", -70)])
+def test_fp32_rows_come_from_and_go_to_their_slots_in_the_gemms(T, H, E, k, W, F, act, cut):
+    """In a step the GEMMs of fp32 experts move the rows; stage by stage copies stand before and behind them.  Tiles of 32 and 64 rows, one and
+    two sets of waves, sources without rows, (cut > 0) rows past the pair capacity, which have no slot, (cut < 0) rows behind the total."""
     from iris_testing_amd.configs import MoEConfig
     from iris_testing_amd.pipeline import DispatchPipeline
     cfg = MoEConfig("case", T, T, H, "f32", E, k, W, F, act)
     world = harness.build_world(cfg, DEV)
-    if cut:
+    if cut < 0:
+        world.S -= cut
+    if cut > 0:
         M = max(world.M - cut, 1)
         world.M, world.recv = M, world.recv[:, :M].contiguous()
     ew, _, _ = harness.expert_weights(cfg, 0, DEV)
