@@ -126,6 +126,117 @@ __global__ __launch_bounds__(SCAN_E * SCAN_SLICES) void scan_hist_kernel(const i
     if (sl == 0) base[(size_t)NG * E + e] = sum[c][SCAN_SLICES];
 }
 
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+constexpr int PACK_ZR = 8;  // consecutive slots of a [W,M,row] buffer that a wave looks through for padding (see pack_tokens_kernel)
+
+
+// rows [size_s, M) of every slot s of a [W,M,row] buffer <- 0, size_s = sum over e of rc[s,e]; one wave per run of
+// PACK_ZR consecutive rows (the slot's size is summed once per run, or twice when the run crosses into the next slot)
+__device__ __forceinline__ int slot_size(const int32_t* __restrict__ rc, int s, int E_l, int lane) {
+    int size = 0;
+    for (int e = lane; e < E_l; e += WAVE) size += rc[s * E_l + e];
+    return wave_sum(size);
+}
+__device__ __forceinline__ void zero_padding_rows(u32x4* __restrict__ buf, const int32_t* __restrict__ rc, int W, int E_l, int M,
+                                                  int row_vecs, int block) {
+    const int wave = threadIdx.x / WAVE, lane = lane_id();
+    const int r0 = (block * (blockDim.x / WAVE) + wave) * PACK_ZR, r1 = min(r0 + PACK_ZR, W * M);
+    if (r0 >= r1) return;
+    int s = r0 / M, m = r0 % M;
+    int size = slot_size(rc, s, E_l, lane);
+    const u32x4 z = {0u, 0u, 0u, 0u};
+    for (int r = r0; r < r1; ++r) {
+        if (m >= size) {
+            u32x4* row = buf + (size_t)r * row_vecs;
+            for (int c = lane; c < row_vecs; c += WAVE) __builtin_nontemporal_store(z, row + c);
+        }
+        if (++m == M && r + 1 < r1) { m = 0; size = slot_size(rc, ++s, E_l, lane); }
+    }
+}
+
+// Expert-major row r of the receive side -> row of the [W,M,H] buffer that holds it (one thread per row, binary search in
+// the (expert, source)-major prefix).  The same index serves the way back: the result row of r returns to the slot its input
+// came from.  Rows past the received total map to row 0; rows the pack dropped (position in the sender's slot at or past
+// the pair capacity M) map to -1: the GEMMs read row 0 for them and store nothing.
+// One launch: every block derives the two prefix tables it needs from recv_counts in LDS (at most
+// MOE_MAX_EXPERTS entries: a wave's scan) instead of waiting for a table kernel; block 0 also leaves the per-expert totals.
+// M = 0: the receive buffer is a padding-free flat payload instead (source-major, expert-minor blocks, the layout
+// reorder_flat_to_token_buf of the reference reads, baseline.py:204-218): the row of (e, s, j) is the exclusive prefix of the
+// counts over flattened (s, e) plus j, and no row can have been dropped.
+// recv_gate / row_gate (both or neither): the gates that arrived with the rows, [rows of the receive buffer], gathered
+// into expert-major order for the GEMM that applies them (0 for rows without a source).  recv_scale / row_scale likewise: the
+// fp8 row scales (rows without a source take that of row 0, whose codes the GEMM reads for them).
+// zbuf (or NULL): the blocks from map_blocks on zero the padding rows of that [W,M,row_vecs] buffer, which depend on the same counts.
+// A launch of its own (256 threads to a block) or, in a step, blocks beside the ranking's (1024).
+struct RecvPrepare {
+    const int32_t* rc;
+    int W, E_l, M, n_rows;
+    int32_t *map, *expert_cnt;
+    const float* recv_gate;
+    float* row_gate;
+    const float* recv_scale;
+    float* row_scale;
+    u32x4* zbuf;
+    int row_vecs, map_blocks;
+};
+__device__ __forceinline__ void recv_prepare_block(const RecvPrepare& a, int block, int32_t* s_row_off /* [MOE_MAX_EXPERTS + 1] */, int32_t* s_src_off) {
+    if (block >= a.map_blocks) {
+        zero_padding_rows(a.zbuf, a.rc, a.W, a.E_l, a.M, a.row_vecs, block - a.map_blocks);
+        return;
+    }
+    const int n = a.W * a.E_l;
+    const bool flat = a.M == 0;
+    if (threadIdx.x < WAVE) {
+        const int lane = lane_id();
+        const int per = (n + WAVE - 1) / WAVE;
+        const int lo = min(lane * per, n), hi = min(lo + per, n);
+        int sum = 0;
+        for (int i = lo; i < hi; ++i) sum += a.rc[(i % a.W) * a.E_l + (i / a.W)];
+        const int incl = wave_incl_scan(sum);
+        int run = incl - sum;
+        for (int i = lo; i < hi; ++i) { s_row_off[i] = run; run += a.rc[(i % a.W) * a.E_l + (i / a.W)]; }
+        if (lane == WAVE - 1) s_row_off[n] = incl;
+        if (flat) {  // exclusive prefix over flattened (s, e): where the block of (s, e) starts in the flat payload
+            int fsum = 0;
+            for (int i = lo; i < hi; ++i) fsum += a.rc[i];
+            const int fincl = wave_incl_scan(fsum);
+            int frun = fincl - fsum;
+            for (int i = lo; i < hi; ++i) { s_src_off[i] = frun; frun += a.rc[i]; }
+        } else {
+            for (int sr = lane; sr < a.W; sr += WAVE) {
+                int r = 0;
+                for (int e = 0; e < a.E_l; ++e) { s_src_off[sr * a.E_l + e] = r; r += a.rc[sr * a.E_l + e]; }
+            }
+        }
+        if (block == 0 && a.expert_cnt)
+            for (int e = lane; e < a.E_l; e += WAVE) {
+                int c = 0;
+                for (int sr = 0; sr < a.W; ++sr) c += a.rc[sr * a.E_l + e];
+                a.expert_cnt[e] = c;
+            }
+    }
+    __syncthreads();
+    const int r = block * blockDim.x + threadIdx.x;
+    if (r >= a.n_rows) return;
+    if (r >= s_row_off[n]) {
+        a.map[r] = 0;
+        if (a.row_gate) a.row_gate[r] = 0.f;
+        if (a.row_scale) a.row_scale[r] = a.recv_scale[0];
+        return;
+    }
+    int lo = 0, hi = n;  // s_row_off[0] = 0 <= r; the last of a run of equal offsets owns the row
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (s_row_off[mid] <= r) lo = mid; else hi = mid;
+    }
+    const int e = lo / a.W, sr = lo % a.W;
+    const int m = s_src_off[sr * a.E_l + e] + (r - s_row_off[lo]);
+    const int row = flat ? m : (m < a.M ? sr * a.M + m : -1);
+    a.map[r] = row;
+    if (a.row_gate) a.row_gate[r] = row >= 0 ? a.recv_gate[row] : 0.f;
+    if (a.row_scale) a.row_scale[r] = a.recv_scale[max(row, 0)];
+}
+
 // ---- 3. stable positions.  A workgroup of 16 waves ranks RBLK consecutive blocks of 64 tokens, 16 / RBLK waves to a block, each with
 // every (16 / RBLK)-th of a token's slots: the waves OR their lane bits into a 64-bit mask per block and expert in LDS (a token holds
 // an expert at most once), and the rank of a slot inside its expert is the rows of the expert in earlier workgroups' blocks +
@@ -136,17 +247,24 @@ __global__ __launch_bounds__(SCAN_E * SCAN_SLICES) void scan_hist_kernel(const i
 // with 16 the popcounts of up to 15 masks per slot and four workgroups in all took 22 us for 4096 tokens x 8 of 256, so 9.
 // (scan and rank took 22 us as launches of their own.)
 // ONE = true (up to 1024 tokens): a single workgroup holds all 16 blocks, counts for itself and is the only launch.
+// SIDE: the blocks from rank_blocks_n on prepare the receive side (in a step, where the received counts are there already: a launch less, 2 to 3 us
+// beside a ranking that leaves the chip idle).
 // base (or NULL): what scan_hist_kernel left, where the sums, which grow with the square of the tokens, are too many (RANK_SUM_CELLS).
-template <bool ONE>
+template <bool ONE, bool SIDE>
 __global__ __launch_bounds__(RANK_WAVES * WAVE) void rank_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict__ hist,
                                                                   const int32_t* __restrict__ base, int T,
                                                                   int k, int E, int W, int NB, int32_t* __restrict__ send_counts,
                                                                   int32_t* __restrict__ expert_offs, int32_t* __restrict__ dst_sizes,
                                                                   int32_t* __restrict__ dst_offsets, int32_t* __restrict__ caps,
-                                                                  int32_t* __restrict__ pos, int32_t* __restrict__ row_token) {
+                                                                  int32_t* __restrict__ pos, int32_t* __restrict__ row_token, int rank_blocks_n,
+                                                                  const RecvPrepare side) {
     constexpr int RBLK = rank_blocks<ONE>(), PARTS = RANK_WAVES / RBLK, SLOTS = MOE_MAX_TOPK / PARTS;
     extern __shared__ unsigned long long masks[];  // [RBLK][E]
     __shared__ int32_t tot[MOE_MAX_EXPERTS], pre[MOE_MAX_EXPERTS], es[MOE_MAX_EXPERTS + 1];
+    if (SIDE && (int)blockIdx.x >= rank_blocks_n) {
+        recv_prepare_block(side, blockIdx.x - rank_blocks_n, es, pre);
+        return;
+    }
     const int tid = threadIdx.x, wave = tid / WAVE, lane = lane_id(), blk = wave / PARTS, part = wave % PARTS;
     const int b0 = blockIdx.x * RBLK, t = (b0 + blk) * CB + lane;
     const bool live = b0 + blk < NB && t < T;
@@ -154,7 +272,7 @@ __global__ __launch_bounds__(RANK_WAVES * WAVE) void rank_kernel(const int32_t* 
 #pragma unroll
     for (int j = 0; j < SLOTS; ++j) mine[j] = (live && j * PARTS + part < k) ? idx[(size_t)t * k + j * PARTS + part] : -1;
     for (int e = tid; e < E; e += blockDim.x) {
-        tot[e] = !ONE && base ? base[(size_t)gridDim.x * E + e] : 0;
+        tot[e] = !ONE && base ? base[(size_t)rank_blocks_n * E + e] : 0;
         pre[e] = !ONE && base ? base[(size_t)blockIdx.x * E + e] : 0;
     }
     for (int i = tid; i < RBLK * E; i += blockDim.x) masks[i] = 0ull;
@@ -392,8 +510,6 @@ __device__ __forceinline__ int source_row(const RowSource& a, int r) {
     }
 }
 
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-
 // Rows of a copy that a wave takes together: of 2 to 4 KB two (eight 16-byte loads of a lane in flight instead of four; 4096 x 2 rows of 3 KB:
 // payload 11.2 -> 10.2 us, unpack 11.6 -> 9.8, return 12.1 -> 10.4), where rows are many enough to keep every place on the chip taken (1024
 // rows one by one or two by two: the same).  Shorter rows gain nothing from four together (8192 x 2 of 1 KB 8.3 -> 9.2) and few rows lose.
@@ -474,7 +590,6 @@ __global__ __launch_bounds__(WPB * WAVE) void gather_rows_kernel(const u32x4* __
 // slots each, which only get zeros where they are padding (a wave per slot was mostly wave start-up: with skewed
 // routing most of the send buffer is padding).  Same bytes in send_buf as the slot-major gather (SRC_PACK), with x
 // read once instead of k times.
-constexpr int PACK_ZR = 8;
 // Waves per token row of the kernels that give a token to a wave: with few tokens a row is cut into runs of columns (64 vectors at
 // least), so that the chip holds some 2048 waves whatever the token count (24 rows of 14 KB, top-8: pack 12.8 -> 7.7 us, combine
 // 23 -> 5.8 us: a wave alone walks its row by 1 to 8 KB a memory round trip).
@@ -803,111 +918,15 @@ int gather_rows(const void* src, void* dst, const RowSource& a, int n_rows, int 
 #undef MOE_GATHER
     return moe_check_launch("gather_rows");
 }
-
-// rows [size_s, M) of every slot s of a [W,M,row] buffer <- 0, size_s = sum over e of rc[s,e]; one wave per run of
-// PACK_ZR consecutive rows (the slot's size is summed once per run, or twice when the run crosses into the next slot)
-__device__ __forceinline__ int slot_size(const int32_t* __restrict__ rc, int s, int E_l, int lane) {
-    int size = 0;
-    for (int e = lane; e < E_l; e += WAVE) size += rc[s * E_l + e];
-    return wave_sum(size);
-}
-__device__ __forceinline__ void zero_padding_rows(u32x4* __restrict__ buf, const int32_t* __restrict__ rc, int W, int E_l, int M,
-                                                  int row_vecs, int block) {
-    const int wave = threadIdx.x / WAVE, lane = lane_id();
-    const int r0 = (block * (blockDim.x / WAVE) + wave) * PACK_ZR, r1 = min(r0 + PACK_ZR, W * M);
-    if (r0 >= r1) return;
-    int s = r0 / M, m = r0 % M;
-    int size = slot_size(rc, s, E_l, lane);
-    const u32x4 z = {0u, 0u, 0u, 0u};
-    for (int r = r0; r < r1; ++r) {
-        if (m >= size) {
-            u32x4* row = buf + (size_t)r * row_vecs;
-            for (int c = lane; c < row_vecs; c += WAVE) __builtin_nontemporal_store(z, row + c);
-        }
-        if (++m == M && r + 1 < r1) { m = 0; size = slot_size(rc, ++s, E_l, lane); }
-    }
-}
-
 __global__ __launch_bounds__(256) void zero_padding_rows_kernel(u32x4* __restrict__ buf, const int32_t* __restrict__ rc, int W, int E_l,
                                                                  int M, int row_vecs) {
     zero_padding_rows(buf, rc, W, E_l, M, row_vecs, blockIdx.x);
 }
 
-// Expert-major row r of the receive side -> row of the [W,M,H] buffer that holds it (one thread per row, binary search in
-// the (expert, source)-major prefix).  The same index serves the way back: the result row of r returns to the slot its input
-// came from.  Rows past the received total map to row 0; rows the pack dropped (position in the sender's slot at or past
-// the pair capacity M) map to -1: the GEMMs read row 0 for them and store nothing.
-// One launch: every block derives the two prefix tables it needs from recv_counts in LDS (at most
-// MOE_MAX_EXPERTS entries: a wave's scan) instead of waiting for a table kernel; block 0 also leaves the per-expert totals.
-// M = 0: the receive buffer is a padding-free flat payload instead (source-major, expert-minor blocks, the layout
-// reorder_flat_to_token_buf of the reference reads, baseline.py:204-218): the row of (e, s, j) is the exclusive prefix of the
-// counts over flattened (s, e) plus j, and no row can have been dropped.
-// recv_gate / row_gate (both or neither): the gates that arrived with the rows, [rows of the receive buffer], gathered
-// into expert-major order for the GEMM that applies them (0 for rows without a source).  recv_scale / row_scale likewise: the
-// fp8 row scales (rows without a source take that of row 0, whose codes the GEMM reads for them).
-// zbuf (or NULL): the blocks from map_blocks on zero the padding rows of that [W,M,row_vecs] buffer, which depend on the same counts.
-__global__ __launch_bounds__(256) void row_map_from_counts_kernel(const int32_t* __restrict__ rc, int W, int E_l, int M, int n_rows,
-                                                                   int32_t* __restrict__ map, int32_t* __restrict__ expert_cnt,
-                                                                   const float* __restrict__ recv_gate, float* __restrict__ row_gate,
-                                                                   const float* __restrict__ recv_scale, float* __restrict__ row_scale,
-                                                                   u32x4* __restrict__ zbuf, int row_vecs, int map_blocks) {
-    if ((int)blockIdx.x >= map_blocks) {
-        zero_padding_rows(zbuf, rc, W, E_l, M, row_vecs, blockIdx.x - map_blocks);
-        return;
-    }
+__global__ __launch_bounds__(256) void row_map_from_counts_kernel(const RecvPrepare a) {
     __shared__ int32_t s_row_off[MOE_MAX_EXPERTS + 1];
     __shared__ int32_t s_src_off[MOE_MAX_EXPERTS];
-    const int n = W * E_l;
-    const bool flat = M == 0;
-    if (threadIdx.x < WAVE) {
-        const int lane = lane_id();
-        const int per = (n + WAVE - 1) / WAVE;
-        const int lo = min(lane * per, n), hi = min(lo + per, n);
-        int sum = 0;
-        for (int i = lo; i < hi; ++i) sum += rc[(i % W) * E_l + (i / W)];
-        const int incl = wave_incl_scan(sum);
-        int run = incl - sum;
-        for (int i = lo; i < hi; ++i) { s_row_off[i] = run; run += rc[(i % W) * E_l + (i / W)]; }
-        if (lane == WAVE - 1) s_row_off[n] = incl;
-        if (flat) {  // exclusive prefix over flattened (s, e): where the block of (s, e) starts in the flat payload
-            int fsum = 0;
-            for (int i = lo; i < hi; ++i) fsum += rc[i];
-            const int fincl = wave_incl_scan(fsum);
-            int frun = fincl - fsum;
-            for (int i = lo; i < hi; ++i) { s_src_off[i] = frun; frun += rc[i]; }
-        } else {
-            for (int sr = lane; sr < W; sr += WAVE) {
-                int r = 0;
-                for (int e = 0; e < E_l; ++e) { s_src_off[sr * E_l + e] = r; r += rc[sr * E_l + e]; }
-            }
-        }
-        if (blockIdx.x == 0 && expert_cnt)
-            for (int e = lane; e < E_l; e += WAVE) {
-                int c = 0;
-                for (int sr = 0; sr < W; ++sr) c += rc[sr * E_l + e];
-                expert_cnt[e] = c;
-            }
-    }
-    __syncthreads();
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= n_rows) return;
-    if (r >= s_row_off[n]) {
-        map[r] = 0;
-        if (row_gate) row_gate[r] = 0.f;
-        if (row_scale) row_scale[r] = recv_scale[0];
-        return;
-    }
-    int lo = 0, hi = n;  // s_row_off[0] = 0 <= r; the last of a run of equal offsets owns the row
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (s_row_off[mid] <= r) lo = mid; else hi = mid;
-    }
-    const int e = lo / W, sr = lo % W;
-    const int m = s_src_off[sr * E_l + e] + (r - s_row_off[lo]);
-    const int row = flat ? m : (m < M ? sr * M + m : -1);
-    map[r] = row;
-    if (row_gate) row_gate[r] = row >= 0 ? recv_gate[row] : 0.f;
-    if (row_scale) row_scale[r] = recv_scale[max(row, 0)];
+    recv_prepare_block(a, blockIdx.x, s_row_off, s_src_off);
 }
 
 int check_rows(const char* who, int dtype, int H) {
@@ -1047,10 +1066,9 @@ extern "C" size_t moe_count_workspace_bytes(int T, int k, int E) {
     return sizeof(int32_t) * (2 * (size_t)E * NB + 2 * (size_t)E + 1);
 }
 
-extern "C" int moe_count_and_offsets(const int32_t* topk_idx, int T, int k, int E, int W, int32_t* send_counts,
-                                     int32_t* expert_offs, int32_t* dst_sizes, int32_t* dst_offsets, int32_t* caps,
-                                     int32_t* pos, int32_t* row_token, void* ws, size_t ws_bytes, moe_stream_t stream) {
-    hipStream_t s = (hipStream_t)stream;
+static int count_and_offsets(const int32_t* topk_idx, int T, int k, int E, int W, int32_t* send_counts, int32_t* expert_offs,
+                             int32_t* dst_sizes, int32_t* dst_offsets, int32_t* caps, int32_t* pos, int32_t* row_token, void* ws,
+                             size_t ws_bytes, const RecvPrepare* side, int side_blocks, hipStream_t s) {
     MOE_REQUIRE(T >= 0 && E > 0 && W > 0, MOE_ERR_INVALID, "count: bad shape T=%d E=%d W=%d", T, E, W);
     MOE_REQUIRE(E % W == 0, MOE_ERR_INVALID, "num_experts_total must be divisible by world_size (E=%d W=%d)", E, W);
     MOE_REQUIRE(k >= 1 && k <= MOE_MAX_TOPK, MOE_ERR_UNSUPPORTED, "count: topk=%d outside [1,%d]", k, MOE_MAX_TOPK);
@@ -1062,9 +1080,13 @@ extern "C" int moe_count_and_offsets(const int32_t* topk_idx, int T, int k, int 
     const int NB = ceil_div(T > 0 ? T : 1, CB);
     int32_t* hist = (int32_t*)ws;
     auto lds = [&](int blocks) { return (size_t)blocks * E * sizeof(unsigned long long); };
+#define MOE_RANK(ONE, SIDE, blocks, hist, base)                                                                                         \
+    rank_kernel<ONE, SIDE><<<(blocks) + side_blocks, RANK_WAVES * WAVE, lds(rank_blocks<ONE>()), s>>>(                                  \
+        topk_idx, hist, base, T, k, E, W, NB, send_counts, expert_offs, dst_sizes, dst_offsets, caps, pos, row_token, blocks,           \
+        side ? *side : RecvPrepare{})
     if (NB <= rank_blocks<true>()) {  // (few tokens: one workgroup holds everything)
-        rank_kernel<true><<<1, RANK_WAVES * WAVE, lds(rank_blocks<true>()), s>>>(topk_idx, nullptr, nullptr, T, k, E, W, NB, send_counts, expert_offs, dst_sizes, dst_offsets,
-                                                           caps, pos, row_token);
+        if (side) MOE_RANK(true, true, 1, nullptr, nullptr);
+        else MOE_RANK(true, false, 1, nullptr, nullptr);
         return moe_check_launch("count_and_offsets");
     }
     block_hist_kernel<<<ceil_div(NB, 4), 256, 4 * E * sizeof(int32_t), s>>>(topk_idx, hist, T, k, E, NB);
@@ -1074,9 +1096,17 @@ extern "C" int moe_count_and_offsets(const int32_t* topk_idx, int T, int k, int 
         base = hist + (size_t)NB * E;
         scan_hist_kernel<<<ceil_div(E, SCAN_E), SCAN_E * SCAN_SLICES, 0, s>>>(hist, base, NB, NG, E);
     }
-    rank_kernel<false><<<NG, RANK_WAVES * WAVE, lds(rank_blocks<false>()), s>>>(
-        topk_idx, hist, base, T, k, E, W, NB, send_counts, expert_offs, dst_sizes, dst_offsets, caps, pos, row_token);
+    if (side) MOE_RANK(false, true, NG, hist, base);
+    else MOE_RANK(false, false, NG, hist, base);
+#undef MOE_RANK
     return moe_check_launch("count_and_offsets");
+}
+
+extern "C" int moe_count_and_offsets(const int32_t* topk_idx, int T, int k, int E, int W, int32_t* send_counts,
+                                     int32_t* expert_offs, int32_t* dst_sizes, int32_t* dst_offsets, int32_t* caps,
+                                     int32_t* pos, int32_t* row_token, void* ws, size_t ws_bytes, moe_stream_t stream) {
+    return count_and_offsets(topk_idx, T, k, E, W, send_counts, expert_offs, dst_sizes, dst_offsets, caps, pos, row_token, ws, ws_bytes, nullptr,
+                             0, (hipStream_t)stream);
 }
 
 // ---- the same entry point for callers that may not allocate: the workspace is a fixed array in the library's own
@@ -1254,18 +1284,25 @@ extern "C" int moe_unpack_expert_major(const void* recv, int dtype, int W, int M
                        S_rows, nullptr, (hipStream_t)stream);
 }
 
+static RecvPrepare recv_prepare_args(const int32_t* rc, int W, int E_l, int M, int n_rows, int32_t* map, int32_t* expert_cnt,
+                                     const float* recv_gate, float* row_gate, const float* recv_scale, float* row_scale, void* zbuf, int row_bytes,
+                                     int threads, int& blocks) {
+    // (at least one block, for the per-expert totals)
+    const int map_blocks = max(ceil_div(n_rows, threads), 1);
+    blocks = map_blocks + (zbuf ? ceil_div(ceil_div(W * M, PACK_ZR), threads / WAVE) : 0);
+    return {rc, W, E_l, M, n_rows, map, expert_cnt, recv_gate, row_gate, recv_scale, row_scale, (u32x4*)zbuf, row_bytes / 16, map_blocks};
+}
+
 static int launch_row_map(const int32_t* rc, int W, int E_l, int M, int n_rows, int32_t* map, int32_t* expert_cnt, const float* recv_gate,
                           float* row_gate, const float* recv_scale, float* row_scale, void* zbuf, int row_bytes, hipStream_t s) {
-    // (at least one block, for the per-expert totals)
-    const int map_blocks = max(ceil_div(n_rows, 256), 1), zero_blocks = zbuf ? ceil_div(ceil_div(W * M, PACK_ZR), 4) : 0;
-    row_map_from_counts_kernel<<<map_blocks + zero_blocks, 256, 0, s>>>(rc, W, E_l, M, n_rows, map, expert_cnt, recv_gate, row_gate, recv_scale,
-                                                                        row_scale, (u32x4*)zbuf, row_bytes / 16, map_blocks);
+    int blocks;
+    const RecvPrepare a = recv_prepare_args(rc, W, E_l, M, n_rows, map, expert_cnt, recv_gate, row_gate, recv_scale, row_scale, zbuf, row_bytes, 256, blocks);
+    row_map_from_counts_kernel<<<blocks, 256, 0, s>>>(a);
     return moe_check_launch("recv_row_map");
 }
 
-extern "C" int moe_recv_prepare(const int32_t* recv_counts, int W, int E_l, int M, int n_rows, const float* recv_gate, const float* recv_scale,
-                                int32_t* row_map, float* row_gate, float* row_scale, int32_t* expert_cnt, void* ret, int dtype, int H,
-                                moe_stream_t stream) {
+static int check_recv_prepare(const int32_t* recv_counts, int W, int E_l, int M, int n_rows, const float* recv_gate, const float* recv_scale,
+                              const int32_t* row_map, const float* row_gate, const float* row_scale, const void* ret, int dtype, int H) {
     MOE_REQUIRE(W > 0 && E_l > 0 && W * E_l <= MOE_MAX_EXPERTS, MOE_ERR_INVALID, "recv_prepare: bad W=%d E_l=%d", W, E_l);
     MOE_REQUIRE(M >= 0 && n_rows >= 0 && recv_counts, MOE_ERR_INVALID, "recv_prepare: bad arguments");
     MOE_REQUIRE((recv_gate == nullptr) == (row_gate == nullptr) && (recv_scale == nullptr) == (row_scale == nullptr), MOE_ERR_INVALID,
@@ -1276,8 +1313,31 @@ extern "C" int moe_recv_prepare(const int32_t* recv_counts, int W, int E_l, int 
         if (rc) return rc;
         MOE_REQUIRE(M >= 1 && (long long)W * M < (1ll << 31), MOE_ERR_UNSUPPORTED, "recv_prepare: %d x %d rows", W, M);
     }
+    return MOE_OK;
+}
+
+extern "C" int moe_recv_prepare(const int32_t* recv_counts, int W, int E_l, int M, int n_rows, const float* recv_gate, const float* recv_scale,
+                                int32_t* row_map, float* row_gate, float* row_scale, int32_t* expert_cnt, void* ret, int dtype, int H,
+                                moe_stream_t stream) {
+    const int rc = check_recv_prepare(recv_counts, W, E_l, M, n_rows, recv_gate, recv_scale, row_map, row_gate, row_scale, ret, dtype, H);
+    if (rc) return rc;
     return launch_row_map(recv_counts, W, E_l, M, n_rows, row_map, expert_cnt, recv_gate, row_gate, recv_scale, row_scale, ret,
                           H * dtype_size(dtype), (hipStream_t)stream);
+}
+
+int moe_count_and_prepare(const moe_step_args* a, hipStream_t s) {
+    const int E_l = a->experts / a->world, M = a->flat ? 0 : a->M;
+    const float *recv_gate = a->gated ? a->recv_gate : nullptr, *recv_scale = a->q_dispatch ? a->recv_scale : nullptr;
+    float *row_gate = a->gated ? a->row_gate : nullptr, *row_scale = a->q_dispatch ? a->xs : nullptr;
+    void* ret = a->flat ? nullptr : a->ret;
+    const int rc = check_recv_prepare(a->recv_counts, a->world, E_l, M, a->S, recv_gate, recv_scale, a->row_map, row_gate, row_scale, ret, a->dtype,
+                                      a->hidden);
+    if (rc) return rc;
+    int blocks;
+    const RecvPrepare side = recv_prepare_args(a->recv_counts, a->world, E_l, M, a->S, a->row_map, a->expert_cnt, recv_gate, row_gate, recv_scale,
+                                               row_scale, ret, a->hidden * dtype_size(a->dtype), RANK_WAVES * WAVE, blocks);
+    return count_and_offsets(a->idx, a->tokens, a->topk, a->experts, a->world, a->send_counts, a->expert_offs, a->dst_sizes, a->dst_offsets, a->caps,
+                             a->pos, a->row_token, a->count_ws, a->count_ws_bytes, &side, blocks, s);
 }
 
 extern "C" int moe_recv_row_map(const int32_t* recv_counts, int W, int E_l, int M, int n_rows, int32_t* row_map,

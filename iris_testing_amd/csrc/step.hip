@@ -1,10 +1,32 @@
 // One step of the hot path as one call: host code only, every stage is an entry point of its own.
 #include "common.h"
 
+// True if nothing that the receive side's preparation reads or writes lies in a buffer of the source side up to the pack: a caller that
+// loops its own rows back (received counts, gates or scales are the sent ones) or shares scratch between the sides needs them in order.
+static bool sides_apart(const moe_step_args* a) {
+    struct Range {
+        const void* at;
+        size_t bytes;
+    };
+    const size_t T = a->tokens, H = a->hidden, E = a->experts, W = a->world, R = T * a->topk, S = a->S, n = W * (size_t)a->M;
+    const size_t row = H * (a->dtype == MOE_BF16 ? 2 : 4);
+    const Range receive[] = {{a->recv_counts, E * 4}, {a->gated ? a->recv_gate : nullptr, n * 4}, {a->q_dispatch ? a->recv_scale : nullptr, n * 4},
+                             {a->row_map, S * 4}, {a->expert_cnt, E / W * 4}, {a->gated ? a->row_gate : nullptr, S * 4},
+                             {a->q_dispatch ? a->xs : nullptr, S * 4}, {a->flat ? nullptr : a->ret, n * row}};
+    const Range source[] = {{a->x, T * row}, {a->idx, R * 4}, {a->gate, R * 4}, {a->send_counts, E * 4}, {a->expert_offs, E * 4},
+                            {a->dst_sizes, W * 4}, {a->dst_offsets, W * 4}, {a->caps, 8}, {a->pos, R * 4}, {a->row_token, R * 4},
+                            {a->count_ws, a->count_ws_bytes}, {a->send, a->flat ? R * row : a->q_dispatch ? n * H : n * row},
+                            {a->send_scale, n * 4}, {a->send_gate, n * 4}, {a->status, 4}};
+    for (const Range& r : receive)
+        for (const Range& q : source)
+            if (r.at && q.at && (uintptr_t)r.at < (uintptr_t)q.at + q.bytes && (uintptr_t)q.at < (uintptr_t)r.at + r.bytes) return false;
+    return true;
+}
+
 // Stage by stage from Python a step costs 8 to 10 foreign calls with some fifteen arguments each (about 80 us of host time);
 // here one, so an eager step of a small model waits for the GPU and not for the host.  The destination side derives the row map, the
-// row scales, the gates and the zeroed padding rows from the received counts in one launch (a launch costs some 4.5 us
-// even when it has nothing to do).
+// row scales, the gates and the zeroed padding rows from the received counts in one launch, the one that ranks the tokens (a launch
+// costs some 4.5 us even when it has nothing to do).
 extern "C" int moe_step(const moe_step_args* a, moe_stream_t stream) {
     MOE_REQUIRE(a, MOE_ERR_INVALID, "step: null arguments");
     const int T = a->tokens, H = a->hidden, E = a->experts, k = a->topk, W = a->world, F = a->ffn, M = a->M, S = a->S;
@@ -21,8 +43,12 @@ extern "C" int moe_step(const moe_step_args* a, moe_stream_t stream) {
     } while (0)
     MOE_STAGE(moe_route_topk(a->x, a->router, a->bias, a->dtype, T, H, E, k, a->logits, a->idx, a->gate, a->route_ws, a->route_ws_bytes,
                              stream));
-    MOE_STAGE(moe_count_and_offsets(a->idx, T, k, E, W, a->send_counts, a->expert_offs, a->dst_sizes, a->dst_offsets, a->caps, a->pos,
-                                    a->row_token, a->count_ws, a->count_ws_bytes, stream));
+    const bool together = a->fused && sides_apart(a);
+    if (together)
+        MOE_STAGE(moe_count_and_prepare(a, (hipStream_t)stream));
+    else
+        MOE_STAGE(moe_count_and_offsets(a->idx, T, k, E, W, a->send_counts, a->expert_offs, a->dst_sizes, a->dst_offsets, a->caps, a->pos,
+                                        a->row_token, a->count_ws, a->count_ws_bytes, stream));
     if (a->q_dispatch)
         MOE_STAGE(moe_pack_tokens_fp8_gated(a->x, T, H, a->idx, a->pos, out_gate, k, E_l, a->dst_sizes, a->dst_offsets, W, M,
                                             (uint8_t*)a->send, a->send_scale, a->gated ? a->send_gate : nullptr, a->status, stream));
@@ -37,11 +63,11 @@ extern "C" int moe_step(const moe_step_args* a, moe_stream_t stream) {
     // fp32 experts: the GEMMs of small launches move the rows themselves (plumbing: 42.9 -> 38 us a step)
     const bool f32_slots = a->f32_weights && !a->fused && !a->quant && a->dtype == MOE_F32 && S > 0;
     // destination: rows in expert-major order
-    if (a->fused)
+    if (a->fused && !together)
         MOE_STAGE(moe_recv_prepare(a->recv_counts, W, E_l, a->flat ? 0 : M, S, a->gated ? a->recv_gate : nullptr,
                                    a->q_dispatch ? a->recv_scale : nullptr, a->row_map, a->gated ? a->row_gate : nullptr,
                                    a->q_dispatch ? a->xs : nullptr, a->expert_cnt, a->flat ? nullptr : a->ret, a->dtype, H, stream));
-    else if (!f32_slots)
+    else if (!a->fused && !f32_slots)
         MOE_STAGE(moe_unpack_expert_major(a->recv, a->dtype, W, M, H, a->recv_counts, E_l, a->rows, S, a->expert_cnt, a->unpack_map, stream));
     const void* src = a->fused ? a->recv : a->rows;
     void* dst = a->fused ? a->ret : a->y;

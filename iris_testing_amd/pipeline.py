@@ -145,7 +145,8 @@ class DispatchPipeline:
         return self._args
 
     def _run(self, s):
-        """The stages of STAGES as one call (the map, scales, gates and padding of the destination side in one launch)."""
+        """The stages of STAGES as one call (the map, scales, gates and padding of the destination side in the ranking launch; the rows of
+        fp32 experts moved by their GEMMs)."""
         L.check(L.lib().moe_step(self._fill(), s))
 
     # each stage is a closure-free method so that callers can time them one by one

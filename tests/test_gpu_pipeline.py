@@ -146,6 +146,35 @@ def test_fp32_rows_come_from_and_go_to_their_slots_in_the_gemms(T, H, E, k, W, F
         assert torch.equal(one[n], stages[n]), f"{n} differs"
 
 
+@pytest.mark.parametrize("tokens,gated", [(40, False), (40, True), (1500, True)])
+def test_rows_looped_back_on_one_rank_are_the_sent_ones(tokens, gated):
+    """The receive side is prepared beside the ranking unless it reads what the source side writes: with one rank the received counts, rows and
+    gates may be the sent buffers themselves, and the step has to give what it gives with copies of them."""
+    from iris_testing_amd.configs import MoEConfig
+    from iris_testing_amd.pipeline import DispatchPipeline
+    cfg = MoEConfig("case", 5, tokens, 256, "bf16", 12, 2, 1, 256, "silu")
+    world = harness.build_world(cfg, DEV)
+    ew, _, _ = harness.expert_weights(cfg, 0, DEV)
+    kw = dict(gated=True, recv_gate=harness.recv_gates(world)) if gated else {}
+    pipe = DispatchPipeline(world, ew, **kw)
+    names = "send_counts pos send expert_cnt row_map hidden ret".split()
+
+    def results():
+        for n in names:
+            getattr(pipe, n).zero_()
+        pipe.step()
+        torch.cuda.synchronize()
+        return {n: getattr(pipe, n).clone() for n in names}
+    apart = results()
+    assert torch.equal(apart["send"], world.recv) and torch.equal(apart["send_counts"], world.recv_counts)
+    world.recv, world.recv_counts = pipe.send, pipe.send_counts
+    if gated:
+        pipe.recv_gate = pipe.send_gate
+    back = results()
+    for n in names:
+        assert torch.equal(back[n], apart[n]), f"{n} differs"
+
+
 def test_entry_point_smoke_runs():
     """The smoke check of the repository's entry module (one small step against the oracle) must keep passing."""
     import importlib
