@@ -250,6 +250,9 @@ __device__ __forceinline__ void recv_prepare_block(const RecvPrepare& a, int blo
 // SIDE: the blocks from rank_blocks_n on prepare the receive side (in a step, where the received counts are there already: a launch less, 2 to 3 us
 // beside a ranking that leaves the chip idle).
 // base (or NULL): what scan_hist_kernel left, where the sums, which grow with the square of the tokens, are too many (RANK_SUM_CELLS).
+// hist == NULL (few enough slots, RANK_SELF_SLOTS): the workgroup counts all slots, those before its blocks and the rest apart, in eight
+// copies of the counters, so that lanes with the same expert seldom meet.
+constexpr int RANK_COPIES = 8;
 template <bool ONE, bool SIDE>
 __global__ __launch_bounds__(RANK_WAVES * WAVE) void rank_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict__ hist,
                                                                   const int32_t* __restrict__ base, int T,
@@ -276,6 +279,10 @@ __global__ __launch_bounds__(RANK_WAVES * WAVE) void rank_kernel(const int32_t* 
         pre[e] = !ONE && base ? base[(size_t)blockIdx.x * E + e] : 0;
     }
     for (int i = tid; i < RBLK * E; i += blockDim.x) masks[i] = 0ull;
+    const int stride = E | 1;  // (odd: the copies of a counter lie in different banks)
+    int32_t* const tab = reinterpret_cast<int32_t*>(masks + RBLK * E);
+    if (!ONE && !hist)
+        for (int i = tid; i < 2 * RANK_COPIES * stride; i += blockDim.x) tab[i] = 0;
     __syncthreads();
     unsigned long long* my = masks + blk * E;
 #pragma unroll
@@ -312,7 +319,30 @@ __global__ __launch_bounds__(RANK_WAVES * WAVE) void rank_kernel(const int32_t* 
                 atomicAdd(&pre[c * V + i], before[i]);
             }
         };
-        if (!base) {
+        if (!hist) {
+            const int n = T * k, limit = min(b0 * CB, T) * k, copy = lane % RANK_COPIES;
+            auto add = [&](int i, int e) {
+                if ((unsigned)e < (unsigned)E) atomicAdd(&tab[((i < limit ? 0 : RANK_COPIES) + copy) * stride + e], 1);
+            };
+            const int vecs = ((uintptr_t)idx & 15) == 0 ? n / 4 : 0;
+#pragma unroll 4
+            for (int i = tid; i < vecs; i += RANK_WAVES * WAVE) {
+                const int4 q = reinterpret_cast<const int4*>(idx)[i];
+                add(4 * i, q.x); add(4 * i + 1, q.y); add(4 * i + 2, q.z); add(4 * i + 3, q.w);
+            }
+            for (int i = 4 * vecs + tid; i < n; i += RANK_WAVES * WAVE) add(i, idx[i]);
+            __syncthreads();
+            for (int e = tid; e < E; e += RANK_WAVES * WAVE) {
+                int before = 0, after = 0;
+#pragma unroll
+                for (int c = 0; c < RANK_COPIES; ++c) {
+                    before += tab[c * stride + e];
+                    after += tab[(RANK_COPIES + c) * stride + e];
+                }
+                pre[e] = before;
+                tot[e] = before + after;
+            }
+        } else if (!base) {
             if (E % 4 == 0 && ((uintptr_t)hist & 15) == 0) sums(std::integral_constant<int, 4>{});
             else sums(std::integral_constant<int, 1>{});
         }
@@ -1058,6 +1088,10 @@ __global__ __launch_bounds__(256) void shuffle_totals_kernel(const int32_t* __re
 // 256 experts 11.7 / 12.7 (8192, 1 M), 13.5 / 13.1 (16384, 4 M), 17.2 / 14.0 (32768, 16 M) and 181 / 43 (262144, 1 G); 512 experts
 // 14.4 / 13.6 (8192, 2 M) and 18.1 / 14.0 (16384, 8 M).
 constexpr long long RANK_SUM_CELLS = 6ll << 20;
+// Slots that every ranking workgroup counts for itself instead of summing up the histogram, which is then no launch.  With the histogram against
+// without, us: 1100 tokens x 1 of 8 8.4 / 3.7, 2048 x 8 of 32 8.7 / 6.8, 8192 x 2 of 256 8.3 / 5.8, 16384 x 2 of 8 9.1 / 6.5, 4096 x 8 of 256
+// 10.5 / 9.0, 8192 x 4 of 512 11.6 / 8.6; but 8192 x 8 of 256 10.8 / 11.9, of 60 9.2 / 11.2, 16384 x 8 of 256 12.6 / 18.0.
+constexpr long long RANK_SELF_SLOTS = 32768;
 
 extern "C" size_t moe_count_workspace_bytes(int T, int k, int E) {
     (void)k;
@@ -1080,24 +1114,30 @@ static int count_and_offsets(const int32_t* topk_idx, int T, int k, int E, int W
     const int NB = ceil_div(T > 0 ? T : 1, CB);
     int32_t* hist = (int32_t*)ws;
     auto lds = [&](int blocks) { return (size_t)blocks * E * sizeof(unsigned long long); };
-#define MOE_RANK(ONE, SIDE, blocks, hist, base)                                                                                         \
-    rank_kernel<ONE, SIDE><<<(blocks) + side_blocks, RANK_WAVES * WAVE, lds(rank_blocks<ONE>()), s>>>(                                  \
+#define MOE_RANK(ONE, SIDE, blocks, hist, base, more)                                                                                    \
+    rank_kernel<ONE, SIDE><<<(blocks) + side_blocks, RANK_WAVES * WAVE, lds(rank_blocks<ONE>()) + (more), s>>>(                           \
         topk_idx, hist, base, T, k, E, W, NB, send_counts, expert_offs, dst_sizes, dst_offsets, caps, pos, row_token, blocks,           \
         side ? *side : RecvPrepare{})
     if (NB <= rank_blocks<true>()) {  // (few tokens: one workgroup holds everything)
-        if (side) MOE_RANK(true, true, 1, nullptr, nullptr);
-        else MOE_RANK(true, false, 1, nullptr, nullptr);
+        if (side) MOE_RANK(true, true, 1, nullptr, nullptr, 0);
+        else MOE_RANK(true, false, 1, nullptr, nullptr, 0);
+        return moe_check_launch("count_and_offsets");
+    }
+    const int NG = ceil_div(NB, rank_blocks<false>());
+    if ((long long)T * k <= RANK_SELF_SLOTS) {
+        const size_t tabs = 2 * RANK_COPIES * (size_t)(E | 1) * sizeof(int32_t);
+        if (side) MOE_RANK(false, true, NG, nullptr, nullptr, tabs);
+        else MOE_RANK(false, false, NG, nullptr, nullptr, tabs);
         return moe_check_launch("count_and_offsets");
     }
     block_hist_kernel<<<ceil_div(NB, 4), 256, 4 * E * sizeof(int32_t), s>>>(topk_idx, hist, T, k, E, NB);
-    const int NG = ceil_div(NB, rank_blocks<false>());
     int32_t* base = nullptr;
     if ((long long)NG * NB * E > RANK_SUM_CELLS) {
         base = hist + (size_t)NB * E;
         scan_hist_kernel<<<ceil_div(E, SCAN_E), SCAN_E * SCAN_SLICES, 0, s>>>(hist, base, NB, NG, E);
     }
-    if (side) MOE_RANK(false, true, NG, hist, base);
-    else MOE_RANK(false, false, NG, hist, base);
+    if (side) MOE_RANK(false, true, NG, hist, base, 0);
+    else MOE_RANK(false, false, NG, hist, base, 0);
 #undef MOE_RANK
     return moe_check_launch("count_and_offsets");
 }

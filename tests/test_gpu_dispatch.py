@@ -555,6 +555,23 @@ def test_counts_and_positions_of_many_tokens(T, E, W, k):
     assert c.caps.tolist() == [max(1, int(sizes.max())), max(1, int(counts.max()))]
 
 
+@pytest.mark.parametrize("T,E,W,k", [(16384, 64, 8, 2), (10923, 60, 4, 3), (4681, 511, 7, 7), (1027, 1, 1, 1)])
+def test_counts_of_slots_that_every_workgroup_counts(T, E, W, k):
+    """Either side of where the ranking workgroups count all slots themselves (32768), an index that 16-byte loads cannot start at, and
+    expert ids that are none, which count nowhere."""
+    test_counts_and_positions_of_many_tokens(T, E, W, k)
+    idx = torch.stack([torch.randperm(max(E, k), generator=torch.Generator().manual_seed(t))[:k] for t in range(T + 1)]).to(torch.int32)
+    idx[:: 97, 0] = -1
+    idx[1:: 89, k - 1] = E
+    both = [ops.count_and_offsets(i, E, W) for i in (idx.to(DEV)[1:], idx[1:].to(DEV))]
+    want = torch.bincount(idx[1:][(idx[1:] >= 0) & (idx[1:] < E)], minlength=E).view(W, -1).to(torch.int32)
+    placed = ((idx[1:] >= 0) & (idx[1:] < E)).to(DEV)
+    for c in both:
+        assert torch.equal(c.send_counts.cpu(), want)
+    assert torch.equal(both[0].pos[placed], both[1].pos[placed])
+    assert torch.equal(both[0].row_token[:int(want.sum())], both[1].row_token[:int(want.sum())])
+
+
 @pytest.mark.parametrize("T,H,k", [(1, 520, 1), (5, 4096, 3), (33, 1032, 8), (700, 264, 2), (2050, 2056, 4)])
 def test_row_copies_and_sums_cut_into_column_runs(T, H, k):
     """Rows cut into runs of columns (whole, ragged, single) where tokens are few, and for the sums where rows are long; pack, combine and the gradient of combine."""
