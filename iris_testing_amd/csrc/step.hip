@@ -1,13 +1,17 @@
 // One step of the hot path as one call: host code only, every stage is an entry point of its own.
 #include "common.h"
 
+struct Range {
+    const void* at;
+    size_t bytes;
+};
+static bool meet(const Range& r, const Range& q) {
+    return r.at && q.at && (uintptr_t)r.at < (uintptr_t)q.at + q.bytes && (uintptr_t)q.at < (uintptr_t)r.at + r.bytes;
+}
+
 // True if nothing that the receive side's preparation reads or writes lies in a buffer of the source side up to the pack: a caller that
 // loops its own rows back (received counts, gates or scales are the sent ones) or shares scratch between the sides needs them in order.
 static bool sides_apart(const moe_step_args* a) {
-    struct Range {
-        const void* at;
-        size_t bytes;
-    };
     const size_t T = a->tokens, H = a->hidden, E = a->experts, W = a->world, R = T * a->topk, S = a->S, n = W * (size_t)a->M;
     const size_t row = H * (a->dtype == MOE_BF16 ? 2 : 4);
     const Range receive[] = {{a->recv_counts, E * 4}, {a->gated ? a->recv_gate : nullptr, n * 4}, {a->q_dispatch ? a->recv_scale : nullptr, n * 4},
@@ -19,8 +23,18 @@ static bool sides_apart(const moe_step_args* a) {
                             {a->send_scale, n * 4}, {a->send_gate, n * 4}, {a->status, 4}};
     for (const Range& r : receive)
         for (const Range& q : source)
-            if (r.at && q.at && (uintptr_t)r.at < (uintptr_t)q.at + q.bytes && (uintptr_t)q.at < (uintptr_t)r.at + r.bytes) return false;
+            if (meet(r, q)) return false;
     return true;
+}
+
+// True if the GEMMs of fp32 experts may move the rows themselves: scratch that takes the place of the received rows once they are unpacked, or of
+// the hidden activation once it is used, needs the copies.
+static bool f32_apart(const moe_step_args* a) {
+    const size_t n = (size_t)a->world * a->M * a->hidden * 4, S = a->S;
+    const Range recv = {a->recv, n}, ret = {a->ret, n}, hidden = {a->hidden_ws, S * a->ffn * 4}, rows = {a->rows, S * a->hidden * 4};
+    const Range counts = {a->recv_counts, (size_t)a->experts * 4}, y = {a->y, S * a->hidden * 4};
+    return !meet(hidden, recv) && !meet(hidden, ret) && !meet(rows, recv) && !meet(y, ret) && !meet(counts, rows) && !meet(counts, hidden) &&
+           !meet(counts, y) && !meet(counts, ret);
 }
 
 // Stage by stage from Python a step costs 8 to 10 foreign calls with some fifteen arguments each (about 80 us of host time);
@@ -61,7 +75,7 @@ extern "C" int moe_step(const moe_step_args* a, moe_stream_t stream) {
         MOE_STAGE(moe_pack_tokens(a->x, a->dtype, T, H, a->idx, a->pos, k, E_l, a->dst_sizes, a->dst_offsets, W, M, a->send, a->status,
                                   stream));
     // fp32 experts: the GEMMs of small launches move the rows themselves (plumbing: 42.9 -> 38 us a step)
-    const bool f32_slots = a->f32_weights && !a->fused && !a->quant && a->dtype == MOE_F32 && S > 0;
+    const bool f32_slots = a->f32_weights && !a->fused && !a->quant && a->dtype == MOE_F32 && S > 0 && f32_apart(a);
     // destination: rows in expert-major order
     if (a->fused && !together)
         MOE_STAGE(moe_recv_prepare(a->recv_counts, W, E_l, a->flat ? 0 : M, S, a->gated ? a->recv_gate : nullptr,

@@ -146,6 +146,26 @@ def test_fp32_rows_come_from_and_go_to_their_slots_in_the_gemms(T, H, E, k, W, F
         assert torch.equal(one[n], stages[n]), f"{n} differs"
 
 
+@pytest.mark.parametrize("over", ["recv", "ret"])
+def test_fp32_scratch_over_rows_that_are_done_with(over):
+    """The hidden activation may lie where the received rows lay (they are unpacked first), and the returned buffer where the hidden activation
+    did: the step then keeps the copies."""
+    from iris_testing_amd.configs import MoEConfig
+    from iris_testing_amd.pipeline import DispatchPipeline
+    cfg = MoEConfig("case", 7, 300, 256, "f32", 8, 2, 4, 128, "gelu")
+    world = harness.build_world(cfg, DEV)
+    ew, _, _ = harness.expert_weights(cfg, 0, DEV)
+    pipe = DispatchPipeline(world, ew)
+    pipe.step()
+    torch.cuda.synchronize()
+    want = {n: getattr(pipe, n).clone() for n in ("rows", "y", "ret")}
+    pipe.hidden = (world.recv if over == "recv" else pipe.ret).view(-1)[:pipe.S * cfg.ffn].view(pipe.S, cfg.ffn)
+    pipe.step()
+    torch.cuda.synchronize()
+    for n in want:
+        assert torch.equal(getattr(pipe, n), want[n]), f"{n} differs"
+
+
 @pytest.mark.parametrize("tokens,gated", [(40, False), (40, True), (1500, True)])
 def test_rows_looped_back_on_one_rank_are_the_sent_ones(tokens, gated):
     """The receive side is prepared beside the ranking unless it reads what the source side writes: with one rank the received counts, rows and
