@@ -498,6 +498,10 @@ typedef struct moe_step_args {
     void* out;
 } moe_step_args;
 int moe_step(const moe_step_args* args /* host */, moe_stream_t stream);
+/* How moe_step would go with these arguments: out[0] = 1 if the receive side is prepared in the launch that ranks the tokens (none of its
+ * buffers meets one of the source side), out[1] = 1 if the GEMMs of fp32 experts move the rows themselves (no buffer lies where another is
+ * still read); 0: stage by stage.  Host-only, looks at addresses and sizes alone; no counterpart in the reference. */
+int moe_step_plan(const moe_step_args* args /* host */, int32_t* out);
 
 #ifdef __cplusplus
 }

@@ -114,6 +114,7 @@ _SIGNATURES = {
     "moe_shuffle_totals": (c_int, [P, c_int, P, c_int, P, P]),
     "moe_expert_forward": (c_int, [P, P, c_int, P, c_int, c_int, c_int, c_int, P, P, c_size_t, P]),
     "moe_step": (c_int, [POINTER(StepArgs), P]),
+    "moe_step_plan": (c_int, [POINTER(StepArgs), P]),
     "moe_grouped_mlp_fp8_mapped": (c_int, [P, c_int, P, P, c_int, c_int, c_int, c_int, P, P, P, P, P, P, P, P, P, P, P, c_int, P, P,
                                            c_size_t, P]),  # (.., xq_ws, xs_ws, hq_ws, hscale_ws, row_gate, out, out_rows, ..)
     "moe_diag_mfma_loop_sink_floats": (c_size_t, []),

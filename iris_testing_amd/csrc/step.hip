@@ -27,14 +27,54 @@ static bool sides_apart(const moe_step_args* a) {
     return true;
 }
 
-// True if the GEMMs of fp32 experts may move the rows themselves: scratch that takes the place of the received rows once they are unpacked, or of
-// the hidden activation once it is used, needs the copies.
+// True if a launch writes nothing that it reads, and nothing twice.
+template <int NR, int NW>
+static bool own_writes(const Range (&reads)[NR], const Range (&writes)[NW]) {
+    for (int i = 0; i < NW; ++i) {
+        for (const Range& r : reads)
+            if (meet(r, writes[i])) return false;
+        for (int j = 0; j < i; ++j)
+            if (meet(writes[j], writes[i])) return false;
+    }
+    return true;
+}
+
+// True if the GEMMs of fp32 experts may move the rows themselves.  One launch then unpacks and runs the up projection, the next runs the
+// down projection and fills the returned buffer: scratch that takes the place of something the other half of such a launch still reads
+// (the hidden activation over the received rows; the returned rows over the hidden activation, or over the counts per expert, by which
+// every workgroup finds its tile) needs the copies, which stand before and behind the GEMMs.
 static bool f32_apart(const moe_step_args* a) {
-    const size_t n = (size_t)a->world * a->M * a->hidden * 4, S = a->S;
-    const Range recv = {a->recv, n}, ret = {a->ret, n}, hidden = {a->hidden_ws, S * a->ffn * 4}, rows = {a->rows, S * a->hidden * 4};
-    const Range counts = {a->recv_counts, (size_t)a->experts * 4}, y = {a->y, S * a->hidden * 4};
-    return !meet(hidden, recv) && !meet(hidden, ret) && !meet(rows, recv) && !meet(y, ret) && !meet(counts, rows) && !meet(counts, hidden) &&
-           !meet(counts, y) && !meet(counts, ret);
+    const size_t H = a->hidden, F = a->ffn, S = a->S, E_l = a->experts / a->world, slots = (size_t)a->world * a->M * H * 4, w = E_l * H * F * 4;
+    const Range recv = {a->recv, slots}, ret = {a->ret, slots}, hidden = {a->hidden_ws, S * F * 4}, rows = {a->rows, S * H * 4}, y = {a->y, S * H * 4};
+    const Range sent = {a->recv_counts, (size_t)a->experts * 4}, counts = {a->expert_cnt, E_l * 4}, w1 = {a->w1, w}, w2 = {a->w2, w};
+    const Range up = {a->act == MOE_ACT_SWIGLU ? a->w_up : nullptr, w};
+    return own_writes({recv, sent, w1, up}, {rows, counts, hidden}) && own_writes({hidden, counts, sent, w2}, {y, ret});
+}
+
+// How a step goes: the receive side prepared in the launch that ranks the tokens; the rows of fp32 experts moved by their GEMMs (plumbing:
+// 42.9 -> 38 us a step).
+struct StepPlan {
+    bool together, f32_slots;
+};
+static int step_plan(const moe_step_args* a, StepPlan* plan) {
+    MOE_REQUIRE(a, MOE_ERR_INVALID, "step: null arguments");
+    MOE_REQUIRE(a->world > 0 && a->experts > 0 && a->experts % a->world == 0, MOE_ERR_INVALID, "step: %d experts on %d ranks", a->experts, a->world);
+    MOE_REQUIRE(a->fused || !(a->flat || a->gated || a->q_dispatch), MOE_ERR_INVALID, "step: flat / gated / q_dispatch are fused modes");
+    MOE_REQUIRE(!a->q_dispatch || (a->quant && !a->flat), MOE_ERR_INVALID, "step: q_dispatch needs fp8 experts and fixed slots");
+    MOE_REQUIRE(!(a->flat && a->gated), MOE_ERR_INVALID, "step: flat and gated are separate modes");
+    plan->together = a->fused && sides_apart(a);
+    plan->f32_slots = a->f32_weights && !a->fused && !a->quant && a->dtype == MOE_F32 && a->S > 0 && f32_apart(a);
+    return MOE_OK;
+}
+
+extern "C" int moe_step_plan(const moe_step_args* a, int32_t* out) {
+    MOE_REQUIRE(out, MOE_ERR_INVALID, "step_plan: null result");
+    StepPlan plan;
+    const int rc = step_plan(a, &plan);
+    if (rc != MOE_OK) return rc;
+    out[0] = plan.together;
+    out[1] = plan.f32_slots;
+    return MOE_OK;
 }
 
 // Stage by stage from Python a step costs 8 to 10 foreign calls with some fifteen arguments each (about 80 us of host time);
@@ -42,23 +82,19 @@ static bool f32_apart(const moe_step_args* a) {
 // row scales, the gates and the zeroed padding rows from the received counts in one launch, the one that ranks the tokens (a launch
 // costs some 4.5 us even when it has nothing to do).
 extern "C" int moe_step(const moe_step_args* a, moe_stream_t stream) {
-    MOE_REQUIRE(a, MOE_ERR_INVALID, "step: null arguments");
+    StepPlan plan;
+    int rc = step_plan(a, &plan);
+    if (rc != MOE_OK) return rc;
     const int T = a->tokens, H = a->hidden, E = a->experts, k = a->topk, W = a->world, F = a->ffn, M = a->M, S = a->S;
-    MOE_REQUIRE(W > 0 && E > 0 && E % W == 0, MOE_ERR_INVALID, "step: %d experts on %d ranks", E, W);
-    MOE_REQUIRE(a->fused || !(a->flat || a->gated || a->q_dispatch), MOE_ERR_INVALID, "step: flat / gated / q_dispatch are fused modes");
-    MOE_REQUIRE(!a->q_dispatch || (a->quant && !a->flat), MOE_ERR_INVALID, "step: q_dispatch needs fp8 experts and fixed slots");
-    MOE_REQUIRE(!(a->flat && a->gated), MOE_ERR_INVALID, "step: flat and gated are separate modes");
     const int E_l = E / W;
     const float* out_gate = a->gated ? a->gate : nullptr;
-    int rc;
 #define MOE_STAGE(call)                           \
     do {                                          \
         if ((rc = (call)) != MOE_OK) return rc;   \
     } while (0)
     MOE_STAGE(moe_route_topk(a->x, a->router, a->bias, a->dtype, T, H, E, k, a->logits, a->idx, a->gate, a->route_ws, a->route_ws_bytes,
                              stream));
-    const bool together = a->fused && sides_apart(a);
-    if (together)
+    if (plan.together)
         MOE_STAGE(moe_count_and_prepare(a, (hipStream_t)stream));
     else
         MOE_STAGE(moe_count_and_offsets(a->idx, T, k, E, W, a->send_counts, a->expert_offs, a->dst_sizes, a->dst_offsets, a->caps, a->pos,
@@ -74,14 +110,12 @@ extern "C" int moe_step(const moe_step_args* a, moe_stream_t stream) {
     else
         MOE_STAGE(moe_pack_tokens(a->x, a->dtype, T, H, a->idx, a->pos, k, E_l, a->dst_sizes, a->dst_offsets, W, M, a->send, a->status,
                                   stream));
-    // fp32 experts: the GEMMs of small launches move the rows themselves (plumbing: 42.9 -> 38 us a step)
-    const bool f32_slots = a->f32_weights && !a->fused && !a->quant && a->dtype == MOE_F32 && S > 0 && f32_apart(a);
     // destination: rows in expert-major order
-    if (a->fused && !together)
+    if (a->fused && !plan.together)
         MOE_STAGE(moe_recv_prepare(a->recv_counts, W, E_l, a->flat ? 0 : M, S, a->gated ? a->recv_gate : nullptr,
                                    a->q_dispatch ? a->recv_scale : nullptr, a->row_map, a->gated ? a->row_gate : nullptr,
                                    a->q_dispatch ? a->xs : nullptr, a->expert_cnt, a->flat ? nullptr : a->ret, a->dtype, H, stream));
-    else if (!a->fused && !f32_slots)
+    else if (!a->fused && !plan.f32_slots)
         MOE_STAGE(moe_unpack_expert_major(a->recv, a->dtype, W, M, H, a->recv_counts, E_l, a->rows, S, a->expert_cnt, a->unpack_map, stream));
     const void* src = a->fused ? a->recv : a->rows;
     void* dst = a->fused ? a->ret : a->y;
@@ -96,7 +130,7 @@ extern "C" int moe_step(const moe_step_args* a, moe_stream_t stream) {
         MOE_STAGE(moe_grouped_mlp_fp8_mapped(src, n_buf, map, a->expert_cnt, S, H, F, E_l, (const uint8_t*)a->w1, a->s1, a->s_up,
                                              (const uint8_t*)a->w2, a->s2, a->xq, a->xs, a->hq, a->hscale, row_gate, dst, n_buf, map,
                                              a->part_ws, a->part_ws_bytes, stream));
-    else if (f32_slots)
+    else if (plan.f32_slots)
         MOE_STAGE(moe_mlp_f32_slots((const float*)a->recv, a->recv_counts, W, M, S, H, F, E_l, a->act, (const float*)a->w1,
                                     (const float*)a->w_up, (const float*)a->w2, (float*)a->rows, a->expert_cnt, (float*)a->hidden_ws,
                                     (float*)a->y, (float*)a->ret, (hipStream_t)stream));
@@ -112,7 +146,7 @@ extern "C" int moe_step(const moe_step_args* a, moe_stream_t stream) {
             MOE_STAGE(moe_grouped_gemm_mapped(a->hidden_ws, S, nullptr, a->w2, a->expert_cnt, S, F, H, E_l, MOE_ACT_NONE, dst, n_buf, map,
                                               a->part_ws, a->part_ws_bytes, stream));
     }
-    if (!a->fused && !f32_slots) MOE_STAGE(moe_return_pack(a->y, a->dtype, S, H, a->recv_counts, W, E_l, M, a->ret, a->ret_map, stream));
+    if (!a->fused && !plan.f32_slots) MOE_STAGE(moe_return_pack(a->y, a->dtype, S, H, a->recv_counts, W, E_l, M, a->ret, a->ret_map, stream));
     // the flat returned payload is indexed by position: one "destination" that holds all experts, offset 0
     if (a->flat)
         return moe_combine(a->returned, a->dtype, 1, T * k, H, a->idx, a->pos, a->gate, a->zero_off, T, k, E, a->out, a->status, stream);

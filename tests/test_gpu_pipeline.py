@@ -146,10 +146,10 @@ def test_fp32_rows_come_from_and_go_to_their_slots_in_the_gemms(T, H, E, k, W, F
         assert torch.equal(one[n], stages[n]), f"{n} differs"
 
 
-@pytest.mark.parametrize("over", ["recv", "ret"])
+@pytest.mark.parametrize("over", ["recv", "ret", "counts"])
 def test_fp32_scratch_over_rows_that_are_done_with(over):
     """The hidden activation may lie where the received rows lay (they are unpacked first), and the returned buffer where the hidden activation
-    did: the step then keeps the copies."""
+    or the counts per expert did: the step then keeps the copies."""
     from iris_testing_amd.configs import MoEConfig
     from iris_testing_amd.pipeline import DispatchPipeline
     cfg = MoEConfig("case", 7, 300, 256, "f32", 8, 2, 4, 128, "gelu")
@@ -159,7 +159,10 @@ def test_fp32_scratch_over_rows_that_are_done_with(over):
     pipe.step()
     torch.cuda.synchronize()
     want = {n: getattr(pipe, n).clone() for n in ("rows", "y", "ret")}
-    pipe.hidden = (world.recv if over == "recv" else pipe.ret).view(-1)[:pipe.S * cfg.ffn].view(pipe.S, cfg.ffn)
+    if over == "counts":
+        pipe.expert_cnt = pipe.ret.view(-1).view(torch.int32)[12:12 + cfg.e_local]
+    else:
+        pipe.hidden = (world.recv if over == "recv" else pipe.ret).view(-1)[:pipe.S * cfg.ffn].view(pipe.S, cfg.ffn)
     pipe.step()
     torch.cuda.synchronize()
     for n in want:

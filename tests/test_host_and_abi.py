@@ -332,3 +332,78 @@ def test_step_takes_the_buffers_of_the_moment(monkeypatch, kind, mode):
     pipe.out.data = keep
     pipe.step()
     assert seen["out"] == keep.data_ptr()
+
+
+# What the launches of a step that may go beside one another read and write (names of moe_step_args): the receive side's preparation, and the
+# source side from the counting to the packing; the two GEMMs of fp32 experts with the copies of the rows in them.
+PREPARE = ("recv_counts recv_gate recv_scale", "row_map expert_cnt row_gate xs ret")
+SOURCE = ("idx x gate", "send_counts expert_offs dst_sizes dst_offsets caps pos row_token count_ws send send_scale send_gate status")
+F32_UP = ("recv recv_counts w1 w_up", "rows expert_cnt hidden_ws")
+F32_DOWN = ("hidden_ws expert_cnt recv_counts w2", "y ret")
+NOT_BESIDE = "router bias logits route_ws s1 s_up s2 xq hq hscale unpack_map ret_map part_ws returned zero_off out"  # other launches alone
+
+
+@pytest.mark.parametrize("mode", ["f32", "f32 swiglu", "bf16", "gated", "flat", "fp8", "fp8 gated", "fp8 rows"])
+def test_step_keeps_launches_apart_whose_buffers_meet(mode):
+    """Every pair of a step's buffers laid over one another, by all and by one value: where one launch writes what another that would go
+    beside it reads or writes, the step goes stage by stage; next to each other they may lie."""
+    import ctypes
+    from iris_testing_amd import _lib as L
+    T, H, E, k, W, F, M, S = 24, 64, 12, 2, 3, 96, 17, 41
+    e_l, f32 = E // W, mode.startswith("f32")
+    flat, gated, q, quant = mode == "flat", "gated" in mode, mode in ("fp8", "fp8 gated"), "fp8" in mode
+    act = L.ACT["swiglu" if quant or "swiglu" in mode else "silu"]
+    B, slots, R = 4 if f32 else 2, W * M, T * k
+    size = dict(x=T * H * B, idx=R * 4, gate=R * 4, send_counts=E * 4, expert_offs=E * 4, dst_sizes=W * 4, dst_offsets=W * 4, caps=8, pos=R * 4,
+                row_token=R * 4, count_ws=4096, send=R * H * B if flat else slots * H * (1 if q else B), status=4, recv_counts=E * 4,
+                recv=S * H * B if flat else slots * H * (1 if q else B), expert_cnt=e_l * 4, ret=(S if flat else slots) * H * B)
+    size.update(dict(send_scale=slots * 4, recv_scale=slots * 4) if q else {}, **(dict(send_gate=slots * 4, recv_gate=slots * 4, row_gate=S * 4) if gated else {}))
+    if f32:
+        size.update(rows=S * H * 4, hidden_ws=S * F * 4, y=S * H * 4, w1=e_l * H * F * 4, w2=e_l * H * F * 4,
+                    **({"w_up": e_l * H * F * 4} if act == L.ACT["swiglu"] else {}))
+    else:
+        size.update(row_map=S * 4, **({"xs": S * 4} if quant else {}))
+    pointers = [n for n, t in L.StepArgs._fields_ if t is ctypes.c_void_p]
+    known = " ".join((*PREPARE, *SOURCE, *F32_UP, *F32_DOWN, NOT_BESIDE)).split()
+    assert set(known) == set(pointers), "a buffer of moe_step_args that this test does not know: say which launches use it"
+    at = {n: (i + 1) << 32 for i, n in enumerate(pointers) if n in size or n in NOT_BESIDE.split()}
+    out = (ctypes.c_int32 * 2)()
+
+    def plan(**moved):
+        a = L.StepArgs(tokens=T, hidden=H, experts=E, topk=k, world=W, ffn=F, act=act, dtype=L.MOE_F32 if f32 else L.MOE_BF16, M=M, S=S, fused=not f32,
+                       flat=flat, gated=gated, quant=quant, q_dispatch=q, f32_weights=f32, count_ws_bytes=size["count_ws"], **{**at, **moved})
+        L.check(L.lib().moe_step_plan(ctypes.byref(a), out))
+        return out[1 if f32 else 0]
+
+    used = lambda names: [n for n in names.split() if n in size and not (n == "xs" and not q) and not (n == "ret" and flat)]  # noqa: E731
+    bad = set()
+    if f32:
+        for reads, writes in (map(used, F32_UP), map(used, F32_DOWN)):
+            bad |= {frozenset((w, n)) for w in writes for n in reads + writes if n != w}
+    else:
+        (pr, pw), (sr, sw) = map(used, PREPARE), map(used, SOURCE)
+        bad |= {frozenset((p, s)) for p in pw for s in sr + sw} | {frozenset((p, s)) for p in pr for s in sw}
+    both_read = {frozenset((p, s)) for p in used(PREPARE[0]) for s in used(SOURCE[0])}  # (either way is right)
+    assert plan() == 1 and len(bad) > 10
+    for p in size:
+        for q_ in size:
+            if p == q_:
+                continue
+            pair = frozenset((p, q_))
+            for over in (at[p], at[p] + size[p] - 4):
+                got = plan(**{q_: over})
+                assert got == 0 if pair in bad else got == 1 or pair in both_read, (p, q_)
+            assert plan(**{q_: at[p] + size[p]}) == 1, (p, q_)
+    for n in NOT_BESIDE.split():
+        assert all(plan(**{n: at[p]}) == 1 for p in size), n
+
+
+def test_step_plan_refuses_what_a_step_refuses():
+    import ctypes
+    from iris_testing_amd import _lib as L
+    out = (ctypes.c_int32 * 2)()
+    a = L.StepArgs(experts=8, world=4, fused=1)
+    assert L.lib().moe_step_plan(ctypes.byref(a), out) == 0 and L.lib().moe_step_plan(ctypes.byref(a), None) == -1 and L.lib().moe_step_plan(None, out) == -1
+    for wrong in (dict(world=0), dict(world=3), dict(experts=0), dict(flat=1, gated=1), dict(q_dispatch=1), dict(fused=0, flat=1)):
+        b = L.StepArgs(**{**dict(experts=8, world=4, fused=1), **wrong})
+        assert L.lib().moe_step_plan(ctypes.byref(b), out) == -1, wrong
