@@ -287,6 +287,12 @@ size_t moe_gemm_part_workspace_bytes(void);
  * out[2] = parts that the K range of every small tile is cut into (1: not cut), out[3] = 64-byte stages of K per part.  Host-only: the
  * functions that the launches and kernels use; no counterpart in the reference. */
 int moe_gemm_launch_plan(int S_rows, int E_l, int K, int N, int act, int fp8, int cus, size_t part_ws_bytes, int tiles, int32_t* out);
+/* How an fp32 grouped GEMM of S_rows rows in E_l groups, K x N, is launched on `cus` compute units.  side 0: rows in expert-major order on
+ * both ends; 1: result rows go to their slots of the returned buffer as well; 2: rows come from their slots of the received buffer.  out[0] =
+ * edge of its square tiles, out[1] = sets of four waves to a tile, out[2], out[3] = workgroups along columns and rows.
+ * MOE_ERR_UNSUPPORTED where such a launch does not move rows (64 x 64 tiles; side 1 with an activation).  Host-only; no counterpart in
+ * the reference. */
+int moe_gemm_f32_plan(int S_rows, int E_l, int K, int N, int act, int side, int cus, int32_t* out);
 /* A plan that launches followed before they handed a part-filled last round to small tiles, kept for its callers: total_tiles large
  * tiles on a grid of `grid` workgroups, k_stages 64-byte stages of K (even), room for max_units part tiles: out[0] = tiles taken whole,
  * out[1] = parts per remaining tile (1: no split), out[2] = K stages per part, out[3] = work units in all. */

@@ -1740,18 +1740,36 @@ constexpr int gg_f32_lds(int R, int KG, bool up) {
     const int KC = 128 / R * KG;
     return (32 * R * (KC + 4) + (up ? 2 : 1) * KC * (32 * R + 16)) * 4;
 }
+// How an fp32 launch goes (the one place where that is decided; moe_gemm_f32_plan shows it).
+struct F32Plan {
+    int tile, sets;
+    int cols, rows;  // workgroups of the tiles
+};
 // 64 x 64 tiles once they give every compute unit two workgroups, 32 x 32 below
-bool gg_f32_big(int S_rows, int N) { return (long long)ceil_div(N, 64) * ceil_div(S_rows, 64) >= 2 * num_cus(); }
+bool gg_f32_big(int S_rows, int N, int cus) { return (long long)ceil_div(N, 64) * ceil_div(S_rows, 64) >= 2 * cus; }
+static int f32_plan(int S_rows, int E_l, int K, int N, int epi, int side, int cus, F32Plan* p) {
+    const bool big = gg_f32_big(S_rows, N, cus);
+    // (a side that a launch does not have would be left out without a word: rows or padding unwritten)
+    MOE_REQUIRE(side == F32_ROWS || !big, MOE_ERR_UNSUPPORTED, "grouped_gemm: 64 x 64 tiles do not move rows (%d rows, %d columns)", S_rows, N);
+    MOE_REQUIRE(side != F32_RETURN || epi == EPI_NONE, MOE_ERR_UNSUPPORTED, "grouped_gemm: results go to their slots without an activation (%d)", epi);
+    // Two sets of waves to a tile up to two workgroups a compute unit (half a tile per group more than the rows fill): 344 tiles, K 1000
+    // 30.4 -> 21.7 us, but 832 tiles, K 1024 51.5 -> 58.0 (one such workgroup fits a compute unit, three of the others do).
+    const bool split = !big && K > 128 && (long long)ceil_div(N, 32) * (ceil_div(S_rows, 32) + E_l / 2) <= 2 * cus;
+    p->tile = big ? 64 : 32;
+    p->sets = split ? 2 : 1;
+    p->cols = ceil_div(N, p->tile);
+    p->rows = ceil_div(S_rows, p->tile) + E_l;
+    return MOE_OK;
+}
 int launch_f32(const float* A, const float* W, const float* U, float* C, const int32_t* cnt, int E_l, int K, int N, int S_rows,
                int epi, hipStream_t s, int side = F32_ROWS, F32Side sd = {}) {
     if (S_rows == 0) return MOE_OK;
     const bool vec = K % 4 == 0 && N % 4 == 0 && (((uintptr_t)(side == F32_UNPACK ? sd.buf : A) | (uintptr_t)W | (uintptr_t)U) & 15) == 0;
-    const bool big = gg_f32_big(S_rows, N);
-    const int tile = big ? 64 : 32;
-    dim3 grid(ceil_div(N, tile), ceil_div(S_rows, tile) + E_l);
-    // Two sets of waves to a tile up to two workgroups a compute unit (half a tile per group more than the rows fill): 344 tiles, K 1000
-    // 30.4 -> 21.7 us, but 832 tiles, K 1024 51.5 -> 58.0 (one such workgroup fits a compute unit, three of the others do).
-    const bool split = !big && K > 128 && (long long)ceil_div(N, 32) * (ceil_div(S_rows, 32) + E_l / 2) <= 2 * num_cus();
+    F32Plan plan;
+    const int rc = f32_plan(S_rows, E_l, K, N, epi, side, num_cus(), &plan);
+    if (rc) return rc;
+    const bool big = plan.tile == 64, split = plan.sets == 2;
+    dim3 grid(plan.cols, plan.rows);
     // (a workgroup for every 16 rows of the returned buffer that S_rows cannot fill, up to a round of the chip)
     sd.tiles_y = grid.y;
     if (side == F32_RETURN) grid.y += std::min(ceil_div(std::max(sd.W * sd.M - S_rows, 1), 16 * (int)grid.x), ceil_div(num_cus(), (int)grid.x));
@@ -1898,6 +1916,16 @@ extern "C" int moe_gemm_launch_plan(int S_rows, int E_l, int K, int N, int act, 
     return MOE_OK;
 }
 
+extern "C" int moe_gemm_f32_plan(int S_rows, int E_l, int K, int N, int act, int side, int cus, int32_t* out) {
+    MOE_REQUIRE(S_rows > 0 && E_l > 0 && K > 0 && N > 0 && act >= EPI_NONE && act <= EPI_SWIGLU && side >= F32_ROWS && side <= F32_UNPACK &&
+                cus > 0 && out, MOE_ERR_INVALID, "gemm_f32_plan: bad arguments");
+    F32Plan p;
+    const int rc = f32_plan(S_rows, E_l, K, N, act, side, cus, &p);
+    if (rc) return rc;
+    out[0] = p.tile; out[1] = p.sets; out[2] = p.cols; out[3] = p.rows;
+    return MOE_OK;
+}
+
 extern "C" size_t moe_gemm_part_workspace_bytes(void) { return gs_workspace_bytes(num_cus()); }
 
 extern "C" int moe_grouped_gemm_mapped(const void* a_base, int a_rows, const int32_t* a_row_map, const void* packed,
@@ -1990,7 +2018,7 @@ int moe_mlp_f32_slots(const float* recv, const int32_t* recv_counts, int W, int 
     MOE_REQUIRE(W > 0 && W * E_l <= MOE_MAX_EXPERTS && M >= 1 && recv_counts && ret, MOE_ERR_INVALID, "return_pack: bad arguments");
     MOE_REQUIRE((long long)W * M < (1ll << 31), MOE_ERR_UNSUPPORTED, "return_pack: W*M too large");
     // (with large tiles the rows' places, looked up slab by slab, cost more than the copies: H 512, F 1024, 54 940 rows 1443 -> 1635 us a step, 14 613 456 -> 480)
-    const bool up = !gg_f32_big(S_rows, F), down = !gg_f32_big(S_rows, H);
+    const bool up = !gg_f32_big(S_rows, F, num_cus()), down = !gg_f32_big(S_rows, H, num_cus());
     int rc = up ? MOE_OK : moe_unpack_expert_major(recv, MOE_F32, W, M, H, recv_counts, E_l, rows, S_rows, expert_cnt, nullptr, s);
     if (rc) return rc;
     rc = launch_f32(rows, w1, w_up, hidden_ws, expert_cnt, E_l, H, F, S_rows, act, s, up ? F32_UNPACK : F32_ROWS,

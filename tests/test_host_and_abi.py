@@ -249,6 +249,34 @@ def test_tile_rule_counts_on_parts_only_where_there_is_room_for_them():
     assert full == ctr + (8 << 20) and differ > 20 and split > 100
 
 
+def test_fp32_launch_moves_rows_or_refuses():
+    """A launch of the fp32 GEMM that cannot move rows (large tiles; an activation on the way to the slots) says so and is not launched
+    without them; one that can covers every tile of any distribution of the rows."""
+    import ctypes
+    import random
+    from iris_testing_amd import _lib as L
+    rnd, out, seen = random.Random(7), (ctypes.c_int32 * 4)(), {"big": 0, "split": 0, "one": 0}
+    for _ in range(3000):
+        S, E_l, K, N = int(2 ** rnd.uniform(0, 15)), rnd.choice([1, 2, 15, 64, 130]), int(2 ** rnd.uniform(0, 12)), int(2 ** rnd.uniform(0, 12))
+        act, cus = rnd.choice(["none", "gelu", "silu", "swiglu"]), rnd.choice([256, 256, 304, 64])
+        args = (S, E_l, K, N, L.ACT[act])
+        assert L.lib().moe_gemm_f32_plan(*args, 0, cus, out) == 0
+        tile, sets, cols, rows = plan = tuple(out)
+        assert tile in (32, 64) and sets in (1, 2) and cols * tile >= N and (sets == 1 or tile == 32 and K > 128)
+        seen["big" if tile == 64 else "split" if sets == 2 else "one"] += 1
+        cnt = [0] * E_l
+        for _ in range(20):
+            cnt[rnd.randrange(E_l)] += S // 20
+        cnt[rnd.randrange(E_l)] += S - sum(cnt)
+        assert sum(-(-c // tile) for c in cnt) <= rows
+        for side in (1, 2):
+            refused = tile == 64 or (side == 1 and act != "none")
+            assert L.lib().moe_gemm_f32_plan(*args, side, cus, out) == (-2 if refused else 0)
+            assert refused or tuple(out) == plan
+    assert min(seen.values()) > 100, seen
+    assert L.lib().moe_gemm_f32_plan(0, 1, 4, 4, 0, 0, 256, out) == -1 and L.lib().moe_gemm_f32_plan(1, 1, 4, 4, 0, 3, 256, out) == -1
+
+
 def test_results_in_one_allocation_do_not_share_a_version_counter():
     """What a caller changes in place must not look changed elsewhere: autograd refuses to use a saved tensor whose counter moved."""
     from iris_testing_amd import ops
