@@ -191,7 +191,7 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
         if (d < 2 * RA) gg_dma16(ap + (d & 1) * ROWB, aoff[d >> 1], la0 + slot * 2 * ASZ + (d & 1) * ASZ + (d >> 1) * 64 * ROWB);
         else if (d < 2 * (RA + RB)) {
             const int e = d - 2 * RA;
-            gg_dma16(bp[e / RB][BN_PAIR ? e % RB : 0], boff[e % RB], lb0 + slot * 2 * BSZ + (e / RB) * BSZ + (e % RB) * 64 * ROWB);
+            gg_dma16(bp[e / RB][BN_PAIR ? e % RB : 0], boff[e % RB], lb0, slot * 2 * BSZ + (e / RB) * BSZ + (e % RB) * 64 * ROWB);
         } else if constexpr (BSA) gg_dma4(sp, soff, ls0 + slot * 256);
     };
 #define GS_PAIR_PTRS(pr)                                                    \

@@ -435,3 +435,28 @@ def test_step_plan_refuses_what_a_step_refuses():
     for wrong in (dict(world=0), dict(world=3), dict(experts=0), dict(flat=1, gated=1), dict(q_dispatch=1), dict(fused=0, flat=1)):
         b = L.StepArgs(**{**dict(experts=8, world=4, fused=1), **wrong})
         assert L.lib().moe_step_plan(ctypes.byref(b), out) == -1, wrong
+
+
+def test_loads_in_inline_assembly_wait_for_their_scalar_base():
+    """A scalar register that a vector instruction wrote may be a load's base five wait states later at the earliest, and the compiler does not
+    count them into an asm statement: every such load's base is moved inside its statement, or the statement waits as long before the load."""
+    def registers(name):  # s[96:99] -> s96 .. s99; an operand is itself
+        m = re.fullmatch(r"s\[(\d+):(\d+)\]", name)
+        return {f"s{i}" for i in range(int(m[1]), int(m[2]) + 1)} if m else {name}
+    seen = 0
+    csrc = os.path.join(ROOT, "iris_testing_amd", "csrc")
+    for name in sorted(os.listdir(csrc)):
+        if not name.endswith((".h", ".hip")):
+            continue
+        for text in re.findall(r'asm volatile\("([^"]*)"', open(os.path.join(csrc, name)).read()):
+            states, moved = 0, set()
+            for op in filter(None, text.split(r"\n\t")):
+                kind, *args = op.replace(",", " ").split()
+                if "load" in kind:
+                    assert kind.startswith(("global_load_lds", "buffer_load")), op
+                    seen += 1
+                    assert registers(args[1]) <= moved or states >= 5, (name, text)
+                elif kind in ("s_mov_b32", "s_mov_b64"):
+                    moved |= registers(args[0])
+                states += int(args[0]) + 1 if kind == "s_nop" else 1
+    assert seen == 3
