@@ -577,7 +577,9 @@ __global__ __launch_bounds__(WPB * WAVE) void gather_rows_kernel(const u32x4* __
         recv_tables(tables, q, a.W, a.E_l);
         a.rc = tables.rc; a.src_off = tables.src_off; a.row_off = tables.row_off; a.flat_off = tables.flat_off;
     }
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = lane_id();
+    // (row by row the wave's number stays in a vector register: in a scalar one the look-up of a row becomes a chain of scalar loads and divisions
+    // that short rows do not cover; 32768 rows of 256 bytes, fixed-slot pack 12.7 us and 11.7, payload 10.3 and 9.8, receive layout 12.9 and 12.1)
+    const int wave = RPW > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE) : threadIdx.x / WAVE, lane = lane_id();
     if constexpr (RPW > 1) {
         for (unsigned r0 = (blockIdx.x * WPB + wave) * RPW; r0 < (unsigned)n_rows; r0 += gridDim.x * WPB * RPW) {
             const u32x4* from[RPW];
