@@ -540,10 +540,15 @@ __device__ __forceinline__ int source_row(const RowSource& a, int r) {
     }
 }
 
-// Rows of a copy that a wave takes together: of 2 to 4 KB two (eight 16-byte loads of a lane in flight instead of four; 4096 x 2 rows of 3 KB:
-// payload 11.2 -> 10.2 us, unpack 11.6 -> 9.8, return 12.1 -> 10.4), where rows are many enough to keep every place on the chip taken (1024
-// rows one by one or two by two: the same).  Shorter rows gain nothing from four together (8192 x 2 of 1 KB 8.3 -> 9.2) and few rows lose.
-inline int copy_rows(int n_rows, int row_vec) { return row_vec > 2 * WAVE && row_vec <= 4 * WAVE && n_rows >= 4096 ? 2 : 1; }
+// Rows of a copy that a wave takes together: of 2 to 4 KB two (eight 16-byte loads of a lane in flight instead of four), from as many rows on as
+// keep every place on the chip taken, up to where the waves of single rows fill the memory's queues by themselves.  One by one / together, us: 4096 rows
+// of 3 KB payload 7.4 / 6.4, unpack 8.1 / 7.7, return 8.1 / 7.8; 8192 of 3.5 KB 13.0 / 11.4, 14.2 / 12.1, 14.5 / 12.8; 12288 of 3 KB 14.6 / 13.3, 16.1 / 14.8,
+// 16.5 / 16.0; but 14800 payload + 9 %, the others equal, 24576 26.8 / 28.2, 28.4 / 30.0, 28.9 / 30.4, 65536 68 / 71, 69 / 74, 70 / 75.  The fixed-slot pack
+// of rows up to 2.5 KB gains at any number (65536 of 2 KB 57 / 51).  Shorter rows gain nothing (8192 of 1 KB 5 to 10 % more).
+inline int copy_rows(int mode, int n_rows, int row_vec) {
+    if (row_vec <= 2 * WAVE || row_vec > 4 * WAVE || n_rows < 4096) return 1;
+    return n_rows <= 12288 || (mode == SRC_PACK && row_vec <= 160) ? 2 : 1;
+}
 // RPW rows of at most 8 / RPW vectors a lane, row j from src[from[j]] (below 0: zeros) to dst[j]; NT_STORE: non-temporal stores
 template <int RPW, bool NT_STORE>
 __device__ __forceinline__ void copy_rows_together(const u32x4* const (&from)[RPW], u32x4* const (&to)[RPW], int row_vec, int lane) {
@@ -943,7 +948,7 @@ int launch_combine(const void* ret, const int32_t* idx, const int32_t* pos, cons
 
 int gather_rows(const void* src, void* dst, const RowSource& a, int n_rows, int row_bytes, hipStream_t s) {
     if (n_rows == 0) return MOE_OK;
-    const int rpw = copy_rows(n_rows, row_bytes / 16), blocks = min(ceil_div(n_rows, 4 * rpw), 65535 * 8);
+    const int rpw = copy_rows(a.mode, n_rows, row_bytes / 16), blocks = min(ceil_div(n_rows, 4 * rpw), 65535 * 8);
 #define MOE_GATHER(R) gather_rows_kernel<4, false, R><<<blocks, 4 * WAVE, 0, s>>>((const u32x4*)src, (u32x4*)dst, a, n_rows, row_bytes / 16, RecvCounts{})
     if (rpw == 2) MOE_GATHER(2);
     else MOE_GATHER(1);
@@ -1284,7 +1289,7 @@ static int recv_driven(const char* who, int mode, const void* src, void* dst, in
     a.W = W; a.E_l = E_l; a.M = M; a.CAP = CAP;
     a.status = status;
     // (one workgroup at least, for pca and the totals; at most what the chip holds at once, which then walks the rows)
-    const int row_vec = H * dtype_size(dtype) / 16, rpw = copy_rows(n_out, row_vec), blocks = max(1, min(ceil_div(n_out, 4 * rpw), 256 * 7));
+    const int row_vec = H * dtype_size(dtype) / 16, rpw = copy_rows(mode, n_out, row_vec), blocks = max(1, min(ceil_div(n_out, 4 * rpw), 256 * 7));
 #define MOE_GATHER(R) gather_rows_kernel<4, true, R><<<blocks, 4 * WAVE, 0, s>>>((const u32x4*)src, (u32x4*)dst, a, n_out, row_vec, q)
     if (rpw == 2) MOE_GATHER(2);
     else MOE_GATHER(1);
@@ -1543,7 +1548,7 @@ extern "C" int moe_a2a_place(const moe_a2a_source* sources, int dtype, int W, in
     for (int s0 = 0; s0 < W; s0 += A2A_SRC) {
         const int ns = min(A2A_SRC, W - s0);
         // (four short rows to a wave where rows are many, see copy_rows: 28672 rows of 1.5 KB, 16384 of them copied 20.8 -> 18.6 us)
-        const int row_vec = H * dtype_size(dtype) / 16, n = E_l * ns * CAP, rpw = n >= 8192 && row_vec <= 2 * WAVE ? 4 : copy_rows(n, row_vec);
+        const int row_vec = H * dtype_size(dtype) / 16, n = E_l * ns * CAP, rpw = n >= 8192 && row_vec <= 2 * WAVE ? 4 : n >= 4096 && row_vec > 2 * WAVE && row_vec <= 4 * WAVE ? 2 : 1;
         const int blocks = min(ceil_div(n, 4 * rpw), 256 * 8);
 #define MOE_PLACE(R)                                                                                                                      \
     a2a_place_kernel<R><<<blocks, 256, 0, (hipStream_t)stream>>>(a2a_slice(sources, s0, ns), s0, ns, W, E_l, CAP, row_vec, (u32x4*)token_buf, \
