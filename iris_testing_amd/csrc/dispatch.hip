@@ -543,11 +543,11 @@ __device__ __forceinline__ int source_row(const RowSource& a, int r) {
 // Rows of a copy that a wave takes together: of 2 to 4 KB two (eight 16-byte loads of a lane in flight instead of four), from as many rows on as
 // keep every place on the chip taken, up to where the waves of single rows fill the memory's queues by themselves.  One by one / together, us: 4096 rows
 // of 3 KB payload 7.4 / 6.4, unpack 8.1 / 7.7, return 8.1 / 7.8; 8192 of 3.5 KB 13.0 / 11.4, 14.2 / 12.1, 14.5 / 12.8; 12288 of 3 KB 14.6 / 13.3, 16.1 / 14.8,
-// 16.5 / 16.0; but 14800 payload + 9 %, the others equal, 24576 26.8 / 28.2, 28.4 / 30.0, 28.9 / 30.4, 65536 68 / 71, 69 / 74, 70 / 75.  The fixed-slot pack
+// 16.5 / 16.0; 13500 payload 3 to 9 % more, the others 1 to 7 % less; but 14800 the others equal, 24576 26.8 / 28.2, 28.4 / 30.0, 28.9 / 30.4, 65536 68 / 71, 69 / 74, 70 / 75.  The fixed-slot pack
 // of rows up to 2.5 KB gains at any number (65536 of 2 KB 57 / 51).  Shorter rows gain nothing (8192 of 1 KB 5 to 10 % more).
 inline int copy_rows(int mode, int n_rows, int row_vec) {
     if (row_vec <= 2 * WAVE || row_vec > 4 * WAVE || n_rows < 4096) return 1;
-    return n_rows <= 12288 || (mode == SRC_PACK && row_vec <= 160) ? 2 : 1;
+    return n_rows <= (mode == SRC_MAP ? 12288 : 14336) || (mode == SRC_PACK && row_vec <= 160) ? 2 : 1;
 }
 // RPW rows of at most 8 / RPW vectors a lane, row j from src[from[j]] (below 0: zeros) to dst[j]; NT_STORE: non-temporal stores
 template <int RPW, bool NT_STORE>
@@ -1030,7 +1030,7 @@ __global__ __launch_bounds__(256) void a2a_place_kernel(const A2aSources q, int 
         for (int i = tid; i < n_sync; i += blockDim.x) token_sync[i] = W;
     }
     __syncthreads();
-    const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE), wpb = blockDim.x / WAVE;
+    const int wave = RPW > 1 ? __builtin_amdgcn_readfirstlane(tid / WAVE) : tid / WAVE, wpb = blockDim.x / WAVE;  // (as in gather_rows_kernel: 65536 rows of 3 KB 67 and 60 us)
     const unsigned n_rows = (unsigned)(E_l * ns * CAP);
     // row r of the launch: (e, s, j); the source's row, or NULL: zeros
     auto row = [&](unsigned r, u32x4*& to) -> const u32x4* {
@@ -1538,6 +1538,19 @@ extern "C" int moe_a2a_max_count(const moe_a2a_source* sources, int W, int E_l, 
     return moe_check_launch("a2a_max_count");
 }
 
+// Rows of the exchange that a wave takes together: two of up to 3 KB (few rows: 4 KB), from where they keep the chip busy to
+// where the waves of single rows do, and four of very many short ones.
+// One by one / together, us (n rows copied, 1.1 to 1.2 n slots): 8192 rows of 1.5 KB 9.2 / 8.4, 2 KB 10.9 / 9.9; 16384 of 1 KB 11.7 / 11.0, 1.5 KB
+// 16.2 / 14.3; 32768 of 512 bytes 14.5 / 14.4, 1.5 KB 23.1 / 19.9, 2.3 KB 27.7 / 26.3; 4096 of 3 KB 9.4 / 7.9; but of 2.3 KB 6.6 / 7.1, 6000 of 2 KB 7.0 / 7.6, 8192 of 1 KB
+// 6.5 / 7.0, of 256 bytes 5.5 / 6.1, 32768 of 256 bytes 10.7 / 12.2, 65536 of 3 KB 60 / 64, 24576 of 3.5 KB 31.5 / 34.7.  Four together cost 0 to 10 % more
+// than two, but 65536 of 512 bytes 25.7 / 23.6 / 22.4 (two, four), of 1 KB 29.3 / 27.0 / 25.5, of 1.5 KB 38.6 / 36.3 / 38.2.
+static int place_rows(int n, int row_vec) {
+    const long long vecs = (long long)n * row_vec;
+    if (row_vec > 2 * WAVE) return n >= (row_vec <= 160 ? 6144 : 4096) && ((row_vec <= 3 * WAVE && vecs <= 8ll << 20) || (row_vec <= 4 * WAVE && n <= 6144)) ? 2 : 1;
+    if (n >= 49152 && row_vec <= 80) return 4;
+    return n >= 8192 && vecs >= (row_vec >= 48 ? 3ll : 4ll) << 18 && vecs <= 8ll << 20 ? 2 : 1;
+}
+
 extern "C" int moe_a2a_place(const moe_a2a_source* sources, int dtype, int W, int E_l, int CAP, int H, void* token_buf, int32_t* pca,
                              int32_t* counts_ready, int n_ready, int32_t* token_sync, int n_sync, moe_stream_t stream) {
     int rc = a2a_check("a2a_place", sources, W, E_l);
@@ -1547,8 +1560,7 @@ extern "C" int moe_a2a_place(const moe_a2a_source* sources, int dtype, int W, in
     MOE_REQUIRE(token_buf && pca, MOE_ERR_INVALID, "a2a_place: null pointer");
     for (int s0 = 0; s0 < W; s0 += A2A_SRC) {
         const int ns = min(A2A_SRC, W - s0);
-        // (four short rows to a wave where rows are many, see copy_rows: 28672 rows of 1.5 KB, 16384 of them copied 20.8 -> 18.6 us)
-        const int row_vec = H * dtype_size(dtype) / 16, n = E_l * ns * CAP, rpw = n >= 8192 && row_vec <= 2 * WAVE ? 4 : n >= 4096 && row_vec > 2 * WAVE && row_vec <= 4 * WAVE ? 2 : 1;
+        const int row_vec = H * dtype_size(dtype) / 16, n = E_l * ns * CAP, rpw = place_rows(n, row_vec);
         const int blocks = min(ceil_div(n, 4 * rpw), 256 * 8);
 #define MOE_PLACE(R)                                                                                                                      \
     a2a_place_kernel<R><<<blocks, 256, 0, (hipStream_t)stream>>>(a2a_slice(sources, s0, ns), s0, ns, W, E_l, CAP, row_vec, (u32x4*)token_buf, \

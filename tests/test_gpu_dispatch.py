@@ -644,7 +644,7 @@ def test_router_segments_by_two_sets_of_waves(T, H, E, k, bias):
 
 @pytest.mark.parametrize("H", [1024, 1032, 2040, 2048, 2056])
 def test_copies_of_many_rows_two_and_four_to_a_wave(H):
-    """Rows of 2 to 4 KB are copied two, the exchange's shorter ones four to a wave when there are many.  A copy moves columns without
+    """Rows of 2 to 4 KB are copied two to a wave when there are many.  A copy moves columns without
     looking at them: the first 64 of every output are those of the same copy of 64-column rows, which go one by one."""
     T, E, W, k, E_l = 2051, 24, 4, 2, 6
     g = torch.Generator(device=DEV).manual_seed(H)
@@ -673,10 +673,10 @@ def test_copies_of_many_rows_two_and_four_to_a_wave(H):
 
 
 @pytest.mark.parametrize("H", [8, 768, 1024, 1032, 2048, 2056])
-def test_exchange_of_many_rows(H):
-    """The exchange by one, two and four rows to a wave, with a source that sends nothing, one whose payload ends early, and an
+def test_exchange_of_many_rows(H, cap=641):
+    """The exchange by one and two rows to a wave, with a source that sends nothing, one whose payload ends early, and an
     odd number of rows."""
-    W, E_l, cap = 5, 3, 641
+    W, E_l = 5, 3
     g = torch.Generator(device=DEV).manual_seed(H)
     counts = torch.randint(0, cap + 1, (W, E_l), generator=torch.Generator().manual_seed(H)).to(torch.int32)
     counts[0, 0], counts[1, 2] = cap, 0
@@ -699,3 +699,9 @@ def test_exchange_of_many_rows(H):
             c = 0 if s == 3 else int(counts[s, e])
             assert torch.equal(out[e, s, :c], rows[s][at:at + c]) and not bool(out[e, s, c:].any()), (s, e)
             at += c
+
+
+@pytest.mark.parametrize("H,cap", [(8, 3281), (640, 3277), (648, 3277), (504, 3276)])
+def test_exchange_of_very_many_short_rows(H, cap):
+    """Either side of where four rows go to a wave: 49152 slots, rows of 1280 bytes."""
+    test_exchange_of_many_rows(H, cap)
