@@ -1752,9 +1752,13 @@ static int f32_plan(int S_rows, int E_l, int K, int N, int epi, int side, int cu
     // (a side that a launch does not have would be left out without a word: rows or padding unwritten)
     MOE_REQUIRE(side == F32_ROWS || !big, MOE_ERR_UNSUPPORTED, "grouped_gemm: 64 x 64 tiles do not move rows (%d rows, %d columns)", S_rows, N);
     MOE_REQUIRE(side != F32_RETURN || epi == EPI_NONE, MOE_ERR_UNSUPPORTED, "grouped_gemm: results go to their slots without an activation (%d)", epi);
-    // Two sets of waves to a tile up to two workgroups a compute unit (half a tile per group more than the rows fill): 344 tiles, K 1000
-    // 30.4 -> 21.7 us, but 832 tiles, K 1024 51.5 -> 58.0 (one such workgroup fits a compute unit, three of the others do).
-    const bool split = !big && K > 128 && (long long)ceil_div(N, 32) * (ceil_div(S_rows, 32) + E_l / 2) <= 2 * cus;
+    // Two sets of waves to a tile where the chip takes all tiles at once: one such workgroup fits a compute unit (82 KB of LDS), three of the others
+    // do.  One set / two, us at K 132, 400 and 1024: 256 tiles ratio 0.95, 0.85 and 0.71, 192 0.90, 0.82, 0.74; but 264 to 420 tiles 1.14, 1.11 and 1.06, 640
+    // 1.35, 1.33 and 1.33.  Counted are the tiles that rows spread at random make: one per group that has any while groups are small, then about half a
+    // tile per group more than the rows fill; near the line either choice is right for about half the spreads.
+    const double per = (double)S_rows / E_l;
+    const double tiles = ceil_div(N, 32) * (E_l == 1 ? (double)ceil_div(S_rows, 32) : per < 16 ? E_l * (1 - exp(-per)) : S_rows / 32.0 + 0.484 * E_l);
+    const bool split = !big && K > 128 && tiles <= (E_l == 1 ? 1.0 : 1.03) * cus;
     p->tile = big ? 64 : 32;
     p->sets = split ? 2 : 1;
     p->cols = ceil_div(N, p->tile);

@@ -277,6 +277,34 @@ def test_fp32_launch_moves_rows_or_refuses():
     assert L.lib().moe_gemm_f32_plan(0, 1, 4, 4, 0, 0, 256, out) == -1 and L.lib().moe_gemm_f32_plan(1, 1, 4, 4, 0, 3, 256, out) == -1
 
 
+def test_fp32_tiles_get_two_sets_of_waves_while_they_are_one_round():
+    """A compute unit holds one workgroup of two sets: with rows spread over the groups at random, they are taken where the tiles
+    are about as many as the compute units or fewer, and only there."""
+    import ctypes
+    import random
+    from iris_testing_amd import _lib as L
+    rnd, out, seen = random.Random(11), (ctypes.c_int32 * 4)(), [0, 0]
+    for _ in range(2000):
+        S, E_l, K, N, cus = int(2 ** rnd.uniform(0, 12)), rnd.choice([1, 2, 15, 32, 64]), rnd.choice([64, 128, 129, 400, 2000]), int(2 ** rnd.uniform(5, 11)), rnd.choice([256, 304, 64])
+        L.check(L.lib().moe_gemm_f32_plan(S, E_l, K, N, L.ACT["none"], 0, cus, out))
+        tile, sets, cols, _ = out
+        if tile != 32:
+            continue
+        tiles = 0
+        for _ in range(8):
+            cnt = [0] * E_l
+            for _ in range(S):
+                cnt[rnd.randrange(E_l)] += 1
+            tiles += cols * sum(-(-c // 32) for c in cnt) / 8
+        slack = 1.0 if E_l == 1 else 1.2
+        if sets == 2:
+            assert K > 128 and tiles <= slack * cus, (S, E_l, K, N, cus, tiles)
+        elif K > 128:
+            assert slack * tiles > cus, (S, E_l, K, N, cus, tiles)
+        seen[sets - 1] += K > 128
+    assert min(seen) > 200, seen
+
+
 def test_results_in_one_allocation_do_not_share_a_version_counter():
     """What a caller changes in place must not look changed elsewhere: autograd refuses to use a saved tensor whose counter moved."""
     from iris_testing_amd import ops
