@@ -1415,16 +1415,20 @@ extern "C" int moe_recv_row_map_flat(const int32_t* recv_counts, int W, int E_l,
     return moe_recv_row_map_gated(recv_counts, W, E_l, 0, n_rows, nullptr, row_map, nullptr, expert_cnt, stream);
 }
 
+// (E_l = 0: no row is one)
+static int zero_padding(void* buf, int dtype, int W, int M, int H, const int32_t* recv_counts, int E_l, hipStream_t s) {
+    const int run = padding_run(W * M, H * dtype_size(dtype));
+    zero_padding_rows_kernel<<<ceil_div(ceil_div(W * M, run), 4), 256, 0, s>>>((u32x4*)buf, recv_counts, W, E_l, M, H * dtype_size(dtype) / 16, run);
+    return moe_check_launch("zero_padding_rows");
+}
+
 extern "C" int moe_zero_padding_rows(void* buf, int dtype, int W, int M, int H, const int32_t* recv_counts, int E_l,
                                      moe_stream_t stream) {
     int rc = check_rows("zero_padding_rows", dtype, H);
     if (rc) return rc;
     MOE_REQUIRE(W > 0 && E_l > 0 && M >= 1 && buf && recv_counts, MOE_ERR_INVALID, "zero_padding_rows: bad arguments");
     MOE_REQUIRE((long long)W * M < (1ll << 31), MOE_ERR_UNSUPPORTED, "zero_padding_rows: too many rows");
-    const int run = padding_run(W * M, H * dtype_size(dtype));
-    zero_padding_rows_kernel<<<ceil_div(ceil_div(W * M, run), 4), 256, 0, (hipStream_t)stream>>>((u32x4*)buf, recv_counts, W, E_l, M,
-                                                                                                 H * dtype_size(dtype) / 16, run);
-    return moe_check_launch("zero_padding_rows");
+    return zero_padding(buf, dtype, W, M, H, recv_counts, E_l, (hipStream_t)stream);
 }
 
 extern "C" int moe_shuffle(const void* token_buf, int dtype, int E_l, int W, int CAP, int H, const int32_t* pca,
@@ -1452,9 +1456,15 @@ extern "C" int moe_shuffle_backward(const void* grad_rows, int dtype, int E_l, i
 
 extern "C" int moe_return_pack(const void* y, int dtype, int S_rows, int H, const int32_t* recv_counts, int W, int E_l,
                                int M, void* ret, int32_t* map_ws, moe_stream_t stream) {
-    (void)S_rows, (void)map_ws;
+    (void)map_ws;
     MOE_REQUIRE(M >= 1, MOE_ERR_INVALID, "return_pack: M=%d", M);
     MOE_REQUIRE((long long)W * M < (1ll << 31), MOE_ERR_UNSUPPORTED, "return_pack: W*M too large");
+    if (S_rows == 0) {  // (a rank that received nothing: no result rows, which then have no storage either, and every slot is padding)
+        const int rc = check_rows("return_pack", dtype, H);
+        if (rc) return rc;
+        MOE_REQUIRE(W > 0 && E_l > 0 && W * E_l <= MOE_MAX_EXPERTS && recv_counts && ret, MOE_ERR_INVALID, "return_pack: bad arguments");
+        return zero_padding(ret, dtype, W, M, H, recv_counts, 0, (hipStream_t)stream);
+    }
     return recv_driven("return_pack", SRC_RETURN, y, ret, dtype, H, {recv_counts, E_l, 1, nullptr, nullptr}, W, E_l, M, 1, W * M, nullptr,
                        (hipStream_t)stream);
 }

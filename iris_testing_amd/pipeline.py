@@ -108,7 +108,7 @@ class DispatchPipeline:
         self.part_ws = torch.empty(self.part_ws_bytes // 4, dtype=torch.float32, device=dev) if self.part_ws_bytes else None
         if weights.dtype == torch.uint8:
             self.xq = torch.empty((S, H), dtype=torch.uint8, device=dev)
-            self.xs = torch.empty((S,), dtype=torch.float32, device=dev)
+            self.xs = torch.empty((max(S, 1),), dtype=torch.float32, device=dev)
             self.hq = torch.empty((S, F), dtype=torch.uint8, device=dev)          # hidden activation: e4m3 codes
             self.hsc = torch.empty((S, F // 32), dtype=torch.uint8, device=dev)   # and one scale byte per row and 32 columns
         # source side again: what comes back ([W,M,H], same slots as `send`) and the combined output

@@ -117,6 +117,36 @@ def test_step_as_one_call_equals_its_stages(name, mode):
         assert torch.equal(one[n], stages[n]), f"{n} differs"
 
 
+@pytest.mark.parametrize("name,mode", [("plumbing", {}), ("small", dict(fused=False)), ("small", {}), ("small", dict(gated=True)),
+                                       ("small", dict(padding_free=True)), ("zipf_k4", {}), ("zipf_k4", dict(fused=False)), ("zipf_k4", dict(fp8_dispatch=False)),
+                                       ("zipf_k4", dict(gated=True)), ("zipf_k4", dict(padding_free=True))])
+def test_step_of_a_rank_that_receives_nothing(name, mode):
+    """No token of any rank chose an expert of this one: what it sends back is all padding, and its source side goes on as ever."""
+    from dataclasses import replace
+    from iris_testing_amd.pipeline import DispatchPipeline
+    cfg = replace(CONFIGS[name], tokens=40)
+    world = harness.build_world(cfg, DEV)
+    ew, _, _ = harness.expert_weights(cfg, 0, DEV)
+    world.recv_counts, world.S = torch.zeros_like(world.recv_counts), 0
+    if mode.get("gated"):
+        mode = dict(mode, recv_gate=harness.recv_gates(world))
+    if mode.get("padding_free"):
+        mode = dict(mode, recv_flat=harness.recv_flat(world))
+    pipe = DispatchPipeline(world, ew, **mode)
+    pipe.returned.copy_(torch.randn(pipe.returned.shape, device=DEV).to(pipe.returned.dtype))
+    outs = []
+    for events in (None, []):
+        pipe.expert_cnt.fill_(7)
+        if pipe.ret is not None:
+            pipe.ret.fill_(3)
+        pipe.out.zero_()
+        pipe.step(events)
+        torch.cuda.synchronize()
+        outs.append(pipe.out.clone())
+        assert not bool(pipe.expert_cnt.any()) and (pipe.ret is None or not bool(pipe.ret.any()))
+    assert torch.equal(*outs) and bool(outs[0].any())
+
+
 @pytest.mark.parametrize("T,H,E,k,W,F,act,cut", [(37, 128, 8, 2, 4, 260, "gelu", 0), (5, 36, 3, 1, 1, 100, "silu", 0), (300, 256, 130, 2, 65, 512, "silu", 3),
                                                  (2000, 132, 24, 4, 8, 200, "gelu", 40), (700, 512, 12, 2, 2, 1024, "silu", 1), (4, 64, 16, 1, 4, 64, "gelu", 0), (40, 252, 8, 2, 2, 130, "swiglu", -70)])
 def test_fp32_rows_come_from_and_go_to_their_slots_in_the_gemms(T, H, E, k, W, F, act, cut):
