@@ -546,6 +546,8 @@ def main():
         "ms_per_step_stream": round(stream_ms_per_step, 4),
         "ms_per_step_graph": None if ms_graph is None else round(ms_graph, 4),
         "roofline": roofline,
+        # (a step is one call: it prepares the receive side in the ranking launch, and its fp32 GEMMs move the rows themselves)
+        "stages_are": "launches of their own, timed one by one; a step merges some of them, so they add up to more than ms_per_step",
         "stages": stages,
     }
 

@@ -1024,13 +1024,15 @@ __global__ void zero_pad_rows_kernel(T* __restrict__ out, int K, int Nreal, int 
 }
 
 // fp32 grouped GEMM (the plumbing workload's experts, and the fp32 gradients to rows): tiles of 32R x 32R rows and columns, four waves
-// of 16R x 16R each, on the fp32 matrix instruction (16x16x4; products and sums of one k after the other, k ascending, the
-// order of a scalar fmaf chain).  Weights in the reference layout [E_l][K][N].
-// Bound at the plumbing sizes (512 rows, K 256 / 512) by the length of its chain: load, LDS, matrix instructions, slab by slab, with few
+// of 16R x 16R each, on the fp32 matrix instruction (16x16x4; products and sums of one k after the other).  Weights in the reference layout [E_l][K][N].
+// A sum is one chain over ascending k, the order of a scalar fmaf chain, with KG = 1; with KG = 2 two such chains, over the even and the odd pieces of
+// 128 of K, added once.  Which of the two a launch takes depends on its rows, groups and columns (f32_plan): the same row may differ
+// by rounding between launches of different sizes.
+// Bound at the plumbing sizes (487 rows, K 256 / 512) by the length of its chain: load, LDS, matrix instructions, slab by slab, with few
 // workgroups in flight; hence the long slabs (R = 1: 128 of K, twice the loads under way) and small tiles (256 workgroups of
-// 32 x 32 where 64 x 64 gives 64).  KG = 2, where there are few tiles: eight waves to a tile, slabs twice as long, every set of four with half of
-// a slab's steps and the second half's sums added at the end: the two GEMMs 22.7 -> 17.1 us (with one set 21.3; on the vector
-// units with 64 x 64 tiles they took 32 and 56 us).
+// 32 x 32 where 64 x 64 gives 64).  KG = 2, where the tiles are one round: eight waves to a tile, slabs twice as long, every set of four with half of
+// a slab's steps and the second half's sums added at the end: the two GEMMs of the plumbing step 8.0 and 12.4 us with one set, 7.4 and 8.7 with two
+// (fastest launches; on the vector units with 64 x 64 tiles they took 32 and 56).
 // R = 2 for launches of many tiles: every operand value out of LDS feeds two matrix instructions.
 // A in LDS as [row][k % 4][k / 4]: the four values a lane needs in four consecutive steps are one 16-byte read; B as
 // [k][column], rows padded so that the four k of a step lie in different banks.

@@ -305,13 +305,15 @@ __global__ __launch_bounds__(NWV * WAVE, (NWV == 4 && TB == 2 ? 2 : 1)) void rou
 // KG = 2: a second set of waves runs the segments 4 to 7 beside the first one's 0 to 3; its chains wait in registers and go through LDS at the
 // end, where the first set adds them in order, so the bits stay (256 tiles: 4096 tokens x 768 33 -> 28 us; 512: 8192 x 768 48 -> 46, half of it from
 // the rows' leaving through LDS in 16-byte pieces; the products run at 0.86 of the fp32 rate, the other 13 us are launch, first loads and stores).
+// The waiting chains fill the 128 registers that four waves to a SIMD leave; one value a lane goes to scratch in front of the slab loop and comes
+// back behind it.
 // Bound by the fp32 rate, which K = 1 MFMAs and vector instructions share (95 us for 4096 x 7168 x 256, measured 143 with the
 // partial sums and the top-k; the 32 x 32 shape reaches 0.95 of the rate from a single chain per wave, 16 x 16 0.82): what counts is how few
 // vector instructions surround the MFMAs.  9218 tokens x 5032, 32 experts 88 -> 60 us and 16384 x 4096, 32 experts 94 -> 55 us
 // (blocks 32 experts wide instead of 64), 2048 x 4096, 256 experts 64 -> 50 us, 9216 x 3072, 256 experts 179 -> 157 us.
 // Slabs of KC h are double-buffered in LDS; the conversion and the writes of the next slab sit piece by piece between this one's
 // MFMAs, whose chain would leave the issue slots empty.
-// NB = 1: one slab in LDS and four workgroups to a compute unit; the others' products cover a workgroup's conversion, writes and barriers.
+// (NB = 2.)  NB = 1: one slab in LDS and four workgroups to a compute unit; the others' products cover a workgroup's conversion, writes and barriers.
 // LDS: tokens as [token][h] (the lane reads eight consecutive h of its token), the router as [h][expert] as it comes.
 template <int SHAPE, int NWE, int KC, int D /* slabs under way in registers */, bool ALL, int NB /* slabs in LDS */, int KG /* sets of waves */>
 __global__ __launch_bounds__(KG * 4 * WAVE, NB == 1 || KG == 2 ? 4 : 2) void route_logits_bf16_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
@@ -348,7 +350,8 @@ __global__ __launch_bounds__(KG * 4 * WAVE, NB == 1 || KG == 2 ? 4 : 2) void rou
         wh[i] = c / (EB / 4);
         wp[i] = w + min(eb0 + c % (EB / 4) * 4, E - 4);
     }
-    static_assert(D == 2 || D == 4, "slab s lies in buffer s % 2 and register set s % D");
+    static_assert((D == 2 || D == 4) && (NB == 1 || NB == 2), "slab s lies in buffer s % NB and register set s % D");
+    static_assert((SHAPE == 16) == (KG == 2), "the two sets' rows leave by their own way, the others' in the 32 x 32 layout");
     rt_u4 xr[D][XPT];
     uint2 wr[D][WPT];
     // (pieces past the end of the rows repeat the last ones; what is past H is not consumed)
@@ -423,7 +426,8 @@ __global__ __launch_bounds__(KG * 4 * WAVE, NB == 1 || KG == 2 ? 4 : 2) void rou
     for (int i = 0; i < WPT; ++i) put_w(0, 0, i);
     fetch(0, D * KC);
     __syncthreads();
-    // slab s (s % D = S) from buffer S % 2; slab s + 1 (register set N) goes to the other one, slab s + 1 + D is requested in its place
+    // slab s (s % D = S) from buffer S % NB.  Slab s + 1 (register set N) goes to the other buffer piece by piece between the products, with NB = 1 to
+    // the same one between two barriers behind them; slab s + 1 + D is requested in its place.
     auto slab = [&](auto idx, int s) {
         constexpr int S = decltype(idx)::value, B = S % NB, N = (S + 1) % D;
         const int n = min(NCH, (H - s * KC) / 8);
@@ -522,7 +526,7 @@ __global__ __launch_bounds__(KG * 4 * WAVE, NB == 1 || KG == 2 ? 4 : 2) void rou
     float* o = ALL ? out : out + (size_t)b8 * T * E;
 #pragma unroll
     for (int v = 0; v < NACC; ++v) {
-        const int t = t0 + wt + (SHAPE == 32 ? 32 * (v / 16) + 8 * (v % 16 / 4) + 4 * (lane / 32) + v % 4 : 16 * (v / 4) + 4 * (lane / 16) + v % 4);
+        const int t = t0 + wt + 32 * (v / 16) + 8 * (v % 16 / 4) + 4 * (lane / 32) + v % 4;
         if (t < T) o[(size_t)t * E + e] = !ALL ? acc[v] : bias ? __fadd_rn(sum[v], be) : sum[v];
     }
 }
@@ -818,8 +822,8 @@ extern "C" int moe_route_topk(const void* x, const void* router, const float* bi
         // it: 16384 tokens, 256 experts 71 -> 63 us (512 h), 108 -> 99 (1024), 180 -> 134 (1536), 215 -> 169 (2048), 541 -> 520
         // (7168); 14336 tokens x 2048 182 -> 167; but 12288 tokens (384 tiles) 156 -> 165, 8192 (256: one to a compute unit) 107 -> 108.
         const bool all32 = E > 64 && tok_blocks * n_e >= 448;
-        // The segments as workgroups: four to a compute unit (of 256; one slab of LDS each) where that takes no more than half the rounds that two (two slabs)
-        // take: 4096 tokens x 7168, 256 experts (1024 workgroups) 154 -> 143 us with the top-k, 8192 x 2048 (2048) 108 -> 102, 12288 x 2048 155 -> 151,
+        // The segments as workgroups: four to a compute unit (of 256; one slab of LDS each) where all fit two to a compute unit anyway (half of the chip stays
+        // idle: single rounds are equal or better so), or where four take no more than half the rounds that two (two slabs) take: 4096 tokens x 7168, 256 experts (1024 workgroups) 154 -> 143 us with the top-k, 8192 x 2048 (2048) 108 -> 102, 12288 x 2048 155 -> 151,
         // 600 x 4096 31.4 -> 30.5; but 9216 x 3072 (2304: three rounds for five) 157 -> 163, 6000 x 4992, 160 experts (1504) 146 -> 161.
         const int wgs = 8 * tok_blocks * n_e, pairs = ceil_div(wgs, 2 * 256);
         const bool four = pairs == 1 || 2 * ceil_div(wgs, 4 * 256) <= pairs;
