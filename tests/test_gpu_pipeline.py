@@ -228,6 +228,82 @@ def test_rows_looped_back_on_one_rank_are_the_sent_ones(tokens, gated):
         assert torch.equal(back[n], apart[n]), f"{n} differs"
 
 
+@pytest.mark.parametrize("mode,shared", [("fp8", "rows counts scale"), ("fp8", "scale"), ("fp8", "counts"), ("fp8 gated", "rows counts scale gate"),
+                                         ("fp8 gated", "gate"), ("gated", "gate"), ("flat", "rows counts"), ("flat", "counts"), ("fp8 flat", "rows counts")])
+def test_one_rank_loops_some_of_its_buffers_back(mode, shared):
+    """As above with fp8 rows and their scales, gates and padding-free payloads, all of them looped back or one alone; what the last step left in
+    the shared buffers is wrong before each step."""
+    from iris_testing_amd.configs import MoEConfig
+    from iris_testing_amd.pipeline import DispatchPipeline
+    fp8, gated, flat = "fp8" in mode, "gated" in mode, "flat" in mode
+    cfg = MoEConfig("case", 5, 300, 256, "bf16", 12, 2, 1, 256, "swiglu" if fp8 else "silu", quant="fp8" if fp8 else "none")
+    world = harness.build_world(cfg, DEV)
+    ew, _, _ = harness.expert_weights(cfg, 0, DEV)
+    kw = dict(gated=True, recv_gate=harness.recv_gates(world)) if gated else dict(padding_free=True, recv_flat=harness.recv_flat(world)) if flat else {}
+    pipe = DispatchPipeline(world, ew, **kw)
+    assert pipe.fp8_dispatch == (fp8 and not flat)
+    names = [n for n in "send_counts pos send payload send_q send_scale send_gate expert_cnt row_map row_gate xs hidden ret ret_flat".split()
+             if isinstance(getattr(pipe, n, None), torch.Tensor)]
+
+    def results():
+        for n in names:
+            getattr(pipe, n).zero_()
+        pipe.step()
+        torch.cuda.synchronize()
+        return {n: getattr(pipe, n).clone() for n in names}
+    apart = results()
+    for what in shared.split():
+        if what == "counts":
+            world.recv_counts = pipe.send_counts
+        elif what == "scale":
+            world.recv_scale = pipe.send_scale
+        elif what == "gate":
+            pipe.recv_gate = pipe.send_gate
+        elif flat:
+            pipe.recv_flat = pipe.payload
+        else:
+            world.recv_q = pipe.send_q
+    back = results()
+    for n in names:
+        assert torch.equal(back[n], apart[n]), f"{n} differs"
+
+
+@pytest.mark.parametrize("over", ["ret over send", "ret over recv", "ret over rows", "ret over counts and rows", "y over recv", "y over rows"])
+def test_fp32_destination_buffers_that_take_each_others_place(over):
+    """Scratch plans that stage by stage are right: a buffer where another lay that is done with by then."""
+    from iris_testing_amd.configs import MoEConfig
+    from iris_testing_amd.pipeline import DispatchPipeline
+    cfg = MoEConfig("case", 7, 300, 256, "f32", 8, 2, 4, 128, "gelu")
+    world = harness.build_world(cfg, DEV)
+    ew, _, _ = harness.expert_weights(cfg, 0, DEV)
+    pipe = DispatchPipeline(world, ew)
+    pipe.step()
+    torch.cuda.synchronize()
+    names = ["hidden", "ret", "out"] + (["y"] if over[0] == "y" else [])
+    want, recv, S = {n: getattr(pipe, n).clone() for n in names}, world.recv.clone(), pipe.S
+    assert pipe.ret.numel() >= 64 + S * cfg.hidden
+    if over == "ret over send":
+        pipe.ret = pipe.send
+    elif over == "ret over recv":
+        pipe.ret = world.recv
+    elif over == "y over recv":
+        pipe.y = world.recv.view(-1)[:S * cfg.hidden].view(S, -1)
+    elif over == "y over rows":
+        pipe.y = pipe.rows
+    else:
+        if "counts" in over:
+            pipe.expert_cnt = pipe.ret.view(-1).view(torch.int32)[:cfg.e_local]
+        pipe.rows = pipe.ret.view(-1)[64:64 + S * cfg.hidden].view(S, -1)
+    for _ in range(3):
+        pipe.ret.fill_(5)
+        pipe.y.fill_(5)
+        world.recv.copy_(recv)
+        pipe.step()
+        torch.cuda.synchronize()
+        for n in names:
+            assert torch.equal(getattr(pipe, n), want[n]), f"{n} differs"
+
+
 def test_entry_point_smoke_runs():
     """The smoke check of the repository's entry module (one small step against the oracle) must keep passing."""
     import importlib
