@@ -199,26 +199,21 @@ enum { EPI_NONE = 0, EPI_GELU = 1, EPI_SILU = 2, EPI_SWIGLU = 3, EPI_GATE = 4 };
 // Written as inline assembly to get the scalar-base + 32-bit-lane-offset form (the builtin expands to a
 // 64-bit per-lane address); M0 holds the LDS byte address of the wave's 1 KB destination.
 // A scalar register that a vector instruction wrote (v_readlane, where the compiler brings a spilled base back) may be a load's base
-// only five wait states later, and the compiler does not count them across the start of such a statement: the base goes
-// through a scalar move first (which needs no wait, and is the wait state that a load needs behind a write of M0).
-__device__ __forceinline__ void gg_dma16(const uint8_t* sbase, uint32_t voff, uint32_t lds_addr) {
-    const uint8_t* b;
-    asm volatile("s_mov_b32 m0, %3\n\ts_mov_b64 %0, %1\n\tglobal_load_lds_dwordx4 %2, %0" : "=&s"(b) : "s"(sbase), "v"(voff), "s"(lds_addr) : "memory");
-}
-
+// only five wait states later, and the compiler does not count them across the start of such a statement.  csrc/build.py goes over the machine
+// code and refuses a library with a load that is too early (there is none within eight).  Moving the base to a scalar register of the statement's
+// own would make that needless, but the loads wait for the move: mixtral's step 8062 -> 8126 us, its training pass 26111 -> 26437.
+// The LDS address is added up in the statement, a constant offset as a literal: with the sums in front of it the compiler keeps one base
+// for every load of a stage and reloads most of them from spills (265 instead of 239 instructions around the 128 MFMAs of two stages).
 __device__ __forceinline__ void gg_dma16(const uint8_t* sbase, uint32_t voff, uint32_t lds_base, uint32_t lds_off) {
-    gg_dma16(sbase, voff, lds_base + lds_off);
+    asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %0"
+                 : : "s"(sbase), "v"(voff), "s"(lds_base), "is"(lds_off) : "memory", "scc");
 }
 
-// The same through a buffer descriptor: bytes at or past its range arrive as zeros.  (The halves of an operand of four registers cannot be
-// named in the statement: the moves go to registers of its own.  The LDS address is added up here, which pays for the second move: the
-// training pass of 32 small experts takes what it took without the moves, with the sum in front of the statement 0.7 % more, with the waits written out 1.2 %.)
+// The same through a buffer descriptor: bytes at or past its range arrive as zeros.
 typedef int gg_i32x4 __attribute__((ext_vector_type(4)));
-typedef int gg_i32x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ void gg_dma16(const gg_i32x4& srd, uint32_t voff, uint32_t lds_base, uint32_t lds_off) {
-    const gg_i32x2 lo = {srd.x, srd.y}, hi = {srd.z, srd.w};
-    asm volatile("s_add_u32 m0, %3, %4\n\ts_mov_b64 s[96:97], %0\n\ts_mov_b64 s[98:99], %1\n\tbuffer_load_dwordx4 %2, s[96:99], 0 offen lds"
-                 : : "s"(lo), "s"(hi), "v"(voff), "s"(lds_base), "s"(lds_off) : "memory", "scc", "s96", "s97", "s98", "s99");
+    asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %0, 0 offen lds"
+                 : : "s"(srd), "v"(voff), "s"(lds_base), "is"(lds_off) : "memory", "scc");
 }
 // Descriptor of `left` bytes at p (none when left <= 0), in scalar registers.
 __device__ __forceinline__ gg_i32x4 gg_range(const uint8_t* p, long long left) {
@@ -257,8 +252,7 @@ __device__ __forceinline__ int gg_lane_now() {
 
 // One dword per lane, HBM -> LDS: lane l's value lands at lds_addr + 4 l.
 __device__ __forceinline__ void gg_dma4(const uint8_t* sbase, uint32_t voff, uint32_t lds_addr) {
-    const uint8_t* b;
-    asm volatile("s_mov_b32 m0, %3\n\ts_mov_b64 %0, %1\n\tglobal_load_lds_dword %2, %0" : "=&s"(b) : "s"(sbase), "v"(voff), "s"(lds_addr) : "memory");
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %1, %0" : : "s"(sbase), "v"(voff), "s"(lds_addr) : "memory");
 }
 
 // a wave-uniform value forced into scalar registers

@@ -384,8 +384,8 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
     // load d (0 .. LPS-1) of one stage: A rounds first, then B rounds
 #define GG_LD(d, ap_, bp_, aoff_, slot)                                                                       \
     do {                                                                                                      \
-        if constexpr ((d) < RA) gg_dma16(ap_, aoff_[(d) < RA ? (d) : 0], la0, ((slot) * ASLOT + (d) * LR * CHUNKS) * 16); \
-        else gg_dma16(BN_RAW && (d) >= RA + RB / 2 ? bp_##2 : bp_, b_off[(d) >= RA ? (d) - RA : 0], lb0, ((slot) * BSLOT + ((d) - RA) * LR * CHUNKS) * 16); \
+        if constexpr ((d) < RA) gg_dma16(ap_, aoff_[(d) < RA ? (d) : 0], la0 + (slot) * ASLOT * 16, (d) * LR * CHUNKS * 16); \
+        else gg_dma16(BN_RAW && (d) >= RA + RB / 2 ? bp_##2 : bp_, b_off[(d) >= RA ? (d) - RA : 0], lb0 + (slot) * BSLOT * 16, ((d) - RA) * LR * CHUNKS * 16); \
     } while (0)
     // loads [first, first + count) of stage `st` (clamped to the last stage: the ring never holds data
     // of another tile, and a repeated load of the last stage lands in a slot nobody reads again)
