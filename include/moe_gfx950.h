@@ -391,9 +391,9 @@ int moe_combine_backward(const void* d_out, const void* ret, int dtype, int W, i
                          const int32_t* pos, const float* gate, const int32_t* dst_sizes, const int32_t* dst_offsets, int T,
                          int k, int E_l, void* d_ret, float* d_gate, moe_stream_t stream);
 
-/* ---- a13: return path and combine (not in the reference; defined by the task statement) -------
+/* ---- a13: return path and combine (not in the reference) -------
  * ret[s, expert_offs_s[e]+j, :] = y[off[e,s]+j, :], zero padding: the [W,M,H] buffer this rank
- * sends back, slot s in the order source s sent its rows. */
+ * sends back, slot s in the order source s sent its rows.  S_rows = 0 (nothing was received; y may be NULL): every slot is padding. */
 int moe_return_pack(const void* y, int dtype, int S_rows, int H, const int32_t* recv_counts, int W, int E_l,
                     int M, void* ret, int32_t* map_ws, moe_stream_t stream);
 
