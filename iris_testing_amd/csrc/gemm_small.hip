@@ -188,10 +188,10 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
     // (bp[stage][matrix of a pair])
     typedef typename std::conditional<BMODE == GG_B_PACKED, const uint8_t*, gg_i32x4>::type bsrc_t;
     auto load = [&](int d, const uint8_t* ap, const bsrc_t (&bp)[2][2], const uint8_t* sp, int slot) {
-        if (d < 2 * RA) gg_dma16(ap + (d & 1) * ROWB, aoff[d >> 1], la0 + slot * 2 * ASZ, (d & 1) * ASZ + (d >> 1) * 64 * ROWB);
+        if (d < 2 * RA) gg_dma16(ap + (d & 1) * ROWB, aoff[d >> 1], la0 + slot * 2 * ASZ + (d & 1) * ASZ + (d >> 1) * 64 * ROWB);
         else if (d < 2 * (RA + RB)) {
             const int e = d - 2 * RA;
-            gg_dma16(bp[e / RB][BN_PAIR ? e % RB : 0], boff[e % RB], lb0 + slot * 2 * BSZ, (e / RB) * BSZ + (e % RB) * 64 * ROWB);
+            gg_dma16(bp[e / RB][BN_PAIR ? e % RB : 0], boff[e % RB], lb0 + slot * 2 * BSZ + (e / RB) * BSZ + (e % RB) * 64 * ROWB);
         } else if constexpr (BSA) gg_dma4(sp, soff, ls0 + slot * 256);
     };
 #define GS_PAIR_PTRS(pr)                                                    \
