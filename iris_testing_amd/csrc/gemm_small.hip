@@ -29,8 +29,8 @@ struct GsShape {
     static constexpr int WM = BM == 32 ? 1 : 2, WN = 4 / WM;  // waves along rows and columns
     static constexpr int WR = BM / WM, WC = GS_BN / WN;       // rows and columns of a wave
     static constexpr int NST = 3;                             // ring slots, a pair of 64-byte stages each (two workgroups fit a compute unit)
-    static constexpr int RA = BM < 64 ? 1 : BM / 64;          // activation loads per wave and stage (1 KB each)
-    static constexpr int RB = GS_BN / 64;
+    static constexpr int RA = BM / 32;                        // activation loads per wave and pair of stages (1 KB each)
+    static constexpr int RB = GS_BN / 64;                     // weight loads per wave and stage
 };
 template <int BM, bool BSA>
 constexpr int gs_lds_bytes() {
@@ -66,7 +66,7 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
     constexpr int MT = FP8 ? 32 : 16, CF = FP8 ? 2 : 1;
     constexpr int TM = S::WR / MT, TN = S::WC / MT;
     constexpr int NST = S::NST, RA = S::RA, RB = S::RB;
-    constexpr int LPS = 2 * (RA + RB) + (BSA ? 1 : 0);
+    constexpr int LPS = RA + 2 * RB + (BSA ? 1 : 0);  // loads per wave and pair
     constexpr int ASZ = BM * ROWB, BSZ = GS_BN * ROWB;  // bytes of a stage (a ring slot holds two)
     constexpr bool QOUT = FP8 && EPI == EPI_SWIGLU;
     static_assert(TM >= 1 && TN >= 1, "wave tile");
@@ -143,7 +143,9 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
     const int nkp = P > 1 ? gg_part_stages(nk, P) : nk;
     const int ks0 = part * nkp, nks = min(nkp, nk - ks0);
 
-    // ---- addresses.  LDS tiles as in the large kernel: 64-byte rows, chunk c of row r at position c ^ gg_swz(r >> 2).
+    // ---- addresses.  LDS tiles: weights as in the large kernel, 64-byte rows, chunk c of row r at position c ^ gg_swz(r >> 2);
+    // activations a pair of stages at a time, 128-byte rows, chunk c of row r at position c ^ gg_swz_wide(r) (in 64-byte pieces, a stage at a
+    // time: 1724 rows x 4096 x 1024 in two groups 24.9 us, now 24.0; 1003 x 4096 x 2048 36 -> 34; 200 x 1024 x 1024 7.2 -> 6.9).
     const int lchunk = (lane & 3) ^ gg_swz(lane >> 4);
     const uint32_t ldk = (uint32_t)(p.K * ES);
     const uint8_t* Ab = (p.a_map ? p.A : p.A + (size_t)row0 * ldk) + (size_t)ks0 * ROWB;
@@ -161,9 +163,8 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
     uint32_t aoff[RA], boff[RB];
 #pragma unroll
     for (int r = 0; r < RA; ++r) {
-        const int wr = BM < 64 ? (wave & 1) : wave;  // (32 rows: two waves move them, the other two repeat that)
-        const int lr = min(r * 64 + wr * WROWS + (lane >> 2), rv - 1);
-        aoff[r] = (uint32_t)(p.a_map ? max(p.a_map[row0 + lr], 0) : lr) * ldk + lchunk * 16;
+        const int ar = (r * 4 + wave) * 8 + (lane >> 3), lr = min(ar, rv - 1);
+        aoff[r] = (uint32_t)(p.a_map ? max(p.a_map[row0 + lr], 0) : lr) * ldk + ((lane & 7) ^ gg_swz_wide(ar)) * 16;
     }
 #pragma unroll
     for (int r = 0; r < RB; ++r) {
@@ -178,7 +179,7 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
     uint8_t* const sA = lds;
     uint8_t* const sB = lds + NST * 2 * ASZ;
     uint32_t* const sS = (uint32_t*)(lds + NST * 2 * (ASZ + BSZ)) + wave * NST * 64;  // (BSA) the wave's scale dwords, one per row
-    const uint32_t la0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr_t)sA) + (BM < 64 ? (wave & 1) : wave) * WROWS * ROWB;
+    const uint32_t la0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr_t)sA) + wave * 1024;
     const uint32_t lb0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr_t)sB) + wave * WROWS * ROWB;
     [[maybe_unused]] const uint32_t ls0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr_t)sS);
     [[maybe_unused]] const uint32_t soff = BSA ? (uint32_t)(row0 + min(wm * S::WR + (lane & (S::WR - 1)), rv - 1)) * (uint32_t)p.bs_pitch : 0u;
@@ -188,9 +189,9 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
     // (bp[stage][matrix of a pair])
     typedef typename std::conditional<BMODE == GG_B_PACKED, const uint8_t*, gg_i32x4>::type bsrc_t;
     auto load = [&](int d, const uint8_t* ap, const bsrc_t (&bp)[2][2], const uint8_t* sp, int slot) {
-        if (d < 2 * RA) gg_dma16(ap + (d & 1) * ROWB, aoff[d >> 1], la0 + slot * 2 * ASZ + (d & 1) * ASZ + (d >> 1) * 64 * ROWB);
-        else if (d < 2 * (RA + RB)) {
-            const int e = d - 2 * RA;
+        if (d < RA) gg_dma16(ap, aoff[d], la0 + slot * 2 * ASZ + d * 4096);
+        else if (d < RA + 2 * RB) {
+            const int e = d - RA;
             gg_dma16(bp[e / RB][BN_PAIR ? e % RB : 0], boff[e % RB], lb0 + slot * 2 * BSZ + (e / RB) * BSZ + (e % RB) * 64 * ROWB);
         } else if constexpr (BSA) gg_dma4(sp, soff, ls0 + slot * 256);
     };
@@ -219,7 +220,8 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
     // and the pair NST behind it is requested into the slot that has just been read out; one barrier per pair (it says that the
     // next pair's loads of every wave have landed and that nobody reads the slot the new loads go to any more).
     const int fpos = (FP8 ? (lane >> 5) : (lane >> 4)) ^ gg_swz(lane >> 2);
-    const uint4* fa = (const uint4*)sA + (wm * S::WR + (lane & (MT - 1))) * CHUNKS;
+    const uint4* fa = (const uint4*)sA + (wm * S::WR + (lane & (MT - 1))) * 2 * CHUNKS;
+    const int fpos_a = (FP8 ? (lane >> 5) : (lane >> 4)) ^ gg_swz_wide(lane);  // (rows of a fragment start at multiples of 16)
     const uint4* fb = (const uint4*)sB + (wn * S::WC + (lane & (MT - 1))) * CHUNKS;
     // (BN_RAW) LDS address of the lane's part of the first of the two fragments of each group of 32 columns (see gg_read_tr)
     constexpr int BTR = BN_PAIR ? 128 : 256;
@@ -240,7 +242,7 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
     auto read = [&](Frag& f, int slot) {
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
-            const uint4* as = fa + (slot * 2 + u) * (ASZ / 16);
+            const uint4* as = fa + slot * (2 * ASZ / 16);
             const uint4* bs = fb + (slot * 2 + u) * (BSZ / 16);
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
@@ -256,7 +258,7 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
-                for (int h = 0; h < CF; ++h) f.a[u][i][h] = as[i * MT * CHUNKS + (fpos ^ (2 * h))];
+                for (int h = 0; h < CF; ++h) f.a[u][i][h] = as[i * MT * 2 * CHUNKS + (fpos_a ^ (CHUNKS * u + 2 * h))];
         }
         if constexpr (BSA) {
             // lane 32 h + r: the scale bytes of row r, block h of either stage (see mma_fp8_k64_bs), in bytes 0 and 2

@@ -230,6 +230,11 @@ __device__ __forceinline__ gg_i32x4 gg_range(const uint8_t* p, long long left) {
 // 32 h .. 32 h + 31: chunk h of rows 0 .. 31) meet 64 different banks each time when the swizzle maps 0, 1, 2, 3 to 0, 3, 2, 1.  With
 // 0, 1, 2, 3 itself lanes 0-3 and 20-23 share their banks: 303 bytes a ns and compute unit instead of 530 (reads alone).
 __device__ __forceinline__ int gg_swz(int r4) { return -r4 & 3; }
+// Tiles of 128-byte rows (a pair of stages, 64 bytes of K each).  A compute unit loads pieces of 64 bytes of rows from its L2 at 66 bytes a ns,
+// pieces of 128 and more at 127 to 135 (loads alone, 256 workgroups of four waves): an activation operand in whole lines costs the load path half.  Chunk c of row r at position c ^ gg_swz_wide(r), c in 0 .. 7.  Two rows span
+// the banks, and the eight even (odd) rows of each such 16 lanes meet eight different positions: rows 0-3 and 12-15 of one chunk have r / 2 % 8 = 0, 1, 6, 7, rows
+// 4-11 of the next chunk 2, 3, 4, 5 with the lowest bit flipped; rows 0-3, 12-15, 20-27 of one chunk (fp8) all eight.
+__device__ __forceinline__ int gg_swz_wide(int r) { return (r >> 1) & 7; }
 
 // Half h of a fragment of a 16 x 16 x 32 MFMA out of an LDS tile whose rows run along k (row pitch PITCH bytes): lanes 16 q ..
 // 16 q + 15 end with k 8 q + 4 h .. + 3 of columns 0 .. 15.  `addr`: the lane's LDS byte address of k = 8 q + (lane % 16) / 4, four
