@@ -7,8 +7,8 @@
 //   * tiles are 256 (or 128) x 256, four wave64s each owning a 128 (64) x 128 block of 16x16x32 (bf16) or
 //     32x32x64 (fp8) MFMAs with the accumulators in the accumulation registers;
 //   * operands go HBM -> LDS directly (global_load_lds, 16 bytes per lane) through a ring of four
-//     64-byte K stages; the loads of a stage are spread evenly over one MFMA block and issued more than two
-//     blocks ahead; an XOR swizzle of the 16-byte chunks keeps MFMA fragment reads bank-conflict free;
+//     64-byte K stages, activations two stages (a cache line of every row) at a time; the loads are spread over the MFMA
+//     blocks, one to two blocks ahead; an XOR swizzle of the 16-byte chunks keeps MFMA fragment reads bank-conflict free;
 //   * one MFMA block per stage: fragment reads and loads are interleaved one by one between its MFMAs;
 //   * weights are re-tiled once into a K-contiguous layout (gate/up interleaved for SwiGLU) so both
 //     MFMA operands are read as 128-bit fragments;
@@ -175,10 +175,10 @@ __device__ __forceinline__ auto gg_stage_src(const uint8_t* base, size_t off, lo
 // NWM x 2 wave64s per workgroup; every wave owns a (BM/NWM) x 128 block of the tile.
 //
 // K moves through LDS in a ring of NRING stages of ROWB bytes per tile row.  A stage is one MFMA block
-// (one 16x16x32 bf16 or 32x32x64 fp8 MFMA per pair of fragments).  The loads of stage s+4 go into the slot of
-// stage s during block s -- every wave took the fragments of stage s into registers one block earlier -- spread
-// over the block, so the load pipe sees a steady stream instead of a burst and every load has more than two
-// blocks of MFMA work to land.
+// (one 16x16x32 bf16 or 32x32x64 fp8 MFMA per pair of fragments).  Every wave takes the fragments of stage s + 1 into registers during
+// block s.  Activations come in pairs of stages (2 p, 2 p + 1): the pair's slots are free after block 2 p, and block 2 p + 1 requests pair p + 2 into
+// them, which block 2 p + 3 reads.  Weights come by stages: block 2 p requests stages 2 p + 3 and 2 p + 4.  The loads of a block stand one by one
+// between its MFMAs, so the load pipe sees a steady stream.  (DW: block s requests stage s + 4 of both.)
 // BSA: the activation operand carries block scales (fp8 down projection: GemmParams::a_bscale), applied by the MFMAs.
 // TRACE: the same kernel with time stamps (GemmParams::trace); product launches never use it.
 template <int BM, int NWM, int EPI, bool FP8, int BMODE = GG_B_PACKED, bool BSA = false, bool TRACE = false>
@@ -215,6 +215,13 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
     constexpr int LR = NW * WROWS;                     // rows fetched per load round (16 per wave)
     constexpr int RA = BM / LR, RB = BN / LR;          // load rounds per stage
     constexpr int LPS = RA + RB;                       // HBM->LDS loads per lane per stage
+    // Activations come a pair of stages at a time, 128 bytes of their rows (whole cache lines) to a load: the load path takes pieces of 64
+    // bytes at half the rate (see gg_swz_wide).  With a stage at a time: 33618 rows in 32 groups x 7168 x (2 x 2048) 1650 us, now 1563; x 2048 x 7168 884 -> 851;
+    // 32972 x 4096 x (2 x 14336) 5519 -> 5300, x 14336 x 4096 2660 -> 2590; fp8 MLP of 81920 x 2048 x 1408 in 15 groups 858 -> 824 (same box each).
+    // (DW: a stage's rows are 512 bytes as it is)
+    constexpr bool WIDE = !DW;
+    constexpr int LA = WIDE ? 2 * RA : RA;             // loads of A per lane: per pair (WIDE) or stage
+    constexpr int LE = WIDE ? 2 * RB : LPS, LO = WIDE ? LA : LPS;  // loads behind the MFMAs of a block in an even, odd slot
     // Where the other instructions of a block sit.  bf16: a 16x16x32 MFMA covers only 16 cycles of other issue,
     // so no MFMA gets more than one: the fragment reads go behind every RSTEP-th MFMA of the first half of the
     // block (they must have landed when the block ends in the hand-over), the loads are spread evenly over the
@@ -224,10 +231,12 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
     constexpr int RPM = NRD > NT / 2 ? 2 : 1;                 // reads behind one MFMA
     constexpr int RFIRST = 0;                                 // first MFMA with a read behind it
     constexpr int RSTEP = (NT / 2) * RPM / NRD > 0 ? (NT / 2) * RPM / NRD : 1;  // MFMAs from one read group to the next
-    constexpr int LFIRST = NT > LPS ? 1 : 0;                  // first MFMA with a load behind it
-    constexpr int LSTEP = (NT - LFIRST) / LPS;                // MFMAs from one load to the next
+    constexpr int LFIRST = NT > LE && NT > LO ? 1 : 0;        // first MFMA with a load behind it
+    // MFMAs from one load to the next.  WIDE: the pair of A is needed when the next block ends, so its loads take the first half of theirs; those of B,
+    // the first of which are as urgent, three quarters (mixtral's gate / up GEMM 5238 -> 5150 us against loads over whole blocks, the others 0.3 %; all within half: 5192)
+    constexpr int LSE = WIDE ? ((NT - LFIRST) / LE * 3 + 3) / 4 : (NT - LFIRST) / LE, LSO = WIDE ? ((NT - LFIRST) / LO + 1) / 2 : (NT - LFIRST) / LO;
     constexpr int ASLOT = BM * CHUNKS, BSLOT = BN * CHUNKS;  // uint4 per ring slot
-    static_assert(TM * MT * NWM == BM && BM % LR == 0 && BN % LR == 0 && NT <= 64 && LSTEP >= 1 && LFIRST + LSTEP * (LPS - 1) < NT && RFIRST + RSTEP * ((NRD - 1) / RPM) < NT, "tile shape");
+    static_assert(TM * MT * NWM == BM && BM % LR == 0 && BN % LR == 0 && NT <= 64 && LSE >= 1 && LFIRST + LSE * (LE - 1) < NT && LSO >= 1 && LFIRST + LSO * (LO - 1) < NT && RFIRST + RSTEP * ((NRD - 1) / RPM) < NT, "tile shape");
     static_assert(CHUNKS == 4 && NRING == 4, "the stage schedule below is written for 64-byte stages in four slots");
 
     __shared__ __align__(1024) uint4 sA[NRING * ASLOT];
@@ -310,7 +319,8 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
     // bytes 32-63 -- the two blocks of 32 k that the scaled form of the instruction scales separately
     constexpr int FSTEP = FP8 ? 2 : 1;  // distance of a lane's second chunk
     const int fpos = (FP8 ? (lane >> 5) : (lane >> 4)) ^ fswz;
-    const uint4* fa = sA + (wm * (BM / NWM) + (lane & (MT - 1))) * CHUNKS;
+    const uint4* fa = sA + (wm * (BM / NWM) + (lane & (MT - 1))) * (WIDE ? 2 * CHUNKS : CHUNKS);
+    [[maybe_unused]] const int fpos_a = (FP8 ? (lane >> 5) : (lane >> 4)) ^ gg_swz_wide(lane);
     const uint4* fb = sB + (wn * (BN / 2) + (lane & (MT - 1))) * CHUNKS;
     const uint32_t la0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr_t)(sA + wave * WROWS * CHUNKS));
     const uint32_t lb0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr_t)(sB + wave * WROWS * CHUNKS));
@@ -362,7 +372,7 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
                                : (size_t)(t).g * p.Npad * p.K * ES + (size_t)(t).nt * BN * ROWB + (size_t)(t).ks0 * b_slab; \
     const uint8_t* Bb_ = p.B + bo0_;                                                                          \
     if constexpr (BT || BN_RAW) dw_left_b = (long long)p.E_l * b_group - (long long)bo0_;                      \
-    uint32_t aoff_[RA];                                                                                     \
+    uint32_t aoff_[LA];                                                                                     \
     const int ln_ = gg_lane_now();  /* lrow and lchunk again, derived per tile */                              \
     if constexpr (DW) {                                                                                      \
         const long long rows_ = g_row_start[(t).g + 1] - (t).ks0;                                            \
@@ -372,53 +382,54 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
             aoff_[r] = (uint32_t)(2 * (r * NW + wave_s) + (ln_ >> 5)) * ldk +                                   \
                        (uint32_t)((ln_ & 31) ^ (2 * (((2 * wave_s + (ln_ >> 5)) & 3) + 4 * (r & 1)))) * 16u;      \
     } else {                                                                                                 \
-        const int lrow_ = wave_s * WROWS + (ln_ >> 2);                                                         \
-        const uint32_t lcb_ = (uint32_t)(((ln_ & 3) ^ gg_swz(ln_ >> 4)) * 16);                                  \
-        _Pragma("unroll") for (int r = 0; r < RA; ++r) {                                                      \
-            const int lr_ = max(min(r * LR + lrow_, (t).rv - 1), 0);  /* tile row this lane fetches, clamped */ \
+        const int lrow_ = wave_s * 8 + (ln_ >> 3);                                                             \
+        const uint32_t lcb_ = (uint32_t)(((ln_ & 7) ^ gg_swz_wide(lrow_)) * 16);                                \
+        _Pragma("unroll") for (int r = 0; r < LA; ++r) {                                                      \
+            const int lr_ = max(min(r * NW * 8 + lrow_, (t).rv - 1), 0);  /* tile row this lane fetches, clamped */ \
             aoff_[r] = (uint32_t)(p.a_map ? max(MAPROW_(t, lr_), 0) : lr_) * ldk + lcb_;                      \
         }                                                                                                     \
     }
     [[maybe_unused]] const ptrdiff_t b2_delta = p.B2 - p.B;
     [[maybe_unused]] long long dw_left_a = 0, dw_left_b = 0;  // (DW) bytes of the operands from the tile's corner to the end of the group
-    // load d (0 .. LPS-1) of one stage: A rounds first, then B rounds
-#define GG_LD(d, ap_, bp_, aoff_, slot)                                                                       \
-    do {                                                                                                      \
-        if constexpr ((d) < RA) gg_dma16(ap_, aoff_[(d) < RA ? (d) : 0], la0 + (slot) * ASLOT * 16, (d) * LR * CHUNKS * 16); \
-        else gg_dma16(BN_RAW && (d) >= RA + RB / 2 ? bp_##2 : bp_, b_off[(d) >= RA ? (d) - RA : 0], lb0 + (slot) * BSLOT * 16, ((d) - RA) * LR * CHUNKS * 16); \
-    } while (0)
-    // loads [first, first + count) of stage `st` (clamped to the last stage: the ring never holds data
-    // of another tile, and a repeated load of the last stage lands in a slot nobody reads again)
-#define GG_STAGE_PTRS(Ab_, Bb_, st, ap_, bp_, nks_)                                            \
-    const int st_ = min((st), (nks_) - 1);                                                     \
-    const auto ap_ = gg_stage_src<DW>(Ab_, (size_t)st_ * (DW ? (size_t)32 * ldk : (size_t)ROWB), dw_left_a);  \
-    const size_t so_ = BT ? (size_t)(p.B2 ? st_ >> 1 : st_) * ROWB : (size_t)st_ * (DW || BN_RAW ? (size_t)32 * ldb : b_slab); \
-    const auto bp_ = gg_stage_src<BMODE != GG_B_PACKED>(BT && p.B2 && (st_ & 1) ? Bb_ + b2_delta : Bb_, so_, dw_left_b);   \
+    // load d of a stage of B (0 .. RB - 1), of a pair of stages or a stage of A (0 .. LA - 1)
+#define GG_LDB(d, bp_, slot) gg_dma16(BN_RAW && (d) >= RB / 2 ? bp_##2 : bp_, b_off[d], lb0 + (slot) * BSLOT * 16, (d) * LR * CHUNKS * 16)
+#define GG_LDA(d, ap_, aoff_, slot) gg_dma16(ap_, aoff_[d], la0 + (slot) * ASLOT * 16, (d) * (WIDE ? NW * 1024 : LR * CHUNKS * 16))
+    // Where stage `st` of B and the stage (WIDE: the pair that starts with it) `st` of A lie, clamped to the tile's last ones: the ring never holds data
+    // of another tile, and a repeated load of the last stage lands in a slot nobody reads again
+#define GG_A_PTR(Ab_, st, ap_, nks_)                                                           \
+    const auto ap_ = gg_stage_src<DW>(Ab_, (size_t)min((st), (nks_) - (WIDE ? 2 : 1)) * (DW ? (size_t)32 * ldk : (size_t)ROWB), dw_left_a);
+#define GG_B_PTRS(Bb_, st, bp_, nks_)                                                          \
+    const int st_##bp_ = min((st), (nks_) - 1);                                                \
+    const size_t so_##bp_ = BT ? (size_t)(p.B2 ? st_##bp_ >> 1 : st_##bp_) * ROWB : (size_t)st_##bp_ * (DW || BN_RAW ? (size_t)32 * ldb : b_slab); \
+    const auto bp_ = gg_stage_src<BMODE != GG_B_PACKED>(BT && p.B2 && (st_##bp_ & 1) ? Bb_ + b2_delta : Bb_, so_##bp_, dw_left_b);   \
     /* (BN_RAW: the second region, in the other matrix or 256 bytes further along the rows) */                  \
-    [[maybe_unused]] const auto bp_##2 = gg_stage_src<BMODE != GG_B_PACKED>(BN_RAW ? Bb_ + (BN_PAIR ? b2_delta : 256) : Bb_, so_, \
+    [[maybe_unused]] const auto bp_##2 = gg_stage_src<BMODE != GG_B_PACKED>(BN_RAW ? Bb_ + (BN_PAIR ? b2_delta : 256) : Bb_, so_##bp_, \
                                                                             dw_left_b - (BN_RAW && !BN_PAIR ? 256 : 0));
-#define GG_ISSUE_RANGE(Ab_, Bb_, aoff_, st, slot, first, count, nks_)                          \
+#define GG_ISSUE_A(Ab_, aoff_, st, slot, nks_)                                                 \
     do {                                                                                       \
-        GG_STAGE_PTRS(Ab_, Bb_, st, ap_i, bp_i, nks_)                                          \
-        if constexpr ((first) + 0 < (first) + (count)) GG_LD((first) + 0 < LPS ? (first) + 0 : 0, ap_i, bp_i, aoff_, slot); \
-        if constexpr ((first) + 1 < (first) + (count)) GG_LD((first) + 1 < LPS ? (first) + 1 : 0, ap_i, bp_i, aoff_, slot); \
-        if constexpr ((first) + 2 < (first) + (count)) GG_LD((first) + 2 < LPS ? (first) + 2 : 0, ap_i, bp_i, aoff_, slot); \
-        if constexpr ((first) + 3 < (first) + (count)) GG_LD((first) + 3 < LPS ? (first) + 3 : 0, ap_i, bp_i, aoff_, slot); \
-        if constexpr ((first) + 4 < (first) + (count)) GG_LD((first) + 4 < LPS ? (first) + 4 : 0, ap_i, bp_i, aoff_, slot); \
-        if constexpr ((first) + 5 < (first) + (count)) GG_LD((first) + 5 < LPS ? (first) + 5 : 0, ap_i, bp_i, aoff_, slot); \
-        if constexpr ((first) + 6 < (first) + (count)) GG_LD((first) + 6 < LPS ? (first) + 6 : 0, ap_i, bp_i, aoff_, slot); \
-        if constexpr ((first) + 7 < (first) + (count)) GG_LD((first) + 7 < LPS ? (first) + 7 : 0, ap_i, bp_i, aoff_, slot); \
-        static_assert((count) <= 8, "GG_ISSUE_RANGE is unrolled for eight loads");             \
+        GG_A_PTR(Ab_, st, ap_i, nks_)                                                          \
+        _Pragma("unroll") for (int d_ = 0; d_ < LA; ++d_) GG_LDA(d_, ap_i, aoff_, slot);        \
     } while (0)
-    // what a tile has in flight before its first MFMA: its first four stages, one per ring slot
+#define GG_ISSUE_B(Bb_, st, slot, nks_)                                                        \
+    do {                                                                                       \
+        GG_B_PTRS(Bb_, st, bp_i, nks_)                                                         \
+        _Pragma("unroll") for (int d_ = 0; d_ < RB; ++d_) GG_LDB(d_, bp_i, slot);               \
+    } while (0)
+    // what a tile has in flight before its first MFMA: its first four stages, one per ring slot (WIDE: the first block requests the fourth stage of B)
 #define GG_PROLOGUE(Ab_, Bb_, aoff_, nks_)                    \
     do {                                                      \
         GG_SC_DMA(0, nks_, 0);                                \
-        GG_ISSUE_RANGE(Ab_, Bb_, aoff_, 0, 0, 0, LPS, nks_);  \
-        GG_ISSUE_RANGE(Ab_, Bb_, aoff_, 1, 1, 0, LPS, nks_);  \
+        GG_ISSUE_A(Ab_, aoff_, 0, 0, nks_);                   \
+        GG_ISSUE_B(Bb_, 0, 0, nks_);                          \
+        if constexpr (!WIDE) GG_ISSUE_A(Ab_, aoff_, 1, 1, nks_); \
+        GG_ISSUE_B(Bb_, 1, 1, nks_);                          \
         GG_SC_DMA(2, nks_, 2);                                \
-        GG_ISSUE_RANGE(Ab_, Bb_, aoff_, 2, 2, 0, LPS, nks_);  \
-        GG_ISSUE_RANGE(Ab_, Bb_, aoff_, 3, 3, 0, LPS, nks_);  \
+        GG_ISSUE_A(Ab_, aoff_, 2, 2, nks_);                   \
+        GG_ISSUE_B(Bb_, 2, 2, nks_);                          \
+        if constexpr (!WIDE) {                                \
+            GG_ISSUE_A(Ab_, aoff_, 3, 3, nks_);               \
+            GG_ISSUE_B(Bb_, 3, 3, nks_);                      \
+        }                                                     \
     } while (0)
 
     // BSA: the block-scale bytes travel with the stages.  One dword per tile row holds the four scale bytes of a PAIR of
@@ -458,14 +469,14 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
     gg_fill_table<BM, DW>(s_tiles, g_tile_start, g_row_start, p.E_l, Nt, p.S_rows, n_tiles, my, (int)gridDim.x, 0, p.dw_rows);
     __syncthreads();
     GgTile cur = gg_walk<BM, DW>(s_tiles, g_tile_start, g_row_start, p.E_l, Nt, p.S_rows, n_tiles, nk, my, (int)gridDim.x, round, round0, p.dw_rows);
-    uint32_t a_off[RA];
+    uint32_t a_off[LA];
     const uint8_t *Ab = p.A, *Bb = p.B;
     if (cur.rv > 0) {
         GG_TILE_PTRS(cur, Ab0, Bb0, a_off0, GG_MAPROW_GLOBAL);
         Ab = Ab0;
         Bb = Bb0;
 #pragma unroll
-        for (int r = 0; r < RA; ++r) a_off[r] = a_off0[r];
+        for (int r = 0; r < LA; ++r) a_off[r] = a_off0[r];
         sc_row0 = cur.row0; sc_rv = cur.rv; sc_ks0 = cur.ks0;
         GG_PROLOGUE(Ab, Bb, a_off, (VARK ? cur.nks : nk));
     }
@@ -495,10 +506,9 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
 
         // ---- One MFMA block per 64-byte stage.  Block s multiplies the fragments of stage s, reads those of
         // stage s+1 (all issued in the first half of the block, so they have landed when the block ends) and
-        // refills slot s % 4, drained one block earlier, with stage s+4, its loads spread between the MFMAs
-        // (a steady stream instead of a burst, each with three blocks of MFMA work to land); the hand-over at
-        // its end waits for the wave's own loads of stage s+2 -- everything issued after them, stages s+3 and
-        // s+4, may stay in flight -- and meets the other waves.  Loads past the end of the tile are clamped
+        // requests what its predecessors have drained the slots for (above); the hand-over at its end waits for the
+        // wave's own loads of stage s+2 -- what was issued after them may stay in flight: behind a block in an even slot its own loads of B, behind one in an
+        // odd slot its own of A and the second half of the B loads before -- and meets the other waves.  Loads past the end of the tile are clamped
         // to its last stage (straight-line code, constant wait counts); in the last block the "next
         // fragments" are whatever the next slot holds and are never used.  Every instruction is pinned by
         // scheduling fences: each read and each load is issued in the shadow of an MFMA.
@@ -512,7 +522,7 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
             uint4& f_ = ro_ < TM ? NA_[ro_ < TM ? ro_ : 0] : NB_[ro_ < TM ? 0 : ro_ - TM];               \
             if constexpr (rh_ == 0) { f_.x = v_.x; f_.y = v_.y; } else { f_.z = v_.x; f_.w = v_.y; }      \
         }                                                                                                \
-        else if constexpr (ro_ < TM) NA_[ro_ * CF + rh_] = nfa_[ro_ * MT * CHUNKS + (fpos ^ (rh_ * FSTEP))];  \
+        else if constexpr (ro_ < TM) NA_[ro_ * CF + rh_] = nfa_[ro_ * MT * 2 * CHUNKS + (fpos_a ^ (nodd_ * CHUNKS + rh_ * FSTEP))];  \
         else NB_[(ro_ - TM) * CF + rh_] = nfb_[(ro_ - TM) * MT * CHUNKS + (fpos ^ (rh_ * FSTEP))];       \
     } while (0)
 #define GG_ML(I, FA_, FB_, NA_, NB_, slot, Z_, EVEN_, SET_)                                                \
@@ -524,8 +534,16 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
             else if constexpr (FP8) mma_fp8_k64<Z_>(acc[pa_][pb_], FB_[2 * pb_], FB_[2 * pb_ + 1], FA_[2 * pa_], FA_[2 * pa_ + 1]); \
             else mma_bf16_k32<Z_>(acc[pa_][pb_], FB_[pb_], FA_[pa_]);                                    \
             __builtin_amdgcn_sched_barrier(0);                                                           \
-            constexpr int ld_ = (I) >= LFIRST && ((I) - LFIRST) % LSTEP == 0 ? ((I) - LFIRST) / LSTEP : LPS;  /* load behind this MFMA */ \
-            if constexpr (ld_ < LPS) GG_LD((ld_ < LPS ? ld_ : 0), ap_, bp_, a_off, slot);                \
+            constexpr int ls_ = (EVEN_) ? LSE : LSO, ln_ = (EVEN_) ? LE : LO;                            \
+            constexpr int ld_ = (I) >= LFIRST && ((I) - LFIRST) % ls_ == 0 ? ((I) - LFIRST) / ls_ : ln_;  /* load behind this MFMA */ \
+            if constexpr (ld_ < ln_) {                                                                   \
+                if constexpr (!WIDE) {                                                                   \
+                    if constexpr (ld_ < RA) GG_LDA((ld_ < RA ? ld_ : 0), ap_, a_off, slot);              \
+                    else GG_LDB((ld_ >= RA ? ld_ - RA : 0), bp_, slot);                                  \
+                } else if constexpr (!(EVEN_)) GG_LDA((ld_ < LA ? ld_ : 0), ap_, a_off, ((slot) + 3) & 3);  \
+                else if constexpr (ld_ < RB) GG_LDB((ld_ < RB ? ld_ : 0), bq_, ((slot) + 3) & 3);          \
+                else GG_LDB((ld_ >= RB && ld_ < 2 * RB ? ld_ - RB : 0), bp_, slot);                       \
+            }                                                                                            \
             constexpr int r0_ = (I) >= RFIRST && ((I) - RFIRST) % RSTEP == 0 ? (((I) - RFIRST) / RSTEP) * RPM : NRD; /* first read */ \
             if constexpr (r0_ < NRD) GG_RD((r0_ < NRD ? r0_ : 0), NA_, NB_);                             \
             if constexpr (RPM > 1 && r0_ + 1 < NRD) GG_RD((r0_ + 1 < NRD ? r0_ + 1 : 0), NA_, NB_);      \
@@ -540,8 +558,11 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
     // SET_: which copy of the block scales (BSA) the stage's pair uses: slot / 2, as a literal (0 where the slot is a run-time value: no BSA there)
 #define GG_STAGE(FA_, FB_, NA_, NB_, SL, EVEN_, s, last, Z_, SET_)                                                \
     do {                                                                                                 \
+        /* WIDE: a block in an even slot requests B's stages s + 3 (into the slot whose fragments its predecessor read last) and s + 4, \
+           one in an odd slot A's pair of stages s + 3 and s + 4 */                                       \
+        GG_B_PTRS(Bb, (s) + 3 - kbase, bq_, nks_ld)                                                       \
         if constexpr (EVEN_) { /* (a block in an even slot) */                                           \
-            /* from block nks - 4 on the loads fetch the next tile, if it is at hand; not in a tile's first block: the  \
+            /* from block nks - 4 on the loads fetch the next tile (but for the last stage of B), if it is at hand; not in a tile's first block: the  \
                row map that the tile's top requested must have landed and been handed over (one block end at least) */ \
             if ((s) == nks - 4 && (s) > 0) {                                                             \
                 const GgTile pk_ = gg_peek<DW>(s_tiles, g_row_start, nk, my, (int)gridDim.x, round, round0); \
@@ -549,19 +570,20 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
                     GG_TILE_PTRS(pk_, Ab_s, Bb_s, a_off_s, GG_MAPROW_LDS);                               \
                     Ab = Ab_s;                                                                           \
                     Bb = Bb_s;                                                                           \
-                    _Pragma("unroll") for (int r = 0; r < RA; ++r) a_off[r] = a_off_s[r];                \
+                    _Pragma("unroll") for (int r = 0; r < LA; ++r) a_off[r] = a_off_s[r];                \
                     kbase = nks;                                                                         \
                     nks_ld = VARK ? pk_.nks : nk;                                                        \
                     seam = true;                                                                         \
                     sc_row0 = pk_.row0; sc_rv = pk_.rv; sc_ks0 = pk_.ks0;                                \
                 }                                                                                        \
             }                                                                                            \
-            /* (the scale dwords of the pair whose even stage this block requests) */                   \
-            GG_SC_DMA((s) + 4 - kbase, nks_ld, SET_ * 2);                                                \
         }                                                                                                \
-        GG_STAGE_PTRS(Ab, Bb, (s) + 4 - kbase, ap_, bp_, nks_ld)                                         \
+        if constexpr (!(EVEN_)) GG_SC_DMA((s) + 3 - kbase, nks_ld, SET_ * 2);  /* (the pair's scale dwords) */ \
+        GG_A_PTR(Ab, (s) + (WIDE ? 3 : 4) - kbase, ap_, nks_ld)                                          \
+        GG_B_PTRS(Bb, (s) + 4 - kbase, bp_, nks_ld)                                                      \
+        [[maybe_unused]] constexpr int nodd_ = (EVEN_) ? 1 : 0;  /* parity of the stage whose fragments are read */ \
         [[maybe_unused]] const int nsl_ = ((SL) + 1) & 3;                                                \
-        const uint4* nfa_ = fa + (((SL) + 1) & 3) * ASLOT;                                               \
+        const uint4* nfa_ = fa + (WIDE ? (((SL) + 1) & 3) >> 1 << 1 : (((SL) + 1) & 3)) * ASLOT;          \
         const uint4* nfb_ = fb + (((SL) + 1) & 3) * BSLOT;                                               \
         /* (written-out MFMAs: two wait states between the vector instructions above and an MFMA that reads their results) */ \
         if constexpr (BSA && NWM == 4) asm volatile("s_nop 1");                                          \
@@ -573,7 +595,7 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
         /* an odd block ends a pair: the next pair's scale dwords, from the other copy, behind its last MFMA */ \
         if constexpr (!(EVEN_)) GG_SC_READ(1 - SET_);                                                    \
         if (!(last) || seam) { /* (the last block hands over too when the next tile's stages are behind it) */ \
-            gg_wait<2 * LPS, 0>();                                                                       \
+            gg_wait<WIDE ? ((EVEN_) ? 2 * RB : RB + LA) : 2 * LPS, 0>();                                 \
             __builtin_amdgcn_s_barrier();                                                                \
         }                                                                                                \
         if constexpr (TRACE) {                                                                           \
@@ -638,7 +660,7 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
                         fA0[i] = make_uint4(lo.x, lo.y, hi.x, hi.y);
                     } else {
 #pragma unroll
-                        for (int h = 0; h < CF; ++h) fA0[i * CF + h] = fa0[i * MT * CHUNKS + (fpos ^ (h * FSTEP))];
+                        for (int h = 0; h < CF; ++h) fA0[i * CF + h] = fa0[i * MT * 2 * CHUNKS + (fpos_a ^ (h * FSTEP))];
                     }
                 }
 #pragma unroll
@@ -714,7 +736,7 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
             Ab = Ab_n;
             Bb = Bb_n;
 #pragma unroll
-            for (int r = 0; r < RA; ++r) a_off[r] = a_off_n[r];
+            for (int r = 0; r < LA; ++r) a_off[r] = a_off_n[r];
             sc_row0 = nxt.row0; sc_rv = nxt.rv; sc_ks0 = nxt.ks0;
             __syncthreads();
             GG_PROLOGUE(Ab, Bb, a_off, (VARK ? nxt.nks : nk));
@@ -931,9 +953,12 @@ __global__ __launch_bounds__(NWM * 2 * WAVE, 1) void grouped_gemm_kernel(const G
 #undef GG_TILE_PTRS
 #undef GG_MAPROW_GLOBAL
 #undef GG_MAPROW_LDS
-#undef GG_LD
-#undef GG_STAGE_PTRS
-#undef GG_ISSUE_RANGE
+#undef GG_LDA
+#undef GG_LDB
+#undef GG_A_PTR
+#undef GG_B_PTRS
+#undef GG_ISSUE_A
+#undef GG_ISSUE_B
 #undef GG_PROLOGUE
 #undef GG_SC_DMA
 #undef GG_SC_READ
