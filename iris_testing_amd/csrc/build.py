@@ -13,7 +13,7 @@ from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB = os.path.join(HERE, "libmoe_gfx950.so")
-SOURCES = ["capi.hip", "route.hip", "dispatch.hip", "grouped_gemm.hip", "gemm_small.hip", "step.hip", "diag.hip"]
+SOURCES = ["capi.hip", "route.hip", "dispatch.hip", "grouped_gemm.hip", "gemm_small.hip", "gemm_duo.hip", "step.hip", "diag.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 LLVM = os.environ.get("ROCM_LLVM", "/opt/rocm/llvm/bin")
 FLAGS = [

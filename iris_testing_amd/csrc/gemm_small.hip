@@ -125,7 +125,7 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
                 int m = in % mt_g;
                 nt = in / mt_g;
                 if constexpr (TAIL) {
-                    gg_patch(in, mt_g, nt_all, m, nt);
+                    gg_patch(in, mt_g, nt_all, tm == 128 ? SUP_DUO : SUP, m, nt);
                     nt = nt * (GG_BN / GS_BN) + tile % (GG_BN / GS_BN);
                 }
                 const int r = m * tm + (TAIL ? tile % subs / (GG_BN / GS_BN) * BM : 0);
@@ -554,43 +554,15 @@ static int gs_dispatch(const GsParams& q, int bm, int epi, void* ws, size_t byte
     return moe_check_launch("grouped_gemm");
 }
 
-// Tile height for a launch (32 or 64 rows), or 0: large tiles.  Both paths' times in us are estimated from what the host knows
-// -- the row total, not its split over the groups (every group adds about half a tile of ragged tail) -- with coefficients
-// fitted to 470 launches drawn over rows 16 .. 16384, 1 .. 32 groups, K and N 512 .. 8192, bf16 and fp8, even and skewed:
-//   large tiles: whole rounds of the persistent grid, each 0.46 us per 64 bytes of K (fp8 a fifth more) and 3.3 us between tiles; a
-//     part-filled last round 0.57 us (256 rows) or 0.33 us (128 rows), or what small tiles take for it where they get it (gg_tail);
-//     6 us for the launch;
-//   small tiles: 0.24 / 0.30 us per 128 bytes of K while every workgroup has a compute unit to itself, then in proportion to
-//     their number (times 1.2, fp8 1.4: the load path is shared); 5 us for the hand-over of a split tile, 7 us for the launch.  Tiles are
-//     split only as far as the launch has a workspace for the parts.
-// Over those launches the choice made from these estimates is within 0.5 % (geometric mean) of the better of the two, 1.19 times
-// faster than large tiles alone and in one launch of 470 more than 6 % slower than them: 27.5 -> 9.0 us at 512 rows x 1024 x 1024
-// (2 groups, bf16), 31 -> 21 us at 512 x 2048 x 4096, 49 -> 20 us for an fp8 MLP of 300 rows; the line lies at about one round of
-// large tiles.
-int gs_choose_bm(int S_rows, int E_l, int K, int ncols, bool fp8, int cus, const void* part_ws, size_t part_ws_bytes) {
-    const double E = std::min(E_l, S_rows), nk = (double)K * (fp8 ? 1 : 2) / ROWB, share = fp8 ? 1.4 : 1.225;
-    const int nt = (ncols + GG_BN - 1) / GG_BN, nts = (ncols + GS_BN - 1) / GS_BN;
-    const double t256 = (S_rows / 256.0 + 0.5 * E) * nt, t128 = (S_rows / 128.0 + 0.5 * E) * nt;
-    const bool small_m = 0.62 * ceil(t128 / cus) < ceil(t256 / cus);
-    const double tiles = small_m ? t128 : t256, rate = fp8 ? 1.2 : 1.0;
-    const double full = floor(tiles / cus), rem = tiles - full * cus;
-    const GgTail tail = gg_tail((int)nk, small_m ? 128 : 256, fp8, cus);
-    double best = 6 + full * (nk * 0.46 * rate + 3.3), last = nk * (small_m ? 0.33 : 0.57) * rate + 5.1;
-    if (E > 1 && tail.worth) {
-        best += 9.2;
-        if (rem <= tail.most) last = std::min(last, 8 + 0.15 * nk * share * std::max(1.0, rem * (small_m ? 4 : 8) / cus));
-    }
-    if (rem > 0.5) best += last;
-    int bm_best = 0;
-    for (int bm : {32, 64}) {
-        const double units = (S_rows / (double)bm + 0.5 * E) * nts;
-        const int room = std::min(gs_slots(bm, cus), gs_max_units(bm, part_ws, part_ws_bytes));
-        const double P = units < room ? std::max(1.0, std::min(std::min(floor(room / units), floor(nk / GS_MIN_PART_STAGES)), (double)GG_MAX_PARTS)) : 1.0;
-        const double x = units * P / cus;
-        const double t = 7.4 + (P > 1 ? 5 : 0) + nk / 2 / P * (bm == 32 ? 0.24 : 0.30) * std::max(1.0, x * share) + 1.5 * std::max(1.0, x / 2);
-        if (t < best) { best = t; bm_best = bm; }
-    }
-    return bm_best;
+// What a launch on tiles of bm rows is taken to cost, in us, for gg_choose (grouped_gemm.hip), which says where the coefficients come from: 0.27 / 0.30 us per
+// 128 bytes of K while every workgroup has a compute unit to itself, then in proportion to their number (times 1.22 to 1.37: the load path is
+// shared), and the hand-over of a split tile.  `tiles`: about as many as there will be.
+double gs_estimate(int bm, double tiles, int nk, bool fp8, int cus, const void* part_ws, size_t part_ws_bytes) {
+    const int room = std::min(gs_slots(bm, cus), gs_max_units(bm, part_ws, part_ws_bytes));
+    const double P = tiles < room ? std::max(1.0, std::min(std::min(floor(room / tiles), floor((double)nk / GS_MIN_PART_STAGES)), (double)GG_MAX_PARTS)) : 1.0;
+    const double x = tiles * P / cus;
+    if (bm == 32) return nk / 2 / P * 0.27 * std::max(1.0, x * (fp8 ? 1.37 : 1.24)) + 0.5 * std::max(1.0, x / 2) + (P > 1 ? 4 : 0);
+    return nk / 2 / P * 0.30 * std::max(1.0, x * (fp8 ? 1.30 : 1.22)) + 1.3 * std::max(1.0, x / 2) + (P > 1 ? 6.5 : 0);
 }
 
 size_t gs_workspace_bytes(int cus) { return GS_CTR_BYTES + std::min<size_t>((size_t)cus * 64 * GS_BN * 4, GS_PART_BYTES); }
@@ -607,7 +579,7 @@ int launch_gemm_tail(const GemmParams& p, bool fp8, int bm_big, int epi, void* w
     q.g = p;
     q.ncols = epi == EPI_SWIGLU ? 2 * p.N : p.N;
     q.big_bm = bm_big;
-    q.big_grid = grid;
+    q.big_grid = bm_big == 128 ? 2 * grid : grid;  // (tiles to a round)
     return fp8 ? gs_dispatch<true>(q, 64, epi, ws, bytes, grid, s) : gs_dispatch<false>(q, 64, epi, ws, bytes, grid, s);
 }
 

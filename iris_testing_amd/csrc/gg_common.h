@@ -301,15 +301,15 @@ __device__ __forceinline__ GgRows gg_rows(const int32_t* cnt, int g, int E_l, in
     return {before + ex, min(c, left - ex), before + min(wave_lane(inc, WAVE - 1), left)};
 }
 
-constexpr int SUP = 16;  // super-tile edge, in large tiles
-// Tile idx of a group of Mt x Nt large tiles in the order they are walked: bands of 16 rows, super-columns of 16 within them.
-__device__ __forceinline__ void gg_patch(int idx, int Mt, int Nt, int& mt, int& nt) {
-    const int band = idx / (SUP * Nt), rem = idx % (SUP * Nt);
-    const int hr = min(SUP, Mt - band * SUP);
-    const int sc = rem / (hr * SUP), rem2 = rem % (hr * SUP);
-    const int wc = min(SUP, Nt - sc * SUP);
-    mt = band * SUP + rem2 / wc;
-    nt = sc * SUP + rem2 % wc;
+constexpr int SUP = 16, SUP_DUO = 8;  // super-tile edge, in tiles: of 256 rows, of 128 (gemm_duo.hip)
+// Tile idx of a group of Mt x Nt large tiles in the order they are walked: bands of `sup` rows, super-columns of `sup` within them.
+__device__ __forceinline__ void gg_patch(int idx, int Mt, int Nt, int sup, int& mt, int& nt) {
+    const int band = idx / (sup * Nt), rem = idx % (sup * Nt);
+    const int hr = min(sup, Mt - band * sup);
+    const int sc = rem / (hr * sup), rem2 = rem % (hr * sup);
+    const int wc = min(sup, Nt - sc * sup);
+    mt = band * sup + rem2 / wc;
+    nt = sc * sup + rem2 % wc;
 }
 
 // Tiles of a launch that the large kernel takes: all of them, or whole rounds of the grid when the rest is left to small tiles.
@@ -347,12 +347,14 @@ __device__ __forceinline__ void gg_zero_tail(const GemmParams& p, int total) {
         *(uint4*)((bf16_t*)p.C + (size_t)(total + i / nv) * p.ldc + (i % nv) * 8) = make_uint4(0, 0, 0, 0);
 }
 
-// gemm_small.hip: the tile height (32 or 64 rows) of the small-tile kernel for a launch, 0 where the large tiles are the
-// better choice; and that launch.
-int gs_choose_bm(int S_rows, int E_l, int K, int ncols, bool fp8, int cus, const void* part_ws, size_t part_ws_bytes);
+// gemm_small.hip: the time of a launch of small tiles (32 or 64 rows) as the choice between the kernels sees it; and that launch.
+double gs_estimate(int bm, double tiles, int nk, bool fp8, int cus, const void* part_ws, size_t part_ws_bytes);
 int gs_plan_parts(long long tiles, int bm, int nk, int cus, const void* part_ws, size_t bytes);  // parts per tile, as its kernel finds them
 size_t gs_workspace_bytes(int cus);  // (what its partial sums take at most)
 int launch_gemm_small(const GemmParams& p, bool fp8, int bm, int epi, void* ws, size_t bytes, int cus, hipStream_t s);
 // The tiles of a launch of large tiles (bm_big rows, grid workgroups) that GemmParams::tail_max left over.
 int launch_gemm_tail(const GemmParams& p, bool fp8, int bm_big, int epi, void* ws, size_t bytes, int grid, hipStream_t s);
+
+// gemm_duo.hip: tiles of 128 rows, two workgroups to a compute unit (GemmParams::tail_max as for 256-row tiles; weight gradients where dw_rows is set).
+int launch_gemm_duo(const GemmParams& p, bool fp8, int epi, int cus, hipStream_t s);
 }  // namespace moe_gg

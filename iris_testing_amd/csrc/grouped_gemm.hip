@@ -4,8 +4,8 @@
 // Replaces the reference's intended expert layer (layers/expert.py:31-60) and grouped_gemm kernel
 // (kernels.py:240-289): out[rows of group g] = tokens[rows of g] @ weights[g], fp32 accumulate,
 // persistent grid walking a tile list that spans all groups.  Differences in kind, not a port:
-//   * tiles are 256 (or 128) x 256, four wave64s each owning a 128 (64) x 128 block of 16x16x32 (bf16) or
-//     32x32x64 (fp8) MFMAs with the accumulators in the accumulation registers;
+//   * tiles are 256 x 256, four wave64s each owning a 128 x 128 block of 16x16x32 (bf16) MFMAs with the accumulators in the
+//     accumulation registers, or eight with 64 x 128 of 32x32x64 (fp8); tiles of 128 x 256 are gemm_duo.hip's;
 //   * operands go HBM -> LDS directly (global_load_lds, 16 bytes per lane) through a ring of four
 //     64-byte K stages, activations two stages (a cache line of every row) at a time; the loads are spread over the MFMA
 //     blocks, one to two blocks ahead; an XOR swizzle of the 16-byte chunks keeps MFMA fragment reads bank-conflict free;
@@ -82,7 +82,7 @@ __device__ __forceinline__ GgTile gg_decode(const int* g_tile_start, const int* 
     const int Mt = (cnt_g + BM - 1) / BM;
     const int idx = lin - g_tile_start[g];
     int mt, nt;
-    gg_patch(idx, Mt, Nt, mt, nt);
+    gg_patch(idx, Mt, Nt, SUP, mt, nt);
     GgTile t;
     t.g = g;
     t.nt = nt;
@@ -1669,29 +1669,60 @@ int round_up(int a, int b) { return (a + b - 1) / b * b; }
 // moe_diag_gemm_trace: where the next forward GEMM launches of this process leave time stamps (not thread-safe: a diagnostic)
 struct { unsigned long long* buf; int flags; } g_trace = {nullptr, 0};
 
-// What a launch of S_rows rows in E_l groups takes: the height of its tiles (32, 64: gemm_small.hip; 128, 256) and, for large ones,
+// What a launch of S_rows rows in E_l groups takes: the height of its tiles (32, 64: gemm_small.hip; 128: gemm_duo.hip; 256: above) and, for large ones,
 // GemmParams::tail_max.  The one place where that is decided (moe_gemm_launch_plan shows it).
+// The host knows the row total, not its split over the groups: every group adds about half a tile of ragged tail.  Of four estimates the smallest decides.
+// Their coefficients (us) are those whose choices were best over 2300 drawn launches, each timed on all four kernels (64 .. 40000 rows, 1 .. 32 groups, K and
+// columns 512 .. 14336, bf16 and fp8, even and skewed): bf16 1.3 % (geometric mean), fp8 0.7 % over the best of the four each time, where the rule before, without
+// the kernel of gemm_duo.hip but with a 128-row form of the one above, was at 6.4 and 3.6 %.  They are no launch's time: what two estimates share is left
+// out.  Tiles of 128 rows: 0.36 us per 64 bytes of K while a compute unit has one, 0.69 for every two; of 256 rows: 0.34 to 0.37, but they start 42 behind (few rounds
+// of few tiles fill the chip badly, and a tile's store and the next one's first stages stand alone on their unit).  So 128-row tiles serve short K at any number
+// of rows and long K up to some two rounds: 16384 rows of 8 groups x 2048 x 2048 139 us on 256-row tiles, 118 on these; 33618 rows of 32 x 7168 x 4096 1543 and 1638.
 struct GgChoice {
     int bm, tail_max;
 };
-static GgChoice gg_choose(int S_rows, int E_l, int K, int nt, int ncols, bool fp8, int grid, const void* part_ws, size_t part_ws_bytes,
-                          bool whole) {
-    whole |= S_rows > GG_SCAN_ROWS;
-    // launches that large tiles would leave mostly idle
-    const int bm_small = whole ? 0 : gs_choose_bm(S_rows, E_l, K, ncols, fp8, grid, part_ws, part_ws_bytes);
-    if (bm_small) return {bm_small, 0};
-    // 256-row or 128-row tiles: the host knows only the total row count, so it compares the estimated number
-    // of rounds of the persistent grid (every group adds about half a tile of ragged tail); a 128-row tile
-    // costs about 0.62 of a 256-row one
-    const double t256 = ((double)S_rows / 256 + 0.5 * E_l) * nt, t128 = ((double)S_rows / 128 + 0.5 * E_l) * nt;
-    const int bm = 0.62 * ceil(t128 / grid) < ceil(t256 / grid) ? 128 : 256;
-    if (whole) return {bm, 0};
-    const GgTail t = gg_tail(K * (fp8 ? 1 : 2) / ROWB, bm, fp8, grid);
-    if (E_l == 1) {  // (no group but this one: the host knows what is left over)
-        const int total = ceil_div(S_rows, bm) * nt;
-        return {bm, gg_whole_tiles(total, grid, t.most) == total ? 0 : t.most};
+constexpr int gg_round(int bm, int cus) { return bm == 128 ? 2 * cus : cus; }  // tiles that run at a time
+static GgChoice gg_choose(int S_rows, int E_l, int K, int nt, int ncols, bool fp8, int cus, const void* part_ws, size_t part_ws_bytes, bool whole) {
+    if (S_rows > GG_SCAN_ROWS) return {256, 0};
+    if (whole) {  // (time stamps: only the kernel above writes them, and only launches whose tiles it fills about as well as half-height ones would)
+        const double t256 = ((double)S_rows / 256 + 0.5 * E_l) * nt, t128 = ((double)S_rows / 128 + 0.5 * E_l) * nt;
+        return {0.62 * ceil(t128 / cus) < ceil(t256 / cus) ? 128 : 256, 0};
     }
-    return {bm, t.worth ? t.most : 0};
+    const int nk = K * (fp8 ? 1 : 2) / ROWB, nts = ceil_div(ncols, 128);
+    const double E = std::min(E_l, S_rows), stream = E * K * ncols * (fp8 ? 1 : 2) / 5.5e6;  // (us that the weights alone take)
+    GgChoice best = {32, 0};
+    // (where the weights are the time, in part out of the infinity cache, the smallest tiles)
+    double least = std::max(gs_estimate(32, (S_rows / 32.0 + 0.5 * E) * nts, nk, fp8, cus, part_ws, part_ws_bytes), 0.4 * stream);
+    auto consider = [&](int bm, double us) {
+        us = std::max(us, 0.4 * stream);
+        if (us < least) { least = us; best.bm = bm; }
+    };
+    consider(64, gs_estimate(64, (S_rows / 64.0 + 0.5 * E) * nts, nk, fp8, cus, part_ws, part_ws_bytes));
+    {
+        const double x = (S_rows / 128.0 + 0.5 * E) * nt / cus, two = std::min(1.0, std::max(0.0, (x - 0.9) / 0.27));
+        consider(128, 1.25 + (1 - two) * 0.36 * nk + two * std::max(1.0, x / 2 + 0.04) * 0.69 * nk + 0.09 * stream);
+    }
+    const GgTail t256 = gg_tail(nk, 256, fp8, cus), t128 = gg_tail(nk, 128, fp8, cus);
+    {
+        double us;
+        if (E == 1) {  // (no group but this one: the host knows the last round)
+            const int total = ceil_div(S_rows, 256) * nt, full = total / cus, rem = total % cus;
+            double last = rem ? 0.37 * nk : 0;
+            if (full && rem && rem <= t256.most) last = std::min(last, 4 + 0.15 * nk * (fp8 ? 1.4 : 1.225) * std::max(1.0, rem * 8.0 / cus));
+            us = 43 + full * 0.34 * nk + last;
+        } else {
+            const double x = (S_rows / 256.0 + 0.5 * E) * nt / cus;
+            us = x <= 1.2 ? 42.5 + 0.37 * nk : 43 + (x + 1) * 0.34 * nk;
+        }
+        consider(256, us + 0.045 * stream);
+    }
+    if (best.bm < 128) return best;
+    const GgTail t = best.bm == 128 ? t128 : t256;
+    if (E_l == 1) {
+        const int total = ceil_div(S_rows, best.bm) * nt;
+        best.tail_max = gg_whole_tiles(total, gg_round(best.bm, cus), t.most) == total ? 0 : t.most;
+    } else best.tail_max = t.worth ? t.most : 0;
+    return best;
 }
 
 template <bool FP8>
@@ -1706,9 +1737,19 @@ int launch_gemm(const GemmParams& p_in, int epi, hipStream_t s, void* part_ws = 
     }
     const GgChoice ch = gg_choose(p.S_rows, p.E_l, p.K, p.Npad / GG_BN, epi == EPI_SWIGLU ? 2 * p.N : p.N, FP8, grid, part_ws, part_ws_bytes, traced);
     if (ch.bm < 128) return launch_gemm_small(p, FP8, ch.bm, epi, part_ws, part_ws_bytes, grid, s);
-    const int bm = ch.bm;
-    const bool small_m = bm == 128;
     p.tail_max = ch.tail_max;
+    if (FP8 && epi == EPI_NONE && !p.a_bscale) return moe_fail(MOE_ERR_INVALID, "grouped_gemm: the fp8 down projection needs block scales");
+    auto tail = [&]() -> int {
+        if (!p.tail_max) return moe_check_launch("grouped_gemm");
+        GemmParams q = p;
+        q.zero_tail = 0;
+        return launch_gemm_tail(q, FP8, ch.bm, epi, part_ws, part_ws_bytes, grid, s);
+    };
+    if (ch.bm == 128) {
+        if (traced) return moe_fail(MOE_ERR_UNSUPPORTED, "grouped_gemm: no time-stamping instantiation for this launch (256-row tiles, no activation or SwiGLU)");
+        const int rc = launch_gemm_duo(p, FP8, epi, grid, s);
+        return rc ? rc : tail();
+    }
     // fp8 without activation is the down projection of the expert MLP: its activation operand is block-scaled
 #define GG_LAUNCH(BMv, NWMv, EPIv, MODEv)                                                                      \
     do {                                                                                                  \
@@ -1721,18 +1762,8 @@ int launch_gemm(const GemmParams& p_in, int epi, hipStream_t s, void* part_ws = 
         }                                                                                                 \
         grouped_gemm_kernel<BMv, NWMv, EPIv, FP8, MODEv, BSAv><<<grid, NWMv * 2 * WAVE, 0, s>>>(p); \
     } while (0)
-#define GG_EPI_MODE(EPIv, MODEv)                     \
-    do {                                             \
-        if (small_m) GG_LAUNCH(128, 2, EPIv, MODEv); \
-        else GG_LAUNCH(256, (FP8 ? (EPIv == EPI_NONE ? GG_FP8_BSA_NWM : GG_FP8_NWM) : GG_BIG_NWM), EPIv, MODEv); \
-    } while (0)
+#define GG_EPI_MODE(EPIv, MODEv) GG_LAUNCH(256, (FP8 ? (EPIv == EPI_NONE ? GG_FP8_BSA_NWM : GG_FP8_NWM) : GG_BIG_NWM), EPIv, MODEv)
 #define GG_EPI(EPIv) GG_EPI_MODE(EPIv, GG_B_PACKED)
-    auto tail = [&]() -> int {
-        if (!p.tail_max) return moe_check_launch("grouped_gemm");
-        GemmParams q = p;
-        q.zero_tail = 0;
-        return launch_gemm_tail(q, FP8, bm, epi, part_ws, part_ws_bytes, grid, s);
-    };
     if constexpr (!FP8) {  // weights in the reference layout
         if (p.b_mode != GG_B_PACKED) {
             if (traced) return moe_fail(MOE_ERR_UNSUPPORTED, "grouped_gemm: no time-stamping instantiation for weights in the reference layout");
@@ -1747,7 +1778,6 @@ int launch_gemm(const GemmParams& p_in, int epi, hipStream_t s, void* part_ws = 
     }
     switch (epi) {
         case EPI_NONE:
-            if (FP8 && !p.a_bscale) return moe_fail(MOE_ERR_INVALID, "grouped_gemm: the fp8 down projection needs block scales");
             GG_EPI(EPI_NONE);
             break;
         // (no fp8 entry point asks for these two: not instantiated)
@@ -1938,7 +1968,7 @@ extern "C" int moe_gemm_launch_plan(int S_rows, int E_l, int K, int N, int act, 
     const void* ws = part_ws_bytes ? out : nullptr;  // (any address: only whether there is one counts)
     const GgChoice ch = gg_choose(S_rows, E_l, K, ceil_div(ncols, GG_BN), ncols, fp8 != 0, cus, ws, part_ws_bytes, false);
     const bool large = ch.bm >= 128;
-    const int whole = large ? gg_whole_tiles(tiles, cus, ch.tail_max) : 0;
+    const int whole = large ? gg_whole_tiles(tiles, gg_round(ch.bm, cus), ch.tail_max) : 0;
     const int small = large ? (tiles - whole) * (ch.bm / 64) * (GG_BN / 128) : tiles;  // small tiles of the launch, or of its last round
     out[0] = ch.bm;
     out[1] = whole;
@@ -2249,7 +2279,13 @@ static int launch_dw(const void* x, const void* dy, const int32_t* expert_cnt, i
     p.A = (const uint8_t*)x; p.B = (const uint8_t*)dy; p.C = dw; p.cnt = expert_cnt;
     p.E_l = E_l; p.K = 64; p.N = N; p.Npad = round_up(N, GG_BN); p.ldc = ldc; p.S_rows = K;
     p.dw_rows = K; p.dw_src_rows = S_rows; p.dw_split = split_F; p.dw_delta = dw_delta; p.c_group_stride = (size_t)K * ldc;
-    grouped_gemm_kernel<256, GG_BIG_NWM, EPI_NONE, false, GG_B_DW><<<num_cus(), GG_BIG_NWM * 2 * WAVE, 0, s>>>(p);
+    // 128-row tiles (gemm_duo.hip) while 256-row ones do not fill the chip, and for short reductions over some rounds of them, where storing tiles is most of
+    // the work.  160 drawn launches: 0.53 to 0.85 of the time at up to half a round (817 rows of 2 groups x 576 x 640 18.2 us -> 10.6) and, up to 300 rows a
+    // group, to five rounds; from 10 rounds or some 2000 rows times rounds on 0.9 to 1.1 (33618 rows of 32 groups x 7168 x 4096: 1780 us, 1900 on these).
+    const int cus = num_cus();
+    const double rounds = (double)E_l * ceil_div(K, 256) * (p.Npad / GG_BN) / cus;
+    if (S_rows <= GG_SCAN_ROWS && (rounds <= 0.9 || (rounds <= 10 && rounds * S_rows / E_l <= 2000))) return launch_gemm_duo(p, false, EPI_NONE, cus, s);
+    grouped_gemm_kernel<256, GG_BIG_NWM, EPI_NONE, false, GG_B_DW><<<cus, GG_BIG_NWM * 2 * WAVE, 0, s>>>(p);
     return moe_check_launch("grouped_gemm_dw");
 }
 
