@@ -6,7 +6,8 @@
 // MFMAs of the others), a plain ring of LDS stages, and the K range of every tile cut into P parts when there are fewer tiles
 // than workgroups the chip can hold.  The parts of a tile leave their fp32 sums in the workspace; the workgroup that finishes
 // last adds them in part order (so the result does not depend on who that is) and applies the epilogue: one launch, where
-// the large-tile path needs a launch for whole tiles, one for the parts and one for their reduction.
+// the large-tile path needs a launch for whole tiles, one for the parts and one for their reduction.  Where every tile has a compute unit
+// to itself, two sets of four waves share one (KG = 2): pairs of stages in turn, each set through its own ring, the sums added at the end.
 #include "gg_common.h"
 #include <algorithm>
 #include <atomic>
@@ -32,10 +33,10 @@ struct GsShape {
     static constexpr int RA = BM / 32;                        // activation loads per wave and pair of stages (1 KB each)
     static constexpr int RB = GS_BN / 64;                     // weight loads per wave and stage
 };
-template <int BM, bool BSA>
+template <int BM, bool BSA, int KG>
 constexpr int gs_lds_bytes() {
     using S = GsShape<BM>;
-    const int ring = S::NST * (BM + GS_BN) * 2 * ROWB + (BSA ? 4 * S::NST * 256 : 0);
+    const int ring = KG * (S::NST * (BM + GS_BN) * 2 * ROWB + (BSA ? 4 * S::NST * 256 : 0));
     const int epi = BM * GS_LDO * 4;
     return ring > epi ? ring : epi;
 }
@@ -57,8 +58,8 @@ __host__ __device__ inline int gs_parts(long long tiles, int slots, int nk, int 
     return P < 1 ? 1 : P;
 }
 
-template <int BM, bool FP8, int EPI, bool BSA, int BMODE, bool TAIL>
-__global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParams q) {
+template <int BM, bool FP8, int EPI, bool BSA, int BMODE, bool TAIL, int KG>
+__global__ __launch_bounds__(GS_THREADS * KG, 2) void gemm_small_kernel(const GsParams q) {
     constexpr bool BT = BMODE == GG_B_T, BN_PAIR = BMODE == GG_B_NP, BN_RAW = BMODE == GG_B_N || BN_PAIR;  // (see GG_B_*)
     static_assert(!FP8 || BMODE == GG_B_PACKED, "raw weights are a bf16 matter");
     using S = GsShape<BM>;
@@ -74,7 +75,8 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
     __shared__ int s_last;
     const GemmParams& p = q.g;
     const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) & 3, kg = KG > 1 ? __builtin_amdgcn_readfirstlane(tid >> 8) : 0;  // (of the set; the set)
+    constexpr int NTH = GS_THREADS * KG;
     const int wm = wave / S::WN, wn = wave % S::WN;
 
     // ---- this workgroup's unit: group, column tile, row tile, part.  Every wave scans the row counts by itself (64 groups at
@@ -176,15 +178,15 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
         else boff[r] = (uint32_t)(r * 64 + wave * WROWS + (lane >> 2)) * ROWB + lchunk * 16;
     }
     static_assert(!BN_RAW || RB == 2, "two loads per wave and stage");
-    uint8_t* const sA = lds;
-    uint8_t* const sB = lds + NST * 2 * ASZ;
-    uint32_t* const sS = (uint32_t*)(lds + NST * 2 * (ASZ + BSZ)) + wave * NST * 64;  // (BSA) the wave's scale dwords, one per row
+    uint8_t* const sA = lds + kg * (gs_lds_bytes<BM, BSA, KG>() / KG);
+    uint8_t* const sB = sA + NST * 2 * ASZ;
+    uint32_t* const sS = (uint32_t*)(sA + NST * 2 * (ASZ + BSZ)) + wave * NST * 64;  // (BSA) the wave's scale dwords, one per row
     const uint32_t la0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr_t)sA) + wave * 1024;
     const uint32_t lb0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr_t)sB) + wave * WROWS * ROWB;
     [[maybe_unused]] const uint32_t ls0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr_t)sS);
     [[maybe_unused]] const uint32_t soff = BSA ? (uint32_t)(row0 + min(wm * S::WR + (lane & (S::WR - 1)), rv - 1)) * (uint32_t)p.bs_pitch : 0u;
 
-    const int npair = nks / 2;
+    const int npair = nks / 2, mine = (npair + KG - 1 - kg) / KG, steps = (npair + KG - 1) / KG;  // pairs of the set (kg, kg + KG, ...), steps of all
     // load d (0 .. LPS - 1) of the pair whose first stage lies at ap / bp: activations, weights, (BSA) scale dwords
     // (bp[stage][matrix of a pair])
     typedef typename std::conditional<BMODE == GG_B_PACKED, const uint8_t*, gg_i32x4>::type bsrc_t;
@@ -196,7 +198,7 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
         } else if constexpr (BSA) gg_dma4(sp, soff, ls0 + slot * 256);
     };
 #define GS_PAIR_PTRS(pr)                                                    \
-    const int st_ = 2 * min((pr), npair - 1);                               \
+    const int st_ = 2 * min((pr) * KG + kg, npair - 1);                     \
     const uint8_t* ap_ = gg_uniform(Ab + (size_t)st_ * ROWB);               \
     bsrc_t bp_[2][2];                                                       \
     _Pragma("unroll") for (int u_ = 0; u_ < 2; ++u_)                         \
@@ -290,6 +292,7 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
         asm volatile("" ::: "memory");
         read(nxt, slot);
         __builtin_amdgcn_sched_barrier(0);
+        if (KG > 1 && s >= mine) return;  // (an odd number of pairs: this set has none left)
         constexpr int NM = 2 * TM * TN, STEP = NM / LPS > 0 ? NM / LPS : 1, PER = (LPS + NM - 1) / NM;  // MFMAs per load, loads per MFMA
 #pragma unroll
         for (int m = 0; m < NM; ++m) {
@@ -308,9 +311,9 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-    for (int s = 0; s < npair; s += 2) {
+    for (int s = 0; s < steps; s += 2) {
         step(f0, f1, s);
-        if (s + 1 < npair) step(f1, f0, s + 1);
+        if (s + 1 < steps) step(f1, f0, s + 1);
     }
     asm volatile("" ::: "memory");
     gg_wait<0, 0>();
@@ -321,7 +324,7 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
     // with the sums read back from there.
     float* const so = (float*)lds;
     constexpr int OCW = EPI == EPI_SWIGLU ? GS_BN / 2 : GS_BN;  // output columns of the tile
-    constexpr int TPR = OCW / 8, RPP = GS_THREADS / TPR;         // threads per row, rows per pass
+    constexpr int TPR = OCW / 8, RPP = NTH / TPR;         // threads per row, rows per pass
     const int oc = (tid % TPR) * 8;                              // the thread's first output column inside the tile
     const int pc = EPI == EPI_SWIGLU ? (oc / 32) * 64 + oc % 32 : oc;  // its packed column inside the tile
     const int gp = nt * GS_BN + pc;
@@ -397,17 +400,28 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
     float* const ws = P > 1 ? (float*)((uint8_t*)p.part_ws + GS_CTR_BYTES) : nullptr;
     constexpr int NQ = FP8 ? 4 : 1;
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+    for (int set = KG - 1; set >= 0; --set) {  // (the second set leaves its sums, the first adds its own)
+        if (set == kg) {
 #pragma unroll
-        for (int j = 0; j < TN; ++j)
+            for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int v = 0; v < NQ; ++v) {
-                // four consecutive rows of the weight tile are four consecutive columns
-                const int r = wm * S::WR + i * MT + (lane & (MT - 1));
-                const int c = gg_packed_col<FP8>(wn * S::WC + j * MT + (FP8 ? 8 * v + 4 * (lane >> 5) : 4 * (lane >> 4)));
-                *(float4*)(so + r * GS_LDO + c) = make_float4(acc[i][j][4 * v], acc[i][j][4 * v + 1], acc[i][j][4 * v + 2], acc[i][j][4 * v + 3]);
-            }
-    __syncthreads();
+                for (int j = 0; j < TN; ++j)
+#pragma unroll
+                    for (int v = 0; v < NQ; ++v) {
+                        // four consecutive rows of the weight tile are four consecutive columns
+                        const int r = wm * S::WR + i * MT + (lane & (MT - 1));
+                        const int c = gg_packed_col<FP8>(wn * S::WC + j * MT + (FP8 ? 8 * v + 4 * (lane >> 5) : 4 * (lane >> 4)));
+                        float4* const at = (float4*)(so + r * GS_LDO + c);
+                        float4 a = make_float4(acc[i][j][4 * v], acc[i][j][4 * v + 1], acc[i][j][4 * v + 2], acc[i][j][4 * v + 3]);
+                        if (KG > 1 && set == 0) {
+                            const float4 b = *at;
+                            a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w;
+                        }
+                        *at = a;
+                    }
+        }
+        __syncthreads();
+    }
     // (whole passes of RPP rows: the threads that hold a block of columns of a row stay together)
     const int r_end = min((rv + RPP - 1) & ~(RPP - 1), BM);
     if (P == 1) {
@@ -424,7 +438,7 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_small_kernel(const GsParam
         return;
     }
     unsigned long long* const o = (unsigned long long*)(ws + (size_t)unit * (BM * GS_BN));
-    for (int i = tid; i < rv * (GS_BN / 2); i += GS_THREADS)
+    for (int i = tid; i < rv * (GS_BN / 2); i += NTH)
         __hip_atomic_store(o + i, *(const unsigned long long*)(so + (i / (GS_BN / 2)) * GS_LDO + 2 * (i % (GS_BN / 2))), __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_AGENT);
     // arrival: the sums above are written through to memory; once they are acknowledged the part counts itself in.  The
@@ -502,7 +516,6 @@ int gs_plan_parts(long long tiles, int bm, int nk, int cus, const void* part_ws,
 template <int BM, bool FP8, int EPI, bool BSA, int BMODE>
 static void gs_launch(const GsParams& q0, void* part_ws, size_t part_ws_bytes, int cus, hipStream_t s) {
     GsParams q = q0;
-    constexpr int lds = gs_lds_bytes<BM, BSA>();
     q.slots = gs_slots(BM, cus);
     q.g.max_units = gs_max_units(BM, part_ws, part_ws_bytes);
     q.g.part_ws = q.g.max_units ? (float*)part_ws : nullptr;
@@ -514,11 +527,18 @@ static void gs_launch(const GsParams& q0, void* part_ws, size_t part_ws_bytes, i
     q.nonce = gs_nonce();
     if constexpr (BM == 64) {
         if (q.big_bm) {
-            gemm_small_kernel<BM, FP8, EPI, BSA, BMODE, true><<<units((long long)q.g.tail_max * (q.big_bm / BM) * (GG_BN / GS_BN)), GS_THREADS, lds, s>>>(q);
+            gemm_small_kernel<BM, FP8, EPI, BSA, BMODE, true, 1><<<units((long long)q.g.tail_max * (q.big_bm / BM) * (GG_BN / GS_BN)), GS_THREADS, gs_lds_bytes<BM, BSA, 1>(), s>>>(q);
             return;
         }
     }
-    gemm_small_kernel<BM, FP8, EPI, BSA, BMODE, false><<<units(ub), GS_THREADS, lds, s>>>(q);
+    // Two sets of waves to a tile where every tile has a compute unit to itself: what bounds such a launch is how long the weights take to come, and two sets
+    // have twice as many stages under way.  Weights from memory: 443 rows of two groups x 2048 x 4096 19.4 -> 18.3 us, x 4096 x 2048 24.6 -> 22.9, 482 of 2 x 3840 x 1664
+    // 25.8 -> 22.8; short K gains nothing (1088: 12.0, 12.0) or pays for adding the sets up (576: 7.6 -> 8.1), and so do groups of a few rows
+    // (77 rows of 32 x 5440 x 896 50.9 -> 53.8); a second round of such workgroups costs 1.04 to 1.36 times.
+    if (ub <= cus && q.g.K * (FP8 ? 1 : 2) >= 54 * ROWB && q.g.S_rows >= 8 * q.g.E_l)
+        gemm_small_kernel<BM, FP8, EPI, BSA, BMODE, false, 2><<<units(ub), GS_THREADS * 2, gs_lds_bytes<BM, BSA, 2>(), s>>>(q);
+    else
+        gemm_small_kernel<BM, FP8, EPI, BSA, BMODE, false, 1><<<units(ub), GS_THREADS, gs_lds_bytes<BM, BSA, 1>(), s>>>(q);
 }
 
 template <bool FP8>

@@ -72,6 +72,19 @@ def test_small_gemm_edges(cnt, K, N, act, workspace):
         assert torch.equal(out.view(torch.int16), first.view(torch.int16))
 
 
+# two sets of waves to a tile (every tile a compute unit to itself, 54 stages of K or more): odd and even numbers of pairs of stages, whole and in parts
+@pytest.mark.parametrize("cnt,K,N,act", [((33, 31), 1728, 200, "silu"), ((64, 0, 17), 1856, 96, "swiglu"), ((70,), 1792, 1032, "none"), ((100, 28), 4160, 136, "gelu")])
+@pytest.mark.parametrize("workspace", [False, True], ids=["whole", "parts"])
+def test_small_gemm_two_sets_of_waves(cnt, K, N, act, workspace):
+    test_small_gemm_edges(cnt, K, N, act, workspace)
+
+
+@pytest.mark.parametrize("cnt,H,F", [((40,), 3456, 3584), ((65, 9), 4224, 128)])
+@pytest.mark.parametrize("workspace", [False, True], ids=["whole", "parts"])
+def test_small_fp8_mlp_two_sets_of_waves(cnt, H, F, workspace):
+    test_small_fp8_mlp_edges(cnt, H, F, workspace)
+
+
 @pytest.mark.parametrize("cnt,H,F", [((1,), 128, 128), ((33, 0, 64), 384, 256), ((65,), 4096, 640), ((20, 7), 2048, 2176),
                                      ((6000,), 2048, 1408)])  # (the last: large tiles with 8 left over)
 @pytest.mark.parametrize("workspace", [False, True], ids=["whole", "parts"])
