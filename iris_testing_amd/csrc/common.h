@@ -101,3 +101,17 @@ static inline int dtype_size(int dtype) { return dtype == MOE_F32 ? 4 : (dtype =
 static inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 // whether 16-byte loads and stores may start at p (NULL: there is nothing to load)
 static inline bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
+// f(k as a constant where kernels have a form for it, else 0)
+template <typename F>
+static inline void with_topk(int k, F&& f) {
+    switch (k) {
+        case 1: return f(std::integral_constant<int, 1>{});
+        case 2: return f(std::integral_constant<int, 2>{});
+        case 4: return f(std::integral_constant<int, 4>{});
+        case 8: return f(std::integral_constant<int, 8>{});
+        case 16: return f(std::integral_constant<int, 16>{});
+        default: return f(std::integral_constant<int, 0>{});
+    }
+}
+template <int KT>
+constexpr int topk_slots() { return KT ? KT : MOE_MAX_TOPK; }

@@ -639,17 +639,48 @@ inline int row_parts(int tokens, int row_vec) {
 inline int combine_parts(int tokens, int row_vec) {
     return tokens < 2048 ? row_parts(tokens, row_vec) : max(1, min(min(16384 / tokens, row_vec / (2 * WAVE)), 4));
 }
-template <int WPB>
+// Columns [c_lo, c_hi) of a token's row to the rows of send that slots(drow) names (k of them; -1: none).  Eight 16-byte loads in flight per lane (fewer
+// at the end of a row, or when the row is shorter than 8 KB), the first ones under way while the slots are looked up.
+// KT: the top-k, or 0 for any.  With few tokens the launch is a chain of round trips to memory, and sixteen slots spelt out, most of them jumped
+// over, are more of them, for instructions: 256 x 1 KB, top-2, 4.3 -> 3.6 us, 512 x 4 KB, top-1, 5.3 -> 4.6, 24 x 14 KB, top-8, 6.7 -> 6.3; with
+// many tokens of short rows they are work: 65536 x 1 KB, top-2, 74 -> 42, 8192 x 1.5 KB, top-2, 13.9 -> 8.6; 4096 x 14 KB, top-8, 115 -> 110.
+template <int KT, typename F>
+__device__ __forceinline__ void pack_row(const u32x4* __restrict__ src, u32x4* __restrict__ send, int k, int row_vec, int c_lo, int c_hi, int lane, F&& slots) {
+    constexpr int KM = topk_slots<KT>();
+    u32x4 v[8];
+    auto load = [&](int c) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (c + u * WAVE < c_hi) v[u] = __builtin_nontemporal_load(src + c + u * WAVE);
+    };
+    if (KT) load(c_lo + lane);
+    int drow[KM];
+    slots(drow);
+    for (int c = c_lo + lane; c < c_hi; c += 8 * WAVE) {
+        if (!KT || c >= c_lo + 8 * WAVE) load(c);
+#pragma unroll
+        for (int j = 0; j < KM; ++j) {
+            if ((KT || j < k) && drow[j] >= 0) {
+                u32x4* o = send + (size_t)drow[j] * row_vec + c;
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    if (c + u * WAVE < c_hi) __builtin_nontemporal_store(v[u], o + u * WAVE);
+            }
+        }
+    }
+}
+template <int WPB, int KT>
 __global__ __launch_bounds__(WPB * WAVE) void pack_tokens_kernel(const u32x4* __restrict__ x, u32x4* __restrict__ send,
                                                                   const int32_t* __restrict__ idx, const int32_t* __restrict__ pos,
                                                                   const int32_t* __restrict__ dst_sizes,
-                                                                  const int32_t* __restrict__ dst_offsets, int T, int k, int E_l,
+                                                                  const int32_t* __restrict__ dst_offsets, int T, int k_rt, int E_l,
                                                                   int W, int M, int row_vec, int32_t* __restrict__ status,
                                                                   const float* __restrict__ gate, float* __restrict__ send_gate, int parts) {
     // gate / send_gate (both or neither): the slot's top-k gate travels with its row, send_gate[d,m] = gate[t,kk], zero
     // in the padding slots -- for a destination that applies the gate to the expert's result before sending it back
     // parts: waves per token, each with its own run of columns (see row_parts)
-    const int wave = threadIdx.x / WAVE, lane = lane_id();
+    constexpr int KM = topk_slots<KT>();
+    const int wave = threadIdx.x / WAVE, lane = lane_id(), k = KT ? KT : k_rt;
     const int n_slots = W * M, n_tok = T * parts;
     const int per = ((row_vec + parts - 1) / parts + WAVE - 1) / WAVE * WAVE;
     const int n_units = n_tok + (n_slots + PACK_ZR - 1) / PACK_ZR;
@@ -673,35 +704,19 @@ __global__ __launch_bounds__(WPB * WAVE) void pack_tokens_kernel(const u32x4* __
         }
         const int r = unit / parts, c_lo = (unit % parts) * per, c_hi = min(c_lo + per, row_vec);
         // destination rows of the token's k slots (-1: beyond the pair capacity, dropped like the gather drops it)
-        int drow[MOE_MAX_TOPK];
+        pack_row<KT>(x + (size_t)r * row_vec, send, k, row_vec, c_lo, c_hi, lane, [&](int (&drow)[KM]) {
 #pragma unroll
-        for (int j = 0; j < MOE_MAX_TOPK; ++j) {
-            drow[j] = -1;
-            if (j < k) {
-                const int d = idx[(size_t)r * k + j] / E_l;
-                const bool d_ok = (unsigned)d < (unsigned)W;  // (an expert id outside [0, W E_l): no slot, and no read of its offset)
-                const int m = pos[(size_t)r * k + j] - dst_offsets[d_ok ? d : 0];
-                if (d_ok && (unsigned)m < (unsigned)M) drow[j] = d * M + m;
-                if (send_gate && drow[j] >= 0 && lane == 0 && c_lo == 0) send_gate[drow[j]] = gate[(size_t)r * k + j];
-            }
-        }
-        const u32x4* src = x + (size_t)r * row_vec;
-        // eight 16-byte loads in flight per lane (fewer at the end of a row, or when the row is shorter than 8 KB)
-        for (int c = c_lo + lane; c < c_hi; c += 8 * WAVE) {
-            u32x4 v[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u)
-                if (c + u * WAVE < c_hi) v[u] = __builtin_nontemporal_load(src + c + u * WAVE);
-#pragma unroll
-            for (int j = 0; j < MOE_MAX_TOPK; ++j) {
-                if (j < k && drow[j] >= 0) {
-                    u32x4* o = send + (size_t)drow[j] * row_vec + c;
-#pragma unroll
-                    for (int u = 0; u < 8; ++u)
-                        if (c + u * WAVE < c_hi) __builtin_nontemporal_store(v[u], o + u * WAVE);
+            for (int j = 0; j < KM; ++j) {
+                drow[j] = -1;
+                if (KT || j < k) {
+                    const int d = idx[(size_t)r * k + j] / E_l;
+                    const bool d_ok = (unsigned)d < (unsigned)W;  // (an expert id outside [0, W E_l): no slot, and no read of its offset)
+                    const int m = pos[(size_t)r * k + j] - dst_offsets[d_ok ? d : 0];
+                    if (d_ok && (unsigned)m < (unsigned)M) drow[j] = d * M + m;
+                    if (send_gate && drow[j] >= 0 && lane == 0 && c_lo == 0) send_gate[drow[j]] = gate[(size_t)r * k + j];
                 }
             }
-        }
+        });
     }
 }
 
@@ -1107,9 +1122,9 @@ extern "C" size_t moe_count_workspace_bytes(int T, int k, int E) {
     return sizeof(int32_t) * (2 * (size_t)E * NB + 2 * (size_t)E + 1);
 }
 
-static int count_and_offsets(const int32_t* topk_idx, int T, int k, int E, int W, int32_t* send_counts, int32_t* expert_offs,
-                             int32_t* dst_sizes, int32_t* dst_offsets, int32_t* caps, int32_t* pos, int32_t* row_token, void* ws,
-                             size_t ws_bytes, const RecvPrepare* side, int side_blocks, hipStream_t s) {
+static int check_count(const int32_t* topk_idx, int T, int k, int E, int W, const int32_t* send_counts, const int32_t* expert_offs,
+                       const int32_t* dst_sizes, const int32_t* dst_offsets, const int32_t* caps, const int32_t* pos, const int32_t* row_token,
+                       const void* ws, size_t ws_bytes) {
     MOE_REQUIRE(T >= 0 && E > 0 && W > 0, MOE_ERR_INVALID, "count: bad shape T=%d E=%d W=%d", T, E, W);
     MOE_REQUIRE(E % W == 0, MOE_ERR_INVALID, "num_experts_total must be divisible by world_size (E=%d W=%d)", E, W);
     MOE_REQUIRE(k >= 1 && k <= MOE_MAX_TOPK, MOE_ERR_UNSUPPORTED, "count: topk=%d outside [1,%d]", k, MOE_MAX_TOPK);
@@ -1118,6 +1133,14 @@ static int count_and_offsets(const int32_t* topk_idx, int T, int k, int E, int W
     MOE_REQUIRE(T == 0 || (topk_idx && pos && row_token), MOE_ERR_INVALID, "count: null pointer");
     MOE_REQUIRE(ws_bytes >= moe_count_workspace_bytes(T, k, E), MOE_ERR_WORKSPACE, "count: workspace %zu < %zu", ws_bytes,
                 moe_count_workspace_bytes(T, k, E));
+    return MOE_OK;
+}
+
+static int count_and_offsets(const int32_t* topk_idx, int T, int k, int E, int W, int32_t* send_counts, int32_t* expert_offs,
+                             int32_t* dst_sizes, int32_t* dst_offsets, int32_t* caps, int32_t* pos, int32_t* row_token, void* ws,
+                             size_t ws_bytes, const RecvPrepare* side, int side_blocks, hipStream_t s) {
+    const int rc = check_count(topk_idx, T, k, E, W, send_counts, expert_offs, dst_sizes, dst_offsets, caps, pos, row_token, ws, ws_bytes);
+    if (rc) return rc;
     const int NB = ceil_div(T > 0 ? T : 1, CB);
     int32_t* hist = (int32_t*)ws;
     auto lds = [&](int blocks) { return (size_t)blocks * E * sizeof(unsigned long long); };
@@ -1216,13 +1239,19 @@ extern "C" int moe_max_floor1(const int32_t* values, int n, int32_t* out, moe_st
     return moe_check_launch("max_floor1");
 }
 
-extern "C" int moe_pack_payload(const void* x, int dtype, int T, int H, const int32_t* row_token, int R, void* payload,
-                                moe_stream_t stream) {
-    int rc = check_rows("pack_payload", dtype, H);
+static int check_pack_payload(const void* x, int dtype, int T, int H, const int32_t* row_token, int R, const void* payload) {
+    const int rc = check_rows("pack_payload", dtype, H);
     if (rc) return rc;
     MOE_REQUIRE(R >= 0 && T >= 0, MOE_ERR_INVALID, "pack_payload: bad shape");
+    MOE_REQUIRE(R == 0 || (x && row_token && payload), MOE_ERR_INVALID, "pack_payload: null pointer");
+    return MOE_OK;
+}
+
+extern "C" int moe_pack_payload(const void* x, int dtype, int T, int H, const int32_t* row_token, int R, void* payload,
+                                moe_stream_t stream) {
+    const int rc = check_pack_payload(x, dtype, T, H, row_token, R, payload);
+    if (rc) return rc;
     if (R == 0) return MOE_OK;
-    MOE_REQUIRE(x && row_token && payload, MOE_ERR_INVALID, "pack_payload: null pointer");
     RowSource a{};
     a.mode = SRC_MAP;
     a.map = row_token;
@@ -1249,10 +1278,9 @@ extern "C" int moe_pack(const void* x, int dtype, int T, int H, const int32_t* r
     return gather_rows(x, send_buf, a, W * M, H * dtype_size(dtype), s);
 }
 
-extern "C" int moe_pack_tokens_gated(const void* x, int dtype, int T, int H, const int32_t* topk_idx, const int32_t* pos,
-                                     const float* gate, int k, int E_l, const int32_t* dst_sizes, const int32_t* dst_offsets, int W,
-                                     int M, void* send_buf, float* send_gate, int32_t* status, moe_stream_t stream) {
-    int rc = check_rows("pack_tokens", dtype, H);
+static int check_pack_tokens(const void* x, int dtype, int T, int H, const int32_t* topk_idx, const int32_t* pos, const float* gate, int k, int E_l,
+                             const int32_t* dst_sizes, const int32_t* dst_offsets, int W, int M, const void* send_buf, const float* send_gate) {
+    const int rc = check_rows("pack_tokens", dtype, H);
     MOE_REQUIRE((gate == nullptr) == (send_gate == nullptr), MOE_ERR_INVALID, "pack_tokens: gate and send_gate go together");
     if (rc) return rc;
     MOE_REQUIRE(W > 0 && M >= 1 && T >= 0 && E_l > 0, MOE_ERR_INVALID, "pack_tokens: bad shape W=%d M=%d E_l=%d", W, M, E_l);
@@ -1260,12 +1288,21 @@ extern "C" int moe_pack_tokens_gated(const void* x, int dtype, int T, int H, con
     MOE_REQUIRE((long long)W * M + T < (1ll << 31), MOE_ERR_UNSUPPORTED, "pack_tokens: W*M + T too large");
     MOE_REQUIRE(send_buf && dst_sizes && dst_offsets, MOE_ERR_INVALID, "pack_tokens: null pointer");
     MOE_REQUIRE(T == 0 || (x && topk_idx && pos), MOE_ERR_INVALID, "pack_tokens: null pointer");
+    return MOE_OK;
+}
+
+extern "C" int moe_pack_tokens_gated(const void* x, int dtype, int T, int H, const int32_t* topk_idx, const int32_t* pos,
+                                     const float* gate, int k, int E_l, const int32_t* dst_sizes, const int32_t* dst_offsets, int W,
+                                     int M, void* send_buf, float* send_gate, int32_t* status, moe_stream_t stream) {
+    const int rc = check_pack_tokens(x, dtype, T, H, topk_idx, pos, gate, k, E_l, dst_sizes, dst_offsets, W, M, send_buf, send_gate);
+    if (rc) return rc;
     const int parts = row_parts(T, H * dtype_size(dtype) / 16);
     const int n_units = T * parts + ceil_div(W * M, PACK_ZR);
     const int blocks = min(ceil_div(n_units, 4), 65535 * 8);
-    pack_tokens_kernel<4><<<blocks, 4 * WAVE, 0, (hipStream_t)stream>>>((const u32x4*)x, (u32x4*)send_buf, topk_idx, pos, dst_sizes,
-                                                                        dst_offsets, T, k, E_l, W, M,
-                                                                        H * dtype_size(dtype) / 16, status, gate, send_gate, parts);
+    with_topk(k, [&](auto kt) {
+        pack_tokens_kernel<4, decltype(kt)::value><<<blocks, 4 * WAVE, 0, (hipStream_t)stream>>>(
+            (const u32x4*)x, (u32x4*)send_buf, topk_idx, pos, dst_sizes, dst_offsets, T, k, E_l, W, M, H * dtype_size(dtype) / 16, status, gate, send_gate, parts);
+    });
     return moe_check_launch("pack_tokens");
 }
 
@@ -1375,7 +1412,8 @@ extern "C" int moe_recv_prepare(const int32_t* recv_counts, int W, int E_l, int 
                           H * dtype_size(dtype), (hipStream_t)stream);
 }
 
-int moe_count_and_prepare(const moe_step_args* a, hipStream_t s) {
+// The receive side's preparation for a step, as blocks of `threads` beside another launch's
+static int step_recv_prepare(const moe_step_args* a, int threads, RecvPrepare* side, int* blocks) {
     const int E_l = a->experts / a->world, M = a->flat ? 0 : a->M;
     const float *recv_gate = a->gated ? a->recv_gate : nullptr, *recv_scale = a->q_dispatch ? a->recv_scale : nullptr;
     float *row_gate = a->gated ? a->row_gate : nullptr, *row_scale = a->q_dispatch ? a->xs : nullptr;
@@ -1383,9 +1421,16 @@ int moe_count_and_prepare(const moe_step_args* a, hipStream_t s) {
     const int rc = check_recv_prepare(a->recv_counts, a->world, E_l, M, a->S, recv_gate, recv_scale, a->row_map, row_gate, row_scale, ret, a->dtype,
                                       a->hidden);
     if (rc) return rc;
+    *side = recv_prepare_args(a->recv_counts, a->world, E_l, M, a->S, a->row_map, a->expert_cnt, recv_gate, row_gate, recv_scale, row_scale, ret,
+                              a->hidden * dtype_size(a->dtype), threads, *blocks);
+    return MOE_OK;
+}
+
+int moe_count_and_prepare(const moe_step_args* a, hipStream_t s) {
+    RecvPrepare side;
     int blocks;
-    const RecvPrepare side = recv_prepare_args(a->recv_counts, a->world, E_l, M, a->S, a->row_map, a->expert_cnt, recv_gate, row_gate, recv_scale,
-                                               row_scale, ret, a->hidden * dtype_size(a->dtype), RANK_WAVES * WAVE, blocks);
+    const int rc = step_recv_prepare(a, RANK_WAVES * WAVE, &side, &blocks);
+    if (rc) return rc;
     return count_and_offsets(a->idx, a->tokens, a->topk, a->experts, a->world, a->send_counts, a->expert_offs, a->dst_sizes, a->dst_offsets, a->caps,
                              a->pos, a->row_token, a->count_ws, a->count_ws_bytes, &side, blocks, s);
 }
