@@ -17,6 +17,9 @@ int moe_check_launch(const char* what);
 
 // dispatch.hip, for step.hip: moe_count_and_offsets and moe_recv_prepare with one launch less
 int moe_count_and_prepare(const moe_step_args* a, hipStream_t s);
+// ... and where moe_count_with_pack says so, the count (with prepare: both) and the bf16 or fp32 pack in one
+bool moe_count_with_pack(int T, int k);
+int moe_count_and_pack(const moe_step_args* a, bool prepare, hipStream_t s);
 // grouped_gemm.hip, for step.hip: moe_unpack_expert_major of fp32 rows, moe_grouped_mlp and moe_return_pack, in two launches where tiles are small (S_rows > 0)
 int moe_mlp_f32_slots(const float* recv, const int32_t* recv_counts, int W, int M, int S_rows, int H, int F, int E_l, int act, const float* w1,
                       const float* w_up, const float* w2, float* rows, int32_t* expert_cnt, float* hidden_ws, float* y, float* ret,

@@ -720,6 +720,125 @@ __global__ __launch_bounds__(WPB * WAVE) void pack_tokens_kernel(const u32x4* __
     }
 }
 
+// Count and pack of few tokens in one launch: every wave works out for itself where its token's rows go, from the expert ids of all slots (a few
+// KB, from L2), so nothing has to wait for a ranking in front.  The row of a slot is the slots of lower experts plus those of its own in earlier
+// tokens; with key = expert * T k + slot (a token holds an expert at most once) that is the number of smaller keys, and the keys below the first of
+// its destination's experts are the rows in front of the destination: a compare, a ballot and a bit count for 64 slots.
+// Block 0 counts the experts and leaves the tables; blocks 1 to side_blocks prepare the receive side (see rank_kernel); the others are the
+// units of pack_tokens_kernel, whose bytes these are.  M = 0: the padding-free payload, row = position.
+// What it saves is the ranking's launch, most of whose time is its start and a chain of small steps.  A step of 256 fp32 tokens x 1 KB, top-2, 34.7 -> 31.8 us;
+// 512 x 4 KB, top-1, 66.6 -> 63.8; 24 x 14 KB, top-8, 352 -> 349; 777 x 4 KB, top-2, flat, 111.5 -> 106.8.
+struct CountOut {
+    int32_t *send_counts, *expert_offs, *dst_sizes, *dst_offsets, *caps, *pos, *row_token;
+};
+template <int KT>
+__global__ __launch_bounds__(256) void count_pack_kernel(const u32x4* __restrict__ x, u32x4* __restrict__ send, const int32_t* __restrict__ idx, int T, int k_rt,
+                                                          int E, int W, int M, int row_vec, const CountOut out, int32_t* __restrict__ status,
+                                                          const float* __restrict__ gate, float* __restrict__ send_gate, int parts, int side_blocks,
+                                                          const RecvPrepare side) {
+    __shared__ int32_t tot[MOE_MAX_EXPERTS], es[MOE_MAX_EXPERTS + 1];
+    extern __shared__ int32_t copies[];  // [RANK_COPIES][E | 1]
+    constexpr int KM = topk_slots<KT>();
+    const int tid = threadIdx.x, lane = lane_id(), k = KT ? KT : k_rt, n = T * k, E_l = E / W;
+    if (blockIdx.x == 0) {
+        const int stride = E | 1;
+        for (int i = tid; i < RANK_COPIES * stride; i += 256) copies[i] = 0;
+        __syncthreads();
+#pragma unroll 4
+        for (int i = tid; i < n; i += 256) {
+            const int e = idx[i];
+            if ((unsigned)e < (unsigned)E) atomicAdd(&copies[lane % RANK_COPIES * stride + e], 1);
+        }
+        __syncthreads();
+        for (int e = tid; e < E; e += 256) {
+            int c = 0;
+#pragma unroll
+            for (int i = 0; i < RANK_COPIES; ++i) c += copies[i * stride + e];
+            tot[e] = c;
+        }
+        __syncthreads();
+        if (tid < WAVE) offsets_body(tot, E, W, es, true, out.send_counts, out.expert_offs, out.dst_sizes, out.dst_offsets, out.caps);
+        return;
+    }
+    if ((int)blockIdx.x <= side_blocks) {
+        recv_prepare_block(side, blockIdx.x - 1, es, tot);
+        return;
+    }
+    // f(keys of 8 x 64 slots: a lane's own; ids outside [0, E) and slots past the end above all others)
+    auto keys = [&](auto f) {
+        for (int i0 = 0; i0 < n; i0 += 8 * WAVE) {
+            unsigned key[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const int i = i0 + u * WAVE + lane;
+                const int e = i < n ? idx[i] : -1;
+                key[u] = (unsigned)e < (unsigned)E ? (unsigned)(e * n + i) : ~0u;
+            }
+            f(key);
+        }
+    };
+    const int n_slots = W * M, n_tok = T * parts, per = ((row_vec + parts - 1) / parts + WAVE - 1) / WAVE * WAVE;
+    const int n_units = n_tok + (n_slots + PACK_ZR - 1) / PACK_ZR, first = ((int)blockIdx.x - 1 - side_blocks) * 4 + tid / WAVE;
+    for (int unit = __builtin_amdgcn_readfirstlane(first); unit < n_units; unit += (gridDim.x - 1 - side_blocks) * 4) {
+        if (unit >= n_tok) {
+            const int s0 = (unit - n_tok) * PACK_ZR, s1 = min(s0 + PACK_ZR, n_slots);
+            int d = s0 / M, m = s0 % M;
+            auto size_of = [&](int q) {
+                int c = 0;
+                keys([&](const unsigned (&key)[8]) {
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) c += __popcll(__ballot(key[u] - (unsigned)(q * E_l * n) < (unsigned)(E_l * n)));
+                });
+                return c;
+            };
+            int cnt = size_of(d);
+            const u32x4 z = {0u, 0u, 0u, 0u};
+            for (int sl = s0; sl < s1; ++sl) {
+                if (m == 0 && cnt > M && status && lane == 0) *status = 1;
+                if (m >= cnt) {
+                    u32x4* o = send + (size_t)sl * row_vec;
+                    for (int c = lane; c < row_vec; c += WAVE) o[c] = z;
+                    if (send_gate && lane == 0) send_gate[sl] = 0.f;
+                }
+                if (++m == M && sl + 1 < s1) { m = 0; cnt = size_of(++d); }
+            }
+            continue;
+        }
+        const int r = unit / parts, c_lo = (unit % parts) * per, c_hi = min(c_lo + per, row_vec);
+        pack_row<KT>(x + (size_t)r * row_vec, send, k, row_vec, c_lo, c_hi, lane, [&](int (&drow)[KM]) {
+            int e[KM], p[KM] = {}, before[KM] = {};
+#pragma unroll
+            for (int j = 0; j < KM; ++j) e[j] = KT || j < k ? idx[r * k + j] : -1;
+            keys([&](const unsigned (&key)[8]) {
+#pragma unroll
+                for (int j = 0; j < KM; ++j) {
+                    if (KT || j < k) {
+                        const unsigned own = (unsigned)(e[j] * n + r * k), dst = (unsigned)(e[j] / E_l * E_l * n);
+#pragma unroll
+                        for (int u = 0; u < 8; ++u) {
+                            p[j] += __popcll(__ballot(key[u] < own));
+                            before[j] += __popcll(__ballot(key[u] < dst));
+                        }
+                    }
+                }
+            });
+#pragma unroll
+            for (int j = 0; j < KM; ++j) {
+                drow[j] = -1;
+                if ((KT || j < k) && (unsigned)e[j] < (unsigned)E) {
+                    const int m = p[j] - before[j];
+                    drow[j] = M == 0 ? p[j] : m < M ? e[j] / E_l * M + m : -1;
+                    if (c_lo == 0 && lane == 0) {
+                        out.pos[r * k + j] = p[j];
+                        out.row_token[p[j]] = r;
+                        if (send_gate && drow[j] >= 0) send_gate[drow[j]] = gate[r * k + j];
+                    }
+                }
+            }
+        });
+    }
+}
+
 // ---- combine: out[t,:] = sum_kk gate[t,kk] * ret[slot(t,kk),:] --------------------------------------
 template <typename XT>
 struct Vec16;
@@ -1115,6 +1234,11 @@ constexpr long long RANK_SUM_CELLS = 6ll << 20;
 // 10.5 / 9.0, 8192 x 4 of 512 11.6 / 8.6; but 8192 x 8 of 256 10.8 / 11.9, of 60 9.2 / 11.2, 16384 x 8 of 256 12.6 / 18.0.
 constexpr long long RANK_SELF_SLOTS = 32768;
 
+// Slots, and slots x top-k (the comparisons of a wave of count_pack_kernel), up to which a step's count goes with its pack.  A step of rows of 2 KB with
+// launches apart against together, us: 2048 x 1 of 8 41.7 / 40.1, 1024 x 2 of 8 43.9 / 42.4, 512 x 4 of 64 48.4 / 47.2, 128 x 8 of 256 52.4 / 51.2; but
+// 2048 x 2 of 8 44.9 / 50.3, of 64 57.2 / 61.0, 4096 x 1 of 256 83.3 / 86.9, 1024 x 4 of 64 57.6 / 59.2, 256 x 8 of 256 58.0 / 59.0.
+constexpr long long COUNT_PACK_SLOTS = 2048, COUNT_PACK_WORK = 8192;
+
 extern "C" size_t moe_count_workspace_bytes(int T, int k, int E) {
     (void)k;
     const size_t NB = (size_t)ceil_div(T > 0 ? T : 1, CB);
@@ -1433,6 +1557,30 @@ int moe_count_and_prepare(const moe_step_args* a, hipStream_t s) {
     if (rc) return rc;
     return count_and_offsets(a->idx, a->tokens, a->topk, a->experts, a->world, a->send_counts, a->expert_offs, a->dst_sizes, a->dst_offsets, a->caps,
                              a->pos, a->row_token, a->count_ws, a->count_ws_bytes, &side, blocks, s);
+}
+
+bool moe_count_with_pack(int T, int k) { return T > 0 && k >= 1 && k <= MOE_MAX_TOPK && (long long)T * k <= COUNT_PACK_SLOTS && (long long)T * k * k <= COUNT_PACK_WORK; }
+
+int moe_count_and_pack(const moe_step_args* a, bool prepare, hipStream_t s) {
+    const int T = a->tokens, k = a->topk, E = a->experts, W = a->world, E_l = E / W, M = a->flat ? 0 : a->M, row_vec = a->hidden * dtype_size(a->dtype) / 16;
+    const float* gate = a->gated ? a->gate : nullptr;
+    float* send_gate = a->gated ? a->send_gate : nullptr;
+    RecvPrepare side{};
+    int blocks = 0, rc = prepare ? step_recv_prepare(a, 256, &side, &blocks) : MOE_OK;
+    if (!rc)
+        rc = check_count(a->idx, T, k, E, W, a->send_counts, a->expert_offs, a->dst_sizes, a->dst_offsets, a->caps, a->pos, a->row_token, a->count_ws,
+                         a->count_ws_bytes);
+    if (!rc)
+        rc = a->flat ? check_pack_payload(a->x, a->dtype, T, a->hidden, a->row_token, T * k, a->send)
+                     : check_pack_tokens(a->x, a->dtype, T, a->hidden, a->idx, a->pos, gate, k, E_l, a->dst_sizes, a->dst_offsets, W, M, a->send, send_gate);
+    if (rc) return rc;
+    const int parts = row_parts(T, row_vec), units = T * parts + ceil_div(W * M, PACK_ZR);
+    const CountOut out = {a->send_counts, a->expert_offs, a->dst_sizes, a->dst_offsets, a->caps, a->pos, a->row_token};
+    with_topk(k, [&](auto kt) {
+        count_pack_kernel<decltype(kt)::value><<<1 + blocks + min(ceil_div(units, 4), 65535 * 8), 256, RANK_COPIES * (size_t)(E | 1) * sizeof(int32_t), s>>>(
+            (const u32x4*)a->x, (u32x4*)a->send, a->idx, T, k, E, W, M, row_vec, out, a->status, gate, send_gate, parts, blocks, side);
+    });
+    return moe_check_launch("count_and_pack");
 }
 
 extern "C" int moe_recv_row_map(const int32_t* recv_counts, int W, int E_l, int M, int n_rows, int32_t* row_map,

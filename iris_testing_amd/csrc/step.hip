@@ -51,10 +51,19 @@ static bool f32_apart(const moe_step_args* a) {
     return own_writes({recv, sent, w1, up}, {rows, counts, hidden}) && own_writes({hidden, counts, sent, w2}, {y, ret});
 }
 
+// True if the count may share a launch with the pack, which then does not read what the count leaves: nothing that the two write is read by
+// either or written twice.
+static bool count_pack_apart(const moe_step_args* a) {
+    const size_t T = a->tokens, H = a->hidden, E = a->experts, W = a->world, R = T * a->topk, n = W * (size_t)a->M, row = H * (a->dtype == MOE_BF16 ? 2 : 4);
+    return own_writes({{a->x, T * row}, {a->idx, R * 4}, {a->gated ? a->gate : nullptr, R * 4}},
+                      {{a->send_counts, E * 4}, {a->expert_offs, E * 4}, {a->dst_sizes, W * 4}, {a->dst_offsets, W * 4}, {a->caps, 8}, {a->pos, R * 4},
+                       {a->row_token, R * 4}, {a->send, (a->flat ? R : n) * row}, {a->gated ? a->send_gate : nullptr, n * 4}, {a->status, 4}});
+}
+
 // How a step goes: the receive side prepared in the launch that ranks the tokens; the rows of fp32 experts moved by their GEMMs (plumbing:
-// 42.9 -> 38 us a step).
+// 42.9 -> 38 us a step); the tokens ranked by the pack.
 struct StepPlan {
-    bool together, f32_slots;
+    bool together, f32_slots, count_pack;
 };
 static int step_plan(const moe_step_args* a, StepPlan* plan) {
     MOE_REQUIRE(a, MOE_ERR_INVALID, "step: null arguments");
@@ -64,6 +73,7 @@ static int step_plan(const moe_step_args* a, StepPlan* plan) {
     MOE_REQUIRE(!(a->flat && a->gated), MOE_ERR_INVALID, "step: flat and gated are separate modes");
     plan->together = a->fused && sides_apart(a);
     plan->f32_slots = a->f32_weights && !a->fused && !a->quant && a->dtype == MOE_F32 && a->S > 0 && f32_apart(a);
+    plan->count_pack = !a->q_dispatch && moe_count_with_pack(a->tokens, a->topk) && count_pack_apart(a);
     return MOE_OK;
 }
 
@@ -94,12 +104,15 @@ extern "C" int moe_step(const moe_step_args* a, moe_stream_t stream) {
     } while (0)
     MOE_STAGE(moe_route_topk(a->x, a->router, a->bias, a->dtype, T, H, E, k, a->logits, a->idx, a->gate, a->route_ws, a->route_ws_bytes,
                              stream));
-    if (plan.together)
+    if (plan.count_pack)
+        MOE_STAGE(moe_count_and_pack(a, plan.together, (hipStream_t)stream));
+    else if (plan.together)
         MOE_STAGE(moe_count_and_prepare(a, (hipStream_t)stream));
     else
         MOE_STAGE(moe_count_and_offsets(a->idx, T, k, E, W, a->send_counts, a->expert_offs, a->dst_sizes, a->dst_offsets, a->caps, a->pos,
                                         a->row_token, a->count_ws, a->count_ws_bytes, stream));
-    if (a->q_dispatch)
+    if (plan.count_pack) {
+    } else if (a->q_dispatch)
         MOE_STAGE(moe_pack_tokens_fp8_gated(a->x, T, H, a->idx, a->pos, out_gate, k, E_l, a->dst_sizes, a->dst_offsets, W, M,
                                             (uint8_t*)a->send, a->send_scale, a->gated ? a->send_gate : nullptr, a->status, stream));
     else if (a->flat)
