@@ -636,6 +636,8 @@ inline int row_parts(int tokens, int row_vec) {
 // The combine's: also with many tokens, so that the rows of fewer tokens are read at a time -- with a row to a wave 4096 x 8 rows of 14 KB
 // are 32768 places in memory at once.  Runs of 2 KB at least and at most four to a row (k = 8: 4096 x 14 KB 104 -> 97 us, 5.5 TB/s;
 // 8192 x 4 KB 61 -> 57; k = 2: 8192 x 8 KB 41 -> 36; eight runs 55 where four take 51 and one 54, runs of 1 KB 20 where one takes 17).
+// The pack's too (2048 x 14 KB, top-4 43.8 -> 39.1 us, 3000 x 10 KB, top-2 23.4 -> 22.3, 2500 x 14 KB, top-8 78 -> 74; 4096 x 14 KB, top-8 127 -> 129 by
+// itself, between the router and the combine 2 us quicker).
 inline int combine_parts(int tokens, int row_vec) {
     return tokens < 2048 ? row_parts(tokens, row_vec) : max(1, min(min(16384 / tokens, row_vec / (2 * WAVE)), 4));
 }
@@ -1420,7 +1422,7 @@ extern "C" int moe_pack_tokens_gated(const void* x, int dtype, int T, int H, con
                                      int M, void* send_buf, float* send_gate, int32_t* status, moe_stream_t stream) {
     const int rc = check_pack_tokens(x, dtype, T, H, topk_idx, pos, gate, k, E_l, dst_sizes, dst_offsets, W, M, send_buf, send_gate);
     if (rc) return rc;
-    const int parts = row_parts(T, H * dtype_size(dtype) / 16);
+    const int row_vec = H * dtype_size(dtype) / 16, parts = combine_parts(T, row_vec);
     const int n_units = T * parts + ceil_div(W * M, PACK_ZR);
     const int blocks = min(ceil_div(n_units, 4), 65535 * 8);
     with_topk(k, [&](auto kt) {
