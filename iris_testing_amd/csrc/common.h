@@ -17,7 +17,7 @@ int moe_check_launch(const char* what);
 
 // dispatch.hip, for step.hip: moe_count_and_offsets and moe_recv_prepare with one launch less
 int moe_count_and_prepare(const moe_step_args* a, hipStream_t s);
-// ... and where moe_count_with_pack says so, the count (with prepare: both) and the bf16 or fp32 pack in one
+// ... and where moe_count_with_pack says so, the count (with prepare: both) and the pack in one
 bool moe_count_with_pack(int T, int k);
 int moe_count_and_pack(const moe_step_args* a, bool prepare, hipStream_t s);
 // grouped_gemm.hip, for step.hip: moe_unpack_expert_major of fp32 rows, moe_grouped_mlp and moe_return_pack, in two launches where tiles are small (S_rows > 0)
@@ -118,3 +118,29 @@ static inline void with_topk(int k, F&& f) {
 }
 template <int KT>
 constexpr int topk_slots() { return KT ? KT : MOE_MAX_TOPK; }
+
+// ---- bf16 rows as e4m3 codes and a scale per row: largest magnitude, codes of eight values -----
+__device__ __forceinline__ float fp8_row_amax(const uint4& v, float amax) {
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        amax = fmaxf(amax, fabsf(__uint_as_float(w[i] << 16)));
+        amax = fmaxf(amax, fabsf(__uint_as_float(w[i] & 0xffff0000u)));
+    }
+    return amax;
+}
+__device__ __forceinline__ uint2 fp8_row_convert(const uint4& v, float inv) {
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+    float f[8];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        f[2 * i] = __fmul_rn(__uint_as_float(w[i] << 16), inv);
+        f[2 * i + 1] = __fmul_rn(__uint_as_float(w[i] & 0xffff0000u), inv);
+    }
+    int lo = 0, hi = 0;
+    lo = __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], lo, false);
+    lo = __builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], lo, true);
+    hi = __builtin_amdgcn_cvt_pk_fp8_f32(f[4], f[5], hi, false);
+    hi = __builtin_amdgcn_cvt_pk_fp8_f32(f[6], f[7], hi, true);
+    return make_uint2((uint32_t)lo, (uint32_t)hi);
+}

@@ -722,6 +722,113 @@ __global__ __launch_bounds__(WPB * WAVE) void pack_tokens_kernel(const u32x4* __
     }
 }
 
+// ---- quantise and pack in one pass: the token rows leave the source as fp8 codes and one scale per row -----------------
+// Per-row quantisation commutes with moving rows: send_q / send_scale hold, slot for slot, what quantize_rows_fp8 would make
+// of the bf16 send buffer (padding slots: codes 0, scale 1, as for an all-zero row) -- so the destination can feed them to
+// the fp8 GEMM as they arrive, and half the bytes cross.  Units [0, T) of the launch are tokens (one wave each: the row is
+// read once, quantised in registers, stored to its k slots); the units after them are runs of PACK_ZR slots that are
+// written only where they are padding.
+// A token: its row of nv 16-byte vectors, asked for before its slots are looked up (NV to a lane in registers; 0: read twice), a form for each usual
+// top-k (see pack_row): 3500 x 4 KB, top-8 22.7 -> 19.7 us, 3000 x 10 KB, top-2 22.0 -> 19.0, 16384 x 2 KB, top-8 44 -> 40; 4096 x 8 KB, top-4 27.7 -> 28.6.
+template <int KT, int NV, typename F>
+__device__ __forceinline__ void pack_row_fp8(const uint4* __restrict__ src, uint8_t* __restrict__ send_q, float* __restrict__ send_scale, int k, int nv,
+                                             int lane, F&& slots) {
+    constexpr int KM = topk_slots<KT>();
+    const size_t cols = (size_t)nv * 8;
+    uint4 held[NV > 0 ? NV : 1];
+    float amax = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const int c = lane + i * WAVE;
+        held[i] = c < nv ? src[c] : make_uint4(0, 0, 0, 0);
+    }
+    int drow[KM];
+    slots(drow);
+    if constexpr (NV > 0) {
+#pragma unroll
+        for (int i = 0; i < NV; ++i) amax = fp8_row_amax(held[i], amax);
+    } else {
+        for (int c = lane; c < nv; c += WAVE) amax = fp8_row_amax(src[c], amax);
+    }
+    amax = __int_as_float(wave_max0(__float_as_int(amax)));  // (never NaN, never below 0: the bits are ordered alike)
+    const bool zero = amax == 0.f;
+    const float inv = zero ? 1.f : __fdiv_rn(448.f, amax);
+    const float sc = zero ? 1.f : __fdiv_rn(amax, 448.f);
+    if constexpr (NV > 0) {
+        uint2 code[NV];
+#pragma unroll
+        for (int i = 0; i < NV; ++i) code[i] = fp8_row_convert(held[i], inv);
+#pragma unroll
+        for (int j = 0; j < KM; ++j) {
+            if ((KT || j < k) && drow[j] >= 0) {
+                uint2* o = (uint2*)(send_q + (size_t)drow[j] * cols);
+#pragma unroll
+                for (int i = 0; i < NV; ++i) {
+                    const int c = lane + i * WAVE;
+                    if (c < nv) o[c] = code[i];
+                }
+                if (lane == 0) send_scale[drow[j]] = sc;
+            }
+        }
+    } else {
+        for (int c = lane; c < nv; c += WAVE) {
+            const uint2 code = fp8_row_convert(src[c], inv);
+#pragma unroll
+            for (int j = 0; j < KM; ++j)
+                if ((KT || j < k) && drow[j] >= 0) ((uint2*)(send_q + (size_t)drow[j] * cols))[c] = code;
+        }
+#pragma unroll
+        for (int j = 0; j < KM; ++j)
+            if ((KT || j < k) && drow[j] >= 0 && lane == 0) send_scale[drow[j]] = sc;
+    }
+}
+template <int KT, int NV>
+__global__ __launch_bounds__(256) void pack_tokens_fp8_kernel(const bf16_t* __restrict__ x, int T, int cols,
+                                                               const int32_t* __restrict__ idx, const int32_t* __restrict__ pos,
+                                                               const int32_t* __restrict__ dst_sizes,
+                                                               const int32_t* __restrict__ dst_offsets, int k_rt, int E_l, int W, int M,
+                                                               uint8_t* __restrict__ send_q, float* __restrict__ send_scale,
+                                                               int32_t* __restrict__ status, const float* __restrict__ gate,
+                                                               float* __restrict__ send_gate) {
+    // (gate / send_gate, both or neither: the slot's top-k gate travels with its row, zero in the padding slots)
+    constexpr int KM = topk_slots<KT>();
+    const int wave = threadIdx.x / WAVE, lane = lane_id(), k = KT ? KT : k_rt;
+    const int nv = cols / 8;  // 16-byte vectors of bf16 per row = 8-byte vectors of codes
+    const int n_slots = W * M;
+    const int n_units = T + (n_slots + PACK_ZR - 1) / PACK_ZR;
+    for (int r = blockIdx.x * 4 + wave; r < n_units; r += gridDim.x * 4) {
+        if (r >= T) {
+            const int s0 = (r - T) * PACK_ZR, s1 = min(s0 + PACK_ZR, n_slots);
+            int d = s0 / M, m = s0 % M;
+            int cnt = dst_sizes[d];
+            for (int sl = s0; sl < s1; ++sl) {
+                if (m == 0 && cnt > M && status && lane == 0) *status = 1;
+                if (m >= cnt) {
+                    uint2* o = (uint2*)(send_q + (size_t)sl * cols);
+                    for (int c = lane; c < nv; c += WAVE) o[c] = make_uint2(0u, 0u);
+                    if (lane == 0) send_scale[sl] = 1.f;
+                    if (send_gate && lane == 0) send_gate[sl] = 0.f;
+                }
+                if (++m == M && sl + 1 < s1) { m = 0; cnt = dst_sizes[++d]; }
+            }
+            continue;
+        }
+        pack_row_fp8<KT, NV>((const uint4*)(x + (size_t)r * cols), send_q, send_scale, k, nv, lane, [&](int (&drow)[KM]) {
+#pragma unroll
+            for (int j = 0; j < KM; ++j) {
+                drow[j] = -1;
+                if (KT || j < k) {
+                    const int d = idx[(size_t)r * k + j] / E_l;
+                    const bool d_ok = (unsigned)d < (unsigned)W;
+                    const int m = pos[(size_t)r * k + j] - dst_offsets[d_ok ? d : 0];
+                    if (d_ok && (unsigned)m < (unsigned)M) drow[j] = d * M + m;
+                    if (send_gate && drow[j] >= 0 && lane == 0) send_gate[drow[j]] = gate[(size_t)r * k + j];
+                }
+            }
+        });
+    }
+}
+
 // Count and pack of few tokens in one launch: every wave works out for itself where its token's rows go, from the expert ids of all slots (a few
 // KB, from L2), so nothing has to wait for a ranking in front.  The row of a slot is the slots of lower experts plus those of its own in earlier
 // tokens; with key = expert * T k + slot (a token holds an expert at most once) that is the number of smaller keys, and the keys below the first of
@@ -729,12 +836,12 @@ __global__ __launch_bounds__(WPB * WAVE) void pack_tokens_kernel(const u32x4* __
 // Block 0 counts the experts and leaves the tables; blocks 1 to side_blocks prepare the receive side (see rank_kernel); the others are the
 // units of pack_tokens_kernel, whose bytes these are.  M = 0: the padding-free payload, row = position.
 // What it saves is the ranking's launch, most of whose time is its start and a chain of small steps.  A step of 256 fp32 tokens x 1 KB, top-2, 34.7 -> 31.8 us;
-// 512 x 4 KB, top-1, 66.6 -> 63.8; 24 x 14 KB, top-8, 352 -> 349; 777 x 4 KB, top-2, flat, 111.5 -> 106.8.
+// 512 x 4 KB, top-1, 66.6 -> 63.8; 24 x 14 KB, top-8, 352 -> 349; 777 x 4 KB, top-2, flat, 111.5 -> 106.8; quantised, 64 x 4 KB, top-2 of 64, 36.9 -> 33.5.
 struct CountOut {
     int32_t *send_counts, *expert_offs, *dst_sizes, *dst_offsets, *caps, *pos, *row_token;
 };
-template <int KT>
-__global__ __launch_bounds__(256) void count_pack_kernel(const u32x4* __restrict__ x, u32x4* __restrict__ send, const int32_t* __restrict__ idx, int T, int k_rt,
+template <int KT, int NV /* -1: the rows as they are, 16-byte vectors; else quantised (pack_row_fp8), 8-byte vectors of codes */>
+__global__ __launch_bounds__(256) void count_pack_kernel(const u32x4* __restrict__ x, void* __restrict__ send, float* __restrict__ send_scale, const int32_t* __restrict__ idx, int T, int k_rt,
                                                           int E, int W, int M, int row_vec, const CountOut out, int32_t* __restrict__ status,
                                                           const float* __restrict__ gate, float* __restrict__ send_gate, int parts, int side_blocks,
                                                           const RecvPrepare side) {
@@ -794,12 +901,14 @@ __global__ __launch_bounds__(256) void count_pack_kernel(const u32x4* __restrict
                 return c;
             };
             int cnt = size_of(d);
-            const u32x4 z = {0u, 0u, 0u, 0u};
+            typedef typename std::conditional<(NV < 0), u32x4, uint2>::type vec;
+            const vec z = {};
             for (int sl = s0; sl < s1; ++sl) {
                 if (m == 0 && cnt > M && status && lane == 0) *status = 1;
                 if (m >= cnt) {
-                    u32x4* o = send + (size_t)sl * row_vec;
+                    vec* o = (vec*)send + (size_t)sl * row_vec;
                     for (int c = lane; c < row_vec; c += WAVE) o[c] = z;
+                    if (NV >= 0 && lane == 0) send_scale[sl] = 1.f;
                     if (send_gate && lane == 0) send_gate[sl] = 0.f;
                 }
                 if (++m == M && sl + 1 < s1) { m = 0; cnt = size_of(++d); }
@@ -807,7 +916,7 @@ __global__ __launch_bounds__(256) void count_pack_kernel(const u32x4* __restrict
             continue;
         }
         const int r = unit / parts, c_lo = (unit % parts) * per, c_hi = min(c_lo + per, row_vec);
-        pack_row<KT>(x + (size_t)r * row_vec, send, k, row_vec, c_lo, c_hi, lane, [&](int (&drow)[KM]) {
+        auto slots = [&](int (&drow)[KM]) {
             int e[KM], p[KM] = {}, before[KM] = {};
 #pragma unroll
             for (int j = 0; j < KM; ++j) e[j] = KT || j < k ? idx[r * k + j] : -1;
@@ -837,7 +946,9 @@ __global__ __launch_bounds__(256) void count_pack_kernel(const u32x4* __restrict
                     }
                 }
             }
-        });
+        };
+        if constexpr (NV < 0) pack_row<KT>(x + (size_t)r * row_vec, (u32x4*)send, k, row_vec, c_lo, c_hi, lane, slots);
+        else pack_row_fp8<KT, NV>((const uint4*)x + (size_t)r * row_vec, (uint8_t*)send, send_scale, k, row_vec, lane, slots);
     }
 }
 
@@ -1439,6 +1550,54 @@ extern "C" int moe_pack_tokens(const void* x, int dtype, int T, int H, const int
                                  status, stream);
 }
 
+// f(16-byte vectors of a row of H bf16 values to a lane, 0: too many for the registers)
+template <typename F>
+static void with_row_vectors(int H, F&& f) {
+    const int nv = ceil_div(H / 8, WAVE);
+    if (nv <= 2) f(std::integral_constant<int, 2>{});
+    else if (nv <= 4) f(std::integral_constant<int, 4>{});
+    else if (nv <= 8) f(std::integral_constant<int, 8>{});
+    else if (nv <= 16) f(std::integral_constant<int, 16>{});
+    else f(std::integral_constant<int, 0>{});
+}
+
+static int check_pack_tokens_fp8(const void* x_bf16, int T, int H, const int32_t* topk_idx, const int32_t* pos, const float* gate, int k, int E_l,
+                                 const int32_t* dst_sizes, const int32_t* dst_offsets, int W, int M, const void* send_q, const float* send_scale,
+                                 const float* send_gate) {
+    MOE_REQUIRE((gate == nullptr) == (send_gate == nullptr), MOE_ERR_INVALID, "pack_tokens_fp8: gate and send_gate go together");
+    MOE_REQUIRE(T >= 0 && H > 0 && H % 8 == 0 && W > 0 && M >= 1 && E_l > 0, MOE_ERR_INVALID, "pack_tokens_fp8: bad shape");
+    MOE_REQUIRE(k >= 1 && k <= MOE_MAX_TOPK, MOE_ERR_UNSUPPORTED, "pack_tokens_fp8: topk=%d outside [1,%d]", k, MOE_MAX_TOPK);
+    MOE_REQUIRE((long long)W * M + T < (1ll << 31), MOE_ERR_UNSUPPORTED, "pack_tokens_fp8: W*M + T too large");
+    MOE_REQUIRE(send_q && send_scale && dst_sizes && dst_offsets, MOE_ERR_INVALID, "pack_tokens_fp8: null pointer");
+    MOE_REQUIRE(T == 0 || (x_bf16 && topk_idx && pos), MOE_ERR_INVALID, "pack_tokens_fp8: null pointer");
+    return MOE_OK;
+}
+
+extern "C" int moe_pack_tokens_fp8(const void* x_bf16, int T, int H, const int32_t* topk_idx, const int32_t* pos, int k, int E_l,
+                                   const int32_t* dst_sizes, const int32_t* dst_offsets, int W, int M, uint8_t* send_q,
+                                   float* send_scale, int32_t* status, moe_stream_t stream) {
+    return moe_pack_tokens_fp8_gated(x_bf16, T, H, topk_idx, pos, nullptr, k, E_l, dst_sizes, dst_offsets, W, M, send_q, send_scale,
+                                     nullptr, status, stream);
+}
+
+extern "C" int moe_pack_tokens_fp8_gated(const void* x_bf16, int T, int H, const int32_t* topk_idx, const int32_t* pos,
+                                         const float* gate, int k, int E_l, const int32_t* dst_sizes, const int32_t* dst_offsets,
+                                         int W, int M, uint8_t* send_q, float* send_scale, float* send_gate, int32_t* status,
+                                         moe_stream_t stream) {
+    const int rc = check_pack_tokens_fp8(x_bf16, T, H, topk_idx, pos, gate, k, E_l, dst_sizes, dst_offsets, W, M, send_q, send_scale, send_gate);
+    if (rc) return rc;
+    const int n_units = T + ceil_div(W * M, PACK_ZR);
+    const int blocks = min(ceil_div(n_units, 4), 65535 * 8);
+    hipStream_t s = (hipStream_t)stream;
+    with_topk(k, [&](auto kt) {
+        with_row_vectors(H, [&](auto nv) {
+            pack_tokens_fp8_kernel<decltype(kt)::value, decltype(nv)::value><<<blocks, 256, 0, s>>>(
+                (const bf16_t*)x_bf16, T, H, topk_idx, pos, dst_sizes, dst_offsets, k, E_l, W, M, send_q, send_scale, status, gate, send_gate);
+        });
+    });
+    return moe_check_launch("pack_tokens_fp8");
+}
+
 static int recv_driven(const char* who, int mode, const void* src, void* dst, int dtype, int H, const RecvCounts& q, int W, int E_l, int M,
                        int CAP, int n_out, int32_t* status, hipStream_t s) {
     int rc = check_rows(who, dtype, H);
@@ -1564,7 +1723,7 @@ int moe_count_and_prepare(const moe_step_args* a, hipStream_t s) {
 bool moe_count_with_pack(int T, int k) { return T > 0 && k >= 1 && k <= MOE_MAX_TOPK && (long long)T * k <= COUNT_PACK_SLOTS && (long long)T * k * k <= COUNT_PACK_WORK; }
 
 int moe_count_and_pack(const moe_step_args* a, bool prepare, hipStream_t s) {
-    const int T = a->tokens, k = a->topk, E = a->experts, W = a->world, E_l = E / W, M = a->flat ? 0 : a->M, row_vec = a->hidden * dtype_size(a->dtype) / 16;
+    const int T = a->tokens, k = a->topk, E = a->experts, W = a->world, E_l = E / W, H = a->hidden, M = a->flat ? 0 : a->M;
     const float* gate = a->gated ? a->gate : nullptr;
     float* send_gate = a->gated ? a->send_gate : nullptr;
     RecvPrepare side{};
@@ -1573,14 +1732,21 @@ int moe_count_and_pack(const moe_step_args* a, bool prepare, hipStream_t s) {
         rc = check_count(a->idx, T, k, E, W, a->send_counts, a->expert_offs, a->dst_sizes, a->dst_offsets, a->caps, a->pos, a->row_token, a->count_ws,
                          a->count_ws_bytes);
     if (!rc)
-        rc = a->flat ? check_pack_payload(a->x, a->dtype, T, a->hidden, a->row_token, T * k, a->send)
-                     : check_pack_tokens(a->x, a->dtype, T, a->hidden, a->idx, a->pos, gate, k, E_l, a->dst_sizes, a->dst_offsets, W, M, a->send, send_gate);
+        rc = a->flat ? check_pack_payload(a->x, a->dtype, T, H, a->row_token, T * k, a->send)
+             : a->q_dispatch
+                 ? check_pack_tokens_fp8(a->x, T, H, a->idx, a->pos, gate, k, E_l, a->dst_sizes, a->dst_offsets, W, M, a->send, a->send_scale, send_gate)
+                 : check_pack_tokens(a->x, a->dtype, T, H, a->idx, a->pos, gate, k, E_l, a->dst_sizes, a->dst_offsets, W, M, a->send, send_gate);
     if (rc) return rc;
-    const int parts = row_parts(T, row_vec), units = T * parts + ceil_div(W * M, PACK_ZR);
     const CountOut out = {a->send_counts, a->expert_offs, a->dst_sizes, a->dst_offsets, a->caps, a->pos, a->row_token};
+    auto launch = [&](auto kt, auto nv, int row_vec, int parts) {
+        const int units = T * parts + ceil_div(W * M, PACK_ZR), grid = 1 + blocks + min(ceil_div(units, 4), 65535 * 8);
+        count_pack_kernel<decltype(kt)::value, decltype(nv)::value><<<grid, 256, RANK_COPIES * (size_t)(E | 1) * sizeof(int32_t), s>>>(
+            (const u32x4*)a->x, a->send, a->send_scale, a->idx, T, k, E, W, M, row_vec, out, a->status, gate, send_gate, parts, blocks, side);
+    };
     with_topk(k, [&](auto kt) {
-        count_pack_kernel<decltype(kt)::value><<<1 + blocks + min(ceil_div(units, 4), 65535 * 8), 256, RANK_COPIES * (size_t)(E | 1) * sizeof(int32_t), s>>>(
-            (const u32x4*)a->x, (u32x4*)a->send, a->idx, T, k, E, W, M, row_vec, out, a->status, gate, send_gate, parts, blocks, side);
+        const int row_vec = H * dtype_size(a->dtype) / 16;
+        if (a->q_dispatch) with_row_vectors(H, [&](auto nv) { launch(kt, nv, H / 8, 1); });
+        else launch(kt, std::integral_constant<int, -1>{}, row_vec, row_parts(T, row_vec));
     });
     return moe_check_launch("count_and_pack");
 }

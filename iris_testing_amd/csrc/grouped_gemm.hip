@@ -1302,31 +1302,6 @@ __global__ __launch_bounds__(256 * KG) void grouped_gemm_f32_kernel(const float*
 // ---- per-row fp8 quantisation of bf16 rows (one wave per row) -------------------------------------
 // Rows of up to 64 * NV * 8 columns are held in registers between the amax pass and the conversion, so
 // they are read from memory once; longer rows are read twice.
-__device__ __forceinline__ float fp8_row_amax(const uint4& v, float amax) {
-    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        amax = fmaxf(amax, fabsf(__uint_as_float(w[i] << 16)));
-        amax = fmaxf(amax, fabsf(__uint_as_float(w[i] & 0xffff0000u)));
-    }
-    return amax;
-}
-__device__ __forceinline__ uint2 fp8_row_convert(const uint4& v, float inv) {
-    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-    float f[8];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        f[2 * i] = __fmul_rn(__uint_as_float(w[i] << 16), inv);
-        f[2 * i + 1] = __fmul_rn(__uint_as_float(w[i] & 0xffff0000u), inv);
-    }
-    int lo = 0, hi = 0;
-    lo = __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], lo, false);
-    lo = __builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], lo, true);
-    hi = __builtin_amdgcn_cvt_pk_fp8_f32(f[4], f[5], hi, false);
-    hi = __builtin_amdgcn_cvt_pk_fp8_f32(f[6], f[7], hi, true);
-    return make_uint2((uint32_t)lo, (uint32_t)hi);
-}
-
 template <int NV>  // 16-byte vectors per lane kept in registers (0: stream the row twice)
 __global__ __launch_bounds__(256) void quantize_rows_fp8_kernel(const bf16_t* __restrict__ x, int rows, int cols,
                                                                  uint8_t* __restrict__ q, float* __restrict__ scale,
@@ -1363,103 +1338,6 @@ __global__ __launch_bounds__(256) void quantize_rows_fp8_kernel(const bf16_t* __
             }
         } else {
             for (int c = lane; c < nv; c += WAVE) dst[c] = fp8_row_convert(src[c], inv);
-        }
-    }
-}
-
-// ---- quantise and pack in one pass: the token rows leave the source as fp8 codes and one scale per row -----------------
-// Per-row quantisation commutes with moving rows: send_q / send_scale hold, slot for slot, what quantize_rows_fp8 would make
-// of the bf16 send buffer (padding slots: codes 0, scale 1, as for an all-zero row) -- so the destination can feed them to
-// the fp8 GEMM as they arrive, and half the bytes cross.  Units [0, T) of the launch are tokens (one wave each: the row is
-// read once, quantised in registers, stored to its k slots); the units after them are runs of PACKQ_ZR slots that are
-// written only where they are padding.
-constexpr int PACKQ_ZR = 8;
-template <int NV>
-__global__ __launch_bounds__(256) void pack_tokens_fp8_kernel(const bf16_t* __restrict__ x, int T, int cols,
-                                                               const int32_t* __restrict__ idx, const int32_t* __restrict__ pos,
-                                                               const int32_t* __restrict__ dst_sizes,
-                                                               const int32_t* __restrict__ dst_offsets, int k, int E_l, int W, int M,
-                                                               uint8_t* __restrict__ send_q, float* __restrict__ send_scale,
-                                                               int32_t* __restrict__ status, const float* __restrict__ gate,
-                                                               float* __restrict__ send_gate) {
-    // (gate / send_gate, both or neither: the slot's top-k gate travels with its row, zero in the padding slots)
-    const int wave = threadIdx.x / WAVE, lane = lane_id();
-    const int nv = cols / 8;  // 16-byte vectors of bf16 per row = 8-byte vectors of codes
-    const int n_slots = W * M;
-    const int n_units = T + (n_slots + PACKQ_ZR - 1) / PACKQ_ZR;
-    for (int r = blockIdx.x * 4 + wave; r < n_units; r += gridDim.x * 4) {
-        if (r >= T) {
-            const int s0 = (r - T) * PACKQ_ZR, s1 = min(s0 + PACKQ_ZR, n_slots);
-            int d = s0 / M, m = s0 % M;
-            int cnt = dst_sizes[d];
-            for (int sl = s0; sl < s1; ++sl) {
-                if (m == 0 && cnt > M && status && lane == 0) *status = 1;
-                if (m >= cnt) {
-                    uint2* o = (uint2*)(send_q + (size_t)sl * cols);
-                    for (int c = lane; c < nv; c += WAVE) o[c] = make_uint2(0u, 0u);
-                    if (lane == 0) send_scale[sl] = 1.f;
-                    if (send_gate && lane == 0) send_gate[sl] = 0.f;
-                }
-                if (++m == M && sl + 1 < s1) { m = 0; cnt = dst_sizes[++d]; }
-            }
-            continue;
-        }
-        int drow[MOE_MAX_TOPK];
-#pragma unroll
-        for (int j = 0; j < MOE_MAX_TOPK; ++j) {
-            drow[j] = -1;
-            if (j < k) {
-                const int d = idx[(size_t)r * k + j] / E_l;
-                const bool d_ok = (unsigned)d < (unsigned)W;
-                const int m = pos[(size_t)r * k + j] - dst_offsets[d_ok ? d : 0];
-                if (d_ok && (unsigned)m < (unsigned)M) drow[j] = d * M + m;
-                if (send_gate && drow[j] >= 0 && lane == 0) send_gate[drow[j]] = gate[(size_t)r * k + j];
-            }
-        }
-        const uint4* src = (const uint4*)(x + (size_t)r * cols);
-        uint4 held[NV > 0 ? NV : 1];
-        float amax = 0.f;
-        if constexpr (NV > 0) {
-#pragma unroll
-            for (int i = 0; i < NV; ++i) {
-                const int c = lane + i * WAVE;
-                held[i] = c < nv ? src[c] : make_uint4(0, 0, 0, 0);
-            }
-#pragma unroll
-            for (int i = 0; i < NV; ++i) amax = fp8_row_amax(held[i], amax);
-        } else {
-            for (int c = lane; c < nv; c += WAVE) amax = fp8_row_amax(src[c], amax);
-        }
-        amax = __int_as_float(wave_max0(__float_as_int(amax)));  // (never NaN, never below 0: the bits are ordered alike)
-        const bool zero = amax == 0.f;
-        const float inv = zero ? 1.f : __fdiv_rn(448.f, amax);
-        const float sc = zero ? 1.f : __fdiv_rn(amax, 448.f);
-        if constexpr (NV > 0) {
-            uint2 code[NV];
-#pragma unroll
-            for (int i = 0; i < NV; ++i) code[i] = fp8_row_convert(held[i], inv);
-#pragma unroll
-            for (int j = 0; j < MOE_MAX_TOPK; ++j) {
-                if (j < k && drow[j] >= 0) {
-                    uint2* o = (uint2*)(send_q + (size_t)drow[j] * cols);
-#pragma unroll
-                    for (int i = 0; i < NV; ++i) {
-                        const int c = lane + i * WAVE;
-                        if (c < nv) o[c] = code[i];
-                    }
-                    if (lane == 0) send_scale[drow[j]] = sc;
-                }
-            }
-        } else {
-            for (int c = lane; c < nv; c += WAVE) {
-                const uint2 code = fp8_row_convert(src[c], inv);
-#pragma unroll
-                for (int j = 0; j < MOE_MAX_TOPK; ++j)
-                    if (j < k && drow[j] >= 0) ((uint2*)(send_q + (size_t)drow[j] * cols))[c] = code;
-            }
-#pragma unroll
-            for (int j = 0; j < MOE_MAX_TOPK; ++j)
-                if (j < k && drow[j] >= 0 && lane == 0) send_scale[drow[j]] = sc;
         }
     }
 }
@@ -2194,37 +2072,6 @@ extern "C" int moe_grouped_mlp_fp8(const void* tokens_bf16, const int32_t* exper
                                    moe_stream_t stream) {
     return moe_grouped_mlp_fp8_mapped(tokens_bf16, S_rows, nullptr, expert_cnt, S_rows, H, F, E_l, wgu_packed, sg, su, wd_packed,
                                       sd, xq_ws, xs_ws, hq_ws, hscale_ws, nullptr, out, S_rows, nullptr, nullptr, 0, stream);
-}
-
-extern "C" int moe_pack_tokens_fp8(const void* x_bf16, int T, int H, const int32_t* topk_idx, const int32_t* pos, int k, int E_l,
-                                   const int32_t* dst_sizes, const int32_t* dst_offsets, int W, int M, uint8_t* send_q,
-                                   float* send_scale, int32_t* status, moe_stream_t stream) {
-    return moe_pack_tokens_fp8_gated(x_bf16, T, H, topk_idx, pos, nullptr, k, E_l, dst_sizes, dst_offsets, W, M, send_q, send_scale,
-                                     nullptr, status, stream);
-}
-
-extern "C" int moe_pack_tokens_fp8_gated(const void* x_bf16, int T, int H, const int32_t* topk_idx, const int32_t* pos,
-                                         const float* gate, int k, int E_l, const int32_t* dst_sizes, const int32_t* dst_offsets,
-                                         int W, int M, uint8_t* send_q, float* send_scale, float* send_gate, int32_t* status,
-                                         moe_stream_t stream) {
-    MOE_REQUIRE((gate == nullptr) == (send_gate == nullptr), MOE_ERR_INVALID, "pack_tokens_fp8: gate and send_gate go together");
-    MOE_REQUIRE(T >= 0 && H > 0 && H % 8 == 0 && W > 0 && M >= 1 && E_l > 0, MOE_ERR_INVALID, "pack_tokens_fp8: bad shape");
-    MOE_REQUIRE(k >= 1 && k <= MOE_MAX_TOPK, MOE_ERR_UNSUPPORTED, "pack_tokens_fp8: topk=%d outside [1,%d]", k, MOE_MAX_TOPK);
-    MOE_REQUIRE((long long)W * M + T < (1ll << 31), MOE_ERR_UNSUPPORTED, "pack_tokens_fp8: W*M + T too large");
-    MOE_REQUIRE(send_q && send_scale && dst_sizes && dst_offsets, MOE_ERR_INVALID, "pack_tokens_fp8: null pointer");
-    MOE_REQUIRE(T == 0 || (x_bf16 && topk_idx && pos), MOE_ERR_INVALID, "pack_tokens_fp8: null pointer");
-    const int n_units = T + ceil_div(W * M, PACKQ_ZR);
-    const int blocks = min(ceil_div(n_units, 4), 65535 * 8);
-    const int nv = ceil_div(H / 8, WAVE);
-    hipStream_t s = (hipStream_t)stream;
-#define GG_PQ(NVv) pack_tokens_fp8_kernel<NVv><<<blocks, 256, 0, s>>>((const bf16_t*)x_bf16, T, H, topk_idx, pos, dst_sizes, dst_offsets, k, E_l, W, M, send_q, send_scale, status, gate, send_gate)
-    if (nv <= 2) GG_PQ(2);
-    else if (nv <= 4) GG_PQ(4);
-    else if (nv <= 8) GG_PQ(8);
-    else if (nv <= 16) GG_PQ(16);
-    else GG_PQ(0);
-#undef GG_PQ
-    return moe_check_launch("pack_tokens_fp8");
 }
 
 extern "C" int moe_grouped_mlp_fp8_q_mapped(const uint8_t* a_q, const float* a_scale, int a_rows, const int32_t* a_row_map,

@@ -55,9 +55,11 @@ static bool f32_apart(const moe_step_args* a) {
 // either or written twice.
 static bool count_pack_apart(const moe_step_args* a) {
     const size_t T = a->tokens, H = a->hidden, E = a->experts, W = a->world, R = T * a->topk, n = W * (size_t)a->M, row = H * (a->dtype == MOE_BF16 ? 2 : 4);
+    const size_t sent = a->flat ? R * row : n * (a->q_dispatch ? H : row);
     return own_writes({{a->x, T * row}, {a->idx, R * 4}, {a->gated ? a->gate : nullptr, R * 4}},
                       {{a->send_counts, E * 4}, {a->expert_offs, E * 4}, {a->dst_sizes, W * 4}, {a->dst_offsets, W * 4}, {a->caps, 8}, {a->pos, R * 4},
-                       {a->row_token, R * 4}, {a->send, (a->flat ? R : n) * row}, {a->gated ? a->send_gate : nullptr, n * 4}, {a->status, 4}});
+                       {a->row_token, R * 4}, {a->send, sent}, {a->q_dispatch ? a->send_scale : nullptr, n * 4}, {a->gated ? a->send_gate : nullptr, n * 4},
+                       {a->status, 4}});
 }
 
 // How a step goes: the receive side prepared in the launch that ranks the tokens; the rows of fp32 experts moved by their GEMMs (plumbing:
@@ -73,7 +75,7 @@ static int step_plan(const moe_step_args* a, StepPlan* plan) {
     MOE_REQUIRE(!(a->flat && a->gated), MOE_ERR_INVALID, "step: flat and gated are separate modes");
     plan->together = a->fused && sides_apart(a);
     plan->f32_slots = a->f32_weights && !a->fused && !a->quant && a->dtype == MOE_F32 && a->S > 0 && f32_apart(a);
-    plan->count_pack = !a->q_dispatch && moe_count_with_pack(a->tokens, a->topk) && count_pack_apart(a);
+    plan->count_pack = moe_count_with_pack(a->tokens, a->topk) && count_pack_apart(a);
     return MOE_OK;
 }
 

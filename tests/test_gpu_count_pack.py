@@ -12,7 +12,7 @@ from iris_testing_amd.configs import CONFIGS  # noqa: E402
 from iris_testing_amd.pipeline import DispatchPipeline  # noqa: E402
 
 DEV = "cuda"
-NAMES = ("logits idx gate send_counts expert_offs dst_sizes dst_offsets caps pos row_token send send_gate payload expert_cnt row_map row_gate rows "
+NAMES = ("logits idx gate send_counts expert_offs dst_sizes dst_offsets caps pos row_token send send_gate send_q send_scale payload expert_cnt row_map row_gate rows "
          "hidden y ret ret_flat out status").split()
 
 
@@ -51,6 +51,17 @@ def test_count_with_the_pack_equals_the_stages(tokens, topk, experts, world, slo
         assert torch.equal(one[n], stages[n]), f"{n} differs"
     if slots and mode != "flat":
         assert one["status"].item() == 1
+
+
+@pytest.mark.parametrize("tokens,topk,experts,world,hidden,mode", [(1, 1, 8, 8, 128, "fixed"), (33, 16, 64, 2, 1152, "fixed"), (100, 3, 27, 3, 2176, "gated"),
+                                                                   (128, 8, 64, 8, 4224, "gated"), (512, 4, 20, 5, 256, "fixed"), (513, 4, 20, 5, 256, "fixed"),
+                                                                   (1024, 2, 8, 2, 8320, "fixed"), (2048, 1, 12, 4, 128, "gated")])
+def test_count_with_the_quantising_pack_equals_the_stages(tokens, topk, experts, world, hidden, mode):
+    pipe = _pipe("zipf_k4", tokens, topk, experts, world, hidden=hidden, mode=mode)
+    assert pipe.fp8_dispatch
+    one, stages = _results(pipe, None), _results(pipe, [])
+    for n in one:
+        assert torch.equal(one[n], stages[n]), f"{n} differs"
 
 
 @pytest.mark.parametrize("tokens,topk", [(1, 2), (100, 5), (1024, 2), (1025, 2)])

@@ -38,3 +38,7 @@ def test_selection_and_pack_for_every_topk(T, H, E, W, dtype, k):
         keep = m < M
         want_gate[d[keep], m[keep]] = gate[keep]
         assert torch.equal(send_gate, want_gate)
+        if dtype == "bf16":
+            q, scale = ops.pack_tokens_fp8(x, idx, n.pos, n.dst_sizes, n.dst_offsets, E // W, M)[:2]
+            want_q, want_scale = ops.quantize_rows_fp8(want.view(W * M, H))
+            assert torch.equal(q.view(torch.uint8).view(W * M, H), want_q.view(torch.uint8)) and torch.equal(scale.view(-1), want_scale.view(-1))
