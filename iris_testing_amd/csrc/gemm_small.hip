@@ -51,11 +51,11 @@ struct GsParams {
 
 // How many parts every tile's K range is cut into.
 __host__ __device__ inline int gs_parts(long long tiles, int slots, int nk, int max_units) {
-    if (tiles <= 0) return 1;
-    const long long most = slots < max_units ? slots : max_units;
-    int P = (int)(most / tiles < GG_MAX_PARTS ? most / tiles : GG_MAX_PARTS);
+    const int most = slots < max_units ? slots : max_units;
+    if (tiles <= 0 || 2 * tiles > most) return 1;  // (nothing to divide: a launch of small tiles is short enough to see the division)
+    int P = most / (int)tiles < GG_MAX_PARTS ? most / (int)tiles : GG_MAX_PARTS;
     while (P > 1 && (gg_part_stages(nk, P) < GS_MIN_PART_STAGES || (P - 1) * gg_part_stages(nk, P) >= nk)) --P;
-    return P < 1 ? 1 : P;
+    return P;
 }
 
 template <int BM, bool FP8, int EPI, bool BSA, int BMODE, bool TAIL, int KG>
@@ -108,7 +108,9 @@ __global__ __launch_bounds__(GS_THREADS * KG, 2) void gemm_small_kernel(const Gs
     const int per = (units + 7) / 8;
     const int unit = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
     if (((int)blockIdx.x >> 3) >= per || unit >= units) return;
-    const int tile = unit / P, part = unit % P, whole = first + tile / subs;
+    int tile = unit, part = 0;
+    if (P > 1) { tile = unit / P; part = unit - tile * P; }
+    const int whole = first + tile / subs;
     int g = 0, row0 = 0, rv = 0, nt = 0;
     {
         int rows = 0, before = 0;
@@ -124,8 +126,9 @@ __global__ __launch_bounds__(GS_THREADS * KG, 2) void gemm_small_kernel(const Gs
                 const int l = __builtin_ctzll(hit);
                 const int mt_g = wave_lane(mt, l), in = whole - wave_lane(t0, l);
                 g = g0 + l;
-                int m = in % mt_g;
-                nt = in / mt_g;
+                int m = 0;
+                nt = in;
+                if (mt_g > 1) { nt = in / mt_g; m = in - nt * mt_g; }
                 if constexpr (TAIL) {
                     gg_patch(in, mt_g, nt_all, tm == 128 ? SUP_DUO : SUP, m, nt);
                     nt = nt * (GG_BN / GS_BN) + tile % (GG_BN / GS_BN);
@@ -163,11 +166,15 @@ __global__ __launch_bounds__(GS_THREADS * KG, 2) void gemm_small_kernel(const Gs
     const uint8_t* Bb = p.B + b_at;
     [[maybe_unused]] const long long b_left = (long long)p.E_l * b_group - (long long)b_at;
     uint32_t aoff[RA], boff[RB];
+    int arow[RA];  // (of the lane's rows: all under way together)
 #pragma unroll
-    for (int r = 0; r < RA; ++r) {
-        const int ar = (r * 4 + wave) * 8 + (lane >> 3), lr = min(ar, rv - 1);
-        aoff[r] = (uint32_t)(p.a_map ? max(p.a_map[row0 + lr], 0) : lr) * ldk + ((lane & 7) ^ gg_swz_wide(ar)) * 16;
+    for (int r = 0; r < RA; ++r) arow[r] = min((r * 4 + wave) * 8 + (lane >> 3), rv - 1);
+    if (p.a_map) {
+#pragma unroll
+        for (int r = 0; r < RA; ++r) arow[r] = p.a_map[row0 + arow[r]];
     }
+#pragma unroll
+    for (int r = 0; r < RA; ++r) aoff[r] = (uint32_t)max(arow[r], 0) * ldk + ((lane & 7) ^ gg_swz_wide((r * 4 + wave) * 8 + (lane >> 3))) * 16;
 #pragma unroll
     for (int r = 0; r < RB; ++r) {
         if constexpr (BT) boff[r] = (uint32_t)gg_packed_col<false>(r * 64 + wave * WROWS + (lane >> 2)) * ldb + lchunk * 16;

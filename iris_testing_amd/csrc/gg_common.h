@@ -340,7 +340,7 @@ __host__ __device__ inline int gg_part_stages(int nk, int P) { return ((nk + P -
 
 // GemmParams::zero_tail, by all workgroups of a launch
 __device__ __forceinline__ void gg_zero_tail(const GemmParams& p, int total) {
-    if (!p.zero_tail || total >= p.S_rows) return;
+    if (__builtin_expect(!p.zero_tail || total >= p.S_rows, 1)) return;
     const int nv = p.N / 8;
     const size_t n = (size_t)(p.S_rows - total) * nv;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
