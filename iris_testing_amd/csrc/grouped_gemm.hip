@@ -1057,7 +1057,10 @@ __global__ void zero_pad_rows_kernel(T* __restrict__ out, int K, int Nreal, int 
 // workgroups in flight; hence the long slabs (R = 1: 128 of K, twice the loads under way) and small tiles (256 workgroups of
 // 32 x 32 where 64 x 64 gives 64).  KG = 2, where the tiles are one round: eight waves to a tile, slabs twice as long, every set of four with half of
 // a slab's steps and the second half's sums added at the end: the two GEMMs of the plumbing step 8.0 and 12.4 us with one set, 7.4 and 8.7 with two
-// (fastest launches; on the vector units with 64 x 64 tiles they took 32 and 56).
+// (fastest launches; on the vector units with 64 x 64 tiles they took 32 and 56).  What of the chain need not wait does not: the weights' first slab is asked for
+// before the rows' places are known, the second slab (R = 1) with the first, and the sources' counts beside the counts per expert.  A plumbing step
+// 33.6 -> 31.1 us; rows x K x N of a group: 256 x 1024 x 256 13.0 -> 11.9, 1000 x 516 x 500 of four 15.9 -> 14.2, 4096 x 256 x 512 of eight 24.8 -> 19.6, 4096 x 512 x 1024
+// (R = 2, whose loads no longer jump either) 55 -> 50.
 // R = 2 for launches of many tiles: every operand value out of LDS feeds two matrix instructions.
 // A in LDS as [row][k % 4][k / 4]: the four values a lane needs in four consecutive steps are one 16-byte read; B as
 // [k][column], rows padded so that the four k of a step lie in different banks.
@@ -1075,21 +1078,22 @@ struct F32Side {
     float* rows;
     int32_t* cnt;
 };
-template <int EPI, int R, int KG, int SIDE = F32_ROWS>
+template <int EPI, int R, int KG, int SIDE, bool VEC /* K, N and the bases allow 16-byte loads */>
 __global__ __launch_bounds__(256 * KG) void grouped_gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ Wt,
                                                                 const float* __restrict__ Wup, float* __restrict__ C,
                                                                 const int32_t* __restrict__ cnt, int E_l, int K, int N,
-                                                                int S_rows, bool vec, const F32Side side) {
+                                                                int S_rows, const F32Side side) {
     // PT: 16-byte units of each operand per thread and slab
     constexpr int TM = 32 * R, KC = 128 / R * KG, NTH = 256 * KG, PT = TM * KC / 4 / NTH, STEPS = KC / 16 / KG;
     constexpr int PA = KC + 4, PB = TM + 16;
     constexpr bool UP = EPI == EPI_SWIGLU;
+    constexpr int D = R == 1 && VEC ? 2 : 1;  // slabs under way (many tiles cover each other's loads)
     extern __shared__ __align__(16) float slab[];
     float *const As = slab, *const Bs = As + TM * PA, *const Us = Bs + KC * PB;
     __shared__ int s_g, s_row0, s_rv, s_first;
     constexpr bool RET = SIDE == F32_RETURN, SRC = SIDE == F32_UNPACK;
     __shared__ int32_t s_from[SIDE ? MOE_MAX_EXPERTS : 1], s_slot[SIDE ? MOE_MAX_EXPERTS : 1], s_at[SIDE ? TM : 1];
-    __shared__ int32_t s_rc[SRC ? MOE_MAX_EXPERTS : 1], s_cnt[SRC ? MOE_MAX_EXPERTS : 1];
+    __shared__ int32_t s_rc[SIDE ? MOE_MAX_EXPERTS : 1], s_cnt[SRC ? MOE_MAX_EXPERTS : 1];
     const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
     if constexpr (RET) {
         if ((int)blockIdx.y >= side.tiles_y) {  // padding rows: a wave's share of all slots, slot by slot
@@ -1104,6 +1108,8 @@ __global__ __launch_bounds__(256 * KG) void grouped_gemm_f32_kernel(const float*
             }
             return;
         }
+        if (wave > 0)  // (while the first wave reads the counts)
+            for (int i = threadIdx.x - WAVE; i < side.W * E_l; i += NTH - WAVE) s_rc[i] = side.rc[i];
     }
     if constexpr (SRC) {
         for (int i = threadIdx.x; i < side.W * E_l; i += NTH) s_rc[i] = side.rc[i];
@@ -1117,7 +1123,6 @@ __global__ __launch_bounds__(256 * KG) void grouped_gemm_f32_kernel(const float*
         __syncthreads();
     }
     const int32_t* const counts = SRC ? s_cnt : cnt;
-    const int32_t* const rc = SRC ? s_rc : side.rc;
     if (wave == 0) {  // which expert's rows: 64 experts at a time, tiles and rows before them by a scan
         int mt = blockIdx.y, rs = 0;
         bool found = false;
@@ -1146,6 +1151,11 @@ __global__ __launch_bounds__(256 * KG) void grouped_gemm_f32_kernel(const float*
     const int row0 = s_row0, rv = s_rv, n0 = blockIdx.x * TM;
     const float* W = Wt + (size_t)g * K * N;
     const float* U = UP ? Wup + (size_t)g * K * N : nullptr;
+    auto handover = [] {  // what went to LDS is there; loads stay under way
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
     auto place = [&](int i) {  // row i of the tile: its slot
         const int r = s_first + i;  // of the expert's rows
         int lo = 0, hi = side.W;    // (the last of a run of equal starts owns the row)
@@ -1156,81 +1166,106 @@ __global__ __launch_bounds__(256 * KG) void grouped_gemm_f32_kernel(const float*
         const int m = s_slot[lo] + r - s_from[lo];
         s_at[i] = (unsigned)m < (unsigned)side.M ? lo * side.M + m : -1;  // (past the pair capacity: the row has no slot)
     };
-    if constexpr (SIDE != F32_ROWS) {
-        // where the rows of every source start among the expert's, and among the slots
-        if (wave == 0) {
-            int run = 0;
-            for (int base = 0; base < side.W; base += WAVE) {
-                const int sr = base + lane;
-                int mine = 0, before = 0;
-                if (sr < side.W) {
-                    mine = rc[sr * E_l + g];
+    // where the rows of every source start among the expert's, and among the slots (the first wave)
+    auto sources = [&] {
+        int run = 0;
+        for (int base = 0; base < side.W; base += WAVE) {
+            const int sr = base + lane;
+            int mine = 0, before = 0;
+            if (sr < side.W) {
+                mine = s_rc[sr * E_l + g];
 #pragma unroll 8
-                    for (int e = 0; e < g; ++e) before += rc[sr * E_l + e];
-                }
-                const int incl = wave_incl_scan(mine);
-                if (sr < side.W) { s_from[sr] = run + incl - mine; s_slot[sr] = before; }
-                run += wave_lane(incl, WAVE - 1);
+                for (int e = 0; e < g; ++e) before += s_rc[sr * E_l + e];
             }
+            const int incl = wave_incl_scan(mine);
+            if (sr < side.W) { s_from[sr] = run + incl - mine; s_slot[sr] = before; }
+            run += wave_lane(incl, WAVE - 1);
         }
-        if constexpr (SRC) {
-            __syncthreads();
-            if ((int)threadIdx.x < rv) place(threadIdx.x);
-            __syncthreads();
-        }
-    }
-    float4 ra[PT], rb[PT], ru[UP ? PT : 1];
-    // (vec: K, N and the bases allow 16-byte loads, so a unit lies wholly inside or outside)
-    auto load = [&](const float* p, int at, int end) {
-        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (vec) {
-            if (at < end) v = *reinterpret_cast<const float4*>(p + at);
-        } else {
+    };
+    // Nothing jumps over a 16-byte load: addresses are clamped into the operand, and what lies outside it becomes zero on the way to LDS -- so that the wait
+    // for one slab's loads can leave the next one's under way (D sets of registers).
+    static_assert(NTH % (KC / 4) == 0 && NTH % (TM / 4) == 0, "a thread's units lie below one another");
+    const int ka = threadIdx.x % (KC / 4) * 4, ra0 = threadIdx.x / (KC / 4);            // A: consecutive threads walk K; units NTH / (KC / 4) rows apart
+    const int nb = n0 + threadIdx.x % (TM / 4) * 4, kb0 = threadIdx.x / (TM / 4);       // W: consecutive threads walk N; units NTH / (TM / 4) of K apart
+    float4 ra[D][PT], rb[D][PT], ru[D][UP ? PT : 1];
+    const float* arow[PT];
+    bool aok[PT];
+    auto load = [&](const float* p, int at, int end, [[maybe_unused]] bool ok) {  // (ok: the row exists)
+        if constexpr (VEC) return *reinterpret_cast<const float4*>(p + (at < end ? at : 0));  // (a unit lies wholly inside or outside)
+        else {  // (value by value, and jumped over: the clamped addresses are more work than the jumps, 2000 x 130 x 131 10.0 us against 9.3)
+            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+            end = ok ? end : 0;
             if (at < end) v.x = p[at];
             if (at + 1 < end) v.y = p[at + 1];
             if (at + 2 < end) v.z = p[at + 2];
             if (at + 3 < end) v.w = p[at + 3];
+            return v;
         }
-        return v;
     };
-    auto fetch = [&](int k0) {
+    auto inside = [](const float4& v, bool ok) { return VEC && !ok ? make_float4(0.f, 0.f, 0.f, 0.f) : v; };
+    auto fetch_w = [&](auto d_c, int k0) {
+        constexpr int d = decltype(d_c)::value;
 #pragma unroll
         for (int q = 0; q < PT; ++q) {
-            const int i = threadIdx.x + q * NTH;
-            const int r = i / (KC / 4), k4 = i % (KC / 4);     // A: consecutive threads walk K
-            if constexpr (SRC) {
-                const int at = s_at[min(r, rv - 1)];
-                ra[q] = load(side.buf + (size_t)max(at, 0) * K, k0 + 4 * k4, r < rv && at >= 0 ? K : 0);
-            } else {
-                ra[q] = load(A + (size_t)(row0 + min(r, rv - 1)) * K, k0 + 4 * k4, r < rv ? K : 0);
-            }
-            const int kb = i / (TM / 4), n4 = i % (TM / 4);     // W: consecutive threads walk N
-            const size_t row = (size_t)min(k0 + kb, K - 1) * N;
-            const int end = k0 + kb < K ? N : 0;
-            rb[q] = load(W + row, n0 + 4 * n4, end);
-            if constexpr (UP) ru[q] = load(U + row, n0 + 4 * n4, end);
+            const int kb = k0 + kb0 + q * (NTH / (TM / 4));
+            const size_t row = (size_t)min(kb, K - 1) * N;
+            rb[d][q] = load(W + row, nb, N, kb < K);
+            if constexpr (UP) ru[d][q] = load(U + row, nb, N, kb < K);
         }
     };
+    auto fetch_a = [&](auto d_c, int k0) {
+        constexpr int d = decltype(d_c)::value;
+#pragma unroll
+        for (int q = 0; q < PT; ++q) ra[d][q] = load(arow[q], k0 + ka, K, aok[q]);
+    };
+    typedef std::integral_constant<int, 0> set0;
+    typedef std::integral_constant<int, D - 1> set1;
+    fetch_w(set0{}, 0);
+    if constexpr (SRC) {
+        if (wave == 0) sources();
+        handover();
+        if ((int)threadIdx.x < rv) place(threadIdx.x);
+        handover();
+    }
+#pragma unroll
+    for (int q = 0; q < PT; ++q) {
+        const int r = ra0 + q * (NTH / (KC / 4)), at = SRC ? s_at[min(r, rv - 1)] : row0 + min(r, rv - 1);
+        aok[q] = r < rv && at >= 0;
+        arow[q] = (SRC ? side.buf : A) + (size_t)max(at, 0) * K;
+    }
+    fetch_a(set0{}, 0);
+    if constexpr (D == 2) {
+        fetch_w(set1{}, KC);
+        fetch_a(set1{}, KC);
+    }
+    if constexpr (RET)
+        if (wave == 0) sources();
     const int half = wave / 4;  // which steps of a slab are this wave's
     const int wm = (wave / 2 % 2) * 16 * R, wn = (wave % 2) * 16 * R, l16 = lane % 16, kg = lane / 16;
     floatx4 acc[R][R] = {}, acu[UP ? R : 1][R] = {};
-    fetch(0);
-    for (int k0 = 0; k0 < K; k0 += KC) {
+    typedef std::integral_constant<bool, true> more;
+    typedef std::integral_constant<bool, false> last;
+    auto slab_pass = [&](auto d_c, auto more_c, int k0) {
+        constexpr int d = decltype(d_c)::value;
 #pragma unroll
         for (int q = 0; q < PT; ++q) {
-            const int i = threadIdx.x + q * NTH;
-            float* a = As + (i / (KC / 4)) * PA + i % (KC / 4);
+            const int r = ra0 + q * (NTH / (KC / 4)), kb = kb0 + q * (NTH / (TM / 4));
+            const float4 va = inside(ra[d][q], aok[q] && k0 + ka < K);
             if constexpr (SRC) {  // (rows are multiples of 16 bytes)
-                const int r = i / (KC / 4), k = k0 + i % (KC / 4) * 4;
-                if (blockIdx.x == 0 && r < rv && k < K) *reinterpret_cast<float4*>(side.rows + (size_t)(row0 + r) * K + k) = ra[q];
+                if (blockIdx.x == 0 && r < rv && k0 + ka < K) *reinterpret_cast<float4*>(side.rows + (size_t)(row0 + r) * K + k0 + ka) = va;
             }
-            a[0] = ra[q].x; a[KC / 4] = ra[q].y; a[2 * (KC / 4)] = ra[q].z; a[3 * (KC / 4)] = ra[q].w;
-            const int b = (i / (TM / 4)) * PB + (i % (TM / 4)) * 4;
-            *reinterpret_cast<float4*>(Bs + b) = rb[q];
-            if constexpr (UP) *reinterpret_cast<float4*>(Us + b) = ru[q];
+            float* a = As + r * PA + ka / 4;
+            a[0] = va.x; a[KC / 4] = va.y; a[2 * (KC / 4)] = va.z; a[3 * (KC / 4)] = va.w;
+            const int b = kb * PB + nb - n0;
+            const bool wok = k0 + kb < K && nb < N;
+            *reinterpret_cast<float4*>(Bs + b) = inside(rb[d][q], wok);
+            if constexpr (UP) *reinterpret_cast<float4*>(Us + b) = inside(ru[d][q], wok);
         }
-        __syncthreads();
-        if (k0 + KC < K) fetch(k0 + KC);
+        handover();
+        if (D == 1 ? k0 + KC < K : decltype(more_c)::value) {
+            fetch_w(d_c, k0 + D * KC);
+            fetch_a(d_c, k0 + D * KC);
+        }
         if constexpr (RET)
             if (k0 == 0 && (int)threadIdx.x < rv) place(threadIdx.x);  // (read behind the barrier below)
         // slab positions past K hold zeros: adding +0 products leaves every sum as it is
@@ -1258,7 +1293,17 @@ __global__ __launch_bounds__(256 * KG) void grouped_gemm_f32_kernel(const float*
         } else {
             for (int s4 = 0; s4 < steps; ++s4) step(half * STEPS + s4);
         }
-        __syncthreads();
+        handover();
+    };
+    if constexpr (D == 2) {
+        int k0 = 0;
+        for (; k0 + KC < K; k0 += 2 * KC) {
+            slab_pass(set0{}, more{}, k0);
+            slab_pass(set1{}, more{}, k0 + KC);
+        }
+        if (k0 < K) slab_pass(set0{}, last{}, k0);
+    } else {
+        for (int k0 = 0; k0 < K; k0 += KC) slab_pass(set0{}, more{}, k0);
     }
     if constexpr (KG == 2) {  // the second half's sums, through LDS
         float* const o = slab + (threadIdx.x & 255) * (R * R * 4 * (UP ? 2 : 1));
@@ -1713,7 +1758,7 @@ int launch_f32(const float* A, const float* W, const float* U, float* C, const i
     sd.tiles_y = grid.y;
     if (side == F32_RETURN) grid.y += std::min(ceil_div(std::max(sd.W * sd.M - S_rows, 1), 16 * (int)grid.x), ceil_div(num_cus(), (int)grid.x));
 #define GG_F32_L(EPI, R, KG, SIDE)                                                                                                   \
-    grouped_gemm_f32_kernel<EPI, R, KG, SIDE><<<grid, 256 * KG, gg_f32_lds(R, KG, EPI == EPI_SWIGLU), s>>>(A, W, U, C, cnt, E_l, K, N, S_rows, vec, sd)
+    (vec ? grouped_gemm_f32_kernel<EPI, R, KG, SIDE, true> : grouped_gemm_f32_kernel<EPI, R, KG, SIDE, false>)<<<grid, 256 * KG, gg_f32_lds(R, KG, EPI == EPI_SWIGLU), s>>>(A, W, U, C, cnt, E_l, K, N, S_rows, sd)
 #define GG_F32_K(EPI, R, KG)                                                                                                         \
     do {                                                                                                                             \
         if (side == F32_UNPACK) GG_F32_L(EPI, R, KG, F32_UNPACK);                                                                    \
