@@ -1256,20 +1256,29 @@ __global__ __launch_bounds__(256) void a2a_place_kernel(const A2aSources q, int 
                                                          u32x4* __restrict__ token_buf, int32_t* __restrict__ pca,
                                                          int32_t* __restrict__ counts_ready, int n_ready,
                                                          int32_t* __restrict__ token_sync, int n_sync) {
-    __shared__ int32_t cnt[MOE_MAX_EXPERTS], off[MOE_MAX_EXPERTS], most;
+    // Every workgroup finds the places of all rows, in front of its first one: all counts and starts in one trip to memory, then a scan for each source.  (Counts, then
+    // starts, then a source's experts one after the other: 24000 rows of 1.5 KB from 8 sources to 32 experts 16.7 us, now 16.1.)
+    __shared__ int32_t cnt[MOE_MAX_EXPERTS], off[MOE_MAX_EXPERTS], start[A2A_SRC];
+    __shared__ bool over[256 / WAVE];
     const int tid = threadIdx.x, lane = lane_id();
-    if (tid == 0) most = 0;
-    __syncthreads();
+    bool mine = false;
     for (int i = tid; i < ns * E_l; i += blockDim.x) {
         const int c = a2a_count(q.src[i / E_l], i % E_l);
         cnt[i] = c;
-        if (c > CAP) atomicMax(&most, c);
+        mine |= c > CAP;
     }
+    if (tid < ns) start[tid] = q.src[tid].payload ? *q.src[tid].start : 0;
+    const bool any = __ballot(mine) != 0;
+    if (lane == 0) over[tid / WAVE] = any;
     __syncthreads();
-    if (most > CAP) return;
-    for (int s = tid; s < ns; s += blockDim.x) {
-        int r = q.src[s].payload ? *q.src[s].start : 0;
-        for (int e = 0; e < E_l; ++e) { off[s * E_l + e] = r; r += cnt[s * E_l + e]; }
+    if (over[0] || over[1] || over[2] || over[3]) return;
+    for (int s = tid / WAVE; s < ns; s += blockDim.x / WAVE) {
+        int run = start[s];
+        for (int e0 = 0; e0 < E_l; e0 += WAVE) {
+            const int e = e0 + lane, c = e < E_l ? cnt[s * E_l + e] : 0, incl = wave_incl_scan(c);
+            if (e < E_l) off[s * E_l + e] = run + incl - c;
+            run += wave_lane(incl, WAVE - 1);
+        }
     }
     if (blockIdx.x == 0) {
         for (int i = tid; i < ns * E_l; i += blockDim.x) pca[(i % E_l) * W + s0 + i / E_l] = cnt[i];
